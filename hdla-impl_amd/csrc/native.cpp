@@ -1,0 +1,501 @@
+// Host path of the Python operators: argument checks, allocations, autograd nodes and calls of the C ABI in native code.
+//
+// A call on a few tokens costs the GPU 4 to 30 microseconds; what it cost the host in Python (shape checks, ctypes
+// marshalling, autograd.Function with its decorators, one tensor allocation at a time) was 25 to 250.  Every operator of
+// the package therefore asks here first.  A function of this module takes the arguments of the public operator as they
+// are, and either runs the whole call or, for anything that is not its case (another dtype or head size, tensors on the
+// CPU, shapes that do not fit, ...), returns None without having touched anything: the Python code of the operator then
+// converts, pads or raises as it always did.  So this file holds no error messages of its own; it only recognises what
+// needs none.
+//
+// The kernels stay behind the C ABI of libhdla_hip.so: `bind` receives the handle of the library the package loaded and
+// looks the entry points up in it.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/GradMode.h>
+#include <c10/hip/HIPStream.h>
+#include <dlfcn.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cstdlib>
+#include <cstring>
+#include <string>
+
+#include "../../include/hdla_hip.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+// ---- the C ABI -------------------------------------------------------------------------------------------------------
+struct Api {
+#define HDLA_FN(name) decltype(&hdla_##name) name
+    HDLA_FN(strerror); HDLA_FN(workspace_bytes); HDLA_FN(boundary_bytes); HDLA_FN(chunk_fwd_b); HDLA_FN(chunk_bwd_b);
+    HDLA_FN(recurrent_fwd); HDLA_FN(param_recurrent_fwd); HDLA_FN(normalize_fwd); HDLA_FN(normalize_bwd);
+    HDLA_FN(normalize_workspace_bytes);
+#undef HDLA_FN
+} api;
+PyObject* error_class = nullptr;                 // _lib.HdlaError
+PyObject* memory_error = nullptr;                // torch.OutOfMemoryError
+
+// what _lib.check raises: "<entry point> failed with code <rc>: <text>"
+struct AbiError : std::runtime_error { using std::runtime_error::runtime_error; };
+void check(int rc, const char* what) {
+    if (rc) throw AbiError(std::string(what) + " failed with code " + std::to_string(rc) + ": " + api.strerror(rc));
+}
+
+// The same on a thread of the autograd engine: the Python exception is set here and carried by the engine to the caller.
+template <typename F> auto in_backward(F fn) {
+    try {
+        return fn();
+    } catch (const AbiError& e) {
+        const PyGILState_STATE gil = PyGILState_Ensure();
+        PyErr_SetString(error_class ? error_class : PyExc_RuntimeError, e.what());
+        python_error err;
+        err.persist();
+        PyGILState_Release(gil);
+        throw err;
+    }
+}
+
+// an autograd function takes defined tensors, or std::optional
+using Maybe = std::optional<Tensor>;
+inline Maybe maybe(const Tensor& t) { return t.defined() ? Maybe(t) : Maybe(); }
+inline Tensor value(const Maybe& t) { return t ? *t : Tensor(); }
+
+inline void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+inline float* fptr(const Tensor& t) { return static_cast<float*>(ptr(t)); }
+inline void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+inline int dtype_code(at::ScalarType t) { return t == at::kBFloat16 ? HDLA_BF16 : HDLA_FP32; }
+inline bool native_dtype(at::ScalarType t) { return t == at::kBFloat16 || t == at::kFloat; }
+inline Tensor bytes_like(const Tensor& t, size_t n) { return at::empty({(int64_t)n}, t.options().dtype(at::kByte)); }
+
+// the package's environment switches, read on every call like the Python code does
+bool env_is(const char* name, std::initializer_list<const char*> values, bool unset) {
+    const char* v = getenv(name);
+    if (!v) return unset;
+    for (const char* x : values) if (!strcmp(v, x)) return true;
+    return false;
+}
+bool keep_forward_default() { return !env_is("HDLA_HIP_KEEP_FORWARD", {"", "0", "false", "False"}, true); }
+bool keep_boundaries_default() { return env_is("HDLA_HIP_INPUTS_ONLY", {"", "0", "false", "False"}, true); }
+// false: the Python code has to look at it (another spelling, a number that is none)
+bool route_and_segments(hdla_dims& d) {
+    const char* r = getenv("HDLA_HIP_ROUTE");
+    if (!r || !*r || !strcmp(r, "auto")) d.route = HDLA_ROUTE_AUTO;
+    else if (!strcmp(r, "classic")) d.route = HDLA_ROUTE_CLASSIC;
+    else if (!strcmp(r, "fused")) d.route = HDLA_ROUTE_FUSED;
+    else return false;
+    const char* s = getenv("HDLA_HIP_SEGMENTS");
+    if (!s) { d.segments = 0; return true; }
+    char* end = nullptr;
+    d.segments = (int32_t)strtol(s, &end, 10);
+    return *s && !*end;
+}
+
+// ---- the chunked operators -------------------------------------------------------------------------------------------
+// a and b, or beta (the other undefined)
+struct ChunkIn {
+    Tensor q, k, v, a, b, beta, gk, h0, cu;
+};
+
+bool chunk_dims(const ChunkIn& x, double scale, hdla_dims& d) {
+    d = hdla_dims{};
+    d.B = (int32_t)x.q.size(0); d.T = (int32_t)x.q.size(1); d.H = (int32_t)x.q.size(2); d.K = (int32_t)x.q.size(3);
+    d.V = (int32_t)x.v.size(3); d.R = 2;
+    d.N = x.cu.defined() ? (int32_t)(x.cu.numel() - 1) : d.B;
+    d.in_dtype = dtype_code(x.q.scalar_type());
+    d.gk_dtype = dtype_code(x.gk.scalar_type());
+    d.scale = (float)scale;
+    d.cu_seqlens = x.cu.defined() ? x.cu.data_ptr<int64_t>() : nullptr;
+    return route_and_segments(d);
+}
+
+Tensor workspace(const hdla_dims& d, int pass, const Tensor& like) {
+    const size_t n = api.workspace_bytes(&d, pass);
+    if (!n) throw AbiError("hdla_workspace_bytes rejected the dimensions (B=" + std::to_string(d.B) + ",T=" + std::to_string(d.T) +
+                           ",H=" + std::to_string(d.H) + ",K=" + std::to_string(d.K) + ",V=" + std::to_string(d.V) +
+                           ",R=" + std::to_string(d.R) + ",N=" + std::to_string(d.N) + ")");
+    return bytes_like(like, n);
+}
+
+// rows outside every sequence of a packed batch are written by nobody: zeros there
+Tensor fresh(const Tensor& like, bool packed) { return packed ? at::zeros_like(like) : at::empty_like(like); }
+
+void chunk_forward(const ChunkIn& x, const hdla_dims& d, bool want_ht, bool want_boundary, Tensor& o, Tensor& ht, Tensor& boundary) {
+    const auto f32 = x.q.options().dtype(at::kFloat);
+    o = fresh(x.v, x.cu.defined());
+    if (want_ht) ht = at::empty({d.N, d.H, d.K, d.V}, f32);
+    const size_t nb = want_boundary ? api.boundary_bytes(&d) : 0;
+    if (nb) boundary = bytes_like(x.q, nb);
+    const Tensor ws = workspace(d, HDLA_PASS_FWD, x.q);
+    check(api.chunk_fwd_b(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.beta), ptr(x.gk), fptr(x.h0), ptr(o), fptr(ht),
+                          ptr(boundary), nb, ptr(ws), (size_t)ws.numel(), stream_of(x.q)), "hdla_chunk_fwd_b");
+}
+
+// The autograd node: the contract of ChunkDPLRDeltaRuleFunction and ChunkHDLAFunction (the inputs and, where the route
+// has one, the record of the states at the segment boundaries are saved; everything else is recomputed).
+struct ChunkFn : torch::autograd::Function<ChunkFn> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Maybe& a, const Maybe& b,
+                                 const Maybe& beta, const Tensor& gk, const Maybe& h0, const Maybe& cu, double scale, bool want_ht) {
+        ChunkIn x{q, k, v, value(a), value(b), value(beta), gk, value(h0), value(cu)};
+        if (h0) x.h0 = h0->to(at::kFloat).contiguous();
+        hdla_dims d;
+        chunk_dims(x, scale, d);
+        Tensor o, ht, boundary;
+        chunk_forward(x, d, want_ht, keep_boundaries_default(), o, ht, boundary);
+        ctx->save_for_backward({q, k, v, x.a, x.b, x.beta, gk, value(h0), x.cu, boundary});
+        ctx->saved_data["scale"] = scale;
+        ctx->set_materialize_grads(false);
+        return want_ht ? variable_list{o, ht} : variable_list{o};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        return in_backward([&] { return gradients(ctx, grads); });
+    }
+    static variable_list gradients(AutogradContext* ctx, const variable_list& grads) {
+        const auto s = ctx->get_saved_variables();
+        ChunkIn x{s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7], s[8]};
+        const Tensor& boundary = s[9];
+        const at::DeviceGuard guard(x.q.device());
+        if (x.h0.defined()) x.h0 = x.h0.to(at::kFloat).contiguous();
+        hdla_dims d;
+        chunk_dims(x, ctx->saved_data["scale"].toDouble(), d);
+        const Tensor d_o = grads[0].defined() ? grads[0].to(x.v.scalar_type()).contiguous() : at::zeros_like(x.v);
+        Tensor dht;
+        if (grads.size() > 1 && grads[1].defined()) dht = grads[1].to(at::kFloat).contiguous();
+        const bool packed = x.cu.defined();
+        const Tensor ws = workspace(d, HDLA_PASS_BWD, x.q);
+        const Tensor dq = fresh(x.q, packed), dk = fresh(x.k, packed), dv = fresh(x.v, packed), dgk = fresh(x.gk, packed);
+        Tensor da, db, dbeta, dh0;
+        if (x.beta.defined()) dbeta = fresh(x.beta, packed);
+        else { da = fresh(x.a, packed); db = fresh(x.b, packed); }
+        if (x.h0.defined()) dh0 = at::empty_like(x.h0);
+        check(api.chunk_bwd_b(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.beta), ptr(x.gk), fptr(x.h0), ptr(d_o), fptr(dht),
+                              ptr(dq), ptr(dk), ptr(dv), ptr(da), ptr(db), ptr(dbeta), ptr(dgk), fptr(dh0), ptr(boundary),
+                              boundary.defined() ? (size_t)boundary.numel() : 0, ptr(ws), (size_t)ws.numel(), stream_of(x.q)),
+              "hdla_chunk_bwd_b");
+        if (dh0.defined()) dh0 = dh0.to(s[7].scalar_type());
+        return {dq, dk, dv, da, db, dbeta, dgk, dh0, Tensor(), Tensor(), Tensor()};
+    }
+};
+
+// ---- reading the Python arguments ------------------------------------------------------------------------------------
+// a plain tensor (or parameter): no subclass, nothing that overrides torch functions
+inline bool is_tensor(PyObject* o) { return THPVariable_CheckExact(o); }
+inline const Tensor& unpack(PyObject* o) { return THPVariable_Unpack(o); }
+inline bool truth(PyObject* o, bool& out) {
+    const int r = PyObject_IsTrue(o);
+    if (r < 0) PyErr_Clear();
+    out = r > 0;
+    return r >= 0;
+}
+inline bool number(PyObject* o, double& out) {
+    out = PyFloat_AsDouble(o);
+    if (out == -1.0 && PyErr_Occurred()) { PyErr_Clear(); return false; }
+    return true;
+}
+inline bool gpu_like(const Tensor& t, const at::Device& dev) { return t.device() == dev && t.layout() == at::kStrided && !t.is_complex(); }
+inline bool same_sizes(const Tensor& t, std::initializer_list<int64_t> s) { return t.sizes() == at::IntArrayRef(s); }
+
+// What the chunked and the token-serial operators have in common: q, k, v, gk, the states and the sequence table.
+// False: not a case of this file.
+bool read_operands(PyObject* pq, PyObject* pk, PyObject* pv, PyObject* pgk, PyObject* ph0, PyObject* pcu, bool serial, ChunkIn& x) {
+    if (!api.strerror || !is_tensor(pq) || !is_tensor(pk) || !is_tensor(pv) || !is_tensor(pgk)) return false;
+    const Tensor &q = unpack(pq), &k = unpack(pk), &v = unpack(pv), &gk = unpack(pgk);
+    const auto dt = q.scalar_type();
+    const at::Device dev = q.device();
+    if (!dev.is_cuda() || !native_dtype(dt) || k.scalar_type() != dt || v.scalar_type() != dt) return false;
+    if (gk.scalar_type() != dt && gk.scalar_type() != at::kFloat) return false;
+    if (q.dim() != 4 || v.dim() != 4 || k.sizes() != q.sizes() || gk.sizes() != q.sizes()) return false;
+    if (!gpu_like(q, dev) || !gpu_like(k, dev) || !gpu_like(v, dev) || !gpu_like(gk, dev)) return false;
+    const int64_t B = q.size(0), T = q.size(1), H = q.size(2), K = q.size(3), V = v.size(3);
+    const auto native = [&](int64_t d) { return d == 64 || d == 128 || (serial && d == 256); };
+    if (!native(K) || !native(V) || v.size(0) != B || v.size(1) != T || v.size(2) != H || B < 1 || T < 1 || H < 1) return false;
+    if (B > INT32_MAX || T > INT32_MAX / 4 || H > 65535) return false;
+    int64_t N = B;
+    if (pcu != Py_None) {
+        if (!is_tensor(pcu)) return false;
+        const Tensor& cu = unpack(pcu);
+        if (cu.device() != dev || cu.scalar_type() != at::kLong || cu.dim() != 1 || cu.numel() < 2 || B != 1) return false;
+        N = cu.numel() - 1;
+        x.cu = cu.contiguous();
+    }
+    if (ph0 != Py_None) {
+        if (!is_tensor(ph0)) return false;
+        const Tensor& h0 = unpack(ph0);
+        if (!gpu_like(h0, dev) || !same_sizes(h0, {N, H, K, V}) || !h0.is_floating_point()) return false;
+        x.h0 = h0;
+    }
+    x.q = q; x.k = k; x.v = v; x.gk = gk;
+    return true;
+}
+bool read_ab(PyObject* pa, PyObject* pb, ChunkIn& x) {
+    if (!is_tensor(pa) || !is_tensor(pb)) return false;
+    const Tensor &a = unpack(pa), &b = unpack(pb);
+    const auto s = x.q.sizes();
+    if (a.scalar_type() != x.q.scalar_type() || b.scalar_type() != x.q.scalar_type() || !gpu_like(a, x.q.device()) || !gpu_like(b, x.q.device()))
+        return false;
+    if (!same_sizes(a, {s[0], 2 * s[1], s[2], s[3]}) || !same_sizes(b, {s[0], 2 * s[1], s[2], s[3]})) return false;
+    x.a = a; x.b = b;
+    return true;
+}
+// beta [B,T,H] or [B,T,H,1]; keeps the tensor as given
+bool read_beta(PyObject* p, ChunkIn& x) {
+    if (!is_tensor(p)) return false;
+    const Tensor& t = unpack(p);
+    const auto s = x.q.sizes();
+    if (t.scalar_type() != x.q.scalar_type() || !gpu_like(t, x.q.device())) return false;
+    if (!same_sizes(t, {s[0], s[1], s[2], 1}) && !same_sizes(t, {s[0], s[1], s[2]})) return false;
+    x.beta = t;
+    return true;
+}
+inline bool wants_grad(const Tensor& t) { return t.defined() && t.requires_grad(); }
+bool any_grad(const ChunkIn& x) {
+    return c10::GradMode::is_enabled() && (wants_grad(x.q) || wants_grad(x.k) || wants_grad(x.v) || wants_grad(x.a) || wants_grad(x.b) ||
+                                           wants_grad(x.beta) || wants_grad(x.gk) || wants_grad(x.h0));
+}
+void make_contiguous(ChunkIn& x) {
+    x.q = x.q.contiguous(); x.k = x.k.contiguous(); x.v = x.v.contiguous(); x.gk = x.gk.contiguous();
+    if (x.a.defined()) { x.a = x.a.contiguous(); x.b = x.b.contiguous(); }
+    if (x.beta.defined()) x.beta = x.beta.contiguous();
+}
+
+PyObject* none() { Py_RETURN_NONE; }
+PyObject* wrap_or_none(const Tensor& t) { return t.defined() ? THPVariable_Wrap(t) : none(); }
+PyObject* pair(const Tensor& a, const Tensor& b) {
+    PyObject* r = PyTuple_New(2);
+    if (!r) return nullptr;
+    PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(a));
+    PyTuple_SET_ITEM(r, 1, wrap_or_none(b));
+    return r;
+}
+
+// runs fn, turning C++ exceptions into Python ones
+template <typename F> PyObject* guarded(F fn) {
+    try {
+        return fn();
+    } catch (const AbiError& e) {
+        PyErr_SetString(error_class ? error_class : PyExc_RuntimeError, e.what());
+    } catch (const c10::OutOfMemoryError& e) {
+        PyErr_SetString(memory_error ? memory_error : PyExc_MemoryError, e.what_without_backtrace());
+    } catch (const c10::Error& e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
+    } catch (const std::exception& e) {
+        if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
+    }
+    return nullptr;
+}
+
+PyObject* run_chunk(ChunkIn& x, PyObject* pscale, PyObject* pwant, PyObject* pkeep) {
+    bool want = false, keep = false;
+    double scale = 0;
+    if (!truth(pwant, want)) return none();
+    if (pkeep == Py_None ? keep_forward_default() : (!truth(pkeep, keep) || keep)) return none();
+    if (pscale == Py_None) scale = std::pow((double)x.q.size(3), -0.5);
+    else if (!number(pscale, scale)) return none();
+    hdla_dims d;
+    return guarded([&]() -> PyObject* {
+        if (!chunk_dims(x, scale, d)) return none();
+        const at::DeviceGuard guard(x.q.device());
+        make_contiguous(x);
+        if (any_grad(x)) {
+            const auto r = ChunkFn::apply(x.q, x.k, x.v, maybe(x.a), maybe(x.b), maybe(x.beta), x.gk, maybe(x.h0), maybe(x.cu), scale, want);
+            return pair(r[0], want ? r[1] : Tensor());
+        }
+        if (x.h0.defined()) x.h0 = x.h0.to(at::kFloat).contiguous();
+        Tensor o, ht, boundary;
+        chunk_forward(x, d, want, false, o, ht, boundary);
+        return pair(o, ht);
+    });
+}
+
+// chunk(q, k, v, a, b, gk, RANK_AB, scale, initial_state, output_final_state, head_first, chunk_size, cu_seqlens, keep_forward)
+PyObject* py_chunk(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 14) return none();
+    ChunkIn x;
+    bool head_first = false;
+    if (!PyLong_CheckExact(a[6]) || PyLong_AsLong(a[6]) != 2 || !PyLong_CheckExact(a[11]) || PyLong_AsLong(a[11]) < 1) { PyErr_Clear(); return none(); }
+    if (!truth(a[10], head_first) || head_first) return none();
+    if (!read_operands(a[0], a[1], a[2], a[5], a[8], a[12], false, x) || !read_ab(a[3], a[4], x)) return none();
+    return run_chunk(x, a[7], a[9], a[13]);
+}
+
+// chunk_hdla(q, k, v, beta, log_f, scale, initial_state, output_final_state, cu_seqlens, keep_forward)
+PyObject* py_chunk_hdla(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 10) return none();
+    ChunkIn x;
+    if (!read_operands(a[0], a[1], a[2], a[4], a[6], a[8], false, x) || !read_beta(a[3], x)) return none();
+    return run_chunk(x, a[5], a[7], a[9]);
+}
+
+// ---- the token-serial operators: no gradients ------------------------------------------------------------------------
+PyObject* run_recurrent(ChunkIn& x, PyObject* pscale, PyObject* pwant, PyObject* preverse) {
+    bool want = false, reverse = false;
+    double scale = 0;
+    if (any_grad(x) || !truth(pwant, want) || !truth(preverse, reverse)) return none();
+    if (pscale == Py_None) scale = std::pow((double)x.q.size(3), -0.5);
+    else if (!number(pscale, scale)) return none();
+    hdla_dims d;
+    return guarded([&]() -> PyObject* {
+        if (!chunk_dims(x, scale, d)) return none();
+        const at::DeviceGuard guard(x.q.device());
+        make_contiguous(x);
+        if (x.h0.defined()) x.h0 = x.h0.to(at::kFloat).contiguous();
+        const Tensor o = fresh(x.v, x.cu.defined());
+        Tensor ht;
+        if (want) ht = at::empty({d.N, d.H, d.K, d.V}, x.q.options().dtype(at::kFloat));
+        if (x.beta.defined())
+            check(api.param_recurrent_fwd(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.beta), ptr(x.gk), reverse, fptr(x.h0), ptr(o), fptr(ht),
+                                          stream_of(x.q)), "hdla_param_recurrent_fwd");
+        else
+            check(api.recurrent_fwd(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.gk), reverse, fptr(x.h0), ptr(o), fptr(ht),
+                                    stream_of(x.q)), "hdla_recurrent_fwd");
+        return pair(o, ht);
+    });
+}
+
+// recurrent(q, k, v, a, b, gk, rank_ab, scale, initial_state, output_final_state, reverse, cu_seqlens, head_first)
+PyObject* py_recurrent(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 13) return none();
+    ChunkIn x;
+    bool head_first = false;
+    if (!PyLong_CheckExact(a[6]) || PyLong_AsLong(a[6]) != 2) { PyErr_Clear(); return none(); }
+    if (!truth(a[12], head_first) || head_first) return none();
+    if (!read_operands(a[0], a[1], a[2], a[5], a[8], a[11], true, x) || !read_ab(a[3], a[4], x)) return none();
+    return run_recurrent(x, a[7], a[9], a[10]);
+}
+
+// recurrent_hdla(q, k, v, beta, log_f, scale, initial_state, output_final_state, reverse, cu_seqlens)
+PyObject* py_recurrent_hdla(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 10) return none();
+    ChunkIn x;
+    if (!read_operands(a[0], a[1], a[2], a[4], a[6], a[9], true, x) || !read_beta(a[3], x)) return none();
+    return run_recurrent(x, a[5], a[7], a[8]);
+}
+
+// ---- the fused normalisation -----------------------------------------------------------------------------------------
+hdla_norm_dims norm_dims(const Tensor& x, const Tensor& w, int gate_pos, double c, double eps, int64_t groups) {
+    hdla_norm_dims d{};
+    const int64_t D = x.size(-1);
+    d.rows = D ? x.numel() / D : 0;
+    d.G = (int32_t)groups; d.E = (int32_t)(D / groups);
+    d.dtype = dtype_code(x.scalar_type());
+    d.weight_dtype = w.defined() ? dtype_code(w.scalar_type()) : HDLA_FP32;
+    d.gate_pos = gate_pos; d.c = (float)c; d.eps = (float)eps;
+    return d;
+}
+Tensor norm_forward(const Tensor& x, const Tensor& w, const Tensor& gate, const hdla_norm_dims& d) {
+    Tensor o = at::empty_like(x);
+    check(api.normalize_fwd(&d, ptr(x), ptr(w), ptr(gate), ptr(o), stream_of(x)), "hdla_normalize_fwd");
+    return o;
+}
+struct NormFn : torch::autograd::Function<NormFn> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, const Maybe& weight, const Maybe& g, int64_t gate_pos, double c, double eps,
+                          int64_t groups) {
+        const Tensor w = value(weight), gate = value(g);
+        ctx->save_for_backward({x, w, gate});
+        ctx->saved_data["p"] = gate_pos; ctx->saved_data["c"] = c; ctx->saved_data["e"] = eps; ctx->saved_data["g"] = groups;
+        return norm_forward(x, w, gate, norm_dims(x, w, (int)gate_pos, c, eps, groups));
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        return in_backward([&] { return gradients(ctx, grads); });
+    }
+    static variable_list gradients(AutogradContext* ctx, const variable_list& grads) {
+        const auto s = ctx->get_saved_variables();
+        const Tensor &x = s[0], &w = s[1], &gate = s[2];
+        const at::DeviceGuard guard(x.device());
+        const hdla_norm_dims d = norm_dims(x, w, (int)ctx->saved_data["p"].toInt(), ctx->saved_data["c"].toDouble(),
+                                           ctx->saved_data["e"].toDouble(), ctx->saved_data["g"].toInt());
+        const Tensor d_o = grads[0].to(x.scalar_type()).contiguous();
+        const Tensor dx = at::empty_like(x);
+        Tensor dgate, dw, ws;
+        if (gate.defined()) dgate = at::empty_like(x);
+        size_t nws = 0;
+        if (w.defined()) {
+            dw = at::empty({x.size(-1)}, x.options().dtype(at::kFloat));
+            nws = api.normalize_workspace_bytes(&d);
+            ws = bytes_like(x, nws < 16 ? 16 : nws);
+        }
+        check(api.normalize_bwd(&d, ptr(x), ptr(w), ptr(gate), ptr(d_o), ptr(dx), ptr(dgate), fptr(dw), ptr(ws), nws, stream_of(x)),
+              "hdla_normalize_bwd");
+        if (dw.defined()) dw = dw.to(w.scalar_type()).reshape(w.sizes());
+        return {dx, dw, dgate, Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+// normalize(x, weight, bias, residual, gate, gate_act, gate_pos, c, eps, use_mean, num_groups, return_residual)
+PyObject* py_normalize(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 12 || !api.strerror || !is_tensor(a[0]) || a[2] != Py_None || a[3] != Py_None || a[9] != Py_False || a[11] != Py_False) return none();
+    Tensor x = unpack(a[0]), w, gate;
+    const at::Device dev = x.device();
+    if (!dev.is_cuda() || !native_dtype(x.scalar_type()) || !gpu_like(x, dev) || x.dim() < 1) return none();
+    const int64_t D = x.size(-1);
+    if (!PyLong_CheckExact(a[10])) return none();
+    const int64_t groups = PyLong_AsLongLong(a[10]);
+    if (groups < 1 || D < 1 || D % groups) { PyErr_Clear(); return none(); }
+    if (a[1] != Py_None) {
+        if (!is_tensor(a[1])) return none();
+        w = unpack(a[1]);
+        if (!gpu_like(w, dev) || !native_dtype(w.scalar_type()) || w.numel() != D) return none();
+    }
+    int64_t pos = 0;
+    if (a[4] != Py_None) {
+        if (!is_tensor(a[4]) || !PyUnicode_Check(a[5]) || PyUnicode_CompareWithASCIIString(a[5], "sigmoid") || !PyUnicode_Check(a[6])) return none();
+        gate = unpack(a[4]);
+        pos = !PyUnicode_CompareWithASCIIString(a[6], "pre") ? 1 : !PyUnicode_CompareWithASCIIString(a[6], "post") ? 2 : 0;
+        if (!pos || !gpu_like(gate, dev) || gate.sizes() != x.sizes() || gate.scalar_type() != x.scalar_type()) return none();
+    }
+    double c = 0, eps = 0;
+    if (!number(a[7], c) || !number(a[8], eps)) return none();
+    return guarded([&]() -> PyObject* {
+        const at::DeviceGuard guard(dev);
+        x = x.contiguous();
+        if (w.defined()) w = w.contiguous();
+        if (gate.defined()) gate = gate.contiguous();
+        if (c10::GradMode::is_enabled() && (wants_grad(x) || wants_grad(w) || wants_grad(gate)))
+            return THPVariable_Wrap(NormFn::apply(x, maybe(w), maybe(gate), pos, c, eps, groups));
+        return THPVariable_Wrap(norm_forward(x, w, gate, norm_dims(x, w, (int)pos, c, eps, groups)));
+    });
+}
+
+// ---- module ----------------------------------------------------------------------------------------------------------
+// bind(handle of libhdla_hip.so, HdlaError, torch.OutOfMemoryError)
+PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 3) { PyErr_SetString(PyExc_TypeError, "bind(handle, error, memory_error)"); return nullptr; }
+    void* h = PyLong_AsVoidPtr(a[0]);
+    if (!h) { if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "no library"); return nullptr; }
+    Api x{};
+#define HDLA_FN(name)                                                                                              \
+    if (!(x.name = reinterpret_cast<decltype(x.name)>(dlsym(h, "hdla_" #name)))) {                                 \
+        PyErr_SetString(a[1], "the library does not export hdla_" #name);                                          \
+        return nullptr;                                                                                            \
+    }
+    HDLA_FN(strerror) HDLA_FN(workspace_bytes) HDLA_FN(boundary_bytes) HDLA_FN(chunk_fwd_b) HDLA_FN(chunk_bwd_b)
+    HDLA_FN(recurrent_fwd) HDLA_FN(param_recurrent_fwd) HDLA_FN(normalize_fwd) HDLA_FN(normalize_bwd)
+    HDLA_FN(normalize_workspace_bytes)
+#undef HDLA_FN
+    Py_INCREF(a[1]);
+    Py_XDECREF(error_class);
+    error_class = a[1];
+    Py_INCREF(a[2]);
+    Py_XDECREF(memory_error);
+    memory_error = a[2];
+    api = x;
+    return none();
+}
+
+#define HDLA_DEF(name, fn) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(fn)), METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {
+    HDLA_DEF("bind", py_bind), HDLA_DEF("chunk", py_chunk), HDLA_DEF("chunk_hdla", py_chunk_hdla), HDLA_DEF("recurrent", py_recurrent),
+    HDLA_DEF("recurrent_hdla", py_recurrent_hdla), HDLA_DEF("normalize", py_normalize), {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__native() { return PyModule_Create(&module); }

@@ -15,6 +15,7 @@ _ROUTES = {"": ROUTE_AUTO, "auto": ROUTE_AUTO, "classic": ROUTE_CLASSIC, "fused"
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB_NAME = "libhdla_hip.so"
 _lib = None
+_native = None
 
 
 class HdlaDims(ctypes.Structure):
@@ -128,6 +129,22 @@ def load():
     lib.hdla_skinny_wgrad_workspace_bytes.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int32, ctypes.c_int32]
     _lib = lib
     return lib
+
+
+def native():
+    """The operators' native host path (csrc/native.cpp), bound to the loaded library.  Its functions take the arguments
+    of the public operators; they return None, having done nothing, for a call that is not theirs."""
+    global _native
+    if _native is None:
+        lib = load()
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise HdlaError(f"the native host path could not be loaded ({e}): build it with the library "
+                            "(make -C hdla-impl_amd/csrc)") from e
+        module.bind(lib._handle, HdlaError, torch.OutOfMemoryError)
+        _native = module
+    return _native
 
 
 def check(rc: int, what: str) -> None:

@@ -249,6 +249,10 @@ def chunk_hrdplr_delta_rule(
     them; False (and None without HDLA_HIP_KEEP_FORWARD=1 in the environment) is the reference's behaviour: only the
     inputs are kept (hrdplr.py:137) and the backward pass recomputes (:161-198).  Results agree to rounding.
     """
+    out = _lib.native().chunk(q, k, v, a, b, gk, RANK_AB, scale, initial_state, output_final_state, head_first, chunk_size,
+                              cu_seqlens, keep_forward)
+    if out is not None:
+        return out
     assert head_first is False or head_first == 0, "only head_first=False is supported (HRDPLR/fwd_func.py:28)"
     assert q.dtype == k.dtype == v.dtype                                                   # hrdplr.py:301
     if RANK_AB not in (1, 2):
@@ -292,10 +296,11 @@ def chunk_hrdplr_delta_rule(
     h0 = initial_state
     if h0 is not None and (Kn != K or Vn != V):
         h0 = F.pad(h0, (0, Vn - V, 0, Kn - K))
-    o, final_state = ChunkDPLRDeltaRuleFunction.apply(
-        _pad_last(q, Kn), _pad_last(k, Kn), _pad_last(v, Vn), _pad_last(a2, Kn), _pad_last(b2, Kn), _pad_last(gk, Kn),
-        scale, h0, output_final_state, 2, head_first, chunk_size, cu_seqlens,
-        _lib.keep_forward_default() if keep_forward is None else bool(keep_forward))
+    ops = [_pad_last(x, n) for x, n in ((q, Kn), (k, Kn), (v, Vn), (a2, Kn), (b2, Kn), (gk, Kn))]
+    keep = _lib.keep_forward_default() if keep_forward is None else bool(keep_forward)
+    out = _lib.native().chunk(*ops, 2, scale, h0, output_final_state, head_first, chunk_size, cu_seqlens, keep)
+    o, final_state = out if out is not None else ChunkDPLRDeltaRuleFunction.apply(
+        *ops, scale, h0, output_final_state, 2, head_first, chunk_size, cu_seqlens, keep)
     if Vn != V:
         o = o[..., :V]
     if final_state is not None and (Kn != K or Vn != V):

@@ -112,6 +112,9 @@ def chunk_hdla_delta_rule(
     b (rounded to q's dtype, as ``hdla_custom.py:301-304`` does) formed inside the kernels.  Returns ``(o, final_state)``
     like the plain operator; gradients flow to q, k, v, beta, log_f and initial_state.  ``keep_forward``: as for
     ``chunk_hrdplr_delta_rule``."""
+    out = _lib.native().chunk_hdla(q, k, v, beta, log_f, scale, initial_state, output_final_state, cu_seqlens, keep_forward)
+    if out is not None:
+        return out
     assert q.dtype == k.dtype == v.dtype
     if q.dim() != 4 or v.dim() != 4:
         raise ValueError("q, k, v must be 4-dimensional [B, T, H, D]")
@@ -149,9 +152,10 @@ def chunk_hdla_delta_rule(
     h0 = initial_state
     if h0 is not None and (Kn != K or Vn != V):
         h0 = F.pad(h0, (0, Vn - V, 0, Kn - K))
-    o, final_state = ChunkHDLAFunction.apply(_pad_last(q, Kn), _pad_last(k, Kn), _pad_last(v, Vn), beta,
-                                             _pad_last(gk, Kn), scale, h0, output_final_state, cu_seqlens,
-                                             _lib.keep_forward_default() if keep_forward is None else bool(keep_forward))
+    ops = (_pad_last(q, Kn), _pad_last(k, Kn), _pad_last(v, Vn), beta, _pad_last(gk, Kn), scale, h0, output_final_state,
+           cu_seqlens, _lib.keep_forward_default() if keep_forward is None else bool(keep_forward))
+    out = _lib.native().chunk_hdla(*ops)
+    o, final_state = out if out is not None else ChunkHDLAFunction.apply(*ops)
     if Vn != V:
         o = o[..., :V]
     if final_state is not None and (Kn != K or Vn != V):
@@ -175,6 +179,9 @@ def fused_recurrent_hdla_delta_rule(
     """``fused_recurrent_dplr_delta_rule(q, k, v, *parameterize_a_b(beta, k, log_f), gk=log_f, rank_ab=2, ...)``
     with a and b (rounded to q's dtype) formed per token inside the kernel.  Inference only: no gradients, like
     the plain recurrent operator (HRDPLR/recurrent.py:219-224)."""
+    out = _lib.native().recurrent_hdla(q, k, v, beta, log_f, scale, initial_state, output_final_state, reverse, cu_seqlens)
+    if out is not None:
+        return out
     assert q.dtype == k.dtype == v.dtype
     if q.dim() != 4 or v.dim() != 4:
         raise ValueError("q, k, v must be 4-dimensional [B, T, H, D]")

@@ -93,6 +93,10 @@ def normalize_fn(
     """``o = c / sqrt(E) * x' / sqrt(mean_E(x'^2) + eps) * weight`` per group of ``E = D / num_groups`` channels of the
     last dimension, with ``x' = x * sigmoid(gate)`` (``gate_pos == "pre"``) or ``o * sigmoid(gate)`` afterwards
     (``"post"``).  Signature of normalize_triton.py:452-465; ``o`` has ``x``'s dtype and shape."""
+    o = _lib.native().normalize(x, weight, bias, residual, gate, gate_act, gate_pos, c, eps, use_mean, num_groups,
+                                return_residual)
+    if o is not None:
+        return o
     assert x.shape[-1] % num_groups == 0, "The last dimension of x must be divisible by num_groups"
     if bias is not None or residual is not None or return_residual or use_mean:
         raise NotImplementedError("hdla_hip.normalize_fn covers the forms the HDLA layer uses: no bias, no residual, "

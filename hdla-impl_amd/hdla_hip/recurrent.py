@@ -86,6 +86,10 @@ def fused_recurrent_dplr_delta_rule(
     ``[N, H, K, V]``, ``cu_seqlens`` packs N sequences into a batch of one; returns ``(o, final_state)`` with
     ``o`` in ``v``'s dtype and ``final_state`` fp32 or ``None``.
     """
+    out = _lib.native().recurrent(q, k, v, a, b, gk, rank_ab, scale, initial_state, output_final_state, reverse, cu_seqlens,
+                                  head_first)
+    if out is not None:
+        return out
     assert head_first == False, ""                                                          # recurrent.py:276
     if cu_seqlens is not None:
         if q.shape[0] != 1:

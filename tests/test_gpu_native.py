@@ -1,0 +1,58 @@
+"""The operators' native host path (csrc/native.cpp): what it takes gives the bits of the Python autograd functions it
+stands in front of, and what is not its case it leaves alone."""
+import pytest
+import torch
+
+from hdla_hip import (ChunkDPLRDeltaRuleFunction, ChunkHDLAFunction, _lib, chunk_hdla_delta_rule, chunk_hrdplr_delta_rule,
+                      fused_recurrent_dplr_delta_rule)
+from hdla_hip.synthetic import make_inputs
+
+DEV = "cuda"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["ab", "beta"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,K,V,cu,state", [(1, 64, 64, None, True), (40, 64, 64, None, False), (33, 128, 64, [0, 5, 5, 33], True)])
+def test_chunked_operators_against_the_python_functions(form, dtype, T, K, V, cu, state):
+    x = make_inputs(41, 1, T, 2, K, V, n_states=None if cu is None else len(cu) - 1)
+    beta = 2 * torch.rand(1, T, 2, 1, generator=torch.Generator().manual_seed(1))
+    names = (x.q, x.k, x.v, x.a, x.b, x.gk) if form == "ab" else (x.q, x.k, x.v, beta, x.gk)
+    # q as a strided view: the native path makes it contiguous itself
+    leaves = [t.to(dtype).to(DEV) for t in names]
+    leaves[0] = torch.stack([leaves[0], leaves[0]], dim=-1)[..., 0]
+    leaves = [t.detach().requires_grad_() for t in leaves]
+    h0 = x.h0.to(DEV).requires_grad_() if state else None
+    cu = None if cu is None else torch.tensor(cu, device=DEV)
+    fn, op, pos = ((ChunkDPLRDeltaRuleFunction, chunk_hrdplr_delta_rule, (2,)) if form == "ab"
+                   else (ChunkHDLAFunction, chunk_hdla_delta_rule, ()))
+    args = (0.5, h0, state) + ((2, False, 16, cu, False) if form == "ab" else (cu, False))
+    if form == "beta":
+        leaves_py = leaves[:3] + [leaves[3].reshape(1, T, 2)] + leaves[4:]
+    else:
+        leaves_py = leaves
+    ref = fn.apply(*leaves_py, *args)
+    got = op(*leaves, *pos, scale=0.5, initial_state=h0, output_final_state=state, cu_seqlens=cu, keep_forward=False)
+    gos = [x.do.to(dtype).to(DEV)] + ([x.dht.to(DEV)] if state else [])
+    wrt = leaves + ([h0] if state else [])
+    g_ref = torch.autograd.grad([t for t in ref if t is not None], wrt, gos)
+    g_got = torch.autograd.grad([t for t in got if t is not None], wrt, gos)
+    for a, b in zip(list(ref) + list(g_ref), list(got) + list(g_got)):
+        assert (a is None and b is None) or torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_outputs_that_no_loss_uses_and_calls_that_are_left_to_python():
+    x = make_inputs(42, 1, 20, 2, 64, 64)
+    leaves = [t.bfloat16().to(DEV).requires_grad_() for t in (x.q, x.k, x.v, x.a, x.b, x.gk)]
+    o, ht = chunk_hrdplr_delta_rule(*leaves, 2, output_final_state=True)
+    only_ht = torch.autograd.grad(ht, leaves, x.dht.to(DEV))                   # no gradient of o: taken as zeros
+    assert all(torch.isfinite(g.float()).all() for g in only_ht) and float(only_ht[1].float().abs().sum()) > 0
+    n = _lib.native()
+    t = [y.detach() for y in leaves]
+    assert n.recurrent(*leaves, 2, None, None, False, False, None, False) is None      # gradients wanted
+    assert n.recurrent(*t, 1, None, None, False, False, None, False) is None           # a and b of one rank
+    assert n.recurrent(*[y.half() for y in t], 2, None, None, False, False, None, False) is None
+    assert n.chunk(*t, 2, None, x.h0, False, False, 16, None, None) is None            # state on the CPU
+    assert n.chunk(*t, 2, None, None, False, False, 16, None, True) is None            # kept forward pass
+    assert torch.equal(fused_recurrent_dplr_delta_rule(*t, 2)[0], n.recurrent(*t, 2, None, None, False, False, None, False)[0])
