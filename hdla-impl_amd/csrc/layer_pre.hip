@@ -23,6 +23,7 @@ struct PreArgs {
     int H, D, ldy, cq, ck, cv, cb;            // column offsets in y; cb < 0: no beta
     int lpr_log2, norm_q, norm_k, norm_v;
     float beta_scale, eps_d;                  // eps_d = D * eps: o = u / sqrt(sum u^2 + D eps)
+    int zero_from;                            // > 0: backward, columns zero_from .. ldy of dy are padding and become zero
 };
 
 typedef unsigned pre_u32x4 __attribute__((ext_vector_type(4)));
@@ -170,6 +171,9 @@ __global__ __launch_bounds__(256) void layer_pre_bwd_kernel(PreArgs p) {
                 const float g = ld_elem(static_cast<const T*>(p.dbeta) + slot);
                 st_elem(static_cast<T*>(p.dy) + row * p.ldy + p.cb + h, g * p.beta_scale * b * (1.f - b));
             }
+            // the padding of the row, shared out over the lanes of its heads
+            if (p.zero_from > 0)
+                for (int c = p.zero_from + h * lpr + sl; c < p.ldy; c += p.H * lpr) st_elem(static_cast<T*>(p.dy) + row * p.ldy + c, 0.f);
         }
     }
 }
@@ -223,6 +227,8 @@ static int pre_config(const hdla_pre_dims* d, PreArgs& a, unsigned& nwg) {
     a.nsg = (a.nslot + rpw - 1) / rpw;
     a.norm_q = d->norm_q != 0; a.norm_k = d->norm_k != 0; a.norm_v = d->norm_v != 0;
     a.beta_scale = d->beta_scale; a.eps_d = d->eps * (float)d->D;
+    if (d->zero_from < 0 || d->zero_from > d->ldy) return HDLA_ERR_SHAPE;
+    a.zero_from = d->zero_from;
     const long long per_wave = a.nsg >= 16384 ? 4 : 1;          // passes per wavefront; few when the problem is small
     long long w = (a.nsg + 4 * per_wave - 1) / (4 * per_wave);
     nwg = (unsigned)(w < 1 ? 1 : (w > 8192 ? 8192 : w));

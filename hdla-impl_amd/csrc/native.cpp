@@ -13,6 +13,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/GradMode.h>
 #include <c10/hip/HIPStream.h>
@@ -38,7 +39,8 @@ struct Api {
 #define HDLA_FN(name) decltype(&hdla_##name) name
     HDLA_FN(strerror); HDLA_FN(workspace_bytes); HDLA_FN(boundary_bytes); HDLA_FN(chunk_fwd_b); HDLA_FN(chunk_bwd_b);
     HDLA_FN(recurrent_fwd); HDLA_FN(param_recurrent_fwd); HDLA_FN(normalize_fwd); HDLA_FN(normalize_bwd);
-    HDLA_FN(normalize_workspace_bytes);
+    HDLA_FN(normalize_workspace_bytes); HDLA_FN(layer_pre_fwd); HDLA_FN(layer_pre_bwd); HDLA_FN(logsigmoid_fwd); HDLA_FN(logsigmoid_bwd);
+    HDLA_FN(skinny_wgrad); HDLA_FN(skinny_wgrad_workspace_bytes); HDLA_FN(sum_partials);
 #undef HDLA_FN
 } api;
 PyObject* error_class = nullptr;                 // _lib.HdlaError
@@ -464,6 +466,276 @@ PyObject* py_normalize(PyObject*, PyObject* const* a, Py_ssize_t n) {
     });
 }
 
+// ---- the layer -------------------------------------------------------------------------------------------------------
+// HDLA_Custom.forward in its common form (bf16, silu activations, one block, beta, output gate, no biases; layer.py checks
+// that) as one call and one autograd node.  What one node buys over one per step: the GEMMs read the inner activations of
+// the low-rank projections where they lie in y and write their gradients where they belong in dy (no copies), the rows of
+// the concatenated weight can be padded to what the GEMMs like, and the host is out of the way (a decode step is ten
+// kernels of 4-10 us each, behind 200 us of Python).
+struct LayerCfg {
+    int64_t H, groups;
+    bool norm_q, norm_v;
+    double beta_scale, c, eps;
+    int gate_pos;
+};
+constexpr int RECURRENT_BELOW = 9;               // see layer.py
+constexpr double PRE_EPS = 1e-5;                 // l2_norm's
+
+// Columns of y: q, k, v (d each), the inner activations of decay and gate (D each), beta (H), padding.
+struct LayerCols {
+    int64_t d, D, H, f0, g0, beta, used, ld;
+    LayerCols(int64_t d_, int64_t H_, bool padded) : d(d_), D(d_ / H_), H(H_) {
+        f0 = 3 * d; g0 = f0 + D; beta = g0 + D; used = beta + H;
+        // The GEMM on x runs at its best on output widths that are whole tiles of 256 (8192 x 3216 x 1024: 82 us, with
+        // 3328 columns 50; its input gradient 60 -> 55, its weight gradient 86 -> 80).  Short calls read the weight once and are
+        // bound by that: there only up to the 16 bytes that rows are aligned to.
+        ld = padded ? (used + 255) / 256 * 256 : (used + 7) / 8 * 8;
+    }
+};
+constexpr int64_t PAD_FROM_ROWS = 1024;
+
+// the concatenated projection weight [ld, d]; rows behind the last projection are zero
+Tensor gather_weights(const Tensor* w, const LayerCols& L) {       // wq, wk, wv, wf0, wg0, wbeta
+    Tensor out = at::empty({L.ld, L.d}, w[0].options());
+    std::vector<Tensor> parts{w[0], w[1], w[2], w[3], w[4], w[5]};
+    if (L.ld > L.used) parts.push_back(at::zeros({L.ld - L.used, L.d}, w[0].options()));
+    at::cat_out(out, parts, 0);
+    return out;
+}
+hdla_pre_dims pre_dims(const LayerCols& L, const LayerCfg& f, int64_t rows) {
+    hdla_pre_dims p{};
+    p.rows = rows; p.H = (int32_t)L.H; p.D = (int32_t)L.D; p.dtype = HDLA_BF16; p.ldy = (int32_t)L.ld;
+    p.col_q = 0; p.col_k = (int32_t)L.d; p.col_v = (int32_t)(2 * L.d); p.col_beta = (int32_t)L.beta;
+    p.norm_q = f.norm_q; p.norm_k = 1; p.norm_v = f.norm_v;
+    p.beta_scale = (float)f.beta_scale; p.eps = (float)PRE_EPS;
+    p.zero_from = (int32_t)L.used;
+    return p;
+}
+// everything between x and the output; what the backward pass needs of it
+struct LayerFwd { Tensor x, w, y, f, g, o, n, out, ht, boundary; ChunkIn op; };
+
+// params: wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo; `w` gathered or undefined
+void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, const Tensor& h0, bool want_ht, bool chunked, bool want_boundary,
+                   LayerFwd& r) {
+    const int64_t B = x3.size(0), T = x3.size(1), d = x3.size(2), rows = B * T;
+    const LayerCols L(d, f.H, r.w.size(0) != LayerCols(d, f.H, false).ld);
+    const auto opt = x3.options();
+    r.x = x3.contiguous().view({rows, d});
+    r.y = at::mm(r.x, r.w.t());
+    const hdla_pre_dims pd = pre_dims(L, f, rows);
+    ChunkIn& in = r.op;
+    in.q = at::empty({B, T, L.H, L.D}, opt); in.k = at::empty({B, T, L.H, L.D}, opt); in.v = at::empty({B, T, L.H, L.D}, opt);
+    in.beta = at::empty({B, T, L.H, 1}, opt);
+    void* const s = stream_of(x3);
+    check(api.layer_pre_fwd(&pd, ptr(r.y), ptr(in.q), ptr(in.k), ptr(in.v), ptr(in.beta), s), "hdla_layer_pre_fwd");
+    r.f = at::mm(r.y.narrow(1, L.f0, L.D), P[6].t());
+    in.gk = at::empty({B, T, L.H, L.D}, opt);
+    check(api.logsigmoid_fwd(HDLA_BF16, r.f.numel(), ptr(r.f), ptr(in.gk), s), "hdla_logsigmoid_fwd");
+    if (h0.defined()) in.h0 = h0.to(at::kFloat).contiguous();
+    hdla_dims cd;
+    chunk_dims(in, 1.0, cd);
+    if (chunked) {
+        chunk_forward(in, cd, want_ht, want_boundary, r.o, r.ht, r.boundary);
+    } else {
+        r.o = at::empty_like(in.v);
+        if (want_ht) r.ht = at::empty({cd.N, cd.H, cd.K, cd.V}, opt.dtype(at::kFloat));
+        check(api.param_recurrent_fwd(&cd, ptr(in.q), ptr(in.k), ptr(in.v), ptr(in.beta), ptr(in.gk), 0, fptr(in.h0), ptr(r.o), fptr(r.ht), s),
+              "hdla_param_recurrent_fwd");
+    }
+    r.g = at::mm(r.y.narrow(1, L.g0, L.D), P[7].t());
+    const Tensor o2 = r.o.view({rows, d});
+    r.n = norm_forward(o2, P[8], r.g, norm_dims(o2, P[8], f.gate_pos, f.c, f.eps, f.groups));
+    r.out = at::mm(r.n, P[9].t()).view({B, T, d});
+}
+
+// dW [n, k] = dY [rows, n]^T X [rows, k].  An output of few tiles would leave most of the chip idle (1024 x 1024 over 8192
+// rows: 54 us): the rows are split over a batch of products whose fp32 results one kernel adds (28 + 4 us).
+Tensor weight_grad(const Tensor& dy, const Tensor& x) {
+    const int64_t rows = dy.size(0), n = dy.size(1), k = x.size(1);
+    const int64_t tiles = ((n + 127) / 128) * ((k + 127) / 128);
+    int64_t S = 1;
+    while (S < 8 && tiles * S * 2 <= 256 && rows % (S * 2) == 0 && rows / (S * 2) >= 1024) S *= 2;
+    if (S == 1 || dy.stride(0) != n || x.stride(0) != k || n * k % 8) return at::mm(dy.t(), x);
+    const Tensor part = at::bmm(dy.view({S, rows / S, n}).transpose(1, 2), x.view({S, rows / S, k}), at::kFloat);
+    const Tensor dw = at::empty({n, k}, dy.options());
+    check(api.sum_partials(fptr(part), (int32_t)S, n * k, ptr(dw), stream_of(dy)), "hdla_sum_partials");
+    return dw;
+}
+// the same for the low-rank projections (hdla_skinny_wgrad)
+Tensor skinny_grad(const Tensor& dy, const Tensor& x0) {
+    const int64_t rows = dy.size(0), K = dy.size(1), N = x0.size(1);
+    const size_t nws = api.skinny_wgrad_workspace_bytes(HDLA_BF16, rows, (int32_t)N, (int32_t)K);
+    const Tensor ws = bytes_like(dy, nws), dw = at::empty({K, N}, dy.options());
+    check(api.skinny_wgrad(HDLA_BF16, rows, (int32_t)N, (int32_t)K, ptr(dy), dy.stride(0), ptr(x0), x0.stride(0), ptr(dw), ptr(ws), nws,
+                           stream_of(dy)), "hdla_skinny_wgrad");
+    return dw;
+}
+
+struct LayerFn : torch::autograd::Function<LayerFn> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& wq, const Tensor& wk, const Tensor& wv, const Tensor& wf0,
+                                 const Tensor& wg0, const Tensor& wbeta, const Tensor& wf1, const Tensor& wg1, const Tensor& wnorm,
+                                 const Tensor& wo, const Maybe& h0, const LayerCfg& f, bool want_ht) {
+        const Tensor P[10] = {wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo};
+        LayerFwd r;
+        r.w = gather_weights(P, LayerCols(x.size(2), f.H, x.size(0) * x.size(1) >= PAD_FROM_ROWS));
+        layer_forward(x, P, f, value(h0), want_ht, true, keep_boundaries_default(), r);
+        ctx->save_for_backward({r.x, r.w, r.y, r.f, r.g, r.o, r.n, r.boundary, r.op.q, r.op.k, r.op.v, r.op.beta, r.op.gk, value(h0), wf1, wg1,
+                                wnorm, wo});
+        ctx->saved_data["c"] = std::vector<double>{f.beta_scale, f.c, f.eps};
+        ctx->saved_data["i"] = std::vector<int64_t>{f.H, f.groups, f.norm_q, f.norm_v, f.gate_pos, x.size(0), x.size(1)};
+        ctx->set_materialize_grads(false);
+        return want_ht ? variable_list{r.out, r.ht} : variable_list{r.out};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        return in_backward([&] { return gradients(ctx, grads); });
+    }
+    static variable_list gradients(AutogradContext* ctx, const variable_list& grads) {
+        const auto s = ctx->get_saved_variables();
+        const Tensor &x = s[0], &w = s[1], &y = s[2], &f = s[3], &g = s[4], &o = s[5], &n = s[6], &boundary = s[7];
+        const Tensor &q = s[8], &k = s[9], &v = s[10], &beta = s[11], &gk = s[12], &h0 = s[13], &wf1 = s[14], &wg1 = s[15], &wnorm = s[16],
+                     &wo = s[17];
+        const at::DeviceGuard guard(x.device());
+        const auto cc = ctx->saved_data["c"].toDoubleVector();
+        const auto ci = ctx->saved_data["i"].toIntVector();
+        const LayerCfg cfg{ci[0], ci[1], ci[2] != 0, ci[3] != 0, cc[0], cc[1], cc[2], (int)ci[4]};
+        const int64_t B = ci[5], T = ci[6], rows = x.size(0), d = x.size(1);
+        const LayerCols L(d, cfg.H, w.size(0) != LayerCols(d, cfg.H, false).ld);
+        void* const stream = stream_of(x);
+        const auto opt = x.options();
+        const auto need = [&](size_t i) { return ctx->needs_input_grad(i); };
+        variable_list out(14);
+
+        // output projection and gated norm
+        const Tensor dout = grads[0].defined() ? grads[0].to(at::kBFloat16).contiguous().view({rows, d}) : at::zeros({rows, d}, opt);
+        if (need(10)) out[10] = weight_grad(dout, n);
+        const Tensor dn = at::mm(dout, wo);
+        const Tensor o2 = o.view({rows, d}), d_o = at::empty({rows, d}, opt), dgate = at::empty({rows, d}, opt);
+        Tensor dwn = at::empty({d}, opt.dtype(at::kFloat));
+        {
+            const hdla_norm_dims nd = norm_dims(o2, wnorm, cfg.gate_pos, cfg.c, cfg.eps, cfg.groups);
+            const size_t nws = api.normalize_workspace_bytes(&nd);
+            const Tensor ws = bytes_like(x, nws < 16 ? 16 : nws);
+            check(api.normalize_bwd(&nd, ptr(o2), ptr(wnorm), ptr(g), ptr(dn), ptr(d_o), ptr(dgate), fptr(dwn), ptr(ws), nws, stream),
+                  "hdla_normalize_bwd");
+        }
+        if (need(9)) out[9] = dwn.to(wnorm.scalar_type()).view(wnorm.sizes());
+
+        // the operator
+        Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), dbeta = at::empty_like(beta), dgk = at::empty_like(gk), dh0;
+        {
+            ChunkIn in{q, k, v, Tensor(), Tensor(), beta, gk, h0, Tensor()};
+            if (h0.defined()) { in.h0 = h0.to(at::kFloat).contiguous(); dh0 = at::empty_like(in.h0); }
+            Tensor dht;
+            if (grads.size() > 1 && grads[1].defined()) dht = grads[1].to(at::kFloat).contiguous();
+            hdla_dims cd;
+            chunk_dims(in, 1.0, cd);
+            const Tensor ws = workspace(cd, HDLA_PASS_BWD, x);
+            check(api.chunk_bwd_b(&cd, ptr(q), ptr(k), ptr(v), nullptr, nullptr, ptr(beta), ptr(gk), fptr(in.h0), ptr(d_o), fptr(dht), ptr(dq),
+                                  ptr(dk), ptr(dv), nullptr, nullptr, ptr(dbeta), ptr(dgk), fptr(dh0), ptr(boundary),
+                                  boundary.defined() ? (size_t)boundary.numel() : 0, ptr(ws), (size_t)ws.numel(), stream), "hdla_chunk_bwd_b");
+            if (dh0.defined()) out[11] = dh0.to(h0.scalar_type());
+        }
+
+        // gradient of y, each part written where it belongs
+        const Tensor dy = at::empty_like(y);
+        const hdla_pre_dims pd = pre_dims(L, cfg, rows);
+        check(api.layer_pre_bwd(&pd, ptr(y), ptr(dq), ptr(dk), ptr(dv), ptr(dbeta), ptr(dy), stream), "hdla_layer_pre_bwd");
+        const Tensor df = at::empty_like(f);
+        check(api.logsigmoid_bwd(HDLA_BF16, f.numel(), ptr(f), ptr(dgk), ptr(df), stream), "hdla_logsigmoid_bwd");
+        Tensor df0 = dy.narrow(1, L.f0, L.D), dg0 = dy.narrow(1, L.g0, L.D);
+        at::mm_out(df0, df, wf1);
+        at::mm_out(dg0, dgate, wg1);
+        if (need(7)) out[7] = skinny_grad(df, y.narrow(1, L.f0, L.D));
+        if (need(8)) out[8] = skinny_grad(dgate, y.narrow(1, L.g0, L.D));
+
+        // the projections of x
+        if (need(1) || need(2) || need(3) || need(4) || need(5) || need(6)) {
+            const Tensor dw = weight_grad(dy, x);
+            const int64_t at_row[7] = {0, d, 2 * d, L.f0, L.g0, L.beta, L.used};
+            for (int i = 0; i < 6; ++i) out[1 + i] = dw.narrow(0, at_row[i], at_row[i + 1] - at_row[i]);
+        }
+        if (need(0)) out[0] = at::mm(dy, w).view({B, T, d});
+        return out;
+    }
+};
+
+// layer(x, (wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo), initial_state, want_state, mode, cache,
+//       H, groups, norm_q, norm_v, beta_scale, c, eps, gate_pos) -> (output, state) or None
+// mode: 0 chunked with gradients and from RECURRENT_BELOW tokens on, else token-serial; 1 chunked; 2 token-serial
+// cache: a two-element list that keeps the concatenated weight between calls without gradients, or None
+PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 14 || !api.strerror || !is_tensor(a[0]) || !PyTuple_CheckExact(a[1]) || PyTuple_GET_SIZE(a[1]) != 10) return none();
+    const Tensor& x = unpack(a[0]);
+    const at::Device dev = x.device();
+    if (!dev.is_cuda() || x.scalar_type() != at::kBFloat16 || !gpu_like(x, dev) || x.dim() != 3 || x.numel() == 0) return none();
+    if (at::autocast::is_autocast_enabled(at::kCUDA)) return none();
+    LayerCfg f{};
+    f.H = PyLong_AsLongLong(a[6]); f.groups = PyLong_AsLongLong(a[7]);
+    f.norm_q = a[8] == Py_True; f.norm_v = a[9] == Py_True;
+    const int mode = (int)PyLong_AsLong(a[4]);
+    f.gate_pos = (int)PyLong_AsLong(a[13]);
+    bool want = false;
+    if (!number(a[10], f.beta_scale) || !number(a[11], f.c) || !number(a[12], f.eps) || !truth(a[3], want) || PyErr_Occurred()) { PyErr_Clear(); return none(); }
+    const int64_t B = x.size(0), T = x.size(1), d = x.size(2);
+    if (f.H < 1 || d % f.H || d % 64 || f.groups < 1 || d % f.groups || B * T > INT32_MAX / 4) return none();
+    const int64_t D = d / f.H;
+    if (D != 64 && D != 128) return none();
+    const int64_t shapes[10][2] = {{d, d}, {d, d}, {d, d}, {D, d}, {D, d}, {f.H, d}, {d, D}, {d, D}, {d, 0}, {d, d}};
+    Tensor P[10];
+    bool op_grad = wants_grad(x), any = op_grad;
+    for (int i = 0; i < 10; ++i) {
+        PyObject* o = PyTuple_GET_ITEM(a[1], i);
+        if (!is_tensor(o)) return none();
+        P[i] = unpack(o);
+        if (P[i].device() != dev || !P[i].is_contiguous()) return none();
+        if (i == 8 ? (P[i].dim() != 1 || P[i].size(0) != d || !native_dtype(P[i].scalar_type()))
+                   : (P[i].scalar_type() != at::kBFloat16 || !same_sizes(P[i], {shapes[i][0], shapes[i][1]}))) return none();
+        any = any || wants_grad(P[i]);
+        op_grad = op_grad || ((i < 4 || i == 5 || i == 6) && wants_grad(P[i]));
+    }
+    Tensor h0;
+    if (a[2] != Py_None) {
+        if (!is_tensor(a[2])) return none();
+        h0 = unpack(a[2]);
+        if (!gpu_like(h0, dev) || !same_sizes(h0, {B, f.H, D, D}) || !h0.is_floating_point()) return none();
+        any = any || wants_grad(h0);
+    }
+    const bool grad = c10::GradMode::is_enabled() && any;
+    const bool chunked = mode == 1 || (mode == 0 && ((c10::GradMode::is_enabled() && op_grad) || T >= RECURRENT_BELOW));
+    if (grad && !chunked) return none();                         // gradients behind the token-serial operator: as the Python code has it
+    if (keep_forward_default() && grad) return none();
+    hdla_dims probe{};
+    if (!route_and_segments(probe)) return none();
+    return guarded([&]() -> PyObject* {
+        const at::DeviceGuard guard(dev);
+        if (grad) {
+            const auto r = LayerFn::apply(x, P[0], P[1], P[2], P[3], P[4], P[5], P[6], P[7], P[8], P[9], maybe(h0), f, want);
+            return pair(r[0], want ? r[1] : Tensor());
+        }
+        LayerFwd r;
+        const LayerCols L(d, f.H, B * T >= PAD_FROM_ROWS);
+        if (PyList_CheckExact(a[5]) && PyList_GET_SIZE(a[5]) == 2) {
+            // the weight of the last call, as long as the parameters are the ones it was built from, unmodified
+            struct { const void* p; uint64_t v; } key[7];
+            for (int i = 0; i < 6; ++i) key[i] = {P[i].data_ptr(), (uint64_t)P[i]._version()};
+            key[6] = {nullptr, (uint64_t)L.ld};
+            PyObject *old_key = PyList_GET_ITEM(a[5], 0), *old = PyList_GET_ITEM(a[5], 1);
+            if (PyBytes_CheckExact(old_key) && PyBytes_GET_SIZE(old_key) == (Py_ssize_t)sizeof key &&
+                !memcmp(PyBytes_AS_STRING(old_key), key, sizeof key) && is_tensor(old)) {
+                r.w = unpack(old);
+            } else {
+                r.w = gather_weights(P, L);
+                PyList_SetItem(a[5], 0, PyBytes_FromStringAndSize(reinterpret_cast<const char*>(key), sizeof key));
+                PyList_SetItem(a[5], 1, THPVariable_Wrap(r.w));
+            }
+        } else {
+            r.w = gather_weights(P, L);
+        }
+        layer_forward(x, P, f, h0, want, chunked, false, r);
+        return pair(r.out, r.ht);
+    });
+}
+
 // ---- module ----------------------------------------------------------------------------------------------------------
 // bind(handle of libhdla_hip.so, HdlaError, torch.OutOfMemoryError)
 PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -478,7 +750,8 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     HDLA_FN(strerror) HDLA_FN(workspace_bytes) HDLA_FN(boundary_bytes) HDLA_FN(chunk_fwd_b) HDLA_FN(chunk_bwd_b)
     HDLA_FN(recurrent_fwd) HDLA_FN(param_recurrent_fwd) HDLA_FN(normalize_fwd) HDLA_FN(normalize_bwd)
-    HDLA_FN(normalize_workspace_bytes)
+    HDLA_FN(normalize_workspace_bytes) HDLA_FN(layer_pre_fwd) HDLA_FN(layer_pre_bwd) HDLA_FN(logsigmoid_fwd) HDLA_FN(logsigmoid_bwd)
+    HDLA_FN(skinny_wgrad) HDLA_FN(skinny_wgrad_workspace_bytes) HDLA_FN(sum_partials)
 #undef HDLA_FN
     Py_INCREF(a[1]);
     Py_XDECREF(error_class);
@@ -493,7 +766,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
 #define HDLA_DEF(name, fn) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(fn)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     HDLA_DEF("bind", py_bind), HDLA_DEF("chunk", py_chunk), HDLA_DEF("chunk_hdla", py_chunk_hdla), HDLA_DEF("recurrent", py_recurrent),
-    HDLA_DEF("recurrent_hdla", py_recurrent_hdla), HDLA_DEF("normalize", py_normalize), {nullptr, nullptr, 0, nullptr}};
+    HDLA_DEF("recurrent_hdla", py_recurrent_hdla), HDLA_DEF("normalize", py_normalize), HDLA_DEF("layer", py_layer), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -159,3 +159,15 @@ extern "C" int hdla_skinny_wgrad(int dtype, int64_t M, int32_t N, int32_t K, con
     e = hipGetLastError();
     return e == hipSuccess ? HDLA_OK : (int)e;
 }
+
+extern "C" int hdla_sum_partials(const float* part, int32_t count, int64_t n, void* out, void* stream) {
+    if (count < 1 || n < 0 || n % 8) return HDLA_ERR_SHAPE;
+    if (n == 0) return HDLA_OK;
+    if (!part || !out) return HDLA_ERR_NULL;
+    if (((reinterpret_cast<uintptr_t>(part) | reinterpret_cast<uintptr_t>(out)) & 15) != 0) return HDLA_ERR_ALIGN;
+    if ((n / 8 + 255) / 256 > 0x7fffffffLL) return HDLA_ERR_SHAPE;
+    hipLaunchKernelGGL(skinny_wgrad_sum_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream), part,
+                       static_cast<bf16*>(out), (long long)n, (int)count);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? HDLA_OK : (int)e;
+}

@@ -9,7 +9,7 @@ from typing import Optional
 import torch
 
 HDLA_BF16, HDLA_FP32 = 0, 1
-HDLA_VERSION = 200          # the header this binding was written against (struct layouts, entry points)
+HDLA_VERSION = 201          # the header this binding was written against (struct layouts, entry points)
 ROUTE_AUTO, ROUTE_CLASSIC, ROUTE_FUSED = 0, 1, 2
 _ROUTES = {"": ROUTE_AUTO, "auto": ROUTE_AUTO, "classic": ROUTE_CLASSIC, "fused": ROUTE_FUSED}
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -44,7 +44,7 @@ class HdlaPreDims(ctypes.Structure):
     """struct hdla_pre_dims of include/hdla_hip.h."""
     _fields_ = [("rows", ctypes.c_int64)] + [(n, ctypes.c_int32) for n in (
         "H", "D", "dtype", "ldy", "col_q", "col_k", "col_v", "col_beta", "norm_q", "norm_k", "norm_v")] + [
-        ("beta_scale", ctypes.c_float), ("eps", ctypes.c_float)]
+        ("beta_scale", ctypes.c_float), ("eps", ctypes.c_float), ("zero_from", ctypes.c_int32)]
 
 
 class HdlaError(RuntimeError):

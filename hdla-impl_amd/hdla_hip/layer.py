@@ -32,10 +32,11 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import _lib
 from .chunk import chunk_hrdplr_delta_rule
 from . import layer_pre as _pre
 from .hdla import chunk_hdla_delta_rule, fused_recurrent_hdla_delta_rule, parameterize_a_b
-from .normalize import get_norm_fn, l2_norm
+from .normalize import GroupRMSNormFusedGate, RMSNormFusedGate, get_norm_fn, l2_norm
 from .recurrent import fused_recurrent_dplr_delta_rule
 
 EMBED_DIM_BASE = 256                 # HRDPLR/normalizations/normalization_utils.py:14
@@ -143,6 +144,10 @@ class HDLA_Custom(nn.Module):
         self.num_blocks = num_blocks
         self.fuse_ab, self.dispatch, self.fuse_pre = fuse_ab, dispatch, fuse_pre
         self._all_silu = all(a in ("silu", "swish") for a in (q_activation, k_activation, v_activation))
+        # the form the native host path runs as one call, as far as the constructor decides it
+        self._common = (self._all_silu and use_beta and use_output_gate and not bias and num_blocks == 1 and not use_offset
+                        and gate_act == "sigmoid" and gate_pos in ("pre", "post"))
+        self._native_cache = [None, None]
         self._init_weights()
 
     # ---- initialisation: hdla_custom.py:159-187 and normalization_utils.py:115-211 (the branches a module of this
@@ -205,6 +210,7 @@ class HDLA_Custom(nn.Module):
     def reset_cache(self):
         """Forget the concatenated projection weight of evaluation mode."""
         self._gathered_key = self._gathered_val = None
+        self._native_cache = [None, None]
 
     def train(self, mode: bool = True):
         self.reset_cache()
@@ -295,6 +301,37 @@ class HDLA_Custom(nn.Module):
             log_f = log_f.masked_fill(~keep, 0)
         return q, k, v, beta, log_f, gate0
 
+    def _native_params(self):
+        """Parameters for the native call, or None where a submodule has been replaced or carries hooks."""
+        mods = self._modules
+        f, g, norm = mods["f_proj"], mods["output_gate"], mods["norm"]
+        if type(f) is not nn.Sequential or type(g) is not nn.Sequential or type(norm) not in (RMSNormFusedGate, GroupRMSNormFusedGate):
+            return None
+        out = []
+        for m in (mods["q_proj"], mods["k_proj"], mods["v_proj"], f._modules["0"], g._modules["0"], mods["bet_proj"], f._modules["1"],
+                  g._modules["1"], norm, mods["o_proj"]):
+            if ((m is not norm and type(m) is not nn.Linear) or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                    or m._backward_pre_hooks):
+                return None
+            p = m._parameters
+            if p["weight"] is None or p.get("bias") is not None:
+                return None
+            out.append(p["weight"])
+        return tuple(out)
+
+    def _forward_native(self, x, state, use_cache):
+        """The whole layer as one native call in its common form (csrc/native.cpp); None where this call is not of it."""
+        params = self._native_params()
+        if params is None:
+            return None
+        norm, grouped = self.norm, type(self.norm) is GroupRMSNormFusedGate
+        groups = norm.num_groups if grouped else 1
+        mode = 0 if self.dispatch == "auto" else (1 if self.training or use_cache else 2)
+        return _lib.native().layer(
+            x, params, state, bool(use_cache), mode, None if self.training else self._native_cache, self.num_heads, groups,
+            bool(self.norm_q), bool(self.norm_v), 2.0 if self.beta_activation == "neg" else 1.0,
+            (self.embed_dim // groups) ** 0.5, norm.eps, 1 if norm.gate_pos == "pre" else 2)
+
     def forward(self, x, attention_mask: Optional[torch.Tensor] = None, past_key_values=None,
                 use_cache: Optional[bool] = False, lower_bound: Optional[torch.Tensor] = None, **kwargs):
         b, n, d = x.shape
@@ -302,6 +339,12 @@ class HDLA_Custom(nn.Module):
         if past_key_values is not None and len(past_key_values) > self.layer_idx:
             recurrent_state = past_key_values[self.layer_idx]["recurrent_state"][0]
             q_offset = past_key_values.get_seq_length(self.layer_idx)
+        if self._common and self.fuse_ab and self.fuse_pre and attention_mask is None and lower_bound is None:
+            out = self._forward_native(x, recurrent_state, use_cache)
+            if out is not None:
+                if past_key_values is not None:
+                    past_key_values.update(recurrent_state=[out[1]], layer_idx=self.layer_idx, offset=n)
+                return out[0], past_key_values
         q, k, v, beta, log_f, gate0 = self.project(x, attention_mask, q_offset, lower_bound)
         dtype = q.dtype
         k, v, beta, log_f = k.to(dtype), v.to(dtype), beta.to(dtype), log_f.to(dtype)

@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-#define HDLA_VERSION 200
+#define HDLA_VERSION 201
 
 enum { HDLA_BF16 = 0, HDLA_FP32 = 1 };
 
@@ -274,10 +274,11 @@ typedef struct hdla_pre_dims {
     int32_t ldy, col_q, col_k, col_v, col_beta;
     int32_t norm_q, norm_k, norm_v;
     float beta_scale, eps;
+    int32_t zero_from;         /* > 0: the backward pass writes zeros to columns zero_from .. ldy of dy as well */
 } hdla_pre_dims;
 int hdla_layer_pre_fwd(const hdla_pre_dims* dims, const void* y, void* q, void* k, void* v, void* beta, void* stream);
 /* Backward pass: from y and the gradients of the four outputs, the gradient of y's four column ranges, written in
- * place into dy [rows, ldy]; the other columns of dy are not touched. */
+ * place into dy [rows, ldy]; the other columns of dy are not touched (but see zero_from). */
 int hdla_layer_pre_bwd(const hdla_pre_dims* dims, const void* y, const void* dq, const void* dk, const void* dv,
                        const void* dbeta, void* dy, void* stream);
 /* log_f = logsigmoid(f) (HRDPLR/hdla_custom.py:219) and its gradient df = dlog_f * sigmoid(-f), elementwise over n
@@ -294,6 +295,9 @@ int hdla_logsigmoid_bwd(int dtype, int64_t n, const void* x, const void* dy, voi
 int hdla_skinny_wgrad(int dtype, int64_t M, int32_t N, int32_t K, const void* dY, int64_t ldy, const void* X0,
                       int64_t ldx, void* dW, void* workspace, size_t workspace_bytes, void* stream);
 size_t hdla_skinny_wgrad_workspace_bytes(int dtype, int64_t M, int32_t N, int32_t K);
+/* out [n] (bf16) = sum of `count` consecutive fp32 partial results part [count][n], added in order; n a multiple of 8,
+ * both 16-byte aligned: the second half of a product whose contraction was split. */
+int hdla_sum_partials(const float* part, int32_t count, int64_t n, void* out, void* stream);
 
 /* Measurement aid; it has no counterpart in the reference.  One launch of a kernel that reads `n_read` (0..3)
  * buffers and writes `n_write` (0..2) buffers of `bytes` bytes each (a multiple of 16; every pointer 16-byte

@@ -56,3 +56,45 @@ def test_outputs_that_no_loss_uses_and_calls_that_are_left_to_python():
     assert n.chunk(*t, 2, None, x.h0, False, False, 16, None, None) is None            # state on the CPU
     assert n.chunk(*t, 2, None, None, False, False, 16, None, True) is None            # kept forward pass
     assert torch.equal(fused_recurrent_dplr_delta_rule(*t, 2)[0], n.recurrent(*t, 2, None, None, False, False, None, False)[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,T,d,H,kw", [
+    (1, 1023, 256, 4, {}),                                          # rows of y padded to 16 bytes only (H = 4: not by themselves)
+    (2, 512, 256, 4, {"gate_pos": "post", "norm_q": True}),         # from 1024 rows on: padded to whole GEMM tiles
+    (4, 2048, 256, 2, {"token_mixer_norm_type": "grouprmsnorm"}),   # the output projection's weight gradient in four row ranges
+])
+def test_layer_as_one_call_against_its_steps(B, T, d, H, kw):
+    """The layer's one native call against the same module run step by step (_common switched off), training and decode.
+    The two differ where the steps round to bf16 in between (H = 4: the elementwise stage in torch's operators)."""
+    from hdla_hip.layer import HDLA_Custom, RecurrentCache
+    from oracle import hrdplr_oracle as O
+    torch.manual_seed(3)
+    m = HDLA_Custom(d, H, token_mixer_init_type=2, rescale_type=0, **kw).to(DEV).bfloat16().train()
+    g = torch.Generator().manual_seed(4)
+    x = torch.randn(B, T, d, generator=g).bfloat16().to(DEV).requires_grad_()
+    do = torch.randn(B, T, d, generator=g).bfloat16().to(DEV)
+    ps = list(m.parameters())
+    res = []
+    for common in (True, False):
+        m._common = common
+        y, _ = m(x)
+        res.append([y.detach()] + list(torch.autograd.grad(y, [x] + ps, do)))
+    assert res[0][0].grad_fn is None
+    errs = [O.rel_l2(a, b) for a, b in zip(*res)]
+    print([f"{e:.1e}" for e in errs], flush=True)
+    assert errs[0] <= 1e-2 and max(errs) <= 2e-2
+    m.eval()
+    outs = []
+    with torch.no_grad():
+        for common in (True, False):
+            m._common = common
+            cache = RecurrentCache()
+            _, cache = m(x[:, :20], past_key_values=cache, use_cache=True)
+            y = [m(x[:, 20 + i:21 + i], past_key_values=cache, use_cache=True)[0] for i in range(2)]
+            m.q_proj.weight.mul_(-1.0)                              # the kept concatenation has to notice
+            y.append(m(x[:, 22:23], past_key_values=cache, use_cache=True)[0])
+            m.q_proj.weight.mul_(-1.0)
+            outs.append(y + [cache[0]["recurrent_state"][0]])
+    for a, b in zip(*outs):
+        assert O.rel_l2(a, b) <= 1e-2
