@@ -38,7 +38,8 @@ int check_dims(const hdla_dims* d, int max_dim = 128) {
 // ---- the fused route (fused_impl.cuh) ----------------------------------------------------------------------------
 constexpr int FUSED_MAX_SEGMENTS = 64;       // the segments are chained serially by every workgroup that needs them: about a
                                              // microsecond a segment, against 2.5 for every chunk a segment is shorter
-constexpr int FUSED_MIN_SEGMENT_CHUNKS = 8;  // a segment pays for its transition matrix: not worth it for a few chunks
+constexpr int FUSED_MIN_SEGMENT_CHUNKS = 4;  // one chunk for each pair of producer waves: shorter segments wait for the same first chunk
+constexpr int FUSED_MIN_CHUNKS = 9;          // sequences of at most 8 chunks stay whole: a second kernel takes as long as they do
 constexpr int FUSED_TARGET_WORKGROUPS = 256; // one workgroup per compute unit
 
 // the shapes the fused kernels are built for
@@ -54,10 +55,39 @@ int fused_segments(const hdla_dims* d) {
     if (d->segments > 0) return d->segments < FUSED_MAX_SEGMENTS ? d->segments : FUSED_MAX_SEGMENTS;
     const long long lanes = (long long)d->N * d->H;
     const long long chunks_per_seq = ((d->T + CHUNK - 1) / CHUNK) / (d->cu_seqlens ? d->N : 1);
-    int nseg = 1;
+    if (chunks_per_seq < FUSED_MIN_CHUNKS) return 1;
+    // A segment takes about 2.2 us a chunk and every segment of the chain 0.9 us: the sum is least near 1.6 sqrt(chunks)
+    // segments, and twice as many pay as long as the chunks are at least a quarter of their square.  Measured (us,
+    // forward pass / training step, 8 chunks a segment at the least -> this rule): 2 lanes of 16 chunks 26/75 -> 20/70,
+    // 8 of 63 44/126 -> 32/96, 16 of 125 50/158 -> 49/141.
+    long long nseg = 1;
     while (nseg * 2 <= FUSED_MAX_SEGMENTS && lanes * nseg * 2 <= FUSED_TARGET_WORKGROUPS &&
-           chunks_per_seq / (nseg * 2) >= FUSED_MIN_SEGMENT_CHUNKS) nseg *= 2;
-    return nseg;
+           chunks_per_seq / (nseg * 2) >= FUSED_MIN_SEGMENT_CHUNKS && nseg * nseg <= chunks_per_seq) nseg *= 2;
+    return (int)nseg;
+}
+
+// ---- time segments of the stand-alone scans (scan_impl.cuh): where a whole sequence per workgroup would leave most of the
+// device idle.  A launch for the segments' records, one that chains them (together 10 us at the least), then the scans on
+// shorter sequences: twice the steps, of which nseg run at once.  Measured (us, forward / backward pass, one segment ->
+// as many as chosen here): fp32, K=V=64, 16 lanes of 63 chunks 156/224 -> 69/157 (8); fp32, K=V=128, 4 lanes of 125
+// chunks 812/896 -> 142/278 (16); bf16, K=V=128, 16 lanes of 313 chunks 293/546 -> 192/546 (8 and 1); bf16, K=128 V=64,
+// 8 lanes of 500 chunks 377/509 -> 154/352 (16 and 8).
+constexpr int SCAN_MAX_SEGMENTS = 32;
+int scan_segments(const hdla_dims* d, bool bwd) {
+    if (d->route != HDLA_ROUTE_AUTO) return 1;
+    if (d->segments > 0) return d->segments < SCAN_MAX_SEGMENTS ? d->segments : SCAN_MAX_SEGMENTS;
+    const bool f32 = d->in_dtype == HDLA_FP32;
+    const long long lanes = (long long)d->N * d->H;
+    const long long chunks = ((d->T + CHUNK - 1) / CHUNK) / (d->cu_seqlens ? d->N : 1);
+    // lanes x segments: beyond 128 the records' launch needs more than one round on the device.  The backward scans of
+    // 2-byte inputs are bound by their traffic from a dozen lanes on, and the reverse records come on top: fewer there.
+    if (bwd && !f32 && lanes > 8) return 1;
+    const long long most = bwd && !f32 ? 64 : 128;
+    // chunks a segment: a step takes 2-4 us with fp32 products, about 0.7 with bf16
+    const long long least = f32 ? 4 : 7;
+    int nseg = 1;
+    while (nseg * 2 <= SCAN_MAX_SEGMENTS && lanes * nseg * 2 <= most && chunks / (nseg * 2) >= least) nseg *= 2;
+    return nseg >= 4 ? nseg : 1;                          // two segments only make up for the second walk
 }
 
 struct FusedLayout {
@@ -156,6 +186,12 @@ int make_layout(const hdla_dims* d, int pass, WsLayout& L, int& nch) {
         L.CHUNK_OFF = take((size_t)(2 * d->N + 1) * 4);          // chunk_off [N+1], then order [N]
         L.CHUNK_SEQ = take((size_t)(nch > 0 ? nch : 1) * 4);
     }
+    const int nseg = pass == HDLA_PASS_FWD || pass == HDLA_PASS_BWD ? scan_segments(d, pass == HDLA_PASS_BWD) : 1;
+    if (nseg > 1) {
+        const size_t recs = (size_t)d->N * d->H * nseg, state = recs * K * V * 4, matrix = recs * K * K * 4;
+        L.SEG_LOC = take(state); L.SEG_TR = take(matrix); L.SEG_IN = take(state);
+        if (pass == HDLA_PASS_BWD) { L.SEG_RLOC = take(state); L.SEG_RTR = take(matrix); L.SEG_RIN = take(state); }
+    }
     L.total = off > 0 ? off : 256;
     return HDLA_OK;
 }
@@ -224,6 +260,12 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
     a.da = static_cast<T*>(da); a.db = static_cast<T*>(db); a.dgk = dgk;
     a.beta = static_cast<const T*>(beta); a.dbeta = static_cast<T*>(dbeta);
     bind_ws(a, d, LP, prep_ws, LS, pass == HDLA_PASS_BWD_KEPT ? workspace : prep_ws, nch);
+    a.seg = SegRec{1, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+    const int nseg = on_kept ? 1 : scan_segments(d, !fwd);
+    if (nseg > 1) {
+        const auto at = [&](size_t o) { return reinterpret_cast<float*>(static_cast<char*>(workspace) + o); };
+        a.seg = SegRec{nseg, at(LP.SEG_LOC), at(LP.SEG_TR), at(LP.SEG_IN), at(LP.SEG_RLOC), at(LP.SEG_RTR), at(LP.SEG_RIN)};
+    }
     hipError_t e;
     if (pass == HDLA_PASS_BWD_KEPT) stages &= ~HDLA_STAGE_PREP;    // the forward pass has run it
     if (d->cu_seqlens && (stages & HDLA_STAGE_PREP)) {
@@ -234,6 +276,10 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
     }
     if (nch > 0 && (stages & HDLA_STAGE_PREP)) {
         e = launch_prep<T>(a, d->K, d->V, pass == HDLA_PASS_FWD ? 0 : pass == HDLA_PASS_BWD ? 1 : 2, stream);
+        if (e != hipSuccess) return (int)e;
+    }
+    if (a.seg.nseg > 1 && (stages & HDLA_STAGE_CHAIN)) {
+        e = launch_scan_segments<T>(a, d->K, d->V, !fwd, stream);
         if (e != hipSuccess) return (int)e;
     }
     // the two scans of the backward pass are independent of each other: one launch when both are asked for

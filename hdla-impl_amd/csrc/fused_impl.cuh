@@ -47,9 +47,7 @@ constexpr int FUSED_ABORTED = 0x48444c00;
 __device__ __forceinline__ void seg_range(const SeqTab& st, int n, int nseg, int seg, int& s0, int& s1) {
     int c0, c1;
     seq_chunks(st, n, c0, c1);
-    const int len = (c1 - c0 + nseg - 1) / nseg;
-    s0 = min(c0 + seg * len, c1);
-    s1 = min(s0 + len, c1);
+    seg_range(c0, c1, nseg, seg, s0, s1);
 }
 
 // LDS of a fused workgroup (byte offsets): per producer one slot = [operands | outbox | solver scratch], then the flags

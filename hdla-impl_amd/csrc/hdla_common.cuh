@@ -270,6 +270,13 @@ __device__ __forceinline__ void seq_bounds(const SeqTab& st, int n, int64_t& bos
     }
 }
 
+// chunk range [s0, s1) of time segment `seg` of the chunks [c0, c1) of a sequence
+__device__ __forceinline__ void seg_range(int c0, int c1, int nseg, int seg, int& s0, int& s1) {
+    const int len = (c1 - c0 + nseg - 1) / nseg;
+    s0 = min(c0 + seg * len, c1);
+    s1 = min(s0 + len, c1);
+}
+
 // ---- per-chunk decay quantities in fragment layout ---------------------------------------------------------
 // lane (g,c) holds token c of the chunk and channels 16*kt + 4g + i.  The 16 lanes of a group are one DPP "row",
 // so prefix sums, suffix sums and sums over the tokens of a chunk are row_shr / row_shl / mirror additions on

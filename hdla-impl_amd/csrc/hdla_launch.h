@@ -15,6 +15,8 @@ template <typename T> hipError_t launch_scan_fwd(const ChunkArgs<T>& a, int K, i
 template <typename T> hipError_t launch_scan_bwd(const ChunkArgs<T>& a, int K, int V, hipStream_t stream);
 // both scans of the backward pass (scan_fwd without the output, scan_bwd) in one launch
 template <typename T> hipError_t launch_scan_pair(const ChunkArgs<T>& a, int K, int V, hipStream_t stream);
+// several time segments per sequence: what the scans above start their segments from
+template <typename T> hipError_t launch_scan_segments(const ChunkArgs<T>& a, int K, int V, bool both, hipStream_t stream);
 template <typename T> hipError_t launch_chunk_grad(const ChunkArgs<T>& a, int K, int V, hipStream_t stream);
 template <typename T> hipError_t launch_recurrent(const RecurrentArgs<T>& a, int K, int V, hipStream_t stream);
 

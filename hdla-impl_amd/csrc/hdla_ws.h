@@ -101,6 +101,8 @@ struct WsLayout {
     // chunk table (only with cu_seqlens)
     size_t CHUNK_OFF;  // int32 [N+1]
     size_t CHUNK_SEQ;  // int32 [nch]
+    // records of the time segments (see SegRec)
+    size_t SEG_LOC, SEG_TR, SEG_IN, SEG_RLOC, SEG_RTR, SEG_RIN;
     size_t total;
 };
 
@@ -111,6 +113,15 @@ struct Ws {
     T* TM;
     int32_t* STRONG;
     int sa_stride;            // bytes between the forward-scan blocks of consecutive (chunk, head) slots
+};
+
+// Time segments of the stand-alone scans (scan_impl.cuh): records per (sequence, head, segment), fp32 tiles in fragment
+// order.  The forward direction's, then the reverse direction's.
+struct SegRec {
+    int nseg;                 // segments per sequence; 1: no records
+    float *loc, *tr, *in;     // [V/16][K/16] state the segment leaves when it starts from zero (the first: from h0);
+                              // [K/16][K/16] its transition matrix; [V/16][K/16] the state that enters it
+    float *rloc, *rtr, *rin;  // the same for the state gradient, from the right (the last: from dht)
 };
 
 template <typename T>
@@ -136,6 +147,7 @@ struct ChunkArgs {            // inputs of the chunked operator + workspace
     float* dh0;               // nullable
     T *dq, *dk, *dv, *da, *db;
     void* dgk;
+    SegRec seg;
 };
 
 template <typename T>

@@ -24,6 +24,16 @@ template <typename T>
 hipError_t launch_scan_pair(const ChunkArgs<T>& a, int K, int V, hipStream_t stream) {
     return launch_scan<T>(a, K, V, SCAN_PAIR, stream);
 }
+template <typename T>
+hipError_t launch_scan_segments(const ChunkArgs<T>& a, int K, int V, bool both, hipStream_t stream) {
+    if (K == 64 && V == 64) return launch_scan_segments_shape<T, 64, 64>(a, both, stream);
+    if (K == 128 && V == 128) return launch_scan_segments_shape<T, 128, 128>(a, both, stream);
+    if (K == 64 && V == 128) return launch_scan_segments_shape<T, 64, 128>(a, both, stream);
+    if (K == 128 && V == 64) return launch_scan_segments_shape<T, 128, 64>(a, both, stream);
+    return hipErrorInvalidValue;
+}
+template hipError_t launch_scan_segments<bf16>(const ChunkArgs<bf16>&, int, int, bool, hipStream_t);
+template hipError_t launch_scan_segments<float>(const ChunkArgs<float>&, int, int, bool, hipStream_t);
 template hipError_t launch_scan_fwd<bf16>(const ChunkArgs<bf16>&, int, int, bool, hipStream_t);
 template hipError_t launch_scan_fwd<float>(const ChunkArgs<float>&, int, int, bool, hipStream_t);
 template hipError_t launch_scan_bwd<bf16>(const ChunkArgs<bf16>&, int, int, hipStream_t);

@@ -3,5 +3,7 @@
 
 namespace hdla {
 template hipError_t launch_scan_shape<bf16, 64, 64>(const ChunkArgs<bf16>&, ScanKind, hipStream_t);
+template hipError_t launch_scan_segments_shape<bf16, 64, 64>(const ChunkArgs<bf16>&, bool, hipStream_t);
 template hipError_t launch_scan_shape<bf16, 64, 128>(const ChunkArgs<bf16>&, ScanKind, hipStream_t);
+template hipError_t launch_scan_segments_shape<bf16, 64, 128>(const ChunkArgs<bf16>&, bool, hipStream_t);
 }  // namespace hdla

@@ -197,18 +197,63 @@ __device__ __forceinline__ void memory_wave(char* smem, int nsteps, int hw, BlkF
 //              [K/32][NWC] tile pairs (1 KiB a pair for 2-byte elements).  v_new is not checkpointed: the
 //              chunk_grad kernel rebuilds it from this checkpoint, w and u;
 //   OUT_GRAD   reverse scan: the same for dS, followed by [NWC] tile pairs of dv_new.
-enum ScanOut { OUT_O, OUT_STATE, OUT_GRAD };
+//   OUT_SUM    summary of a time segment: no outbox, the record is written at the end
+enum ScanOut { OUT_O, OUT_STATE, OUT_GRAD, OUT_SUM };
 template <typename T, int K, int V, int NWC, int SLOT_, ScanOut OUT> struct ScanLds {
     static constexpr int ES = sizeof(T), NM = ScanCfg<T, K, V, NWC>::NM, SLOT = SLOT_;
     static constexpr int OROW = 16 * NWC * ES + 16;
     static constexpr int OB_HC = (K / 32) * NWC * PAIR * ES;
-    static constexpr int OB = OUT == OUT_O ? CH * OROW : OUT == OUT_STATE ? OB_HC : OB_HC + NWC * PAIR * ES;
+    static constexpr int OB = OUT == OUT_SUM ? 0 : OUT == OUT_O ? CH * OROW : OUT == OUT_STATE ? OB_HC : OB_HC + NWC * PAIR * ES;
     static constexpr int BYTES = NSLOT * SLOT + (NM ? 2 * OB : 0);
 };
 
+// ---- time segments -------------------------------------------------------------------------------------------
+// Few (sequence, head) pairs leave most of the device idle while each of them walks its chunks one after the other, at
+// 0.5 to 4 us a chunk.  There a sequence is cut into nseg time segments: the state leaving a segment is affine in the
+// state entering it, S_out = M S_in + S_loc, and so is the state gradient on the way back.  A first launch walks all
+// segments at once from a zero state (OUT_SUM: no output but the record) and, on K more columns that start as the
+// identity and take no input of the chunks, for M; scan_chain_kernel chains the records into the states that enter the
+// segments; then the scans run as they do for whole sequences, every segment from its own state.  Twice the steps,
+// nseg times as many of them at once (scan_segments in api.hip says when).
+//
+// At the end of a segment: column block j of the state, or (trans) of the transition matrix X, whose tile (kt, j) is kept
+// with rows k, inner k', which is how the chain takes it.
+template <typename T, int K>
+__device__ __forceinline__ void store_record(const f32x4 (&S)[K / 16], float* loc, float* tr, int64_t rec, int V, int j, bool trans) {
+    constexpr int KT = K / 16;
+    if (trans) {
+        const Frag<float> ident = ident_frag<float>();
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) {
+            Frag<float> f;
+            f.v = S[kt];
+            f = transpose(f, ident);                      // exact: fp32 products with ones and zeros
+            *reinterpret_cast<f32x4*>(tr + rec * (K * K) + (kt * KT + j) * TILE + 4 * lane_id()) = f.v;
+        }
+    } else {
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) *reinterpret_cast<f32x4*>(loc + rec * (K * V) + (j * KT + kt) * TILE + 4 * lane_id()) = S[kt];
+    }
+}
+// the columns a segment starts from when it does not start from h0 / dht: the chained state, zeros, or the identity
+template <typename T, int K, bool SUM>
+__device__ __forceinline__ void load_entry(f32x4 (&S)[K / 16], const float* in, int64_t rec, int V, int j, bool trans) {
+    const int l = lane_id(), g = l >> 4, c = l & 15;
+#pragma unroll
+    for (int kt = 0; kt < K / 16; ++kt) {
+        if (!SUM) S[kt] = *reinterpret_cast<const f32x4*>(in + rec * (K * V) + (j * (K / 16) + kt) * TILE + 4 * l);
+        else if (trans) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) S[kt][i] = (16 * kt + 4 * g + i == 16 * j + c) ? 1.f : 0.f;
+        } else S[kt] = zero4();
+    }
+}
+
 // ---- forward -------------------------------------------------------------------------------------------------
-template <typename T, int K, int V, int NWC, bool WRITE_O>
-__device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem, int n, int split) {
+// split: which of the SPLIT groups of NWC column blocks; from SPLIT on (OUT_SUM only), of the transition matrix's
+template <typename T, int K, int V, int NWC, ScanOut OUT>
+__device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem, int n, int seg, int split) {
+    constexpr bool WRITE_O = OUT == OUT_O, SUM = OUT == OUT_SUM;
     typedef ScanCfg<T, K, V, NWC> C;
     constexpr int KT = K / 16, KT2 = KT / 2, VT = V / 16, NM = C::NM, ES = sizeof(T);
     constexpr BlkF B = blk_fwd(K, sizeof(T), WRITE_O);
@@ -216,19 +261,24 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
     constexpr bool PIPE_UPD = PIPE && C::early_update_reads(WRITE_O);
     constexpr int NIB = B.SIZE / 1024, SLOT = B.SIZE + C::OWN_FWD, NI = SLOT / 1024;
     constexpr bool OWN_LDS = C::OWN_FWD > 0;
-    typedef ScanLds<T, K, V, NWC, SLOT, WRITE_O ? OUT_O : OUT_STATE> L;
+    typedef ScanLds<T, K, V, NWC, SLOT, OUT> L;
     constexpr int OROW = L::OROW, OB_HC = L::OB_HC, OB = L::OB;
     char* const outbox = smem + NSLOT * SLOT;
 
     const int h = blockIdx.x;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int vt0 = split * NWC;                          // first column block of this workgroup
+    const bool trans = SUM && split >= C::SPLIT;
+    const int vt0 = (trans ? split - C::SPLIT : split) * NWC;     // first column block of this workgroup
+    const int own0 = trans ? 0 : vt0;                     // of its tiles of u^T, v^T (transition columns take none: never used)
     const int l = lane_id(), g = l >> 4, c = l & 15;
     const int H = p.H;
-    int c0, c1;
-    seq_chunks(p.st, n, c0, c1);
+    int cs, ce, c0, c1;
+    seq_chunks(p.st, n, cs, ce);
+    seg_range(cs, ce, p.seg.nseg, seg, c0, c1);
     int64_t bos, eos;
     seq_bounds(p.st, n, bos, eos);
+    bos += (int64_t)(c0 - cs) * CH;                       // the segment's first token
+    const int64_t rec = ((int64_t)n * p.H + h) * p.seg.nseg + seg;
     const int64_t chw0 = (int64_t)h * p.st.nch;
     const int nchunks = c1 - c0, last = c1 - 1;
     // block of step t; steps past the end of the sequence are clamped, so every load is unconditional (a load
@@ -238,8 +288,8 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
         // (the forward pass's blocks are B.SIZE apart; those the backward pass reads may be a forward pass's, further apart)
         const char* b = reinterpret_cast<const char*>(p.ws.W) + chw * (WRITE_O ? B.SIZE : p.ws.sa_stride);
         if constexpr (OWN_LDS)
-            return BlockFwd<NIB, C::OWN_UT, C::OWN_VTT>{b, reinterpret_cast<const char*>(p.ws.UT + (chw * VT + vt0) * PAIR),
-                                                        reinterpret_cast<const char*>(p.ws.VTT + (chw * VT + vt0) * TILE)};
+            return BlockFwd<NIB, C::OWN_UT, C::OWN_VTT>{b, reinterpret_cast<const char*>(p.ws.UT + (chw * VT + own0) * PAIR),
+                                                        reinterpret_cast<const char*>(p.ws.VTT + (chw * VT + own0) * TILE)};
         else
             return BlockOne{b};
     };
@@ -248,6 +298,7 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
         if (nchunks <= 0) return;
         const int hw = wv - NWC;
         memory_wave<T, NI, NM ? NM : 1, NM ? C::DR_SHARE : NSLOT, SLOT, 0>(smem, nchunks, hw, blk, [&](int t) __attribute__((always_inline)) {
+            if (SUM) return;
             const int cid = c0 + t;
             const char* ob = outbox + (t & 1) * OB;
             if (WRITE_O) {
@@ -285,7 +336,9 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
     const int64_t soff = ((int64_t)n * H + h) * K * V + 16 * vt + c;
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) S[kt] = zero4();
-    if (p.h0) {
+    if (seg > 0) {
+        load_entry<T, K, SUM>(S, p.seg.in, rec, V, vt, trans);
+    } else if (p.h0) {
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
@@ -295,8 +348,8 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
     auto load_own = [&](Own& o, int t) __attribute__((always_inline)) {
         if constexpr (!OWN_LDS) {
             const int64_t chw = chw0 + min(c0 + t, last);
-            ld_pair(p.ws.UT + (chw * VT + vt) * PAIR, o.ut[0], o.ut[1]);
-            o.vtt = ld_tile(p.ws.VTT + (chw * VT + vt) * TILE);
+            ld_pair(p.ws.UT + (chw * VT + own0 + wv % VT) * PAIR, o.ut[0], o.ut[1]);
+            o.vtt = ld_tile(p.ws.VTT + (chw * VT + own0 + wv % VT) * TILE);
         }
     };
 
@@ -322,6 +375,7 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
             ld_pair(reinterpret_cast<const T*>(slot + B.SIZE) + wv * PAIR, own.ut[0], own.ut[1]);
             own.vtt = ld_tile(reinterpret_cast<const T*>(slot + B.SIZE + C::OWN_UT) + wv * TILE);
         }
+        if (SUM && trans) { own.ut[0] = zero_frag<T>(); own.ut[1] = zero_frag<T>(); own.vtt = zero_frag<T>(); }
         const T* sBGT = reinterpret_cast<const T*>(slot + B.BGT);
         const T* sKGT = reinterpret_cast<const T*>(slot + B.KGT);
         const float* sEGL = reinterpret_cast<const float*>(slot + B.EGL);
@@ -381,7 +435,7 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
             __builtin_amdgcn_sched_barrier(0);
         }
         const Frag<T> vnb[2] = {to_frag<T>(vn[0]), to_frag<T>(vn[1])};
-        if (!WRITE_O) {
+        if (OUT == OUT_STATE) {
             // checkpoint of the entering state, as the fragments held here (tile pairs, 16 bytes per lane, whole
             // cache lines): the chunk_grad kernel turns them the way it needs them
             T* hc = NM ? reinterpret_cast<T*>(ob) + wv * PAIR : p.ws.HC + chw * (K * V) + vt * PAIR;
@@ -477,7 +531,9 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
         }
         if (NM) lds_barrier();                            // hands the last outbox to the memory waves
     }
-    if (p.ht) {
+    if (SUM) {
+        store_record<T, K>(S, p.seg.loc, p.seg.tr, rec, V, vt, trans);
+    } else if (p.ht && seg == p.seg.nseg - 1) {
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
@@ -487,8 +543,9 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
 
 // ---- backward ------------------------------------------------------------------------------------------------
 // Step t handles chunk c1-1-t.
-template <typename T, int K, int V, int NWC>
-__device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem, int n, int split) {
+template <typename T, int K, int V, int NWC, ScanOut OUT>
+__device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem, int n, int seg, int split) {
+    constexpr bool SUM = OUT == OUT_SUM;
     typedef ScanCfg<T, K, V, NWC> C;
     constexpr int KT = K / 16, KT2 = KT / 2, VT = V / 16, NM = C::NM, ES = sizeof(T);
     // LDS slot: [BG | WT] (BGT and W of the forward-scan block, transposed on their way in) | EGL | QGT | AQBT
@@ -498,19 +555,23 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
     constexpr bool PIPE = C::pipelined(false);
     constexpr bool PIPE_UPD = PIPE && C::early_update_reads(false);
     constexpr int NI = B.SIZE / 1024, SLOT = B.SIZE;
-    typedef ScanLds<T, K, V, NWC, SLOT, OUT_GRAD> L;
+    typedef ScanLds<T, K, V, NWC, SLOT, OUT> L;
     constexpr int OB_HC = L::OB_HC, OB = L::OB;
     char* const outbox = smem + NSLOT * SLOT;
 
     const int h = blockIdx.x;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int vt0 = split * NWC;
+    const bool trans = SUM && split >= C::SPLIT;
+    const int vt0 = (trans ? split - C::SPLIT : split) * NWC;
     const int l = lane_id(), g = l >> 4, c = l & 15;
     const int H = p.H;
-    int c0, c1;
-    seq_chunks(p.st, n, c0, c1);
+    int cs, ce, c0, c1;
+    seq_chunks(p.st, n, cs, ce);
+    seg_range(cs, ce, p.seg.nseg, seg, c0, c1);
     int64_t bos, eos;
     seq_bounds(p.st, n, bos, eos);
+    bos += (int64_t)(c0 - cs) * CH;
+    const int64_t rec = ((int64_t)n * p.H + h) * p.seg.nseg + seg;
     const int64_t chw0 = (int64_t)h * p.st.nch;
     const int nchunks = c1 - c0, first = c1 - 1;
     auto blk = [&](int t) __attribute__((always_inline)) {
@@ -522,6 +583,7 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
         if (nchunks <= 0) return;
         const int hw = wv - NWC;
         memory_wave<T, NI, NM ? NM : 1, NM ? C::DR_SHARE : NSLOT, SLOT, NT>(smem, nchunks, hw, blk, [&](int t) __attribute__((always_inline)) {
+            if (SUM) return;
             const int cid = first - t;
             const char* ob = outbox + (t & 1) * OB;
             char* hc = reinterpret_cast<char*>(p.ws.DHC + (chw0 + cid) * (K * V) + vt0 * PAIR);
@@ -544,7 +606,9 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
     const int64_t soff = ((int64_t)n * H + h) * K * V + 16 * vt + c;
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) dS[kt] = zero4();
-    if (p.dht) {
+    if (seg < p.seg.nseg - 1) {
+        load_entry<T, K, SUM>(dS, p.seg.rin, rec, V, vt, trans);
+    } else if (p.dht) {
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
@@ -556,7 +620,7 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
         const int cid = max(first - t, c0);
         const int64_t tok0 = bos + (int64_t)(cid - c0) * CH;
         const int len = (int)min((int64_t)CH, eos - tok0);
-        don = ld_frag(p.dout + ((tok0 + min(c, len - 1)) * H + h) * V + 16 * vt + 4 * g);
+        don = ld_frag(p.dout + ((tok0 + min(c, len - 1)) * H + h) * V + 16 * (trans ? 0 : vt) + 4 * g);
     };
 
     Frag<T> aq[2], bg[2][KT];                             // phase-1 operands; when pipelined, read a step ahead
@@ -596,7 +660,7 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) dsb[kt] = to_frag<T>(dS[kt]);
         const int len = (int)min((int64_t)CH, eos - (bos + (int64_t)(cid - c0) * CH));
-        if (c >= len) don = zero_frag<T>();
+        if (c >= len || trans) don = zero_frag<T>();
         const Frag<T> doT = transpose(don, ident);          // rows value, inner token
         // dv_new_s^T (rows value, inner token) = do^T A_qb^s + dS^T bg_s^T
         f32x4 dvn[2];
@@ -618,12 +682,14 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
         }
         const Frag<T> dvb[2] = {to_frag<T>(dvn[0]), to_frag<T>(dvn[1])};
         // gradient of the state leaving the chunk and of v_new, as the fragments held here (tile pairs)
+        if constexpr (!SUM) {
         T* dhc = NM ? reinterpret_cast<T*>(ob) + wv * PAIR : p.ws.DHC + chw * (K * V) + vt * PAIR;
         T* dvp = NM ? reinterpret_cast<T*>(ob + OB_HC) + wv * PAIR : p.ws.DVN + chw * (2 * CH * V) + vt * PAIR;
         constexpr int HSTR = (NM ? NWC : VT) * PAIR;
 #pragma unroll
         for (int kp = 0; kp < KT2; ++kp) st_pair2(dhc + kp * HSTR, dsb[2 * kp], dsb[2 * kp + 1]);
         st_pair2(dvp, dvb[0], dvb[1]);
+        }
         // dS <- exp(g_last) dS + qg^T do + sum_s w_s^T dv_new_s
 #pragma unroll
         for (int kp = 0; kp < KT2; ++kp) {
@@ -700,7 +766,9 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
         }
         if (NM) lds_barrier();
     }
-    if (p.dh0) {
+    if (SUM) {
+        store_record<T, K>(dS, p.seg.rloc, p.seg.rtr, rec, V, vt, trans);
+    } else if (p.dh0 && seg == 0) {
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
@@ -709,21 +777,24 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
 }
 
 // ---- kernels ---------------------------------------------------------------------------------------------------
-// grid = (H, directions * SPLIT, N): blockIdx.y = direction * SPLIT + split; blockIdx.z counts the sequences, packed
-// ones from the longest down.  Workgroups start in the order of their linear index (x fastest): the workgroups of one
-// (sequence, head) are H apart, which puts them on the same XCD (and its L2, where they share the chunk blocks) when H
-// is a multiple of 8, and when the launch has more workgroups than the device holds at once, the long sequences,
-// which decide when the launch ends, start first and the short ones fill in behind them.
-__device__ __forceinline__ int scan_sequence(const SeqTab& st) { return st.cu ? st.order[blockIdx.z] : (int)blockIdx.z; }
+// grid = (H, directions * SPLIT, N * segments): blockIdx.y = direction * SPLIT + split; blockIdx.z counts the sequences
+// (segment fastest), packed ones from the longest down.  Workgroups start in the order of their linear index (x fastest):
+// the workgroups of one (sequence, head) are H apart, which puts them on the same XCD (and its L2, where they share the
+// chunk blocks) when H is a multiple of 8, and when the launch has more workgroups than the device holds at once, the long
+// sequences, which decide when the launch ends, start first and the short ones fill in behind them.
+__device__ __forceinline__ int scan_sequence(const SeqTab& st, int z) { return st.cu ? st.order[z] : z; }
 template <typename T, int K, int V, int NWC, bool WRITE_O>
 __global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_fwd_kernel(ChunkArgs<T> p) {
-    __shared__ __attribute__((aligned(16))) char smem[ScanLds<T, K, V, NWC, blk_fwd(K, sizeof(T), WRITE_O).SIZE + ScanCfg<T, K, V, NWC>::OWN_FWD, WRITE_O ? OUT_O : OUT_STATE>::BYTES];
-    scan_fwd_body<T, K, V, NWC, WRITE_O>(p, smem, scan_sequence(p.st), blockIdx.y);
+    constexpr ScanOut OUT = WRITE_O ? OUT_O : OUT_STATE;
+    __shared__ __attribute__((aligned(16))) char smem[ScanLds<T, K, V, NWC, blk_fwd(K, sizeof(T), WRITE_O).SIZE + ScanCfg<T, K, V, NWC>::OWN_FWD, OUT>::BYTES];
+    const int z = blockIdx.z / p.seg.nseg, seg = blockIdx.z % p.seg.nseg;
+    scan_fwd_body<T, K, V, NWC, OUT>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
 }
 template <typename T, int K, int V, int NWC>
 __global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_bwd_kernel(ChunkArgs<T> p) {
     __shared__ __attribute__((aligned(16))) char smem[ScanLds<T, K, V, NWC, slot_bwd(K, sizeof(T)).SIZE, OUT_GRAD>::BYTES];
-    scan_bwd_body<T, K, V, NWC>(p, smem, scan_sequence(p.st), blockIdx.y);
+    const int z = blockIdx.z / p.seg.nseg, seg = blockIdx.z % p.seg.nseg;
+    scan_bwd_body<T, K, V, NWC, OUT_GRAD>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
 }
 // Both scans of the backward pass in one launch: they depend on the prep kernel only, not on each other.
 template <typename T, int K, int V, int NWC>
@@ -732,16 +803,78 @@ __global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_pair_ke
     constexpr int NB = ScanLds<T, K, V, NWC, slot_bwd(K, sizeof(T)).SIZE, OUT_GRAD>::BYTES;
     constexpr int SPLIT = ScanCfg<T, K, V, NWC>::SPLIT;
     __shared__ __attribute__((aligned(16))) char smem[NF > NB ? NF : NB];
-    const int n = scan_sequence(p.st);
-    if (blockIdx.y < SPLIT) scan_fwd_body<T, K, V, NWC, false>(p, smem, n, blockIdx.y);
-    else scan_bwd_body<T, K, V, NWC>(p, smem, n, blockIdx.y - SPLIT);
+    const int z = blockIdx.z / p.seg.nseg, seg = blockIdx.z % p.seg.nseg;
+    const int n = scan_sequence(p.st, z);
+    if (blockIdx.y < SPLIT) scan_fwd_body<T, K, V, NWC, OUT_STATE>(p, smem, n, seg, blockIdx.y);
+    else scan_bwd_body<T, K, V, NWC, OUT_GRAD>(p, smem, n, seg, blockIdx.y - SPLIT);
+}
+// The segments' records: grid = (H, directions * (V + K) / 16 / NWC, N * (segments - 1)); forward the segments before the
+// last, in reverse those behind the first.
+template <typename T, int K, int V, int NWC, bool BOTH>
+__global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_sum_kernel(ChunkArgs<T> p) {
+    constexpr int NF = ScanLds<T, K, V, NWC, blk_fwd(K, sizeof(T), false).SIZE + ScanCfg<T, K, V, NWC>::OWN_FWD, OUT_SUM>::BYTES;
+    constexpr int NB = ScanLds<T, K, V, NWC, slot_bwd(K, sizeof(T)).SIZE, OUT_SUM>::BYTES;
+    constexpr int SPLIT = ScanCfg<T, K, V, NWC>::SPLIT, COLS = (V + K) / 16 / NWC;
+    __shared__ __attribute__((aligned(16))) char smem[BOTH && NB > NF ? NB : NF];
+    const int z = blockIdx.z / (p.seg.nseg - 1), seg = blockIdx.z % (p.seg.nseg - 1);
+    const int n = scan_sequence(p.st, z), split = blockIdx.y % COLS;
+    if (!BOTH || (int)blockIdx.y < COLS) {
+        if (seg == 0 && split >= SPLIT) return;           // starts from h0: nobody asks for its transition
+        scan_fwd_body<T, K, V, NWC, OUT_SUM>(p, smem, n, seg, split);
+    } else {
+        if (seg + 1 == p.seg.nseg - 1 && split >= SPLIT) return;
+        scan_bwd_body<T, K, V, NWC, OUT_SUM>(p, smem, n, seg + 1, split);
+    }
+}
+// The records chained into what enters the segments, X <- M_s X + X_loc(s) from the segment that starts the sequence (or, in
+// reverse, ends it): grid = (H, directions * V/16, N), one wave per 16 rows of the state's column block.  A chain of
+// dependent steps, so a step is kept short: the wave's rows of the next transition matrix are requested a step ahead, the
+// waves exchange their rows through LDS (split operands: the error of fp32 products), one barrier a step.
+template <typename T, int K, int V>
+__global__ __launch_bounds__(64 * (K / 16)) void scan_chain_kernel(ChunkArgs<T> p) {
+    constexpr int KT = K / 16, VT = V / 16;
+    __shared__ __attribute__((aligned(16))) Split<T> sx[2][KT][64];
+    const int h = blockIdx.x, vt = blockIdx.y % VT, n = blockIdx.z, nseg = p.seg.nseg;
+    const bool rev = blockIdx.y >= VT;
+    const int kt = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane_id();
+    const float* const loc = rev ? p.seg.rloc : p.seg.loc;
+    const float* const tr = rev ? p.seg.rtr : p.seg.tr;
+    float* const in = rev ? p.seg.rin : p.seg.in;
+    const int64_t rec0 = ((int64_t)n * p.H + h) * nseg;
+    // step i handles the i-th segment from the start of the chain
+    auto rec = [&](int i) { return rec0 + (rev ? nseg - 1 - i : i); };
+    const int own = (vt * KT + kt) * TILE + 4 * l;
+    auto request = [&](int i, f32x4 (&m)[KT], f32x4& a) __attribute__((always_inline)) {
+        i = min(i, nseg - 2);                             // past the end: never used
+        a = *reinterpret_cast<const f32x4*>(loc + rec(i) * (K * V) + own);
+#pragma unroll
+        for (int ki = 0; ki < KT; ++ki) m[ki] = *reinterpret_cast<const f32x4*>(tr + rec(i) * (K * K) + (kt * KT + ki) * TILE + 4 * l);
+    };
+    f32x4 x = *reinterpret_cast<const f32x4*>(loc + rec(0) * (K * V) + own);
+    f32x4 m[KT], add;
+    request(1, m, add);
+    for (int i = 1; i < nseg; ++i) {
+        *reinterpret_cast<f32x4*>(in + rec(i) * (K * V) + own) = x;
+        if (i == nseg - 1) break;
+        Split<T> xs;
+        split(x, xs);
+        sx[i & 1][kt][l] = xs;
+        __syncthreads();
+        x = add;
+        Split<T> q[KT];
+#pragma unroll
+        for (int ki = 0; ki < KT; ++ki) split(m[ki], q[ki]);
+        request(i + 1, m, add);
+#pragma unroll
+        for (int ki = 0; ki < KT; ++ki) x = mm3(sx[i & 1][ki][l], q[ki], x);
+    }
 }
 
 // ---- launchers -------------------------------------------------------------------------------------------------
 template <typename T, int K, int V, int NWC>
 static hipError_t launch_scan_nwc(const ChunkArgs<T>& a, ScanKind kind, hipStream_t stream) {
     typedef ScanCfg<T, K, V, NWC> C;
-    dim3 grid(a.H, C::SPLIT * (kind == SCAN_PAIR ? 2 : 1), a.st.N), block(C::THREADS);
+    dim3 grid(a.H, C::SPLIT * (kind == SCAN_PAIR ? 2 : 1), a.st.N * a.seg.nseg), block(C::THREADS);
     switch (kind) {
         case SCAN_FWD_O: hipLaunchKernelGGL((scan_fwd_kernel<T, K, V, NWC, true>), grid, block, 0, stream, a); break;
         case SCAN_FWD: hipLaunchKernelGGL((scan_fwd_kernel<T, K, V, NWC, false>), grid, block, 0, stream, a); break;
@@ -758,7 +891,7 @@ template <typename T, int K, int V>
 hipError_t launch_scan_shape(const ChunkArgs<T>& a, ScanKind kind, hipStream_t stream) {
     constexpr int VT = V / 16;
     if constexpr (sizeof(T) == 2) {
-        const int lanes = a.H * a.st.N * (kind == SCAN_PAIR ? 2 : 1);
+        const int lanes = a.H * a.st.N * a.seg.nseg * (kind == SCAN_PAIR ? 2 : 1);
         if (lanes * 4 <= SCAN_TARGET_WORKGROUPS) return launch_scan_nwc<T, K, V, VT / 4>(a, kind, stream);
         // eight computing waves leave no room for memory waves: V = 128 is always split at least in two
         if (lanes * 2 <= SCAN_TARGET_WORKGROUPS || VT == 8) return launch_scan_nwc<T, K, V, VT / 2>(a, kind, stream);
@@ -767,6 +900,19 @@ hipError_t launch_scan_shape(const ChunkArgs<T>& a, ScanKind kind, hipStream_t s
     } else {
         return launch_scan_nwc<T, K, V, VT>(a, kind, stream);
     }
+}
+
+template <typename T, int K, int V>
+hipError_t launch_scan_segments_shape(const ChunkArgs<T>& a, bool both, hipStream_t stream) {
+    constexpr int NWC = 4;                                // column blocks per workgroup: each fetches the chunks' operands once for them
+    typedef ScanCfg<T, K, V, NWC> C;
+    dim3 grid(a.H, (V + K) / 16 / NWC * (both ? 2 : 1), a.st.N * (a.seg.nseg - 1)), block(C::THREADS);
+    if (both) hipLaunchKernelGGL((scan_sum_kernel<T, K, V, NWC, true>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((scan_sum_kernel<T, K, V, NWC, false>), grid, block, 0, stream, a);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((scan_chain_kernel<T, K, V>), dim3(a.H, V / 16 * (both ? 2 : 1), a.st.N), dim3(64 * (K / 16)), 0, stream, a);
+    return hipGetLastError();
 }
 
 }  // namespace hdla

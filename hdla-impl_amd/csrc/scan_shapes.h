@@ -8,5 +8,8 @@ namespace hdla {
 enum ScanKind { SCAN_FWD_O, SCAN_FWD, SCAN_BWD, SCAN_PAIR };   // forward scan with / without the output, reverse, both
 
 template <typename T, int K, int V> hipError_t launch_scan_shape(const ChunkArgs<T>& a, ScanKind kind, hipStream_t stream);
+// several time segments: the segments' records (forward direction, or with `both` the reverse one too), then the states
+// (and state gradients) that enter them
+template <typename T, int K, int V> hipError_t launch_scan_segments_shape(const ChunkArgs<T>& a, bool both, hipStream_t stream);
 
 }  // namespace hdla

@@ -98,3 +98,25 @@ def test_layer_as_one_call_against_its_steps(B, T, d, H, kw):
             outs.append(y + [cache[0]["recurrent_state"][0]])
     for a, b in zip(*outs):
         assert O.rel_l2(a, b) <= 1e-2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,K,V,segments", [(torch.bfloat16, 128, 128, 4), (torch.bfloat16, 128, 64, 7), (torch.bfloat16, 64, 128, 2),
+                                                (torch.float32, 64, 64, 4), (torch.float32, 128, 128, 3), (torch.float32, 64, 128, 5)])
+@pytest.mark.parametrize("T,cu", [(145, None), (150, [0, 33, 33, 40, 150])])
+def test_time_segments_of_the_stand_alone_scans(dtype, K, V, segments, T, cu, monkeypatch):
+    """The scans cut into time segments (ragged last chunks, segments without chunks, an empty sequence, segments longer and
+    shorter than the scans' rings) against whole sequences."""
+    from oracle import hrdplr_oracle as O
+    x = make_inputs(44, 1, T, 2, K, V, gk_div=4.0, n_states=None if cu is None else len(cu) - 1)
+    leaves = [t.to(dtype).to(DEV).requires_grad_() for t in (x.q, x.k, x.v, x.a, x.b, x.gk)]
+    h0 = x.h0.to(DEV).requires_grad_()
+    cu = None if cu is None else torch.tensor(cu, device=DEV)
+    res = []
+    for n in (segments, 1):
+        monkeypatch.setenv("HDLA_HIP_SEGMENTS", str(n))
+        o, ht = chunk_hrdplr_delta_rule(*leaves, 2, scale=0.7, initial_state=h0, output_final_state=True, cu_seqlens=cu)
+        res.append([o.detach(), ht.detach()] + list(torch.autograd.grad([o, ht], leaves + [h0], [x.do.to(dtype).to(DEV), x.dht.to(DEV)])))
+    errs = [O.rel_l2(a, b) for a, b in zip(*res)]
+    print([f"{e:.1e}" for e in errs], flush=True)
+    assert max(errs) <= (6e-3 if dtype == torch.bfloat16 else 3e-6)
