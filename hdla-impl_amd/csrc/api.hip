@@ -223,6 +223,15 @@ void bind_ws(ChunkArgs<T>& a, const hdla_dims* d, const WsLayout& LP, void* prep
     a.st.nch = nch;
 }
 
+template <typename T> PackedOut packed_outputs(const hdla_dims* d, const ChunkArgs<T>& a) {
+    PackedOut out{};
+    const long long rows = (long long)d->T * d->H, k = rows * d->K * sizeof(T), v = rows * d->V * sizeof(T);
+    out.add(a.o, v);
+    out.add(a.dq, k); out.add(a.dk, k); out.add(a.dv, v); out.add(a.da, 2 * k); out.add(a.db, 2 * k);
+    out.add(a.dgk, rows * d->K * (a.gk_f32 ? 4 : 2)); out.add(a.dbeta, rows * sizeof(T));
+    return out;
+}
+
 inline bool bad_ws(const void* p, size_t have, size_t need) {
     return !p || (reinterpret_cast<uintptr_t>(p) & 255) || have < need;
 }
@@ -271,7 +280,7 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
     if (d->cu_seqlens && (stages & HDLA_STAGE_PREP)) {
         char* base = static_cast<char*>(prep_ws);
         e = launch_chunk_table(d->cu_seqlens, d->N, d->T, nch, reinterpret_cast<int32_t*>(base + LP.CHUNK_OFF),
-                               reinterpret_cast<int32_t*>(base + LP.CHUNK_SEQ), stream);
+                               reinterpret_cast<int32_t*>(base + LP.CHUNK_SEQ), packed_outputs(d, a), stream);
         if (e != hipSuccess) return (int)e;
     }
     if (nch > 0 && (stages & HDLA_STAGE_PREP)) {
@@ -348,7 +357,7 @@ int run_fused(const hdla_dims* d, bool fwd, const void* q, const void* k, const 
     hipError_t e;
     if (d->cu_seqlens && (stages & HDLA_STAGE_PREP)) {
         e = launch_chunk_table(d->cu_seqlens, d->N, d->T, L.nch, reinterpret_cast<int32_t*>(base + L.CHUNK_OFF),
-                               reinterpret_cast<int32_t*>(base + L.CHUNK_SEQ), stream);
+                               reinterpret_cast<int32_t*>(base + L.CHUNK_SEQ), packed_outputs(d, a), stream);
         if (e != hipSuccess) return (int)e;
     }
     if (fwd) {

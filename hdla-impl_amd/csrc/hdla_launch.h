@@ -6,7 +6,16 @@
 
 namespace hdla {
 
-hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int32_t* chunk_off, int32_t* chunk_seq, hipStream_t stream);
+// Outputs of a call on a packed batch.  The kernels write the rows of the sequences; a table that is not a partition of the
+// tokens (it may come unchecked from the device) leaves rows that belong to none, and these are to read as zeros.
+struct PackedOut {
+    void* p[7];
+    long long bytes[7];       // multiples of 2
+    int n;
+    void add(void* q, long long b) { if (q) { p[n] = q; bytes[n++] = b; } }
+};
+hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int32_t* chunk_off, int32_t* chunk_seq, const PackedOut& out,
+                              hipStream_t stream);
 
 // K, V in {64, 128}; returns hipErrorInvalidValue for any other pair.
 // mode: 0 = for the forward pass, 1 = for the backward pass, 2 = forward pass whose workspace the backward pass will use

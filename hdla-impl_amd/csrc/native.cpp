@@ -127,12 +127,9 @@ Tensor workspace(const hdla_dims& d, int pass, const Tensor& like) {
     return bytes_like(like, n);
 }
 
-// rows outside every sequence of a packed batch are written by nobody: zeros there
-Tensor fresh(const Tensor& like, bool packed) { return packed ? at::zeros_like(like) : at::empty_like(like); }
-
 void chunk_forward(const ChunkIn& x, const hdla_dims& d, bool want_ht, bool want_boundary, Tensor& o, Tensor& ht, Tensor& boundary) {
     const auto f32 = x.q.options().dtype(at::kFloat);
-    o = fresh(x.v, x.cu.defined());
+    o = at::empty_like(x.v);
     if (want_ht) ht = at::empty({d.N, d.H, d.K, d.V}, f32);
     const size_t nb = want_boundary ? api.boundary_bytes(&d) : 0;
     if (nb) boundary = bytes_like(x.q, nb);
@@ -171,12 +168,11 @@ struct ChunkFn : torch::autograd::Function<ChunkFn> {
         const Tensor d_o = grads[0].defined() ? grads[0].to(x.v.scalar_type()).contiguous() : at::zeros_like(x.v);
         Tensor dht;
         if (grads.size() > 1 && grads[1].defined()) dht = grads[1].to(at::kFloat).contiguous();
-        const bool packed = x.cu.defined();
         const Tensor ws = workspace(d, HDLA_PASS_BWD, x.q);
-        const Tensor dq = fresh(x.q, packed), dk = fresh(x.k, packed), dv = fresh(x.v, packed), dgk = fresh(x.gk, packed);
+        const Tensor dq = at::empty_like(x.q), dk = at::empty_like(x.k), dv = at::empty_like(x.v), dgk = at::empty_like(x.gk);
         Tensor da, db, dbeta, dh0;
-        if (x.beta.defined()) dbeta = fresh(x.beta, packed);
-        else { da = fresh(x.a, packed); db = fresh(x.b, packed); }
+        if (x.beta.defined()) dbeta = at::empty_like(x.beta);
+        else { da = at::empty_like(x.a); db = at::empty_like(x.b); }
         if (x.h0.defined()) dh0 = at::empty_like(x.h0);
         check(api.chunk_bwd_b(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.beta), ptr(x.gk), fptr(x.h0), ptr(d_o), fptr(dht),
                               ptr(dq), ptr(dk), ptr(dv), ptr(da), ptr(db), ptr(dbeta), ptr(dgk), fptr(dh0), ptr(boundary),
@@ -349,7 +345,7 @@ PyObject* run_recurrent(ChunkIn& x, PyObject* pscale, PyObject* pwant, PyObject*
         const at::DeviceGuard guard(x.q.device());
         make_contiguous(x);
         if (x.h0.defined()) x.h0 = x.h0.to(at::kFloat).contiguous();
-        const Tensor o = fresh(x.v, x.cu.defined());
+        const Tensor o = x.cu.defined() ? at::zeros_like(x.v) : at::empty_like(x.v);     // rows of no sequence stay zero
         Tensor ht;
         if (want) ht = at::empty({d.N, d.H, d.K, d.V}, x.q.options().dtype(at::kFloat));
         if (x.beta.defined())

@@ -355,12 +355,15 @@ constexpr int ORDER_MAX_N = 2048;      // beyond this many sequences they are ta
 constexpr int TABLE_THREADS = 256;
 // Workgroup 0 builds the table; with at most ORDER_MAX_N sequences, workgroups 1 .. ceil(N / 256) rank the sequences by
 // their chunk counts, one sequence a thread (they form the counts from cu themselves, so they wait for nobody).
+// Workgroup 0 also looks whether the table is a partition of the T tokens, which it is unless the caller made a mistake, and
+// only if it is not clears the outputs `out` (clearing them for every call took 88 of 2050 us of a training step on 16384
+// tokens, H = 16, K = V = 128).
 __global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const int64_t* cu, int N, int T, int nch, int32_t* chunk_off,
-                                                                          int32_t* chunk_seq) {
+                                                                          int32_t* chunk_seq, PackedOut out) {
     constexpr int LONG_SEQ = 64, LONG_LIST = 512;
     __shared__ long long strip[2][TABLE_THREADS];
     __shared__ __attribute__((aligned(16))) int32_t len[ORDER_MAX_N];
-    __shared__ int n_long, long_seq[LONG_LIST], long_c0[LONG_LIST], long_c1[LONG_LIST];
+    __shared__ int n_gaps, n_long, long_seq[LONG_LIST], long_c0[LONG_LIST], long_c1[LONG_LIST];
     const int t = threadIdx.x;
     auto chunks_of = [&](int n) {
         int64_t bos, eos;
@@ -393,11 +396,16 @@ __global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const 
     const int per = (N + TABLE_THREADS - 1) / TABLE_THREADS;
     const int n0 = min(t * per, N), n1 = min(n0 + per, N);
     long long own = 0;
+    int gaps = t == 0 && (cu[0] != 0 || cu[N] != T);
 #pragma unroll 8
-    for (int n = n0; n < n1; ++n) own += chunks_of(n);
+    for (int n = n0; n < n1; ++n) {
+        own += chunks_of(n);
+        gaps |= cu[n + 1] < cu[n];
+    }
     strip[0][t] = own;
-    if (t == 0) n_long = 0;
+    if (t == 0) { n_long = 0; n_gaps = 0; }
     __syncthreads();
+    if (gaps) atomicAdd(&n_gaps, 1);                      // read behind the barriers of the scan below
     int cur = 0;
     for (int d = 1; d < TABLE_THREADS; d <<= 1) {         // inclusive scan, one doubling step per round
         strip[cur ^ 1][t] = strip[cur][t] + (t >= d ? strip[cur][t - d] : 0);
@@ -426,6 +434,9 @@ __global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const 
         for (int cid = long_c0[i] + t; cid < long_c1[i]; cid += TABLE_THREADS) chunk_seq[cid] = long_seq[i];
     if (N > ORDER_MAX_N)                                  // too many to rank: as they come
         for (int n = t; n < N; n += TABLE_THREADS) order[n] = n;
+    if (n_gaps)
+        for (int i = 0; i < out.n; ++i)
+            for (long long e = t; e < out.bytes[i] / 2; e += TABLE_THREADS) static_cast<uint16_t*>(out.p[i])[e] = 0;
 }
 
 template <typename T, int K, int V, bool HD>
@@ -463,9 +474,10 @@ hipError_t launch_prep(const ChunkArgs<T>& a, int K, int V, int mode, hipStream_
 template hipError_t launch_prep<bf16>(const ChunkArgs<bf16>&, int, int, int, hipStream_t);
 template hipError_t launch_prep<float>(const ChunkArgs<float>&, int, int, int, hipStream_t);
 
-hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int32_t* chunk_off, int32_t* chunk_seq, hipStream_t stream) {
+hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int32_t* chunk_off, int32_t* chunk_seq, const PackedOut& out,
+                              hipStream_t stream) {
     const int rankers = N <= ORDER_MAX_N ? (N + TABLE_THREADS - 1) / TABLE_THREADS : 0;
-    hipLaunchKernelGGL(build_chunk_table_kernel, dim3(1 + rankers), dim3(TABLE_THREADS), 0, stream, cu, N, T, nch, chunk_off, chunk_seq);
+    hipLaunchKernelGGL(build_chunk_table_kernel, dim3(1 + rankers), dim3(TABLE_THREADS), 0, stream, cu, N, T, nch, chunk_off, chunk_seq, out);
     return hipGetLastError();
 }
 

@@ -203,7 +203,7 @@ def check_cu_seqlens(cu_seqlens: torch.Tensor, T: int) -> None:
     """Validate a packed-sequence table that is still on the CPU (free: no device synchronisation): it must start at
     0, end at T and never decrease.  A table that already lives on the GPU is not read back; the kernels force its
     entries into [0, T], so a bad one cannot cause an access outside the tensors, but rows that belong to no sequence
-    are then left unwritten in the outputs."""
+    are then zeros in the outputs."""
     if cu_seqlens.dim() != 1 or cu_seqlens.numel() < 2:
         raise ValueError(f"cu_seqlens must be a 1-d tensor of N+1 >= 2 entries, got shape {tuple(cu_seqlens.shape)}")
     if cu_seqlens.is_cuda:

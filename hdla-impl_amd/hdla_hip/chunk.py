@@ -80,8 +80,7 @@ def chunk_hrdplr_fwd(q, k, v, a, b, gk, scale, initial_state, output_final_state
     N = B if cu_seqlens is None else cu_seqlens.numel() - 1
     with torch.cuda.device(q.device):
         dims = _dims(q, v, gk, scale, cu_seqlens, N)
-        # with a packed-sequence table that was not validated on the host, rows outside every sequence stay unwritten
-        o = torch.zeros_like(v) if cu_seqlens is not None else torch.empty_like(v)
+        o = torch.empty_like(v)
         ht = torch.empty(N, H, K, V, dtype=torch.float32, device=q.device) if output_final_state else None
         if keep:
             ws = _lib.workspace(dims, _lib.PASS_FWD_KEEP, q.device)
@@ -142,8 +141,7 @@ def chunk_hrdplr_bwd(q, k, v, a, b, gk, scale, initial_state, do, dht, cu_seqlen
     B, T, H, K = q.shape
     V = v.shape[-1]
     N = B if cu_seqlens is None else cu_seqlens.numel() - 1
-    # rows outside every sequence of a packed batch stay unwritten: they must not carry garbage upstream
-    new = torch.zeros_like if cu_seqlens is not None else torch.empty_like
+    new = torch.empty_like
     with torch.cuda.device(q.device):
         dims = _dims(q, v, gk, scale, cu_seqlens, N)
         ws = _lib.workspace(dims, 1, q.device)

@@ -101,6 +101,29 @@ def test_layer_as_one_call_against_its_steps(B, T, d, H, kw):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("K", [64, 128])
+def test_rows_of_no_sequence_are_zeros(K):
+    """A table that comes unchecked from the device and leaves rows out (gaps at both ends and between, where it falls):
+    outputs and gradients read zero there, and the covered rows are those of the same sequences by themselves."""
+    T, H = 60, 2
+    cu = torch.tensor([3, 20, 14, 14, 30, 41], device=DEV)          # sequences 3..20, 14..14, 14..30 (overlapping), 30..41
+    x = make_inputs(43, 1, T, H, K, K, n_states=5)
+    leaves = [t.bfloat16().to(DEV).requires_grad_() for t in (x.q, x.k, x.v, x.a, x.b, x.gk)]
+    junk = [torch.full((1 << 22,), float("nan"), device=DEV) for _ in range(8)]         # what recycled memory may hold
+    del junk
+    o, _ = chunk_hrdplr_delta_rule(*leaves, 2, cu_seqlens=cu)
+    g = torch.autograd.grad(o, leaves, x.do.bfloat16().to(DEV))
+    inside = torch.zeros(T, dtype=torch.bool, device=DEV)
+    inside[3:41] = True
+    for t in (o, *g):
+        r = 2 if t.shape[1] == 2 * T else 1
+        rows = inside.repeat_interleave(r)
+        assert bool((t[0, ~rows] == 0).all()) and torch.isfinite(t.float()).all()
+    alone, _ = chunk_hrdplr_delta_rule(*[t[:, 30 * (t.shape[1] // T):41 * (t.shape[1] // T)] for t in leaves], 2)
+    assert torch.equal(alone, o[:, 30:41])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype,K,V,segments", [(torch.bfloat16, 128, 128, 4), (torch.bfloat16, 128, 64, 7), (torch.bfloat16, 64, 128, 2),
                                                 (torch.float32, 64, 64, 4), (torch.float32, 128, 128, 3), (torch.float32, 64, 128, 5)])
 @pytest.mark.parametrize("T,cu", [(145, None), (150, [0, 33, 33, 40, 150])])
