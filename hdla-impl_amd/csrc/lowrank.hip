@@ -1,0 +1,328 @@
+// Matrix products of the HDLA layer for which a BLAS call is the wrong tool.
+//
+// layer_up: the second halves of the layer's two low-rank projections (f_proj and output_gate, HRDPLR/hdla_custom.py:117-121,
+// 151-155: Linear(head_dim -> embed_dim)) and log_f = logsigmoid(f) (:219), in one launch.  x0 [M, D] -> [M, d] with D = 64
+// or 128 is bound by what it writes (M x d, three times).  As two BLAS calls and an elementwise kernel it took
+// 14.6 + 9.1 + 10.1 us at M = 8192, d = 1024, and in a decode step three launches of 4.5 us and 40 us of host time.
+// layer_down: their input gradients, dx0 [M, D] = dY [M, d] W [d, D], with dY = dlog_f sigmoid(-f) formed on the way in for
+// the first (before: 12 + 12 us and a pass of its own for dY, 10.7 us).
+// rows_gemm: y [M, N] = x [M, K] W [N, K]^T for at most 64 rows, i.e. the large projections of a decode step: a stream of W,
+// all of the chip's workgroups on it, where the BLAS call costs 20 us of host time and 10 us (16 x 6416 x 2048).
+//
+// bf16 in and out, fp32 accumulation.  Operands are read 16 bytes a lane; the eight elements are two fragments whose inner
+// index is permuted the same way on both sides (elements 8j..8j+3 and 8j+4..8j+7, see ld_two_tiles in skinny.hip), which a
+// sum over that index does not notice.
+#include "hdla_common.cuh"
+#include "../../include/hdla_hip.h"
+
+namespace hdla {
+
+struct TwoTiles { Frag<bf16> a, b; };
+__device__ __forceinline__ TwoTiles ld16(const bf16* p) {
+    const s16x8 x = *reinterpret_cast<const s16x8*>(p);
+    TwoTiles t;
+    t.a.v = __builtin_shufflevector(x, x, 0, 1, 2, 3);
+    t.b.v = __builtin_shufflevector(x, x, 4, 5, 6, 7);
+    return t;
+}
+// column 8g + i (tile a) and 8g + 4 + i (tile b) of a 32-column block, row c: eight consecutive elements of a row
+__device__ __forceinline__ void st16(bf16* p, f32x4 a, f32x4 b) {
+    const Frag<bf16> fa = to_frag<bf16>(a), fb = to_frag<bf16>(b);
+    *reinterpret_cast<s16x8*>(p) = __builtin_shufflevector(fa.v, fb.v, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+// row of a 32-row block that lane c of a fragment holds, for tile a (+ 4 for tile b)
+__device__ __forceinline__ int row8(int c) { return 8 * (c >> 2) + (c & 3); }
+
+// log(sigmoid(x)) as logsigmoid_kernel<bf16> forms it (layer_pre.hip)
+__device__ __forceinline__ float logsig(float x) {
+    const float e = __expf(-fabsf(x));
+    return fminf(x, 0.f) - (e < 1e-4f ? e : __logf(1.f + e));
+}
+
+struct UpArgs {
+    const bf16 *x0[2], *w[2];             // inner activations [M, D] (rows ldx apart), weights [d, D]: decay, gate
+    bf16 *f, *log_f, *gate;               // [M, d]; f may be null (nothing but log_f is asked for)
+    long long ldx;
+    int M, d;
+};
+// A wave per 16 rows and 64 columns; blockIdx.y: decay or gate.
+template <int D>
+__global__ __launch_bounds__(256) void layer_up_kernel(UpArgs p) {
+    constexpr int KB = D / 32;
+    const int l = lane_id(), g = l >> 4, c = l & 15, which = blockIdx.y;
+    const long long unit = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int cbs = p.d / 64;
+    const long long r0 = unit / cbs * 16;
+    const int n0 = (int)(unit % cbs) * 64;
+    if (r0 >= p.M) return;
+    const bool ok = r0 + c < p.M;
+    const bf16* x = p.x0[which] + min(r0 + c, (long long)p.M - 1) * p.ldx + 8 * g;
+    const bf16* w = p.w[which] + (long long)(n0 + row8(c)) * D + 8 * g;
+    TwoTiles xf[KB], wf[2][2][KB];
+#pragma unroll
+    for (int k = 0; k < KB; ++k) xf[k] = ld16(x + 32 * k);
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int k = 0; k < KB; ++k) wf[b][h][k] = ld16(w + (32 * b + 4 * h) * D + 32 * k);
+    const long long out = (r0 + c) * p.d + n0 + 8 * g;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        f32x4 acc[2] = {zero4(), zero4()};
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int k = 0; k < KB; ++k) {
+                acc[h] = mm(xf[k].a, wf[b][h][k].a, acc[h]);
+                acc[h] = mm(xf[k].b, wf[b][h][k].b, acc[h]);
+            }
+        if (!ok) continue;
+        if (which == 1) {
+            st16(p.gate + out + 32 * b, acc[0], acc[1]);
+        } else {
+            if (p.f) st16(p.f + out + 32 * b, acc[0], acc[1]);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const f32x4 r = to_f32(to_frag<bf16>(acc[h]));         // f as the stored tensor has it
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[h][i] = logsig(r[i]);
+            }
+            st16(p.log_f + out + 32 * b, acc[0], acc[1]);
+        }
+    }
+}
+
+struct DownArgs {
+    const bf16 *dy[2], *f, *w[2];         // dlog_f, dgate [M, d]; f [M, d]; weights [d, D]
+    bf16* dx[2];                          // [M, D], rows ldx apart
+    long long ldx;
+    int M, d;
+};
+// A workgroup per 16 MT rows; its four waves share out the columns of dY and add up through LDS; blockIdx.y: decay or gate.
+// W has the contraction index outermost: its tiles are turned by a product with the identity, once for MT row tiles.
+template <int D, int MT>
+__global__ __launch_bounds__(256) void layer_down_kernel(DownArgs p) {
+    constexpr int DB = D / 32;
+    __shared__ f32x4 red[3][MT * 2 * DB][64];
+    const int wv = threadIdx.x >> 6, l = lane_id(), g = l >> 4, c = l & 15, which = blockIdx.y;
+    const long long r0 = (long long)blockIdx.x * (16 * MT);
+    const Frag<bf16> id = ident_frag<bf16>();
+    f32x4 acc[MT][2 * DB];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int b = 0; b < 2 * DB; ++b) acc[m][b] = zero4();
+    const bf16* dy[MT];
+    const bf16* fr[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const long long row = min(r0 + 16 * m + c, (long long)p.M - 1);   // rows past the end: computed, not stored
+        dy[m] = p.dy[which] + row * p.d + 8 * g;
+        fr[m] = p.f + row * p.d + 8 * g;
+    }
+#pragma unroll 2
+    for (int n0 = 32 * wv; n0 < p.d; n0 += 128) {
+        TwoTiles y[MT], ff[MT], wt[2][DB];
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            y[m] = ld16(dy[m] + n0);
+            if (which == 0) ff[m] = ld16(fr[m] + n0);
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int b = 0; b < DB; ++b) wt[h][b] = ld16(p.w[which] + (long long)(n0 + row8(c) + 4 * h) * D + 32 * b + 8 * g);
+        if (which == 0) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                // df = dlog_f sigmoid(-f), rounded as the stored gradient would be
+                auto one = [](Frag<bf16>& d, Frag<bf16> f) __attribute__((always_inline)) {
+                    f32x4 x = to_f32(d), z = to_f32(f);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) x[i] *= 1.f / (1.f + __expf(z[i]));
+                    d = to_frag<bf16>(x);
+                };
+                one(y[m].a, ff[m].a);
+                one(y[m].b, ff[m].b);
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int b = 0; b < DB; ++b) {
+                const Frag<bf16> ta = transpose(wt[h][b].a, id), tb = transpose(wt[h][b].b, id);
+#pragma unroll
+                for (int m = 0; m < MT; ++m) {
+                    const Frag<bf16> x = h == 0 ? y[m].a : y[m].b;
+                    acc[m][2 * b] = mm(x, ta, acc[m][2 * b]);
+                    acc[m][2 * b + 1] = mm(x, tb, acc[m][2 * b + 1]);
+                }
+            }
+    }
+    if (wv) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int b = 0; b < 2 * DB; ++b) red[wv - 1][m * 2 * DB + b][l] = acc[m][b];
+    }
+    __syncthreads();
+    if (wv) return;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        if (r0 + 16 * m + c >= p.M) continue;
+#pragma unroll
+        for (int b = 0; b < DB; ++b) {
+            f32x4 s[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int i = m * 2 * DB + 2 * b + h;
+                s[h] = acc[m][2 * b + h] + red[0][i][l] + red[1][i][l] + red[2][i][l];
+            }
+            st16(p.dx[which] + (r0 + 16 * m + c) * p.ldx + 32 * b + 8 * g, s[0], s[1]);
+        }
+    }
+}
+
+// y [M, N] = x [M, K] W [N, K]^T, M <= 16 MT.  A workgroup per 16 rows of W; its four waves take every fourth 32-column
+// block of K and add up through LDS.  Bound by the stream of W, of which a wave keeps UNR blocks in flight; from some 16
+// million weights on by the x that every workgroup reads again (from L2), which is where the BLAS library's larger tiles
+// win (1 x 12576 x 4096: 35 us here, 26 there).
+template <int MT>
+__global__ __launch_bounds__(256) void rows_gemm_kernel(const bf16* __restrict__ x, long long ldx, const bf16* __restrict__ w, long long ldw,
+                                                        bf16* __restrict__ y, long long ldy, int M, int N, int K) {
+    constexpr int UNR = MT <= 2 ? 8 : 4;
+    __shared__ f32x4 red[3][MT][64];
+    const int wv = threadIdx.x >> 6, l = lane_id(), g = l >> 4, c = l & 15;
+    const int n0 = blockIdx.x * 16;
+    const bf16* wr = w + (long long)min(n0 + c, N - 1) * ldw + 8 * g;
+    const bf16* xr[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) xr[m] = x + (long long)min(16 * m + c, M - 1) * ldx + 8 * g;
+    f32x4 acc[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[m] = zero4();
+    int k = 32 * wv;
+    for (; k + 128 * (UNR - 1) < K; k += 128 * UNR) {
+        TwoTiles a[UNR], b[UNR][MT];
+#pragma unroll
+        for (int u = 0; u < UNR; ++u) {
+            a[u] = ld16(wr + k + 128 * u);
+#pragma unroll
+            for (int m = 0; m < MT; ++m) b[u][m] = ld16(xr[m] + k + 128 * u);
+        }
+        __builtin_amdgcn_sched_barrier(0);                // all of them requested before the first is waited for
+#pragma unroll
+        for (int u = 0; u < UNR; ++u)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                acc[m] = mm(b[u][m].a, a[u].a, acc[m]);
+                acc[m] = mm(b[u][m].b, a[u].b, acc[m]);
+            }
+    }
+    for (; k < K; k += 128) {
+        const TwoTiles a = ld16(wr + k);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const TwoTiles b = ld16(xr[m] + k);
+            acc[m] = mm(b.a, a.a, acc[m]);
+            acc[m] = mm(b.b, a.b, acc[m]);
+        }
+    }
+    if (wv) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) red[wv - 1][m][l] = acc[m];
+    }
+    __syncthreads();
+    if (wv) return;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const f32x4 s = acc[m] + red[0][m][l] + red[1][m][l] + red[2][m][l];
+        if (16 * m + c >= M) continue;
+        bf16* o = y + (long long)(16 * m + c) * ldy + n0 + 4 * g;
+        if (n0 + 4 * g + 3 < N) st_frag(o, to_frag<bf16>(s));
+        else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) if (n0 + 4 * g + i < N) st_elem(o + i, s[i]);
+        }
+    }
+}
+
+static bool lr_al(const void* p, int a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
+static int lr_check(const hdla_up_dims* q) {
+    if (!q) return HDLA_ERR_NULL;
+    if (q->rows < 0 || q->rows > 0x7fffffff || (q->D != 64 && q->D != 128) || q->d <= 0 || q->d % 128) return HDLA_ERR_SHAPE;
+    if (q->ld < q->D || q->ld % 8 || q->col_f < 0 || q->col_g < 0 || q->col_f % 8 || q->col_g % 8) return HDLA_ERR_ALIGN;
+    if (q->col_f + q->D > q->ld || q->col_g + q->D > q->ld) return HDLA_ERR_SHAPE;
+    return HDLA_OK;
+}
+
+}  // namespace hdla
+
+using namespace hdla;
+
+extern "C" int hdla_layer_up_fwd(const hdla_up_dims* dims, const void* y, const void* wf, const void* wg, void* f, void* log_f, void* gate,
+                                 void* stream) {
+    const int rc = lr_check(dims);
+    if (rc) return rc;
+    if (dims->rows == 0) return HDLA_OK;
+    if (!y || !wf || !wg || !log_f || !gate) return HDLA_ERR_NULL;
+    for (const void* p : {y, wf, wg, (const void*)f, (const void*)log_f, (const void*)gate}) if (!lr_al(p, 16)) return HDLA_ERR_ALIGN;
+    const long long units = (dims->rows + 15) / 16 * (dims->d / 64);
+    if ((units + 3) / 4 > 0x7fffffffLL) return HDLA_ERR_SHAPE;
+    UpArgs a{};
+    a.x0[0] = static_cast<const bf16*>(y) + dims->col_f; a.x0[1] = static_cast<const bf16*>(y) + dims->col_g;
+    a.w[0] = static_cast<const bf16*>(wf); a.w[1] = static_cast<const bf16*>(wg);
+    a.f = static_cast<bf16*>(f); a.log_f = static_cast<bf16*>(log_f); a.gate = static_cast<bf16*>(gate);
+    a.ldx = dims->ld; a.M = (int)dims->rows; a.d = dims->d;
+    const dim3 grid((unsigned)((units + 3) / 4), 2), block(256);
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    if (dims->D == 64) hipLaunchKernelGGL(layer_up_kernel<64>, grid, block, 0, s, a);
+    else hipLaunchKernelGGL(layer_up_kernel<128>, grid, block, 0, s, a);
+    return (int)hipGetLastError();
+}
+
+extern "C" int hdla_layer_down(const hdla_up_dims* dims, const void* wf, const void* wg, const void* f, const void* dlog_f, const void* dgate,
+                               void* dy, void* stream) {
+    const int rc = lr_check(dims);
+    if (rc) return rc;
+    if (dims->rows == 0) return HDLA_OK;
+    if (!wf || !wg || !f || !dlog_f || !dgate || !dy) return HDLA_ERR_NULL;
+    for (const void* p : {wf, wg, f, dlog_f, dgate, (const void*)dy}) if (!lr_al(p, 16)) return HDLA_ERR_ALIGN;
+    DownArgs a{};
+    a.dy[0] = static_cast<const bf16*>(dlog_f); a.dy[1] = static_cast<const bf16*>(dgate); a.f = static_cast<const bf16*>(f);
+    a.w[0] = static_cast<const bf16*>(wf); a.w[1] = static_cast<const bf16*>(wg);
+    a.dx[0] = static_cast<bf16*>(dy) + dims->col_f; a.dx[1] = static_cast<bf16*>(dy) + dims->col_g;
+    a.ldx = dims->ld; a.M = (int)dims->rows; a.d = dims->d;
+    const dim3 block(256);
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    // row tiles a workgroup: what the registers hold; few rows are spread over more workgroups
+    const bool wide = dims->rows >= 4096;
+    const auto grid = [&](int mt) { return dim3((unsigned)((dims->rows + 16 * mt - 1) / (16 * mt)), 2); };
+    if (dims->D == 64) {
+        if (wide) hipLaunchKernelGGL((layer_down_kernel<64, 2>), grid(2), block, 0, s, a);
+        else hipLaunchKernelGGL((layer_down_kernel<64, 1>), grid(1), block, 0, s, a);
+    } else {
+        if (wide) hipLaunchKernelGGL((layer_down_kernel<128, 2>), grid(2), block, 0, s, a);
+        else hipLaunchKernelGGL((layer_down_kernel<128, 1>), grid(1), block, 0, s, a);
+    }
+    return (int)hipGetLastError();
+}
+
+extern "C" int hdla_rows_gemm(int32_t M, int32_t N, int32_t K, const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, int64_t ldy,
+                              void* stream) {
+    if (M < 0 || M > 64 || N < 1 || K < 32 || K % 32) return HDLA_ERR_SHAPE;
+    if (M == 0) return HDLA_OK;
+    if (ldx < K || ldw < K || ldy < N) return HDLA_ERR_SHAPE;
+    if (!x || !w || !y) return HDLA_ERR_NULL;
+    if (!lr_al(x, 16) || !lr_al(w, 16) || !lr_al(y, 8) || ldx % 8 || ldw % 8 || ldy % 4) return HDLA_ERR_ALIGN;
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    const bf16 *xp = static_cast<const bf16*>(x), *wp = static_cast<const bf16*>(w);
+    bf16* yp = static_cast<bf16*>(y);
+    const dim3 grid((N + 15) / 16), block(256);
+    if (M <= 16) hipLaunchKernelGGL(rows_gemm_kernel<1>, grid, block, 0, s, xp, (long long)ldx, wp, (long long)ldw, yp, (long long)ldy, M, N, K);
+    else if (M <= 32) hipLaunchKernelGGL(rows_gemm_kernel<2>, grid, block, 0, s, xp, (long long)ldx, wp, (long long)ldw, yp, (long long)ldy, M, N, K);
+    else hipLaunchKernelGGL(rows_gemm_kernel<4>, grid, block, 0, s, xp, (long long)ldx, wp, (long long)ldw, yp, (long long)ldy, M, N, K);
+    return (int)hipGetLastError();
+}

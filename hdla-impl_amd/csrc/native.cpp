@@ -39,8 +39,8 @@ struct Api {
 #define HDLA_FN(name) decltype(&hdla_##name) name
     HDLA_FN(strerror); HDLA_FN(workspace_bytes); HDLA_FN(boundary_bytes); HDLA_FN(chunk_fwd_b); HDLA_FN(chunk_bwd_b);
     HDLA_FN(recurrent_fwd); HDLA_FN(param_recurrent_fwd); HDLA_FN(normalize_fwd); HDLA_FN(normalize_bwd);
-    HDLA_FN(normalize_workspace_bytes); HDLA_FN(layer_pre_fwd); HDLA_FN(layer_pre_bwd); HDLA_FN(logsigmoid_fwd); HDLA_FN(logsigmoid_bwd);
-    HDLA_FN(skinny_wgrad); HDLA_FN(skinny_wgrad_workspace_bytes); HDLA_FN(sum_partials);
+    HDLA_FN(normalize_workspace_bytes); HDLA_FN(layer_pre_fwd); HDLA_FN(layer_pre_bwd); HDLA_FN(layer_up_fwd); HDLA_FN(layer_down);
+    HDLA_FN(layer_up_wgrad); HDLA_FN(layer_up_wgrad_workspace_bytes); HDLA_FN(rows_gemm); HDLA_FN(sum_partials);
 #undef HDLA_FN
 } api;
 PyObject* error_class = nullptr;                 // _lib.HdlaError
@@ -507,41 +507,57 @@ hdla_pre_dims pre_dims(const LayerCols& L, const LayerCfg& f, int64_t rows) {
     p.zero_from = (int32_t)L.used;
     return p;
 }
+hdla_up_dims up_dims(const LayerCols& L, int64_t rows) {
+    hdla_up_dims u{};
+    u.rows = rows; u.d = (int32_t)L.d; u.D = (int32_t)L.D; u.ld = L.ld; u.col_f = (int32_t)L.f0; u.col_g = (int32_t)L.g0;
+    return u;
+}
+// x w^T.  For the few rows of a decode step by hdla_rows_gemm, which is a launch where the BLAS call is 19 us of host time
+// (measured, us, here / there: 16 x 1024 x 1024 4.5/19, 16 x 6416 x 2048 12/19, 16 x 4096 x 4096 12/19, 64 x 2048 x 2048 13/19;
+// beyond the products below the GPU's own time decides, and the BLAS kernels' larger tiles with it: 1 x 12576 x 4096 35/26).
+Tensor project(const Tensor& x, const Tensor& w) {
+    const int64_t M = x.size(0), tiles = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+    if (M > 64 || tiles * w.numel() > (int64_t(32) << 20)) return at::mm(x, w.t());
+    const Tensor y = at::empty({x.size(0), w.size(0)}, x.options());
+    check(api.rows_gemm((int32_t)x.size(0), (int32_t)w.size(0), (int32_t)w.size(1), ptr(x), x.stride(0), ptr(w), w.stride(0), ptr(y), y.stride(0),
+                        stream_of(x)), "hdla_rows_gemm");
+    return y;
+}
 // everything between x and the output; what the backward pass needs of it
 struct LayerFwd { Tensor x, w, y, f, g, o, n, out, ht, boundary; ChunkIn op; };
 
-// params: wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo; `w` gathered or undefined
-void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, const Tensor& h0, bool want_ht, bool chunked, bool want_boundary,
-                   LayerFwd& r) {
+// params: wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo; r.w gathered; keep: a backward pass follows
+void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, const Tensor& h0, bool want_ht, bool chunked, bool keep, LayerFwd& r) {
     const int64_t B = x3.size(0), T = x3.size(1), d = x3.size(2), rows = B * T;
     const LayerCols L(d, f.H, r.w.size(0) != LayerCols(d, f.H, false).ld);
     const auto opt = x3.options();
     r.x = x3.contiguous().view({rows, d});
-    r.y = at::mm(r.x, r.w.t());
+    r.y = project(r.x, r.w);
     const hdla_pre_dims pd = pre_dims(L, f, rows);
     ChunkIn& in = r.op;
     in.q = at::empty({B, T, L.H, L.D}, opt); in.k = at::empty({B, T, L.H, L.D}, opt); in.v = at::empty({B, T, L.H, L.D}, opt);
     in.beta = at::empty({B, T, L.H, 1}, opt);
     void* const s = stream_of(x3);
     check(api.layer_pre_fwd(&pd, ptr(r.y), ptr(in.q), ptr(in.k), ptr(in.v), ptr(in.beta), s), "hdla_layer_pre_fwd");
-    r.f = at::mm(r.y.narrow(1, L.f0, L.D), P[6].t());
+    const hdla_up_dims ud = up_dims(L, rows);
+    if (keep) r.f = at::empty({rows, d}, opt);
     in.gk = at::empty({B, T, L.H, L.D}, opt);
-    check(api.logsigmoid_fwd(HDLA_BF16, r.f.numel(), ptr(r.f), ptr(in.gk), s), "hdla_logsigmoid_fwd");
+    r.g = at::empty({rows, d}, opt);
+    check(api.layer_up_fwd(&ud, ptr(r.y), ptr(P[6]), ptr(P[7]), ptr(r.f), ptr(in.gk), ptr(r.g), s), "hdla_layer_up_fwd");
     if (h0.defined()) in.h0 = h0.to(at::kFloat).contiguous();
     hdla_dims cd;
     chunk_dims(in, 1.0, cd);
     if (chunked) {
-        chunk_forward(in, cd, want_ht, want_boundary, r.o, r.ht, r.boundary);
+        chunk_forward(in, cd, want_ht, keep && keep_boundaries_default(), r.o, r.ht, r.boundary);
     } else {
         r.o = at::empty_like(in.v);
         if (want_ht) r.ht = at::empty({cd.N, cd.H, cd.K, cd.V}, opt.dtype(at::kFloat));
         check(api.param_recurrent_fwd(&cd, ptr(in.q), ptr(in.k), ptr(in.v), ptr(in.beta), ptr(in.gk), 0, fptr(in.h0), ptr(r.o), fptr(r.ht), s),
               "hdla_param_recurrent_fwd");
     }
-    r.g = at::mm(r.y.narrow(1, L.g0, L.D), P[7].t());
     const Tensor o2 = r.o.view({rows, d});
     r.n = norm_forward(o2, P[8], r.g, norm_dims(o2, P[8], f.gate_pos, f.c, f.eps, f.groups));
-    r.out = at::mm(r.n, P[9].t()).view({B, T, d});
+    r.out = project(r.n, P[9]).view({B, T, d});
 }
 
 // dW [n, k] = dY [rows, n]^T X [rows, k].  An output of few tiles would leave most of the chip idle (1024 x 1024 over 8192
@@ -557,16 +573,6 @@ Tensor weight_grad(const Tensor& dy, const Tensor& x) {
     check(api.sum_partials(fptr(part), (int32_t)S, n * k, ptr(dw), stream_of(dy)), "hdla_sum_partials");
     return dw;
 }
-// the same for the low-rank projections (hdla_skinny_wgrad)
-Tensor skinny_grad(const Tensor& dy, const Tensor& x0) {
-    const int64_t rows = dy.size(0), K = dy.size(1), N = x0.size(1);
-    const size_t nws = api.skinny_wgrad_workspace_bytes(HDLA_BF16, rows, (int32_t)N, (int32_t)K);
-    const Tensor ws = bytes_like(dy, nws), dw = at::empty({K, N}, dy.options());
-    check(api.skinny_wgrad(HDLA_BF16, rows, (int32_t)N, (int32_t)K, ptr(dy), dy.stride(0), ptr(x0), x0.stride(0), ptr(dw), ptr(ws), nws,
-                           stream_of(dy)), "hdla_skinny_wgrad");
-    return dw;
-}
-
 struct LayerFn : torch::autograd::Function<LayerFn> {
     static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& wq, const Tensor& wk, const Tensor& wv, const Tensor& wf0,
                                  const Tensor& wg0, const Tensor& wbeta, const Tensor& wf1, const Tensor& wg1, const Tensor& wnorm,
@@ -574,7 +580,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
         const Tensor P[10] = {wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo};
         LayerFwd r;
         r.w = gather_weights(P, LayerCols(x.size(2), f.H, x.size(0) * x.size(1) >= PAD_FROM_ROWS));
-        layer_forward(x, P, f, value(h0), want_ht, true, keep_boundaries_default(), r);
+        layer_forward(x, P, f, value(h0), want_ht, true, true, r);
         ctx->save_for_backward({r.x, r.w, r.y, r.f, r.g, r.o, r.n, r.boundary, r.op.q, r.op.k, r.op.v, r.op.beta, r.op.gk, value(h0), wf1, wg1,
                                 wnorm, wo});
         ctx->saved_data["c"] = std::vector<double>{f.beta_scale, f.c, f.eps};
@@ -636,13 +642,16 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
         const Tensor dy = at::empty_like(y);
         const hdla_pre_dims pd = pre_dims(L, cfg, rows);
         check(api.layer_pre_bwd(&pd, ptr(y), ptr(dq), ptr(dk), ptr(dv), ptr(dbeta), ptr(dy), stream), "hdla_layer_pre_bwd");
-        const Tensor df = at::empty_like(f);
-        check(api.logsigmoid_bwd(HDLA_BF16, f.numel(), ptr(f), ptr(dgk), ptr(df), stream), "hdla_logsigmoid_bwd");
-        Tensor df0 = dy.narrow(1, L.f0, L.D), dg0 = dy.narrow(1, L.g0, L.D);
-        at::mm_out(df0, df, wf1);
-        at::mm_out(dg0, dgate, wg1);
-        if (need(7)) out[7] = skinny_grad(df, y.narrow(1, L.f0, L.D));
-        if (need(8)) out[8] = skinny_grad(dgate, y.narrow(1, L.g0, L.D));
+        const hdla_up_dims ud = up_dims(L, rows);
+        check(api.layer_down(&ud, ptr(wf1), ptr(wg1), ptr(f), ptr(dgk), ptr(dgate), ptr(dy), stream), "hdla_layer_down");
+        if (need(7) || need(8)) {
+            out[7] = at::empty_like(wf1);
+            out[8] = at::empty_like(wg1);
+            const size_t nws = api.layer_up_wgrad_workspace_bytes(&ud);
+            const Tensor ws = bytes_like(x, nws);
+            check(api.layer_up_wgrad(&ud, ptr(y), ptr(f), ptr(dgk), ptr(dgate), ptr(out[7]), ptr(out[8]), ptr(ws), nws, stream),
+                  "hdla_layer_up_wgrad");
+        }
 
         // the projections of x
         if (need(1) || need(2) || need(3) || need(4) || need(5) || need(6)) {
@@ -673,7 +682,7 @@ PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     bool want = false;
     if (!number(a[10], f.beta_scale) || !number(a[11], f.c) || !number(a[12], f.eps) || !truth(a[3], want) || PyErr_Occurred()) { PyErr_Clear(); return none(); }
     const int64_t B = x.size(0), T = x.size(1), d = x.size(2);
-    if (f.H < 1 || d % f.H || d % 64 || f.groups < 1 || d % f.groups || B * T > INT32_MAX / 4) return none();
+    if (f.H < 1 || d % f.H || d % 128 || f.groups < 1 || d % f.groups || B * T > INT32_MAX / 4) return none();
     const int64_t D = d / f.H;
     if (D != 64 && D != 128) return none();
     const int64_t shapes[10][2] = {{d, d}, {d, d}, {d, d}, {D, d}, {D, d}, {f.H, d}, {d, D}, {d, D}, {d, 0}, {d, d}};
@@ -746,8 +755,8 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     HDLA_FN(strerror) HDLA_FN(workspace_bytes) HDLA_FN(boundary_bytes) HDLA_FN(chunk_fwd_b) HDLA_FN(chunk_bwd_b)
     HDLA_FN(recurrent_fwd) HDLA_FN(param_recurrent_fwd) HDLA_FN(normalize_fwd) HDLA_FN(normalize_bwd)
-    HDLA_FN(normalize_workspace_bytes) HDLA_FN(layer_pre_fwd) HDLA_FN(layer_pre_bwd) HDLA_FN(logsigmoid_fwd) HDLA_FN(logsigmoid_bwd)
-    HDLA_FN(skinny_wgrad) HDLA_FN(skinny_wgrad_workspace_bytes) HDLA_FN(sum_partials)
+    HDLA_FN(normalize_workspace_bytes) HDLA_FN(layer_pre_fwd) HDLA_FN(layer_pre_bwd) HDLA_FN(layer_up_fwd) HDLA_FN(layer_down)
+    HDLA_FN(layer_up_wgrad) HDLA_FN(layer_up_wgrad_workspace_bytes) HDLA_FN(rows_gemm) HDLA_FN(sum_partials)
 #undef HDLA_FN
     Py_INCREF(a[1]);
     Py_XDECREF(error_class);

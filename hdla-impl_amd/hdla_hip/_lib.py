@@ -47,6 +47,12 @@ class HdlaPreDims(ctypes.Structure):
         ("beta_scale", ctypes.c_float), ("eps", ctypes.c_float), ("zero_from", ctypes.c_int32)]
 
 
+class HdlaUpDims(ctypes.Structure):
+    """struct hdla_up_dims of include/hdla_hip.h."""
+    _fields_ = [("rows", ctypes.c_int64), ("d", ctypes.c_int32), ("D", ctypes.c_int32), ("ld", ctypes.c_int64),
+                ("col_f", ctypes.c_int32), ("col_g", ctypes.c_int32)]
+
+
 class HdlaError(RuntimeError):
     pass
 
@@ -127,6 +133,19 @@ def load():
                                       ctypes.c_int64, P, P, ctypes.c_size_t, P]
     lib.hdla_skinny_wgrad_workspace_bytes.restype = ctypes.c_size_t
     lib.hdla_skinny_wgrad_workspace_bytes.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int32, ctypes.c_int32]
+    UF = ctypes.POINTER(HdlaUpDims)
+    lib.hdla_layer_up_fwd.restype = ctypes.c_int
+    lib.hdla_layer_up_fwd.argtypes = [UF] + [P] * 7
+    lib.hdla_layer_down.restype = ctypes.c_int
+    lib.hdla_layer_down.argtypes = [UF] + [P] * 7
+    lib.hdla_layer_up_wgrad.restype = ctypes.c_int
+    lib.hdla_layer_up_wgrad.argtypes = [UF] + [P] * 7 + [ctypes.c_size_t, P]
+    lib.hdla_layer_up_wgrad_workspace_bytes.restype = ctypes.c_size_t
+    lib.hdla_layer_up_wgrad_workspace_bytes.argtypes = [UF]
+    lib.hdla_rows_gemm.restype = ctypes.c_int
+    lib.hdla_rows_gemm.argtypes = [ctypes.c_int32] * 3 + [P, ctypes.c_int64, P, ctypes.c_int64, P, ctypes.c_int64, P]
+    lib.hdla_sum_partials.restype = ctypes.c_int
+    lib.hdla_sum_partials.argtypes = [P, ctypes.c_int32, ctypes.c_int64, P, P]
     _lib = lib
     return lib
 

@@ -299,6 +299,34 @@ size_t hdla_skinny_wgrad_workspace_bytes(int dtype, int64_t M, int32_t N, int32_
  * both 16-byte aligned: the second half of a product whose contraction was split. */
 int hdla_sum_partials(const float* part, int32_t count, int64_t n, void* out, void* stream);
 
+/* The second halves of the layer's two low-rank projections (f_proj and output_gate, HRDPLR/hdla_custom.py:117-121,151-155)
+ * with log_f = logsigmoid(f) (:219), bf16.  Their inner activations are column ranges col_f .. + D and col_g .. + D of
+ * y [rows, ld] (a projection output); weights [d, D] row-major; D = 64 or 128, d a multiple of 128; ld, col_f, col_g
+ * multiples of 8.  f [rows, d] (NULL where no backward pass follows), log_f and gate [rows, d] are written. */
+typedef struct hdla_up_dims {
+    int64_t rows;
+    int32_t d, D;
+    int64_t ld;
+    int32_t col_f, col_g;
+} hdla_up_dims;
+int hdla_layer_up_fwd(const hdla_up_dims* dims, const void* y, const void* wf, const void* wg, void* f, void* log_f,
+                      void* gate, void* stream);
+/* The gradient of the inner activations, written into the two column ranges of dy [rows, ld] (the others are not
+ * touched): (dlog_f sigmoid(-f)) wf and dgate wg, with dlog_f, dgate [rows, d] and f as the forward pass left it. */
+int hdla_layer_down(const hdla_up_dims* dims, const void* wf, const void* wg, const void* f, const void* dlog_f,
+                    const void* dgate, void* dy, void* stream);
+/* The weight gradients of both, dwf = (dlog_f sigmoid(-f))^T y[:, col_f ..] and dwg = dgate^T y[:, col_g ..], each [d, D]:
+ * hdla_skinny_wgrad for the pair.  workspace: hdla_layer_up_wgrad_workspace_bytes() bytes, 16-byte aligned. */
+int hdla_layer_up_wgrad(const hdla_up_dims* dims, const void* y, const void* f, const void* dlog_f, const void* dgate,
+                        void* dwf, void* dwg, void* workspace, size_t workspace_bytes, void* stream);
+size_t hdla_layer_up_wgrad_workspace_bytes(const hdla_up_dims* dims);
+
+/* y [M, N] = x [M, K] w [N, K]^T in bf16 for M <= 64 rows and K a multiple of 32 (the large projections of a decode step;
+ * nn.Linear without bias).  ldx, ldw: row strides in elements, multiples of 8; ldy: a multiple of 4; x, w 16-byte, y 8-byte
+ * aligned. */
+int hdla_rows_gemm(int32_t M, int32_t N, int32_t K, const void* x, int64_t ldx, const void* w, int64_t ldw, void* y,
+                   int64_t ldy, void* stream);
+
 /* Measurement aid; it has no counterpart in the reference.  One launch of a kernel that reads `n_read` (0..3)
  * buffers and writes `n_write` (0..2) buffers of `bytes` bytes each (a multiple of 16; every pointer 16-byte
  * aligned) and does nothing else.  Supported mixes (reads:writes): 1:0, 0:1, 1:1, 2:1, 3:1, 1:2; others return
