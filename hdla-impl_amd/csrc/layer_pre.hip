@@ -61,7 +61,12 @@ template <> struct PrePiece<float> {
     }
 };
 
-template <typename T> __device__ __forceinline__ float pre_sigmoid(float x) { return 1.f / (1.f + exp_t<T>(-x)); }
+// fp32: the division; bf16 results: the hardware reciprocal (one unit in the last place of fp32, a tenth of the
+// instructions; the exponential before it is as close)
+template <typename T> __device__ __forceinline__ float pre_sigmoid(float x) {
+    const float d = 1.f + exp_t<T>(-x);
+    return sizeof(T) == 2 ? __builtin_amdgcn_rcpf(d) : 1.f / d;
+}
 
 // u = silu(x) in place; returns nothing.  sg[j] keeps sigmoid(x) for the backward pass.
 template <typename T, int N> __device__ __forceinline__ void silu_fwd(float (&x)[N], float (&sg)[N]) {

@@ -38,8 +38,10 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 template <typename T> struct Piece;
 template <> struct Piece<bf16> {
     static constexpr int N = 8;
-    static __device__ __forceinline__ void ld(const void* base, long long elem, float (&f)[8]) {
-        const u32x4 r = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(static_cast<const bf16*>(base) + elem));
+    static __device__ __forceinline__ u32x4 raw(const void* base, long long elem) {
+        return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(static_cast<const bf16*>(base) + elem));
+    }
+    static __device__ __forceinline__ void unpack(u32x4 r, float (&f)[8]) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             f[2 * i] = __uint_as_float(r[i] << 16);
@@ -55,10 +57,12 @@ template <> struct Piece<bf16> {
 };
 template <> struct Piece<float> {
     static constexpr int N = 4;
-    static __device__ __forceinline__ void ld(const void* base, long long elem, float (&f)[4]) {
-        const f32x4 r = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(static_cast<const float*>(base) + elem));
+    static __device__ __forceinline__ u32x4 raw(const void* base, long long elem) {
+        return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(static_cast<const float*>(base) + elem));
+    }
+    static __device__ __forceinline__ void unpack(u32x4 r, float (&f)[4]) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) f[i] = r[i];
+        for (int i = 0; i < 4; ++i) f[i] = __uint_as_float(r[i]);
     }
     static __device__ __forceinline__ void st(void* base, long long elem, const float (&f)[4]) {
         f32x4 r;
@@ -68,13 +72,31 @@ template <> struct Piece<float> {
     }
 };
 
+// N consecutive weights, 16 bytes a load
 template <int N> __device__ __forceinline__ void ld_weight(const void* w, int w_f32, int col, float (&f)[N]) {
+    if (w_f32) {
 #pragma unroll
-    for (int i = 0; i < N; ++i)
-        f[i] = w_f32 ? static_cast<const float*>(w)[col + i] : bf2f(static_cast<const bf16*>(w)[col + i].x);
+        for (int i = 0; i < N; i += 4) {
+            const f32x4 r = *reinterpret_cast<const f32x4*>(static_cast<const float*>(w) + col + i);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) f[i + j] = r[j];
+        }
+    } else {
+        // (fp32 data next to bf16 weights: N = 4, eight bytes)
+#pragma unroll
+        for (int i = 0; i < N; i += 4) {
+            const f32x4 r = to_f32(ld_frag(static_cast<const bf16*>(w) + col + i));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) f[i + j] = r[j];
+        }
+    }
 }
 
-__device__ __forceinline__ float sigmoid_f(float x) { return 1.f / (1.f + __expf(-x)); }
+// fp32: the division; bf16 results: the hardware reciprocal (one unit in the last place of fp32, a tenth of the
+// instructions; the exponential before it is as close)
+template <typename T> __device__ __forceinline__ float sigmoid_t(float x);
+template <> __device__ __forceinline__ float sigmoid_t<float>(float x) { return 1.f / (1.f + __expf(-x)); }
+template <> __device__ __forceinline__ float sigmoid_t<bf16>(float x) { return __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
 
 // Where a lane stands: lane sl of the LPR lanes across one group, group position rw of the 64/LPR groups of a pass;
 // `wave` counts passes' owners (wavefronts, or workgroups when a workgroup shares one long group).
@@ -125,6 +147,25 @@ __global__ __launch_bounds__(256) void normalize_fwd_kernel(NormArgs p) {
     const int E = p.E;
     // the launch makes nwave * rpw a multiple of G: the group index of a lane's slots never changes
     const int g = (int)((L.wave * L.rpw + L.rw) % p.G);
+    // A pass's pieces are requested while the pass before it is worked on (the first one's before the weights): otherwise a
+    // wavefront with two passes waits for HBM twice (8192 x 1024: 18.2 -> 13 us).  The largest rows have no registers for it.
+    constexpr bool AHEAD = NV <= 4;
+    u32x4 rx[NV], rg[NV];
+    auto request = [&](long long sg) __attribute__((always_inline)) {
+        const long long slot = sg * L.rpw + L.rw;
+        const bool live = sg < p.nsg && slot < p.nslot;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int e = (i * L.lpr + L.sl) * N;
+            rx[i] = u32x4{0, 0, 0, 0};
+            rg[i] = u32x4{0, 0, 0, 0};
+            if (live && e < E) {
+                rx[i] = Piece<T>::raw(p.x, slot * E + e);
+                if (p.gate_pos) rg[i] = Piece<T>::raw(p.gate, slot * E + e);
+            }
+        }
+    };
+    if (AHEAD) request(L.wave);
     float w[NV][N];
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -138,24 +179,20 @@ __global__ __launch_bounds__(256) void normalize_fwd_kernel(NormArgs p) {
     for (long long sg = L.wave; sg < p.nsg; sg += L.nwave) {
         const long long slot = sg * L.rpw + L.rw;
         const bool live = slot < p.nslot;
+        if (!AHEAD) request(sg);
         float x[NV][N], gs[NV][N];
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
-            const int e = (i * L.lpr + L.sl) * N;
-            if (live && e < E) {
-                Piece<T>::ld(p.x, slot * E + e, x[i]);
-                if (p.gate_pos) Piece<T>::ld(p.gate, slot * E + e, gs[i]);
-            } else {
-#pragma unroll
-                for (int j = 0; j < N; ++j) { x[i][j] = 0.f; gs[i][j] = 0.f; }
-            }
+            Piece<T>::unpack(rx[i], x[i]);
+            Piece<T>::unpack(rg[i], gs[i]);
         }
+        if (AHEAD) request(sg + L.nwave);
         float ss = 0.f;
 #pragma unroll
         for (int i = 0; i < NV; ++i)
 #pragma unroll
             for (int j = 0; j < N; ++j) {
-                if (p.gate_pos) gs[i][j] = sigmoid_f(gs[i][j]);
+                if (p.gate_pos) gs[i][j] = sigmoid_t<T>(gs[i][j]);
                 if (pre) x[i][j] *= gs[i][j];
                 ss += x[i][j] * x[i][j];
             }
@@ -185,6 +222,25 @@ __global__ __launch_bounds__(256) void normalize_bwd_kernel(NormArgs p) {
     const bool pre = p.gate_pos == 1, post = p.gate_pos == 2, has_w = p.weight != nullptr;
     const int E = p.E;
     const int g = (int)((L.wave * L.rpw + L.rw) % p.G);
+    constexpr bool AHEAD = NV <= 2;                       // see the forward kernel
+    u32x4 rx[NV], rg[NV], rd[NV];
+    auto request = [&](long long sg) __attribute__((always_inline)) {
+        const long long slot = sg * L.rpw + L.rw;
+        const bool live = sg < p.nsg && slot < p.nslot;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int e = (i * L.lpr + L.sl) * N;
+            rx[i] = u32x4{0, 0, 0, 0};
+            rg[i] = u32x4{0, 0, 0, 0};
+            rd[i] = u32x4{0, 0, 0, 0};
+            if (live && e < E) {
+                rx[i] = Piece<T>::raw(p.x, slot * E + e);
+                rd[i] = Piece<T>::raw(p.d_o, slot * E + e);
+                if (p.gate_pos) rg[i] = Piece<T>::raw(p.gate, slot * E + e);
+            }
+        }
+    };
+    if (AHEAD) request(L.wave);
     float w[NV][N], dw[NV][N];
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -200,26 +256,22 @@ __global__ __launch_bounds__(256) void normalize_bwd_kernel(NormArgs p) {
     for (long long sg = L.wave; sg < p.nsg; sg += L.nwave) {
         const long long slot = sg * L.rpw + L.rw;
         const bool live = slot < p.nslot;
+        if (!AHEAD) request(sg);
         float x[NV][N], gs[NV][N], dr[NV][N];
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
-            const int e = (i * L.lpr + L.sl) * N;
-            if (live && e < E) {
-                Piece<T>::ld(p.x, slot * E + e, x[i]);
-                Piece<T>::ld(p.d_o, slot * E + e, dr[i]);
-                if (p.gate_pos) Piece<T>::ld(p.gate, slot * E + e, gs[i]);
-            } else {
-#pragma unroll
-                for (int j = 0; j < N; ++j) { x[i][j] = 0.f; gs[i][j] = 0.f; dr[i][j] = 0.f; }
-            }
+            Piece<T>::unpack(rx[i], x[i]);
+            Piece<T>::unpack(rd[i], dr[i]);
+            Piece<T>::unpack(rg[i], gs[i]);
         }
+        if (AHEAD) request(sg + L.nwave);
         // x: the normalised quantity (gated when the gate comes first); dr: gradient of x / sigma before the weight
         float ss = 0.f, sd = 0.f;
 #pragma unroll
         for (int i = 0; i < NV; ++i)
 #pragma unroll
             for (int j = 0; j < N; ++j) {
-                if (p.gate_pos) gs[i][j] = sigmoid_f(gs[i][j]);
+                if (p.gate_pos) gs[i][j] = sigmoid_t<T>(gs[i][j]);
                 if (pre) x[i][j] *= gs[i][j];
                 dr[i][j] *= p.cn;
                 if (post) dr[i][j] *= gs[i][j];
@@ -310,6 +362,7 @@ __global__ __launch_bounds__(256) void normalize_dw_kernel(const float* __restri
     f32x4 acc = zero4();
     if (col < D) {
         const int g = (int)(col / E), e = (int)(col % E);
+#pragma unroll 8
         for (long long idx = g + (long long)rl * G; idx < nrow; idx += 64LL * G)
             acc += *reinterpret_cast<const f32x4*>(partial + idx * E + e);
     }

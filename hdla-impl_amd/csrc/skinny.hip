@@ -73,7 +73,7 @@ __global__ __launch_bounds__(256) void skinny_wgrad_kernel(WgradArgs p) {
                 f32x4 d = to_f32(x[a]);
                 const f32x4 t = to_f32(f[a]);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) d[i] *= 1.f / (1.f + __expf(t[i]));
+                for (int i = 0; i < 4; ++i) d[i] *= __builtin_amdgcn_rcpf(1.f + __expf(t[i]));
                 x[a] = to_frag<bf16>(d);
             }
         }
