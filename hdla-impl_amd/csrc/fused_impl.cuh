@@ -31,6 +31,8 @@
 #include "hdla_common.cuh"
 #include "fused_shapes.h"
 
+#include <type_traits>
+
 namespace hdla {
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
@@ -101,16 +103,18 @@ __device__ __forceinline__ void signal_add(int* flag) {
     if (lane_id() == 0) __hip_atomic_fetch_add(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// the log-decay of four channels as it sits in memory (element type or fp32), converted and masked only where it is used
+// the log-decay of four channels as it sits in memory (element type or fp32), converted only where it is used
 template <typename T, bool GKF32> struct GkRaw {
     typedef Frag<T> type;
     static __device__ __forceinline__ type load(const char* p) { return ld_frag(reinterpret_cast<const T*>(p)); }
-    static __device__ __forceinline__ f32x4 value(type x, bool ok) { return ok ? to_f32(x) : zero4(); }
+    static __device__ __forceinline__ f32x4 value(type x) { return to_f32(x); }
+    static __device__ __forceinline__ void mask(type& x, bool ok) { x.v = ok ? x.v : zero_frag<T>().v; }
 };
 template <typename T> struct GkRaw<T, true> {
     typedef f32x4 type;
     static __device__ __forceinline__ type load(const char* p) { return *reinterpret_cast<const f32x4*>(p); }
-    static __device__ __forceinline__ f32x4 value(type x, bool ok) { return ok ? x : zero4(); }
+    static __device__ __forceinline__ f32x4 value(type x) { return x; }
+    static __device__ __forceinline__ void mask(type& x, bool ok) { x = ok ? x : zero4(); }
 };
 
 // F(I16) for lane (g, c), like ident_frag() but from the caller's lane coordinates
@@ -159,9 +163,10 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
     int c0, c1;
     seq_chunks(p.st, n, c0, c1);
 
-    // rows of the previous chunk's results, left in the outbox by the consumers, out to global memory (forward pass);
-    // each wave of the pair takes half of the rows
-    auto copy_out = [&](int cid) __attribute__((always_inline)) {
+    // rows [rb, rb + NR) of the previous chunk's results, left in the outbox by the consumers, out to global memory
+    // (forward pass)
+    auto copy_out = [&](int cid, int rb, auto nr) __attribute__((always_inline)) {
+        constexpr int NR = decltype(nr)::value;
         if constexpr (FWD) {
             // the lane's offsets below are formed afresh in every call: hoisted out of the chunk loop they would be held
             // in registers through all of it
@@ -170,11 +175,10 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
             const int64_t tok0 = bos + (int64_t)(cid - c0) * CH;
             const int len = (int)min((int64_t)CH, eos - tok0);
             const int64_t chw = (int64_t)h * p.st.nch + cid;
-            const int rb = half * (CH / 2);
             if (seg == 0) {
                 constexpr int LPR = V * (int)sizeof(T) / 16, RPI = 64 / LPR;
 #pragma unroll
-                for (int r0 = 0; r0 < CH / 2; r0 += RPI) {
+                for (int r0 = 0; r0 < NR; r0 += RPI) {
                     const int r = rb + r0 + l / LPR, e = (l % LPR) * 16;
                     const i32x4 x = *reinterpret_cast<const i32x4*>(slot + L::OBOX + r * L::OROW + e);
                     if (r < len) *reinterpret_cast<i32x4*>(reinterpret_cast<char*>(p.o + ((tok0 + r) * H + h) * V) + e) = x;
@@ -183,14 +187,14 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
                 constexpr int LPO = V * 4 / 16, RPO = 64 / LPO;
                 char* ol = reinterpret_cast<char*>(a.ol + chw * (CH * V));
 #pragma unroll
-                for (int r0 = 0; r0 < CH / 2; r0 += RPO) {
+                for (int r0 = 0; r0 < NR; r0 += RPO) {
                     const int r = rb + r0 + l / LPO, e = (l % LPO) * 16;
                     *reinterpret_cast<i32x4*>(ol + r * (V * 4) + e) = *reinterpret_cast<const i32x4*>(slot + L::OBOX + r * L::OROW + e);
                 }
                 constexpr int LPG = K * (int)sizeof(T) / 16, RPG = 64 / LPG;
                 char* gw = reinterpret_cast<char*>(a.gw + chw * (CH * K));
 #pragma unroll
-                for (int r0 = 0; r0 < CH / 2; r0 += RPG) {
+                for (int r0 = 0; r0 < NR; r0 += RPG) {
                     const int r = rb + r0 + l / LPG, e = (l % LPG) * 16;
                     *reinterpret_cast<i32x4*>(gw + r * (K * (int)sizeof(T)) + e) = *reinterpret_cast<const i32x4*>(slot + L::GBOX + r * L::GROW + e);
                 }
@@ -260,11 +264,9 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
             }
         }
     };
-    auto sel = [](Frag<T> f, bool ok) __attribute__((always_inline)) {
-        Frag<T> r;
-        r.v = ok ? f.v : zero_frag<T>().v;
-        return r;
-    };
+    // rows past the end of a ragged chunk become zeros, in place and only there (a uniform branch: whole chunks pay nothing)
+    auto mask = [](Frag<T>& f, bool ok) __attribute__((always_inline)) { f.v = ok ? f.v : zero_frag<T>().v; };
+    auto mask_gk = [](typename GkRaw<T, GKF32>::type& x, bool ok) __attribute__((always_inline)) { GkRaw<T, GKF32>::mask(x, ok); };
     if (pp < nst) request(pp, true);
 
     int it = 0, prev_cid = -1;
@@ -290,34 +292,30 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
         const Frag<T> ident = ident_of<T>(g, c);
         const bool rowok = c < len;
 
-        // ---- the slot: wait until the consumers have left the chunk it held ---------------------------------------------
-        // (at the top, so that every tile can go to the slot as it is formed instead of being held in registers; the
-        // consumers are through with the slot a step of theirs after this pair's last signal, long before this pair is
-        // back here, unless they are what limits the kernel anyway)
-        if (!wait_ge(f_consumed, VT * it, f_abort)) { if (l == 0) *a.err = FUSED_ABORTED + 1; return; }
-        __builtin_amdgcn_sched_barrier(0);
-        // The rows the consumers left in the outbox for that chunk go out first (the consumers write the outbox again
-        // only after both signals at the end).
-        if (it > 0) copy_out(prev_cid);
-        prev_cid = cid;
-        __builtin_amdgcn_sched_barrier(0);
-        request(t, false);                                // the rest of this chunk's inputs, behind those stores
+        request(t, false);                                // the rest of this chunk's inputs
         __builtin_amdgcn_sched_barrier(0);
         // (ag^T waits in the slot where w will go: w = Tm ag is formed further down, when the inverse is there)
         T* const sWW = reinterpret_cast<T*>(slot + (REV ? SB.W : BF.W));
 
-        // ---- own channel tiles: decays, parts of the score tiles, gated copies (prep.hip, phases A and C) -------------
+        // ---- own channel tiles: decays, parts of the score tiles (prep.hip, phase A) -------------------------------------
+        // Nothing here needs the slot: the consumers are through with the chunk it held by the time the gated copies below
+        // are to go there (waiting for them first left a pair idle for a fifth of its time).
+        f32x4 egi[KH], edn[KH];
         f32x4 aqk = zero4(), aqb[2] = {zero4(), zero4()}, aak[2] = {zero4(), zero4()};
         f32x4 aab[2][2] = {{zero4(), zero4()}, {zero4(), zero4()}};
         f32x4 aqbT[2] = {zero4(), zero4()};
-        float big = 0.f;                                  // see strong_decay()
+        bool strong = false;                              // a channel decays beyond the safe range (uniform over the wave)
         float beta_t = 0.f, s_t = 0.f;
         if (HD) {
+            if (len < CH) {
+#pragma unroll
+                for (int j = 0; j < KH; ++j) { mask_gk(ng[j], rowok); mask_gk(og[j], rowok); mask(nk[j], rowok); mask(ok_[j], rowok); }
+            }
             beta_t = rowok ? ld_elem(&nbeta) : 0.f;
 #pragma unroll
             for (int j = 0; j < KH; ++j) {
-                const f32x4 g4 = GkRaw<T, GKF32>::value(ng[j], rowok), gx = GkRaw<T, GKF32>::value(og[j], rowok);
-                const f32x4 k4 = to_f32(sel(nk[j], rowok)), kx = to_f32(sel(ok_[j], rowok));
+                const f32x4 g4 = GkRaw<T, GKF32>::value(ng[j]), gx = GkRaw<T, GKF32>::value(og[j]);
+                const f32x4 k4 = to_f32(nk[j]), kx = to_f32(ok_[j]);
                 const f32x4 kf = k4 * k4 * exp4<T>(g4) + kx * kx * exp4<T>(gx);
                 s_t += kf[0] + kf[1] + kf[2] + kf[3];
             }
@@ -327,8 +325,8 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
         // the operands of channel tile j as the products take them: as loaded, or (HDLA parameterisation) formed from k,
         // gk, beta and s
         auto operands = [&](int j, f32x4 g4, Frag<T>& rq, Frag<T>& rk, Frag<T> (&ra)[2], Frag<T> (&rb)[2]) __attribute__((always_inline)) {
-            rq = sel(nq[j], rowok);
-            rk = sel(nk[j], rowok);
+            rq = nq[j];
+            rk = nk[j];
             if (HD) {
                 const f32x4 kk = to_f32(rk), f4 = exp4<T>(g4);
                 ra[0] = to_frag<T>(kk * (-beta_t));
@@ -336,39 +334,44 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
                 rb[0] = to_frag<T>(f4 * kk);
                 rb[1] = rk;
             } else {
-                ra[0] = sel(na[0][j], rowok);
-                ra[1] = sel(na[1][j], rowok);
-                rb[0] = sel(nb[0][j], rowok);
-                rb[1] = sel(nb[1][j], rowok);
+                ra[0] = na[0][j];
+                ra[1] = na[1][j];
+                rb[0] = nb[0][j];
+                rb[1] = nb[1][j];
             }
         };
         auto decays = [&](int j, f32x4& gi, f32x4& ge) __attribute__((always_inline)) {
-            const f32x4 g4 = GkRaw<T, GKF32>::value(ng[j], rowok);
+            const f32x4 g4 = GkRaw<T, GKF32>::value(ng[j]);
             gi = scan16_incl(g4);
             ge = gi - g4;
         };
 #pragma unroll
         for (int j = 0; j < KH; ++j) {
-            const f32x4 g4 = GkRaw<T, GKF32>::value(ng[j], rowok);
+            if (len < CH) {
+                mask_gk(ng[j], rowok);
+                mask(nq[j], rowok);
+                mask(nk[j], rowok);
+                if (!HD) { mask(na[0][j], rowok); mask(na[1][j], rowok); mask(nb[0][j], rowok); mask(nb[1][j], rowok); }
+            }
+            const f32x4 g4 = GkRaw<T, GKF32>::value(ng[j]);
             Frag<T> rq, rk, ra[2], rb[2];
             operands(j, g4, rq, rk, ra, rb);
-            const f32x4 gi = scan16_incl(g4), ge = gi - g4;
-            const f32x4 m = bcast16<MID>(gi);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) big = fmaxf(big, fmaxf(fabsf(gi[i] - m[i]), fabsf(ge[i] - m[i])));
+            const TileDecay e(g4, c);
+            strong |= e.strong;
+            egi[j] = e.egi;
+            edn[j] = e.edn;
             // One row-side operand at a time against the three inner-side ones, the scheduler kept from interleaving the
             // groups (each tile still gets its products in the order of the channel tiles): all six split operands
             // at once are more registers than three waves per SIMD leave.
             {
-                const f32x4 ek = exp4<T>(m - gi);
                 Split<T> kh, bh[2];
-                split(to_f32(rk) * ek, kh);
-                split(to_f32(rb[0]) * ek, bh[0]);
-                split(to_f32(rb[1]) * ek, bh[1]);
+                split(to_f32(rk) * e.ek, kh);
+                split(to_f32(rb[0]) * e.ek, bh[0]);
+                split(to_f32(rb[1]) * e.ek, bh[1]);
                 __builtin_amdgcn_sched_barrier(0);
                 {
                     Split<T> qh;
-                    split(to_f32(rq) * exp4<T>(gi - m) * scale, qh);
+                    split(to_f32(rq) * e.eq * scale, qh);
                     if (FWD) aqk = mm3(qh, kh, aqk);
 #pragma unroll
                     for (int s = 0; s < 2; ++s) {
@@ -377,55 +380,20 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);
-                const f32x4 ea = exp4<T>(ge - m);
 #pragma unroll
                 for (int r = 0; r < 2; ++r) {
                     Split<T> ah;
-                    split(to_f32(ra[r]) * ea, ah);
+                    split(to_f32(ra[r]) * e.ea, ah);
                     if (!REV) aak[r] = mm3(ah, kh, aak[r]);
                     aab[r][0] = mm3(ah, bh[0], aab[r][0]);
                     aab[r][1] = mm3(ah, bh[1], aab[r][1]);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
-            pin(rq); pin(rk); pin(ra[0]); pin(ra[1]); pin(rb[0]); pin(rb[1]);
-            const f32x4 q4 = to_f32(rq), k4 = to_f32(rk);
-            const f32x4 a0 = to_f32(ra[0]), a1 = to_f32(ra[1]), b0 = to_f32(rb[0]), b1 = to_f32(rb[1]);
-            // the gated copies, while the operands are at hand: each tile goes to its half of the stored pair
-            // (scheduling barriers: the products above, the copies below and the next tile are kept apart, or their
-            // temporaries would all be live at once)
-            __builtin_amdgcn_sched_barrier(0);
-            const f32x4 gl = bcast16<CH - 1>(gi);
-            const f32x4 egi = exp4<T>(gi), edn = exp4<T>(gl - gi);
-            // e^{ge} of a token is e^{gi} of the token before it (1 for the first), e^{gl} is e^{gi} of the last token:
-            // lane moves in place of two more rounds of exponentials
-            f32x4 ege = dpp0<0x111>(egi);                 // row_shr:1 (lanes of one token group are a DPP row)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) ege[i] = c == 0 ? 1.f : ege[i];
-            const f32x4 egl = bcast16<CH - 1>(egi);
-            st_pair(sWW + (0 * KT2 + half) * PAIR, j, transpose(to_frag<T>(a0 * ege), ident));
-            st_pair(sWW + (1 * KT2 + half) * PAIR, j, transpose(to_frag<T>(a1 * ege), ident));
-            const Frag<T> fqg = to_frag<T>(q4 * egi * scale);
-            const Frag<T> fbg[2] = {to_frag<T>(b0 * edn), to_frag<T>(b1 * edn)};
-            if (!REV) {
-                st_pair(reinterpret_cast<T*>(slot + BF.KGT) + half * PAIR, j, transpose(to_frag<T>(k4 * edn), ident));
-                st_pair(reinterpret_cast<T*>(slot + BF.BGT) + (0 * KT2 + half) * PAIR, j, transpose(fbg[0], ident));
-                st_pair(reinterpret_cast<T*>(slot + BF.BGT) + (1 * KT2 + half) * PAIR, j, transpose(fbg[1], ident));
-                st_pair(reinterpret_cast<T*>(slot + BF.QG) + half * PAIR, j, fqg);
-            } else {
-                // the reverse scan takes bg as it is and w transposed (the stand-alone kernel turns the stored tiles on
-                // their way into LDS: the same values)
-                st_pair(reinterpret_cast<T*>(slot + SB.BGT) + (0 * KT2 + half) * PAIR, j, fbg[0]);
-                st_pair(reinterpret_cast<T*>(slot + SB.BGT) + (1 * KT2 + half) * PAIR, j, fbg[1]);
-                st_pair(reinterpret_cast<T*>(slot + SB.QGT) + half * PAIR, j, transpose(fqg, ident));
-            }
-            if (c == 0) *reinterpret_cast<f32x4*>(slot + (REV ? SB.EGL : BF.EGL) + (16 * (kt0 + j) + 4 * g) * 4) = egl;
-            __builtin_amdgcn_sched_barrier(0);
         }
         // Each wave decides for its own channels (the parts of the score tiles add up whichever way they were formed).
         // Where a channel decays too strongly for the single centre, what was accumulated above may hold infinities: it
         // is thrown away and the parts are formed again by passes whose exponents cannot overflow (see DecayPass).
-        const bool strong = __any(big > SAFE_RANGE) != 0;  // the same answer on every lane of the wave
         if (strong) {
             aqk = zero4();
 #pragma unroll
@@ -467,11 +435,6 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
                 }
             }
         }
-        // the first tile's inputs are used up: the next chunk's may come
-        __builtin_amdgcn_sched_barrier(0);
-        if (t + FNP < nst) request(t + FNP, true);
-        __builtin_amdgcn_sched_barrier(0);
-
         // ---- the other wave's parts travel to the lead ------------------------------------------------------------------
         // tile order in the scratch: A_ab (4), then A_ak (2; the reverse kernel: A_qb^T), A_qb (2), A_qk: as many as the mode forms
         constexpr int NPART = REV ? 6 : FWD ? 9 : 8;    // A_ab, (A_ak), A_qb or its transpose, (A_qk)
@@ -484,18 +447,55 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
             signal_set(f_part, it + 1);
         }
 
+        // ---- the slot: wait until the consumers have left the chunk it held ---------------------------------------------
+        if (!wait_ge(f_consumed, VT * it, f_abort)) { if (l == 0) *a.err = FUSED_ABORTED + 1; return; }
+        __builtin_amdgcn_sched_barrier(0);
+        // ---- gated copies of the own channel tiles (prep.hip, phase C), each to its half of the stored pair --------------
+#pragma unroll
+        for (int j = 0; j < KH; ++j) {
+            pin(nq[j]); pin(nk[j]);                       // converted again, not kept converted from above
+            if (!HD) { pin(na[0][j]); pin(na[1][j]); pin(nb[0][j]); pin(nb[1][j]); }
+            Frag<T> rq, rk, ra[2], rb[2];
+            operands(j, GkRaw<T, GKF32>::value(ng[j]), rq, rk, ra, rb);
+            const f32x4 one = {1.f, 1.f, 1.f, 1.f}, ege = prev_token(egi[j], one), egl = bcast16<CH - 1>(egi[j]);
+            st_pair(sWW + (0 * KT2 + half) * PAIR, j, transpose(to_frag<T>(to_f32(ra[0]) * ege), ident));
+            st_pair(sWW + (1 * KT2 + half) * PAIR, j, transpose(to_frag<T>(to_f32(ra[1]) * ege), ident));
+            const Frag<T> fqg = to_frag<T>(to_f32(rq) * egi[j] * scale);
+            const Frag<T> fbg[2] = {to_frag<T>(to_f32(rb[0]) * edn[j]), to_frag<T>(to_f32(rb[1]) * edn[j])};
+            if (!REV) {
+                st_pair(reinterpret_cast<T*>(slot + BF.KGT) + half * PAIR, j, transpose(to_frag<T>(to_f32(rk) * edn[j]), ident));
+                st_pair(reinterpret_cast<T*>(slot + BF.BGT) + (0 * KT2 + half) * PAIR, j, transpose(fbg[0], ident));
+                st_pair(reinterpret_cast<T*>(slot + BF.BGT) + (1 * KT2 + half) * PAIR, j, transpose(fbg[1], ident));
+                st_pair(reinterpret_cast<T*>(slot + BF.QG) + half * PAIR, j, fqg);
+            } else {
+                // the reverse scan takes bg as it is and w transposed (the stand-alone kernel turns the stored tiles on
+                // their way into LDS: the same values)
+                st_pair(reinterpret_cast<T*>(slot + SB.BGT) + (0 * KT2 + half) * PAIR, j, fbg[0]);
+                st_pair(reinterpret_cast<T*>(slot + SB.BGT) + (1 * KT2 + half) * PAIR, j, fbg[1]);
+                st_pair(reinterpret_cast<T*>(slot + SB.QGT) + half * PAIR, j, transpose(fqg, ident));
+            }
+            if (c == 0) *reinterpret_cast<f32x4*>(slot + (REV ? SB.EGL : BF.EGL) + (16 * (kt0 + j) + 4 * g) * 4) = egl;
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // the inputs are used up: the next chunk's first ones may come
+        if (t + FNP < nst) request(t + FNP, true);
+        __builtin_amdgcn_sched_barrier(0);
+
         Frag<T> vT[VH];
         if (!REV) {
 #pragma unroll
             for (int j = 0; j < VH; ++j) {
-                vT[j] = transpose(sel(nv[j], rowok), ident);
+                if (len < CH) mask(nv[j], rowok);
+                vT[j] = transpose(nv[j], ident);
                 st_frag(reinterpret_cast<T*>(slot + L::VTT) + (vt0 + j) * TILE + 4 * l, vT[j]);
             }
         }
         if (REV || CKPT) {
-            // rows past the end of a ragged chunk were taken as zeros
 #pragma unroll
-            for (int j = 0; j < VH; ++j) st_frag(reinterpret_cast<T*>(slot + L::DOT) + (vt0 + j) * TILE + 4 * l, transpose(sel(ndo[j], rowok), ident));
+            for (int j = 0; j < VH; ++j) {
+                if (len < CH) mask(ndo[j], rowok);
+                st_frag(reinterpret_cast<T*>(slot + L::DOT) + (vt0 + j) * TILE + 4 * l, transpose(ndo[j], ident));
+            }
         }
 
         // ---- the lead: whole score tiles, (I - A_ab)^-1 by forward substitution (prep.hip, phase B) ---------------------
@@ -611,6 +611,9 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
             }
             signal_set(f_inv, it + 1);
         } else {
+            // while the lead solves: the rows the consumers left in the outbox for the chunk the slot held (they write the
+            // outbox again only after both signals at the end)
+            if (it > 0) copy_out(prev_cid, 0, std::integral_constant<int, CH>());
             if (!wait_ge(f_inv, it + 1, f_abort)) { if (l == 0) *a.err = FUSED_ABORTED + 1; return; }
 #pragma unroll
             for (int s = 0; s < 2; ++s) ld_pair(sPub + s * PAIR, tm[s][0], tm[s][1]);
@@ -651,11 +654,12 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
             }
         }
         signal_add(f_ready);
+        prev_cid = cid;
     }
-    // the last chunk's rows
+    // the last chunk's rows, half by each wave
     if (FWD && it > 0) {
         if (!wait_ge(f_consumed, VT * it, f_abort)) { if (l == 0) *a.err = FUSED_ABORTED + 1; return; }
-        copy_out(prev_cid);
+        copy_out(prev_cid, half * (CH / 2), std::integral_constant<int, CH / 2>());
     }
 }
 
