@@ -74,16 +74,17 @@ def interface_bytes(kernel, pass_, K, V, es, gs, frac_seg=0.0):
         return inputs + 16 * V * es + TM + HC + DHC + DVN + outs
     # fused route: the scans' operands stay in LDS.  frac_seg = share of the chunks that lie in segments > 0 (their local
     # output rows, fp32, and the 16 x K block G go through the workspace to the kernel that chains the segments)
+    # (each kernel of the backward pass reads what it needs of the record the forward kernel leaves: TM, A_ak, A_qb, G)
     if kernel == "fused_fwd":
-        return inputs + (1 - frac_seg) * 16 * V * es + frac_seg * (16 * V * 4 + 16 * K * es)
+        return inputs + (1 - frac_seg) * 16 * V * es + frac_seg * (16 * V * 4 + 16 * K * es) + 2 * TM
     if kernel == "fixup":
         return frac_seg * (16 * V * 4 + 16 * K * es + 16 * V * es)
     if kernel == "fused_ckpt":
-        return inputs + 16 * V * es + HC + TM
+        return inputs - 16 * K * es + 16 * V * es + TM + 512 * es + frac_seg * 16 * K * es + HC
     if kernel == "fused_sum":
         return inputs
     if kernel == "fused_rev":
-        return inputs - 16 * V * es + 16 * V * es + DHC + DVN          # q, k, gk, a, b and do in; dS checkpoint and dv_new out
+        return inputs - 16 * K * es - 16 * V * es + 16 * V * es + TM + AQB + DHC + DVN   # q, gk, a, b and do in; dS checkpoint and dv_new out
     raise ValueError(kernel)
 
 
@@ -774,9 +775,9 @@ def run_chunk_workload(wl, cfg, steps, warmup, dev, keep_variant=True):
 
     sec = time_steps(step, steps, warmup)
     # the same step on the other routes the library has for this shape (reported beside `value`, never as it): strictly
-    # the inputs kept between the passes (the fused route's default hands the states at the time-segment boundaries, 64 KiB
-    # per sequence, head and segment, from the forward to the backward pass; without them the backward pass re-derives
-    # them with one more pass over the inputs), and the classic launch plan (separate prep and scan kernels)
+    # the inputs kept between the passes (the fused route's default hands the forward pass's record, 37 % of the inputs'
+    # bytes, to the backward pass; without it the backward pass re-derives it with one more pass over the inputs), and the
+    # classic launch plan (separate prep and scan kernels)
     variants = {}
     if keep_variant:
         from hdla_hip import _lib as _l

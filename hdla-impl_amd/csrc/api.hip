@@ -93,6 +93,7 @@ int scan_segments(const hdla_dims* d, bool bwd) {
 struct FusedLayout {
     size_t OL, GW, SLOC, MSEG, RSEG, SIN, ERR;                 // fused kernels' own
     size_t HC, DHC, DVN, TM, UT, W, STRONG;                    // what chunk_grad reads (backward pass)
+    size_t MT, AQ;                                             // and the rest of the record
     size_t CHUNK_OFF, CHUNK_SEQ;
     size_t total;
     int nch, nseg;
@@ -120,6 +121,9 @@ int make_fused_layout(const hdla_dims* d, int pass, FusedLayout& L) {
     } else {
         L.RSEG = take(recs * K * V * 4);
         L.SIN = take(recs * K * V * 4);
+        L.MT = take(recs * K * K * 4);
+        L.GW = L.nseg > 1 ? take(chw * 16 * K * es) : 0;
+        L.AQ = take(chw * 1024 * es);
         L.HC = take(chw * K * V * es);
         L.DHC = take(chw * K * V * es);
         L.DVN = take(chw * 2 * 16 * V * es);
@@ -138,6 +142,22 @@ int make_fused_layout(const hdla_dims* d, int pass, FusedLayout& L) {
 size_t fused_boundary_bytes(const hdla_dims* d) {
     const int nseg = fused_segments(d);
     return nseg > 1 ? (size_t)d->N * d->H * nseg * d->K * d->V * 4 : 0;
+}
+// The record a forward pass hands to the backward pass: the boundary states (first, so that a record is a boundary), the
+// segments' transitions, and per (chunk, head) what the score tiles come to (fused_impl.cuh).
+struct FusedRecord { size_t SIN, MT, GW, TM, AQ, STRONG, total; };
+FusedRecord fused_record(const hdla_dims* d, const FusedLayout& L) {
+    FusedRecord r{};
+    size_t off = 0;
+    auto take = [&](size_t bytes) { const size_t o = off; off += up256(bytes); return o; };
+    const size_t chw = (size_t)d->H * (size_t)L.nch, recs = (size_t)d->N * d->H * L.nseg;
+    r.SIN = take(fused_boundary_bytes(d));
+    if (L.nseg > 1) { r.MT = take(recs * d->K * d->K * 4); r.GW = take(chw * 16 * d->K * 2); }
+    r.TM = take(chw * 1024 * 2);
+    r.AQ = take(chw * 1024 * 2);
+    r.STRONG = take(chw * 4);
+    r.total = off;
+    return r;
 }
 
 // pass: HDLA_PASS_FWD, _BWD, _FWD_KEEP (a forward pass that leaves what the backward pass needs of it), _BWD_KEPT (the
@@ -313,9 +333,10 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
     return HDLA_OK;
 }
 
-// The fused route's launch sequences.  Forward: fused kernel (+ fixup kernel when there are several segments); it
-// leaves the states entering the segments in `boundary` when given.  Backward: (without `boundary`: summary pass +
-// chaining, to re-derive those states) checkpoint kernel, reverse kernel, chunk_grad.
+// The fused route's launch sequences.  Forward: fused kernel (+ fixup kernel when there are several segments).  When
+// `boundary` is given it leaves the states entering the segments there, or, if there is room for it, the whole record.
+// Backward: (without a record: summary pass, which writes one to the workspace; without the states: chaining) checkpoint
+// kernel, reverse kernel, chunk_grad.
 int run_fused(const hdla_dims* d, bool fwd, const void* q, const void* k, const void* v, const void* a_, const void* b,
               const void* beta, const void* gk, const float* h0, void* o, float* ht, const void* d_o, const float* dht,
               void* dq, void* dk, void* dv, void* da, void* db, void* dbeta, void* dgk, float* dh0, void* boundary,
@@ -328,6 +349,9 @@ int run_fused(const hdla_dims* d, bool fwd, const void* q, const void* k, const 
     if (bad_ws(workspace, workspace_bytes, L.total)) return HDLA_ERR_WORKSPACE;
     if (boundary && (L.nseg > 1) && (boundary_bytes < fused_boundary_bytes(d) || (reinterpret_cast<uintptr_t>(boundary) & 15)))
         return HDLA_ERR_WORKSPACE;
+    const FusedRecord R = fused_record(d, L);
+    char* const rec = boundary && boundary_bytes >= R.total ? static_cast<char*>(boundary) : nullptr;
+    if (rec && (reinterpret_cast<uintptr_t>(rec) & 15)) return HDLA_ERR_WORKSPACE;
     char* base = static_cast<char*>(workspace);
     FusedArgs<T> f{};
     ChunkArgs<T>& a = f.c;
@@ -341,9 +365,18 @@ int run_fused(const hdla_dims* d, bool fwd, const void* q, const void* k, const 
     a.da = static_cast<T*>(da); a.db = static_cast<T*>(db); a.dgk = dgk;
     a.beta = static_cast<const T*>(beta); a.dbeta = static_cast<T*>(dbeta);
     a.ws.HC = reinterpret_cast<T*>(base + L.HC); a.ws.DHC = reinterpret_cast<T*>(base + L.DHC);
-    a.ws.DVN = reinterpret_cast<T*>(base + L.DVN); a.ws.TM = reinterpret_cast<T*>(base + L.TM);
+    a.ws.DVN = reinterpret_cast<T*>(base + L.DVN);
     a.ws.UT = reinterpret_cast<T*>(base + L.UT); a.ws.W = reinterpret_cast<T*>(base + L.W);
-    a.ws.STRONG = reinterpret_cast<int32_t*>(base + L.STRONG);
+    f.gw = reinterpret_cast<T*>(base + L.GW);
+    if (rec) {
+        a.ws.TM = reinterpret_cast<T*>(rec + R.TM); a.ws.STRONG = reinterpret_cast<int32_t*>(rec + R.STRONG);
+        f.aq = reinterpret_cast<T*>(rec + R.AQ);
+        if (L.nseg > 1) { f.mt = reinterpret_cast<float*>(rec + R.MT); f.gw = reinterpret_cast<T*>(rec + R.GW); }
+    } else if (!fwd) {
+        a.ws.TM = reinterpret_cast<T*>(base + L.TM); a.ws.STRONG = reinterpret_cast<int32_t*>(base + L.STRONG);
+        f.aq = reinterpret_cast<T*>(base + L.AQ);
+        f.mt = reinterpret_cast<float*>(base + L.MT);
+    }
     a.ws.sa_stride = 2 * d->K * 16 * 2;                            // chunk_grad's view of w: [2][K/16] tiles per slot
     a.st.cu = d->cu_seqlens;
     a.st.chunk_off = d->cu_seqlens ? reinterpret_cast<const int32_t*>(base + L.CHUNK_OFF) : nullptr;
@@ -361,7 +394,7 @@ int run_fused(const hdla_dims* d, bool fwd, const void* q, const void* k, const 
         if (e != hipSuccess) return (int)e;
     }
     if (fwd) {
-        f.ol = reinterpret_cast<float*>(base + L.OL); f.gw = reinterpret_cast<T*>(base + L.GW);
+        f.ol = reinterpret_cast<float*>(base + L.OL);
         f.sin_out = static_cast<float*>(boundary);
         if (stages & HDLA_STAGE_SCAN_FWD) {
             e = launch_fused<T>(f, d->K, d->V, FUSED_FWD, stream);
@@ -373,20 +406,21 @@ int run_fused(const hdla_dims* d, bool fwd, const void* q, const void* k, const 
         }
         return HDLA_OK;
     }
+    f.sin = static_cast<const float*>(boundary);
+    // no record: one pass over the inputs for it, and its segments chained into the states that enter them (a caller that
+    // runs the stages one by one may leave this one out once the workspace holds them; one segment has no stage of its own
+    // for it)
+    if (!rec && (stages & (L.nseg > 1 ? HDLA_STAGE_CHAIN : HDLA_STAGE_SCAN_FWD))) {
+        e = launch_fused<T>(f, d->K, d->V, FUSED_SUM, stream);
+        if (e != hipSuccess) return (int)e;
+    }
     if (L.nseg > 1 && !boundary) {
-        // inputs only: one pass for the segment records, chained into the states entering the segments (a caller that
-        // runs the stages one by one may leave this one out once the workspace holds them)
         f.sin_out = reinterpret_cast<float*>(base + L.SIN);
-        f.gw = nullptr;
         if (stages & HDLA_STAGE_CHAIN) {
-            e = launch_fused<T>(f, d->K, d->V, FUSED_SUM, stream);
-            if (e != hipSuccess) return (int)e;
             e = launch_fixup<T>(f, d->K, d->V, stream);
             if (e != hipSuccess) return (int)e;
         }
         f.sin = f.sin_out;
-    } else {
-        f.sin = static_cast<const float*>(boundary);
     }
     if (stages & HDLA_STAGE_SCAN_FWD) {
         e = launch_fused<T>(f, d->K, d->V, FUSED_CKPT, stream);
@@ -468,6 +502,13 @@ size_t hdla_boundary_bytes(const hdla_dims* dims) {
     bool fused;
     if (check_dims(dims) || pick_route(dims, fused) || !fused) return 0;
     return fused_boundary_bytes(dims);
+}
+
+size_t hdla_record_bytes(const hdla_dims* dims) {
+    bool fused;
+    FusedLayout L;
+    if (check_dims(dims) || pick_route(dims, fused) || !fused || make_fused_layout(dims, HDLA_PASS_BWD, L)) return 0;
+    return fused_record(dims, L).total;
 }
 
 int hdla_workspace_layout(const hdla_dims* dims, int pass, hdla_ws_layout* out) {

@@ -26,8 +26,6 @@ namespace hdla {
 
 constexpr int NW = 4;     // wavefronts per (chunk, head)
 
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-
 // LDS of a workgroup (byte offsets)
 template <typename T, int K, int V> struct CgLds {
     static constexpr int ES = sizeof(T);

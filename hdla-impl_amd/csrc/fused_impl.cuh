@@ -21,6 +21,14 @@
 //                   segment from the right, d S_in(s) = M_s^T d S_in(s+1) + R_s, which the reverse kernel's consumers
 //                   chain themselves before they start.
 //
+// What the backward pass's two kernels take over from the forward pass (or from the summary pass, which is the forward
+// kernel without its outputs): the record.  Per (chunk, head), 2-byte elements: (I - A_ab)^-1, A_ak, A_qb (8 tiles of
+// 16 x 16) and in segments > 0 G (16 x K); per segment M.  That is 6 KB beside the 16 KB of a chunk's inputs at K = V = 64,
+// and it is all that takes a producer pair its time: the score products and the triangular solve were three quarters of
+// each of the two kernels.  With the record a producer only forms the gated copies, w and
+// u (fused_replay), and nothing of M is computed twice.  Measured (4 x 2048 tokens, 16 heads, K = V = 64):
+// checkpoint kernel 76 -> 57 us, reverse kernel 69 -> 54 us (with the loads of rows_to_tiles), the forward kernel pays 2 us.
+//
 // Synchronisation.  Producers and consumers run at their own pace; a slot is handed over through two counters in LDS
 // that only ever grow: ready[p] (+1 per wave of pair p and chunk completed) and consumed[p] (consumer-steps finished on
 // slot p); the waves of a pair hand each other the parts and the inverse the same way (part[p], inv[p]).
@@ -34,8 +42,6 @@
 #include <type_traits>
 
 namespace hdla {
-
-typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int FNP = 4;                    // producer pairs = LDS slots
 constexpr int FLDP = 36;                  // padded row length of the 32 x 32 matrices of the triangular solve
@@ -52,31 +58,34 @@ __device__ __forceinline__ void seg_range(const SeqTab& st, int n, int nseg, int
     seg_range(c0, c1, nseg, seg, s0, s1);
 }
 
-// LDS of a fused workgroup (byte offsets): per producer one slot = [operands | outbox | solver scratch], then the flags
+// LDS of a fused workgroup (byte offsets): per producer pair one slot = [operands | outbox | solver scratch], then the flags
 template <typename T, int K, int V, int MODE> struct FusedLds {
     static constexpr int ES = sizeof(T), TB = TILE * ES, KT = K / 16, VT = V / 16;
-    static constexpr bool REV = MODE == FUSED_REV;
-    static constexpr BlkF BF = blk_fwd(K, ES, true);
+    static constexpr bool REV = MODE == FUSED_REV, FWD = MODE == FUSED_FWD, SOLVES = FWD || MODE == FUSED_SUM;
+    static constexpr BlkF BF = blk_fwd(K, ES, SOLVES);
     static constexpr SlotB SB = slot_bwd(K, ES);
-    // forward direction: the forward-scan block, then u^T (VT tile pairs), v^T (VT tiles), and in checkpoint mode do^T
-    // (VT tiles) and the inverse for chunk_grad
-    static constexpr int UT = BF.SIZE, VTT = UT + 2 * VT * TB, DOT_F = VTT + VT * TB;
+    // forward direction: the forward-scan block, then u^T (VT tile pairs), v^T (VT tiles); checkpoint kernel: do^T (VT
+    // tiles); where the score tiles are solved: (I - A_ab)^-1 as chunk_grad reads it (2 tile pairs) and A_ak (a tile pair)
+    static constexpr int UT = BF.SIZE, VTT = UT + 2 * VT * TB, FWD_END = VTT + VT * TB;
+    static constexpr int TMB = FWD_END, AKB = TMB + 4 * TB;
     // reverse direction: the reverse-scan slot, then do^T
-    static constexpr int DOT = REV ? SB.SIZE : DOT_F;
-    static constexpr int TMB = DOT_F + VT * TB;          // checkpoint mode: (I - A_ab)^-1 as chunk_grad reads it (2 tile pairs)
-    static constexpr int OPER = REV ? SB.SIZE + VT * TB : (MODE == FUSED_CKPT ? TMB + 4 * TB : DOT_F);
+    static constexpr int DOT = REV ? SB.SIZE : FWD_END;
+    static constexpr int OPER = SOLVES ? AKB + 2 * TB : DOT + VT * TB;
     // outbox of the forward pass: 16 rows of o (fp32 in segments > 0, element type in segment 0) and 16 rows of G
     static constexpr int OROW = V * 4 + 16, GROW = K * ES + 16;
-    static constexpr int OBOX = OPER, GBOX = OBOX + (MODE == FUSED_FWD ? CH * OROW : 0);
-    static constexpr int SOLVE = GBOX + (MODE == FUSED_FWD ? CH * GROW : 0);
-    static constexpr int SLOT = SOLVE + 2 * 32 * FLDP * 4;
+    static constexpr int OBOX = OPER, GBOX = OBOX + (FWD ? CH * OROW : 0);
+    static constexpr int SOLVE = GBOX + (FWD ? CH * GROW : 0);
+    static constexpr int SLOT = SOLVE + (SOLVES ? 2 * 32 * FLDP * 4 : 0);
     // int ready[4], consumed[4], abort, -, -, -, part[4], inv[4], strong[4] (per producer pair; see fused_producer), then
     // two counters of the reverse kernel's consumers (records staged, records used: fused_consumer_rev)
     static constexpr int FLAGS = FNP * SLOT;
     // reverse kernel: transition records of the segments to the right, as split operands, for the consumers' chain
     // (CHAIN_STAGE records of K x K at a time: every consumer wave needs them whole, each loads a quarter)
     static constexpr int CHAIN_STAGE = 2;
-    static constexpr int CHAIN = FLAGS + 128;
+    // scratch of the producers for their loads (rows_to_tiles): one area a wave; where the waves of a pair solve, one a pair
+    // for its lead, the other wave has the second half of the solver scratch, which is free until that wave itself fills it with its parts
+    static constexpr int ROWS = FLAGS + 128, ROWS_B = (SOLVES ? FNP : 2 * FNP) * ROWS_SCRATCH;
+    static constexpr int CHAIN = ROWS + ROWS_B;
     static constexpr int BYTES = CHAIN + (REV ? CHAIN_STAGE * 2 * KT * KT * TB : 0);
 };
 
@@ -103,16 +112,27 @@ __device__ __forceinline__ void signal_add(int* flag) {
     if (lane_id() == 0) __hip_atomic_fetch_add(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// the log-decay of four channels as it sits in memory (element type or fp32), converted only where it is used
+// the log-decays of four channels as they sit in memory (element type or fp32), converted only where they are used, and of
+// the wave's share of a chunk as loaded (a row's 32 channels: 64 bytes as one piece a lane, or 128 bytes as two)
 template <typename T, bool GKF32> struct GkRaw {
     typedef Frag<T> type;
-    static __device__ __forceinline__ type load(const char* p) { return ld_frag(reinterpret_cast<const T*>(p)); }
+    typedef i32x4 rows;
+    static __device__ __forceinline__ void load(const char* p, int l, uint32_t row_ch, rows& x) { x = *reinterpret_cast<const i32x4*>(at(p, 2 * row_ch + 16 * (l & 3))); }
+    static __device__ __forceinline__ void tiles(char* scratch, int l, rows x, type (&f)[2]) { rows_to_tiles(scratch, l, x, f[0], f[1]); }
     static __device__ __forceinline__ f32x4 value(type x) { return to_f32(x); }
     static __device__ __forceinline__ void mask(type& x, bool ok) { x.v = ok ? x.v : zero_frag<T>().v; }
 };
 template <typename T> struct GkRaw<T, true> {
     typedef f32x4 type;
-    static __device__ __forceinline__ type load(const char* p) { return *reinterpret_cast<const f32x4*>(p); }
+    struct rows { f32x4 x[2]; };
+    static __device__ __forceinline__ void load(const char* p, int l, uint32_t row_ch, rows& x) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) x.x[j] = *reinterpret_cast<const f32x4*>(at(p, 4 * row_ch + 64 * j + 16 * (l & 3)));
+    }
+    static __device__ __forceinline__ void tiles(char* scratch, int l, const rows& x, type (&f)[2]) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) f[j] = rows_to_tile(scratch, l, x.x[j]);
+    }
     static __device__ __forceinline__ f32x4 value(type x) { return x; }
     static __device__ __forceinline__ void mask(type& x, bool ok) { x = ok ? x : zero4(); }
 };
@@ -139,10 +159,10 @@ template <typename T, bool GKF32, int K, int V, int MODE, bool HD>
 __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem, int n, int h, int seg, int s0, int s1, int pp, int half) {
     static_assert(K == 64 && sizeof(T) == 2 && V % 32 == 0, "a producer pair holds all channels of a chunk: K = 64, 2-byte elements");
     typedef FusedLds<T, K, V, MODE> L;
-    constexpr bool REV = MODE == FUSED_REV, CKPT = MODE == FUSED_CKPT, FWD = MODE == FUSED_FWD;
+    constexpr bool FWD = MODE == FUSED_FWD;
+    static_assert(L::SOLVES, "the backward pass's kernels read what this producer solves for (fused_replay)");
     constexpr int KT = K / 16, VT = V / 16, KT2 = KT / 2, KH = 2, VH = VT / 2;
     constexpr BlkF BF = L::BF;
-    constexpr SlotB SB = L::SB;
     const ChunkArgs<T>& p = a.c;
     char* slot = smem + pp * L::SLOT;
     // the pair's scratch: first the other wave's parts of the nine score tiles (fp32, 9 KiB); then, in the same bytes,
@@ -202,76 +222,64 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
         }
     };
 
-    // The wave's share of the chunk's inputs as loaded, four elements a lane (lane (g,c): token c, channels 16kt + 4g ..):
-    // requested one chunk of this pair ahead, as soon as the registers are free, so that the round trip to HBM runs
-    // behind the rest of the previous chunk.  Nothing is done to them at the load (a select or a conversion would wait
-    // for the data).  With the HDLA parameterisation the sum over ALL channels of k^2 f is needed: the other half's k and
-    // gk come along.
-    Frag<T> nq[KH], nk[KH], na[2][KH], nb[2][KH], nv[VH], ndo[VH], ok_[KH];
-    typename GkRaw<T, GKF32>::type ng[KH], og[KH];
+    // The wave's share of the chunk's inputs as loaded, 16 bytes a lane (rows_to_tiles): requested one chunk of this pair
+    // ahead, as soon as the registers are free, so that the round trip to HBM runs behind the rest of the previous chunk.
+    // With the HDLA parameterisation the sum over ALL channels of k^2 f is needed: the other half's k and gk come along.
+    // In parts, by what three waves per SIMD have registers for: 0 beside the score tiles, 1 when those are done with; v (2)
+    // only behind the scores of its own chunk; the decays once more (3) where the strong-decay passes want them.
+    i32x4 xq, xk, xa[2], xb[2], xv, xok;
+    typename GkRaw<T, GKF32>::rows xg, xog;
     T nbeta;
-    // first: the first own channel tile's operands (requested a chunk ahead); !first: everything else of the chunk
-    // (requested when its turn begins: it arrives behind the work on the first tile).  More a chunk ahead would be more
-    // registers held through the whole chunk than three waves per SIMD leave.
-    auto request = [&](int t, bool first) __attribute__((always_inline)) {
-        const int cid = REV ? s1 - 1 - t : s0 + t;
+    char* const sX = lead ? smem + L::ROWS + pp * ROWS_SCRATCH : smem + pp * L::SLOT + L::SOLVE + 32 * FLDP * 4;
+    static_assert(K / 2 == 32 && V / 2 == 32, "half a row of any operand is 64 bytes");
+    auto request = [&](int t, int part) __attribute__((always_inline)) {
+        const int cid = s0 + t;
         const int64_t tok0 = bos + (int64_t)(cid - c0) * CH;
         const int len = (int)min((int64_t)CH, eos - tok0);
-        // uniform base of the chunk's first row + a 32-bit byte offset per lane, formed afresh in every call (see copy_out);
+        // uniform base of the chunk's first row + a 32-bit offset per lane, formed afresh in every call (see copy_out);
         // rows past the end alias the last valid row and are masked at use
-        int cc = c, gg = g;
-        asm volatile("" : "+v"(cc), "+v"(gg));
-        const uint32_t row = (uint32_t)min(cc, max(len, 1) - 1);
+        int ll = l;
+        asm volatile("" : "+v"(ll));
+        const uint32_t row = (uint32_t)min(ll >> 2, max(len, 1) - 1), last = (uint32_t)(max(len, 1) - 1), piece = 16 * (ll & 3);
         constexpr uint32_t ES = sizeof(T), GS = GKF32 ? 4 : 2;
-        const uint32_t qe = row * (uint32_t)(H * K) + 4 * gg, ae = row * (uint32_t)(RANK * H * K) + 4 * gg;
-        const uint32_t ve = row * (uint32_t)(H * V) + 4 * gg;
-        const int64_t qb = (tok0 * H + h) * K, ab = (tok0 * RANK * H + h) * K, vb = (tok0 * H + h) * V;
-        const char* gkp = reinterpret_cast<const char*>(p.gk) + qb * GS;
-        if (!first) {
-            if (!REV) {
-#pragma unroll
-                for (int j = 0; j < VH; ++j) nv[j] = ld_frag(at(p.v + vb, (ve + 16 * (vt0 + j)) * ES));
-            }
-            if (REV || CKPT) {
-#pragma unroll
-                for (int j = 0; j < VH; ++j) ndo[j] = ld_frag(at(p.dout + vb, (ve + 16 * (vt0 + j)) * ES));
-            }
+        if (part == 2) {
+            xv = *reinterpret_cast<const i32x4*>(at(p.v + (tok0 * H + h) * V, (row * (uint32_t)(H * V) + 16 * vt0) * ES + piece));
+            return;
         }
-        if (HD && first) nbeta = *at(p.beta + tok0 * H + h, row * (uint32_t)H * ES);
-#pragma unroll
-        for (int j = 0; j < KH; ++j) {
-            const uint32_t ko = 16 * (kt0 + j), kx = 16 * (KH - kt0 + j);
-            if (HD && first) {
-                // the sum over all channels comes before everything else: k and gk of every tile a chunk ahead
-                if (j > 0) {
-                    ng[j] = GkRaw<T, GKF32>::load(gkp + (qe + ko) * GS);
-                    nk[j] = ld_frag(at(p.k + qb, (qe + ko) * ES));
-                }
-                og[j] = GkRaw<T, GKF32>::load(gkp + (qe + kx) * GS);
-                ok_[j] = ld_frag(at(p.k + qb, (qe + kx) * ES));
-            }
-            if ((j == 0) != first) continue;
-            nq[j] = ld_frag(at(p.q + qb, (qe + ko) * ES));
-            if (!(HD && j > 0)) {
-                ng[j] = GkRaw<T, GKF32>::load(gkp + (qe + ko) * GS);
-                nk[j] = ld_frag(at(p.k + qb, (qe + ko) * ES));
-            }
+        const uint32_t qo = (row * (uint32_t)(H * K) + 16 * kt0) * ES + piece, ao = (row * (uint32_t)(RANK * H * K) + 16 * kt0) * ES + piece;
+        const int64_t qb = (tok0 * H + h) * K, ab = (tok0 * RANK * H + h) * K;
+        const char* gkp = reinterpret_cast<const char*>(p.gk) + qb * GS;
+        auto rows = [](const T* b, uint32_t off) __attribute__((always_inline)) { return *reinterpret_cast<const i32x4*>(at(b, off)); };
+        if (part != 1) GkRaw<T, GKF32>::load(gkp, ll, row * (uint32_t)(H * K) + 16 * kt0, xg);
+        if (part == 3) return;
+        if (part == 0) {
+            xk = rows(p.k + qb, qo);
             if (!HD) {
-                na[0][j] = ld_frag(at(p.a + ab, (ae + ko) * ES));
-                na[1][j] = ld_frag(at(p.a + ab, (ae + (uint32_t)(H * K) + ko) * ES));
-                nb[0][j] = ld_frag(at(p.b + ab, (ae + ko) * ES));
-                nb[1][j] = ld_frag(at(p.b + ab, (ae + (uint32_t)(H * K) + ko) * ES));
+#pragma unroll
+                for (int r = 0; r < 2; ++r) xb[r] = rows(p.b + ab, ao + r * (uint32_t)(H * K) * ES);
             }
+            return;
+        }
+        if (HD) {
+            const uint32_t other = 16 * (KH - kt0);
+            nbeta = *at(p.beta + tok0 * H + h, min((uint32_t)(ll & 15), last) * (uint32_t)H * ES);
+            GkRaw<T, GKF32>::load(gkp, ll, row * (uint32_t)(H * K) + other, xog);
+            xok = rows(p.k + qb, qo + (other - 16 * kt0) * ES);
+        }
+        xq = rows(p.q + qb, qo);
+        if (!HD) {
+#pragma unroll
+            for (int r = 0; r < 2; ++r) xa[r] = rows(p.a + ab, ao + r * (uint32_t)(H * K) * ES);
         }
     };
     // rows past the end of a ragged chunk become zeros, in place and only there (a uniform branch: whole chunks pay nothing)
     auto mask = [](Frag<T>& f, bool ok) __attribute__((always_inline)) { f.v = ok ? f.v : zero_frag<T>().v; };
     auto mask_gk = [](typename GkRaw<T, GKF32>::type& x, bool ok) __attribute__((always_inline)) { GkRaw<T, GKF32>::mask(x, ok); };
-    if (pp < nst) request(pp, true);
+    if (pp < nst) { request(pp, 0); request(pp, 1); }
 
     int it = 0, prev_cid = -1;
     for (int t = pp; t < nst; t += FNP, ++it) {
-        const int cid = REV ? s1 - 1 - t : s0 + t;
+        const int cid = s0 + t;
         const int64_t tok0 = bos + (int64_t)(cid - c0) * CH;
         const int len = (int)min((int64_t)CH, eos - tok0);
         const int64_t chw = (int64_t)h * p.st.nch + cid;
@@ -292,10 +300,25 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
         const Frag<T> ident = ident_of<T>(g, c);
         const bool rowok = c < len;
 
-        request(t, false);                                // the rest of this chunk's inputs
+        Frag<T> nq[KH], nk[KH], na[2][KH], nb[2][KH], ok_[KH];
+        typename GkRaw<T, GKF32>::type ng[KH], og[KH];
+        GkRaw<T, GKF32>::tiles(sX, l, xg, ng);
+        rows_to_tiles(sX, l, xk, nk[0], nk[1]);
+        if (!HD) {
+#pragma unroll
+            for (int r = 0; r < 2; ++r) rows_to_tiles(sX, l, xb[r], nb[r][0], nb[r][1]);
+        } else {
+            GkRaw<T, GKF32>::tiles(sX, l, xog, og);
+            rows_to_tiles(sX, l, xok, ok_[0], ok_[1]);
+        }
+        rows_to_tiles(sX, l, xq, nq[0], nq[1]);
+        if (!HD) {
+#pragma unroll
+            for (int r = 0; r < 2; ++r) rows_to_tiles(sX, l, xa[r], na[r][0], na[r][1]);
+        }
         __builtin_amdgcn_sched_barrier(0);
         // (ag^T waits in the slot where w will go: w = Tm ag is formed further down, when the inverse is there)
-        T* const sWW = reinterpret_cast<T*>(slot + (REV ? SB.W : BF.W));
+        T* const sWW = reinterpret_cast<T*>(slot + BF.W);
 
         // ---- own channel tiles: decays, parts of the score tiles (prep.hip, phase A) -------------------------------------
         // Nothing here needs the slot: the consumers are through with the chunk it held by the time the gated copies below
@@ -303,7 +326,6 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
         f32x4 egi[KH], edn[KH];
         f32x4 aqk = zero4(), aqb[2] = {zero4(), zero4()}, aak[2] = {zero4(), zero4()};
         f32x4 aab[2][2] = {{zero4(), zero4()}, {zero4(), zero4()}};
-        f32x4 aqbT[2] = {zero4(), zero4()};
         bool strong = false;                              // a channel decays beyond the safe range (uniform over the wave)
         float beta_t = 0.f, s_t = 0.f;
         if (HD) {
@@ -353,9 +375,11 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
                 mask(nk[j], rowok);
                 if (!HD) { mask(na[0][j], rowok); mask(na[1][j], rowok); mask(nb[0][j], rowok); mask(nb[1][j], rowok); }
             }
+            if (HD) pin(ng[j]);                           // e^{gk} formed again, not kept from the sum above
             const f32x4 g4 = GkRaw<T, GKF32>::value(ng[j]);
             Frag<T> rq, rk, ra[2], rb[2];
             operands(j, g4, rq, rk, ra, rb);
+            if (HD) __builtin_amdgcn_sched_barrier(0);
             const TileDecay e(g4, c);
             strong |= e.strong;
             egi[j] = e.egi;
@@ -375,8 +399,7 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
                     if (FWD) aqk = mm3(qh, kh, aqk);
 #pragma unroll
                     for (int s = 0; s < 2; ++s) {
-                        if (!REV) aqb[s] = mm3(qh, bh[s], aqb[s]);
-                        if (REV) aqbT[s] = mm3(bh[s], qh, aqbT[s]);
+                        aqb[s] = mm3(qh, bh[s], aqb[s]);
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -384,7 +407,7 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
                 for (int r = 0; r < 2; ++r) {
                     Split<T> ah;
                     split(to_f32(ra[r]) * e.ea, ah);
-                    if (!REV) aak[r] = mm3(ah, kh, aak[r]);
+                    aak[r] = mm3(ah, kh, aak[r]);
                     aab[r][0] = mm3(ah, bh[0], aab[r][0]);
                     aab[r][1] = mm3(ah, bh[1], aab[r][1]);
                     __builtin_amdgcn_sched_barrier(0);
@@ -395,10 +418,15 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
         // Where a channel decays too strongly for the single centre, what was accumulated above may hold infinities: it
         // is thrown away and the parts are formed again by passes whose exponents cannot overflow (see DecayPass).
         if (strong) {
+            if (!HD) {                                    // (not held through the common path)
+                request(t, 3);
+                GkRaw<T, GKF32>::tiles(sX, l, xg, ng);
+                if (len < CH) { mask_gk(ng[0], rowok); mask_gk(ng[1], rowok); }
+            }
             aqk = zero4();
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
-                aqb[s] = zero4(); aak[s] = zero4(); aqbT[s] = zero4(); aab[0][s] = zero4(); aab[1][s] = zero4();
+                aqb[s] = zero4(); aak[s] = zero4(); aab[0][s] = zero4(); aab[1][s] = zero4();
             }
 #pragma unroll 1
             for (int ps = 0; ps < DecayPass::COUNT; ++ps) {
@@ -419,15 +447,14 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
 #pragma unroll
                     for (int s = 0; s < 2; ++s) {
                         split(to_f32(rb[s]) * ek, bh[s]);
-                        if (!REV) aqb[s] = mm3(qh, bh[s], aqb[s]);
-                        if (REV) aqbT[s] = mm3(bh[s], qh, aqbT[s]);
+                        aqb[s] = mm3(qh, bh[s], aqb[s]);
                         __builtin_amdgcn_sched_barrier(0);
                     }
 #pragma unroll
                     for (int r = 0; r < 2; ++r) {
                         Split<T> ah;
                         split(to_f32(ra[r]) * ea, ah);
-                        if (!REV) aak[r] = mm3(ah, kh, aak[r]);
+                        aak[r] = mm3(ah, kh, aak[r]);
                         aab[r][0] = mm3(ah, bh[0], aab[r][0]);
                         aab[r][1] = mm3(ah, bh[1], aab[r][1]);
                         __builtin_amdgcn_sched_barrier(0);
@@ -436,10 +463,10 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
             }
         }
         // ---- the other wave's parts travel to the lead ------------------------------------------------------------------
-        // tile order in the scratch: A_ab (4), then A_ak (2; the reverse kernel: A_qb^T), A_qb (2), A_qk: as many as the mode forms
-        constexpr int NPART = REV ? 6 : FWD ? 9 : 8;    // A_ab, (A_ak), A_qb or its transpose, (A_qk)
+        // tile order in the scratch: A_ab (4), A_ak (2), A_qb (2), A_qk (where the outputs are formed)
+        constexpr int NPART = FWD ? 9 : 8;
         if (!lead) {
-            f32x4* const tiles[9] = {&aab[0][0], &aab[0][1], &aab[1][0], &aab[1][1], REV ? &aqbT[0] : &aak[0], REV ? &aqbT[1] : &aak[1],
+            f32x4* const tiles[9] = {&aab[0][0], &aab[0][1], &aab[1][0], &aab[1][1], &aak[0], &aak[1],
                                      &aqb[0], &aqb[1], &aqk};
 #pragma unroll
             for (int i = 0; i < NPART; ++i) *reinterpret_cast<f32x4*>(sP + (i * 64 + l) * 4) = *tiles[i];
@@ -447,6 +474,8 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
             signal_set(f_part, it + 1);
         }
 
+        request(t, 2);
+        __builtin_amdgcn_sched_barrier(0);
         // ---- the slot: wait until the consumers have left the chunk it held ---------------------------------------------
         if (!wait_ge(f_consumed, VT * it, f_abort)) { if (l == 0) *a.err = FUSED_ABORTED + 1; return; }
         __builtin_amdgcn_sched_barrier(0);
@@ -454,55 +483,40 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
 #pragma unroll
         for (int j = 0; j < KH; ++j) {
             pin(nq[j]); pin(nk[j]);                       // converted again, not kept converted from above
-            if (!HD) { pin(na[0][j]); pin(na[1][j]); pin(nb[0][j]); pin(nb[1][j]); }
+            if (HD) pin(ng[j]);
+            else { pin(na[0][j]); pin(na[1][j]); pin(nb[0][j]); pin(nb[1][j]); }
             Frag<T> rq, rk, ra[2], rb[2];
-            operands(j, GkRaw<T, GKF32>::value(ng[j]), rq, rk, ra, rb);
+            operands(j, HD ? GkRaw<T, GKF32>::value(ng[j]) : zero4(), rq, rk, ra, rb);
             const f32x4 one = {1.f, 1.f, 1.f, 1.f}, ege = prev_token(egi[j], one), egl = bcast16<CH - 1>(egi[j]);
             st_pair(sWW + (0 * KT2 + half) * PAIR, j, transpose(to_frag<T>(to_f32(ra[0]) * ege), ident));
             st_pair(sWW + (1 * KT2 + half) * PAIR, j, transpose(to_frag<T>(to_f32(ra[1]) * ege), ident));
             const Frag<T> fqg = to_frag<T>(to_f32(rq) * egi[j] * scale);
             const Frag<T> fbg[2] = {to_frag<T>(to_f32(rb[0]) * edn[j]), to_frag<T>(to_f32(rb[1]) * edn[j])};
-            if (!REV) {
-                st_pair(reinterpret_cast<T*>(slot + BF.KGT) + half * PAIR, j, transpose(to_frag<T>(to_f32(rk) * edn[j]), ident));
-                st_pair(reinterpret_cast<T*>(slot + BF.BGT) + (0 * KT2 + half) * PAIR, j, transpose(fbg[0], ident));
-                st_pair(reinterpret_cast<T*>(slot + BF.BGT) + (1 * KT2 + half) * PAIR, j, transpose(fbg[1], ident));
-                st_pair(reinterpret_cast<T*>(slot + BF.QG) + half * PAIR, j, fqg);
-            } else {
-                // the reverse scan takes bg as it is and w transposed (the stand-alone kernel turns the stored tiles on
-                // their way into LDS: the same values)
-                st_pair(reinterpret_cast<T*>(slot + SB.BGT) + (0 * KT2 + half) * PAIR, j, fbg[0]);
-                st_pair(reinterpret_cast<T*>(slot + SB.BGT) + (1 * KT2 + half) * PAIR, j, fbg[1]);
-                st_pair(reinterpret_cast<T*>(slot + SB.QGT) + half * PAIR, j, transpose(fqg, ident));
-            }
-            if (c == 0) *reinterpret_cast<f32x4*>(slot + (REV ? SB.EGL : BF.EGL) + (16 * (kt0 + j) + 4 * g) * 4) = egl;
+            st_pair(reinterpret_cast<T*>(slot + BF.KGT) + half * PAIR, j, transpose(to_frag<T>(to_f32(rk) * edn[j]), ident));
+            st_pair(reinterpret_cast<T*>(slot + BF.BGT) + (0 * KT2 + half) * PAIR, j, transpose(fbg[0], ident));
+            st_pair(reinterpret_cast<T*>(slot + BF.BGT) + (1 * KT2 + half) * PAIR, j, transpose(fbg[1], ident));
+            st_pair(reinterpret_cast<T*>(slot + BF.QG) + half * PAIR, j, fqg);
+            if (c == 0) *reinterpret_cast<f32x4*>(slot + BF.EGL + (16 * (kt0 + j) + 4 * g) * 4) = egl;
             __builtin_amdgcn_sched_barrier(0);
         }
-        // the inputs are used up: the next chunk's first ones may come
-        if (t + FNP < nst) request(t + FNP, true);
-        __builtin_amdgcn_sched_barrier(0);
-
         Frag<T> vT[VH];
-        if (!REV) {
+        rows_to_tiles(slot + L::UT + vt0 * PAIR * (int)sizeof(T), l, xv, vT[0], vT[1]);   // (where u of these tiles goes later)
 #pragma unroll
-            for (int j = 0; j < VH; ++j) {
-                if (len < CH) mask(nv[j], rowok);
-                vT[j] = transpose(nv[j], ident);
-                st_frag(reinterpret_cast<T*>(slot + L::VTT) + (vt0 + j) * TILE + 4 * l, vT[j]);
-            }
+        for (int j = 0; j < VH; ++j) {
+            if (len < CH) mask(vT[j], rowok);
+            vT[j] = transpose(vT[j], ident);
+            st_frag(reinterpret_cast<T*>(slot + L::VTT) + (vt0 + j) * TILE + 4 * l, vT[j]);
         }
-        if (REV || CKPT) {
-#pragma unroll
-            for (int j = 0; j < VH; ++j) {
-                if (len < CH) mask(ndo[j], rowok);
-                st_frag(reinterpret_cast<T*>(slot + L::DOT) + (vt0 + j) * TILE + 4 * l, transpose(ndo[j], ident));
-            }
-        }
+        // the inputs are used up: the next chunk's may come
+        __builtin_amdgcn_sched_barrier(0);
+        if (t + FNP < nst) request(t + FNP, 0);
+        __builtin_amdgcn_sched_barrier(0);
 
         // ---- the lead: whole score tiles, (I - A_ab)^-1 by forward substitution (prep.hip, phase B) ---------------------
         Frag<T> tm[2][2], aakf[2];
         if (lead) {
             if (!wait_ge(f_part, it + 1, f_abort)) { if (l == 0) *a.err = FUSED_ABORTED + 1; return; }
-            f32x4* const tiles[9] = {&aab[0][0], &aab[0][1], &aab[1][0], &aab[1][1], REV ? &aqbT[0] : &aak[0], REV ? &aqbT[1] : &aak[1],
+            f32x4* const tiles[9] = {&aab[0][0], &aab[0][1], &aab[1][0], &aab[1][1], &aak[0], &aak[1],
                                      &aqb[0], &aqb[1], &aqk};
             // the lower channel tiles' part first, as a single wave adds them
 #pragma unroll
@@ -510,22 +524,17 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
                 const f32x4 o = *reinterpret_cast<const f32x4*>(sP + (i * 64 + l) * 4);
                 *tiles[i] = half == 0 ? *tiles[i] + o : o + *tiles[i];
             }
-            if (CKPT && l == 0) p.ws.STRONG[chw] = (strong || *f_strong != 0) ? 1 : 0;
+            if (p.ws.TM && l == 0) p.ws.STRONG[chw] = (strong || *f_strong != 0) ? 1 : 0;
             // causal masks: lane (g,c) reg i is entry (row c, inner 4g+i)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int j = 4 * g + i;
-                const bool le = j <= c, lt = j < c, tle = c <= j;
+                const bool le = j <= c, lt = j < c;
                 if (!le) { aqk[i] = 0.f; aqb[0][i] = 0.f; aqb[1][i] = 0.f; }
                 if (!lt) { aak[0][i] = 0.f; aak[1][i] = 0.f; aab[0][0][i] = 0.f; aab[0][1][i] = 0.f; aab[1][0][i] = 0.f; aab[1][1][i] = 0.f; }
-                if (!tle) { aqbT[0][i] = 0.f; aqbT[1][i] = 0.f; }
             }
-            if (!REV) {
-                if (FWD) st_frag(reinterpret_cast<T*>(slot + BF.AQK) + 4 * l, to_frag<T>(aqk));
-                st_pair2(reinterpret_cast<T*>(slot + BF.AQB), to_frag<T>(aqb[0]), to_frag<T>(aqb[1]));
-            } else {
-                st_pair2(reinterpret_cast<T*>(slot + SB.AQBT), to_frag<T>(aqbT[0]), to_frag<T>(aqbT[1]));
-            }
+            if (FWD) st_frag(reinterpret_cast<T*>(slot + BF.AQK) + 4 * l, to_frag<T>(aqk));
+            st_pair2(reinterpret_cast<T*>(slot + BF.AQB), to_frag<T>(aqb[0]), to_frag<T>(aqb[1]));
             aakf[0] = to_frag<T>(aak[0]);
             aakf[1] = to_frag<T>(aak[1]);
             // (all of the other wave's parts have been read: the scratch may be written)
@@ -601,13 +610,13 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
 #pragma unroll
             for (int s = 0; s < 2; ++s) st_pair2(sPub + s * PAIR, tm[s][0], tm[s][1]);
             st_pair2(sPub + 2 * PAIR, aakf[0], aakf[1]);
-            if (CKPT) {
-                // What the checkpoint pass leaves in the workspace for chunk_grad ((I - A_ab)^-1 here, u and where needed w
-                // below) goes there from the consumers, which have no loads to wait for: a store issued here would stand
-                // behind the next chunk's loads in this wave's in-order memory counter.
+            if (p.ws.TM) {
+                // the record goes out from the consumers, which have no loads to wait for: a store issued here would stand
+                // behind the next chunk's loads in this wave's in-order memory counter
                 T* tmw = reinterpret_cast<T*>(slot + L::TMB);
 #pragma unroll
                 for (int s = 0; s < 2; ++s) st_pair2(tmw + s * PAIR, transpose(tm[s][0], ident), transpose(tm[s][1], ident));
+                st_pair2(reinterpret_cast<T*>(slot + L::AKB), aakf[0], aakf[1]);
             }
             signal_set(f_inv, it + 1);
         } else {
@@ -619,6 +628,9 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
             for (int s = 0; s < 2; ++s) ld_pair(sPub + s * PAIR, tm[s][0], tm[s][1]);
             ld_pair(sPub + 2 * PAIR, aakf[0], aakf[1]);
         }
+        __builtin_amdgcn_sched_barrier(0);
+        if (t + FNP < nst) request(t + FNP, 1);
+        __builtin_amdgcn_sched_barrier(0);
         // ---- w = Tm ag for the own channel tiles, in place of ag^T -------------------------------------------------------
         {
             Frag<T> agT[2][2], fw[2][2];
@@ -633,25 +645,20 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
                     fw[s][e] = to_frag<T>(w);
                 }
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                if (!REV) st_pair2(sWW + (s * KT2 + half) * PAIR, fw[s][0], fw[s][1]);
-                else st_pair2(sWW + (s * KT2 + half) * PAIR, transpose(fw[s][0], ident), transpose(fw[s][1], ident));
-            }
+            for (int s = 0; s < 2; ++s) st_pair2(sWW + (s * KT2 + half) * PAIR, fw[s][0], fw[s][1]);
         }
         // ---- u = Tm (A_ak v) for the own value tiles, transposed (prep.hip, phase D) ------------------------------------
-        if (!REV) {
 #pragma unroll
-            for (int j = 0; j < VH; ++j) {
-                const Frag<T> mT[2] = {to_frag<T>(mm(vT[j], aakf[0], zero4())), to_frag<T>(mm(vT[j], aakf[1], zero4()))};
-                Frag<T> fu[2];
+        for (int j = 0; j < VH; ++j) {
+            const Frag<T> mT[2] = {to_frag<T>(mm(vT[j], aakf[0], zero4())), to_frag<T>(mm(vT[j], aakf[1], zero4()))};
+            Frag<T> fu[2];
 #pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    f32x4 uT = mm(mT[0], tm[s][0], zero4());
-                    uT = mm(mT[1], tm[s][1], uT);
-                    fu[s] = to_frag<T>(uT);
-                }
-                st_pair2(reinterpret_cast<T*>(slot + L::UT) + (vt0 + j) * PAIR, fu[0], fu[1]);
+            for (int s = 0; s < 2; ++s) {
+                f32x4 uT = mm(mT[0], tm[s][0], zero4());
+                uT = mm(mT[1], tm[s][1], uT);
+                fu[s] = to_frag<T>(uT);
             }
+            st_pair2(reinterpret_cast<T*>(slot + L::UT) + (vt0 + j) * PAIR, fu[0], fu[1]);
         }
         signal_add(f_ready);
         prev_cid = cid;
@@ -663,20 +670,266 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
     }
 }
 
+// ---- producers of the backward pass's kernels ----------------------------------------------------------------------
+// The same pairs, slots and shares of a chunk, with the score tiles' results read from the record: nothing is exchanged
+// between the waves of a pair and nothing is solved, a wave forms the gated copies, w and (checkpoint kernel) u of its own
+// tiles.  What is left is mostly traffic (29 KB a chunk and head each, at K = V = 64): a wave requests the whole of its next
+// chunk as soon as this one's is unpacked, long before it waits for the slot, and holds its results in registers until then.
+template <typename T, bool GKF32, int K, int V, int MODE, bool HD>
+__device__ __forceinline__ void fused_replay(const FusedArgs<T>& a, char* smem, int n, int h, int seg, int s0, int s1, int pp, int half) {
+    static_assert(K == 64 && sizeof(T) == 2 && V % 32 == 0, "a producer pair holds all channels of a chunk: K = 64, 2-byte elements");
+    typedef FusedLds<T, K, V, MODE> L;
+    constexpr bool REV = MODE == FUSED_REV;
+    static_assert(REV || MODE == FUSED_CKPT, "the backward pass's kernels");
+    constexpr int VT = V / 16, KT2 = K / 32, KH = 2, VH = VT / 2;
+    constexpr BlkF BF = L::BF;
+    constexpr SlotB SB = L::SB;
+    const ChunkArgs<T>& p = a.c;
+    int* const flags = reinterpret_cast<int*>(smem + L::FLAGS);
+    int* const f_ready = flags + pp, * const f_consumed = flags + 4 + pp, * const f_abort = flags + 8;
+    int l = lane_id(), g = l >> 4, c = l & 15;
+    const int H = p.H;
+    // (The read-first-lane keeps the optimiser from turning "load, splat" into a vector load of the kernel argument: that
+    // ties it to its neighbour st.cu in one memory object, which then goes to LDS, and what depends on st.cu becomes
+    // per-lane control flow that reads the absent table of an unpacked batch.)
+    const float scale = __int_as_float(uniform(__float_as_int(p.scale)));
+    const int nst = s1 - s0;
+    const int kt0 = half * KH, vt0 = half * VH;
+    int64_t bos, eos;
+    seq_bounds(p.st, n, bos, eos);
+    int c0, c1;
+    seq_chunks(p.st, n, c0, c1);
+
+    // the wave's share of a chunk's inputs as loaded (see fused_producer), and the record's tiles
+    i32x4 xq, xk, xa[2], xb[2], xv, xdo, xok, xtm[2], xaq;
+    typename GkRaw<T, GKF32>::rows xg, xog;
+    T nbeta;
+    char* const sX = smem + L::ROWS + (2 * pp + half) * ROWS_SCRATCH;
+    static_assert(K / 2 == 32 && V / 2 == 32, "half a row of any operand is 64 bytes");
+    constexpr bool WITH_K = HD || !REV;                   // the reverse kernel needs k only to form a and b from it
+    auto request = [&](int t) __attribute__((always_inline)) {
+        const int cid = REV ? s1 - 1 - t : s0 + t;
+        const int64_t tok0 = bos + (int64_t)(cid - c0) * CH;
+        const int len = (int)min((int64_t)CH, eos - tok0);
+        const int64_t chw = (int64_t)h * p.st.nch + cid;
+        // uniform base + a 32-bit byte offset per lane, formed afresh in every call (hoisted out of the chunk loop they would
+        // be held in registers through all of it); rows past the end alias the last valid row and are masked at use
+        int ll = l;
+        asm volatile("" : "+v"(ll));
+        const uint32_t row = (uint32_t)min(ll >> 2, max(len, 1) - 1), last = (uint32_t)(max(len, 1) - 1), piece = 16 * (ll & 3);
+        constexpr uint32_t ES = sizeof(T), GS = GKF32 ? 4 : 2;
+        const uint32_t qo = (row * (uint32_t)(H * K) + 16 * kt0) * ES + piece, ao = (row * (uint32_t)(RANK * H * K) + 16 * kt0) * ES + piece;
+        const uint32_t vo = (row * (uint32_t)(H * V) + 16 * vt0) * ES + piece, lo = (uint32_t)ll * 16;
+        const int64_t qb = (tok0 * H + h) * K, ab = (tok0 * RANK * H + h) * K, vb = (tok0 * H + h) * V;
+        const char* gkp = reinterpret_cast<const char*>(p.gk) + qb * GS;
+        auto rows = [](const T* b, uint32_t off) __attribute__((always_inline)) { return *reinterpret_cast<const i32x4*>(at(b, off)); };
+        GkRaw<T, GKF32>::load(gkp, ll, row * (uint32_t)(H * K) + 16 * kt0, xg);
+        if (WITH_K) xk = rows(p.k + qb, qo);
+        if (HD) {
+            const uint32_t other = 16 * (KH - kt0);
+            nbeta = *at(p.beta + tok0 * H + h, min((uint32_t)(ll & 15), last) * (uint32_t)H * ES);
+            GkRaw<T, GKF32>::load(gkp, ll, row * (uint32_t)(H * K) + other, xog);
+            xok = rows(p.k + qb, qo + (other - 16 * kt0) * ES);
+        } else {
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                xa[r] = rows(p.a + ab, ao + r * (uint32_t)(H * K) * ES);
+                xb[r] = rows(p.b + ab, ao + r * (uint32_t)(H * K) * ES);
+            }
+        }
+        if (REV) xq = rows(p.q + qb, qo);
+        else xv = rows(p.v + vb, vo);
+        xdo = rows(p.dout + vb, vo);
+        const T* tm = p.ws.TM + chw * 1024;
+        xtm[0] = rows(tm, lo);
+        xtm[1] = rows(tm + PAIR, lo);
+        xaq = rows(a.aq + chw * 1024 + (REV ? PAIR : 0), lo);
+    };
+    auto mask = [](Frag<T>& f, bool ok) __attribute__((always_inline)) { f.v = ok ? f.v : zero_frag<T>().v; };
+    auto mask_gk = [](typename GkRaw<T, GKF32>::type& x, bool ok) __attribute__((always_inline)) { GkRaw<T, GKF32>::mask(x, ok); };
+    if (pp < nst) request(pp);
+
+    int it = 0;
+    for (int t = pp; t < nst; t += FNP, ++it) {
+        const int cid = REV ? s1 - 1 - t : s0 + t;
+        const int64_t tok0 = bos + (int64_t)(cid - c0) * CH;
+        const int len = (int)min((int64_t)CH, eos - tok0);
+        asm volatile("" : "+v"(l));                       // lane-only values formed afresh for every chunk (see fused_producer)
+        g = l >> 4;
+        c = l & 15;
+        char* slot;
+        {
+            int so = pp * L::SLOT;
+            asm volatile("" : "+s"(so));
+            slot = smem + so;
+        }
+        const Frag<T> ident = ident_of<T>(g, c);
+        const bool rowok = c < len;
+        Frag<T> nq[KH], nk[KH], na[2][KH], nb[2][KH], nv[VH], ndo[VH], ok_[KH], ntm[2][2], naq[2];
+        typename GkRaw<T, GKF32>::type ng[KH], og[KH];
+        GkRaw<T, GKF32>::tiles(sX, l, xg, ng);
+        if (WITH_K) rows_to_tiles(sX, l, xk, nk[0], nk[1]);
+        if (HD) {
+            GkRaw<T, GKF32>::tiles(sX, l, xog, og);
+            rows_to_tiles(sX, l, xok, ok_[0], ok_[1]);
+        } else {
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                rows_to_tiles(sX, l, xa[r], na[r][0], na[r][1]);
+                rows_to_tiles(sX, l, xb[r], nb[r][0], nb[r][1]);
+            }
+        }
+        if (REV) rows_to_tiles(sX, l, xq, nq[0], nq[1]);
+        else rows_to_tiles(sX, l, xv, nv[0], nv[1]);
+        rows_to_tiles(sX, l, xdo, ndo[0], ndo[1]);
+        auto pair = [](i32x4 x, Frag<T>& f0, Frag<T>& f1) __attribute__((always_inline)) {
+            const s16x8 y = __builtin_bit_cast(s16x8, x);
+            f0.v = __builtin_shufflevector(y, y, 0, 1, 2, 3);
+            f1.v = __builtin_shufflevector(y, y, 4, 5, 6, 7);
+        };
+        pair(xtm[0], ntm[0][0], ntm[0][1]);
+        pair(xtm[1], ntm[1][0], ntm[1][1]);
+        pair(xaq, naq[0], naq[1]);
+        const T bt = nbeta;
+        // (everything requested has arrived: the next chunk's inputs may be)
+        __builtin_amdgcn_sched_barrier(0);
+        if (t + FNP < nst) request(t + FNP);
+        __builtin_amdgcn_sched_barrier(0);
+        if (len < CH) {
+#pragma unroll
+            for (int j = 0; j < KH; ++j) {
+                mask_gk(ng[j], rowok);
+                if (WITH_K) mask(nk[j], rowok);
+                if (HD) { mask_gk(og[j], rowok); mask(ok_[j], rowok); }
+                else { mask(na[0][j], rowok); mask(na[1][j], rowok); mask(nb[0][j], rowok); mask(nb[1][j], rowok); }
+                if (REV) mask(nq[j], rowok);
+            }
+#pragma unroll
+            for (int j = 0; j < VH; ++j) {
+                if (!REV) mask(nv[j], rowok);
+                mask(ndo[j], rowok);
+            }
+        }
+        float beta_t = 0.f, s_t = 0.f;
+        if (HD) {
+            beta_t = rowok ? ld_elem(&bt) : 0.f;
+#pragma unroll
+            for (int j = 0; j < KH; ++j) {
+                const f32x4 g4 = GkRaw<T, GKF32>::value(ng[j]), gx = GkRaw<T, GKF32>::value(og[j]);
+                const f32x4 k4 = to_f32(nk[j]), kx = to_f32(ok_[j]);
+                const f32x4 kf = k4 * k4 * exp4<T>(g4) + kx * kx * exp4<T>(gx);
+                s_t += kf[0] + kf[1] + kf[2] + kf[3];
+            }
+            s_t += __shfl_xor(s_t, 16);
+            s_t += __shfl_xor(s_t, 32);
+        }
+        // ---- gated copies of the own channel tiles (prep.hip, phase C) ---------------------------------------------------
+        Frag<T> agT[2][KH], fb[2][KH], fx[KH];            // fb, fx: bg^T, kg^T (checkpoint kernel); bg, qg^T (reverse kernel)
+        f32x4 egl[KH];
+#pragma unroll
+        for (int j = 0; j < KH; ++j) {
+            const f32x4 g4 = GkRaw<T, GKF32>::value(ng[j]), one = {1.f, 1.f, 1.f, 1.f};
+            const f32x4 gi = scan16_incl(g4), egi = exp4<T>(gi), edn = exp4<T>(bcast16<CH - 1>(gi) - gi);
+            const f32x4 ege = prev_token(egi, one);
+            egl[j] = bcast16<CH - 1>(egi);
+            Frag<T> ra[2], rb[2];
+            if (HD) {
+                const f32x4 kk = to_f32(nk[j]), f4 = exp4<T>(g4);
+                ra[0] = to_frag<T>(kk * (-beta_t));
+                ra[1] = to_frag<T>(kk * ((beta_t * s_t - f4) * beta_t));
+                rb[0] = to_frag<T>(f4 * kk);
+                rb[1] = nk[j];
+            } else {
+#pragma unroll
+                for (int r = 0; r < 2; ++r) { ra[r] = na[r][j]; rb[r] = nb[r][j]; }
+            }
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                agT[r][j] = transpose(to_frag<T>(to_f32(ra[r]) * ege), ident);
+                fb[r][j] = to_frag<T>(to_f32(rb[r]) * edn);
+                if (!REV) fb[r][j] = transpose(fb[r][j], ident);
+            }
+            if constexpr (REV) fx[j] = transpose(to_frag<T>(to_f32(nq[j]) * egi * scale), ident);
+            else fx[j] = transpose(to_frag<T>(to_f32(nk[j]) * edn), ident);
+        }
+        // ---- w = Tm ag for the own channel tiles (reverse kernel: w^T), u = Tm (A_ak v) for the own value tiles -----------
+        Frag<T> tm[2][2], fw[2][KH], vT[VH], doT[VH], fu[VH][2], aq[2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int r = 0; r < 2; ++r) tm[s][r] = transpose(ntm[s][r], ident);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) aq[s] = REV ? transpose(naq[s], ident) : naq[s];
+#pragma unroll
+        for (int j = 0; j < VH; ++j) {
+            doT[j] = transpose(ndo[j], ident);
+            if (!REV) vT[j] = transpose(nv[j], ident);
+        }
+#pragma unroll
+        for (int j = 0; j < KH; ++j)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                f32x4 w;
+                if (REV) {
+                    w = mm(agT[0][j], tm[s][0], zero4());
+                    w = mm(agT[1][j], tm[s][1], w);
+                } else {
+                    w = mm(tm[s][0], agT[0][j], zero4());
+                    w = mm(tm[s][1], agT[1][j], w);
+                }
+                fw[s][j] = to_frag<T>(w);
+            }
+        if (!REV) {
+#pragma unroll
+            for (int j = 0; j < VH; ++j) {
+                const Frag<T> mT[2] = {to_frag<T>(mm(vT[j], aq[0], zero4())), to_frag<T>(mm(vT[j], aq[1], zero4()))};
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    f32x4 uT = mm(mT[0], tm[s][0], zero4());
+                    uT = mm(mT[1], tm[s][1], uT);
+                    fu[j][s] = to_frag<T>(uT);
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // ---- the slot --------------------------------------------------------------------------------------------------------
+        if (!wait_ge(f_consumed, VT * it, f_abort)) { if (l == 0) *a.err = FUSED_ABORTED + 1; return; }
+        T* const sW = reinterpret_cast<T*>(slot + (REV ? SB.W : BF.W)), * const sB = reinterpret_cast<T*>(slot + (REV ? SB.BGT : BF.BGT));
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            st_pair2(sW + (s * KT2 + half) * PAIR, fw[s][0], fw[s][1]);
+            st_pair2(sB + (s * KT2 + half) * PAIR, fb[s][0], fb[s][1]);
+        }
+        st_pair2(reinterpret_cast<T*>(slot + (REV ? SB.QGT : BF.KGT)) + half * PAIR, fx[0], fx[1]);
+        if (REV && half == 0) st_pair2(reinterpret_cast<T*>(slot + SB.AQBT), aq[0], aq[1]);
+        if (c == 0) {
+#pragma unroll
+            for (int j = 0; j < KH; ++j) *reinterpret_cast<f32x4*>(slot + (REV ? SB.EGL : BF.EGL) + (16 * (kt0 + j) + 4 * g) * 4) = egl[j];
+        }
+#pragma unroll
+        for (int j = 0; j < VH; ++j) {
+            st_frag(reinterpret_cast<T*>(slot + L::DOT) + (vt0 + j) * TILE + 4 * l, doT[j]);
+            if (!REV) {
+                st_frag(reinterpret_cast<T*>(slot + L::VTT) + (vt0 + j) * TILE + 4 * l, vT[j]);
+                st_pair2(reinterpret_cast<T*>(slot + L::UT) + (vt0 + j) * PAIR, fu[j][0], fu[j][1]);
+            }
+        }
+        signal_add(f_ready);
+    }
+}
+
 // ---- consumers, forward direction ----------------------------------------------------------------------------------
 // Fragment-order records in the workspace (256 fp32 per tile, lane l owns elements 4l..4l+3), per (sequence, head,
 // segment):
-//   sloc  [V/16][K/16] tiles  F(S^T): the state leaving the segment (started from h0 / the given boundary in segment
-//                             0 and in checkpoint mode, from zero otherwise)
-//   mseg  [K/16][K/16] tiles  the segment's transition M (segments > 0).  Forward pass: tile (kt, k't) = F(M block),
-//                             rows k, inner k'; checkpoint mode: the transposed block, rows k', inner k
-//   rseg  [V/16][K/16] tiles  F(R^T), R = sum_t G_t^T do_t (checkpoint mode, segments > 0)
+//   sloc  [V/16][K/16] tiles  F(S^T): the state leaving the segment (started from h0 in segment 0, from zero otherwise)
+//   mseg  [K/16][K/16] tiles  the segment's transition M (segments > 0): tile (kt, k't) = F(M block), rows k, inner k'
+//   mt    [K/16][K/16] tiles  the same with the blocks transposed, rows k', inner k (part of the record)
+//   rseg  [V/16][K/16] tiles  F(R^T), R = sum_t G_t^T do_t (checkpoint kernel, segments > 0)
 //   sin   [V/16][K/16] tiles  F(S_in^T): the state entering the segment (segments > 0)
-// W_GLOBAL: chunk_grad reads w from the workspace where it cannot rebuild it (chunk_grad_body.inc: REBUILD_W)
-template <typename T, int K, int V, int MODE, bool W_GLOBAL>
+template <typename T, int K, int V, int MODE>
 __device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* smem, int n, int h, int seg, int s0, int s1, int wv) {
     typedef FusedLds<T, K, V, MODE> L;
-    constexpr bool CKPT = MODE == FUSED_CKPT, FWD = MODE == FUSED_FWD;
+    constexpr bool FWD = MODE == FUSED_FWD;
     constexpr int KT = K / 16, VT = V / 16, KT2 = KT / 2;
     static_assert(KT == VT, "consumer j owns column block j of the state and of the transition matrix");
     constexpr BlkF BF = L::BF;
@@ -690,28 +943,19 @@ __device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* 
     const int64_t soff = ((int64_t)n * H + h) * K * V + 16 * vt + c;
 
     // state block: lane (g,c) reg i of tile kt = S[16kt + 4g + i][16vt + c]; likewise M with column 16vt + c
-    f32x4 S[KT], M[KT], R[VT];
+    f32x4 S[KT], M[KT];
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) {
         S[kt] = zero4();
 #pragma unroll
         for (int i = 0; i < 4; ++i) M[kt][i] = (16 * kt + 4 * g + i == 16 * vt + c) ? 1.f : 0.f;
     }
+    if (seg == 0 && p.h0) {
 #pragma unroll
-    for (int j = 0; j < VT; ++j) R[j] = zero4();
-    if (seg == 0) {
-        if (p.h0) {
+        for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-            for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) S[kt][i] = p.h0[soff + (int64_t)(16 * kt + 4 * g + i) * V];
-        }
-    } else if (CKPT) {
-        const float* sin = a.sin + rec * (K * V);
-#pragma unroll
-        for (int kt = 0; kt < KT; ++kt) S[kt] = *reinterpret_cast<const f32x4*>(sin + (vt * KT + kt) * TILE + 4 * l);
+            for (int i = 0; i < 4; ++i) S[kt][i] = p.h0[soff + (int64_t)(16 * kt + 4 * g + i) * V];
     }
-    const Frag<T> ident = ident_frag<T>();
 
     for (int t = 0; t < nst; ++t) {
         const int pp = t & (FNP - 1), it = t / FNP;
@@ -764,27 +1008,14 @@ __device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* 
             o = mm(aqk, vtt, o);
         }
         const Frag<T> vnb[2] = {to_frag<T>(vn[0]), to_frag<T>(vn[1])};
-        if (CKPT) {
-            T* hc = p.ws.HC + chw * (K * V) + vt * PAIR;
-#pragma unroll
-            for (int kp = 0; kp < KT2; ++kp) st_pair2(hc + kp * (VT * PAIR), sb[2 * kp], sb[2 * kp + 1]);
-            // the producer's results that chunk_grad reads: between the waves the two tile pairs of (I - A_ab)^-1 and,
-            // where chunk_grad does not rebuild them, this wave's tiles of u and the 2 KT/2 pairs of w
-            if (W_GLOBAL) st_pair2(p.ws.UT + (chw * VT + vt) * PAIR, ut[0], ut[1]);
-            if (wv < 2) {
-                Frag<T> t0, t1;
-                ld_pair(reinterpret_cast<const T*>(slot + L::TMB) + wv * PAIR, t0, t1);
-                st_pair2(p.ws.TM + chw * 1024 + wv * PAIR, t0, t1);
-            }
-            if (W_GLOBAL) {
-                static_assert(!W_GLOBAL || 2 * KT2 == VT, "one pair of w per consumer");
-                T* wg = p.ws.W + chw * (p.ws.sa_stride / (int)sizeof(T));
-#pragma unroll
-                for (int s = 0; s < 2; ++s)
-#pragma unroll
-                    for (int kp = 0; kp < KT2; ++kp)
-                        if (wv == s * KT2 + kp) st_pair2(wg + (s * KT2 + kp) * PAIR, w[s][2 * kp], w[s][2 * kp + 1]);
-            }
+        if (p.ws.TM) {
+            // the record, a tile pair by each wave: (I - A_ab)^-1, A_ak, A_qb
+            static_assert(VT == 4, "four tile pairs");
+            const int src = wv < 2 ? L::TMB + wv * PAIR * (int)sizeof(T) : wv == 2 ? L::AKB : BF.AQB;
+            T* dst = (wv < 2 ? p.ws.TM : a.aq) + chw * 1024 + (wv & 1) * PAIR;
+            Frag<T> t0, t1;
+            ld_pair(reinterpret_cast<const T*>(slot + src), t0, t1);
+            st_pair2(dst, t0, t1);
         }
         if (FWD) {
             o = mm(aqb[0], vnb[0], o);
@@ -820,12 +1051,7 @@ __device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* 
             G = mm(aqb[1], vpb[1], G);
             const Frag<T> Gf = to_frag<T>(G);             // rows token, inner k' (the block's columns)
             if (FWD) st_frag(reinterpret_cast<T*>(smem + pp * L::SLOT + L::GBOX + c * L::GROW) + 16 * wv + 4 * g, Gf);
-            if (CKPT) {
-                // R[k'][v] += sum_tok G[tok][k'] do[tok][v]
-                const Frag<T> GT = transpose(Gf, ident);
-#pragma unroll
-                for (int j = 0; j < VT; ++j) R[j] = mm(GT, ld_tile(reinterpret_cast<const T*>(slot + L::DOT) + j * TILE), R[j]);
-            }
+            else st_frag(a.gw + (chw * CH + c) * K + 16 * wv + 4 * g, Gf);
 #pragma unroll
             for (int kt = 0; kt < KT; ++kt) {
                 f32x4 x = M[kt] * egl[kt];
@@ -839,7 +1065,7 @@ __device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* 
 
     // ---- what the segment leaves behind ------------------------------------------------------------------------------
     if (a.nseg == 1) {
-        if (p.ht && !CKPT) {
+        if (FWD && p.ht) {
 #pragma unroll
             for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
@@ -847,11 +1073,9 @@ __device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* 
         }
         return;
     }
-    if (!CKPT) {
-        float* sloc = a.sloc + rec * (K * V);
+    float* sloc = a.sloc + rec * (K * V);
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt) *reinterpret_cast<f32x4*>(sloc + (vt * KT + kt) * TILE + 4 * l) = S[kt];
-    }
+    for (int kt = 0; kt < KT; ++kt) *reinterpret_cast<f32x4*>(sloc + (vt * KT + kt) * TILE + 4 * l) = S[kt];
     if (pblk) {
         float* mseg = a.mseg + rec * (K * K);
         const Frag<float> identf = ident_frag<float>();
@@ -859,18 +1083,135 @@ __device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* 
         for (int kt = 0; kt < KT; ++kt) {
             Frag<float> f;
             f.v = M[kt];
-            if (!CKPT) f = transpose(f, identf);          // exact: fp32 products with ones and zeros
+            if (a.mt) *reinterpret_cast<f32x4*>(a.mt + rec * (K * K) + (kt * KT + wv) * TILE + 4 * l) = f.v;
+            f = transpose(f, identf);                     // exact: fp32 products with ones and zeros
             *reinterpret_cast<f32x4*>(mseg + (kt * KT + wv) * TILE + 4 * l) = f.v;
         }
-        if (CKPT) {
-            float* rseg = a.rseg + rec * (K * V);
+    }
+}
+
+// ---- consumers, checkpoint kernel ------------------------------------------------------------------------------------
+// The state walk of the forward direction from the true entering state, leaving the state entering every chunk for
+// chunk_grad, and R from the record's G.
+// W_GLOBAL: chunk_grad reads u and w from the workspace where it cannot rebuild them (chunk_grad_body.inc: REBUILD_W)
+template <typename T, int K, int V, bool W_GLOBAL>
+__device__ __forceinline__ void fused_consumer_ckpt(const FusedArgs<T>& a, char* smem, int n, int h, int seg, int s0, int s1, int wv) {
+    typedef FusedLds<T, K, V, FUSED_CKPT> L;
+    constexpr int KT = K / 16, VT = V / 16, KT2 = KT / 2;
+    static_assert(KT == VT, "consumer j owns column block j of the state and of G");
+    constexpr BlkF BF = L::BF;
+    const ChunkArgs<T>& p = a.c;
+    int* const flags = reinterpret_cast<int*>(smem + L::FLAGS);
+    const int l = lane_id(), g = l >> 4, c = l & 15;
+    const int H = p.H, vt = wv;
+    const int nst = s1 - s0;
+    const bool later = seg > 0;                           // uniform over the workgroup
+    const int64_t rec = ((int64_t)n * H + h) * a.nseg + seg;
+    const int64_t soff = ((int64_t)n * H + h) * K * V + 16 * vt + c;
+
+    f32x4 S[KT], R[VT];
 #pragma unroll
-            for (int j = 0; j < VT; ++j) {
-                Frag<float> f;
-                f.v = R[j];
-                f = transpose(f, identf);
-                *reinterpret_cast<f32x4*>(rseg + (j * KT + wv) * TILE + 4 * l) = f.v;
-            }
+    for (int kt = 0; kt < KT; ++kt) S[kt] = zero4();
+#pragma unroll
+    for (int j = 0; j < VT; ++j) R[j] = zero4();
+    if (later) {
+        const float* sin = a.sin + rec * (K * V);
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) S[kt] = *reinterpret_cast<const f32x4*>(sin + (vt * KT + kt) * TILE + 4 * l);
+    } else if (p.h0) {
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) S[kt][i] = p.h0[soff + (int64_t)(16 * kt + 4 * g + i) * V];
+    }
+    const Frag<T> ident = ident_frag<T>();
+    // rows token, inner k' (the block's columns), requested a chunk ahead
+    const T* gw = a.gw + ((int64_t)h * p.st.nch + s0) * (CH * K) + c * K + 16 * wv + 4 * g;
+    Frag<T> gn = zero_frag<T>();
+    if (later) gn = ld_frag(gw);
+
+    for (int t = 0; t < nst; ++t) {
+        const int pp = t & (FNP - 1), it = t / FNP;
+        if (!wait_ge(&flags[pp], 2 * (it + 1), &flags[8])) { if (l == 0) *a.err = FUSED_ABORTED + 2; return; }
+        const char* slot = smem + pp * L::SLOT;
+        const int cid = s0 + t;
+        const int64_t chw = (int64_t)h * p.st.nch + cid;
+        const T* sW = reinterpret_cast<const T*>(slot + BF.W);
+        const T* sBGT = reinterpret_cast<const T*>(slot + BF.BGT);
+        const T* sKGT = reinterpret_cast<const T*>(slot + BF.KGT);
+        const float* sEGL = reinterpret_cast<const float*>(slot + BF.EGL);
+        Frag<T> w[2][KT], kgt[KT], bgt[2][KT], ut[2], vtt, dot[VT];
+        f32x4 egl[KT];
+#pragma unroll
+        for (int kp = 0; kp < KT2; ++kp) {
+            ld_pair(sW + (0 * KT2 + kp) * PAIR, w[0][2 * kp], w[0][2 * kp + 1]);
+            ld_pair(sW + (1 * KT2 + kp) * PAIR, w[1][2 * kp], w[1][2 * kp + 1]);
+        }
+        ld_pair(reinterpret_cast<const T*>(slot + L::UT) + wv * PAIR, ut[0], ut[1]);
+        vtt = ld_tile(reinterpret_cast<const T*>(slot + L::VTT) + wv * TILE);
+#pragma unroll
+        for (int kp = 0; kp < KT2; ++kp) {
+            ld_pair(sKGT + kp * PAIR, kgt[2 * kp], kgt[2 * kp + 1]);
+            ld_pair(sBGT + (0 * KT2 + kp) * PAIR, bgt[0][2 * kp], bgt[0][2 * kp + 1]);
+            ld_pair(sBGT + (1 * KT2 + kp) * PAIR, bgt[1][2 * kp], bgt[1][2 * kp + 1]);
+            egl[2 * kp] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (2 * kp) + 4 * g);
+            egl[2 * kp + 1] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (2 * kp + 1) + 4 * g);
+        }
+        Frag<T> gt = gn;
+        if (later) {
+#pragma unroll
+            for (int j = 0; j < VT; ++j) dot[j] = ld_tile(reinterpret_cast<const T*>(slot + L::DOT) + j * TILE);
+            gt = transpose(gn, ident);
+            if (t + 1 < nst) gn = ld_frag(gw + (int64_t)(t + 1) * (CH * K));
+        }
+        // the stand-alone scan's step (scan_impl.cuh), operation for operation
+        Frag<T> sb[KT];
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) sb[kt] = to_frag<T>(S[kt]);
+        f32x4 vn[2] = {to_f32(ut[0]), to_f32(ut[1])};
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) {
+            vn[0] = mm(sb[kt], w[0][kt], vn[0]);
+            vn[1] = mm(sb[kt], w[1][kt], vn[1]);
+        }
+        const Frag<T> vnb[2] = {to_frag<T>(vn[0]), to_frag<T>(vn[1])};
+        T* hc = p.ws.HC + chw * (K * V) + vt * PAIR;
+#pragma unroll
+        for (int kp = 0; kp < KT2; ++kp) st_pair2(hc + kp * (VT * PAIR), sb[2 * kp], sb[2 * kp + 1]);
+        if (W_GLOBAL) {
+            static_assert(2 * KT2 == VT, "one pair of w per consumer");
+            st_pair2(p.ws.UT + (chw * VT + vt) * PAIR, ut[0], ut[1]);
+            T* wg = p.ws.W + chw * (p.ws.sa_stride / (int)sizeof(T));
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int kp = 0; kp < KT2; ++kp)
+                    if (wv == s * KT2 + kp) st_pair2(wg + (s * KT2 + kp) * PAIR, w[s][2 * kp], w[s][2 * kp + 1]);
+        }
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) {
+            f32x4 x = S[kt] * egl[kt];
+            x = mm(vtt, kgt[kt], x);
+            x = mm(vnb[0], bgt[0][kt], x);
+            x = mm(vnb[1], bgt[1][kt], x);
+            S[kt] = x;
+        }
+        if (later) {
+            // R[k'][v] += sum_tok G[tok][k'] do[tok][v]
+#pragma unroll
+            for (int j = 0; j < VT; ++j) R[j] = mm(gt, dot[j], R[j]);
+        }
+        signal_add(&flags[4 + pp]);
+    }
+    if (later) {
+        float* rseg = a.rseg + rec * (K * V);
+        const Frag<float> identf = ident_frag<float>();
+#pragma unroll
+        for (int j = 0; j < VT; ++j) {
+            Frag<float> f;
+            f.v = R[j];
+            f = transpose(f, identf);
+            *reinterpret_cast<f32x4*>(rseg + (j * KT + wv) * TILE + 4 * l) = f.v;
         }
     }
 }
@@ -929,7 +1270,7 @@ __device__ __forceinline__ void fused_consumer_rev(const FusedArgs<T>& a, char* 
 #pragma unroll
             for (int b = 0; b < STG; ++b) {
                 if (b < ns) {
-                    const float* mrec = a.mseg + (rec0 + step[b]) * (K * K) + wv * NQ * TILE + 4 * l;
+                    const float* mrec = a.mt + (rec0 + step[b]) * (K * K) + wv * NQ * TILE + 4 * l;
 #pragma unroll
                     for (int i = 0; i < NQ; ++i) mq[b][i] = *reinterpret_cast<const f32x4*>(mrec + i * TILE);
                 }
@@ -1062,9 +1403,12 @@ __global__ __launch_bounds__(64 * (V / 16 + 2 * FNP)) void fused_kernel(FusedArg
     __syncthreads();
     if (wv < V / 16) {
         if constexpr (MODE == FUSED_REV) fused_consumer_rev<T, K, V>(a, smem, n, h, seg, s0, s1, wv);
-        else fused_consumer_fwd<T, K, V, MODE, MODE == FUSED_CKPT && (HD || GKF32)>(a, smem, n, h, seg, s0, s1, wv);
+        else if constexpr (MODE == FUSED_CKPT) fused_consumer_ckpt<T, K, V, HD || GKF32>(a, smem, n, h, seg, s0, s1, wv);
+        else fused_consumer_fwd<T, K, V, MODE>(a, smem, n, h, seg, s0, s1, wv);
     } else {
-        fused_producer<T, GKF32, K, V, MODE, HD>(a, smem, n, h, seg, s0, s1, (wv - V / 16) >> 1, (wv - V / 16) & 1);
+        const int pp = (wv - V / 16) >> 1, half = (wv - V / 16) & 1;
+        if constexpr (L::SOLVES) fused_producer<T, GKF32, K, V, MODE, HD>(a, smem, n, h, seg, s0, s1, pp, half);
+        else fused_replay<T, GKF32, K, V, MODE, HD>(a, smem, n, h, seg, s0, s1, pp, half);
     }
 }
 
@@ -1102,7 +1446,7 @@ __global__ __launch_bounds__(256) void fixup_kernel(FusedArgs<T> a) {
         const int per = (s1 - s0 + FIXUP_PARTS - 1) / FIXUP_PARTS;
         s0 = min(s0 + part * per, s1);
         s1 = min(s0 + per, s1);
-        if (s1 <= s0 || (part > 0 && !a.gw)) return;
+        if (s1 <= s0 || (part > 0 && !a.ol)) return;
     } else if (!p.ht || part > 0) return;
     const int64_t rec0 = ((int64_t)n * H + h) * a.nseg;
     const int64_t soff = ((int64_t)n * H + h) * K * V + 16 * vt + c;
@@ -1126,7 +1470,7 @@ __global__ __launch_bounds__(256) void fixup_kernel(FusedArgs<T> a) {
             for (int j = 0; j < VT; ++j) OLr[b][j] = *reinterpret_cast<const f32x4*>(ol + 16 * j);
         }
     };
-    const bool outputs = target < a.nseg && a.gw != nullptr;
+    const bool outputs = target < a.nseg && a.ol != nullptr;
     if (outputs) request(s0 + wv);
 
     // S[kt]: lane (g,c) reg i = S[16kt + 4g + i][16vt + c].  Segment 0 ran from the initial state itself; only where it
@@ -1221,7 +1565,7 @@ __global__ __launch_bounds__(256) void fixup_kernel(FusedArgs<T> a) {
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) *reinterpret_cast<f32x4*>(so + kt * TILE + 4 * l) = S[kt];
     }
-    if (!a.gw) return;                                    // chaining only (the backward pass re-deriving the states)
+    if (!a.ol) return;                                    // chaining only (the backward pass re-deriving the states)
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) st_tile(sS + (vt * KT + kt) * TILE, to_frag<T>(S[kt]));
     __syncthreads();

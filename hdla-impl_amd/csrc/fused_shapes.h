@@ -5,9 +5,9 @@
 
 namespace hdla {
 
-// FUSED_FWD: forward pass (o, or o_local and G for segments > 0; segment records).  FUSED_SUM: the segment records only
-// (what a backward pass runs first when the forward pass left no boundary record).  FUSED_CKPT: the backward pass's
-// forward half: state checkpoints, (I - A_ab)^-1, u, strong-decay flags, and the records the reverse half chains.
+// FUSED_FWD: forward pass (o, or o_local and G for segments > 0; segment records; with ws.TM set: the record for the backward
+// pass).  FUSED_SUM: the same without the outputs (what a backward pass runs first when the forward pass left no record).
+// FUSED_CKPT: the backward pass's forward half: state checkpoints, u and w where chunk_grad reads them, R of the segments.
 // FUSED_REV: the reverse scan of the state gradient: dS checkpoints, dv_new, dh0.
 enum FusedMode { FUSED_FWD = 0, FUSED_SUM = 1, FUSED_CKPT = 2, FUSED_REV = 3 };
 
@@ -21,8 +21,11 @@ struct FusedArgs {
     float* rseg;           // [N][H][nseg][K*V]
     const float* sin;      // [N][H][nseg][K*V]  states entering the segments (read by FUSED_CKPT)
     float* sin_out;        // the same record, written by fixup_kernel (nullable)
-    float* ol;             // [H][nch][16][V] fp32  local outputs of segments > 0 (forward pass)
-    T* gw;                 // [H][nch][16][K]       G of segments > 0 (forward pass); null: fixup_kernel only chains
+    float* ol;             // [H][nch][16][V] fp32  local outputs of segments > 0 (forward pass); null: fixup_kernel only chains
+    // the record (with c.ws.TM and c.ws.STRONG): written by FUSED_FWD and FUSED_SUM, read by FUSED_CKPT and FUSED_REV
+    float* mt;             // [N][H][nseg][K*K]     transposed transitions of segments > 0 (nullable)
+    T* gw;                 // [H][nch][16][K]       G of segments > 0 (the forward pass's fixup_kernel needs it as well)
+    T* aq;                 // [H][nch][2][2 tiles]  A_ak, A_qb
     int* err;              // set nonzero by a wave whose bounded wait ran out
 };
 

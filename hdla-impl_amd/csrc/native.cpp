@@ -37,7 +37,7 @@ using torch::autograd::variable_list;
 // ---- the C ABI -------------------------------------------------------------------------------------------------------
 struct Api {
 #define HDLA_FN(name) decltype(&hdla_##name) name
-    HDLA_FN(strerror); HDLA_FN(workspace_bytes); HDLA_FN(boundary_bytes); HDLA_FN(chunk_fwd_b); HDLA_FN(chunk_bwd_b);
+    HDLA_FN(strerror); HDLA_FN(workspace_bytes); HDLA_FN(record_bytes); HDLA_FN(chunk_fwd_b); HDLA_FN(chunk_bwd_b);
     HDLA_FN(recurrent_fwd); HDLA_FN(param_recurrent_fwd); HDLA_FN(normalize_fwd); HDLA_FN(normalize_bwd);
     HDLA_FN(normalize_workspace_bytes); HDLA_FN(layer_pre_fwd); HDLA_FN(layer_pre_bwd); HDLA_FN(layer_up_fwd); HDLA_FN(layer_down);
     HDLA_FN(layer_up_wgrad); HDLA_FN(layer_up_wgrad_workspace_bytes); HDLA_FN(rows_gemm); HDLA_FN(sum_partials);
@@ -131,7 +131,7 @@ void chunk_forward(const ChunkIn& x, const hdla_dims& d, bool want_ht, bool want
     const auto f32 = x.q.options().dtype(at::kFloat);
     o = at::empty_like(x.v);
     if (want_ht) ht = at::empty({d.N, d.H, d.K, d.V}, f32);
-    const size_t nb = want_boundary ? api.boundary_bytes(&d) : 0;
+    const size_t nb = want_boundary ? api.record_bytes(&d) : 0;
     if (nb) boundary = bytes_like(x.q, nb);
     const Tensor ws = workspace(d, HDLA_PASS_FWD, x.q);
     check(api.chunk_fwd_b(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.beta), ptr(x.gk), fptr(x.h0), ptr(o), fptr(ht),
@@ -139,7 +139,7 @@ void chunk_forward(const ChunkIn& x, const hdla_dims& d, bool want_ht, bool want
 }
 
 // The autograd node: the contract of ChunkDPLRDeltaRuleFunction and ChunkHDLAFunction (the inputs and, where the route
-// has one, the record of the states at the segment boundaries are saved; everything else is recomputed).
+// has one, the record for the backward pass are saved; everything else is recomputed).
 struct ChunkFn : torch::autograd::Function<ChunkFn> {
     static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Maybe& a, const Maybe& b,
                                  const Maybe& beta, const Tensor& gk, const Maybe& h0, const Maybe& cu, double scale, bool want_ht) {
@@ -753,7 +753,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
         PyErr_SetString(a[1], "the library does not export hdla_" #name);                                          \
         return nullptr;                                                                                            \
     }
-    HDLA_FN(strerror) HDLA_FN(workspace_bytes) HDLA_FN(boundary_bytes) HDLA_FN(chunk_fwd_b) HDLA_FN(chunk_bwd_b)
+    HDLA_FN(strerror) HDLA_FN(workspace_bytes) HDLA_FN(record_bytes) HDLA_FN(chunk_fwd_b) HDLA_FN(chunk_bwd_b)
     HDLA_FN(recurrent_fwd) HDLA_FN(param_recurrent_fwd) HDLA_FN(normalize_fwd) HDLA_FN(normalize_bwd)
     HDLA_FN(normalize_workspace_bytes) HDLA_FN(layer_pre_fwd) HDLA_FN(layer_pre_bwd) HDLA_FN(layer_up_fwd) HDLA_FN(layer_down)
     HDLA_FN(layer_up_wgrad) HDLA_FN(layer_up_wgrad_workspace_bytes) HDLA_FN(rows_gemm) HDLA_FN(sum_partials)

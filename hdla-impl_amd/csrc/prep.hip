@@ -376,7 +376,6 @@ __global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const 
         // order, so that when there are more workgroups than compute units the long sequences are not the ones that
         // wait.  All counts go to LDS (entries past N hold -1 and rank behind everything); a thread reads them four at
         // a time against its own.
-        typedef int i32x4 __attribute__((ext_vector_type(4)));
         for (int n = t; n < ORDER_MAX_N; n += TABLE_THREADS) len[n] = n < N ? (int)min(chunks_of(n), (long long)0x7fffffff) : -1;
         __syncthreads();
         const int n = ((int)blockIdx.x - 1) * TABLE_THREADS + t;

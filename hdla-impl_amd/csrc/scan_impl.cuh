@@ -39,7 +39,6 @@
 
 namespace hdla {
 
-typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 // workgroup barrier that orders LDS accesses only: global loads issued before it may still be outstanding
 __device__ __forceinline__ void lds_barrier() {

@@ -9,7 +9,7 @@ from typing import Optional
 import torch
 
 HDLA_BF16, HDLA_FP32 = 0, 1
-HDLA_VERSION = 201          # the header this binding was written against (struct layouts, entry points)
+HDLA_VERSION = 202          # the header this binding was written against (struct layouts, entry points)
 ROUTE_AUTO, ROUTE_CLASSIC, ROUTE_FUSED = 0, 1, 2
 _ROUTES = {"": ROUTE_AUTO, "auto": ROUTE_AUTO, "classic": ROUTE_CLASSIC, "fused": ROUTE_FUSED}
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -96,6 +96,8 @@ def load():
     lib.hdla_param_chunk_bwd.argtypes = [F] + [P] * 14 + [P, ctypes.c_size_t, P]
     lib.hdla_boundary_bytes.restype = ctypes.c_size_t
     lib.hdla_boundary_bytes.argtypes = [F]
+    lib.hdla_record_bytes.restype = ctypes.c_size_t
+    lib.hdla_record_bytes.argtypes = [F]
     lib.hdla_chunk_fwd_b.restype = ctypes.c_int
     lib.hdla_chunk_fwd_b.argtypes = [F] + [P] * 10 + [P, ctypes.c_size_t, P, ctypes.c_size_t, P]
     lib.hdla_chunk_bwd_b.restype = ctypes.c_int
@@ -206,15 +208,22 @@ def make_dims(B, T, H, K, V, R, N, in_dtype, gk_dtype, scale, cu_seqlens: Option
 
 
 def keep_boundaries_default() -> bool:
-    """Whether the forward pass of the chunked operators hands the states at the time-segment boundaries (fused route:
-    64 KiB per sequence, head and segment) to the backward pass, which otherwise re-derives them from the inputs with
-    one more pass.  On by default; HDLA_HIP_INPUTS_ONLY=1 keeps strictly the inputs between the passes."""
+    """Whether the forward pass of the chunked operators hands its record (fused route: the states at the time-segment
+    boundaries and what the chunks' score tiles come to, 37 % of the inputs' bytes) to the backward pass, which otherwise
+    re-derives it from the inputs with one more pass.  On by default; HDLA_HIP_INPUTS_ONLY=1 keeps strictly the inputs
+    between the passes."""
     return os.environ.get("HDLA_HIP_INPUTS_ONLY", "0") in ("", "0", "false", "False")
 
 
 def boundary(dims: HdlaDims, device) -> Optional[torch.Tensor]:
-    """An empty boundary record for these dimensions, or None where the route has none."""
+    """Room for the states at the segment boundaries for these dimensions, or None where the route has none."""
     n = load().hdla_boundary_bytes(ctypes.byref(dims))
+    return torch.empty(n, dtype=torch.uint8, device=device) if n else None
+
+
+def record(dims: HdlaDims, device) -> Optional[torch.Tensor]:
+    """Room for the forward pass's record (boundary states included), or None where the route has none."""
+    n = load().hdla_record_bytes(ctypes.byref(dims))
     return torch.empty(n, dtype=torch.uint8, device=device) if n else None
 
 

@@ -72,7 +72,7 @@ def chunk_hrdplr_fwd(q, k, v, a, b, gk, scale, initial_state, output_final_state
                      beta=None, want_boundary=False):
     """Forward launch sequence (HRDPLR/hrdplr.py:25-99) on native shapes: returns (o, final_state), with ``keep`` also
     the workspace the backward pass can run on instead of recomputing it (``hdla_chunk_fwd_keep``), with
-    ``want_boundary`` also the record of the states at the time-segment boundaries (None where the route has none).
+    ``want_boundary`` also the record for the backward pass (None where the route has none).
     With ``beta`` a and b are formed in the kernels (they may be None)."""
     lib = _lib.load()
     B, T, H, K = q.shape
@@ -90,7 +90,7 @@ def chunk_hrdplr_fwd(q, k, v, a, b, gk, scale, initial_state, output_final_state
             _lib.check(rc, "hdla_chunk_fwd_keep")
             return o, ht, ws
         ws = _lib.workspace(dims, _lib.PASS_FWD, q.device)
-        bnd = _lib.boundary(dims, q.device) if want_boundary else None
+        bnd = _lib.record(dims, q.device) if want_boundary else None
         rc = lib.hdla_chunk_fwd_b(ctypes.byref(dims), _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(a), _lib.ptr(b),
                                   _lib.ptr(beta), _lib.ptr(gk), _lib.ptr(initial_state), _lib.ptr(o), _lib.ptr(ht),
                                   _lib.ptr(bnd), 0 if bnd is None else bnd.numel(),
@@ -186,8 +186,8 @@ class ChunkDPLRDeltaRuleFunction(torch.autograd.Function):
                                                         want_boundary=True)
         else:
             o, final_state = chunk_hrdplr_fwd(q, k, v, a, b, gk, scale, h0, output_final_state, cu_seqlens)
-        # the inputs (hrdplr.py:137) and, where the route cuts sequences into time segments, the states at the segment
-        # boundaries (64 KiB per sequence, head and segment; HDLA_HIP_INPUTS_ONLY=1: not even those)
+        # the inputs (hrdplr.py:137) and, where the route has one, the forward pass's record (37 % of the inputs' bytes;
+        # HDLA_HIP_INPUTS_ONLY=1: strictly the inputs)
         ctx.save_for_backward(q, k, v, a, b, gk, initial_state, cu_seqlens, boundary)
         ctx.scale = scale
         ctx.chunk_size = chunk_size

@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-#define HDLA_VERSION 201
+#define HDLA_VERSION 202
 
 enum { HDLA_BF16 = 0, HDLA_FP32 = 1 };
 
@@ -153,8 +153,14 @@ int hdla_chunk_bwd(const hdla_dims* dims, const void* q, const void* k, const vo
  * (which is what hdla_chunk_bwd does, and hdla_chunk_bwd_b with boundary = NULL).  The reference keeps the inputs only
  * (ctx.save_for_backward, HRDPLR/hrdplr.py:137) and recomputes everything (:161-198); the record is what this route
  * adds to that.  hdla_boundary_bytes returns 0 where the route has no such record (classic route, one segment):
- * boundary is then ignored. */
+ * boundary is then ignored.
+ * With boundary_bytes >= hdla_record_bytes(dims) in both calls the forward pass leaves there, beside those states, what
+ * the score tiles of every chunk come to ((I - A_ab)^-1, A_ak, A_qb, the segments' transitions and their outputs per unit
+ * of entering state: 6 KiB per (16-token chunk, head) at K = V = 64, 37 % of the inputs' bytes), which makes the backward
+ * pass's first two kernels a third faster; without it the backward pass forms the same in its workspace first.
+ * hdla_record_bytes returns 0 on the classic route only. */
 size_t hdla_boundary_bytes(const hdla_dims* dims);
+size_t hdla_record_bytes(const hdla_dims* dims);
 int hdla_chunk_fwd_b(const hdla_dims* dims, const void* q, const void* k, const void* v, const void* a, const void* b,
                      const void* beta, const void* gk, const float* h0, void* o, float* ht, void* boundary,
                      size_t boundary_bytes, void* workspace, size_t workspace_bytes, void* stream);
@@ -208,9 +214,10 @@ enum {
     HDLA_STAGE_SCAN_BWD = 4,    /* reverse state-gradient scan (pass 1 only) */
     HDLA_STAGE_CHUNK_GRAD = 8,  /* per-chunk gradient assembly (pass 1 only) */
     HDLA_STAGE_CHAIN = 16,      /* fused route with several segments only.  Pass 0: the kernel that chains the segments and
-                                 * completes the outputs.  Pass 1: what a backward pass without a boundary record runs first
-                                 * (summary kernel + chaining); it leaves the states entering the segments in the workspace,
-                                 * where later calls without this stage find them */
+                                 * completes the outputs.  Pass 1: what a backward pass without a record runs first
+                                 * (summary kernel + chaining); it leaves the record and the states entering the segments in
+                                 * the workspace, where later calls without this stage find them (with one segment the
+                                 * summary kernel is part of HDLA_STAGE_SCAN_FWD) */
     HDLA_STAGE_ALL = 31
 };
 int hdla_chunk_stages(const hdla_dims* dims, int pass, int stages, const void* q, const void* k, const void* v,

@@ -1,0 +1,61 @@
+"""The fused route's record (what the forward pass leaves for the backward pass): a backward pass that reads it gives the
+gradients of one that forms it itself first, and both those of the classic route."""
+import ctypes
+
+import pytest
+import torch
+
+from hdla_hip import _lib
+from hdla_hip.synthetic import make_inputs
+from oracle import hrdplr_oracle as O
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _call(x, cu, segments, route, with_record, beta):
+    lib, P = _lib.load(), _lib.ptr
+    B, T, H, K = x["q"].shape
+    V, N = x["v"].shape[-1], x["h0"].shape[0]
+    dims = _lib.make_dims(B, T, H, K, V, 2, N, torch.bfloat16, x["gk"].dtype, 0.7, cu, route=route, segments=segments)
+    s = _lib.current_stream(torch.device(DEV))
+    rec = _lib.record(dims, DEV) if with_record else None
+    assert not with_record or rec is not None
+    nrec = 0 if rec is None else rec.numel()
+    a, b, bt = (None, None, x["beta"]) if beta else (x["a"], x["b"], None)
+    o, ht = torch.zeros_like(x["v"]), torch.empty_like(x["h0"])
+    ws = _lib.workspace(dims, 0, DEV)
+    _lib.check(lib.hdla_chunk_fwd_b(ctypes.byref(dims), P(x["q"]), P(x["k"]), P(x["v"]), P(a), P(b), P(bt), P(x["gk"]), P(x["h0"]), P(o),
+                                    P(ht), P(rec), nrec, P(ws), ws.numel(), s), "fwd")
+    g = {n: torch.zeros_like(x[n]) for n in (("q", "k", "v", "beta", "gk") if beta else ("q", "k", "v", "a", "b", "gk"))}
+    g["h0"] = torch.empty_like(x["h0"])
+    ws = _lib.workspace(dims, 1, DEV)
+    _lib.check(lib.hdla_chunk_bwd_b(ctypes.byref(dims), P(x["q"]), P(x["k"]), P(x["v"]), P(a), P(b), P(bt), P(x["gk"]), P(x["h0"]),
+                                    P(x["do"]), P(x["dht"]), P(g["q"]), P(g["k"]), P(g["v"]), P(g.get("a")), P(g.get("b")),
+                                    P(g.get("beta")), P(g["gk"]), P(g["h0"]), P(rec), nrec, P(ws), ws.numel(), s), "bwd")
+    torch.cuda.synchronize()
+    return {"o": o, "ht": ht, **g}
+
+
+@pytest.mark.parametrize("beta", [False, True])
+@pytest.mark.parametrize("gk_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,T,H,cu,segments,gk_div", [
+    (1, 5, 2, None, 1, 2.0), (2, 16, 1, None, 1, 2.0), (1, 129, 3, None, 1, 2.0), (2, 203, 2, None, 2, 8.0), (1, 1000, 2, None, 8, 8.0),
+    (1, 300, 2, (0, 37, 37, 200, 300), 3, 8.0), (1, 150, 2, None, 2, 0.05)])
+def test_backward_pass_from_the_record(B, T, H, cu, segments, gk_div, gk_dtype, beta):
+    n_states = B if cu is None else len(cu) - 1
+    inp = make_inputs(31, B, T, H, 64, 64, gk_div=gk_div, n_states=n_states)
+    x = {n: getattr(inp, n).to(DEV).to(torch.bfloat16 if n not in ("h0", "dht", "gk") else gk_dtype if n == "gk" else torch.float32)
+         for n in ("q", "k", "v", "a", "b", "gk", "h0", "do", "dht")}
+    if beta:
+        x["k"] = torch.nn.functional.normalize(x["k"].float(), dim=-1).bfloat16()
+        x["beta"] = torch.rand(B, T, H, generator=torch.Generator().manual_seed(3)).bfloat16().to(DEV)
+    cud = None if cu is None else torch.tensor(cu, dtype=torch.int64, device=DEV)
+    kept = _call(x, cud, segments, _lib.ROUTE_FUSED, True, beta)
+    formed = _call(x, cud, segments, _lib.ROUTE_FUSED, False, beta)
+    classic = _call(x, cud, 0, _lib.ROUTE_CLASSIC, False, beta)
+    for n in kept:
+        print(n, f"{O.rel_l2(kept[n], formed[n]):.1e} {O.rel_l2(kept[n], classic[n]):.1e}", flush=True)
+        assert torch.isfinite(kept[n].float()).all(), n
+        assert O.rel_l2(kept[n], formed[n]) <= 1e-3, n
+        assert O.rel_l2(kept[n], classic[n]) <= (6e-3 if segments > 1 else 2e-3), n
