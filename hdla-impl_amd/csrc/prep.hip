@@ -53,10 +53,6 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void 
     const int H = p.H;
     const bool rowok = c < cp.len;
     const int64_t tok = cp.tok0 + min(c, cp.len - 1);   // rows past the end alias the last valid row, masked by rowok
-    const int64_t qoff = (tok * H + h) * K + 4 * g;                 // + 16*kt
-    const int64_t aoff0 = ((tok * RANK + 0) * H + h) * K + 4 * g;
-    const int64_t aoff1 = ((tok * RANK + 1) * H + h) * K + 4 * g;
-    const int64_t voff = (tok * H + h) * V + 4 * g;
     const int64_t chw = (int64_t)h * p.st.nch + cid;                // chunk-head slot in the workspace
     const float scale = p.scale;
 
@@ -67,68 +63,133 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void 
     // the inputs of the chunk stay in registers (as loaded) for the second use in phase C: the working set of the
     // resident waves is larger than the L2, so a second load would come from HBM again
     Frag<T> rq[KTW], rk[KTW], ra[2][KTW], rb[2][KTW];       // own channel tiles; index kt below is local, kt0 + kt global
+    // us, a fragment's lanes loading for themselves -> TileLoad: K=V=128 bf16, 16384 tokens of 16 heads, forward / backward mode
+    // 248 / 253 -> 236 / 239; with the HDLA parameterisation, where a wave also read the other one's channels of k and gk for s,
+    // 5003 tokens of 16 heads 85 -> 72.  What is left is the traffic: 70 KB a chunk and head, 239 us at a large copy's rate.
+    typedef std::conditional_t<GKF32, float, bf16> G;
+    typedef TileLoad<T, 2> Load;
+    typedef TileLoad<G, 2> LoadG;
+    char* const scratch = reinterpret_cast<char*>(sT);               // free until phase B
+    static_assert(ROWS_SCRATCH <= sizeof(sTw[0]), "");
+    const T* const qrow = p.q + (cp.tok0 * H + h) * K + 16 * kt0;
+    const T* const krow = p.k + (cp.tok0 * H + h) * K + 16 * kt0;
+    const G* const grow = reinterpret_cast<const G*>(p.gk) + (cp.tok0 * H + h) * K + 16 * kt0;
+    const T* const arow = HD ? nullptr : p.a + (cp.tok0 * RANK * H + h) * K + 16 * kt0;
+    const T* const brow = HD ? nullptr : p.b + (cp.tok0 * RANK * H + h) * K + 16 * kt0;
+    const T* const vrow = p.v + (cp.tok0 * H + h) * V + 16 * vt0;
     // v is used last (phase D) but requested first: the barriers in between would otherwise keep its loads, and a
     // full round trip to HBM, behind everything else
     Frag<T> rv[VTW];
+    Load lv[VTW / 2];
 #pragma unroll
-    for (int vt = 0; vt < VTW; ++vt) rv[vt] = ld_frag_sel(p.v + voff + 16 * (vt0 + vt), rowok);
+    for (int vp = 0; vp < VTW / 2; ++vp) lv[vp].load(vrow + 32 * vp, H * V, cp.len, l);
     // HDLA parameterisation: a_1 = -beta k, a_2 = beta k (beta s - f), b_1 = f k, b_2 = k with f = exp(gk) and
-    // s = sum over ALL channels of k^2 f (a wave reads the other waves' channels of k and gk for it as well)
+    // s = sum over ALL channels of k^2 f (two waves exchange their channels' parts)
     float beta_t = 0.f, s_t = 0.f;
+    if (HD) beta_t = rowok ? ld_elem(p.beta + tok * H + h) : 0.f;
+    f32x4 gks[HD ? KTW : 1];
     if (HD) {
-        beta_t = rowok ? ld_elem(p.beta + tok * H + h) : 0.f;
 #pragma unroll
-        for (int kt = 0; kt < K / 16; ++kt) {
-            const f32x4 g4 = ld_gk4<GKF32>(p.gk, qoff + 16 * kt, rowok);
-            const f32x4 k4 = to_f32(ld_frag_sel(p.k + qoff + 16 * kt, rowok));
-            const f32x4 kf = k4 * k4 * exp4<T>(g4);
-            s_t += kf[0] + kf[1] + kf[2] + kf[3];
+        for (int kp = 0; kp < KTW / 2; ++kp) {
+            LoadG lg;
+            Load lk;
+            lg.load(grow + 32 * kp, H * K, cp.len, l);
+            lk.load(krow + 32 * kp, H * K, cp.len, l);
+            Frag<G> fg[2];
+            Frag<T> f[2];
+            lg.tiles(scratch, cp.len, l, fg);
+            lk.tiles(scratch, cp.len, l, f);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int kt = 2 * kp + e;
+                gks[kt] = to_f32(fg[e]);
+                rk[kt] = f[e];
+                const f32x4 k4 = to_f32(f[e]), kf = k4 * k4 * exp4<T>(gks[kt]);
+                s_t += kf[0] + kf[1] + kf[2] + kf[3];
+            }
         }
         s_t += __shfl_xor(s_t, 16);
         s_t += __shfl_xor(s_t, 32);
+        if (NWP > 1) {                                    // sPart is free until the score tiles are summed
+            if (g == 0) sPart[w * CH + c] = s_t;
+            __syncthreads();
+            s_t = 0.f;
+#pragma unroll
+            for (int ww = 0; ww < NWP; ++ww) s_t += sPart[ww * CH + c];
+            __syncthreads();
+        }
     }
 #pragma unroll
-    for (int kt = 0; kt < KTW; ++kt) {
-        const int ko = 16 * (kt0 + kt);
-        const f32x4 g4 = ld_gk4<GKF32>(p.gk, qoff + ko, rowok);
-        rq[kt] = ld_frag_sel(p.q + qoff + ko, rowok);
-        rk[kt] = ld_frag_sel(p.k + qoff + ko, rowok);
-        if (HD) {
-            const f32x4 kk = to_f32(rk[kt]), f4 = exp4<T>(g4);
-            ra[0][kt] = to_frag<T>(kk * (-beta_t));
-            ra[1][kt] = to_frag<T>(kk * ((beta_t * s_t - f4) * beta_t));
-            rb[0][kt] = to_frag<T>(f4 * kk);
-            rb[1][kt] = rk[kt];
-        } else {
-            ra[0][kt] = ld_frag_sel(p.a + aoff0 + ko, rowok);
-            ra[1][kt] = ld_frag_sel(p.a + aoff1 + ko, rowok);
-            rb[0][kt] = ld_frag_sel(p.b + aoff0 + ko, rowok);
-            rb[1][kt] = ld_frag_sel(p.b + aoff1 + ko, rowok);
-        }
-        gi[kt] = scan16_incl(g4);
-        ge[kt] = gi[kt] - g4;
-        // Every score is a dense product of operands decayed relative to the middle of the chunk: exp(gi_i - gi_j) =
-        // exp(gi_i - m) exp(m - gi_j) with m = gi of token MID.  That is done here for every chunk, tile by tile as the
-        // inputs arrive; it is only valid while the exponents stay within +-SAFE_RANGE, which is checked afterwards.
-        const f32x4 m = bcast16<MID>(gi[kt]);
-        const f32x4 eq = exp4<T>(gi[kt] - m), ek = exp4<T>(m - gi[kt]), ea = exp4<T>(ge[kt] - m);
-        const f32x4 q4 = to_f32(rq[kt]), k4 = to_f32(rk[kt]);
-        const f32x4 a0 = to_f32(ra[0][kt]), a1 = to_f32(ra[1][kt]), b0 = to_f32(rb[0][kt]), b1 = to_f32(rb[1][kt]);
-        Split<T> qh, kh, ah[2], bh[2];
-        split(q4 * eq * scale, qh);
-        split(k4 * ek, kh);
-        split(a0 * ea, ah[0]);
-        split(a1 * ea, ah[1]);
-        split(b0 * ek, bh[0]);
-        split(b1 * ek, bh[1]);
-        aqk = mm3(qh, kh, aqk);
+    for (int kp = 0; kp < KTW / 2; ++kp) {
+        Load lq, lk, la[2], lb[2];
+        LoadG lg;
+        Frag<T> fq[2], fk[2], fa[2][2], fb[2][2];
+        Frag<G> fg[2];
+        lq.load(qrow + 32 * kp, H * K, cp.len, l);
+        if (!HD) {
+            lg.load(grow + 32 * kp, H * K, cp.len, l);
+            lk.load(krow + 32 * kp, H * K, cp.len, l);
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            aqb[s] = mm3(qh, bh[s], aqb[s]);
-            aak[s] = mm3(ah[s], kh, aak[s]);
-#pragma unroll
-            for (int r = 0; r < 2; ++r) aab[r][s] = mm3(ah[r], bh[s], aab[r][s]);
+            for (int r = 0; r < 2; ++r) {
+                la[r].load(arow + r * H * K + 32 * kp, RANK * H * K, cp.len, l);
+                lb[r].load(brow + r * H * K + 32 * kp, RANK * H * K, cp.len, l);
+            }
+            lg.tiles(scratch, cp.len, l, fg);
+            lk.tiles(scratch, cp.len, l, fk);
         }
+        lq.tiles(scratch, cp.len, l, fq);
+        if (!HD) {
+#pragma unroll
+            for (int r = 0; r < 2; ++r) { la[r].tiles(scratch, cp.len, l, fa[r]); lb[r].tiles(scratch, cp.len, l, fb[r]); }
+        }
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int kt = 2 * kp + e;
+            const f32x4 g4 = HD ? gks[HD ? kt : 0] : to_f32(fg[e]);
+            rq[kt] = fq[e];
+            if (HD) {
+                const f32x4 kk = to_f32(rk[kt]), f4 = exp4<T>(g4);
+                ra[0][kt] = to_frag<T>(kk * (-beta_t));
+                ra[1][kt] = to_frag<T>(kk * ((beta_t * s_t - f4) * beta_t));
+                rb[0][kt] = to_frag<T>(f4 * kk);
+                rb[1][kt] = rk[kt];
+            } else {
+                rk[kt] = fk[e];
+#pragma unroll
+                for (int r = 0; r < 2; ++r) { ra[r][kt] = fa[r][e]; rb[r][kt] = fb[r][e]; }
+            }
+            gi[kt] = scan16_incl(g4);
+            ge[kt] = gi[kt] - g4;
+            // Every score is a dense product of operands decayed relative to the middle of the chunk: exp(gi_i - gi_j) =
+            // exp(gi_i - m) exp(m - gi_j) with m = gi of token MID.  That is done here for every chunk, tile by tile as the
+            // inputs arrive; it is only valid while the exponents stay within +-SAFE_RANGE, which is checked afterwards.
+            const f32x4 m = bcast16<MID>(gi[kt]);
+            const f32x4 eq = exp4<T>(gi[kt] - m), ek = exp4<T>(m - gi[kt]), ea = exp4<T>(ge[kt] - m);
+            const f32x4 q4 = to_f32(rq[kt]), k4 = to_f32(rk[kt]);
+            const f32x4 a0 = to_f32(ra[0][kt]), a1 = to_f32(ra[1][kt]), b0 = to_f32(rb[0][kt]), b1 = to_f32(rb[1][kt]);
+            Split<T> qh, kh, ah[2], bh[2];
+            split(q4 * eq * scale, qh);
+            split(k4 * ek, kh);
+            split(a0 * ea, ah[0]);
+            split(a1 * ea, ah[1]);
+            split(b0 * ek, bh[0]);
+            split(b1 * ek, bh[1]);
+            aqk = mm3(qh, kh, aqk);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                aqb[s] = mm3(qh, bh[s], aqb[s]);
+                aak[s] = mm3(ah[s], kh, aak[s]);
+#pragma unroll
+                for (int r = 0; r < 2; ++r) aab[r][s] = mm3(ah[r], bh[s], aab[r][s]);
+            }
+        }
+    }
+#pragma unroll
+    for (int vp = 0; vp < VTW / 2; ++vp) {
+        Frag<T> f[2];
+        lv[vp].tiles(scratch, cp.len, l, f);
+        rv[2 * vp] = f[0];
+        rv[2 * vp + 1] = f[1];
     }
     // Each wave decides for its own channels (the parts of the score tiles add up whichever way they were formed); the
     // backward pass records the decision per (chunk, head) for the chunk_grad kernels.  Where a channel decays too
