@@ -70,6 +70,11 @@ template <typename T, int K, int V, int NWC> struct ScanCfg {
     static constexpr bool pipelined(bool with_o) { return KB <= 128 || (KB <= 256 && !(NWC == 8 && with_o)); }
     // ... and whether that includes the operands of the state update
     static constexpr bool early_update_reads(bool with_o) { return KB <= 128 || (KB <= 256 && NWC <= 4 && (NM == 0 || with_o)); }
+    // Issued a few at a time between the products, or all of them before the phase.  4-byte elements have twice the bytes and
+    // four times the cycles a product to hide them behind; with 2-byte ones it is not the issue of the reads that a step waits
+    // for.  Measured, before the phase -> spread: fp32 K = V = 64, 2 x 1003 tokens of 8 heads, records 45 -> 39 us, forward
+    // scan 22.5 -> 21.0, scan pair 27.7 -> 26.3; bf16 K = V = 128, 2 x 1537 tokens of 8 heads, records 25.6 -> 27.5, pair 82 -> 84.
+    static constexpr bool SPREAD = sizeof(T) == 4;
 };
 
 // A shared operand block as the loading waves see it: NI pieces of 1 KiB, lane l taking 16 bytes of each.  The
@@ -256,7 +261,7 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
     typedef ScanCfg<T, K, V, NWC> C;
     constexpr int KT = K / 16, KT2 = KT / 2, VT = V / 16, NM = C::NM, ES = sizeof(T);
     constexpr BlkF B = blk_fwd(K, sizeof(T), WRITE_O);
-    constexpr bool PIPE = C::pipelined(WRITE_O);
+    constexpr bool PIPE = C::pipelined(WRITE_O), SPREAD = C::SPREAD;
     constexpr bool PIPE_UPD = PIPE && C::early_update_reads(WRITE_O);
     constexpr int NIB = B.SIZE / 1024, SLOT = B.SIZE + C::OWN_FWD, NI = SLOT / 1024;
     constexpr bool OWN_LDS = C::OWN_FWD > 0;
@@ -391,45 +396,51 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
             egl[2 * kp + 1] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (2 * kp + 1) + 4 * g);
         };
         if (WRITE_O) {
-            if (PIPE) {
+            if (PIPE && !SPREAD) {
 #pragma unroll
                 for (int kp = 0; kp < KT2; ++kp) read_qg(kp);
             }
             ld_pair(reinterpret_cast<const T*>(slot + B.AQB), aqb[0], aqb[1]);
             aqk = ld_tile(reinterpret_cast<const T*>(slot + B.AQK));
         }
-        if (PIPE_UPD) {
+        if (PIPE_UPD && !SPREAD) {
 #pragma unroll
             for (int kp = 0; kp < KT2; ++kp) read_upd(kp);
         }
-        if (PIPE) __builtin_amdgcn_sched_barrier(0);      // the reads above stay above the products below
+        if (PIPE && !SPREAD) __builtin_amdgcn_sched_barrier(0);   // the reads above stay above the products below
         Frag<T> sb[KT];
-#pragma unroll
-        for (int kt = 0; kt < KT; ++kt) sb[kt] = to_frag<T>(S[kt]);
-        // v_new^T (rows value, inner token) = u^T + S^T w^T
+        // v_new^T (rows value, inner token) = u^T + S^T w^T; what is read on the way is used a group of products later or after
         f32x4 vn[2] = {to_f32(own.ut[0]), to_f32(own.ut[1])};
 #pragma unroll
         for (int kp = 0; kp < KT2; ++kp) {
+            if (PIPE && SPREAD && WRITE_O) read_qg(kp);
+            if (PIPE_UPD && SPREAD && !WRITE_O) read_upd(kp);
             if (!PIPE) read_w(slot, kp);
+            if (PIPE && SPREAD) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int kt = 2 * kp; kt < 2 * kp + 2; ++kt) {
+                sb[kt] = to_frag<T>(S[kt]);
                 vn[0] = mm(sb[kt], w[0][kt], vn[0]);
                 vn[1] = mm(sb[kt], w[1][kt], vn[1]);
             }
+            if (PIPE && SPREAD) __builtin_amdgcn_sched_barrier(0);
         }
         f32x4 o = zero4();
         if (WRITE_O) {
             // o (rows token, inner value) = qg S + A_qk v + sum_s A_qb^s v_new_s; the first two terms here
 #pragma unroll
             for (int kp = 0; kp < KT2; ++kp) {
+                if (PIPE_UPD && SPREAD) read_upd(kp);
                 if (!PIPE) read_qg(kp);
+                if (PIPE && SPREAD) __builtin_amdgcn_sched_barrier(0);
                 o = mm(qg[2 * kp], sb[2 * kp], o);
                 o = mm(qg[2 * kp + 1], sb[2 * kp + 1], o);
+                if (PIPE && SPREAD) __builtin_amdgcn_sched_barrier(0);
             }
             o = mm(aqk, own.vtt, o);
         }
-        if (PIPE) {
-            __builtin_amdgcn_sched_barrier(0);
+        if (PIPE) __builtin_amdgcn_sched_barrier(0);
+        if (PIPE && !SPREAD) {
             read_w_all(slot_next);                        // the products above have taken their operands already
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -455,6 +466,10 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
 #pragma unroll
         for (int kp = 0; kp < KT2; ++kp) {
             if (!PIPE_UPD) read_upd(kp);
+            if (PIPE && SPREAD) {                             // (those of phase 1, whose products have taken them already)
+                read_w(slot_next, kp);
+                __builtin_amdgcn_sched_barrier(0);
+            }
 #pragma unroll
             for (int kt = 2 * kp; kt < 2 * kp + 2; ++kt) {
                 f32x4 x = S[kt] * egl[kt];
@@ -463,6 +478,7 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
                 x = mm(vnb[1], bgt[1][kt], x);
                 S[kt] = x;
             }
+            if (PIPE && SPREAD) __builtin_amdgcn_sched_barrier(0);
         }
     };
 
@@ -551,7 +567,7 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
     constexpr SlotB B = slot_bwd(K, sizeof(T));
     constexpr int SBWD = blk_bwd(K, sizeof(T)).SIZE, NT = B.NIF;
     const int SFWD = p.ws.sa_stride;
-    constexpr bool PIPE = C::pipelined(false);
+    constexpr bool PIPE = C::pipelined(false), SPREAD = C::SPREAD;
     constexpr bool PIPE_UPD = PIPE && C::early_update_reads(false);
     constexpr int NI = B.SIZE / 1024, SLOT = B.SIZE;
     typedef ScanLds<T, K, V, NWC, SLOT, OUT> L;
@@ -649,32 +665,34 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
             egl[2 * kp] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (2 * kp) + 4 * g);
             egl[2 * kp + 1] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (2 * kp + 1) + 4 * g);
         };
-        if (PIPE_UPD) {
+        if (PIPE_UPD && !SPREAD) {
 #pragma unroll
             for (int kp = 0; kp < KT2; ++kp) read_upd(kp);
         }
-        if (PIPE) __builtin_amdgcn_sched_barrier(0);
-        else ld_pair(reinterpret_cast<const T*>(slot + B.AQBT), aq[0], aq[1]);
+        if (!PIPE) ld_pair(reinterpret_cast<const T*>(slot + B.AQBT), aq[0], aq[1]);
+        else if (!SPREAD) __builtin_amdgcn_sched_barrier(0);
         Frag<T> dsb[KT];
-#pragma unroll
-        for (int kt = 0; kt < KT; ++kt) dsb[kt] = to_frag<T>(dS[kt]);
         const int len = (int)min((int64_t)CH, eos - (bos + (int64_t)(cid - c0) * CH));
         if (c >= len || trans) don = zero_frag<T>();
         const Frag<T> doT = transpose(don, ident);          // rows value, inner token
-        // dv_new_s^T (rows value, inner token) = do^T A_qb^s + dS^T bg_s^T
+        // dv_new_s^T (rows value, inner token) = do^T A_qb^s + dS^T bg_s^T; what is read here is used a phase later
         f32x4 dvn[2];
         dvn[0] = mm(doT, aq[0], zero4());
         dvn[1] = mm(doT, aq[1], zero4());
 #pragma unroll
         for (int kp = 0; kp < KT2; ++kp) {
+            if (PIPE_UPD && SPREAD) read_upd(kp);
             if (!PIPE) read_bg(slot, kp);
+            if (PIPE && SPREAD) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int kt = 2 * kp; kt < 2 * kp + 2; ++kt) {
+                dsb[kt] = to_frag<T>(dS[kt]);
                 dvn[0] = mm(dsb[kt], bg[0][kt], dvn[0]);
                 dvn[1] = mm(dsb[kt], bg[1][kt], dvn[1]);
             }
+            if (PIPE && SPREAD) __builtin_amdgcn_sched_barrier(0);
         }
-        if (PIPE) {
+        if (PIPE && !SPREAD) {
             __builtin_amdgcn_sched_barrier(0);
             read_p1_all(slot_next);
             __builtin_amdgcn_sched_barrier(0);
@@ -693,6 +711,11 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
 #pragma unroll
         for (int kp = 0; kp < KT2; ++kp) {
             if (!PIPE_UPD) read_upd(kp);
+            if (PIPE && SPREAD) {                             // (those of phase 1, whose products have taken them already)
+                if (kp == 0) ld_pair(reinterpret_cast<const T*>(slot_next + B.AQBT), aq[0], aq[1]);
+                read_bg(slot_next, kp);
+                __builtin_amdgcn_sched_barrier(0);
+            }
 #pragma unroll
             for (int kt = 2 * kp; kt < 2 * kp + 2; ++kt) {
                 f32x4 x = dS[kt] * egl[kt];
@@ -701,6 +724,7 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
                 x = mm(dvb[1], wt[1][kt], x);
                 dS[kt] = x;
             }
+            if (PIPE && SPREAD) __builtin_amdgcn_sched_barrier(0);
         }
     };
 
