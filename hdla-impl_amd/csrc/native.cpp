@@ -198,7 +198,11 @@ inline bool number(PyObject* o, double& out) {
     if (out == -1.0 && PyErr_Occurred()) { PyErr_Clear(); return false; }
     return true;
 }
-inline bool gpu_like(const Tensor& t, const at::Device& dev) { return t.device() == dev && t.layout() == at::kStrided && !t.is_complex(); }
+// (a tensor that carries a forward-mode tangent or is the wrapper of a function transform goes to the Python code, whose autograd
+// functions refuse it: here a call without gradients would drop the tangent)
+inline bool gpu_like(const Tensor& t, const at::Device& dev) {
+    return t.device() == dev && t.layout() == at::kStrided && !t.is_complex() && t.has_storage() && !t._fw_grad(/*level=*/0).defined();
+}
 inline bool same_sizes(const Tensor& t, std::initializer_list<int64_t> s) { return t.sizes() == at::IntArrayRef(s); }
 
 // What the chunked and the token-serial operators have in common: q, k, v, gk, the states and the sequence table.
@@ -692,7 +696,7 @@ PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
         PyObject* o = PyTuple_GET_ITEM(a[1], i);
         if (!is_tensor(o)) return none();
         P[i] = unpack(o);
-        if (P[i].device() != dev || !P[i].is_contiguous()) return none();
+        if (!gpu_like(P[i], dev) || !P[i].is_contiguous()) return none();
         if (i == 8 ? (P[i].dim() != 1 || P[i].size(0) != d || !native_dtype(P[i].scalar_type()))
                    : (P[i].scalar_type() != at::kBFloat16 || !same_sizes(P[i], {shapes[i][0], shapes[i][1]}))) return none();
         any = any || wants_grad(P[i]);

@@ -143,3 +143,36 @@ def test_time_segments_of_the_stand_alone_scans(dtype, K, V, segments, T, cu, mo
     errs = [O.rel_l2(a, b) for a, b in zip(*res)]
     print([f"{e:.1e}" for e in errs], flush=True)
     assert max(errs) <= (6e-3 if dtype == torch.bfloat16 else 3e-6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("call", ["chunk", "recurrent", "norm", "layer"])
+@pytest.mark.parametrize("transform", ["dual", "vmap"])
+def test_forward_mode_and_transforms_are_refused(call, transform):
+    """The operators have no forward-mode rule: a tangent on an input that needs no gradient is refused, not dropped."""
+    import torch.autograd.forward_ad as fwad
+    from hdla_hip.layer import HDLA_Custom
+    from hdla_hip.normalize import normalize_fn
+    g = torch.Generator(device="cuda").manual_seed(2)
+    rn = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    q, a = rn(2, 1, 32, 2, 64), rn(1, 64, 2, 64)
+    layer = HDLA_Custom(256, 4, token_mixer_init_type=2, rescale_type=0).cuda().bfloat16().eval().requires_grad_(False)
+    w = torch.ones(64, device="cuda")
+
+    def run(x):
+        if call == "chunk":
+            return chunk_hrdplr_delta_rule(x, q[0], q[0], a, a, -q[0].abs(), 2, scale=1.0)[0]
+        if call == "recurrent":
+            return fused_recurrent_dplr_delta_rule(x, q[0], q[0], a, a, -q[0].abs(), 2, scale=1.0)[0]
+        if call == "norm":
+            return normalize_fn(x, w, gate=q[0], gate_pos="pre", c=8.0, eps=1e-5)
+        return layer(x)[0]
+
+    x = rn(2, 2, 32, 256) if call == "layer" else q
+    run(x[0])                                                 # accepted as it is
+    with pytest.raises((RuntimeError, NotImplementedError)):
+        if transform == "vmap":
+            torch.func.vmap(run)(x)
+        else:
+            with fwad.dual_level():
+                run(fwad.make_dual(x[0], torch.ones_like(x[0])))
