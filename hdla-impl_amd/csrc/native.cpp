@@ -40,7 +40,7 @@ struct Api {
     HDLA_FN(strerror); HDLA_FN(workspace_bytes); HDLA_FN(record_bytes); HDLA_FN(chunk_fwd_b); HDLA_FN(chunk_bwd_b);
     HDLA_FN(recurrent_fwd); HDLA_FN(param_recurrent_fwd); HDLA_FN(normalize_fwd); HDLA_FN(normalize_bwd);
     HDLA_FN(normalize_workspace_bytes); HDLA_FN(layer_pre_fwd); HDLA_FN(layer_pre_bwd); HDLA_FN(layer_up_fwd); HDLA_FN(layer_down);
-    HDLA_FN(layer_up_wgrad); HDLA_FN(layer_up_wgrad_workspace_bytes); HDLA_FN(rows_gemm); HDLA_FN(sum_partials);
+    HDLA_FN(layer_up_wgrad); HDLA_FN(layer_up_wgrad_workspace_bytes); HDLA_FN(rows_gemm); HDLA_FN(sum_partials); HDLA_FN(stack_rows);
 #undef HDLA_FN
 } api;
 PyObject* error_class = nullptr;                 // _lib.HdlaError
@@ -496,10 +496,16 @@ constexpr int64_t PAD_FROM_ROWS = 1024;
 
 // the concatenated projection weight [ld, d]; rows behind the last projection are zero
 Tensor gather_weights(const Tensor* w, const LayerCols& L) {       // wq, wk, wv, wf0, wg0, wbeta
-    Tensor out = at::empty({L.ld, L.d}, w[0].options());
-    std::vector<Tensor> parts{w[0], w[1], w[2], w[3], w[4], w[5]};
-    if (L.ld > L.used) parts.push_back(at::zeros({L.ld - L.used, L.d}, w[0].options()));
-    at::cat_out(out, parts, 0);
+    const Tensor out = at::empty({L.ld, L.d}, w[0].options());
+    const void* parts[6];
+    int64_t rows[6];
+    std::vector<Tensor> whole(6);                                  // (a parameter may be a view at any address)
+    for (int i = 0; i < 6; ++i) {
+        whole[i] = reinterpret_cast<uintptr_t>(w[i].data_ptr()) % 16 ? w[i].detach().clone() : w[i];
+        parts[i] = whole[i].data_ptr();
+        rows[i] = whole[i].size(0);
+    }
+    check(api.stack_rows(parts, rows, 6, L.d, ptr(out), L.ld, stream_of(out)), "hdla_stack_rows");
     return out;
 }
 hdla_pre_dims pre_dims(const LayerCols& L, const LayerCfg& f, int64_t rows) {
@@ -760,7 +766,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HDLA_FN(strerror) HDLA_FN(workspace_bytes) HDLA_FN(record_bytes) HDLA_FN(chunk_fwd_b) HDLA_FN(chunk_bwd_b)
     HDLA_FN(recurrent_fwd) HDLA_FN(param_recurrent_fwd) HDLA_FN(normalize_fwd) HDLA_FN(normalize_bwd)
     HDLA_FN(normalize_workspace_bytes) HDLA_FN(layer_pre_fwd) HDLA_FN(layer_pre_bwd) HDLA_FN(layer_up_fwd) HDLA_FN(layer_down)
-    HDLA_FN(layer_up_wgrad) HDLA_FN(layer_up_wgrad_workspace_bytes) HDLA_FN(rows_gemm) HDLA_FN(sum_partials)
+    HDLA_FN(layer_up_wgrad) HDLA_FN(layer_up_wgrad_workspace_bytes) HDLA_FN(rows_gemm) HDLA_FN(sum_partials) HDLA_FN(stack_rows)
 #undef HDLA_FN
     Py_INCREF(a[1]);
     Py_XDECREF(error_class);

@@ -9,7 +9,7 @@ from typing import Optional
 import torch
 
 HDLA_BF16, HDLA_FP32 = 0, 1
-HDLA_VERSION = 202          # the header this binding was written against (struct layouts, entry points)
+HDLA_VERSION = 203          # the header this binding was written against (struct layouts, entry points)
 ROUTE_AUTO, ROUTE_CLASSIC, ROUTE_FUSED = 0, 1, 2
 _ROUTES = {"": ROUTE_AUTO, "auto": ROUTE_AUTO, "classic": ROUTE_CLASSIC, "fused": ROUTE_FUSED}
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -148,6 +148,8 @@ def load():
     lib.hdla_rows_gemm.argtypes = [ctypes.c_int32] * 3 + [P, ctypes.c_int64, P, ctypes.c_int64, P, ctypes.c_int64, P]
     lib.hdla_sum_partials.restype = ctypes.c_int
     lib.hdla_sum_partials.argtypes = [P, ctypes.c_int32, ctypes.c_int64, P, P]
+    lib.hdla_stack_rows.restype = ctypes.c_int
+    lib.hdla_stack_rows.argtypes = [P, P, ctypes.c_int32, ctypes.c_int64, P, ctypes.c_int64, P]
     _lib = lib
     return lib
 

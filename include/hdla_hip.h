@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-#define HDLA_VERSION 202
+#define HDLA_VERSION 203
 
 enum { HDLA_BF16 = 0, HDLA_FP32 = 1 };
 
@@ -305,6 +305,9 @@ size_t hdla_skinny_wgrad_workspace_bytes(int dtype, int64_t M, int32_t N, int32_
 /* out [n] (bf16) = sum of `count` consecutive fp32 partial results part [count][n], added in order; n a multiple of 8,
  * both 16-byte aligned: the second half of a product whose contraction was split. */
 int hdla_sum_partials(const float* part, int32_t count, int64_t n, void* out, void* stream);
+/* out [total_rows, width] (2-byte elements) = the rows of parts[0 .. count) one part behind the other, parts[m] being [rows[m], width],
+ * then zeros; count <= 8, width a multiple of 8, everything contiguous and 16-byte aligned.  parts and rows are host arrays. */
+int hdla_stack_rows(const void* const* parts, const int64_t* rows, int32_t count, int64_t width, void* out, int64_t total_rows, void* stream);
 
 /* The second halves of the layer's two low-rank projections (f_proj and output_gate, HRDPLR/hdla_custom.py:117-121,151-155)
  * with log_f = logsigmoid(f) (:219), bf16.  Their inner activations are column ranges col_f .. + D and col_g .. + D of

@@ -60,3 +60,20 @@ def test_rows_gemm(M, N, K):
     assert bool((y[M:] == 7.0).all() and (y[:, N:] == 7.0).all())
     assert lib.hdla_rows_gemm(65, N, K, P(x), K + 8, P(w), K, P(y), N + 4, st) == -2
     assert lib.hdla_rows_gemm(M, N, K - 8, P(x), K + 8, P(w), K, P(y), N + 4, st) == -2
+
+
+@pytest.mark.parametrize("rows,width,pad", [((1,), 8, 0), ((3, 0, 5), 24, 1), ((64, 64, 64, 16, 16, 4), 256, 12), ((129, 1, 1, 1, 1, 1, 1, 1), 1016, 0),
+                                            ((1024, 1024, 1024, 64, 64, 16), 1024, 112)])
+def test_stacked_rows(rows, width, pad):
+    """Whole pieces copied, so bit for bit; what lies behind the output stays."""
+    lib, st = _lib.load(), _lib.current_stream(DEV)
+    parts = [_rn(7 + i, r, width) for i, r in enumerate(rows)]
+    total = sum(rows) + pad
+    buf = torch.full(((total + 3) * width,), 7.0, dtype=torch.bfloat16, device=DEV)
+    pp = (ctypes.c_void_p * len(rows))(*[t.data_ptr() for t in parts])
+    rr = (ctypes.c_int64 * len(rows))(*rows)
+    assert lib.hdla_stack_rows(pp, rr, len(rows), width, P(buf), total, st) == 0
+    want = torch.cat(parts + [torch.zeros(pad, width, dtype=torch.bfloat16, device=DEV)])
+    assert torch.equal(buf[:total * width].view(total, width), want) and (buf[total * width:] == 7.0).all()
+    assert lib.hdla_stack_rows(pp, rr, len(rows), width, P(buf), sum(rows) - 1, st) != 0
+    assert lib.hdla_stack_rows(pp, rr, len(rows), width - 1, P(buf), total, st) != 0
