@@ -16,6 +16,7 @@
 #include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/GradMode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <dlfcn.h>
 #include <torch/csrc/Exceptions.h>
@@ -602,6 +603,9 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
         return in_backward([&] { return gradients(ctx, grads); });
     }
     static variable_list gradients(AutogradContext* ctx, const variable_list& grads) {
+        // backward() may be called inside an autocast region although the forward pass ran outside one.  The engine carries that
+        // state to this thread, and torch's products below would come out in the region's type where kernels read bf16.
+        const c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::DispatchKey::AutocastCUDA);
         const auto s = ctx->get_saved_variables();
         const Tensor &x = s[0], &w = s[1], &y = s[2], &f = s[3], &g = s[4], &o = s[5], &n = s[6], &boundary = s[7];
         const Tensor &q = s[8], &k = s[9], &v = s[10], &beta = s[11], &gk = s[12], &h0 = s[13], &wf1 = s[14], &wg1 = s[15], &wnorm = s[16],

@@ -1,0 +1,58 @@
+"""The native host path in the surroundings a training program puts it in: autocast, activation checkpointing, hooks, parameters at
+any address, more than one stream, more than one thread."""
+import sys
+import threading
+import time
+
+import pytest
+import torch
+import torch.nn as nn
+
+from hdla_hip import _lib, chunk_hdla_delta_rule, chunk_hrdplr_delta_rule
+from hdla_hip.layer import HDLA_Custom, RecurrentCache
+from hdla_hip.normalize import normalize_fn
+from hdla_hip.synthetic import make_inputs
+from oracle import hrdplr_oracle as O
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _layer(d=256, H=4, **kw):
+    torch.manual_seed(3)
+    return HDLA_Custom(d, H, token_mixer_init_type=2, rescale_type=0, **kw).to(DEV).bfloat16().train()
+
+
+def _x(B, T, d=256, seed=4, grad=True):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randn(B, T, d, generator=g).bfloat16().to(DEV).requires_grad_(grad), torch.randn(B, T, d, generator=g).bfloat16().to(DEV)
+
+
+def _operands(T=70, H=2, K=64, seed=41):
+    x = make_inputs(seed, 1, T, H, K, K)
+    return [t.bfloat16().to(DEV).requires_grad_() for t in (x.q, x.k, x.v, x.a, x.b, x.gk)], x.do.bfloat16().to(DEV)
+
+
+# ---- autocast -------------------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("what", ["layer", "operator", "norm"])
+def test_backward_inside_an_autocast_region(what, dtype):
+    """A forward pass outside autocast (or in a region that switches it off) and backward() inside one, whose products torch
+    would run in that region's type: the gradients are those of a backward pass outside."""
+    if what == "layer":
+        m, (x, do) = _layer(), _x(2, 40)
+        leaves, run = [x] + list(m.parameters()), lambda: m(x)[0]
+    elif what == "operator":
+        leaves, do = _operands()
+        run = lambda: chunk_hrdplr_delta_rule(*leaves, 2, scale=0.5)[0]
+    else:
+        (x, do), (gate, _) = _x(2, 40), _x(2, 40, seed=5)
+        w = torch.ones(256, device=DEV, requires_grad=True)
+        leaves, run = [x, gate, w], lambda: normalize_fn(x, w, gate=gate, gate_pos="pre", c=16.0, eps=1e-5)
+    ref = torch.autograd.grad(run(), leaves, do)
+    with torch.autocast("cuda", dtype=dtype):
+        with torch.autocast("cuda", enabled=False):
+            y = run()
+        got = torch.autograd.grad(y, leaves, do)
+    for a, b in zip(ref, got):
+        assert a.dtype == b.dtype and torch.equal(a, b)
