@@ -245,10 +245,10 @@ void bind_ws(ChunkArgs<T>& a, const hdla_dims* d, const WsLayout& LP, void* prep
 
 template <typename T> PackedOut packed_outputs(const hdla_dims* d, const ChunkArgs<T>& a) {
     PackedOut out{};
-    const long long rows = (long long)d->T * d->H, k = rows * d->K * sizeof(T), v = rows * d->V * sizeof(T);
+    const long long H = d->H, k = H * d->K * (long long)sizeof(T), v = H * d->V * (long long)sizeof(T);
     out.add(a.o, v);
     out.add(a.dq, k); out.add(a.dk, k); out.add(a.dv, v); out.add(a.da, 2 * k); out.add(a.db, 2 * k);
-    out.add(a.dgk, rows * d->K * (a.gk_f32 ? 4 : 2)); out.add(a.dbeta, rows * sizeof(T));
+    out.add(a.dgk, H * d->K * (a.gk_f32 ? 4 : 2)); out.add(a.dbeta, H * (long long)sizeof(T));
     return out;
 }
 

@@ -10,9 +10,9 @@ namespace hdla {
 // tokens (it may come unchecked from the device) leaves rows that belong to none, and these are to read as zeros.
 struct PackedOut {
     void* p[7];
-    long long bytes[7];       // multiples of 2
+    long long row[7];         // bytes a token, multiples of 2
     int n;
-    void add(void* q, long long b) { if (q) { p[n] = q; bytes[n++] = b; } }
+    void add(void* q, long long b) { if (q) { p[n] = q; row[n++] = b; } }
 };
 hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int32_t* chunk_off, int32_t* chunk_seq, const PackedOut& out,
                               hipStream_t stream);
