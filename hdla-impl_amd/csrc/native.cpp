@@ -204,6 +204,7 @@ inline bool number(PyObject* o, double& out) {
 inline bool gpu_like(const Tensor& t, const at::Device& dev) {
     return t.device() == dev && t.layout() == at::kStrided && !t.is_complex() && t.has_storage() && !t._fw_grad(/*level=*/0).defined();
 }
+inline bool off_grid(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0; }
 inline bool same_sizes(const Tensor& t, std::initializer_list<int64_t> s) { return t.sizes() == at::IntArrayRef(s); }
 
 // What the chunked and the token-serial operators have in common: q, k, v, gk, the states and the sequence table.
@@ -502,7 +503,7 @@ Tensor gather_weights(const Tensor* w, const LayerCols& L) {       // wq, wk, wv
     int64_t rows[6];
     std::vector<Tensor> whole(6);                                  // (a parameter may be a view at any address)
     for (int i = 0; i < 6; ++i) {
-        whole[i] = reinterpret_cast<uintptr_t>(w[i].data_ptr()) % 16 ? w[i].detach().clone() : w[i];
+        whole[i] = off_grid(w[i]) ? w[i].detach().clone() : w[i];
         parts[i] = whole[i].data_ptr();
         rows[i] = whole[i].size(0);
     }
@@ -526,9 +527,10 @@ hdla_up_dims up_dims(const LayerCols& L, int64_t rows) {
 // x w^T.  For the few rows of a decode step by hdla_rows_gemm, which is a launch where the BLAS call is 19 us of host time
 // (measured, us, here / there: 16 x 1024 x 1024 4.5/19, 16 x 6416 x 2048 12/19, 16 x 4096 x 4096 12/19, 64 x 2048 x 2048 13/19;
 // beyond the products below the GPU's own time decides, and the BLAS kernels' larger tiles with it: 1 x 12576 x 4096 35/26).
+constexpr int64_t FEW_ROWS = 64;
 Tensor project(const Tensor& x, const Tensor& w) {
     const int64_t M = x.size(0), tiles = M <= 16 ? 1 : M <= 32 ? 2 : 4;
-    if (M > 64 || tiles * w.numel() > (int64_t(32) << 20)) return at::mm(x, w.t());
+    if (M > FEW_ROWS || tiles * w.numel() > (int64_t(32) << 20)) return at::mm(x, w.t());
     const Tensor y = at::empty({x.size(0), w.size(0)}, x.options());
     check(api.rows_gemm((int32_t)x.size(0), (int32_t)w.size(0), (int32_t)w.size(1), ptr(x), x.stride(0), ptr(w), w.stride(0), ptr(y), y.stride(0),
                         stream_of(x)), "hdla_rows_gemm");
@@ -712,6 +714,10 @@ PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
         any = any || wants_grad(P[i]);
         op_grad = op_grad || ((i < 4 || i == 5 || i == 6) && wants_grad(P[i]));
     }
+    // Kernels of this library read these 16 bytes at a time; the BLAS calls of the Python code take them at any address.  (The
+    // weights that multiply x are copied together anyway, gather_weights.)
+    const bool few = B * T <= FEW_ROWS;
+    if (off_grid(P[6]) || off_grid(P[7]) || (few && (off_grid(P[9]) || (x.is_contiguous() && off_grid(x))))) return none();
     Tensor h0;
     if (a[2] != Py_None) {
         if (!is_tensor(a[2])) return none();
