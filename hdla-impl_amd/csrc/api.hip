@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 
 #include "fused_shapes.h"
@@ -73,11 +74,14 @@ int fused_segments(const hdla_dims* d) {
 // chunks 812/896 -> 142/278 (16); bf16, K=V=128, 16 lanes of 313 chunks 293/546 -> 192/546 (8 and 1); bf16, K=128 V=64,
 // 8 lanes of 500 chunks 377/509 -> 154/352 (16 and 8).
 constexpr int SCAN_MAX_SEGMENTS = 32;
+// Records (lanes x segments) of a segment count asked for: a record is a state and a matrix of K x K, a few of them per pass, and
+// a sequence's segments share a grid dimension with the sequences (65535).  The device is full long before this many.
+constexpr long long SCAN_MAX_RECORDS = 4096;
 int scan_segments(const hdla_dims* d, bool bwd) {
     if (d->route != HDLA_ROUTE_AUTO) return 1;
-    if (d->segments > 0) return d->segments < SCAN_MAX_SEGMENTS ? d->segments : SCAN_MAX_SEGMENTS;
-    const bool f32 = d->in_dtype == HDLA_FP32;
     const long long lanes = (long long)d->N * d->H;
+    if (d->segments > 0) return (int)std::max(1LL, std::min<long long>({d->segments, SCAN_MAX_SEGMENTS, SCAN_MAX_RECORDS / lanes}));
+    const bool f32 = d->in_dtype == HDLA_FP32;
     const long long chunks = ((d->T + CHUNK - 1) / CHUNK) / (d->cu_seqlens ? d->N : 1);
     // lanes x segments: beyond 128 the records' launch needs more than one round on the device.  The backward scans of
     // 2-byte inputs are bound by their traffic from a dozen lanes on, and the reverse records come on top: fewer there.

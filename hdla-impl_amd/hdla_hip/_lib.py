@@ -198,7 +198,8 @@ def default_route() -> int:
 
 
 def default_segments() -> int:
-    """Time segments per sequence on the fused route: environment variable HDLA_HIP_SEGMENTS, 0 = the library chooses."""
+    """Time segments per sequence, of the fused kernels and of the stand-alone scans: environment variable HDLA_HIP_SEGMENTS,
+    0 = the library chooses."""
     return int(os.environ.get("HDLA_HIP_SEGMENTS", "0"))
 
 

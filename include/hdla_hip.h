@@ -80,7 +80,8 @@ typedef struct hdla_dims {
     float scale;               /* applied to q (HRDPLR/hrdplr.py:302) */
     const int64_t* cu_seqlens; /* DEVICE int64[N+1] cumulative sequence starts on the T axis, or NULL */
     int32_t route;             /* HDLA_ROUTE_*; 0 = the library chooses */
-    int32_t segments;          /* fused route: time segments per sequence (at most 64); 0 = the library chooses */
+    int32_t segments;          /* time segments per sequence; 0 = the library chooses.  Fused route: at most 64.  Scans of the
+                                * classic kernels under HDLA_ROUTE_AUTO: at most 32, and 4096 over all sequences and heads */
 } hdla_dims;
 
 /* Byte offsets of the named intermediates inside the workspace (0 = not part of this pass); for tests and

@@ -121,6 +121,18 @@ def test_bad_dims_are_rejected_before_launch(kw, code):
     assert len(lib.hdla_strerror(rc)) > 8
 
 
+@pytest.mark.parametrize("N,H,asked,want", [(1, 2, 7, 7), (4, 16, 100, 32), (256, 16, 32, 1), (100, 8, 32, 5), (4096, 1, 32, 1),
+                                            (65535, 1, 32, 1), (65535, 16, 1000, 1)])
+def test_segments_asked_for_of_the_stand_alone_scans_are_bounded(N, H, asked, want):
+    """A segment count meant for the fused route reaches the scans as well: their records stay few (grids of N x segments
+    and workspaces with them), down to whole sequences for many sequences."""
+    K = V = 128
+    size = lambda segments: _lib.load().hdla_workspace_bytes(ctypes.byref(_lib.HdlaDims(N, 32, H, K, V, 2, N, 0, 0, 1.0, None, 0, segments)), 0)
+    record = (2 * K * V + K * K) * 4
+    assert size(asked) - size(1) == (N * H * want * record if want > 1 else 0)
+
+
+
 def test_null_misaligned_and_small_workspace():
     lib = _lib.load()
     d = _dims()
