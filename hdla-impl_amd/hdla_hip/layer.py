@@ -302,21 +302,34 @@ class HDLA_Custom(nn.Module):
         return q, k, v, beta, log_f, gate0
 
     def _native_params(self):
-        """Parameters for the native call, or None where a submodule has been replaced or carries hooks."""
-        mods = self._modules
-        f, g, norm = mods["f_proj"], mods["output_gate"], mods["norm"]
-        if type(f) is not nn.Sequential or type(g) is not nn.Sequential or type(norm) not in (RMSNormFusedGate, GroupRMSNormFusedGate):
+        """Parameters for the native call, or None where something that it stands in for has been replaced or carries hooks."""
+        own, cls = self.__dict__, type(self)
+        if (cls.project is not _PROJECT or cls._up is not _UP or cls._gathered is not _GATHERED or "project" in own or "_up" in own
+                or "_gathered" in own or nn.Linear.forward is not _LINEAR or nn.Module.__call__ is not _MODULE_CALL):
             return None
-        out = []
-        for m in (mods["q_proj"], mods["k_proj"], mods["v_proj"], f._modules["0"], g._modules["0"], mods["bet_proj"], f._modules["1"],
-                  g._modules["1"], norm, mods["o_proj"]):
-            if ((m is not norm and type(m) is not nn.Linear) or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
-                    or m._backward_pre_hooks):
+        if not own["use_beta"] or not own["use_output_gate"] or own["use_offset"] or own["num_blocks"] != 1 or any(_GLOBAL_HOOKS):
+            return None
+        mods = own["_modules"]
+        f, g, norm = mods.get("f_proj"), mods.get("output_gate"), mods.get("norm")
+        if type(f) is not nn.Sequential or type(g) is not nn.Sequential or len(f._modules) != 2 or len(g._modules) != 2:
+            return None
+        if type(norm) not in _NORMS or type(norm).forward is not _NORMS[type(norm)]:
+            return None
+        if norm.gate_act != "sigmoid" or norm.gate_pos not in ("pre", "post"):
+            return None
+        (f0, f1), (g0, g1), out = f._modules.values(), g._modules.values(), []
+        for m in (mods.get("q_proj"), mods.get("k_proj"), mods.get("v_proj"), f0, g0, mods.get("bet_proj"), f1, g1, norm,
+                  mods.get("o_proj")):
+            if type(m) is not nn.Linear and m is not norm:
                 return None
-            p = m._parameters
-            if p["weight"] is None or p.get("bias") is not None:
+            d = m.__dict__
+            if "forward" in d or d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"]:
                 return None
-            out.append(p["weight"])
+            p = d["_parameters"]
+            w = p.get("weight")
+            if w is None or p.get("bias") is not None:
+                return None
+            out.append(w)
         return tuple(out)
 
     def _forward_native(self, x, state, use_cache):
@@ -324,13 +337,13 @@ class HDLA_Custom(nn.Module):
         params = self._native_params()
         if params is None:
             return None
-        norm, grouped = self.norm, type(self.norm) is GroupRMSNormFusedGate
-        groups = norm.num_groups if grouped else 1
+        norm = self.norm
+        groups, width = (norm.num_groups, norm.num_channels) if type(norm) is GroupRMSNormFusedGate else (1, norm.dim)
         mode = 0 if self.dispatch == "auto" else (1 if self.training or use_cache else 2)
         return _lib.native().layer(
             x, params, state, bool(use_cache), mode, None if self.training else self._native_cache, self.num_heads, groups,
             bool(self.norm_q), bool(self.norm_v), 2.0 if self.beta_activation == "neg" else 1.0,
-            (self.embed_dim // groups) ** 0.5, norm.eps, 1 if norm.gate_pos == "pre" else 2)
+            (width // groups) ** 0.5, norm.eps, 1 if norm.gate_pos == "pre" else 2)
 
     def forward(self, x, attention_mask: Optional[torch.Tensor] = None, past_key_values=None,
                 use_cache: Optional[bool] = False, lower_bound: Optional[torch.Tensor] = None, **kwargs):
@@ -380,3 +393,12 @@ class HDLA_Custom(nn.Module):
         else:
             output = self.norm(output)
         return self.o_proj(output), past_key_values
+
+
+# What the native call stands in for, as written here and in torch: it steps back where any of it is another function by now (a
+# subclass or an instance that overrides a step, a module whose forward has been replaced, a patched class).
+_PROJECT, _UP, _GATHERED = HDLA_Custom.project, HDLA_Custom._up, HDLA_Custom._gathered
+_NORMS = {t: t.forward for t in (RMSNormFusedGate, GroupRMSNormFusedGate)}
+_LINEAR, _MODULE_CALL = nn.Linear.forward, nn.Module.__call__
+_GLOBAL_HOOKS = [getattr(nn.modules.module, n, {}) for n in ("_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks",
+                                                            "_global_backward_pre_hooks")]
