@@ -280,6 +280,20 @@ PyObject* pair(const Tensor& a, const Tensor& b) {
     return r;
 }
 
+// The interpreter lock is given back while a call allocates and launches, as torch's own operators do: nothing in between touches
+// a Python object (what does, such as a saved-tensor hook, takes the lock itself).
+struct Unlocked {
+    PyThreadState* const state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+    Unlocked() = default;
+    Unlocked(const Unlocked&) = delete;
+    Unlocked& operator=(const Unlocked&) = delete;
+};
+template <typename F> auto unlocked(F fn) {
+    const Unlocked u;
+    return fn();
+}
+
 // runs fn, turning C++ exceptions into Python ones
 template <typename F> PyObject* guarded(F fn) {
     try {
@@ -290,6 +304,8 @@ template <typename F> PyObject* guarded(F fn) {
         PyErr_SetString(memory_error ? memory_error : PyExc_MemoryError, e.what_without_backtrace());
     } catch (const c10::Error& e) {
         PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
+    } catch (python_error& e) {                           // raised by Python code on the way (a saved-tensor hook)
+        e.restore();
     } catch (const std::exception& e) {
         if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
     }
@@ -306,15 +322,20 @@ PyObject* run_chunk(ChunkIn& x, PyObject* pscale, PyObject* pwant, PyObject* pke
     hdla_dims d;
     return guarded([&]() -> PyObject* {
         if (!chunk_dims(x, scale, d)) return none();
-        const at::DeviceGuard guard(x.q.device());
-        make_contiguous(x);
-        if (any_grad(x)) {
-            const auto r = ChunkFn::apply(x.q, x.k, x.v, maybe(x.a), maybe(x.b), maybe(x.beta), x.gk, maybe(x.h0), maybe(x.cu), scale, want);
-            return pair(r[0], want ? r[1] : Tensor());
-        }
-        if (x.h0.defined()) x.h0 = x.h0.to(at::kFloat).contiguous();
-        Tensor o, ht, boundary;
-        chunk_forward(x, d, want, false, o, ht, boundary);
+        Tensor o, ht;
+        unlocked([&] {
+            const at::DeviceGuard guard(x.q.device());
+            make_contiguous(x);
+            if (any_grad(x)) {
+                const auto r = ChunkFn::apply(x.q, x.k, x.v, maybe(x.a), maybe(x.b), maybe(x.beta), x.gk, maybe(x.h0), maybe(x.cu), scale, want);
+                o = r[0];
+                if (want) ht = r[1];
+                return;
+            }
+            if (x.h0.defined()) x.h0 = x.h0.to(at::kFloat).contiguous();
+            Tensor boundary;
+            chunk_forward(x, d, want, false, o, ht, boundary);
+        });
         return pair(o, ht);
     });
 }
@@ -348,18 +369,20 @@ PyObject* run_recurrent(ChunkIn& x, PyObject* pscale, PyObject* pwant, PyObject*
     hdla_dims d;
     return guarded([&]() -> PyObject* {
         if (!chunk_dims(x, scale, d)) return none();
-        const at::DeviceGuard guard(x.q.device());
-        make_contiguous(x);
-        if (x.h0.defined()) x.h0 = x.h0.to(at::kFloat).contiguous();
-        const Tensor o = x.cu.defined() ? at::zeros_like(x.v) : at::empty_like(x.v);     // rows of no sequence stay zero
-        Tensor ht;
-        if (want) ht = at::empty({d.N, d.H, d.K, d.V}, x.q.options().dtype(at::kFloat));
-        if (x.beta.defined())
-            check(api.param_recurrent_fwd(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.beta), ptr(x.gk), reverse, fptr(x.h0), ptr(o), fptr(ht),
-                                          stream_of(x.q)), "hdla_param_recurrent_fwd");
-        else
-            check(api.recurrent_fwd(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.gk), reverse, fptr(x.h0), ptr(o), fptr(ht),
-                                    stream_of(x.q)), "hdla_recurrent_fwd");
+        Tensor o, ht;
+        unlocked([&] {
+            const at::DeviceGuard guard(x.q.device());
+            make_contiguous(x);
+            if (x.h0.defined()) x.h0 = x.h0.to(at::kFloat).contiguous();
+            o = x.cu.defined() ? at::zeros_like(x.v) : at::empty_like(x.v);      // rows of no sequence stay zero
+            if (want) ht = at::empty({d.N, d.H, d.K, d.V}, x.q.options().dtype(at::kFloat));
+            if (x.beta.defined())
+                check(api.param_recurrent_fwd(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.beta), ptr(x.gk), reverse, fptr(x.h0), ptr(o), fptr(ht),
+                                              stream_of(x.q)), "hdla_param_recurrent_fwd");
+            else
+                check(api.recurrent_fwd(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.gk), reverse, fptr(x.h0), ptr(o), fptr(ht),
+                                        stream_of(x.q)), "hdla_recurrent_fwd");
+        });
         return pair(o, ht);
     });
 }
@@ -458,13 +481,15 @@ PyObject* py_normalize(PyObject*, PyObject* const* a, Py_ssize_t n) {
     double c = 0, eps = 0;
     if (!number(a[7], c) || !number(a[8], eps)) return none();
     return guarded([&]() -> PyObject* {
-        const at::DeviceGuard guard(dev);
-        x = x.contiguous();
-        if (w.defined()) w = w.contiguous();
-        if (gate.defined()) gate = gate.contiguous();
-        if (c10::GradMode::is_enabled() && (wants_grad(x) || wants_grad(w) || wants_grad(gate)))
-            return THPVariable_Wrap(NormFn::apply(x, maybe(w), maybe(gate), pos, c, eps, groups));
-        return THPVariable_Wrap(norm_forward(x, w, gate, norm_dims(x, w, (int)pos, c, eps, groups)));
+        return THPVariable_Wrap(unlocked([&] {
+            const at::DeviceGuard guard(dev);
+            x = x.contiguous();
+            if (w.defined()) w = w.contiguous();
+            if (gate.defined()) gate = gate.contiguous();
+            if (c10::GradMode::is_enabled() && (wants_grad(x) || wants_grad(w) || wants_grad(gate)))
+                return NormFn::apply(x, maybe(w), maybe(gate), pos, c, eps, groups);
+            return norm_forward(x, w, gate, norm_dims(x, w, (int)pos, c, eps, groups));
+        }));
     });
 }
 
@@ -732,31 +757,43 @@ PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     hdla_dims probe{};
     if (!route_and_segments(probe)) return none();
     return guarded([&]() -> PyObject* {
-        const at::DeviceGuard guard(dev);
+        Tensor out, ht;
         if (grad) {
-            const auto r = LayerFn::apply(x, P[0], P[1], P[2], P[3], P[4], P[5], P[6], P[7], P[8], P[9], maybe(h0), f, want);
-            return pair(r[0], want ? r[1] : Tensor());
+            unlocked([&] {
+                const at::DeviceGuard guard(dev);
+                const auto r = LayerFn::apply(x, P[0], P[1], P[2], P[3], P[4], P[5], P[6], P[7], P[8], P[9], maybe(h0), f, want);
+                out = r[0];
+                if (want) ht = r[1];
+            });
+            return pair(out, ht);
         }
         LayerFwd r;
         const LayerCols L(d, f.H, B * T >= PAD_FROM_ROWS);
-        if (PyList_CheckExact(a[5]) && PyList_GET_SIZE(a[5]) == 2) {
-            // the weight of the last call, as long as the parameters are the ones it was built from, unmodified
-            struct { const void* p; uint64_t v; } key[7];
+        // the weight of the last call, as long as the parameters are the ones it was built from, unmodified
+        const bool cached = PyList_CheckExact(a[5]) && PyList_GET_SIZE(a[5]) == 2;
+        struct { const void* p; uint64_t v; } key[7];
+        if (cached) {
             for (int i = 0; i < 6; ++i) key[i] = {P[i].data_ptr(), (uint64_t)P[i]._version()};
             key[6] = {nullptr, (uint64_t)L.ld};
             PyObject *old_key = PyList_GET_ITEM(a[5], 0), *old = PyList_GET_ITEM(a[5], 1);
             if (PyBytes_CheckExact(old_key) && PyBytes_GET_SIZE(old_key) == (Py_ssize_t)sizeof key &&
-                !memcmp(PyBytes_AS_STRING(old_key), key, sizeof key) && is_tensor(old)) {
-                r.w = unpack(old);
-            } else {
-                r.w = gather_weights(P, L);
-                PyList_SetItem(a[5], 0, PyBytes_FromStringAndSize(reinterpret_cast<const char*>(key), sizeof key));
-                PyList_SetItem(a[5], 1, THPVariable_Wrap(r.w));
-            }
-        } else {
-            r.w = gather_weights(P, L);
+                !memcmp(PyBytes_AS_STRING(old_key), key, sizeof key) && is_tensor(old)) r.w = unpack(old);
         }
-        layer_forward(x, P, f, h0, want, chunked, false, r);
+        const bool built = !r.w.defined();
+        unlocked([&] {
+            const at::DeviceGuard guard(dev);
+            if (built) r.w = gather_weights(P, L);
+            layer_forward(x, P, f, h0, want, chunked, false, r);
+        });
+        if (cached && built && PyList_GET_SIZE(a[5]) == 2) {
+            // (key and weight one behind the other, with the lock held: another thread sees both or neither)
+            PyObject* const k = PyBytes_FromStringAndSize(reinterpret_cast<const char*>(key), sizeof key);
+            if (!k) return nullptr;
+            PyObject* const w = THPVariable_Wrap(r.w);
+            if (!w) { Py_DECREF(k); return nullptr; }
+            PyList_SetItem(a[5], 0, k);
+            PyList_SetItem(a[5], 1, w);
+        }
         return pair(r.out, r.ht);
     });
 }

@@ -91,3 +91,58 @@ def test_layer_tensors_off_the_16_byte_grid(which, B, T):
     # (the same products by other kernels: their results may round to another bf16 value, and so on down the layer)
     for a, b in zip(ref, both(x)):
         assert O.rel_l2(b, a) <= 2e-2
+
+
+@pytest.mark.parametrize("call", ["chunk", "chunk_grad", "chunk_hdla", "recurrent", "normalize", "layer"])
+def test_other_threads_run_during_a_call(call):
+    """A native call gives the interpreter lock back while it allocates and launches, as torch's own operators do."""
+    x = make_inputs(42, 1, 64, 2, 64, 64)
+    t = [y.bfloat16().to(DEV) for y in (x.q, x.k, x.v, x.a, x.b, x.gk)]
+    g = [y.clone().requires_grad_() for y in t]
+    beta = torch.rand(1, 64, 2, 1, device=DEV).bfloat16()
+    m, (lx, _) = _layer(), _x(2, 8, grad=False)
+    n, row = _lib.native(), torch.randn(8, 64, device=DEV).bfloat16()
+    one = {
+        "chunk": lambda: n.chunk(*t, 2, None, None, False, False, 16, None, False),
+        "chunk_grad": lambda: n.chunk(*g, 2, None, None, False, False, 16, None, False),
+        "chunk_hdla": lambda: n.chunk_hdla(t[0], t[1], t[2], beta, t[5], None, None, False, None, False),
+        "recurrent": lambda: n.recurrent(*t, 2, None, None, False, False, None, False),
+        "normalize": lambda: n.normalize(row, None, None, None, None, "sigmoid", "pre", 1.0, 1e-5, False, 1, False),
+        "layer": lambda: m._forward_native(lx, None, False),
+    }[call]
+    assert one() is not None
+    count, stop = [0], threading.Event()
+
+    def other():
+        while not stop.is_set():
+            count[0] += 1
+            time.sleep(0)
+
+    th = threading.Thread(target=other)
+    old = sys.getswitchinterval()
+    sys.setswitchinterval(30.0)              # from here on a thread runs Python only when another one lets go of the lock itself
+    try:
+        th.start()
+        before = count[0]
+        for _ in range(5000):
+            one()
+            if count[0] != before:
+                break
+        ran = count[0] - before
+    finally:
+        stop.set()
+        th.join()
+        sys.setswitchinterval(old)
+    assert ran > 0
+
+
+def test_an_exception_of_a_saved_tensor_hook_comes_through():
+    ops, _ = _operands()
+
+    def refuse(t):
+        raise KeyError("not today")
+
+    with pytest.raises(KeyError, match="not today"):
+        with torch.autograd.graph.saved_tensors_hooks(refuse, lambda t: t):
+            chunk_hrdplr_delta_rule(*ops, 2)
+    assert torch.isfinite(chunk_hrdplr_delta_rule(*ops, 2)[0].float()).all()
