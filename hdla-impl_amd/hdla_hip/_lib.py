@@ -4,6 +4,7 @@ The library is the only compute path: if it cannot be loaded every operator rais
 """
 import ctypes
 import os
+import warnings
 from typing import Optional
 
 import torch
@@ -154,19 +155,32 @@ def load():
     return lib
 
 
+class _NoNative:
+    """What stands in for the native host path where that cannot be loaded: nothing is its case."""
+
+    def _not_mine(self, *args):
+        return None
+
+    chunk = chunk_hdla = recurrent = recurrent_hdla = normalize = layer = _not_mine
+
+
 def native():
     """The operators' native host path (csrc/native.cpp), bound to the loaded library.  Its functions take the arguments
-    of the public operators; they return None, having done nothing, for a call that is not theirs."""
+    of the public operators; they return None, having done nothing, for a call that is not theirs.  It is built against one
+    torch's C++ headers: where it cannot be loaded, a warning says so once and every call takes the Python code behind it,
+    which runs the same kernels with more host time."""
     global _native
     if _native is None:
         lib = load()
         try:
             from . import _native as module
         except ImportError as e:
-            raise HdlaError(f"the native host path could not be loaded ({e}): build it with the library "
-                            "(make -C hdla-impl_amd/csrc)") from e
-        module.bind(lib._handle, HdlaError, torch.OutOfMemoryError)
-        _native = module
+            warnings.warn(f"hdla_hip: the native host path could not be loaded ({e}); calls go through the slower Python host code. "
+                          "Build it for this torch with: make -C hdla-impl_amd/csrc", RuntimeWarning, stacklevel=2)
+            _native = _NoNative()
+        else:
+            module.bind(lib._handle, HdlaError, torch.OutOfMemoryError)
+            _native = module
     return _native
 
 

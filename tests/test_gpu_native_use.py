@@ -146,3 +146,14 @@ def test_an_exception_of_a_saved_tensor_hook_comes_through():
         with torch.autograd.graph.saved_tensors_hooks(refuse, lambda t: t):
             chunk_hrdplr_delta_rule(*ops, 2)
     assert torch.isfinite(chunk_hrdplr_delta_rule(*ops, 2)[0].float()).all()
+
+
+def test_operators_and_layer_without_the_native_host_path(monkeypatch):
+    ops, do = _operands()
+    m, (x, ldo) = _layer(), _x(2, 40)
+    run = lambda: torch.autograd.grad(chunk_hrdplr_delta_rule(*ops, 2)[0], ops, do)
+    ref, lref = run(), torch.autograd.grad(m(x)[0], [x, m.o_proj.weight], ldo)
+    monkeypatch.setattr(_lib, "_native", _lib._NoNative())
+    assert all(torch.equal(a, b) for a, b in zip(ref, run()))
+    for a, b in zip(lref, torch.autograd.grad(m(x)[0], [x, m.o_proj.weight], ldo)):
+        assert O.rel_l2(a, b) <= 2e-2                                  # (the layer's steps round to bf16 in between)

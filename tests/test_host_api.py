@@ -329,6 +329,25 @@ def test_missing_library_fails_loudly(monkeypatch):
         _lib.load()
 
 
+def test_a_native_host_path_that_does_not_load_leaves_the_python_code(monkeypatch):
+    """The library is required; the host path beside it, which is bound to one torch's C++ interface, is not."""
+    import sys
+    import warnings
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.setitem(sys.modules, "hdla_hip._native", None)              # its import fails
+    monkeypatch.delattr(hdla_hip, "_native", raising=False)
+    with pytest.warns(RuntimeWarning, match="native host path"):
+        n = _lib.native()
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _lib.native() is n                                           # said once
+    for f in ("chunk", "chunk_hdla", "recurrent", "recurrent_hdla", "normalize", "layer"):
+        assert getattr(n, f)(1, 2, 3) is None
+    x = make_inputs(5, 1, 4, 1, 64, 64)
+    with pytest.raises(_lib.HdlaError, match="GPU only"):
+        chunk_hrdplr_delta_rule(x.q, x.k, x.v, x.a, x.b, x.gk, 2)
+
+
 def test_product_code_does_not_import_the_oracle():
     pkg = os.path.join(ROOT, "hdla-impl_amd")
     for dirpath, _, files in os.walk(pkg):
