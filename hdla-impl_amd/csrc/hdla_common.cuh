@@ -260,6 +260,28 @@ template <bool GKF32> __device__ __forceinline__ void st_gk4(void* base, int64_t
     else st_frag(reinterpret_cast<bf16*>(base) + elem_off, to_frag<bf16>(x));
 }
 
+// ---- x = 1 / (1 + e): sigmoids of N values, whose exponentials e^-x are in e -------------------------------
+// The quotient is one step of Newton's method on the hardware reciprocal: for every fp32 number from 1 to 2^126 that is, bit for
+// bit, the IEEE quotient (all 1,056,964,609 of them compared; the reciprocal alone is another number for 113,107,050), in three
+// instructions instead of ten.  Beyond (x < -87.3, where it is subnormal or zero), if the wave finds any such value, the division.
+// Measured, 8192 x 1024 bf16, division / this / the reciprocal alone: layer_pre forward 27.6 / 22.5 / 21.8 us, backward 30.6 / 28.1 /
+// 27.8; a layer training step is 1.8 % slower with the division than with the reciprocal, with this 0.6 %.
+template <int N> __device__ __forceinline__ void sigmoid_of_exp(const float (&e)[N], float (&x)[N]) {
+    float big = 0.f;
+#pragma unroll
+    for (int j = 0; j < N; ++j) { x[j] = 1.f + e[j]; big = fmaxf(big, x[j]); }
+    if (__any(big > 0x1p126f)) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) x[j] = 1.f / x[j];
+    } else {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const float r = __builtin_amdgcn_rcpf(x[j]);
+            x[j] = __builtin_fmaf(__builtin_fmaf(-x[j], r, 1.f), r, r);
+        }
+    }
+}
+
 // ---- exp: fast hardware exp2 for the bf16 path, full-accuracy expf for the fp32 path -----------------------
 template <typename T> __device__ __forceinline__ float exp_t(float x);
 template <> __device__ __forceinline__ float exp_t<bf16>(float x) { return __expf(x); }

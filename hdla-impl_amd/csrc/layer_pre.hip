@@ -61,17 +61,20 @@ template <> struct PrePiece<float> {
     }
 };
 
-// fp32: the division; bf16 results: the hardware reciprocal (one unit in the last place of fp32, a tenth of the
-// instructions; the exponential before it is as close)
-template <typename T> __device__ __forceinline__ float pre_sigmoid(float x) {
-    const float d = 1.f + exp_t<T>(-x);
-    return sizeof(T) == 2 ? __builtin_amdgcn_rcpf(d) : 1.f / d;
+template <typename T> __device__ __forceinline__ float pre_sigmoid(float x) { return 1.f / (1.f + exp_t<T>(-x)); }
+
+template <typename T, int N> __device__ __forceinline__ void pre_sigmoids(const float (&x)[N], float (&s)[N]) {
+    float e[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) e[j] = exp_t<T>(-x[j]);
+    sigmoid_of_exp<N>(e, s);
 }
 
 // u = silu(x) in place; returns nothing.  sg[j] keeps sigmoid(x) for the backward pass.
 template <typename T, int N> __device__ __forceinline__ void silu_fwd(float (&x)[N], float (&sg)[N]) {
+    pre_sigmoids<T, N>(x, sg);
 #pragma unroll
-    for (int j = 0; j < N; ++j) { sg[j] = pre_sigmoid<T>(x[j]); x[j] *= sg[j]; }
+    for (int j = 0; j < N; ++j) x[j] *= sg[j];
 }
 
 template <typename T>
@@ -191,11 +194,17 @@ __global__ __launch_bounds__(256) void logsigmoid_kernel(const void* x, const vo
     for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < npiece; i += stride) {
         float f[N], g[N];
         PrePiece<T>::ld(x, i * N, f);
-        if (BWD) PrePiece<T>::ld(dy, i * N, g);
+        if (BWD) {
+            PrePiece<T>::ld(dy, i * N, g);
+            float s[N];
 #pragma unroll
-        for (int j = 0; j < N; ++j) {
-            if (BWD) f[j] = g[j] * pre_sigmoid<T>(-f[j]);
-            else {
+            for (int j = 0; j < N; ++j) f[j] = -f[j];
+            pre_sigmoids<T, N>(f, s);
+#pragma unroll
+            for (int j = 0; j < N; ++j) f[j] = g[j] * s[j];
+        } else {
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
                 // log(1 + e) for e = exp(-|f|) in (0, 1]: the accurate routine for fp32 results; for bf16 results the
                 // hardware logarithm, with the first term of the series where 1 + e would round e away
                 const float e = exp_t<T>(-fabsf(f[j]));

@@ -142,9 +142,14 @@ __global__ __launch_bounds__(256) void layer_down_kernel(DownArgs p) {
             for (int m = 0; m < MT; ++m) {
                 // df = dlog_f sigmoid(-f), rounded as the stored gradient would be
                 auto one = [](Frag<bf16>& d, Frag<bf16> f) __attribute__((always_inline)) {
-                    f32x4 x = to_f32(d), z = to_f32(f);
+                    f32x4 x = to_f32(d);
+                    const f32x4 z = to_f32(f);
+                    float e[4], s[4];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) x[i] *= __builtin_amdgcn_rcpf(1.f + __expf(z[i]));
+                    for (int i = 0; i < 4; ++i) e[i] = __expf(z[i]);
+                    sigmoid_of_exp<4>(e, s);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) x[i] *= s[i];
                     d = to_frag<bf16>(x);
                 };
                 one(y[m].a, ff[m].a);

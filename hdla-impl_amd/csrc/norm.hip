@@ -92,11 +92,13 @@ template <int N> __device__ __forceinline__ void ld_weight(const void* w, int w_
     }
 }
 
-// fp32: the division; bf16 results: the hardware reciprocal (one unit in the last place of fp32, a tenth of the
-// instructions; the exponential before it is as close)
-template <typename T> __device__ __forceinline__ float sigmoid_t(float x);
-template <> __device__ __forceinline__ float sigmoid_t<float>(float x) { return 1.f / (1.f + __expf(-x)); }
-template <> __device__ __forceinline__ float sigmoid_t<bf16>(float x) { return __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
+// x = sigmoid(x)
+template <int N> __device__ __forceinline__ void sigmoids(float (&x)[N]) {
+    float e[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) e[j] = __expf(-x[j]);
+    sigmoid_of_exp<N>(e, x);
+}
 
 // Where a lane stands: lane sl of the LPR lanes across one group, group position rw of the 64/LPR groups of a pass;
 // `wave` counts passes' owners (wavefronts, or workgroups when a workgroup shares one long group).
@@ -189,13 +191,14 @@ __global__ __launch_bounds__(256) void normalize_fwd_kernel(NormArgs p) {
         if (AHEAD) request(sg + L.nwave);
         float ss = 0.f;
 #pragma unroll
-        for (int i = 0; i < NV; ++i)
+        for (int i = 0; i < NV; ++i) {
+            if (p.gate_pos) sigmoids<N>(gs[i]);
 #pragma unroll
             for (int j = 0; j < N; ++j) {
-                if (p.gate_pos) gs[i][j] = sigmoid_t<T>(gs[i][j]);
                 if (pre) x[i][j] *= gs[i][j];
                 ss += x[i][j] * x[i][j];
             }
+        }
         float unused = 0.f;
         group_sum(L, ss, unused, sred, buf);
         const float rs = p.cn / sqrtf(ss * p.inv_e + p.eps);
@@ -268,16 +271,17 @@ __global__ __launch_bounds__(256) void normalize_bwd_kernel(NormArgs p) {
         // x: the normalised quantity (gated when the gate comes first); dr: gradient of x / sigma before the weight
         float ss = 0.f, sd = 0.f;
 #pragma unroll
-        for (int i = 0; i < NV; ++i)
+        for (int i = 0; i < NV; ++i) {
+            if (p.gate_pos) sigmoids<N>(gs[i]);
 #pragma unroll
             for (int j = 0; j < N; ++j) {
-                if (p.gate_pos) gs[i][j] = sigmoid_t<T>(gs[i][j]);
                 if (pre) x[i][j] *= gs[i][j];
                 dr[i][j] *= p.cn;
                 if (post) dr[i][j] *= gs[i][j];
                 ss += x[i][j] * x[i][j];
                 sd += x[i][j] * dr[i][j] * w[i][j];
             }
+        }
         group_sum(L, ss, sd, sred, buf);
         const float inv = 1.f / sqrtf(ss * p.inv_e + p.eps);          // 1 / sigma
         const float proj = sd * inv * p.inv_e;                         // sum(r * dr * w) / E, r = x / sigma

@@ -72,8 +72,12 @@ __global__ __launch_bounds__(256) void skinny_wgrad_kernel(WgradArgs p) {
             for (int a = 0; a < 2; ++a) {
                 f32x4 d = to_f32(x[a]);
                 const f32x4 t = to_f32(f[a]);
+                float e[4], s[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) d[i] *= __builtin_amdgcn_rcpf(1.f + __expf(t[i]));
+                for (int i = 0; i < 4; ++i) e[i] = __expf(t[i]);
+                sigmoid_of_exp<4>(e, s);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) d[i] *= s[i];
                 x[a] = to_frag<bf16>(d);
             }
         }
