@@ -39,8 +39,7 @@ int check_dims(const hdla_dims* d, int max_dim = 128) {
 // ---- the fused route (fused_impl.cuh) ----------------------------------------------------------------------------
 constexpr int FUSED_MAX_SEGMENTS = 64;       // the segments are chained serially by every workgroup that needs them: about a
                                              // microsecond a segment, against 2.5 for every chunk a segment is shorter
-constexpr int FUSED_MIN_SEGMENT_CHUNKS = 4;  // one chunk for each pair of producer waves: shorter segments wait for the same first chunk
-constexpr int FUSED_MIN_CHUNKS = 9;          // sequences of at most 8 chunks stay whole: a second kernel takes as long as they do
+constexpr int FUSED_MIN_SEGMENT_CHUNKS = 8;  // fewer would cost precision, see fused_segments
 constexpr int FUSED_TARGET_WORKGROUPS = 256; // one workgroup per compute unit
 
 // the shapes the fused kernels are built for
@@ -51,20 +50,21 @@ int pick_route(const hdla_dims* d, bool& fused) {
     if (d->route == HDLA_ROUTE_FUSED && !fused) return HDLA_ERR_ROUTE;
     return HDLA_OK;
 }
-// time segments per sequence: as many as give every compute unit a workgroup, within the limits above
+// Time segments per sequence: as many as give every compute unit a workgroup, of eight chunks at the least.  Segments of four
+// chunks are faster where few (sequence, head) lanes leave the device idle (us, forward pass / training step, eight -> four:
+// 2 lanes of 16 chunks 26/75 -> 20/70, 8 of 63 44/126 -> 32/96, 16 of 125 50/158 -> 49/141), but the states entering the later
+// segments reach the outputs through G, which is rounded to 2 bytes once more than what a whole scan multiplies: with twice the
+// segments the gradients are further from a float64 evaluation (mean of 12 inputs: by 0.3 to 0.4 % of the error for 2 lanes of 16
+// chunks, by 0.1 to 0.2 % for 16 of 125, by 0.04 to 0.09 % for 8 of 63; standard errors 0.15, 0.02, 0.02 %).  Splitting the
+// entering states and the transitions into two 2-byte halves each takes half of that away, for 3 us of a forward pass of 81.
 int fused_segments(const hdla_dims* d) {
     if (d->segments > 0) return d->segments < FUSED_MAX_SEGMENTS ? d->segments : FUSED_MAX_SEGMENTS;
     const long long lanes = (long long)d->N * d->H;
     const long long chunks_per_seq = ((d->T + CHUNK - 1) / CHUNK) / (d->cu_seqlens ? d->N : 1);
-    if (chunks_per_seq < FUSED_MIN_CHUNKS) return 1;
-    // A segment takes about 2.2 us a chunk and every segment of the chain 0.9 us: the sum is least near 1.6 sqrt(chunks)
-    // segments, and twice as many pay as long as the chunks are at least a quarter of their square.  Measured (us,
-    // forward pass / training step, 8 chunks a segment at the least -> this rule): 2 lanes of 16 chunks 26/75 -> 20/70,
-    // 8 of 63 44/126 -> 32/96, 16 of 125 50/158 -> 49/141.
-    long long nseg = 1;
+    int nseg = 1;
     while (nseg * 2 <= FUSED_MAX_SEGMENTS && lanes * nseg * 2 <= FUSED_TARGET_WORKGROUPS &&
-           chunks_per_seq / (nseg * 2) >= FUSED_MIN_SEGMENT_CHUNKS && nseg * nseg <= chunks_per_seq) nseg *= 2;
-    return (int)nseg;
+           chunks_per_seq / (nseg * 2) >= FUSED_MIN_SEGMENT_CHUNKS) nseg *= 2;
+    return nseg;
 }
 
 // ---- time segments of the stand-alone scans (scan_impl.cuh): where a whole sequence per workgroup would leave most of the

@@ -121,6 +121,14 @@ def test_bad_dims_are_rejected_before_launch(kw, code):
     assert len(lib.hdla_strerror(rc)) > 8
 
 
+@pytest.mark.parametrize("N,T,H,want", [(1, 240, 2, 1), (1, 256, 2, 2), (2, 1000, 4, 4), (1, 2000, 16, 8), (4, 2048, 16, 4), (1, 65536, 2, 64),
+                                        (16, 512, 16, 1)])
+def test_segments_of_the_fused_route_hold_eight_chunks(N, T, H, want):
+    """Shorter ones would be faster for few sequences and heads, and less precise."""
+    n = _lib.load().hdla_boundary_bytes(ctypes.byref(_lib.HdlaDims(N, T, H, 64, 64, 2, N, 0, 0, 1.0, None, 0, 0)))
+    assert n == (N * H * want * 64 * 64 * 4 if want > 1 else 0)
+
+
 @pytest.mark.parametrize("N,H,asked,want", [(1, 2, 7, 7), (4, 16, 100, 32), (256, 16, 32, 1), (100, 8, 32, 5), (4096, 1, 32, 1),
                                             (65535, 1, 32, 1), (65535, 16, 1000, 1)])
 def test_segments_asked_for_of_the_stand_alone_scans_are_bounded(N, H, asked, want):
