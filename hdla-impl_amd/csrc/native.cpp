@@ -120,6 +120,14 @@ bool chunk_dims(const ChunkIn& x, double scale, hdla_dims& d) {
     return route_and_segments(d);
 }
 
+// The launch plan of a backward pass is that of its forward pass, whatever the environment says by then: the record is laid out by it.
+void keep_plan(AutogradContext* ctx, const hdla_dims& d) { ctx->saved_data["plan"] = std::vector<int64_t>{d.route, d.segments}; }
+void kept_plan(AutogradContext* ctx, hdla_dims& d) {
+    const auto plan = ctx->saved_data["plan"].toIntVector();
+    d.route = (int32_t)plan[0];
+    d.segments = (int32_t)plan[1];
+}
+
 Tensor workspace(const hdla_dims& d, int pass, const Tensor& like) {
     const size_t n = api.workspace_bytes(&d, pass);
     if (!n) throw AbiError("hdla_workspace_bytes rejected the dimensions (B=" + std::to_string(d.B) + ",T=" + std::to_string(d.T) +
@@ -148,6 +156,7 @@ struct ChunkFn : torch::autograd::Function<ChunkFn> {
         if (h0) x.h0 = h0->to(at::kFloat).contiguous();
         hdla_dims d;
         chunk_dims(x, scale, d);
+        keep_plan(ctx, d);
         Tensor o, ht, boundary;
         chunk_forward(x, d, want_ht, keep_boundaries_default(), o, ht, boundary);
         ctx->save_for_backward({q, k, v, x.a, x.b, x.beta, gk, value(h0), x.cu, boundary});
@@ -166,6 +175,7 @@ struct ChunkFn : torch::autograd::Function<ChunkFn> {
         if (x.h0.defined()) x.h0 = x.h0.to(at::kFloat).contiguous();
         hdla_dims d;
         chunk_dims(x, ctx->saved_data["scale"].toDouble(), d);
+        kept_plan(ctx, d);
         const Tensor d_o = grads[0].defined() ? grads[0].to(x.v.scalar_type()).contiguous() : at::zeros_like(x.v);
         Tensor dht;
         if (grads.size() > 1 && grads[1].defined()) dht = grads[1].to(at::kFloat).contiguous();
@@ -562,7 +572,7 @@ Tensor project(const Tensor& x, const Tensor& w) {
     return y;
 }
 // everything between x and the output; what the backward pass needs of it
-struct LayerFwd { Tensor x, w, y, f, g, o, n, out, ht, boundary; ChunkIn op; };
+struct LayerFwd { Tensor x, w, y, f, g, o, n, out, ht, boundary; ChunkIn op; hdla_dims dims; };
 
 // params: wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo; r.w gathered; keep: a backward pass follows
 void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, const Tensor& h0, bool want_ht, bool chunked, bool keep, LayerFwd& r) {
@@ -583,7 +593,7 @@ void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, const T
     r.g = at::empty({rows, d}, opt);
     check(api.layer_up_fwd(&ud, ptr(r.y), ptr(P[6]), ptr(P[7]), ptr(r.f), ptr(in.gk), ptr(r.g), s), "hdla_layer_up_fwd");
     if (h0.defined()) in.h0 = h0.to(at::kFloat).contiguous();
-    hdla_dims cd;
+    hdla_dims& cd = r.dims;
     chunk_dims(in, 1.0, cd);
     if (chunked) {
         chunk_forward(in, cd, want_ht, keep && keep_boundaries_default(), r.o, r.ht, r.boundary);
@@ -619,6 +629,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
         LayerFwd r;
         r.w = gather_weights(P, LayerCols(x.size(2), f.H, x.size(0) * x.size(1) >= PAD_FROM_ROWS));
         layer_forward(x, P, f, value(h0), want_ht, true, true, r);
+        keep_plan(ctx, r.dims);
         ctx->save_for_backward({r.x, r.w, r.y, r.f, r.g, r.o, r.n, r.boundary, r.op.q, r.op.k, r.op.v, r.op.beta, r.op.gk, value(h0), wf1, wg1,
                                 wnorm, wo});
         ctx->saved_data["c"] = std::vector<double>{f.beta_scale, f.c, f.eps};
@@ -672,6 +683,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
             if (grads.size() > 1 && grads[1].defined()) dht = grads[1].to(at::kFloat).contiguous();
             hdla_dims cd;
             chunk_dims(in, 1.0, cd);
+            kept_plan(ctx, cd);
             const Tensor ws = workspace(cd, HDLA_PASS_BWD, x);
             check(api.chunk_bwd_b(&cd, ptr(q), ptr(k), ptr(v), nullptr, nullptr, ptr(beta), ptr(gk), fptr(in.h0), ptr(d_o), fptr(dht), ptr(dq),
                                   ptr(dk), ptr(dv), nullptr, nullptr, ptr(dbeta), ptr(dgk), fptr(dh0), ptr(boundary),

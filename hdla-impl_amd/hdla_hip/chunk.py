@@ -63,9 +63,9 @@ def _rank2(x: torch.Tensor, rank: int) -> torch.Tensor:
     return torch.stack([x, torch.zeros_like(x)], dim=2).reshape(B, 2 * T, H, K)
 
 
-def _dims(q, v, gk, scale, cu_seqlens, n_seq):
+def _dims(q, v, gk, scale, cu_seqlens, n_seq, plan=(None, None)):
     B, T, H, K = q.shape
-    return _lib.make_dims(B, T, H, K, v.shape[-1], 2, n_seq, q.dtype, gk.dtype, scale, cu_seqlens)
+    return _lib.make_dims(B, T, H, K, v.shape[-1], 2, n_seq, q.dtype, gk.dtype, scale, cu_seqlens, *plan)
 
 
 def chunk_hrdplr_fwd(q, k, v, a, b, gk, scale, initial_state, output_final_state, cu_seqlens=None, keep=False,
@@ -134,16 +134,17 @@ def chunk_hrdplr_bwd_kept(q, k, v, a, b, gk, scale, initial_state, do, dht, kept
 
 
 def chunk_hrdplr_bwd(q, k, v, a, b, gk, scale, initial_state, do, dht, cu_seqlens=None, want_dh0=True,
-                     keep_workspace=False, beta=None, boundary=None):
+                     keep_workspace=False, beta=None, boundary=None, plan=(None, None)):
     """Backward launch sequence (HRDPLR/hrdplr.py:149-284) on native shapes.  Returns (dq, dk, dv, da, db, dgk, dh0), or
-    with ``beta`` (dq, dk, dv, dbeta, dgk, dh0).  ``boundary``: the record a forward pass left (see chunk_hrdplr_fwd)."""
+    with ``beta`` (dq, dk, dv, dbeta, dgk, dh0).  ``boundary``: the record a forward pass left (see chunk_hrdplr_fwd), ``plan``
+    the route and segments it ran with."""
     lib = _lib.load()
     B, T, H, K = q.shape
     V = v.shape[-1]
     N = B if cu_seqlens is None else cu_seqlens.numel() - 1
     new = torch.empty_like
     with torch.cuda.device(q.device):
-        dims = _dims(q, v, gk, scale, cu_seqlens, N)
+        dims = _dims(q, v, gk, scale, cu_seqlens, N, plan)
         ws = _lib.workspace(dims, 1, q.device)
         dq, dk, dv, dgk = new(q), new(k), new(v), new(gk)
         da = db = dbeta = None
@@ -189,6 +190,7 @@ class ChunkDPLRDeltaRuleFunction(torch.autograd.Function):
         # the inputs (hrdplr.py:137) and, where the route has one, the forward pass's record (37 % of the inputs' bytes;
         # HDLA_HIP_INPUTS_ONLY=1: strictly the inputs)
         ctx.save_for_backward(q, k, v, a, b, gk, initial_state, cu_seqlens, boundary)
+        ctx.plan = _lib.default_route(), _lib.default_segments()
         ctx.scale = scale
         ctx.chunk_size = chunk_size
         ctx.output_final_state = output_final_state
@@ -212,7 +214,8 @@ class ChunkDPLRDeltaRuleFunction(torch.autograd.Function):
                                                                  cu_seqlens, want_dh0=initial_state is not None)
         else:
             dq, dk, dv, da, db, dgk, dh0 = chunk_hrdplr_bwd(q, k, v, a, b, gk, ctx.scale, h0, do, dht, cu_seqlens,
-                                                            want_dh0=initial_state is not None, boundary=boundary)
+                                                            want_dh0=initial_state is not None, boundary=boundary,
+                                                            plan=ctx.plan)
         if dh0 is not None:
             dh0 = dh0.to(initial_state.dtype)
         # one slot per forward argument (hrdplr.py:284), plus one each for cu_seqlens and keep_forward

@@ -45,9 +45,9 @@ def _fwd(q, k, v, beta, gk, scale, initial_state, output_final_state, cu_seqlens
                             want_boundary=want_boundary)
 
 
-def _bwd(q, k, v, beta, gk, scale, initial_state, do, dht, cu_seqlens, want_dh0, boundary=None):
+def _bwd(q, k, v, beta, gk, scale, initial_state, do, dht, cu_seqlens, want_dh0, boundary=None, plan=(None, None)):
     return chunk_hrdplr_bwd(q, k, v, None, None, gk, scale, initial_state, do, dht, cu_seqlens, want_dh0=want_dh0,
-                            beta=beta, boundary=boundary)
+                            beta=beta, boundary=boundary, plan=plan)
 
 
 class ChunkHDLAFunction(torch.autograd.Function):
@@ -69,6 +69,7 @@ class ChunkHDLAFunction(torch.autograd.Function):
         else:
             o, final_state = _fwd(q, k, v, beta, gk, scale, h0, output_final_state, cu_seqlens)
         ctx.save_for_backward(q, k, v, beta, gk, initial_state, cu_seqlens, boundary)
+        ctx.plan = _lib.default_route(), _lib.default_segments()
         ctx.scale = scale
         return o.to(q.dtype), final_state
 
@@ -88,7 +89,7 @@ class ChunkHDLAFunction(torch.autograd.Function):
                                                                 cu_seqlens, want_dh0=initial_state is not None, beta=beta)
         else:
             dq, dk, dv, dbeta, dgk, dh0 = _bwd(q, k, v, beta, gk, ctx.scale, h0, do, dht, cu_seqlens,
-                                               want_dh0=initial_state is not None, boundary=boundary)
+                                               want_dh0=initial_state is not None, boundary=boundary, plan=ctx.plan)
         if dh0 is not None:
             dh0 = dh0.to(initial_state.dtype)
         return dq.to(q), dk.to(k), dv.to(v), dbeta.to(beta), dgk.to(gk), None, dh0, None, None, None

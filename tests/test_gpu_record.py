@@ -59,3 +59,35 @@ def test_backward_pass_from_the_record(B, T, H, cu, segments, gk_div, gk_dtype, 
         assert torch.isfinite(kept[n].float()).all(), n
         assert O.rel_l2(kept[n], formed[n]) <= 1e-3, n
         assert O.rel_l2(kept[n], classic[n]) <= (6e-3 if segments > 1 else 2e-3), n
+
+
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("form", ["ab", "beta", "layer"])
+def test_the_environment_may_change_between_the_passes(form, native, monkeypatch):
+    """The record is laid out by the forward pass's route and segments: the backward pass runs with these, not with what the
+    environment asks for by then."""
+    from hdla_hip import chunk_hdla_delta_rule, chunk_hrdplr_delta_rule
+    from hdla_hip.layer import HDLA_Custom
+    if not native:
+        monkeypatch.setattr(_lib, "_native", _lib._NoNative())
+    x = make_inputs(46, 1, 600, 2, 64, 64)
+    t = [y.bfloat16().to(DEV).requires_grad_() for y in (x.q, x.k, x.v, x.a, x.b, x.gk)]
+    do = x.do.bfloat16().to(DEV)
+    if form == "layer":
+        torch.manual_seed(1)
+        m = HDLA_Custom(128, 2, token_mixer_init_type=2, rescale_type=0).to(DEV).bfloat16().train()
+        leaves = [torch.randn(1, 600, 128, device=DEV).bfloat16().requires_grad_(), *m.parameters()]
+        do, run = torch.randn(1, 600, 128, device=DEV).bfloat16(), lambda: m(leaves[0])[0]
+    elif form == "ab":
+        leaves, run = t, lambda: chunk_hrdplr_delta_rule(*t, 2, scale=0.7)[0]
+    else:
+        leaves = [*t[:3], torch.rand(1, 600, 2, 1, device=DEV).bfloat16().requires_grad_(), t[5]]
+        run = lambda: chunk_hdla_delta_rule(*leaves, scale=0.7)[0]
+    monkeypatch.setenv("HDLA_HIP_SEGMENTS", "4")
+    ref = torch.autograd.grad(run(), leaves, do)
+    for env in ({"HDLA_HIP_SEGMENTS": "2"}, {"HDLA_HIP_SEGMENTS": "8"}, {"HDLA_HIP_ROUTE": "classic"}):
+        with monkeypatch.context() as c:
+            y = run()
+            for name, value in env.items():
+                c.setenv(name, value)
+            assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(y, leaves, do), ref)), env
