@@ -102,6 +102,7 @@ struct FusedLayout {
     size_t total;
     int nch, nseg;
 };
+constexpr int PASS_BWD_RECORD = -2;          // a backward pass that is given the record (hdla_record_workspace_bytes)
 int make_fused_layout(const hdla_dims* d, int pass, FusedLayout& L) {
     const int rc = check_dims(d);
     if (rc) return rc;
@@ -117,24 +118,28 @@ int make_fused_layout(const hdla_dims* d, int pass, FusedLayout& L) {
     size_t off = 0;
     auto take = [&](size_t bytes) { const size_t o = off; off += up256(bytes); return o; };
     L.ERR = take(256);
-    L.SLOC = take(recs * K * V * 4);
-    L.MSEG = take(recs * K * K * 4);
+    if (pass != PASS_BWD_RECORD) {                            // of the passes that form the segments' records
+        L.SLOC = take(recs * K * V * 4);
+        L.MSEG = take(recs * K * K * 4);
+    }
     if (pass == HDLA_PASS_FWD) {
         L.OL = take(chw * 16 * V * 4);
         L.GW = take(chw * 16 * K * es);
     } else {
         L.RSEG = take(recs * K * V * 4);
-        L.SIN = take(recs * K * V * 4);
-        L.MT = take(recs * K * K * 4);
-        L.GW = L.nseg > 1 ? take(chw * 16 * K * es) : 0;
-        L.AQ = take(chw * 1024 * es);
+        if (pass == HDLA_PASS_BWD) {                               // what a record holds
+            L.SIN = take(recs * K * V * 4);
+            L.MT = take(recs * K * K * 4);
+            L.GW = L.nseg > 1 ? take(chw * 16 * K * es) : 0;
+            L.AQ = take(chw * 1024 * es);
+            L.TM = take(chw * 1024 * es);
+            L.STRONG = take(chw * 4);
+        }
         L.HC = take(chw * K * V * es);
         L.DHC = take(chw * K * V * es);
         L.DVN = take(chw * 2 * 16 * V * es);
-        L.TM = take(chw * 1024 * es);
         L.UT = take(chw * 2 * V * 16 * es);
         L.W = take(chw * 2 * K * 16 * es);
-        L.STRONG = take(chw * 4);
     }
     if (d->cu_seqlens) {
         L.CHUNK_OFF = take((size_t)(2 * d->N + 1) * 4);
@@ -348,13 +353,15 @@ int run_fused(const hdla_dims* d, bool fwd, const void* q, const void* k, const 
               int stages = HDLA_STAGE_ALL) {
     typedef bf16 T;
     FusedLayout L;
-    const int rc = make_fused_layout(d, fwd ? HDLA_PASS_FWD : HDLA_PASS_BWD, L);
+    int rc = make_fused_layout(d, fwd ? HDLA_PASS_FWD : HDLA_PASS_BWD, L);
+    if (rc) return rc;
+    const FusedRecord R = fused_record(d, L);
+    char* const rec = boundary && boundary_bytes >= R.total ? static_cast<char*>(boundary) : nullptr;
+    if (!fwd && rec) rc = make_fused_layout(d, PASS_BWD_RECORD, L);
     if (rc) return rc;
     if (bad_ws(workspace, workspace_bytes, L.total)) return HDLA_ERR_WORKSPACE;
     if (boundary && (L.nseg > 1) && (boundary_bytes < fused_boundary_bytes(d) || (reinterpret_cast<uintptr_t>(boundary) & 15)))
         return HDLA_ERR_WORKSPACE;
-    const FusedRecord R = fused_record(d, L);
-    char* const rec = boundary && boundary_bytes >= R.total ? static_cast<char*>(boundary) : nullptr;
     if (rec && (reinterpret_cast<uintptr_t>(rec) & 15)) return HDLA_ERR_WORKSPACE;
     char* base = static_cast<char*>(workspace);
     FusedArgs<T> f{};
@@ -513,6 +520,12 @@ size_t hdla_record_bytes(const hdla_dims* dims) {
     FusedLayout L;
     if (check_dims(dims) || pick_route(dims, fused) || !fused || make_fused_layout(dims, HDLA_PASS_BWD, L)) return 0;
     return fused_record(dims, L).total;
+}
+
+size_t hdla_record_workspace_bytes(const hdla_dims* dims) {
+    FusedLayout L;
+    if (!hdla_record_bytes(dims)) return hdla_workspace_bytes(dims, HDLA_PASS_BWD);
+    return make_fused_layout(dims, PASS_BWD_RECORD, L) ? 0 : L.total;
 }
 
 int hdla_workspace_layout(const hdla_dims* dims, int pass, hdla_ws_layout* out) {

@@ -38,7 +38,7 @@ using torch::autograd::variable_list;
 // ---- the C ABI -------------------------------------------------------------------------------------------------------
 struct Api {
 #define HDLA_FN(name) decltype(&hdla_##name) name
-    HDLA_FN(strerror); HDLA_FN(workspace_bytes); HDLA_FN(record_bytes); HDLA_FN(chunk_fwd_b); HDLA_FN(chunk_bwd_b);
+    HDLA_FN(strerror); HDLA_FN(workspace_bytes); HDLA_FN(record_bytes); HDLA_FN(record_workspace_bytes); HDLA_FN(chunk_fwd_b); HDLA_FN(chunk_bwd_b);
     HDLA_FN(recurrent_fwd); HDLA_FN(param_recurrent_fwd); HDLA_FN(normalize_fwd); HDLA_FN(normalize_bwd);
     HDLA_FN(normalize_workspace_bytes); HDLA_FN(layer_pre_fwd); HDLA_FN(layer_pre_bwd); HDLA_FN(layer_up_fwd); HDLA_FN(layer_down);
     HDLA_FN(layer_up_wgrad); HDLA_FN(layer_up_wgrad_workspace_bytes); HDLA_FN(rows_gemm); HDLA_FN(sum_partials); HDLA_FN(stack_rows);
@@ -128,8 +128,9 @@ void kept_plan(AutogradContext* ctx, hdla_dims& d) {
     d.segments = (int32_t)plan[1];
 }
 
-Tensor workspace(const hdla_dims& d, int pass, const Tensor& like) {
-    const size_t n = api.workspace_bytes(&d, pass);
+// with_record: of a backward pass that is given the forward pass's record
+Tensor workspace(const hdla_dims& d, int pass, const Tensor& like, bool with_record = false) {
+    const size_t n = with_record ? api.record_workspace_bytes(&d) : api.workspace_bytes(&d, pass);
     if (!n) throw AbiError("hdla_workspace_bytes rejected the dimensions (B=" + std::to_string(d.B) + ",T=" + std::to_string(d.T) +
                            ",H=" + std::to_string(d.H) + ",K=" + std::to_string(d.K) + ",V=" + std::to_string(d.V) +
                            ",R=" + std::to_string(d.R) + ",N=" + std::to_string(d.N) + ")");
@@ -179,7 +180,7 @@ struct ChunkFn : torch::autograd::Function<ChunkFn> {
         const Tensor d_o = grads[0].defined() ? grads[0].to(x.v.scalar_type()).contiguous() : at::zeros_like(x.v);
         Tensor dht;
         if (grads.size() > 1 && grads[1].defined()) dht = grads[1].to(at::kFloat).contiguous();
-        const Tensor ws = workspace(d, HDLA_PASS_BWD, x.q);
+        const Tensor ws = workspace(d, HDLA_PASS_BWD, x.q, boundary.defined());
         const Tensor dq = at::empty_like(x.q), dk = at::empty_like(x.k), dv = at::empty_like(x.v), dgk = at::empty_like(x.gk);
         Tensor da, db, dbeta, dh0;
         if (x.beta.defined()) dbeta = at::empty_like(x.beta);
@@ -684,7 +685,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
             hdla_dims cd;
             chunk_dims(in, 1.0, cd);
             kept_plan(ctx, cd);
-            const Tensor ws = workspace(cd, HDLA_PASS_BWD, x);
+            const Tensor ws = workspace(cd, HDLA_PASS_BWD, x, boundary.defined());
             check(api.chunk_bwd_b(&cd, ptr(q), ptr(k), ptr(v), nullptr, nullptr, ptr(beta), ptr(gk), fptr(in.h0), ptr(d_o), fptr(dht), ptr(dq),
                                   ptr(dk), ptr(dv), nullptr, nullptr, ptr(dbeta), ptr(dgk), fptr(dh0), ptr(boundary),
                                   boundary.defined() ? (size_t)boundary.numel() : 0, ptr(ws), (size_t)ws.numel(), stream), "hdla_chunk_bwd_b");
@@ -822,7 +823,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
         PyErr_SetString(a[1], "the library does not export hdla_" #name);                                          \
         return nullptr;                                                                                            \
     }
-    HDLA_FN(strerror) HDLA_FN(workspace_bytes) HDLA_FN(record_bytes) HDLA_FN(chunk_fwd_b) HDLA_FN(chunk_bwd_b)
+    HDLA_FN(strerror) HDLA_FN(workspace_bytes) HDLA_FN(record_bytes) HDLA_FN(record_workspace_bytes) HDLA_FN(chunk_fwd_b) HDLA_FN(chunk_bwd_b)
     HDLA_FN(recurrent_fwd) HDLA_FN(param_recurrent_fwd) HDLA_FN(normalize_fwd) HDLA_FN(normalize_bwd)
     HDLA_FN(normalize_workspace_bytes) HDLA_FN(layer_pre_fwd) HDLA_FN(layer_pre_bwd) HDLA_FN(layer_up_fwd) HDLA_FN(layer_down)
     HDLA_FN(layer_up_wgrad) HDLA_FN(layer_up_wgrad_workspace_bytes) HDLA_FN(rows_gemm) HDLA_FN(sum_partials) HDLA_FN(stack_rows)

@@ -10,7 +10,7 @@ from typing import Optional
 import torch
 
 HDLA_BF16, HDLA_FP32 = 0, 1
-HDLA_VERSION = 203          # the header this binding was written against (struct layouts, entry points)
+HDLA_VERSION = 204          # the header this binding was written against (struct layouts, entry points)
 ROUTE_AUTO, ROUTE_CLASSIC, ROUTE_FUSED = 0, 1, 2
 _ROUTES = {"": ROUTE_AUTO, "auto": ROUTE_AUTO, "classic": ROUTE_CLASSIC, "fused": ROUTE_FUSED}
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -99,6 +99,8 @@ def load():
     lib.hdla_boundary_bytes.argtypes = [F]
     lib.hdla_record_bytes.restype = ctypes.c_size_t
     lib.hdla_record_bytes.argtypes = [F]
+    lib.hdla_record_workspace_bytes.restype = ctypes.c_size_t
+    lib.hdla_record_workspace_bytes.argtypes = [F]
     lib.hdla_chunk_fwd_b.restype = ctypes.c_int
     lib.hdla_chunk_fwd_b.argtypes = [F] + [P] * 10 + [P, ctypes.c_size_t, P, ctypes.c_size_t, P]
     lib.hdla_chunk_bwd_b.restype = ctypes.c_int
@@ -273,8 +275,10 @@ def current_stream(device) -> ctypes.c_void_p:
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
-def workspace(dims: HdlaDims, pass_: int, device) -> torch.Tensor:
-    n = load().hdla_workspace_bytes(ctypes.byref(dims), pass_)
+def workspace(dims: HdlaDims, pass_: int, device, with_record: bool = False) -> torch.Tensor:
+    """Scratch of a pass; ``with_record``: of a backward pass that is given the forward pass's record."""
+    lib = load()
+    n = lib.hdla_record_workspace_bytes(ctypes.byref(dims)) if with_record else lib.hdla_workspace_bytes(ctypes.byref(dims), pass_)
     if n == 0:
         raise HdlaError("hdla_workspace_bytes rejected the dimensions "
                         f"(B={dims.B},T={dims.T},H={dims.H},K={dims.K},V={dims.V},R={dims.R},N={dims.N})")

@@ -145,7 +145,7 @@ def chunk_hrdplr_bwd(q, k, v, a, b, gk, scale, initial_state, do, dht, cu_seqlen
     new = torch.empty_like
     with torch.cuda.device(q.device):
         dims = _dims(q, v, gk, scale, cu_seqlens, N, plan)
-        ws = _lib.workspace(dims, 1, q.device)
+        ws = _lib.workspace(dims, _lib.PASS_BWD, q.device, with_record=boundary is not None)
         dq, dk, dv, dgk = new(q), new(k), new(v), new(gk)
         da = db = dbeta = None
         if beta is None:

@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-#define HDLA_VERSION 203
+#define HDLA_VERSION 204
 
 enum { HDLA_BF16 = 0, HDLA_FP32 = 1 };
 
@@ -159,9 +159,12 @@ int hdla_chunk_bwd(const hdla_dims* dims, const void* q, const void* k, const vo
  * the score tiles of every chunk come to ((I - A_ab)^-1, A_ak, A_qb, the segments' transitions and their outputs per unit
  * of entering state: 6 KiB per (16-token chunk, head) at K = V = 64, 37 % of the inputs' bytes), which makes the backward
  * pass's first two kernels a third faster; without it the backward pass forms the same in its workspace first.
- * hdla_record_bytes returns 0 on the classic route only. */
+ * hdla_record_bytes returns 0 on the classic route only.
+ * hdla_record_workspace_bytes: the scratch hdla_chunk_bwd_b needs when it is given a whole record, i.e. that of HDLA_PASS_BWD
+ * without room for what the record holds (where there is no record, that of HDLA_PASS_BWD). */
 size_t hdla_boundary_bytes(const hdla_dims* dims);
 size_t hdla_record_bytes(const hdla_dims* dims);
+size_t hdla_record_workspace_bytes(const hdla_dims* dims);
 int hdla_chunk_fwd_b(const hdla_dims* dims, const void* q, const void* k, const void* v, const void* a, const void* b,
                      const void* beta, const void* gk, const float* h0, void* o, float* ht, void* boundary,
                      size_t boundary_bytes, void* workspace, size_t workspace_bytes, void* stream);

@@ -91,3 +91,30 @@ def test_the_environment_may_change_between_the_passes(form, native, monkeypatch
             for name, value in env.items():
                 c.setenv(name, value)
             assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(y, leaves, do), ref)), env
+
+
+@pytest.mark.parametrize("T,segments,cu", [(5, 1, None), (600, 4, None), (500, 3, [0, 100, 100, 411, 500])])
+def test_the_scratch_beside_a_record_is_enough(T, segments, cu):
+    """hdla_record_workspace_bytes bytes and not one more are touched, and the gradients are those on a whole workspace."""
+    x = make_inputs(47, 1, T, 2, 64, 64, n_states=None if cu is None else len(cu) - 1)
+    t = [y.bfloat16().to(DEV) for y in (x.q, x.k, x.v, x.a, x.b, x.gk)]
+    do, h0, dht = x.do.bfloat16().to(DEV), x.h0.to(DEV), x.dht.to(DEV)
+    table = None if cu is None else torch.tensor(cu, device=DEV)
+    lib, P, plan = _lib.load(), _lib.ptr, (_lib.ROUTE_FUSED, segments)
+    dims = _lib.make_dims(1, T, 2, 64, 64, 2, h0.shape[0], torch.bfloat16, torch.bfloat16, 0.7, table, *plan)
+    rec = _lib.record(dims, DEV)
+    s, o, ws = _lib.current_stream(torch.device(DEV)), torch.empty_like(t[2]), _lib.workspace(dims, 0, DEV)
+    _lib.check(lib.hdla_chunk_fwd_b(ctypes.byref(dims), *[P(y) for y in t[:5]], None, P(t[5]), P(h0), P(o), None, P(rec), rec.numel(), P(ws),
+                                    ws.numel(), s), "fwd")
+    res = []
+    small = lib.hdla_record_workspace_bytes(ctypes.byref(dims))
+    for n in (lib.hdla_workspace_bytes(ctypes.byref(dims), 1), small):
+        ws = torch.full((n + 4096,), 0xa5, dtype=torch.uint8, device=DEV)
+        g = [torch.empty_like(y) for y in t] + [torch.empty_like(h0)]
+        run = lambda have: lib.hdla_chunk_bwd_b(ctypes.byref(dims), *[P(y) for y in t[:5]], None, P(t[5]), P(h0), P(do), P(dht),
+                                                *[P(y) for y in g[:5]], None, P(g[5]), P(g[6]), P(rec), rec.numel(), P(ws), have, s)
+        _lib.check(run(n), "bwd")
+        assert bool((ws[n:] == 0xa5).all())
+        res.append(g)
+    assert run(small - 256) == -5
+    assert all(torch.equal(a, b) for a, b in zip(*res))

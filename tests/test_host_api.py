@@ -106,6 +106,20 @@ def test_routes_workspaces_and_boundary_records():
     assert f(ctypes.byref(d4), ok, ok, ok, ok, ok, None, ok, None, ok, None, ctypes.c_void_p(4096 + 8), 1 << 30, ok, 1 << 40, None) == -5
 
 
+def test_scratch_of_a_backward_pass_that_is_given_the_record():
+    """No room for what the record holds: states and transitions of the segments, G, and per (chunk, head) eight tiles and a flag."""
+    lib = _lib.load()
+    W, R, S = (lambda d, f=f: f(ctypes.byref(d)) for f in (lambda d: lib.hdla_workspace_bytes(d, 1), lib.hdla_record_bytes,
+                                                         lib.hdla_record_workspace_bytes))
+    d = _dims(B=4, N=4, T=2048, H=16)
+    segments, chunks = 4 * 16 * 4, 8192
+    assert W(d) - S(d) == 4 * segments * 64 * 64 * 4 + chunks * (16 * 64 * 2 + 2 * 1024 * 2 + 4)
+    assert R(d) == 2 * segments * 64 * 64 * 4 + chunks * (16 * 64 * 2 + 2 * 1024 * 2 + 4)
+    for none in (_dims(route=_lib.ROUTE_CLASSIC), _dims(K=128, V=128), _dims(in_dtype=torch.float32, gk_dtype=torch.float32)):
+        assert R(none) == 0 and S(none) == W(none) > 0
+    assert S(_dims(K=96)) == 0
+
+
 @pytest.mark.parametrize("kw,code", [
     (dict(K=96), -2), (dict(V=32), -2), (dict(R=1), -3), (dict(R=3), -3), (dict(H=0), -2), (dict(T=-1), -2),
     (dict(in_dtype=torch.float32, gk_dtype=torch.bfloat16), -4), (dict(N=3), -7), (dict(B=2, cu_seqlens=256), -7),
