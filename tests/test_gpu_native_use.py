@@ -93,6 +93,99 @@ def test_layer_tensors_off_the_16_byte_grid(which, B, T):
         assert O.rel_l2(b, a) <= 2e-2
 
 
+# ---- activation checkpointing, saved-tensor hooks, hooks on the layer -------------------------------------------------
+@pytest.mark.parametrize("reentrant", [False, True])
+def test_layer_and_operator_under_activation_checkpointing(reentrant):
+    from torch.utils.checkpoint import checkpoint
+    m, (x, do) = _layer(), _x(2, 40)
+    leaves = [x] + list(m.parameters())
+    ref = torch.autograd.grad(m(x)[0], leaves, do)
+    for p in leaves:
+        p.grad = None
+    checkpoint(lambda t: m(t)[0], x, use_reentrant=reentrant).backward(do)
+    assert all(torch.equal(p.grad, g) for p, g in zip(leaves, ref))
+    ops, do = _operands()
+    ref = torch.autograd.grad(chunk_hrdplr_delta_rule(*ops, 2)[0], ops, do)
+    checkpoint(lambda *t: chunk_hrdplr_delta_rule(*t, 2)[0], *ops, use_reentrant=reentrant).backward(do)
+    assert all(torch.equal(p.grad, g) for p, g in zip(ops, ref))
+
+
+def test_saved_tensors_on_the_host():
+    m, (x, do) = _layer(), _x(2, 40)
+    leaves = [x] + list(m.parameters())
+    ref = torch.autograd.grad(m(x)[0], leaves, do)
+    with torch.autograd.graph.save_on_cpu():
+        y = m(x)[0]
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(y, leaves, do), ref))
+
+
+def test_hooks_on_the_layer_and_on_its_gradients():
+    m, (x, do) = _layer(), _x(2, 40)
+    ref = torch.autograd.grad(m(x)[0], [x, m.o_proj.weight], do)
+    seen = []
+    m.register_forward_hook(lambda mod, a, out: (out[0] * 2, out[1]))
+    m.register_full_backward_hook(lambda mod, gi, go: seen.append(len(gi)))
+    m.o_proj.weight.register_hook(lambda g: g * 4)
+    got = torch.autograd.grad(m(x)[0], [x, m.o_proj.weight], do)
+    assert seen == [1] and torch.equal(got[0], 2 * ref[0]) and torch.equal(got[1], 8 * ref[1])
+
+
+# ---- streams and threads ----------------------------------------------------------------------------------------------
+def _step(m, x, do, n=3):
+    """n training steps and cached decode steps on the current stream; what they give."""
+    out = []
+    for _ in range(n):
+        y = m(x)[0]
+        out += [y.detach(), *torch.autograd.grad(y, [x] + list(m.parameters()), do)]
+    m.eval()
+    with torch.no_grad():
+        cache = RecurrentCache()
+        for i in range(n):
+            out.append(m(x[:, 20 * i:20 * i + 20 if i == 0 else 20 * i + 1], past_key_values=cache, use_cache=True)[0])
+    m.train()
+    return out
+
+
+def test_calls_on_a_second_stream():
+    """Whole steps on a stream that is not the default one, with the default stream allocating and writing at the same time."""
+    m, (x, do) = _layer(), _x(2, 70)
+    ref = _step(m, x, do)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        got = _step(m, x, do)
+    for _ in range(20):
+        torch.full((1 << 22,), float("nan"), device=DEV)
+    torch.cuda.current_stream().wait_stream(s)
+    assert all(torch.equal(a, b) for a, b in zip(ref, got))
+
+
+def test_threads_with_a_stream_each():
+    n = 4
+    ms, xs = [_layer() for _ in range(n)], [_x(2, 70, seed=10 + i) for i in range(n)]
+    refs = [_step(m, *x) for m, x in zip(ms, xs)]
+    torch.cuda.synchronize()
+    got, errors = [None] * n, []
+
+    def work(i):
+        try:
+            s = torch.cuda.Stream()
+            with torch.cuda.stream(s):
+                got[i] = _step(ms[i], *xs[i])
+            s.synchronize()
+        except Exception as e:                                     # reported by the main thread
+            errors.append(e)
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(n)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not errors
+    for r, g in zip(refs, got):
+        assert all(torch.equal(a, b) for a, b in zip(r, g))
+
+
 @pytest.mark.parametrize("call", ["chunk", "chunk_grad", "chunk_hdla", "recurrent", "normalize", "layer"])
 def test_other_threads_run_during_a_call(call):
     """A native call gives the interpreter lock back while it allocates and launches, as torch's own operators do."""
