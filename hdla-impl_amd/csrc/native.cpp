@@ -721,7 +721,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
 // layer(x, (wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo), initial_state, want_state, mode, cache,
 //       H, groups, norm_q, norm_v, beta_scale, c, eps, gate_pos) -> (output, state) or None
 // mode: 0 chunked with gradients and from RECURRENT_BELOW tokens on, else token-serial; 1 chunked; 2 token-serial
-// cache: a two-element list that keeps the concatenated weight between calls without gradients, or None
+// cache: a list [key, weight] x 2 that keeps the concatenated weight, narrow and padded, between calls without gradients, or None
 PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 14 || !api.strerror || !is_tensor(a[0]) || !PyTuple_CheckExact(a[1]) || PyTuple_GET_SIZE(a[1]) != 10) return none();
     const Tensor& x = unpack(a[0]);
@@ -783,12 +783,14 @@ PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
         LayerFwd r;
         const LayerCols L(d, f.H, B * T >= PAD_FROM_ROWS);
         // the weight of the last call, as long as the parameters are the ones it was built from, unmodified
-        const bool cached = PyList_CheckExact(a[5]) && PyList_GET_SIZE(a[5]) == 2;
+        // (each width has its own place: a captured graph of decode steps goes on reading the one while long calls use the other)
+        const bool cached = PyList_CheckExact(a[5]) && PyList_GET_SIZE(a[5]) == 4;
+        const Py_ssize_t slot = B * T >= PAD_FROM_ROWS ? 2 : 0;
         struct { const void* p; uint64_t v; } key[7];
         if (cached) {
             for (int i = 0; i < 6; ++i) key[i] = {P[i].data_ptr(), (uint64_t)P[i]._version()};
             key[6] = {nullptr, (uint64_t)L.ld};
-            PyObject *old_key = PyList_GET_ITEM(a[5], 0), *old = PyList_GET_ITEM(a[5], 1);
+            PyObject *old_key = PyList_GET_ITEM(a[5], slot), *old = PyList_GET_ITEM(a[5], slot + 1);
             if (PyBytes_CheckExact(old_key) && PyBytes_GET_SIZE(old_key) == (Py_ssize_t)sizeof key &&
                 !memcmp(PyBytes_AS_STRING(old_key), key, sizeof key) && is_tensor(old)) r.w = unpack(old);
         }
@@ -798,14 +800,14 @@ PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
             if (built) r.w = gather_weights(P, L);
             layer_forward(x, P, f, h0, want, chunked, false, r);
         });
-        if (cached && built && PyList_GET_SIZE(a[5]) == 2) {
+        if (cached && built && PyList_GET_SIZE(a[5]) == 4) {
             // (key and weight one behind the other, with the lock held: another thread sees both or neither)
             PyObject* const k = PyBytes_FromStringAndSize(reinterpret_cast<const char*>(key), sizeof key);
             if (!k) return nullptr;
             PyObject* const w = THPVariable_Wrap(r.w);
             if (!w) { Py_DECREF(k); return nullptr; }
-            PyList_SetItem(a[5], 0, k);
-            PyList_SetItem(a[5], 1, w);
+            PyList_SetItem(a[5], slot, k);
+            PyList_SetItem(a[5], slot + 1, w);
         }
         return pair(r.out, r.ht);
     });

@@ -147,7 +147,7 @@ class HDLA_Custom(nn.Module):
         # the form the native host path runs as one call, as far as the constructor decides it
         self._common = (self._all_silu and use_beta and use_output_gate and not bias and num_blocks == 1 and not use_offset
                         and gate_act == "sigmoid" and gate_pos in ("pre", "post"))
-        self._native_cache = [None, None]
+        self._native_cache = [None] * 4
         self._init_weights()
 
     # ---- initialisation: hdla_custom.py:159-187 and normalization_utils.py:115-211 (the branches a module of this
@@ -208,9 +208,9 @@ class HDLA_Custom(nn.Module):
         return self._gathered_val
 
     def reset_cache(self):
-        """Forget the concatenated projection weight of evaluation mode."""
+        """Forget the concatenated projection weight of evaluation mode (a captured graph that reads it must be captured anew)."""
         self._gathered_key = self._gathered_val = None
-        self._native_cache = [None, None]
+        self._native_cache = [None] * 4
 
     def train(self, mode: bool = True):
         self.reset_cache()

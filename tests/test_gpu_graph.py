@@ -103,3 +103,32 @@ def test_decode_step_replay_carries_the_state():
         torch.cuda.synchronize()
         o_ref, S_ref = fused_recurrent_hdla_delta_rule(*new, scale=1.0, initial_state=S_ref, output_final_state=True)
         assert torch.equal(static_out[0], o_ref) and torch.equal(S, S_ref), f"decode replay {i}"
+
+
+def test_layer_decode_replay_between_long_prefills():
+    """A captured decode step of the layer reads the concatenated weight that evaluation mode keeps: long calls in between, which
+    use a padded one, must leave it where it is."""
+    from hdla_hip.layer import HDLA_Custom, RecurrentCache
+    torch.manual_seed(5)
+    m = HDLA_Custom(256, 4, token_mixer_init_type=2, rescale_type=0).to(DEV).bfloat16().eval()
+    x = torch.randn(3, 1, 256, device=DEV).bfloat16()
+    prompt = torch.randn(1, 1100, 256, device=DEV).bfloat16()
+    state = torch.randn(3, 4, 64, 64, device=DEV)
+
+    def step(x, state):
+        cache = RecurrentCache()
+        cache.update(recurrent_state=[state])
+        y, cache = m(x, past_key_values=cache, use_cache=True)
+        return [y, cache[0]["recurrent_state"][0]]
+
+    with torch.no_grad():
+        g, static_out = _capture(lambda: step(x, state))
+        for i in range(4):
+            m(prompt, past_key_values=RecurrentCache(), use_cache=True)
+            junk = [torch.full((1 << 20,), float("nan"), device=DEV) for _ in range(8)]
+            x.copy_(torch.randn(3, 1, 256, generator=torch.Generator().manual_seed(i)))
+            g.replay()
+            torch.cuda.synchronize()
+            got = [t.clone() for t in static_out]
+            del junk
+            assert all(torch.equal(a, b) for a, b in zip(got, step(x, state))), f"replay {i}"
