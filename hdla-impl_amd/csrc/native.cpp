@@ -17,6 +17,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <dlfcn.h>
 #include <torch/csrc/Exceptions.h>
@@ -795,12 +796,17 @@ PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
                 !memcmp(PyBytes_AS_STRING(old_key), key, sizeof key) && is_tensor(old)) r.w = unpack(old);
         }
         const bool built = !r.w.defined();
+        bool keep = false;
         unlocked([&] {
             const at::DeviceGuard guard(dev);
-            if (built) r.w = gather_weights(P, L);
+            if (built) {
+                r.w = gather_weights(P, L);
+                // (one gathered under capture is not there before the graph is replayed, and belongs to it)
+                keep = cached && c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None;
+            }
             layer_forward(x, P, f, h0, want, chunked, false, r);
         });
-        if (cached && built && PyList_GET_SIZE(a[5]) == 4) {
+        if (keep && PyList_GET_SIZE(a[5]) == 4) {
             // (key and weight one behind the other, with the lock held: another thread sees both or neither)
             PyObject* const k = PyBytes_FromStringAndSize(reinterpret_cast<const char*>(key), sizeof key);
             if (!k) return nullptr;

@@ -204,6 +204,10 @@ class HDLA_Custom(nn.Module):
             with torch.no_grad():
                 w = torch.cat([m.weight for m in heads], dim=0)
                 b = torch.cat([m.bias for m in heads], dim=0) if heads[0].bias is not None else None
+            if w.is_cuda:
+                with torch.cuda.device(w.device):
+                    if torch.cuda.is_current_stream_capturing():           # not there before the graph is replayed
+                        return w, b
             self._gathered_key, self._gathered_val = key, (w, b)
         return self._gathered_val
 

@@ -132,3 +132,23 @@ def test_layer_decode_replay_between_long_prefills():
             got = [t.clone() for t in static_out]
             del junk
             assert all(torch.equal(a, b) for a, b in zip(got, step(x, state))), f"replay {i}"
+
+
+@pytest.mark.parametrize("common", [True, False])                 # one native call, the steps
+def test_layer_first_called_under_capture(common):
+    """What evaluation mode keeps must not come from a capture: it is not there before the graph is replayed."""
+    from hdla_hip.layer import HDLA_Custom
+    torch.manual_seed(6)
+    ms = [HDLA_Custom(256, 4, token_mixer_init_type=2, rescale_type=0).to(DEV).bfloat16().eval() for _ in range(2)]
+    ms[1].load_state_dict(ms[0].state_dict())
+    x = torch.randn(3, 1, 256, device=DEV).bfloat16()
+    for m in ms:
+        m._common = common
+    with torch.no_grad():
+        ref = ms[0](x)[0]
+        g, out = _capture(lambda: ms[1](x)[0], warmup=0)
+        assert torch.equal(ms[1](x)[0], ref)
+        for _ in range(3):
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, ref) and torch.equal(ms[1](x)[0], ref)
