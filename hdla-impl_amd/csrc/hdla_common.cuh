@@ -458,7 +458,11 @@ template <int N> __device__ __forceinline__ bool strong_decay(const f32x4 (&gi)[
 // An exponential is 16 cycles of a SIMD (a quarter-rate instruction) and a multiplication before it; but ge of a token is
 // gi of the token before it, and the second group is the first times e^{m} and e^{gl-m}: three exponentials and lane moves
 // in place of seven.  Products of two factors of the safe range stay inside that of fp32; a tile beyond it (its scores
-// take the strong-decay route) forms the second group directly.
+// take the strong-decay route) forms the second group directly.  A product carries one rounding of 2^-24 more than an exponential,
+// and the backward kernels form their factors directly: beside operands of 8 bits neither is seen.  Errors against a float64
+// evaluation, mean of 12 training steps of 4 x 512 tokens, 16 heads, relative to those with every factor an exponential of its own:
+// 1.0000 (outputs), 0.9999 to 1.0002 (final state, gradients), standard errors up to 0.0002; the products save 1.3 us of a training
+// step of 4 x 2048 tokens and 0.3 us of a forward pass.
 // Measured on 8192 tokens x 16 heads, K = V = 64 (with the producers' reordering in the fused kernels that came with it):
 // forward 75.2 -> 73.8 us, checkpoints 78.6 -> 76.1, reverse 70.7 -> 69.0.
 constexpr float LOG2E = 1.44269504088896340736f;

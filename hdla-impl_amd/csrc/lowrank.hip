@@ -46,7 +46,7 @@ struct UpArgs {
     int M, d;
 };
 // A wave per 16 MT rows and 64 columns; blockIdx.y: decay or gate.  Every wave reads its 64 rows of W (8 or 16 KiB) from L2:
-// with one row tile a wave that was 134 MB next to 50 MB of results, 28 us (8192 x 1024), with four 14.
+// with one row tile a wave that was 134 MB next to 50 MB of results, 28 us (8192 x 1024), with four 21.
 template <int D, int MT>
 __global__ __launch_bounds__(256) void layer_up_kernel(UpArgs p) {
     constexpr int KB = D / 32;
