@@ -81,6 +81,9 @@ class RecurrentCache:
 class HDLA_Custom(nn.Module):
     """S[t] = (I - beta k k^T) Diag(f) (I - beta k k^T) S[t-1] + k v^T,  o[t] = S[t]^T q[t]   (hdla_custom.py:46-62,270-288)."""
 
+    # what a module that was pickled whole before there was a native call does not bring along: it runs as steps
+    _common, _native_cache = False, None
+
     def __init__(
         self,
         embed_dim: int,

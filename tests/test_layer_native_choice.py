@@ -119,3 +119,20 @@ def test_the_scale_of_the_norm_is_its_own(native):
     for kw, c in (({}, 128 ** 0.5), ({"token_mixer_norm_type": "grouprmsnorm"}, 8.0)):
         m = _layer(**kw)
         assert _taken(m, native) and native.calls[-1][11] == c
+
+
+def test_a_module_pickled_before_there_was_a_native_call(native):
+    import io
+    m = _layer()
+    for n in ("_common", "_native_cache"):
+        del m.__dict__[n]
+    buf = io.BytesIO()
+    torch.save(m, buf)
+    buf.seek(0)
+    old = torch.load(buf, weights_only=False)                      # written right here
+    assert not old._common and old._native_cache is None
+    with pytest.raises(AttributeError, match="normalize"):         # the steps (the recorder has nothing but the layer's call)
+        old(torch.zeros(1, 4, 128))
+    assert not native.calls
+    old.eval()
+    assert len(old._native_cache) == 4
