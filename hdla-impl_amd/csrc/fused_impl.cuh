@@ -119,6 +119,7 @@ template <typename T, bool GKF32> struct GkRaw {
     typedef i32x4 rows;
     static __device__ __forceinline__ void load(const char* p, int l, uint32_t row_ch, rows& x) { x = *reinterpret_cast<const i32x4*>(at(p, 2 * row_ch + 16 * (l & 3))); }
     static __device__ __forceinline__ void tiles(char* scratch, int l, rows x, type (&f)[2]) { rows_to_tiles(scratch, l, x, f[0], f[1]); }
+    static __device__ __forceinline__ void drop(rows& x) { forget(x); }
     static __device__ __forceinline__ f32x4 value(type x) { return to_f32(x); }
     static __device__ __forceinline__ void mask(type& x, bool ok) { x.v = ok ? x.v : zero_frag<T>().v; }
 };
@@ -133,6 +134,7 @@ template <typename T> struct GkRaw<T, true> {
 #pragma unroll
         for (int j = 0; j < 2; ++j) f[j] = rows_to_tile(scratch, l, x.x[j]);
     }
+    static __device__ __forceinline__ void drop(rows& x) { forget(x.x[0]); forget(x.x[1]); }
     static __device__ __forceinline__ f32x4 value(type x) { return x; }
     static __device__ __forceinline__ void mask(type& x, bool ok) { x = ok ? x : zero4(); }
 };
@@ -276,6 +278,16 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
     auto mask = [](Frag<T>& f, bool ok) __attribute__((always_inline)) { f.v = ok ? f.v : zero_frag<T>().v; };
     auto mask_gk = [](typename GkRaw<T, GKF32>::type& x, bool ok) __attribute__((always_inline)) { GkRaw<T, GKF32>::mask(x, ok); };
     if (pp < nst) { request(pp, 0); request(pp, 1); }
+    // (the requested inputs are forgotten where the wave ends early, and where they may or may not be requested again: otherwise
+    // their old values stay in registers through the whole chunk)
+    auto forget_first = [&]() __attribute__((always_inline)) { GkRaw<T, GKF32>::drop(xg); forget(xk); forget(xb[0]); forget(xb[1]); };
+    auto forget_rest = [&]() __attribute__((always_inline)) { GkRaw<T, GKF32>::drop(xog); forget(xok); forget(xq); forget(xa[0]); forget(xa[1]); };
+    auto gave_up = [&]() __attribute__((always_inline)) {
+        if (l == 0) *a.err = FUSED_ABORTED + 1;
+        forget_first();
+        forget_rest();
+        forget(xv);
+    };
 
     int it = 0, prev_cid = -1;
     for (int t = pp; t < nst; t += FNP, ++it) {
@@ -396,20 +408,15 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
                 {
                     Split<T> qh;
                     split(to_f32(rq) * e.eq * scale, qh);
-                    if (FWD) aqk = mm3(qh, kh, aqk);
-#pragma unroll
-                    for (int s = 0; s < 2; ++s) {
-                        aqb[s] = mm3(qh, bh[s], aqb[s]);
-                    }
+                    if constexpr (FWD) mm_split<3>(qh, {&kh, &bh[0], &bh[1]}, {&aqk, &aqb[0], &aqb[1]});
+                    else mm_split<2>(qh, {&bh[0], &bh[1]}, {&aqb[0], &aqb[1]});
                 }
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int r = 0; r < 2; ++r) {
                     Split<T> ah;
                     split(to_f32(ra[r]) * e.ea, ah);
-                    aak[r] = mm3(ah, kh, aak[r]);
-                    aab[r][0] = mm3(ah, bh[0], aab[r][0]);
-                    aab[r][1] = mm3(ah, bh[1], aab[r][1]);
+                    mm_split<3>(ah, {&kh, &bh[0], &bh[1]}, {&aak[r], &aab[r][0], &aab[r][1]});
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
@@ -442,21 +449,21 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
                     Split<T> qh, kh, bh[2];
                     split(to_f32(rk) * ek, kh);
                     split(to_f32(rq) * eq * scale, qh);
-                    if (FWD) aqk = mm3(qh, kh, aqk);
+                    if (FWD) aqk = mm_split(qh, kh, aqk);
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int s = 0; s < 2; ++s) {
                         split(to_f32(rb[s]) * ek, bh[s]);
-                        aqb[s] = mm3(qh, bh[s], aqb[s]);
+                        aqb[s] = mm_split(qh, bh[s], aqb[s]);
                         __builtin_amdgcn_sched_barrier(0);
                     }
 #pragma unroll
                     for (int r = 0; r < 2; ++r) {
                         Split<T> ah;
                         split(to_f32(ra[r]) * ea, ah);
-                        aak[r] = mm3(ah, kh, aak[r]);
-                        aab[r][0] = mm3(ah, bh[0], aab[r][0]);
-                        aab[r][1] = mm3(ah, bh[1], aab[r][1]);
+                        aak[r] = mm_split(ah, kh, aak[r]);
+                        aab[r][0] = mm_split(ah, bh[0], aab[r][0]);
+                        aab[r][1] = mm_split(ah, bh[1], aab[r][1]);
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 }
@@ -477,7 +484,7 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
         request(t, 2);
         __builtin_amdgcn_sched_barrier(0);
         // ---- the slot: wait until the consumers have left the chunk it held ---------------------------------------------
-        if (!wait_ge(f_consumed, VT * it, f_abort)) { if (l == 0) *a.err = FUSED_ABORTED + 1; return; }
+        if (!wait_ge(f_consumed, VT * it, f_abort)) { gave_up(); return; }
         __builtin_amdgcn_sched_barrier(0);
         // ---- gated copies of the own channel tiles (prep.hip, phase C), each to its half of the stored pair --------------
 #pragma unroll
@@ -488,13 +495,12 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
             Frag<T> rq, rk, ra[2], rb[2];
             operands(j, HD ? GkRaw<T, GKF32>::value(ng[j]) : zero4(), rq, rk, ra, rb);
             const f32x4 one = {1.f, 1.f, 1.f, 1.f}, ege = prev_token(egi[j], one), egl = bcast16<CH - 1>(egi[j]);
-            st_pair(sWW + (0 * KT2 + half) * PAIR, j, transpose(to_frag<T>(to_f32(ra[0]) * ege), ident));
-            st_pair(sWW + (1 * KT2 + half) * PAIR, j, transpose(to_frag<T>(to_f32(ra[1]) * ege), ident));
+            st_pair2(sWW + (j * KT2 + half) * PAIR, transpose(to_frag<T>(to_f32(ra[0]) * ege), ident),
+                     transpose(to_frag<T>(to_f32(ra[1]) * ege), ident));
             const Frag<T> fqg = to_frag<T>(to_f32(rq) * egi[j] * scale);
             const Frag<T> fbg[2] = {to_frag<T>(to_f32(rb[0]) * edn[j]), to_frag<T>(to_f32(rb[1]) * edn[j])};
             st_pair(reinterpret_cast<T*>(slot + BF.KGT) + half * PAIR, j, transpose(to_frag<T>(to_f32(rk) * edn[j]), ident));
-            st_pair(reinterpret_cast<T*>(slot + BF.BGT) + (0 * KT2 + half) * PAIR, j, transpose(fbg[0], ident));
-            st_pair(reinterpret_cast<T*>(slot + BF.BGT) + (1 * KT2 + half) * PAIR, j, transpose(fbg[1], ident));
+            st_pair2(reinterpret_cast<T*>(slot + BF.BGT) + (kt0 + j) * PAIR, transpose(fbg[0], ident), transpose(fbg[1], ident));
             st_pair(reinterpret_cast<T*>(slot + BF.QG) + half * PAIR, j, fqg);
             if (c == 0) *reinterpret_cast<f32x4*>(slot + BF.EGL + (16 * (kt0 + j) + 4 * g) * 4) = egl;
             __builtin_amdgcn_sched_barrier(0);
@@ -509,13 +515,14 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
         }
         // the inputs are used up: the next chunk's may come
         __builtin_amdgcn_sched_barrier(0);
+        forget_first();
         if (t + FNP < nst) request(t + FNP, 0);
         __builtin_amdgcn_sched_barrier(0);
 
         // ---- the lead: whole score tiles, (I - A_ab)^-1 by forward substitution (prep.hip, phase B) ---------------------
         Frag<T> tm[2][2], aakf[2];
         if (lead) {
-            if (!wait_ge(f_part, it + 1, f_abort)) { if (l == 0) *a.err = FUSED_ABORTED + 1; return; }
+            if (!wait_ge(f_part, it + 1, f_abort)) { gave_up(); return; }
             f32x4* const tiles[9] = {&aab[0][0], &aab[0][1], &aab[1][0], &aab[1][1], &aak[0], &aak[1],
                                      &aqb[0], &aqb[1], &aqk};
             // the lower channel tiles' part first, as a single wave adds them
@@ -593,10 +600,10 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
                 Split<T> pa, pb;
                 split(tllT, pa);
                 split(ahl, pb);
-                const f32x4 xT = mm3(pa, pb, zero4());    // (A_HL T_LL)^T = T_LL^T A_HL^T
+                const f32x4 xT = mm_split(pa, pb, zero4());    // (A_HL T_LL)^T = T_LL^T A_HL^T
                 split(thh, pa);
                 split(xT, pb);
-                const f32x4 thl = mm3(pa, pb, zero4());   // T_HH (A_HL T_LL)
+                const f32x4 thl = mm_split(pa, pb, zero4());   // T_HH (A_HL T_LL)
                 *reinterpret_cast<f32x4*>(&sT[(16 * rr + 8 + ii) * FLDP + 16 * ss + j0]) = thl;
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -623,26 +630,25 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
             // while the lead solves: the rows the consumers left in the outbox for the chunk the slot held (they write the
             // outbox again only after both signals at the end)
             if (it > 0) copy_out(prev_cid, 0, std::integral_constant<int, CH>());
-            if (!wait_ge(f_inv, it + 1, f_abort)) { if (l == 0) *a.err = FUSED_ABORTED + 1; return; }
+            if (!wait_ge(f_inv, it + 1, f_abort)) { gave_up(); return; }
 #pragma unroll
             for (int s = 0; s < 2; ++s) ld_pair(sPub + s * PAIR, tm[s][0], tm[s][1]);
             ld_pair(sPub + 2 * PAIR, aakf[0], aakf[1]);
         }
         __builtin_amdgcn_sched_barrier(0);
+        forget_rest();
         if (t + FNP < nst) request(t + FNP, 1);
         __builtin_amdgcn_sched_barrier(0);
         // ---- w = Tm ag for the own channel tiles, in place of ag^T -------------------------------------------------------
         {
             Frag<T> agT[2][2], fw[2][2];
-            ld_pair(sWW + (0 * KT2 + half) * PAIR, agT[0][0], agT[0][1]);
-            ld_pair(sWW + (1 * KT2 + half) * PAIR, agT[1][0], agT[1][1]);
+            ld_pair(sWW + half * PAIR, agT[0][0], agT[1][0]);
+            ld_pair(sWW + (KT2 + half) * PAIR, agT[0][1], agT[1][1]);
 #pragma unroll
             for (int e = 0; e < 2; ++e)
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
-                    f32x4 w = mm(tm[s][0], agT[0][e], zero4());
-                    w = mm(tm[s][1], agT[1][e], w);
-                    fw[s][e] = to_frag<T>(w);
+                    fw[s][e] = to_frag<T>(mm2(tm[s][0], tm[s][1], agT[0][e], agT[1][e], zero4()));
                 }
 #pragma unroll
             for (int s = 0; s < 2; ++s) st_pair2(sWW + (s * KT2 + half) * PAIR, fw[s][0], fw[s][1]);
@@ -654,9 +660,7 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
             Frag<T> fu[2];
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
-                f32x4 uT = mm(mT[0], tm[s][0], zero4());
-                uT = mm(mT[1], tm[s][1], uT);
-                fu[s] = to_frag<T>(uT);
+                fu[s] = to_frag<T>(mm2(mT[0], mT[1], tm[s][0], tm[s][1], zero4()));
             }
             st_pair2(reinterpret_cast<T*>(slot + L::UT) + (vt0 + j) * PAIR, fu[0], fu[1]);
         }
@@ -869,15 +873,7 @@ __device__ __forceinline__ void fused_replay(const FusedArgs<T>& a, char* smem, 
         for (int j = 0; j < KH; ++j)
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
-                f32x4 w;
-                if (REV) {
-                    w = mm(agT[0][j], tm[s][0], zero4());
-                    w = mm(agT[1][j], tm[s][1], w);
-                } else {
-                    w = mm(tm[s][0], agT[0][j], zero4());
-                    w = mm(tm[s][1], agT[1][j], w);
-                }
-                fw[s][j] = to_frag<T>(w);
+                fw[s][j] = to_frag<T>(REV ? mm2(agT[0][j], agT[1][j], tm[s][0], tm[s][1], zero4()) : mm2(tm[s][0], tm[s][1], agT[0][j], agT[1][j], zero4()));
             }
         if (!REV) {
 #pragma unroll
@@ -885,9 +881,7 @@ __device__ __forceinline__ void fused_replay(const FusedArgs<T>& a, char* smem, 
                 const Frag<T> mT[2] = {to_frag<T>(mm(vT[j], aq[0], zero4())), to_frag<T>(mm(vT[j], aq[1], zero4()))};
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
-                    f32x4 uT = mm(mT[0], tm[s][0], zero4());
-                    uT = mm(mT[1], tm[s][1], uT);
-                    fu[j][s] = to_frag<T>(uT);
+                    fu[j][s] = to_frag<T>(mm2(mT[0], mT[1], tm[s][0], tm[s][1], zero4()));
                 }
             }
         }
@@ -897,8 +891,14 @@ __device__ __forceinline__ void fused_replay(const FusedArgs<T>& a, char* smem, 
         T* const sW = reinterpret_cast<T*>(slot + (REV ? SB.W : BF.W)), * const sB = reinterpret_cast<T*>(slot + (REV ? SB.BGT : BF.BGT));
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
-            st_pair2(sW + (s * KT2 + half) * PAIR, fw[s][0], fw[s][1]);
-            st_pair2(sB + (s * KT2 + half) * PAIR, fb[s][0], fb[s][1]);
+            // the operand of the v_new products pairs two channel tiles, that of the state update the two ranks of a channel tile
+            if (REV) {
+                st_pair2(sW + (kt0 + s) * PAIR, fw[0][s], fw[1][s]);
+                st_pair2(sB + (s * KT2 + half) * PAIR, fb[s][0], fb[s][1]);
+            } else {
+                st_pair2(sW + (s * KT2 + half) * PAIR, fw[s][0], fw[s][1]);
+                st_pair2(sB + (kt0 + s) * PAIR, fb[0][s], fb[1][s]);
+            }
         }
         st_pair2(reinterpret_cast<T*>(slot + (REV ? SB.QGT : BF.KGT)) + half * PAIR, fx[0], fx[1]);
         if (REV && half == 0) st_pair2(reinterpret_cast<T*>(slot + SB.AQBT), aq[0], aq[1]);
@@ -985,8 +985,8 @@ __device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* 
 #pragma unroll
         for (int kp = 0; kp < KT2; ++kp) {
             ld_pair(sKGT + kp * PAIR, kgt[2 * kp], kgt[2 * kp + 1]);
-            ld_pair(sBGT + (0 * KT2 + kp) * PAIR, bgt[0][2 * kp], bgt[0][2 * kp + 1]);
-            ld_pair(sBGT + (1 * KT2 + kp) * PAIR, bgt[1][2 * kp], bgt[1][2 * kp + 1]);
+            ld_pair(sBGT + (2 * kp) * PAIR, bgt[0][2 * kp], bgt[1][2 * kp]);
+            ld_pair(sBGT + (2 * kp + 1) * PAIR, bgt[0][2 * kp + 1], bgt[1][2 * kp + 1]);
             egl[2 * kp] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (2 * kp) + 4 * g);
             egl[2 * kp + 1] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (2 * kp + 1) + 4 * g);
         }
@@ -995,17 +995,21 @@ __device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* 
         Frag<T> sb[KT];
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) sb[kt] = to_frag<T>(S[kt]);
-        f32x4 vn[2] = {to_f32(ut[0]), to_f32(ut[1])};
+        // first what is one product a sum, then the rest in twos: one change of instruction for all accumulators (see mm2)
+        f32x4 x[KT + 1];
+        x[KT] = FWD ? mm(aqk, vtt, zero4()) : zero4();
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt) {
-            vn[0] = mm(sb[kt], w[0][kt], vn[0]);
-            vn[1] = mm(sb[kt], w[1][kt], vn[1]);
+        for (int kt = 0; kt < KT; ++kt) x[kt] = mm(vtt, kgt[kt], S[kt] * egl[kt]);
+        settle<T>(x);
+        f32x4 vn[2] = {to_f32(ut[0]), to_f32(ut[1])}, o = x[KT];
+#pragma unroll
+        for (int kp = 0; kp < KT2; ++kp) {
+            vn[0] = mm2(sb[2 * kp], sb[2 * kp + 1], w[0][2 * kp], w[0][2 * kp + 1], vn[0]);
+            vn[1] = mm2(sb[2 * kp], sb[2 * kp + 1], w[1][2 * kp], w[1][2 * kp + 1], vn[1]);
         }
-        f32x4 o = zero4();
         if (FWD) {
 #pragma unroll
-            for (int kt = 0; kt < KT; ++kt) o = mm(qg[kt], sb[kt], o);
-            o = mm(aqk, vtt, o);
+            for (int kp = 0; kp < KT2; ++kp) o = mm2(qg[2 * kp], qg[2 * kp + 1], sb[2 * kp], sb[2 * kp + 1], o);
         }
         const Frag<T> vnb[2] = {to_frag<T>(vn[0]), to_frag<T>(vn[1])};
         if (p.ws.TM) {
@@ -1018,20 +1022,13 @@ __device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* 
             st_pair2(dst, t0, t1);
         }
         if (FWD) {
-            o = mm(aqb[0], vnb[0], o);
-            o = mm(aqb[1], vnb[1], o);
+            o = mm2(aqb[0], aqb[1], vnb[0], vnb[1], o);
             char* ob = smem + pp * L::SLOT + L::OBOX + c * L::OROW;
             if (seg == 0) st_frag(reinterpret_cast<T*>(ob) + 16 * wv + 4 * g, to_frag<T>(o));
             else *reinterpret_cast<f32x4*>(ob + (16 * wv + 4 * g) * 4) = o;
         }
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt) {
-            f32x4 x = S[kt] * egl[kt];
-            x = mm(vtt, kgt[kt], x);
-            x = mm(vnb[0], bgt[0][kt], x);
-            x = mm(vnb[1], bgt[1][kt], x);
-            S[kt] = x;
-        }
+        for (int kt = 0; kt < KT; ++kt) S[kt] = mm2(vnb[0], vnb[1], bgt[0][kt], bgt[1][kt], x[kt]);
         // ---- the transition matrix's column block: the same update without the chunk's own input --------------------
         if (pblk) {
             Frag<T> mb[KT];
@@ -1039,26 +1036,20 @@ __device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* 
             for (int kt = 0; kt < KT; ++kt) mb[kt] = to_frag<T>(M[kt]);
             f32x4 vp[2] = {zero4(), zero4()};
 #pragma unroll
-            for (int kt = 0; kt < KT; ++kt) {
-                vp[0] = mm(mb[kt], w[0][kt], vp[0]);
-                vp[1] = mm(mb[kt], w[1][kt], vp[1]);
+            for (int kp = 0; kp < KT2; ++kp) {
+                vp[0] = mm2(mb[2 * kp], mb[2 * kp + 1], w[0][2 * kp], w[0][2 * kp + 1], vp[0]);
+                vp[1] = mm2(mb[2 * kp], mb[2 * kp + 1], w[1][2 * kp], w[1][2 * kp + 1], vp[1]);
             }
             f32x4 G = zero4();
 #pragma unroll
-            for (int kt = 0; kt < KT; ++kt) G = mm(qg[kt], mb[kt], G);
+            for (int kp = 0; kp < KT2; ++kp) G = mm2(qg[2 * kp], qg[2 * kp + 1], mb[2 * kp], mb[2 * kp + 1], G);
             const Frag<T> vpb[2] = {to_frag<T>(vp[0]), to_frag<T>(vp[1])};
-            G = mm(aqb[0], vpb[0], G);
-            G = mm(aqb[1], vpb[1], G);
+            G = mm2(aqb[0], aqb[1], vpb[0], vpb[1], G);
             const Frag<T> Gf = to_frag<T>(G);             // rows token, inner k' (the block's columns)
             if (FWD) st_frag(reinterpret_cast<T*>(smem + pp * L::SLOT + L::GBOX + c * L::GROW) + 16 * wv + 4 * g, Gf);
             else st_frag(a.gw + (chw * CH + c) * K + 16 * wv + 4 * g, Gf);
 #pragma unroll
-            for (int kt = 0; kt < KT; ++kt) {
-                f32x4 x = M[kt] * egl[kt];
-                x = mm(vpb[0], bgt[0][kt], x);
-                x = mm(vpb[1], bgt[1][kt], x);
-                M[kt] = x;
-            }
+            for (int kt = 0; kt < KT; ++kt) M[kt] = mm2(vpb[0], vpb[1], bgt[0][kt], bgt[1][kt], M[kt] * egl[kt]);
         }
         signal_add(&flags[4 + pp]);
     }
@@ -1152,8 +1143,8 @@ __device__ __forceinline__ void fused_consumer_ckpt(const FusedArgs<T>& a, char*
 #pragma unroll
         for (int kp = 0; kp < KT2; ++kp) {
             ld_pair(sKGT + kp * PAIR, kgt[2 * kp], kgt[2 * kp + 1]);
-            ld_pair(sBGT + (0 * KT2 + kp) * PAIR, bgt[0][2 * kp], bgt[0][2 * kp + 1]);
-            ld_pair(sBGT + (1 * KT2 + kp) * PAIR, bgt[1][2 * kp], bgt[1][2 * kp + 1]);
+            ld_pair(sBGT + (2 * kp) * PAIR, bgt[0][2 * kp], bgt[1][2 * kp]);
+            ld_pair(sBGT + (2 * kp + 1) * PAIR, bgt[0][2 * kp + 1], bgt[1][2 * kp + 1]);
             egl[2 * kp] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (2 * kp) + 4 * g);
             egl[2 * kp + 1] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (2 * kp + 1) + 4 * g);
         }
@@ -1168,11 +1159,15 @@ __device__ __forceinline__ void fused_consumer_ckpt(const FusedArgs<T>& a, char*
         Frag<T> sb[KT];
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) sb[kt] = to_frag<T>(S[kt]);
+        f32x4 x[KT];
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) x[kt] = mm(vtt, kgt[kt], S[kt] * egl[kt]);
+        settle<T>(x);
         f32x4 vn[2] = {to_f32(ut[0]), to_f32(ut[1])};
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt) {
-            vn[0] = mm(sb[kt], w[0][kt], vn[0]);
-            vn[1] = mm(sb[kt], w[1][kt], vn[1]);
+        for (int kp = 0; kp < KT2; ++kp) {
+            vn[0] = mm2(sb[2 * kp], sb[2 * kp + 1], w[0][2 * kp], w[0][2 * kp + 1], vn[0]);
+            vn[1] = mm2(sb[2 * kp], sb[2 * kp + 1], w[1][2 * kp], w[1][2 * kp + 1], vn[1]);
         }
         const Frag<T> vnb[2] = {to_frag<T>(vn[0]), to_frag<T>(vn[1])};
         T* hc = p.ws.HC + chw * (K * V) + vt * PAIR;
@@ -1189,13 +1184,7 @@ __device__ __forceinline__ void fused_consumer_ckpt(const FusedArgs<T>& a, char*
                     if (wv == s * KT2 + kp) st_pair2(wg + (s * KT2 + kp) * PAIR, w[s][2 * kp], w[s][2 * kp + 1]);
         }
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt) {
-            f32x4 x = S[kt] * egl[kt];
-            x = mm(vtt, kgt[kt], x);
-            x = mm(vnb[0], bgt[0][kt], x);
-            x = mm(vnb[1], bgt[1][kt], x);
-            S[kt] = x;
-        }
+        for (int kt = 0; kt < KT; ++kt) S[kt] = mm2(vnb[0], vnb[1], bgt[0][kt], bgt[1][kt], x[kt]);
         if (later) {
             // R[k'][v] += sum_tok G[tok][k'] do[tok][v]
 #pragma unroll
@@ -1314,7 +1303,7 @@ __device__ __forceinline__ void fused_consumer_rev(const FusedArgs<T>& a, char* 
                             Split<T> q;
                             q.hi = ld_frag(sM + ((b * 2 + 0) * KT * KT + ki * KT + ko) * TILE);
                             q.lo = ld_frag(sM + ((b * 2 + 1) * KT * KT + ki * KT + ko) * TILE);
-                            acc = mm3(xs[ki], q, acc);
+                            acc = mm_split(xs[ki], q, acc);
                         }
                         dS[ko] = acc;
                     }
@@ -1344,8 +1333,8 @@ __device__ __forceinline__ void fused_consumer_rev(const FusedArgs<T>& a, char* 
             ld_pair(sBG + (0 * KT2 + kp) * PAIR, bg[0][2 * kp], bg[0][2 * kp + 1]);
             ld_pair(sBG + (1 * KT2 + kp) * PAIR, bg[1][2 * kp], bg[1][2 * kp + 1]);
             ld_pair(sQGT + kp * PAIR, qgt[2 * kp], qgt[2 * kp + 1]);
-            ld_pair(sWT + (0 * KT2 + kp) * PAIR, wt[0][2 * kp], wt[0][2 * kp + 1]);
-            ld_pair(sWT + (1 * KT2 + kp) * PAIR, wt[1][2 * kp], wt[1][2 * kp + 1]);
+            ld_pair(sWT + (2 * kp) * PAIR, wt[0][2 * kp], wt[1][2 * kp]);
+            ld_pair(sWT + (2 * kp + 1) * PAIR, wt[0][2 * kp + 1], wt[1][2 * kp + 1]);
             egl[2 * kp] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (2 * kp) + 4 * g);
             egl[2 * kp + 1] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (2 * kp + 1) + 4 * g);
         }
@@ -1353,13 +1342,18 @@ __device__ __forceinline__ void fused_consumer_rev(const FusedArgs<T>& a, char* 
         Frag<T> dsb[KT];
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) dsb[kt] = to_frag<T>(dS[kt]);
-        f32x4 dvn[2];
-        dvn[0] = mm(doT, aq[0], zero4());
-        dvn[1] = mm(doT, aq[1], zero4());
+        // (products one by one before those in twos, as in the forward direction; x: dv_new of both ranks, then the state)
+        f32x4 x[2 + KT];
+        x[0] = mm(doT, aq[0], zero4());
+        x[1] = mm(doT, aq[1], zero4());
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt) {
-            dvn[0] = mm(dsb[kt], bg[0][kt], dvn[0]);
-            dvn[1] = mm(dsb[kt], bg[1][kt], dvn[1]);
+        for (int kt = 0; kt < KT; ++kt) x[2 + kt] = mm(doT, qgt[kt], dS[kt] * egl[kt]);
+        settle<T>(x);
+        f32x4 dvn[2] = {x[0], x[1]};
+#pragma unroll
+        for (int kp = 0; kp < KT2; ++kp) {
+            dvn[0] = mm2(dsb[2 * kp], dsb[2 * kp + 1], bg[0][2 * kp], bg[0][2 * kp + 1], dvn[0]);
+            dvn[1] = mm2(dsb[2 * kp], dsb[2 * kp + 1], bg[1][2 * kp], bg[1][2 * kp + 1], dvn[1]);
         }
         const Frag<T> dvb[2] = {to_frag<T>(dvn[0]), to_frag<T>(dvn[1])};
         T* dhc = p.ws.DHC + chw * (K * V) + vt * PAIR;
@@ -1368,13 +1362,7 @@ __device__ __forceinline__ void fused_consumer_rev(const FusedArgs<T>& a, char* 
         for (int kp = 0; kp < KT2; ++kp) st_pair2(dhc + kp * (VT * PAIR), dsb[2 * kp], dsb[2 * kp + 1]);
         st_pair2(dvp, dvb[0], dvb[1]);
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt) {
-            f32x4 x = dS[kt] * egl[kt];
-            x = mm(doT, qgt[kt], x);
-            x = mm(dvb[0], wt[0][kt], x);
-            x = mm(dvb[1], wt[1][kt], x);
-            dS[kt] = x;
-        }
+        for (int kt = 0; kt < KT; ++kt) dS[kt] = mm2(dvb[0], dvb[1], wt[0][kt], wt[1][kt], x[2 + kt]);
         signal_add(&flags[4 + pp]);
     }
     if (seg == 0 && p.dh0) {
@@ -1533,7 +1521,7 @@ __global__ __launch_bounds__(256) void fixup_kernel(FusedArgs<T> a) {
 #pragma unroll
         for (int b = 0; b < FIXUP_STAGE; ++b) {
             if (b < ns) {
-                // X^T <- X^T Q^T + A^T in split 2-byte products (three per tile pair: the error of fp32 products); tile
+                // X^T <- X^T Q^T + A^T in split 2-byte products (the error of fp32 products); tile
                 // (out, in) of the record is at index out * KT + in
                 Split<T> xs[KT];
 #pragma unroll
@@ -1546,7 +1534,7 @@ __global__ __launch_bounds__(256) void fixup_kernel(FusedArgs<T> a) {
                         Split<T> q;
                         q.hi = ld_tile(sM[b][0] + (ko * KT + ki) * TILE);
                         q.lo = ld_tile(sM[b][1] + (ko * KT + ki) * TILE);
-                        acc = mm3(xs[ki], q, acc);
+                        acc = mm_split(xs[ki], q, acc);
                     }
                     S[ko] = acc;
                 }
@@ -1586,7 +1574,7 @@ __global__ __launch_bounds__(256) void fixup_kernel(FusedArgs<T> a) {
                 for (int j = 0; j < VT; ++j) {
                     f32x4 o = OLr[b][j];
 #pragma unroll
-                    for (int kt = 0; kt < KT; ++kt) o = mm(G[b][kt], Sb[j][kt], o);
+                    for (int kt = 0; kt < KT; kt += 2) o = mm2(G[b][kt], G[b][kt + 1], Sb[j][kt], Sb[j][kt + 1], o);
                     st_frag(reinterpret_cast<T*>(st + c * OROW) + 16 * j + 4 * g, to_frag<T>(o));
                 }
                 // whole rows, 16 bytes a lane (the wave's own staging area: LDS accesses of one wave complete in order)

@@ -76,6 +76,10 @@ __device__ __forceinline__ void pin(Frag<bf16>& x) { asm volatile("" : "+v"(x.v)
 __device__ __forceinline__ void pin(f32x4& x) { asm volatile("" : "+v"(x)); }
 __device__ __forceinline__ void pin(Frag<float>&) {}     // fp32 operands are used as they are: nothing to hoist
 
+// The value of x is not needed any more; x is left with whatever its registers hold (no instruction).  For what is refilled under a
+// condition: without this the old value stays in its registers until then, for the case that it is not.
+template <typename X> __device__ __forceinline__ void forget(X& x) { asm volatile("" : "=v"(x)); }
+
 __device__ __forceinline__ f32x4 zero4() { f32x4 z = {0.f, 0.f, 0.f, 0.f}; return z; }
 
 // ---- the tile product --------------------------------------------------------------------------------------
@@ -89,13 +93,42 @@ __device__ __forceinline__ f32x4 mm(Frag<float> frows, Frag<float> finner, f32x4
     return acc;
 }
 
-// (The 16x16x32 bf16 MFMA of gfx950 would do two of these products in the time of one.  It is not used: built with
-// it, the state scans gave wrong results that depended on the register allocation, while a kernel of nothing but
-// such products was exact; the cause was not established, and no kernel here is bound by its matrix products.)
+// Two products of 2-byte operands in one instruction, acc += P0 Q0^T + P1 Q1^T: the 16x16x32 MFMA, whose operands are two
+// tiles' fragments side by side (which inner index a lane's element stands for is free as long as both operands agree).
+// Measured, cycles of a SIMD an instruction: 16 either way, also in a chain through the accumulator, so it is two products
+// in the time of one.
+// An accumulator must not go from mm to mm2 or back without settle(): a result is handed to the next product's accumulator
+// inside the matrix unit, which works between two instructions of one shape, and the compiler, which takes the two shapes for one
+// in this respect, inserts no wait.  Measured: with less than 5 wait states in between the second product adds to another
+// number (back to back, a relative difference of 0.5 to 0.6; from 5 on none); results used as operands, or by vector
+// instructions, are waited for correctly.  test_mfma_chains.py looks through the built kernels for such pairs.
+// Where it counts: the fused kernels' waves wait mostly for the instructions of the others on their SIMD.  Forward kernel, 4 x 2048
+// tokens of 16 heads, K = V = 64: 354 -> 222 products a chunk and head, 72.2 -> 69.5 us (the chain of a consumer's step half as long).
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ bf16x8 side_by_side(Frag<bf16> x, Frag<bf16> y) {
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(x.v, y.v, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+__device__ __forceinline__ f32x4 mm2(Frag<bf16> p0, Frag<bf16> p1, Frag<bf16> q0, Frag<bf16> q1, f32x4 acc) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(side_by_side(q0, q1), side_by_side(p0, p1), acc, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mm2(Frag<float> p0, Frag<float> p1, Frag<float> q0, Frag<float> q1, f32x4 acc) {
+    return mm(p1, q1, mm(p0, q0, acc));
+}
+// the accumulators x have left the matrix unit: 8 wait states between what produced them and what uses them
+template <typename T, int N> __device__ __forceinline__ void settle(f32x4 (&x)[N]) {
+    if constexpr (sizeof(T) == 2) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) asm volatile("" : "+v"(x[i]));
+        asm volatile("s_nop 7");
+#pragma unroll
+        for (int i = 0; i < N; ++i) asm volatile("" : "+v"(x[i]));
+    }
+}
 
 // Split operands for the score products of the bf16 path: x = hi + lo with both halves bf16, and
-// P Q^T ~ Ph Qh^T + Ph Ql^T + Pl Qh^T, which removes the rounding of the decayed operands (the largest single
-// contribution to the forward error) at the price of two more MFMAs per product.  fp32 operands need no split.
+// P Q^T ~ (Ph + Pl) (Qh + Ql)^T, which removes the rounding of the decayed operands (the largest single
+// contribution to the forward error) at the price of one more MFMA per product: [Ph Ph] [Qh Ql]^T and [Pl Pl] [Qh Ql]^T.
+// fp32 operands need no split.
 template <typename T> struct Split;
 template <> struct Split<bf16> { Frag<bf16> hi, lo; };
 template <> struct Split<float> { Frag<float> hi; };
@@ -104,12 +137,19 @@ __device__ __forceinline__ void split(f32x4 x, Split<bf16>& s) {
     s.lo = to_frag<bf16>(x - to_f32(s.hi));
 }
 __device__ __forceinline__ void split(f32x4 x, Split<float>& s) { s.hi.v = x; }
-__device__ __forceinline__ f32x4 mm3(const Split<bf16>& p, const Split<bf16>& q, f32x4 acc) {
-    acc = mm(p.lo, q.hi, acc);
-    acc = mm(p.hi, q.lo, acc);
-    return mm(p.hi, q.hi, acc);
+__device__ __forceinline__ f32x4 mm_split(const Split<bf16>& p, const Split<bf16>& q, f32x4 acc) {
+    acc = mm2(p.lo, p.lo, q.hi, q.lo, acc);
+    return mm2(p.hi, p.hi, q.hi, q.lo, acc);
 }
-__device__ __forceinline__ f32x4 mm3(const Split<float>& p, const Split<float>& q, f32x4 acc) { return mm(p.hi, q.hi, acc); }
+__device__ __forceinline__ f32x4 mm_split(const Split<float>& p, const Split<float>& q, f32x4 acc) { return mm(p.hi, q.hi, acc); }
+// one p against several q: the halves of p one after the other, so that only one is held twice at a time
+template <int N> __device__ __forceinline__ void mm_split(const Split<bf16>& p, const Split<bf16>* const (&q)[N], f32x4* const (&acc)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) *acc[i] = mm2(p.lo, p.lo, q[i]->hi, q[i]->lo, *acc[i]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < N; ++i) *acc[i] = mm2(p.hi, p.hi, q[i]->hi, q[i]->lo, *acc[i]);
+}
 
 // F(I16): used to transpose a tile with one product, F(X^T) = mm(F(I), F(X)).
 template <typename T> __device__ __forceinline__ Frag<T> ident_frag() {

@@ -174,13 +174,13 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void 
             split(a1 * ea, ah[1]);
             split(b0 * ek, bh[0]);
             split(b1 * ek, bh[1]);
-            aqk = mm3(qh, kh, aqk);
+            aqk = mm_split(qh, kh, aqk);
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
-                aqb[s] = mm3(qh, bh[s], aqb[s]);
-                aak[s] = mm3(ah[s], kh, aak[s]);
+                aqb[s] = mm_split(qh, bh[s], aqb[s]);
+                aak[s] = mm_split(ah[s], kh, aak[s]);
 #pragma unroll
-                for (int r = 0; r < 2; ++r) aab[r][s] = mm3(ah[r], bh[s], aab[r][s]);
+                for (int r = 0; r < 2; ++r) aab[r][s] = mm_split(ah[r], bh[s], aab[r][s]);
             }
         }
     }
@@ -221,21 +221,21 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void 
                 Split<T> qh, kh, bh[2];
                 split(to_f32(rk[kt]) * ek, kh);
                 split(to_f32(rq[kt]) * eq * scale, qh);
-                aqk = mm3(qh, kh, aqk);
+                aqk = mm_split(qh, kh, aqk);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
                     split(to_f32(rb[s][kt]) * ek, bh[s]);
-                    aqb[s] = mm3(qh, bh[s], aqb[s]);
+                    aqb[s] = mm_split(qh, bh[s], aqb[s]);
                     __builtin_amdgcn_sched_barrier(0);
                 }
 #pragma unroll
                 for (int r = 0; r < 2; ++r) {
                     Split<T> ah;
                     split(to_f32(ra[r][kt]) * ea, ah);
-                    aak[r] = mm3(ah, kh, aak[r]);
-                    aab[r][0] = mm3(ah, bh[0], aab[r][0]);
-                    aab[r][1] = mm3(ah, bh[1], aab[r][1]);
+                    aak[r] = mm_split(ah, kh, aak[r]);
+                    aab[r][0] = mm_split(ah, bh[0], aab[r][0]);
+                    aab[r][1] = mm_split(ah, bh[1], aab[r][1]);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
@@ -332,10 +332,10 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void 
         Split<T> pa, pb;
         split(tllT, pa);
         split(ahl, pb);
-        const f32x4 xT = mm3(pa, pb, zero4());   // (A_HL T_LL)^T = T_LL^T A_HL^T
+        const f32x4 xT = mm_split(pa, pb, zero4());   // (A_HL T_LL)^T = T_LL^T A_HL^T
         split(thh, pa);
         split(xT, pb);
-        const f32x4 thl = mm3(pa, pb, zero4());  // T_HH (A_HL T_LL)
+        const f32x4 thl = mm_split(pa, pb, zero4());  // T_HH (A_HL T_LL)
         *reinterpret_cast<f32x4*>(&sT[(16 * rr + 8 + ii) * LDP + 16 * ss + j0]) = thl;
         __syncthreads();
     }

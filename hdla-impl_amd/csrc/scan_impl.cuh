@@ -922,7 +922,7 @@ __global__ __launch_bounds__(64 * (K / 16)) void scan_chain_kernel(ChunkArgs<T> 
             for (int ki = 0; ki < KT; ++ki) split(m[ki], q[ki]);
             request(i + 1, m, add);
 #pragma unroll
-            for (int ki = 0; ki < KT; ++ki) x = mm3(sx[i & 1][ki][l], q[ki], x);
+            for (int ki = 0; ki < KT; ++ki) x = mm_split(sx[i & 1][ki][l], q[ki], x);
         }
     }
 }
