@@ -87,8 +87,9 @@ int scan_segments(const hdla_dims* d, bool bwd) {
     // 2-byte inputs are bound by their traffic from a dozen lanes on, and the reverse records come on top: fewer there.
     if (bwd && !f32 && lanes > 8) return 1;
     const long long most = bwd && !f32 ? 64 : 128;
-    // chunks a segment: a step takes 2-4 us with fp32 products, about 0.7 with bf16
-    const long long least = f32 ? 4 : 7;
+    // chunks a segment: a step takes 2-4 us with fp32 products, about 0.7 with bf16, 0.55 in the forward pass's scan (K = V = 128, 16 lanes of
+    // 97 chunks: 57 us in 8 segments, 52 in 4, 55 whole)
+    const long long least = f32 ? 4 : bwd ? 7 : 13;
     int nseg = 1;
     while (nseg * 2 <= SCAN_MAX_SEGMENTS && lanes * nseg * 2 <= most && chunks / (nseg * 2) >= least) nseg *= 2;
     return nseg >= 4 ? nseg : 1;                          // two segments only make up for the second walk
@@ -195,8 +196,12 @@ int make_layout(const hdla_dims* d, int pass, WsLayout& L, int& nch) {
         L.SA_STRIDE = bf.SIZE;
         L.W = sa + bf.W; L.BGT = sa + bf.BGT; L.KGT = sa + bf.KGT; L.EGL = sa + bf.EGL;
         if (with_o) { L.QG = sa + bf.QG; L.AQB = sa + bf.AQB; L.AQK = sa + bf.AQK; }
-        L.UT = take(chw * 2 * V * 16 * es);
-        L.VTT = take(chw * V * 16 * es);
+        if (pass == HDLA_PASS_FWD && es == 2) {
+            L.TM = take(chw * 1536 * es);                         // the scan forms u itself (scan_out.cuh)
+        } else {
+            L.UT = take(chw * 2 * V * 16 * es);
+            L.VTT = take(chw * V * 16 * es);
+        }
     }
     if (bwd_parts) {
         const BlkB bb = blk_bwd(d->K, (int)es);
@@ -326,7 +331,7 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
         e = launch_scan_pair<T>(a, d->K, d->V, stream);
         if (e != hipSuccess) return (int)e;
     } else if (stages & HDLA_STAGE_SCAN_FWD) {
-        e = launch_scan_fwd<T>(a, d->K, d->V, fwd, stream);
+        e = fwd ? launch_scan_out<T>(a, d->K, d->V, pass == HDLA_PASS_FWD_KEEP, stream) : launch_scan_fwd<T>(a, d->K, d->V, stream);
         if (e != hipSuccess) return (int)e;
     }
     if (!fwd) {

@@ -20,11 +20,14 @@ hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int32_t*
 // K, V in {64, 128}; returns hipErrorInvalidValue for any other pair.
 // mode: 0 = for the forward pass, 1 = for the backward pass, 2 = forward pass whose workspace the backward pass will use
 template <typename T> hipError_t launch_prep(const ChunkArgs<T>& a, int K, int V, int mode, hipStream_t stream);
-template <typename T> hipError_t launch_scan_fwd(const ChunkArgs<T>& a, int K, int V, bool write_o, hipStream_t stream);
+// the two scans of the backward pass
+template <typename T> hipError_t launch_scan_fwd(const ChunkArgs<T>& a, int K, int V, hipStream_t stream);
+// the scan of the forward pass, with the output (kept: after launch_prep of mode 2, otherwise of mode 0)
+template <typename T> hipError_t launch_scan_out(const ChunkArgs<T>& a, int K, int V, bool kept, hipStream_t stream);
 template <typename T> hipError_t launch_scan_bwd(const ChunkArgs<T>& a, int K, int V, hipStream_t stream);
-// both scans of the backward pass (scan_fwd without the output, scan_bwd) in one launch
+// both in one launch
 template <typename T> hipError_t launch_scan_pair(const ChunkArgs<T>& a, int K, int V, hipStream_t stream);
-// several time segments per sequence: what the scans above start their segments from
+// several time segments per sequence: what the scans above start their segments from (both: of the backward pass; else of launch_scan_out)
 template <typename T> hipError_t launch_scan_segments(const ChunkArgs<T>& a, int K, int V, bool both, hipStream_t stream);
 template <typename T> hipError_t launch_chunk_grad(const ChunkArgs<T>& a, int K, int V, hipStream_t stream);
 template <typename T> hipError_t launch_recurrent(const RecurrentArgs<T>& a, int K, int V, hipStream_t stream);

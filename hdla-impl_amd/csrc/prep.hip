@@ -25,6 +25,8 @@ template <typename T, bool GKF32, int K, int V, int MODE, bool HD>
 __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void prep_kernel(ChunkArgs<T> p) {
     constexpr bool BWD = MODE == PREP_BWD;                // neither the output's score tiles nor qg are needed
     constexpr bool WB = MODE != PREP_FWD;                 // the backward pass's extras are
+    // the forward pass's scan of 2-byte elements forms u itself and takes the ranks of b^T side by side (scan_out.cuh): v is not read
+    constexpr bool SCAN_U = MODE == PREP_FWD && sizeof(T) == 2;
     constexpr int NWP = K / 64;                       // waves per (chunk, head)
     constexpr int KTW = 4, VT = V / 16, VTW = VT / NWP, KT2 = K / 32;
     constexpr int SAS = blk_fwd(K, sizeof(T), !BWD).SIZE / (int)sizeof(T);   // elements between (chunk, head) slots
@@ -81,6 +83,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void 
     // full round trip to HBM, behind everything else
     Frag<T> rv[VTW];
     Load lv[VTW / 2];
+    if (!SCAN_U)
 #pragma unroll
     for (int vp = 0; vp < VTW / 2; ++vp) lv[vp].load(vrow + 32 * vp, H * V, cp.len, l);
     // HDLA parameterisation: a_1 = -beta k, a_2 = beta k (beta s - f), b_1 = f k, b_2 = k with f = exp(gk) and
@@ -184,6 +187,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void 
             }
         }
     }
+    if (!SCAN_U)
 #pragma unroll
     for (int vp = 0; vp < VTW / 2; ++vp) {
         Frag<T> f[2];
@@ -367,9 +371,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void 
                                     transpose(to_frag<T>(to_f32(ra[1][kt]) * ege), ident)};
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
-                f32x4 w = mm(tm[s][0], agT[0], zero4());
-                w = mm(tm[s][1], agT[1], w);
-                fw[s][e] = to_frag<T>(w);
+                fw[s][e] = to_frag<T>(mm2(tm[s][0], tm[s][1], agT[0], agT[1], zero4()));
             }
             fqg[e] = to_frag<T>(to_f32(rq[kt]) * egi * scale);
             const Frag<T> kg = to_frag<T>(to_f32(rk[kt]) * edn);
@@ -385,7 +387,8 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void 
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             st_pair2(p.ws.W + chw * SAS + (s * KT2 + kp) * PAIR, fw[s][0], fw[s][1]);
-            st_pair2(p.ws.BGT + chw * SAS + (s * KT2 + kp) * PAIR, fbgT[s][0], fbgT[s][1]);
+            if (SCAN_U) st_pair2(p.ws.BGT + chw * SAS + (2 * kp + s) * PAIR, fbgT[0][s], fbgT[1][s]);   // (s: the tile of the pair)
+            else st_pair2(p.ws.BGT + chw * SAS + (s * KT2 + kp) * PAIR, fbgT[s][0], fbgT[s][1]);
         }
         st_pair2(p.ws.KGT + chw * SAS + kp * PAIR, fkgT[0], fkgT[1]);
         if (!BWD) st_pair2(p.ws.QG + chw * SAS + kp * PAIR, fqg[0], fqg[1]);
@@ -394,6 +397,15 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void 
 
     // ---- phase D: u = Tm (A_ak v), kept transposed (rows value, inner token) ---------------------------------
     const Frag<T> aakf[2] = {to_frag<T>(aak[0]), to_frag<T>(aak[1])};
+    if (SCAN_U) {
+        if (w == NWP - 1) {
+            T* tma = p.ws.TM + chw * (3 * PAIR);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) st_pair2(tma + s * PAIR, tm[s][0], tm[s][1]);
+            st_pair2(tma + 2 * PAIR, aakf[0], aakf[1]);
+        }
+        return;
+    }
 #pragma unroll
     for (int vl = 0; vl < VTW; ++vl) {
         const int vt = vt0 + vl;
@@ -403,9 +415,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void 
         Frag<T> fu[2];
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
-            f32x4 uT = mm(mT[0], tm[s][0], zero4());
-            uT = mm(mT[1], tm[s][1], uT);
-            fu[s] = to_frag<T>(uT);
+            fu[s] = to_frag<T>(mm2(mT[0], mT[1], tm[s][0], tm[s][1], zero4()));
         }
         st_pair2(p.ws.UT + (chw * VT + vt) * PAIR, fu[0], fu[1]);
     }

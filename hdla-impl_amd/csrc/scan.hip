@@ -13,8 +13,19 @@ static hipError_t launch_scan(const ChunkArgs<T>& a, int K, int V, ScanKind kind
 }
 
 template <typename T>
-hipError_t launch_scan_fwd(const ChunkArgs<T>& a, int K, int V, bool write_o, hipStream_t stream) {
-    return launch_scan<T>(a, K, V, write_o ? SCAN_FWD_O : SCAN_FWD, stream);
+hipError_t launch_scan_fwd(const ChunkArgs<T>& a, int K, int V, hipStream_t stream) {
+    return launch_scan<T>(a, K, V, SCAN_FWD, stream);
+}
+template <typename T>
+hipError_t launch_scan_out(const ChunkArgs<T>& a, int K, int V, bool kept, hipStream_t stream) {
+    if constexpr (sizeof(T) == 2) {
+        if (K == 64 && V == 64) return launch_scan_out_shape<64, 64>(a, kept, stream);
+        if (K == 128 && V == 128) return launch_scan_out_shape<128, 128>(a, kept, stream);
+        if (K == 64 && V == 128) return launch_scan_out_shape<64, 128>(a, kept, stream);
+        if (K == 128 && V == 64) return launch_scan_out_shape<128, 64>(a, kept, stream);
+        return hipErrorInvalidValue;
+    }
+    return launch_scan<T>(a, K, V, SCAN_FWD_O, stream);
 }
 template <typename T>
 hipError_t launch_scan_bwd(const ChunkArgs<T>& a, int K, int V, hipStream_t stream) {
@@ -26,6 +37,15 @@ hipError_t launch_scan_pair(const ChunkArgs<T>& a, int K, int V, hipStream_t str
 }
 template <typename T>
 hipError_t launch_scan_segments(const ChunkArgs<T>& a, int K, int V, bool both, hipStream_t stream) {
+    if constexpr (sizeof(T) == 2) {
+        if (!both) {
+            if (K == 64 && V == 64) return launch_scan_out_segments_shape<64, 64>(a, stream);
+            if (K == 128 && V == 128) return launch_scan_out_segments_shape<128, 128>(a, stream);
+            if (K == 64 && V == 128) return launch_scan_out_segments_shape<64, 128>(a, stream);
+            if (K == 128 && V == 64) return launch_scan_out_segments_shape<128, 64>(a, stream);
+            return hipErrorInvalidValue;
+        }
+    }
     if (K == 64 && V == 64) return launch_scan_segments_shape<T, 64, 64>(a, both, stream);
     if (K == 128 && V == 128) return launch_scan_segments_shape<T, 128, 128>(a, both, stream);
     if (K == 64 && V == 128) return launch_scan_segments_shape<T, 64, 128>(a, both, stream);
@@ -34,8 +54,10 @@ hipError_t launch_scan_segments(const ChunkArgs<T>& a, int K, int V, bool both, 
 }
 template hipError_t launch_scan_segments<bf16>(const ChunkArgs<bf16>&, int, int, bool, hipStream_t);
 template hipError_t launch_scan_segments<float>(const ChunkArgs<float>&, int, int, bool, hipStream_t);
-template hipError_t launch_scan_fwd<bf16>(const ChunkArgs<bf16>&, int, int, bool, hipStream_t);
-template hipError_t launch_scan_fwd<float>(const ChunkArgs<float>&, int, int, bool, hipStream_t);
+template hipError_t launch_scan_fwd<bf16>(const ChunkArgs<bf16>&, int, int, hipStream_t);
+template hipError_t launch_scan_fwd<float>(const ChunkArgs<float>&, int, int, hipStream_t);
+template hipError_t launch_scan_out<bf16>(const ChunkArgs<bf16>&, int, int, bool, hipStream_t);
+template hipError_t launch_scan_out<float>(const ChunkArgs<float>&, int, int, bool, hipStream_t);
 template hipError_t launch_scan_bwd<bf16>(const ChunkArgs<bf16>&, int, int, hipStream_t);
 template hipError_t launch_scan_bwd<float>(const ChunkArgs<float>&, int, int, hipStream_t);
 template hipError_t launch_scan_pair<bf16>(const ChunkArgs<bf16>&, int, int, hipStream_t);

@@ -933,7 +933,10 @@ static hipError_t launch_scan_nwc(const ChunkArgs<T>& a, ScanKind kind, hipStrea
     typedef ScanCfg<T, K, V, NWC> C;
     dim3 grid(a.H, C::SPLIT * (kind == SCAN_PAIR ? 2 : 1), a.st.N * a.seg.nseg), block(C::THREADS);
     switch (kind) {
-        case SCAN_FWD_O: hipLaunchKernelGGL((scan_fwd_kernel<T, K, V, NWC, true>), grid, block, 0, stream, a); break;
+        case SCAN_FWD_O:
+            if constexpr (sizeof(T) == 4) hipLaunchKernelGGL((scan_fwd_kernel<T, K, V, NWC, true>), grid, block, 0, stream, a);
+            else return hipErrorInvalidValue;             // scan_out.cuh
+            break;
         case SCAN_FWD: hipLaunchKernelGGL((scan_fwd_kernel<T, K, V, NWC, false>), grid, block, 0, stream, a); break;
         case SCAN_BWD: hipLaunchKernelGGL((scan_bwd_kernel<T, K, V, NWC>), grid, block, 0, stream, a); break;
         case SCAN_PAIR: hipLaunchKernelGGL((scan_pair_kernel<T, K, V, NWC>), grid, block, 0, stream, a); break;
@@ -965,7 +968,8 @@ hipError_t launch_scan_segments_shape(const ChunkArgs<T>& a, bool both, hipStrea
     typedef ScanCfg<T, K, V, NWC> C;
     dim3 grid(a.H, (V + K) / 16 / NWC * (both ? 2 : 1), a.st.N * (a.seg.nseg - 1)), block(C::THREADS);
     if (both) hipLaunchKernelGGL((scan_sum_kernel<T, K, V, NWC, true>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((scan_sum_kernel<T, K, V, NWC, false>), grid, block, 0, stream, a);
+    else if constexpr (sizeof(T) == 4) hipLaunchKernelGGL((scan_sum_kernel<T, K, V, NWC, false>), grid, block, 0, stream, a);
+    else return hipErrorInvalidValue;                     // scan_out.cuh
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((scan_chain_kernel<T, K, V>), dim3(a.H, V / 16 * (both ? 2 : 1), a.st.N), dim3(64 * (K / 16)), 0, stream, a);

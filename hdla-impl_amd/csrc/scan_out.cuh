@@ -1,0 +1,421 @@
+// The forward pass's scan for 2-byte elements: the state recurrence and the output o (HRDPLR/fwd_triton.py:808-1095), and the
+// records of time segments in the forward direction.  (4-byte elements and the scans of the backward pass: scan_impl.cuh.)  Computing
+// waves hold a 16-column block of the fp32 state for the whole sequence; those of NWC blocks and NM waves that move data make a workgroup.
+//
+// A sequence is a chain of steps, and up to some 32 heads in flight the time is the number of steps of the longest sequence times
+// the time of one, whatever the traffic (0.69 us at K = V = 128 in the form of scan_impl.cuh, with 4 heads as with 32).  What a step costs
+// is the instructions of a wave that has its SIMD to itself, some five cycles each, the latencies of the chain through the state (product ->
+// conversion -> product -> exchange -> product), and what waits at its barrier.  So:
+//  * products in twos (mm2), those with one product a sum first, one settle; b^T is stored with the two ranks of a channel tile side by
+//    side, as the state update takes it; the walk is compiled without branches;
+//  * at K = 128 two waves share a column block, a half of its channels each: half of the conversions, decays and products per wave, against
+//    one exchange of v_new's parts through LDS, at the barrier that a step has anyway;
+//  * the chunks' blocks go from global memory straight to LDS (global_load_lds), SLOTS chunks ahead, by waves that do nothing else;
+//  * u = Tm (A_ak v) is formed here by a wave of its own, a chunk ahead, from the chunk's (I - A_ab)^-1 and A_ak and the workgroup's columns
+//    of v (in the computing waves it cost 0.14 us a step: a chain of five dependent products).  The kernel that prepares the
+//    chunks does not read v and writes 3 KB instead of u and v^T, 12 KB of its 70 a chunk and head at K = V = 128: 236 -> 192 us for 16384
+//    tokens of 16 heads.  The products and roundings are the ones it had.
+// Measured, us, before -> after, 2048 tokens a sequence: K = V = 128, 16 heads 88 -> 73, 32 heads 92 -> 79, 64 heads 105 -> 101, 128 heads
+// 167 -> 146; K = 64, V = 128, 128 heads 116 -> 98; K = 128, V = 64, 32 heads 87 -> 72.  From 48 heads on a step waits for its loads: 82 us
+// of the 101 where they never leave the L2, 70 without them; touching the blocks' lines 12 chunks ahead made it 105.
+#pragma once
+#include "hdla_common.cuh"
+#include "hdla_launch.h"
+#include "scan_impl.cuh"
+
+namespace hdla {
+
+template <int K, int V, int NWC, bool SUM> struct OutCfg {
+    static constexpr int VT = V / 16, SPLIT = VT / NWC, KT = K / 16;
+    static constexpr BlkF B = blk_fwd(K, 2, true);
+    // 1-KiB pieces of a chunk's block that the scan needs (records: without q's and the scores')
+    static constexpr int NI = (SUM ? B.EGL + 1024 : B.SIZE) / 1024, SLOT = NI * 1024;
+    // computing waves of a column block, each holding KH channel tiles of the state
+    static constexpr int PARTS = K / 64, KH = KT / PARTS, NC = NWC * PARTS;
+    static constexpr int NL = 2, NM = NL + 2;             // waves that load, with the one that forms u and the one that copies the output out
+    static constexpr int CNT = (NI + NL - 1) / NL;        // loads of a wave per chunk (the last pieces may be fetched twice)
+    static constexpr int THREADS = 64 * (NC + NM);
+    static constexpr int OROW = 16 * NWC * 2 + 16, OB = SUM ? 0 : CH * OROW;   // output rows of a step, padded; two of them
+    static constexpr int UB = NWC * 1536;                 // u^T (a pair) and v^T (a tile) of the column blocks; two chunks' of them
+    // what the waves of a column block hand each other: two tiles each, and from the second one its part of the output; two steps' of it
+    static constexpr int XP = (SUM ? 4 : 5) * 1024, XB = PARTS > 1 ? NWC * XP : 0;
+    static constexpr int REST = 2 * (OB + UB + XB);
+    // as many slots as LDS holds, or as half of it does where that is enough (two workgroups on a compute unit)
+    static constexpr int ROOM = (4 * SLOT + REST <= 80 * 1024 ? 80 : 160) * 1024 - REST;
+    static constexpr int SLOTS = ROOM / SLOT < 8 ? ROOM / SLOT : 8;
+    static_assert(SLOTS >= 3 && (SLOTS - 1) * CNT < 63, "a chunk to read, the next one, and one on its way; the memory counter's range");
+    static constexpr int OUTBOX = SLOTS * SLOT, UBUF = OUTBOX + 2 * OB, XBUF = UBUF + 2 * UB, BYTES = XBUF + 2 * XB;
+};
+
+// all but the last n of this wave's memory accesses are complete
+template <int N> __device__ __forceinline__ void wait_loads() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0f70);
+    asm volatile("" ::: "memory");
+}
+
+// KEPT: on a workspace that the backward pass will read (PREP_KEEP): u and v^T are there, and b^T's pairs are of two channel tiles, as the
+// scans of the backward pass take them.  The same products in the same order: the same bits.
+template <int K, int V, int NWC, bool SUM, bool KEPT>
+__device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* smem, int n, int seg, int split) {
+    typedef OutCfg<K, V, NWC, SUM> C;
+    typedef bf16 T;
+    constexpr int KT = C::KT, KT2 = KT / 2, SLOTS = C::SLOTS, SLOT = C::SLOT, PARTS = C::PARTS, KH = C::KH, KH2 = KH / 2;
+    constexpr BlkF B = C::B;
+    const int h = blockIdx.x;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool trans = SUM && split >= C::SPLIT;          // columns of the segment's transition matrix
+    const int vt0 = (trans ? split - C::SPLIT : split) * NWC;
+    const int l = lane_id(), g = l >> 4, c = l & 15;
+    const int H = p.H;
+    int cs, ce, c0, c1;
+    seq_chunks(p.st, n, cs, ce);
+    seg_range(cs, ce, p.seg.nseg, seg, c0, c1);
+    int64_t bos, eos;
+    seq_bounds(p.st, n, bos, eos);
+    bos += (int64_t)(c0 - cs) * CH;                       // the segment's first token
+    const int64_t rec = ((int64_t)n * H + h) * p.seg.nseg + seg;
+    const int64_t chw0 = (int64_t)h * p.st.nch + c0;
+    const int nchunks = c1 - c0, last = nchunks - 1;
+
+    if (wv >= C::NC) {
+        // ---- waves that move data.  Barriers: one closing the prologue, one per step, one handing over the last output; the computing
+        // waves execute the same sequence.  From the barrier of step t on chunk t + 1 is in LDS and the slot of chunk t is free.
+        if (nchunks <= 0) return;
+        const int hw = wv - C::NC;
+        if (hw < C::NL) {
+            const char* const blk = reinterpret_cast<const char*>(p.ws.W) + chw0 * B.SIZE + l * 16;
+            int slot = 0;
+            auto load = [&](int t) __attribute__((always_inline)) {
+                // past the end: the last chunk again, never looked at
+                const char* const bt = blk + (int64_t)min(t, last) * B.SIZE;
+#pragma unroll
+                for (int j = 0; j < C::CNT; ++j) {
+                    const int i = min(hw + j * C::NL, C::NI - 1);
+                    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(bt + i * 1024),
+                                                     (__attribute__((address_space(3))) void*)(smem + slot * SLOT + i * 1024), 16, 0, 0);
+                }
+                slot = slot + 1 == SLOTS ? 0 : slot + 1;
+            };
+#pragma unroll
+            for (int d = 0; d < SLOTS; ++d) load(d);
+            wait_loads<(SLOTS - 1) * C::CNT>();           // chunk 0 is there
+            __builtin_amdgcn_s_barrier();
+            for (int t = 0; t < nchunks; ++t) {
+                wait_loads<(SLOTS - 2) * C::CNT>();       // chunk t + 1
+                __builtin_amdgcn_s_barrier();
+                load(t + SLOTS);                          // where chunk t was
+            }
+            if (!SUM) __builtin_amdgcn_s_barrier();
+            wait_loads<0>();                              // nothing may arrive in LDS that is no longer this workgroup's
+        } else if (hw == C::NL) {
+            // v^T and u = Tm (A_ak v) of the workgroup's column blocks, a chunk ahead, with the roundings of the kernel that prepared the
+            // chunk in u's place.  The operands come through registers, UD chunks ahead.
+            constexpr int UD = 3;
+            struct Own { i32x4 tm[3], ut[KEPT ? NWC : 1]; Frag<T> v[NWC]; };
+            const Frag<T> ident = ident_frag<T>();
+            auto request = [&](int t) __attribute__((always_inline)) {
+                t = min(t, last);
+                const int64_t tok0 = bos + (int64_t)t * CH;
+                const int len = (int)min((int64_t)CH, eos - tok0);
+                Own o;
+                if constexpr (KEPT) {
+#pragma unroll
+                    for (int j = 0; j < NWC; ++j) {
+                        o.ut[j] = *reinterpret_cast<const i32x4*>(p.ws.UT + ((chw0 + t) * (V / 16) + vt0 + j) * PAIR + 8 * l);
+                        o.v[j] = ld_tile(p.ws.VTT + ((chw0 + t) * (V / 16) + vt0 + j) * TILE);
+                    }
+                    return o;
+                }
+#pragma unroll
+                for (int i = 0; i < 3; ++i) o.tm[i] = *reinterpret_cast<const i32x4*>(p.ws.TM + (chw0 + t) * (3 * PAIR) + i * PAIR + 8 * l);
+#pragma unroll
+                for (int j = 0; j < NWC; ++j)
+                    o.v[j] = ld_frag(p.v + ((tok0 + min(c, len - 1)) * H + h) * V + 16 * (trans ? 0 : vt0 + j) + 4 * g);
+                return o;
+            };
+            auto pair = [](i32x4 x, Frag<T>& f0, Frag<T>& f1) __attribute__((always_inline)) {
+                const s16x8 y = __builtin_bit_cast(s16x8, x);
+                f0.v = __builtin_shufflevector(y, y, 0, 1, 2, 3);
+                f1.v = __builtin_shufflevector(y, y, 4, 5, 6, 7);
+            };
+            auto form = [&](int t, const Own& o) __attribute__((always_inline)) {
+                const int len = (int)min((int64_t)CH, eos - (bos + (int64_t)min(t, last) * CH));
+                T* const ub = reinterpret_cast<T*>(smem + C::UBUF + (t & 1) * C::UB);
+                if constexpr (KEPT) {
+#pragma unroll
+                    for (int j = 0; j < NWC; ++j) {
+                        *reinterpret_cast<i32x4*>(ub + j * (3 * TILE) + 8 * l) = o.ut[j];
+                        st_tile(ub + j * (3 * TILE) + PAIR, o.v[j]);
+                    }
+                    return;
+                }
+                Frag<T> tm[2][2], aak[2], vT[NWC], mT[NWC][2];
+                pair(o.tm[0], tm[0][0], tm[0][1]);
+                pair(o.tm[1], tm[1][0], tm[1][1]);
+                pair(o.tm[2], aak[0], aak[1]);
+#pragma unroll
+                for (int j = 0; j < NWC; ++j) vT[j] = transpose((c >= len || trans) ? zero_frag<T>() : o.v[j], ident);
+#pragma unroll
+                for (int j = 0; j < NWC; ++j)
+#pragma unroll
+                    for (int r = 0; r < 2; ++r) mT[j][r] = to_frag<T>(mm(vT[j], aak[r], zero4()));
+#pragma unroll
+                for (int j = 0; j < NWC; ++j) {
+                    st_tile(ub + j * (3 * TILE) + PAIR, vT[j]);
+                    st_pair2(ub + j * (3 * TILE), to_frag<T>(mm2(mT[j][0], mT[j][1], tm[0][0], tm[0][1], zero4())),
+                             to_frag<T>(mm2(mT[j][0], mT[j][1], tm[1][0], tm[1][1], zero4())));
+                }
+            };
+            Own own[UD];                                  // chunk t in own[t % UD]
+#pragma unroll
+            for (int d = 0; d < UD; ++d) own[d] = request(d);
+            form(0, own[0]);
+            own[0] = request(UD);
+            lds_barrier();
+            auto step = [&](int t, Own& o) __attribute__((always_inline)) {
+                form(t + 1, o);
+                o = request(t + 1 + UD);
+                lds_barrier();
+            };
+            // (unrolled: a register moved on while its load is on the way would wait for it)
+            int t0 = 0;
+#pragma unroll 1
+            for (; t0 + UD <= nchunks; t0 += UD) {
+#pragma unroll
+                for (int j = 0; j < UD; ++j) step(t0 + j, own[(j + 1) % UD]);
+            }
+#pragma unroll
+            for (int j = 0; j < UD - 1; ++j)
+                if (t0 + j < nchunks) step(t0 + j, own[(j + 1) % UD]);
+            if (!SUM) lds_barrier();
+        } else {
+            __builtin_amdgcn_s_barrier();
+            for (int t = 0; t <= nchunks; ++t) {
+                if (t == nchunks && SUM) break;
+                lds_barrier();
+                if (SUM || t == 0) continue;
+                // rows of o: 16-byte pieces, LPR lanes a row
+                constexpr int LPR = 2 * NWC, RPI = 64 / LPR;
+                const int64_t tok0 = bos + (int64_t)(t - 1) * CH;
+                const int len = (int)min((int64_t)CH, eos - tok0);
+                const char* ob = smem + C::OUTBOX + ((t - 1) & 1) * C::OB;
+#pragma unroll
+                for (int r0 = 0; r0 < CH; r0 += RPI) {
+                    const int r = r0 + l / LPR, e = (l % LPR) * 16;
+                    if (r < len) {
+                        const i32x4 x = *reinterpret_cast<const i32x4*>(ob + r * C::OROW + e);
+                        *reinterpret_cast<i32x4*>(reinterpret_cast<char*>(p.o + ((tok0 + r) * H + h) * V + 16 * vt0) + e) = x;
+                    }
+                }
+            }
+        }
+        return;
+    }
+
+    // ---- computing wave: channel tiles kt0 .. kt0 + KH of column block vt.  Lane (g,c) reg i of S[k] = S[16 (kt0 + k) + 4g + i][16vt + c]
+    const int col = wv / PARTS, part = wv % PARTS, kt0 = part * KH;
+    const int vt = vt0 + col;
+    f32x4 S[KH];
+    const int64_t soff = ((int64_t)n * H + h) * K * V + 16 * vt + c;
+#pragma unroll
+    for (int k = 0; k < KH; ++k) {
+        const int kt = kt0 + k;
+        S[k] = zero4();
+        if (seg > 0) {
+            if (!SUM) S[k] = *reinterpret_cast<const f32x4*>(p.seg.in + rec * (K * V) + (vt * KT + kt) * TILE + 4 * l);
+            else if (trans) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) S[k][i] = (16 * kt + 4 * g + i == 16 * vt + c) ? 1.f : 0.f;
+            }
+        } else if (p.h0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) S[k][i] = p.h0[soff + (int64_t)(16 * kt + 4 * g + i) * V];
+        }
+    }
+    // The walk, compiled for each part by itself: a wave alone on its SIMD pays some five cycles for every instruction, branches more
+    auto walk = [&](auto part_) __attribute__((always_inline)) {
+        constexpr int part = decltype(part_)::value, kt0 = part * KH;
+        constexpr bool first = part == 0, from_u = part == PARTS - 1;   // the wave with the output, and the one that starts v_new from u
+        // A chunk's operands, read as soon as the chunk before has been through with their registers: half a step and more before they are used
+        Frag<T> w[2][KH], qg[SUM ? 1 : KH], kgt[KH], bgt[2][KH], aqk, aqb[2], ut[2], vtt;
+        f32x4 egl[KH];
+        // (the lane's offset is all of an address that the wave holds in vector registers: the rest is the slot's and immediate)
+        const uint32_t lo = 16 * l, ge = 16 * g;
+        auto pair_at = [&](uint32_t so, int off, Frag<T>& f0, Frag<T>& f1) __attribute__((always_inline)) {
+            const s16x8 y = *reinterpret_cast<const s16x8*>(smem + so + lo + off);
+            f0.v = __builtin_shufflevector(y, y, 0, 1, 2, 3);
+            f1.v = __builtin_shufflevector(y, y, 4, 5, 6, 7);
+        };
+        auto read_u = [&](int t) __attribute__((always_inline)) {
+            const T* ub = reinterpret_cast<const T*>(smem + C::UBUF + (t & 1) * C::UB) + col * (3 * TILE);
+            if constexpr (from_u) ld_pair(ub, ut[0], ut[1]);
+            vtt = ld_tile(ub + PAIR);
+        };
+        auto read_first = [&](uint32_t so) __attribute__((always_inline)) {
+#pragma unroll
+            for (int kp = 0; kp < KH2; ++kp) {
+                pair_at(so, B.W + (part * KH2 + kp) * 1024, w[0][2 * kp], w[0][2 * kp + 1]);
+                pair_at(so, B.W + (KT2 + part * KH2 + kp) * 1024, w[1][2 * kp], w[1][2 * kp + 1]);
+            }
+#pragma unroll
+            for (int kp = 0; kp < KH2; ++kp) {
+                if constexpr (!SUM) pair_at(so, B.QG + (part * KH2 + kp) * 1024, qg[2 * kp], qg[2 * kp + 1]);
+                pair_at(so, B.KGT + (part * KH2 + kp) * 1024, kgt[2 * kp], kgt[2 * kp + 1]);
+            }
+#pragma unroll
+            for (int k = 0; k < KH; ++k) egl[k] = *reinterpret_cast<const f32x4*>(smem + so + ge + B.EGL + 64 * (kt0 + k));
+            if constexpr (!SUM && first) aqk.v = *reinterpret_cast<const s16x4*>(smem + so + lo / 2 + B.AQK);
+        };
+        auto read_rest = [&](uint32_t so) __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < KH; ++k) {
+                if constexpr (!KEPT) pair_at(so, B.BGT + (kt0 + k) * 1024, bgt[0][k], bgt[1][k]);
+                else if (k % 2 == 0) {
+                    pair_at(so, B.BGT + (kt0 + k) * 512, bgt[0][k], bgt[0][k + 1]);
+                    pair_at(so, B.BGT + (KT + kt0 + k) * 512, bgt[1][k], bgt[1][k + 1]);
+                }
+            }
+            if constexpr (!SUM && first) pair_at(so, B.AQB, aqb[0], aqb[1]);
+        };
+        // the column block's area: the parts of the first wave, then those of the second
+        char* const xcol = smem + C::XBUF + col * C::XP + l * 16;
+        lds_barrier();
+        read_u(0);
+        read_first(0);
+        read_rest(0);
+        uint32_t so = 0;
+#pragma unroll 1
+        for (int t = 0; t < nchunks; ++t) {
+            so = so == (SLOTS - 1) * SLOT ? 0 : so + SLOT;
+            char* const xt = xcol + (t & 1) * C::XB;
+            // ---- own channels' part of v_new^T (rows value, inner token) = u^T + S^T w^T, and of qg S
+            Frag<T> sb[KH];
+            f32x4 vn[2] = {zero4(), zero4()}, o = zero4();
+            if constexpr (from_u) { vn[0] = to_f32(ut[0]); vn[1] = to_f32(ut[1]); }
+#pragma unroll
+            for (int kp = 0; kp < KH2; ++kp) {
+                sb[2 * kp] = to_frag<T>(S[2 * kp]);
+                sb[2 * kp + 1] = to_frag<T>(S[2 * kp + 1]);
+                vn[0] = mm2(sb[2 * kp], sb[2 * kp + 1], w[0][2 * kp], w[0][2 * kp + 1], vn[0]);
+                vn[1] = mm2(sb[2 * kp], sb[2 * kp + 1], w[1][2 * kp], w[1][2 * kp + 1], vn[1]);
+            }
+            if constexpr (!SUM) {
+#pragma unroll
+                for (int kp = 0; kp < KH2; ++kp) o = mm2(qg[2 * kp], qg[2 * kp + 1], sb[2 * kp], sb[2 * kp + 1], o);
+            }
+            // ---- what is one product a sum: the chunk's own part of the state, A_qk v
+            f32x4 x[KH + 1];
+#pragma unroll
+            for (int k = 0; k < KH; ++k) x[k] = mm(vtt, kgt[k], S[k] * egl[k]);
+            x[KH] = zero4();
+            if constexpr (!SUM && first) x[KH] = mm(aqk, vtt, x[KH]);
+            if constexpr (PARTS > 1) {
+                *reinterpret_cast<f32x4*>(xt + part * 2048) = vn[0];
+                *reinterpret_cast<f32x4*>(xt + part * 2048 + 1024) = vn[1];
+                if constexpr (!SUM && !first) *reinterpret_cast<f32x4*>(xt + 4096) = o;
+            }
+            // the parts are there; so are chunk t + 1 and its u, and chunk t has been read by all
+            lds_barrier();
+            f32x4 ov[2], oo;
+            if constexpr (PARTS > 1) {
+                ov[0] = *reinterpret_cast<const f32x4*>(xt + (1 - part) * 2048);
+                ov[1] = *reinterpret_cast<const f32x4*>(xt + (1 - part) * 2048 + 1024);
+                if constexpr (!SUM && first) oo = *reinterpret_cast<const f32x4*>(xt + 4096);
+            }
+            __builtin_amdgcn_sched_barrier(0);            // (before the reads of the next chunk: they are what is waited for)
+            read_u(t + 1);
+            read_first(so);
+            __builtin_amdgcn_sched_barrier(0);
+            settle<T>(x);
+            if constexpr (PARTS > 1) {
+                vn[0] += ov[0];
+                vn[1] += ov[1];
+            }
+            const Frag<T> vnb[2] = {to_frag<T>(vn[0]), to_frag<T>(vn[1])};
+            // ---- S <- exp(g_last) S + kg^T v + sum_s bg_s^T v_new_s
+#pragma unroll
+            for (int k = 0; k < KH; ++k) S[k] = mm2(vnb[0], vnb[1], bgt[0][k], bgt[1][k], x[k]);
+            if constexpr (!SUM && first) {
+                // o (rows token, inner value) = A_qk v + qg S + sum_s A_qb^s v_new_s
+                if constexpr (PARTS > 1) o += oo;
+                o = mm2(aqb[0], aqb[1], vnb[0], vnb[1], o + x[KH]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            read_rest(so);
+            if constexpr (!SUM && first) st_frag(reinterpret_cast<T*>(smem + C::OUTBOX + (t & 1) * C::OB + c * C::OROW) + 16 * col + 4 * g, to_frag<T>(o));
+        }
+        if (!SUM) lds_barrier();                          // hands over the last output
+    };
+    if (nchunks > 0) {
+        if (PARTS == 1 || part == 0) walk(std::integral_constant<int, 0>());
+        else walk(std::integral_constant<int, PARTS - 1>());
+    }
+    if (SUM) {
+        // the record: column block vt of the state, or (trans) of the transition matrix, whose tile (kt, vt) is kept with rows k, inner k'
+        const Frag<float> identf = ident_frag<float>();
+#pragma unroll
+        for (int k = 0; k < KH; ++k) {
+            const int kt = kt0 + k;
+            if (trans) {
+                Frag<float> f;
+                f.v = S[k];
+                f = transpose(f, identf);                 // exact: fp32 products with ones and zeros
+                *reinterpret_cast<f32x4*>(p.seg.tr + rec * (K * K) + (kt * KT + vt) * TILE + 4 * l) = f.v;
+            } else {
+                *reinterpret_cast<f32x4*>(p.seg.loc + rec * (K * V) + (vt * KT + kt) * TILE + 4 * l) = S[k];
+            }
+        }
+    } else if (p.ht && seg == p.seg.nseg - 1) {
+#pragma unroll
+        for (int k = 0; k < KH; ++k)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) p.ht[soff + (int64_t)(16 * (kt0 + k) + 4 * g + i) * V] = S[k][i];
+    }
+}
+
+// grid = (H, SPLIT, N * segments), as the other scans' (scan_impl.cuh)
+template <int K, int V, int NWC, bool KEPT>
+__global__ __launch_bounds__((OutCfg<K, V, NWC, false>::THREADS)) void scan_out_kernel(ChunkArgs<bf16> p) {
+    __shared__ __attribute__((aligned(16))) char smem[OutCfg<K, V, NWC, false>::BYTES];
+    const int z = blockIdx.z / p.seg.nseg, seg = blockIdx.z % p.seg.nseg;
+    scan_out_body<K, V, NWC, false, KEPT>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
+}
+// the segments' records in the forward direction: grid = (H, (V + K) / 16 / NWC, N * (segments - 1))
+template <int K, int V, int NWC>
+__global__ __launch_bounds__((OutCfg<K, V, NWC, true>::THREADS)) void scan_out_sum_kernel(ChunkArgs<bf16> p) {
+    __shared__ __attribute__((aligned(16))) char smem[OutCfg<K, V, NWC, true>::BYTES];
+    const int z = blockIdx.z / (p.seg.nseg - 1), seg = blockIdx.z % (p.seg.nseg - 1);
+    if (seg == 0 && (int)blockIdx.y >= OutCfg<K, V, NWC, true>::SPLIT) return;   // starts from h0: nobody asks for its transition
+    scan_out_body<K, V, NWC, true, false>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
+}
+
+template <int K, int V, int NWC> static hipError_t launch_scan_out_nwc(const ChunkArgs<bf16>& a, bool kept, hipStream_t stream) {
+    typedef OutCfg<K, V, NWC, false> C;
+    const dim3 grid(a.H, C::SPLIT, a.st.N * a.seg.nseg), block(C::THREADS);
+    if (kept) hipLaunchKernelGGL((scan_out_kernel<K, V, NWC, true>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((scan_out_kernel<K, V, NWC, false>), grid, block, 0, stream, a);
+    return hipGetLastError();
+}
+// Column blocks a workgroup: as few as give each workgroup a compute unit of its own (every workgroup fetches the chunks' blocks for
+// itself).  K = V = 128, 128 heads, 2 and 4 blocks: 193 and 146 us; 64 heads: 101 and 114.
+template <int K, int V> hipError_t launch_scan_out_shape(const ChunkArgs<bf16>& a, bool kept, hipStream_t stream) {
+    constexpr int VT = V / 16;
+    const int lanes = a.H * a.st.N * a.seg.nseg;
+    if constexpr (VT == 4)
+        if (lanes * 4 <= SCAN_TARGET_WORKGROUPS) return launch_scan_out_nwc<K, V, 1>(a, kept, stream);
+    if (lanes * (VT / 2) <= SCAN_TARGET_WORKGROUPS) return launch_scan_out_nwc<K, V, 2>(a, kept, stream);
+    return launch_scan_out_nwc<K, V, 4>(a, kept, stream);
+}
+// the segments' records, chained into what enters the segments
+template <int K, int V> hipError_t launch_scan_out_segments_shape(const ChunkArgs<bf16>& a, hipStream_t stream) {
+    constexpr int NWC = 4;
+    typedef OutCfg<K, V, NWC, true> C;
+    hipLaunchKernelGGL((scan_out_sum_kernel<K, V, NWC>), dim3(a.H, (V + K) / 16 / NWC, a.st.N * (a.seg.nseg - 1)), dim3(C::THREADS), 0, stream, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((scan_chain_kernel<bf16, K, V>), dim3(a.H, V / 16, a.st.N), dim3(64 * (K / 16)), 0, stream, a);
+    return hipGetLastError();
+}
+
+}  // namespace hdla

@@ -92,7 +92,9 @@ typedef struct hdla_dims {
  * is the offset for slot 0 and consecutive slots are SA_STRIDE bytes apart; likewise QGT, AQBT
  * with SB_STRIDE.  On the fused route the scans' operands never reach the workspace: only TM, HC, DHC, DVN, STRONG
  * (and W, UT where chunk_grad reads them instead of rebuilding them: the hdla_param_ forms, fp32 decays beside bf16
- * inputs) are written, in the backward pass. */
+ * inputs) are written, in the backward pass.  In a forward pass on bf16 inputs (HDLA_PASS_FWD, classic route) the scan forms u
+ * itself: there is no UT and no VTT, TM holds three tile pairs a slot, the blocks of (I - A_ab)^-1 (not transposed: rows i, inner j) and
+ * the two ranks of A_ak, and the tile pairs of BGT are the two ranks of a channel tile. */
 typedef struct hdla_ws_layout {
     int64_t nch;               /* chunk slots per head */
     int64_t W, UT, KGT, BGT, VTT, EGL, QG, AQK, AQB, AQBT, QGT, TM, HC, DHC, DVN;
@@ -130,7 +132,7 @@ int hdla_chunk_fwd(const hdla_dims* dims, const void* q, const void* k, const vo
  * workspace: the kernels use an array of HDLA_STATIC_WORKSPACE_BYTES bytes that is part of the library's device
  * code (every GPU the library runs on holds it until the process ends); the call allocates and frees nothing.
  * A shape whose hdla_workspace_bytes(dims, 0) exceeds that size is refused with HDLA_ERR_STATIC_LIMIT (K = V = 64,
- * bf16: up to 3276 (16-token chunk, head) pairs, e.g. one sequence of 3276 tokens with 16 heads).  All calls on
+ * bf16, classic route: up to 3855 (16-token chunk, head) pairs, e.g. one sequence of 3840 tokens with 16 heads).  All calls on
  * one GPU share the array: calls that may overlap on one GPU (different streams, different threads) race; calls
  * on one stream are safe.  The array's device address is looked up on the first call on each device; make that
  * call outside graph capture. */
