@@ -44,9 +44,25 @@ constexpr int FUSED_TARGET_WORKGROUPS = 256; // one workgroup per compute unit
 
 // the shapes the fused kernels are built for
 bool fused_shape(const hdla_dims* d) { return d->in_dtype == HDLA_BF16 && d->K == 64 && d->V == 64; }
-// whether the plain entry points take the fused route for these dimensions; HDLA_ROUTE_FUSED on another shape is an error
-int pick_route(const hdla_dims* d, bool& fused) {
-    fused = d->route != HDLA_ROUTE_CLASSIC && fused_shape(d);
+// Few short sequences, where the choice is the library's (neither route nor segments asked for): the classic kernels.  A fused workgroup
+// takes some 8 us for each round of four chunks of its segment, which is never shorter than eight chunks; the classic kernels prepare all
+// chunks at once and then walk them at 0.35 us each.  Below six chunks there is little to walk either way, from 32 on there are four fused
+// segments, and beyond 64 lanes the classic kernels' traffic counts.  Measured, us on the device, forward pass / training step, fused ->
+// classic: 2 lanes of 16 chunks 27/55 -> 20/46, 8 of 12 28/60 -> 19/44, 16 of 24 34/75 -> 25/65, 64 of 8 22/60 -> 22/56, 64 of 24 37/97 -> 34/95; but
+// 8 of 4 22/35 and 22/37, 32 of 32 31/82 and 33/85, 64 of 48 47/140 and 49/160, 128 of 8 23/69 and 30/76.
+constexpr int SHORT_MIN_CHUNKS = 6, SHORT_MAX_CHUNKS = 4 * FUSED_MIN_SEGMENT_CHUNKS - 1, SHORT_MAX_LANES = 64;
+bool few_short_sequences(const hdla_dims* d, int least = SHORT_MIN_CHUNKS) {
+    if (!fused_shape(d) || d->route != HDLA_ROUTE_AUTO || d->segments > 0) return false;
+    const long long chunks = ((d->T + CHUNK - 1) / CHUNK) / (d->cu_seqlens ? std::max(d->N, 1) : 1);
+    return (long long)d->N * d->H <= SHORT_MAX_LANES && chunks >= least && chunks <= SHORT_MAX_CHUNKS;
+}
+// (The forward pass alone costs the same on both routes below six chunks; it takes the classic kernels there too, so that a prompt cut into
+// pieces comes out in the bits of the whole one.)
+int short_least(int pass) { return pass == HDLA_PASS_FWD ? 1 : SHORT_MIN_CHUNKS; }
+// whether the plain entry points take the fused route for these dimensions; HDLA_ROUTE_FUSED on another shape is an error.
+// with_boundary: a boundary (or record) buffer is given: then it is the fused route's.
+int pick_route(const hdla_dims* d, int pass, bool with_boundary, bool& fused) {
+    fused = d->route != HDLA_ROUTE_CLASSIC && fused_shape(d) && (with_boundary || !few_short_sequences(d, short_least(pass)));
     if (d->route == HDLA_ROUTE_FUSED && !fused) return HDLA_ERR_ROUTE;
     return HDLA_OK;
 }
@@ -505,25 +521,28 @@ size_t hdla_workspace_bytes(const hdla_dims* dims, int pass) {
     if (pass < HDLA_PASS_FWD || pass > HDLA_PASS_BWD_KEPT) return 0;
     if (check_dims(dims)) return 0;
     bool fused;
-    if (pick_route(dims, fused)) return 0;
+    if (pick_route(dims, pass, true, fused)) return 0;
+    size_t need = 0;
     if (fused && (pass == HDLA_PASS_FWD || pass == HDLA_PASS_BWD)) {
         FusedLayout F;
-        return make_fused_layout(dims, pass, F) ? 0 : F.total;
+        if (make_fused_layout(dims, pass, F)) return 0;
+        need = F.total;
+        if (!few_short_sequences(dims, short_least(pass))) return need;   // (of these the call decides: enough for either)
     }
     if (make_layout(dims, pass, L, nch)) return 0;
-    return L.total;
+    return std::max(need, L.total);
 }
 
 size_t hdla_boundary_bytes(const hdla_dims* dims) {
     bool fused;
-    if (check_dims(dims) || pick_route(dims, fused) || !fused) return 0;
+    if (check_dims(dims) || pick_route(dims, HDLA_PASS_FWD, true, fused) || !fused) return 0;
     return fused_boundary_bytes(dims);
 }
 
 size_t hdla_record_bytes(const hdla_dims* dims) {
     bool fused;
     FusedLayout L;
-    if (check_dims(dims) || pick_route(dims, fused) || !fused || make_fused_layout(dims, HDLA_PASS_BWD, L)) return 0;
+    if (check_dims(dims) || pick_route(dims, HDLA_PASS_BWD, false, fused) || !fused || make_fused_layout(dims, HDLA_PASS_BWD, L)) return 0;
     return fused_record(dims, L).total;
 }
 
@@ -541,7 +560,7 @@ int hdla_workspace_layout(const hdla_dims* dims, int pass, hdla_ws_layout* out) 
     int rc = check_dims(dims);
     if (rc) return rc;
     bool fused;
-    rc = pick_route(dims, fused);
+    rc = pick_route(dims, pass, false, fused);
     if (rc) return rc;
     if (fused && (pass == HDLA_PASS_FWD || pass == HDLA_PASS_BWD)) {
         FusedLayout F;
@@ -582,7 +601,7 @@ static int chunk_fwd_any(const hdla_dims* dims, const void* q, const void* k, co
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (beta) { a = nullptr; b = nullptr; }
     bool fused;
-    rc = pick_route(dims, fused);
+    rc = pick_route(dims, HDLA_PASS_FWD, boundary != nullptr, fused);
     if (rc) return rc;
     if (fused)
         return run_fused(dims, true, q, k, v, a, b, beta, gk, h0, o, ht, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
@@ -608,7 +627,7 @@ static int chunk_bwd_any(const hdla_dims* dims, const void* q, const void* k, co
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (beta) { a = nullptr; b = nullptr; da = nullptr; db = nullptr; }
     bool fused;
-    rc = pick_route(dims, fused);
+    rc = pick_route(dims, HDLA_PASS_BWD, boundary != nullptr, fused);
     if (rc) return rc;
     if (fused)
         return run_fused(dims, false, q, k, v, a, b, beta, gk, h0, nullptr, nullptr, d_o, dht, dq, dk, dv, da, db, dbeta, dgk,
@@ -729,7 +748,7 @@ int hdla_chunk_stages(const hdla_dims* dims, int pass, int stages, const void* q
     if (pass == 0 ? !o : (!d_o || !dq || !dk || !dv || !da || !db || !dgk)) return HDLA_ERR_NULL;
     hipStream_t s = static_cast<hipStream_t>(stream);
     bool fused;
-    const int rr = pick_route(dims, fused);
+    const int rr = pick_route(dims, pass, false, fused);
     if (rr) return rr;
     if (fused)
         return run_fused(dims, pass == 0, q, k, v, a, b, nullptr, gk, h0, o, ht, d_o, dht, dq, dk, dv, da, db, nullptr, dgk, dh0,
