@@ -7,7 +7,7 @@
 // layer_down: their input gradients, dx0 [M, D] = dY [M, d] W [d, D], with dY = dlog_f sigmoid(-f) formed on the way in for
 // the first (before: 12 + 12 us and a pass of its own for dY, 10.7 us).
 // rows_gemm: y [M, N] = x [M, K] W [N, K]^T for at most 64 rows, i.e. the large projections of a decode step: a stream of W,
-// all of the chip's workgroups on it, where the BLAS call costs 20 us of host time and 10 us (16 x 6416 x 2048).
+// all of the chip's workgroups on it, where the BLAS call costs 20 us of host time and 6 to 13 us (16 x 6416 x 2048; here 5 to 9).
 //
 // bf16 in and out, fp32 accumulation.  Operands are read 16 bytes a lane; the eight elements are two fragments whose inner
 // index is permuted the same way on both sides (elements 8j..8j+3 and 8j+4..8j+7, see ld_two_tiles in skinny.hip), which a
@@ -193,67 +193,89 @@ __global__ __launch_bounds__(256) void layer_down_kernel(DownArgs p) {
     }
 }
 
-// y [M, N] = x [M, K] W [N, K]^T, M <= 16 MT.  A workgroup per 16 rows of W; its four waves take every fourth 32-column
-// block of K and add up through LDS.  Bound by the stream of W, of which a wave keeps UNR blocks in flight; from some 16
-// million weights on by the x that every workgroup reads again (from L2), which is where the BLAS library's larger tiles
-// win (1 x 12576 x 4096: 35 us here, 26 there).
-template <int MT>
-__global__ __launch_bounds__(256) void rows_gemm_kernel(const bf16* __restrict__ x, long long ldx, const bf16* __restrict__ w, long long ldw,
-                                                        bf16* __restrict__ y, long long ldy, int M, int N, int K) {
-    constexpr int UNR = MT <= 2 ? 8 : 4;
-    __shared__ f32x4 red[3][MT][64];
-    const int wv = threadIdx.x >> 6, l = lane_id(), g = l >> 4, c = l & 15;
-    const int n0 = blockIdx.x * 16;
-    const bf16* wr = w + (long long)min(n0 + c, N - 1) * ldw + 8 * g;
-    const bf16* xr[MT];
+// y [M, N] = x [M, K] W [N, K]^T, M <= 16 MT.  A workgroup per 16 RT rows of W; its eight waves take an eighth of K each and
+// add up through LDS.
+//
+// What bounds it is the path from memory into the compute unit, and on that the order of the lanes: a fragment's lane order
+// (16 rows, 16 bytes of each) puts the four lanes that the address unit takes at a time into four cache lines, at a quarter of the
+// rate.  So a request is 64 bytes of 16 rows with the four lanes of a row side by side, and the pieces change lanes through
+// 1 KiB of LDS that only their wave uses; what a wave asks for is one stretch of a row (a whole cache line in two requests),
+// UNR blocks of it at a time.  Measured (us; every fourth block, lanes in fragment order -> this; weights in the last-level
+// cache, then from HBM): 16 x 6416 x 2048 9.1 -> 5.0, 12.0 -> 9.0; 16 x 2048 x 2048 5.2 -> 3.2, 6.9 -> 5.3; 64 x 2048 x 2048
+// 11.0 -> 5.6, 13.8 -> 8.3; 16 x 512 x 512, one launch's time, 2.65 -> 2.3.  (The 26 MB of the first at copy rate: 5.4.)
+// UNR: a wave's whole share of K up to 2048 (16 rows) in one or two goes; twice as many is no faster (16 x 6416 x 2048 5.0,
+// 64 x 6416 x 2048 7.6 -> 8.7) and asks twice for K = 512 what is there once (1 -> 2 blocks a wave too many, 2.5 -> 3.0 for 32 rows).
+constexpr int RW = 8;                                     // waves
+// a wave's LDS writes before its reads of what its other lanes wrote, and the other way round: the hardware keeps the order
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+template <int MT, int RT, int UNR>
+__global__ __launch_bounds__(64 * RW) void rows_gemm_kernel(const bf16* __restrict__ x, long long ldx, const bf16* __restrict__ w, long long ldw,
+                                                            bf16* __restrict__ y, long long ldy, int M, int N, int K) {
+    constexpr int TURN = RT + MT, SUMS = RT * MT;         // KiB a wave: to change lanes in, of sums
+    static_assert(SUMS <= RW, "a wave per tile of the result");
+    __shared__ __attribute__((aligned(16))) char sm[RW * (TURN > SUMS ? TURN : SUMS) * 1024];
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane_id(), g = l >> 4, c = l & 15;
+    const int n0 = blockIdx.x * (16 * RT), row = l >> 2, piece = l & 3;
+    // row r's pieces p lie at 4 r + (p ^ r / 4): 16 lanes of either order meet each bank once
+    char* const put = sm + wv * (TURN * 1024) + ((4 * row + (piece ^ (row >> 2))) << 4);
+    const char* const get = sm + wv * (TURN * 1024) + ((4 * c + (g ^ (c >> 2))) << 4);
+    const bf16* from[TURN];                               // rows past the end: read again, not stored
 #pragma unroll
-    for (int m = 0; m < MT; ++m) xr[m] = x + (long long)min(16 * m + c, M - 1) * ldx + 8 * g;
-    f32x4 acc[MT];
+    for (int i = 0; i < TURN; ++i)
+        from[i] = (i < RT ? w + (long long)min(n0 + 16 * i + row, N - 1) * ldw : x + (long long)min(16 * (i - RT) + row, M - 1) * ldx) + 8 * piece;
+    const int nb = K / 32, per = (nb + RW - 1) / RW, end = min(nb, (wv + 1) * per);
+    f32x4 acc[RT][MT];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) acc[m] = zero4();
-    int k = 32 * wv;
-    for (; k + 128 * (UNR - 1) < K; k += 128 * UNR) {
-        TwoTiles a[UNR], b[UNR][MT];
+    for (int r = 0; r < RT; ++r)
 #pragma unroll
-        for (int u = 0; u < UNR; ++u) {
-            a[u] = ld16(wr + k + 128 * u);
-#pragma unroll
-            for (int m = 0; m < MT; ++m) b[u][m] = ld16(xr[m] + k + 128 * u);
-        }
-        __builtin_amdgcn_sched_barrier(0);                // all of them requested before the first is waited for
+        for (int m = 0; m < MT; ++m) acc[r][m] = zero4();
+    // (no branch around a block's products: its requests would be moved behind it)
+    auto blocks = [&](int b0, bool whole) __attribute__((always_inline)) {
+        s16x8 in[UNR][TURN];
 #pragma unroll
         for (int u = 0; u < UNR; ++u)
 #pragma unroll
-            for (int m = 0; m < MT; ++m) {
-                acc[m] = mm(b[u][m].a, a[u].a, acc[m]);
-                acc[m] = mm(b[u][m].b, a[u].b, acc[m]);
-            }
-    }
-    for (; k < K; k += 128) {
-        const TwoTiles a = ld16(wr + k);
+            for (int i = 0; i < TURN; ++i) in[u][i] = *reinterpret_cast<const s16x8*>(from[i] + 32 * (whole ? b0 + u : min(b0 + u, end - 1)));
+        __builtin_amdgcn_sched_barrier(0);                // all of them requested before the first is waited for
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            const TwoTiles b = ld16(xr[m] + k);
-            acc[m] = mm(b.a, a.a, acc[m]);
-            acc[m] = mm(b.b, a.b, acc[m]);
+        for (int u = 0; u < UNR; ++u) {
+            const s16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+            wave_lds_fence();                             // (the reads of the block before)
+#pragma unroll
+            for (int i = 0; i < TURN; ++i) *reinterpret_cast<s16x8*>(put + 1024 * i) = whole || b0 + u < end ? in[u][i] : zero;
+            wave_lds_fence();
+            TwoTiles t[TURN];
+#pragma unroll
+            for (int i = 0; i < TURN; ++i) t[i] = ld16(reinterpret_cast<const bf16*>(get + 1024 * i));
+#pragma unroll
+            for (int r = 0; r < RT; ++r)
+#pragma unroll
+                for (int m = 0; m < MT; ++m) acc[r][m] = mm2(t[RT + m].a, t[RT + m].b, t[r].a, t[r].b, acc[r][m]);
         }
-    }
-    if (wv) {
+    };
+    int b0 = wv * per;
+    for (; b0 + UNR <= end; b0 += UNR) blocks(b0, true);
+    if (b0 < end) blocks(b0, false);
+    __syncthreads();                                      // the sums lie where the others changed lanes
+    f32x4* const red = reinterpret_cast<f32x4*>(sm);
 #pragma unroll
-        for (int m = 0; m < MT; ++m) red[wv - 1][m][l] = acc[m];
-    }
+    for (int i = 0; i < SUMS; ++i) red[(wv * SUMS + i) * 64 + l] = acc[i / MT][i % MT];
     __syncthreads();
-    if (wv) return;
+    if (wv >= SUMS) return;
+    f32x4 s = red[wv * 64 + l];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        const f32x4 s = acc[m] + red[0][m][l] + red[1][m][l] + red[2][m][l];
-        if (16 * m + c >= M) continue;
-        bf16* o = y + (long long)(16 * m + c) * ldy + n0 + 4 * g;
-        if (n0 + 4 * g + 3 < N) st_frag(o, to_frag<bf16>(s));
-        else {
+    for (int i = 1; i < RW; ++i) s += red[(i * SUMS + wv) * 64 + l];
+    const int m = 16 * (wv % MT) + c, n = n0 + 16 * (wv / MT) + 4 * g;
+    if (m >= M) return;
+    bf16* o = y + (long long)m * ldy + n;
+    if (n + 3 < N) st_frag(o, to_frag<bf16>(s));
+    else {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) if (n0 + 4 * g + i < N) st_elem(o + i, s[i]);
-        }
+        for (int i = 0; i < 4; ++i) if (n + i < N) st_elem(o + i, s[i]);
     }
 }
 
@@ -390,9 +412,20 @@ extern "C" int hdla_rows_gemm(int32_t M, int32_t N, int32_t K, const void* x, in
     const hipStream_t s = static_cast<hipStream_t>(stream);
     const bf16 *xp = static_cast<const bf16*>(x), *wp = static_cast<const bf16*>(w);
     bf16* yp = static_cast<bf16*>(y);
-    const dim3 grid((N + 15) / 16), block(256);
-    if (M <= 16) hipLaunchKernelGGL(rows_gemm_kernel<1>, grid, block, 0, s, xp, (long long)ldx, wp, (long long)ldw, yp, (long long)ldy, M, N, K);
-    else if (M <= 32) hipLaunchKernelGGL(rows_gemm_kernel<2>, grid, block, 0, s, xp, (long long)ldx, wp, (long long)ldw, yp, (long long)ldy, M, N, K);
-    else hipLaunchKernelGGL(rows_gemm_kernel<4>, grid, block, 0, s, xp, (long long)ldx, wp, (long long)ldw, yp, (long long)ldy, M, N, K);
+    // Two tiles of W's rows a workgroup where the x that every workgroup reads is as much as that (more than 16 rows of it), once
+    // one tile each is more than a workgroup a compute unit.  One tile / two, weights in the last-level cache, us: K = 2048, 64 rows,
+    // 4096 columns 6.5 / 7.3, 5120 9.2 / 7.4, 6416 9.4 / 7.5; 32 rows 4.4 / 5.9, 6.6 / 6.1, 6.5 / 6.25.
+    const bool two = M > 16 && N > 16 * 256;
+    const dim3 grid((N + (two ? 31 : 15)) / (two ? 32 : 16)), block(64 * RW);
+#define HDLA_ROWS(MT, RT, UNR) \
+    hipLaunchKernelGGL((rows_gemm_kernel<MT, RT, UNR>), grid, block, 0, s, xp, (long long)ldx, wp, (long long)ldw, yp, (long long)ldy, M, N, K)
+    if (M <= 16 && K <= 64 * RW) HDLA_ROWS(1, 1, 2);
+    else if (M <= 16) HDLA_ROWS(1, 1, 4);
+    else if (M <= 32 && !two && K <= 64 * RW) HDLA_ROWS(2, 1, 2);
+    else if (M <= 32 && !two) HDLA_ROWS(2, 1, 4);
+    else if (M <= 32) HDLA_ROWS(2, 2, 4);
+    else if (!two) HDLA_ROWS(4, 1, 2);
+    else HDLA_ROWS(4, 2, 2);
+#undef HDLA_ROWS
     return (int)hipGetLastError();
 }

@@ -561,13 +561,14 @@ hdla_up_dims up_dims(const LayerCols& L, int64_t rows) {
     u.rows = rows; u.d = (int32_t)L.d; u.D = (int32_t)L.D; u.ld = L.ld; u.col_f = (int32_t)L.f0; u.col_g = (int32_t)L.g0;
     return u;
 }
-// x w^T.  For the few rows of a decode step by hdla_rows_gemm, which is a launch where the BLAS call is 19 us of host time
-// (measured, us, here / there: 16 x 1024 x 1024 4.5/19, 16 x 6416 x 2048 12/19, 16 x 4096 x 4096 12/19, 64 x 2048 x 2048 13/19;
-// beyond the products below the GPU's own time decides, and the BLAS kernels' larger tiles with it: 1 x 12576 x 4096 35/26).
+// x w^T.  For the few rows of a decode step by hdla_rows_gemm, which is a launch where the BLAS call is 19 us of host time.
+// GPU time alone (us, here / there, weights from HBM): 16 x 6416 x 2048 9.0/13.0,
+// 64 x 6416 x 2048 12.1/13.5, 64 x 4096 x 4096 14.6/15.0, 16 x 12576 x 4096 24.4/27.0; with more than 16 rows of x, which every
+// workgroup reads, the BLAS kernels' larger tiles win from there on: 32 x 12576 x 4096 29.3/25.1, 64 rows 35.4/26.6.
 constexpr int64_t FEW_ROWS = 64;
 Tensor project(const Tensor& x, const Tensor& w) {
-    const int64_t M = x.size(0), tiles = M <= 16 ? 1 : M <= 32 ? 2 : 4;
-    if (M > FEW_ROWS || tiles * w.numel() > (int64_t(32) << 20)) return at::mm(x, w.t());
+    const int64_t M = x.size(0), most = (M <= 16 ? int64_t(64) : int64_t(16)) << 20;
+    if (M > FEW_ROWS || w.numel() > most) return at::mm(x, w.t());
     const Tensor y = at::empty({x.size(0), w.size(0)}, x.options());
     check(api.rows_gemm((int32_t)x.size(0), (int32_t)w.size(0), (int32_t)w.size(1), ptr(x), x.stride(0), ptr(w), w.stride(0), ptr(y), y.stride(0),
                         stream_of(x)), "hdla_rows_gemm");

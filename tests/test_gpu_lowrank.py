@@ -62,6 +62,20 @@ def test_rows_gemm(M, N, K):
     assert lib.hdla_rows_gemm(M, N, K - 8, P(x), K + 8, P(w), K, P(y), N + 4, st) == -2
 
 
+@pytest.mark.parametrize("M", [16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(4095, 64), (4096, 512), (4116, 544), (4127, 2080)])
+def test_rows_gemm_many_columns(M, N, K):
+    """Both sides of the line from which a workgroup takes 32 rows of W, with a last one of few; blocks of K that the waves share unevenly."""
+    lib, st = _lib.load(), _lib.current_stream(DEV)
+    ld = (N + 3) // 4 * 4
+    x, w = _rn(8, M, K), _rn(9, N, K)
+    y = torch.full((M + 1, ld), 7.0, dtype=torch.bfloat16, device=DEV)
+    assert lib.hdla_rows_gemm(M, N, K, P(x), K, P(w), K, P(y), ld, st) == 0
+    # bf16 result of an exact sum of K products, up to K fp32 roundings: half a bf16 step each way, 2^-9 at most, on average 2^-9 / sqrt(3)
+    assert O.rel_l2(y[:M, :N], x.double() @ w.double().t()) <= 2e-3
+    assert bool((y[M:] == 7.0).all() and (y[:, N:] == 7.0).all())
+
+
 @pytest.mark.parametrize("rows,width,pad", [((1,), 8, 0), ((3, 0, 5), 24, 1), ((64, 64, 64, 16, 16, 4), 256, 12), ((129, 1, 1, 1, 1, 1, 1, 1), 1016, 0),
                                             ((1024, 1024, 1024, 64, 64, 16), 1024, 112)])
 def test_stacked_rows(rows, width, pad):
