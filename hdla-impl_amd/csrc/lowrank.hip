@@ -45,25 +45,25 @@ struct UpArgs {
     long long ldx;
     int M, d;
 };
-// A wave per 16 MT rows and 64 columns; blockIdx.y: decay or gate.  Every wave reads its 64 rows of W (8 or 16 KiB) from L2:
+// A wave per 16 MT rows and 32 NB columns; blockIdx.y: decay or gate.  Every wave reads its 64 rows of W (8 or 16 KiB) from L2:
 // with one row tile a wave that was 134 MB next to 50 MB of results, 28 us (8192 x 1024), with four 21.
-template <int D, int MT>
+template <int D, int MT, int NB>
 __global__ __launch_bounds__(256) void layer_up_kernel(UpArgs p) {
     constexpr int KB = D / 32;
     const int l = lane_id(), g = l >> 4, c = l & 15, which = blockIdx.y;
-    const long long unit = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int cbs = p.d / 64;
+    const long long unit = (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    const int cbs = p.d / (32 * NB);
     const long long r0 = unit / cbs * (16 * MT);
-    const int n0 = (int)(unit % cbs) * 64;
+    const int n0 = (int)(unit % cbs) * (32 * NB);
     if (r0 >= p.M) return;
     const bf16* w = p.w[which] + (long long)(n0 + row8(c)) * D + 8 * g;
-    TwoTiles xf[MT][KB], wf[2][2][KB];
+    TwoTiles xf[MT][KB], wf[NB][2][KB];
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int k = 0; k < KB; ++k) xf[m][k] = ld16(p.x0[which] + min(r0 + 16 * m + c, (long long)p.M - 1) * p.ldx + 8 * g + 32 * k);
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < NB; ++b)
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(256) void layer_up_kernel(UpArgs p) {
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
+        for (int b = 0; b < NB; ++b) {
             f32x4 acc[2] = {zero4(), zero4()};
 #pragma unroll
             for (int h = 0; h < 2; ++h)
@@ -299,23 +299,26 @@ extern "C" int hdla_layer_up_fwd(const hdla_up_dims* dims, const void* y, const 
     if (dims->rows == 0) return HDLA_OK;
     if (!y || !wf || !wg || !log_f || !gate) return HDLA_ERR_NULL;
     for (const void* p : {y, wf, wg, (const void*)f, (const void*)log_f, (const void*)gate}) if (!lr_al(p, 16)) return HDLA_ERR_ALIGN;
-    // four row tiles a wave where that leaves enough waves for the device
+    // four row tiles a wave where that leaves enough waves for the device; few rows: half the columns a wave, a compute unit each
     const int mt = (dims->rows + 63) / 64 * (dims->d / 64) >= 1024 ? 4 : 1;
-    const long long units = (dims->rows + 16 * mt - 1) / (16 * mt) * (dims->d / 64);
-    if ((units + 3) / 4 > 0x7fffffffLL) return HDLA_ERR_SHAPE;
+    const bool few = (dims->rows + 15) / 16 * (dims->d / 64) <= 256;
+    const long long units = (dims->rows + 16 * mt - 1) / (16 * mt) * (dims->d / (few ? 32 : 64)), each = few ? 1 : 4;
+    if ((units + each - 1) / each > 0x7fffffffLL) return HDLA_ERR_SHAPE;
     UpArgs a{};
     a.x0[0] = static_cast<const bf16*>(y) + dims->col_f; a.x0[1] = static_cast<const bf16*>(y) + dims->col_g;
     a.w[0] = static_cast<const bf16*>(wf); a.w[1] = static_cast<const bf16*>(wg);
     a.f = static_cast<bf16*>(f); a.log_f = static_cast<bf16*>(log_f); a.gate = static_cast<bf16*>(gate);
     a.ldx = dims->ld; a.M = (int)dims->rows; a.d = dims->d;
-    const dim3 grid((unsigned)((units + 3) / 4), 2), block(256);
+    const dim3 grid((unsigned)((units + each - 1) / each), 2), block((unsigned)(64 * each));
     const hipStream_t s = static_cast<hipStream_t>(stream);
     if (dims->D == 64) {
-        if (mt == 4) hipLaunchKernelGGL((layer_up_kernel<64, 4>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((layer_up_kernel<64, 1>), grid, block, 0, s, a);
+        if (mt == 4) hipLaunchKernelGGL((layer_up_kernel<64, 4, 2>), grid, block, 0, s, a);
+        else if (few) hipLaunchKernelGGL((layer_up_kernel<64, 1, 1>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((layer_up_kernel<64, 1, 2>), grid, block, 0, s, a);
     } else {
-        if (mt == 4) hipLaunchKernelGGL((layer_up_kernel<128, 4>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((layer_up_kernel<128, 1>), grid, block, 0, s, a);
+        if (mt == 4) hipLaunchKernelGGL((layer_up_kernel<128, 4, 2>), grid, block, 0, s, a);
+        else if (few) hipLaunchKernelGGL((layer_up_kernel<128, 1, 1>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((layer_up_kernel<128, 1, 2>), grid, block, 0, s, a);
     }
     return (int)hipGetLastError();
 }

@@ -43,6 +43,7 @@ struct Api {
     HDLA_FN(recurrent_fwd); HDLA_FN(param_recurrent_fwd); HDLA_FN(normalize_fwd); HDLA_FN(normalize_bwd);
     HDLA_FN(normalize_workspace_bytes); HDLA_FN(layer_pre_fwd); HDLA_FN(layer_pre_bwd); HDLA_FN(layer_up_fwd); HDLA_FN(layer_down);
     HDLA_FN(layer_up_wgrad); HDLA_FN(layer_up_wgrad_workspace_bytes); HDLA_FN(rows_gemm); HDLA_FN(sum_partials); HDLA_FN(stack_rows);
+    HDLA_FN(layer_step);
 #undef HDLA_FN
 } api;
 PyObject* error_class = nullptr;                 // _lib.HdlaError
@@ -509,8 +510,8 @@ PyObject* py_normalize(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // HDLA_Custom.forward in its common form (bf16, silu activations, one block, beta, output gate, no biases; layer.py checks
 // that) as one call and one autograd node.  What one node buys over one per step: the GEMMs read the inner activations of
 // the low-rank projections where they lie in y and write their gradients where they belong in dy (no copies), the rows of
-// the concatenated weight can be padded to what the GEMMs like, and the host is out of the way (a decode step is ten
-// kernels of 4-10 us each, behind 200 us of Python).
+// the concatenated weight can be padded to what the GEMMs like, and the host is out of the way (200 us of Python
+// around a decode step's kernels of 4-10 us each).
 struct LayerCfg {
     int64_t H, groups;
     bool norm_q, norm_v;
@@ -577,6 +578,41 @@ Tensor project(const Tensor& x, const Tensor& w) {
 // everything between x and the output; what the backward pass needs of it
 struct LayerFwd { Tensor x, w, y, f, g, o, n, out, ht, boundary; ChunkIn op; hdla_dims dims; };
 
+// A few tokens: what is between the projections in one to three launches, without the tensors that the steps would hand on.  (Many
+// tokens are better off with what does not depend on the state done for all of them at once.)  One token after a cached state, us a
+// call, as six launches and eleven tensors -> as this (batch x channels, heads): 1 x 512, 8 37.8 -> 23.9, 16 x 2048, 16 36.9 -> 25.2,
+// 25 x 4096, 32 67.7 -> 54.5, 256 x 1024, 16 71 -> 57, 256 x 4096, 32 281 -> 249.  The low-rank products in the same launch or in
+// one before it: 23.9 / 26.8, 25.2 / 27.0, 54.5 / 55.9, 57 / 60, 249 / 252; the other way round only at 256 x 2048, 32: 85.3 / 84.5.
+void layer_step(const Tensor* P, const LayerCfg& f, const LayerCols& L, const hdla_pre_dims& pd, int64_t T, const Tensor& h0, bool want_ht,
+                LayerFwd& r) {
+    const int64_t rows = pd.rows, N = rows / T;
+    void* const s = stream_of(r.x);
+    const auto opt = r.x.options();
+    const bool in_step = T == 1, norm_in_step = f.groups == L.H;
+    r.n = at::empty({rows, L.d}, opt);
+    const hdla_up_dims ud = up_dims(L, rows);
+    const hdla_norm_dims nd = norm_dims(r.n, P[8], f.gate_pos, f.c, f.eps, f.groups);
+    const int64_t parts = (norm_in_step ? 0 : 2) + (in_step ? 0 : norm_in_step ? 2 : 1);     // gate, o, log_f as far as they are handed on
+    Tensor between;
+    if (parts) between = at::empty({parts, rows * L.d}, opt);
+    char* room = static_cast<char*>(ptr(between));
+    void *gate = nullptr, *o = ptr(r.n), *log_f = nullptr;
+    const auto take = [&] { void* const p = room; room += rows * L.d * 2; return p; };
+    if (!norm_in_step) o = take();
+    if (!norm_in_step || !in_step) gate = take();
+    if (!in_step) {
+        log_f = take();
+        check(api.layer_up_fwd(&ud, ptr(r.y), ptr(P[6]), ptr(P[7]), nullptr, log_f, gate, s), "hdla_layer_up_fwd");
+    }
+    Tensor state;
+    if (h0.defined()) state = h0.to(at::kFloat).contiguous();
+    if (want_ht) r.ht = at::empty({N, L.H, L.D, L.D}, opt.dtype(at::kFloat));
+    check(api.layer_step(&pd, in_step ? &ud : nullptr, norm_in_step ? &nd : nullptr, (int32_t)T, ptr(r.y), in_step ? ptr(P[6]) : nullptr,
+                         in_step ? ptr(P[7]) : nullptr, log_f, gate, norm_in_step ? ptr(P[8]) : nullptr, fptr(state), o, fptr(r.ht), s),
+          "hdla_layer_step");
+    if (!norm_in_step) check(api.normalize_fwd(&nd, o, ptr(P[8]), gate, ptr(r.n), s), "hdla_normalize_fwd");
+}
+
 // params: wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo; r.w gathered; keep: a backward pass follows
 void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, const Tensor& h0, bool want_ht, bool chunked, bool keep, LayerFwd& r) {
     const int64_t B = x3.size(0), T = x3.size(1), d = x3.size(2), rows = B * T;
@@ -585,6 +621,11 @@ void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, const T
     r.x = x3.contiguous().view({rows, d});
     r.y = project(r.x, r.w);
     const hdla_pre_dims pd = pre_dims(L, f, rows);
+    if (!chunked && T < RECURRENT_BELOW) {
+        layer_step(P, f, L, pd, T, h0, want_ht, r);
+        r.out = project(r.n, P[9]).view({B, T, d});
+        return;
+    }
     ChunkIn& in = r.op;
     in.q = at::empty({B, T, L.H, L.D}, opt); in.k = at::empty({B, T, L.H, L.D}, opt); in.v = at::empty({B, T, L.H, L.D}, opt);
     in.beta = at::empty({B, T, L.H, 1}, opt);
@@ -835,7 +876,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HDLA_FN(strerror) HDLA_FN(workspace_bytes) HDLA_FN(record_bytes) HDLA_FN(record_workspace_bytes) HDLA_FN(chunk_fwd_b) HDLA_FN(chunk_bwd_b)
     HDLA_FN(recurrent_fwd) HDLA_FN(param_recurrent_fwd) HDLA_FN(normalize_fwd) HDLA_FN(normalize_bwd)
     HDLA_FN(normalize_workspace_bytes) HDLA_FN(layer_pre_fwd) HDLA_FN(layer_pre_bwd) HDLA_FN(layer_up_fwd) HDLA_FN(layer_down)
-    HDLA_FN(layer_up_wgrad) HDLA_FN(layer_up_wgrad_workspace_bytes) HDLA_FN(rows_gemm) HDLA_FN(sum_partials) HDLA_FN(stack_rows)
+    HDLA_FN(layer_up_wgrad) HDLA_FN(layer_up_wgrad_workspace_bytes) HDLA_FN(rows_gemm) HDLA_FN(sum_partials) HDLA_FN(stack_rows) HDLA_FN(layer_step)
 #undef HDLA_FN
     Py_INCREF(a[1]);
     Py_XDECREF(error_class);

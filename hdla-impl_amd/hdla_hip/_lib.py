@@ -147,6 +147,8 @@ def load():
     lib.hdla_layer_up_wgrad.argtypes = [UF] + [P] * 7 + [ctypes.c_size_t, P]
     lib.hdla_layer_up_wgrad_workspace_bytes.restype = ctypes.c_size_t
     lib.hdla_layer_up_wgrad_workspace_bytes.argtypes = [UF]
+    lib.hdla_layer_step.restype = ctypes.c_int
+    lib.hdla_layer_step.argtypes = [PF, UF, NF, ctypes.c_int32] + [P] * 10
     lib.hdla_rows_gemm.restype = ctypes.c_int
     lib.hdla_rows_gemm.argtypes = [ctypes.c_int32] * 3 + [P, ctypes.c_int64, P, ctypes.c_int64, P, ctypes.c_int64, P]
     lib.hdla_sum_partials.restype = ctypes.c_int

@@ -339,6 +339,16 @@ int hdla_layer_up_wgrad(const hdla_up_dims* dims, const void* y, const void* f, 
                         void* dwf, void* dwg, void* workspace, size_t workspace_bytes, void* stream);
 size_t hdla_layer_up_wgrad_workspace_bytes(const hdla_up_dims* dims);
 
+/* hdla_layer_pre_fwd and hdla_param_recurrent_fwd (scale 1, forward) in one launch, for sequences of T tokens each (rows = N T);
+ * bf16, D 64 or 128; h0, ht: [N, H, D, D] or NULL (h0 == NULL: zeros).
+ * norm given (one group a head: G = H, E = D, with a gate): hdla_normalize_fwd as well, o is the normalised and gated output and
+ * weight its weight [H D] or NULL.
+ * up given (T = 1): hdla_layer_up_fwd as well, wf and wg are its weights; log_f is not used and gate, unless NULL, written.
+ * Without it log_f and (with norm) gate [rows, H, D] are inputs. */
+int hdla_layer_step(const hdla_pre_dims* pre, const hdla_up_dims* up, const hdla_norm_dims* norm, int32_t T, const void* y,
+                    const void* wf, const void* wg, const void* log_f, void* gate, const void* weight, const float* h0, void* o,
+                    float* ht, void* stream);
+
 /* y [M, N] = x [M, K] w [N, K]^T in bf16 for M <= 64 rows and K a multiple of 32 (the large projections of a decode step;
  * nn.Linear without bias).  ldx, ldw: row strides in elements, multiples of 8; ldy: a multiple of 4; x, w 16-byte, y 8-byte
  * aligned. */

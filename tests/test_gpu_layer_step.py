@@ -1,0 +1,118 @@
+"""The layer's decode step between the projections in one launch (csrc/layer_step.hip) against the three kernels that it stands
+for, run one after the other."""
+import ctypes
+
+import pytest
+import torch
+
+from hdla_hip import _lib
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda")
+
+
+P = _lib.ptr
+
+
+def _rn(seed, *shape):
+    return torch.randn(*shape, generator=torch.Generator(device=DEV).manual_seed(seed), device=DEV)
+
+
+def _rel(a, b):
+    a, b = a.double(), b.double()
+    return float((a - b).norm() / b.norm())
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("N,T,H,norm_q,norm_v,gate_pos,weight,state", [
+    (1, 1, 2, True, False, 1, "bf16", True), (3, 1, 6, True, True, 2, "fp32", True), (2, 2, 4, False, True, 1, None, False),
+    (2, 8, 16, True, False, 2, "bf16", True), (40, 1, 8, False, False, 1, "fp32", False)])
+def test_layer_step(D, N, T, H, norm_q, norm_v, gate_pos, weight, state):
+    lib, st, ref = _lib.load(), _lib.current_stream(DEV), ctypes.byref
+    rows, d = N * T, H * D
+    f0, ld = (3 * d + H + 1 + 7) // 8 * 8, (3 * d + H + 1 + 7) // 8 * 8 + 2 * D + 8
+    y = _rn(1, rows, ld).bfloat16()
+    y[0, d:d + D] = 0.                                          # a head of k of length nought, values at the ends of the activations
+    y[0, 0:4] = torch.tensor([80., -80., 3e4, -3e4])
+    wf, wg = (_rn(6, d, D) * .2).bfloat16(), (_rn(7, d, D) * .2).bfloat16()
+    w = None if weight is None else (1. + .1 * _rn(4, d)).to(torch.bfloat16 if weight == "bf16" else torch.float32)
+    h0 = _rn(5, N, H, D, D) if state else None
+    pre = _lib.HdlaPreDims(rows, H, D, _lib.dtype_code(torch.bfloat16), ld, 2 * d, d, 0, 3 * d + 1, norm_q, 1, norm_v, 2.0, 1e-5, 0)   # v, k, q: any columns
+    up = _lib.HdlaUpDims(rows, d, D, ld, f0, f0 + D)
+    nd = _lib.HdlaNormDims(rows, H, D, _lib.dtype_code(torch.bfloat16), _lib.dtype_code(torch.float32) if weight == "fp32" else _lib.dtype_code(torch.bfloat16), gate_pos, D ** .5, 1e-5)
+
+    # the kernels that it stands for
+    new = lambda *s: torch.empty(*s, device=DEV, dtype=torch.bfloat16)
+    q, k, v, log_f, gate, ro, rn = (new(rows, H, D) for _ in range(7))
+    beta, rht = new(rows, H), torch.empty(N, H, D, D, device=DEV)
+    assert lib.hdla_layer_up_fwd(ref(up), P(y), P(wf), P(wg), None, P(log_f), P(gate), st) == 0
+    assert lib.hdla_layer_pre_fwd(ref(pre), P(y), P(q), P(k), P(v), P(beta), st) == 0
+    cd = _lib.make_dims(N, T, H, D, D, 2, N, torch.bfloat16, torch.bfloat16, 1.0, None)
+    assert lib.hdla_param_recurrent_fwd(ref(cd), P(q), P(k), P(v), P(beta), P(log_f), 0, P(h0), P(ro), P(rht), st) == 0
+    assert lib.hdla_normalize_fwd(ref(nd), P(ro), P(w), P(gate), P(rn), st) == 0
+    # Sums over a head run in another order, 2^-24 each; where that moves one of the values that are rounded to bf16 across the middle
+    # between two of its numbers (one in 2^10, sums of 128 terms), it moves by 2^-8 of itself.  Not more than a hundredth of all does.
+    tol = 2 ** -8 * .1
+
+    def run(norm, with_up, want_ht=True):
+        o, ht, g = torch.full((rows + 1, H, D), 7., device=DEV, dtype=torch.bfloat16), torch.empty_like(rht), new(rows, H, D)
+        assert lib.hdla_layer_step(ref(pre), ref(up) if with_up else None, ref(nd) if norm else None, T, P(y), P(wf) if with_up else None,
+                                   P(wg) if with_up else None, None if with_up else P(log_f), P(g) if with_up else P(gate), P(w) if norm else None,
+                                   P(h0), P(o), P(ht) if want_ht else None, st) == 0
+        assert bool((o[rows:] == 7.).all())
+        assert _rel(o[:rows], rn if norm else ro) <= tol
+        assert not want_ht or _rel(ht, rht) <= tol
+        assert not with_up or _rel(g, gate) <= tol
+        return o
+
+    first = run(True, False)
+    assert torch.equal(first, run(True, False, False))          # with no final state asked for
+    run(False, False)
+    if T == 1:
+        run(True, True)
+        run(False, True)
+    bad = lambda pre, up, nd, T, y=P(y): lib.hdla_layer_step(pre, up, nd, T, y, P(wf), P(wg), P(log_f), P(gate), None, None, P(ro), None, st)
+    assert bad(ref(pre), None, None, 0) == -2 and bad(ref(pre), None, None, rows + 1) == -2 and bad(ref(pre), ref(up), None, 2) == -2
+    assert bad(ref(pre), None, ref(_lib.HdlaNormDims(rows, 2 * H, D // 2, _lib.dtype_code(torch.bfloat16), _lib.dtype_code(torch.bfloat16), 1, 1., 1e-5)), T) == -2
+    assert bad(ref(pre), None, None, T, None) != 0 and bad(ref(pre), None, None, T, ctypes.c_void_p(y.data_ptr() + 2)) != 0
+
+
+@pytest.mark.parametrize("norm", ["rmsnorm", "grouprmsnorm"])
+@pytest.mark.parametrize("B,T,H", [(3, 1, 4), (65, 1, 2), (2, 8, 4), (2, 9, 4)])
+def test_layer_routes(B, T, H, norm):
+    """Both sides of the lines that the native call chooses by (tokens, rows, the norm's groups) next to the layer's Python
+    code, and replays of a captured step."""
+    from hdla_hip.layer import HDLA_Custom, RecurrentCache
+    torch.manual_seed(3)
+    with torch.device("cuda"):
+        m = HDLA_Custom(64 * H, H, token_mixer_init_type=2, rescale_type=0, token_mixer_norm_type=norm).to(torch.bfloat16).eval()
+    x, s0 = _rn(9, B, T, 64 * H).bfloat16(), _rn(10, B, H, 64, 64)
+
+    def step():
+        cache = RecurrentCache()
+        cache.update(recurrent_state=[s0], layer_idx=0, offset=T)
+        o, cache = m(x, past_key_values=cache, use_cache=True)
+        return o, cache[0]["recurrent_state"][0]
+
+    with torch.no_grad():
+        a, sa = step()
+        m._forward_native = lambda *_: None
+        b, sb = step()
+        del m._forward_native
+        # Both are rounded to bf16 nine times on the way (y, q, k, v, f, the decay, the gate, o, the norm's output), each time by up to
+        # 2^-9, 2^-9 / sqrt(3) in the mean, and in part at other places: sqrt(2 * 9) of that
+        assert _rel(a, b) <= 5e-3 and _rel(sa, sb) <= 5e-3
+        g, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            step()
+        torch.cuda.current_stream().wait_stream(side)
+        with torch.cuda.graph(g):
+            c, sc = step()
+        for i in range(3):
+            s0.mul_(.5)
+            x.neg_()
+            want, ws = step()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(c, want) and torch.equal(sc, ws)
