@@ -83,7 +83,7 @@ int fused_segments(const hdla_dims* d) {
     return nseg;
 }
 
-// ---- time segments of the stand-alone scans (scan_impl.cuh): where a whole sequence per workgroup would leave most of the
+// ---- time segments of the stand-alone scans (scan_impl.cuh, scan_out.cuh, scan_grad.cuh): where a whole sequence per workgroup would leave most of the
 // device idle.  A launch for the segments' records, one that chains them (together 10 us at the least), then the scans on
 // shorter sequences: twice the steps, of which nseg run at once.  Measured (us, forward / backward pass, one segment ->
 // as many as chosen here): fp32, K=V=64, 16 lanes of 63 chunks 156/224 -> 69/157 (8); fp32, K=V=128, 4 lanes of 125

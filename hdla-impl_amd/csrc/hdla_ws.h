@@ -115,7 +115,7 @@ struct Ws {
     int sa_stride;            // bytes between the forward-scan blocks of consecutive (chunk, head) slots
 };
 
-// Time segments of the stand-alone scans (scan_impl.cuh): records per (sequence, head, segment), fp32 tiles in fragment
+// Time segments of the stand-alone scans (scan_impl.cuh, scan_out.cuh, scan_grad.cuh): records per (sequence, head, segment), fp32 tiles in fragment
 // order.  The forward direction's, then the reverse direction's.
 struct SegRec {
     int nseg;                 // segments per sequence; 1: no records

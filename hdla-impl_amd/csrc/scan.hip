@@ -1,15 +1,23 @@
-// Host-side dispatch of the scan kernels by head shape (kernels: scan_impl.cuh, compiled in scan_*.hip).
+// Host-side dispatch of the scan kernels by head shape (kernels: scan_out.cuh and scan_grad.cuh, fp32 scan_impl.cuh; compiled in scan_*.hip).
 #include "scan_shapes.h"
 
 namespace hdla {
 
 template <typename T>
 static hipError_t launch_scan(const ChunkArgs<T>& a, int K, int V, ScanKind kind, hipStream_t stream) {
-    if (K == 64 && V == 64) return launch_scan_shape<T, 64, 64>(a, kind, stream);
-    if (K == 128 && V == 128) return launch_scan_shape<T, 128, 128>(a, kind, stream);
-    if (K == 64 && V == 128) return launch_scan_shape<T, 64, 128>(a, kind, stream);
-    if (K == 128 && V == 64) return launch_scan_shape<T, 128, 64>(a, kind, stream);
-    return hipErrorInvalidValue;
+    if constexpr (sizeof(T) == 2) {
+        if (K == 64 && V == 64) return launch_scan_grad_shape<64, 64>(a, kind, stream);
+        if (K == 128 && V == 128) return launch_scan_grad_shape<128, 128>(a, kind, stream);
+        if (K == 64 && V == 128) return launch_scan_grad_shape<64, 128>(a, kind, stream);
+        if (K == 128 && V == 64) return launch_scan_grad_shape<128, 64>(a, kind, stream);
+        return hipErrorInvalidValue;
+    } else {
+        if (K == 64 && V == 64) return launch_scan_shape<T, 64, 64>(a, kind, stream);
+        if (K == 128 && V == 128) return launch_scan_shape<T, 128, 128>(a, kind, stream);
+        if (K == 64 && V == 128) return launch_scan_shape<T, 64, 128>(a, kind, stream);
+        if (K == 128 && V == 64) return launch_scan_shape<T, 128, 64>(a, kind, stream);
+        return hipErrorInvalidValue;
+    }
 }
 
 template <typename T>
@@ -38,19 +46,18 @@ hipError_t launch_scan_pair(const ChunkArgs<T>& a, int K, int V, hipStream_t str
 template <typename T>
 hipError_t launch_scan_segments(const ChunkArgs<T>& a, int K, int V, bool both, hipStream_t stream) {
     if constexpr (sizeof(T) == 2) {
-        if (!both) {
-            if (K == 64 && V == 64) return launch_scan_out_segments_shape<64, 64>(a, stream);
-            if (K == 128 && V == 128) return launch_scan_out_segments_shape<128, 128>(a, stream);
-            if (K == 64 && V == 128) return launch_scan_out_segments_shape<64, 128>(a, stream);
-            if (K == 128 && V == 64) return launch_scan_out_segments_shape<128, 64>(a, stream);
-            return hipErrorInvalidValue;
-        }
+        if (K == 64 && V == 64) return both ? launch_scan_grad_segments_shape<64, 64>(a, stream) : launch_scan_out_segments_shape<64, 64>(a, stream);
+        if (K == 128 && V == 128) return both ? launch_scan_grad_segments_shape<128, 128>(a, stream) : launch_scan_out_segments_shape<128, 128>(a, stream);
+        if (K == 64 && V == 128) return both ? launch_scan_grad_segments_shape<64, 128>(a, stream) : launch_scan_out_segments_shape<64, 128>(a, stream);
+        if (K == 128 && V == 64) return both ? launch_scan_grad_segments_shape<128, 64>(a, stream) : launch_scan_out_segments_shape<128, 64>(a, stream);
+        return hipErrorInvalidValue;
+    } else {
+        if (K == 64 && V == 64) return launch_scan_segments_shape<T, 64, 64>(a, both, stream);
+        if (K == 128 && V == 128) return launch_scan_segments_shape<T, 128, 128>(a, both, stream);
+        if (K == 64 && V == 128) return launch_scan_segments_shape<T, 64, 128>(a, both, stream);
+        if (K == 128 && V == 64) return launch_scan_segments_shape<T, 128, 64>(a, both, stream);
+        return hipErrorInvalidValue;
     }
-    if (K == 64 && V == 64) return launch_scan_segments_shape<T, 64, 64>(a, both, stream);
-    if (K == 128 && V == 128) return launch_scan_segments_shape<T, 128, 128>(a, both, stream);
-    if (K == 64 && V == 128) return launch_scan_segments_shape<T, 64, 128>(a, both, stream);
-    if (K == 128 && V == 64) return launch_scan_segments_shape<T, 128, 64>(a, both, stream);
-    return hipErrorInvalidValue;
 }
 template hipError_t launch_scan_segments<bf16>(const ChunkArgs<bf16>&, int, int, bool, hipStream_t);
 template hipError_t launch_scan_segments<float>(const ChunkArgs<float>&, int, int, bool, hipStream_t);

@@ -1,14 +1,13 @@
-// Scan kernels, bf16 inputs, head sizes K=128 V=64, K=128 V=128 (see scan_impl.cuh, scan_out.cuh).
-#include "scan_impl.cuh"
-#include "scan_out.cuh"
+// Scan kernels, bf16 inputs, head sizes K=128 V=64, K=128 V=128 (see scan_out.cuh, scan_grad.cuh).
+#include "scan_grad.cuh"
 
 namespace hdla {
-template hipError_t launch_scan_shape<bf16, 128, 64>(const ChunkArgs<bf16>&, ScanKind, hipStream_t);
-template hipError_t launch_scan_segments_shape<bf16, 128, 64>(const ChunkArgs<bf16>&, bool, hipStream_t);
-template hipError_t launch_scan_shape<bf16, 128, 128>(const ChunkArgs<bf16>&, ScanKind, hipStream_t);
-template hipError_t launch_scan_segments_shape<bf16, 128, 128>(const ChunkArgs<bf16>&, bool, hipStream_t);
 template hipError_t launch_scan_out_shape<128, 64>(const ChunkArgs<bf16>&, bool, hipStream_t);
 template hipError_t launch_scan_out_segments_shape<128, 64>(const ChunkArgs<bf16>&, hipStream_t);
+template hipError_t launch_scan_grad_shape<128, 64>(const ChunkArgs<bf16>&, ScanKind, hipStream_t);
+template hipError_t launch_scan_grad_segments_shape<128, 64>(const ChunkArgs<bf16>&, hipStream_t);
 template hipError_t launch_scan_out_shape<128, 128>(const ChunkArgs<bf16>&, bool, hipStream_t);
 template hipError_t launch_scan_out_segments_shape<128, 128>(const ChunkArgs<bf16>&, hipStream_t);
+template hipError_t launch_scan_grad_shape<128, 128>(const ChunkArgs<bf16>&, ScanKind, hipStream_t);
+template hipError_t launch_scan_grad_segments_shape<128, 128>(const ChunkArgs<bf16>&, hipStream_t);
 }  // namespace hdla

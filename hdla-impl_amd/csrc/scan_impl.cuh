@@ -5,40 +5,25 @@
 // scan_bwd replaces HRDPLR/bwd_triton.py:127-222 (reverse recurrence of the state gradient, dh checkpoints,
 // dh0) fused with the dv_new part of HRDPLR/bwd_triton.py:30-105.
 //
-// A computing wave owns one 16-column block of the fp32 state of a (sequence, head) for the whole sequence, in
+// A wave owns one 16-column block of the fp32 state of a (sequence, head) for the whole sequence, in
 // registers as the row fragment of S^T (rows = value column, inner = channel), which is at once the operand
 // layout of the next product: w S, qg S and the rank updates chain through registers with no cross-lane
 // movement.  A workgroup holds NWC such waves; a head's V/16 column blocks are split over (V/16)/NWC workgroups.
 //
-// What bounds a step without the measures below is not arithmetic but memory: one compute unit sustains only a few
-// tens of GB/s of loads that miss to HBM however many it has in flight, a wave may have at most 63 memory
-// instructions outstanding and they complete in order, and all column blocks of a head need the same w / kg / bg /
-// qg tiles.  Hence
-//  * few heads are spread over many compute units (the split above, chosen by the launcher from the number of
-//    heads), each workgroup fetching the chunk's shared operand block (one contiguous block per chunk, written
-//    by the prep kernel) once for its NWC waves;
-//  * the block goes through LDS.  Three LDS slots rotate with ONE LDS-only barrier per chunk (global loads stay
-//    in flight across it):
-//       step t:  barrier                      block t+1 (written during step t-1) becomes visible
-//                share of block t+2 -> slot (t+2) % 3          (its last readers finished before the barrier)
-//                read the operands of the state update of chunk t from slot t % 3
-//                phase 1: v_new (operands already in registers, read during step t-1)
-//                read the phase-1 operands of chunk t+1 from slot (t+1) % 3
-//                phase 2: state update
-//    so every LDS read has a phase of matrix products between its issue and its first use;
-//  * for 2-byte inputs, four "memory waves" per workgroup do nothing but move data: they hold the register ring
-//    of block shares (6 chunks in flight), hand them to LDS, and copy the results, which the computing waves
-//    leave in an LDS outbox laid out like the chunk's record in global memory, out to global memory a step later.
-//    The computing waves then touch global memory only for the few tiles that are theirs alone (rows of do in the
-//    reverse scan; tiles of u^T and v^T in the forward scans, and for K = 64 these too travel through LDS with the
-//    block).  Without memory waves (fp32 inputs, or eight computing waves) the computing waves do all of that
-//    themselves.
+// This file: 4-byte elements, and the chaining of the segments' records for both element sizes (2-byte elements: scan_out.cuh,
+// scan_grad.cuh).  All column blocks of a head need the same w / kg / bg / qg tiles: a workgroup fetches the chunk's shared operand block
+// (one contiguous block per chunk, written by the prep kernel) once for its NWC waves, which hold a register ring of their shares of the
+// blocks to come and hand them to LDS.  Three LDS slots rotate with ONE LDS-only barrier per chunk (global loads stay in flight across it):
+//    step t:  barrier                      block t+1 (written during step t-1) becomes visible
+//             share of block t+2 -> slot (t+2) % 3          (its last readers finished before the barrier)
+//             phase 1: v_new (operands already in registers, read during step t-1); the operands of the state update from slot t % 3
+//             phase 2: state update; the phase-1 operands of chunk t+1 from slot (t+1) % 3
+// so every LDS read has a phase of matrix products between its issue and its first use.
 #pragma once
 #include "hdla_common.cuh"
 #include "scan_shapes.h"
 
 namespace hdla {
-
 
 // workgroup barrier that orders LDS accesses only: global loads issued before it may still be outstanding
 __device__ __forceinline__ void lds_barrier() {
@@ -52,54 +37,26 @@ constexpr int NSLOT = 3;
 template <typename T, int K, int V, int NWC> struct ScanCfg {
     static constexpr int VT = V / 16, SPLIT = VT / NWC;   // workgroups per head
     static constexpr int KB = K * (int)sizeof(T);         // bytes of one operand row
-    static constexpr int NM = (sizeof(T) == 2 && NWC <= 4) ? 4 : 0;   // memory waves
-    static constexpr int THREADS = 64 * (NWC + NM);
-    static constexpr int NLD = NM ? NM : NWC;             // waves that split the loading of a block
-    // forward scans with memory waves (rows of 128 bytes: the larger ones have no registers to spare): the tiles of
-    // u^T and v^T of the workgroup's column blocks travel through LDS with the shared block (appended to it), so
-    // that the computing waves issue no global loads at all
-    static constexpr int OWN_UT = (NM && KB <= 128) ? NWC * PAIR * (int)sizeof(T) : 0, OWN_VTT = (NM && KB <= 128) ? NWC * TILE * (int)sizeof(T) : 0;
-    static constexpr int OWN_FWD = (OWN_UT + OWN_VTT + 1023) & ~1023;
-    // Depth of the register ring of block shares (chunks in flight from global memory) and of the computing
-    // waves' own tiles; multiples of the number of slots so that slot numbers are static in the unrolled loops;
-    // 0: no ring, one chunk at a time.
-    static constexpr int DR_SHARE = NM ? 6 : (KB <= 128 ? 6 : KB <= 256 ? 3 : 0);
-    static constexpr int DR_OWN = NM ? (KB <= 128 ? 6 : 3) : DR_SHARE;
+    static constexpr int THREADS = 64 * NWC;
+    // Depth of the register ring of block shares (chunks in flight from global memory) and of the waves' own tiles; a multiple of the
+    // number of slots so that slot numbers are static in the unrolled loops; 0: no ring, one chunk at a time.
+    static constexpr int DR = KB <= 256 ? 3 : 0;
     // Whether LDS reads are issued a phase ahead of their use as described above, or left where the compiler
     // puts them (the shapes whose operands would not fit the register file twice over) ...
-    static constexpr bool pipelined(bool with_o) { return KB <= 128 || (KB <= 256 && !(NWC == 8 && with_o)); }
-    // ... and whether that includes the operands of the state update
-    static constexpr bool early_update_reads(bool with_o) { return KB <= 128 || (KB <= 256 && NWC <= 4 && (NM == 0 || with_o)); }
-    // Issued a few at a time between the products, or all of them before the phase.  4-byte elements have twice the bytes and
-    // four times the cycles a product to hide them behind; with 2-byte ones it is not the issue of the reads that a step waits
-    // for.  Measured, before the phase -> spread: fp32 K = V = 64, 2 x 1003 tokens of 8 heads, records 45 -> 39 us, forward
-    // scan 22.5 -> 21.0, scan pair 27.7 -> 26.3; bf16 K = V = 128, 2 x 1537 tokens of 8 heads, records 25.6 -> 27.5, pair 82 -> 84.
-    static constexpr bool SPREAD = sizeof(T) == 4;
+    static constexpr bool pipelined(bool with_o) { return KB <= 256 && !(NWC == 8 && with_o); }
+    // ... and whether that includes the operands of the state update.  They are issued a few at a time between the products, not all of them
+    // before the phase: K = V = 64, 2 x 1003 tokens of 8 heads, before the phase -> spread: records 45 -> 39 us, forward scan 22.5 -> 21.0,
+    // scan pair 27.7 -> 26.3.
+    static constexpr bool early_update_reads() { return KB <= 256 && NWC <= 4; }
 };
 
-// A shared operand block as the loading waves see it: NI pieces of 1 KiB, lane l taking 16 bytes of each.  The
-// first NT pieces hold tiles that are handed to LDS transposed, so a lane must hold whole fragments of them: for
-// 2-byte elements a piece is a tile pair in its stored order; for 4-byte elements a piece is one tile of a pair,
-// 16 of every 32 bytes.
-template <int ES> __device__ __forceinline__ int piece_off(int i, int l, bool tiles) {
-    if (ES == 4 && tiles) return (i >> 1) * 2048 + l * 32 + (i & 1) * 16;
-    return i * 1024 + l * 16;
-}
+// A shared operand block as the waves that load it see it: NI pieces of 1 KiB, lane l taking 16 bytes of each.  The first NT pieces hold
+// tiles that are handed to LDS transposed, so a lane must hold whole fragments of them: such a piece is one tile of a pair, 16 of every 32 bytes.
+__device__ __forceinline__ int piece_off(int i, int l, bool tiles) { return tiles ? (i >> 1) * 2048 + l * 32 + (i & 1) * 16 : i * 1024 + l * 16; }
 // the whole block is contiguous in global memory (forward scans)
 struct BlockOne {
     const char* p;
     __device__ __forceinline__ const char* piece(int i, int l, bool) const { return p + i * 1024 + l * 16; }
-};
-// forward scan with memory waves: the block, then the workgroup's tiles of u^T, then those of v^T (the last piece may
-// reach past them: those lanes read inside the tiles again, what they leave in LDS is never looked at)
-template <int NIB, int UTB, int VTB> struct BlockFwd {
-    const char *b, *ut, *vtt;
-    __device__ __forceinline__ const char* piece(int i, int l, bool) const {
-        if (i < NIB) return b + i * 1024 + l * 16;
-        const int off = (i - NIB) * 1024 + l * 16;
-        if (off < UTB) return ut + off;
-        return vtt + (off - UTB) % VTB;
-    }
 };
 // reverse scan: W and BGT (NIF pieces) and the piece holding EGL come from the forward-scan block of the (chunk,
 // head), the rest is the reverse-scan block
@@ -108,28 +65,17 @@ template <typename T, int K> struct BlockTwo {
     __device__ __forceinline__ const char* piece(int i, int l, bool tiles) const {
         constexpr SlotB S = slot_bwd(K, sizeof(T));
         static_assert(S.EGL_SRC % 1024 == 0, "EGL starts a piece");
-        if (i < S.NIF) return f + piece_off<sizeof(T)>(i, l, tiles);
+        if (i < S.NIF) return f + piece_off(i, l, tiles);
         if (i == S.NIF) return f + S.EGL_SRC + l * 16;
         return r + (i - S.NIF - 1) * 1024 + l * 16;
     }
 };
 
-// 16 bytes of fragments of type T, each tile transposed (a product with the identity: exact)
+// 16 bytes of fragments, the tile transposed (a product with the identity: exact)
 template <typename T> __device__ __forceinline__ i32x4 transpose_piece(i32x4 x) {
-    const Frag<T> ident = ident_frag<T>();
-    if constexpr (sizeof(T) == 2) {
-        const s16x8 y = __builtin_bit_cast(s16x8, x);
-        Frag<T> f0, f1;
-        f0.v = __builtin_shufflevector(y, y, 0, 1, 2, 3);
-        f1.v = __builtin_shufflevector(y, y, 4, 5, 6, 7);
-        f0 = transpose(f0, ident);
-        f1 = transpose(f1, ident);
-        return __builtin_bit_cast(i32x4, __builtin_shufflevector(f0.v, f1.v, 0, 1, 2, 3, 4, 5, 6, 7));
-    } else {
-        Frag<T> f;
-        f.v = __builtin_bit_cast(f32x4, x);
-        return __builtin_bit_cast(i32x4, transpose(f, ident).v);
-    }
+    Frag<T> f;
+    f.v = __builtin_bit_cast(f32x4, x);
+    return __builtin_bit_cast(i32x4, transpose(f, ident_frag<T>()).v);
 }
 
 // one wave's share of a shared operand block: the pieces w, w+NLD, ... of its NI pieces
@@ -151,65 +97,19 @@ template <typename T, int NI, int NLD, int NT = 0> struct Share {
         for (int j = 0; j < CNT; ++j) {
             const int i = min(w + j * NLD, NI - 1);
             const bool tiles = j * NLD < NT;
-            *reinterpret_cast<i32x4*>(slot + piece_off<sizeof(T)>(i, l, tiles)) = tiles ? transpose_piece<T>(a[j]) : a[j];
+            *reinterpret_cast<i32x4*>(slot + piece_off(i, l, tiles)) = tiles ? transpose_piece<T>(a[j]) : a[j];
         }
     }
 };
 
-// A memory wave.  blk(t): block of step t (clamped to the last step by the caller); out(t): copy the outbox of
-// step t to global memory.  Barriers: one closing the prologue, one per step, one handing over the last outbox;
-// the computing waves execute exactly the same sequence.
-template <typename T, int NI, int NM, int DR, int SLOT, int NT, typename BlkFn, typename OutFn>
-__device__ __forceinline__ void memory_wave(char* smem, int nsteps, int hw, BlkFn blk, OutFn out) {
-    static_assert(DR % NSLOT == 0 && DR >= NSLOT, "ring depth must be a multiple of the slot count");
-    Share<T, NI, NM, NT> sh[DR];
-#pragma unroll
-    for (int d = 0; d < DR; ++d) sh[d].load(blk(d), hw);
-    sh[0].to_lds(smem, hw);
-    sh[1].to_lds(smem + SLOT, hw);
-    sh[0].load(blk(DR), hw);
-    sh[1].load(blk(DR + 1), hw);
-    lds_barrier();
-    const int nfull = nsteps / DR;
-#pragma unroll 1
-    for (int gi = 0; gi < nfull; ++gi) {
-#pragma unroll
-        for (int j = 0; j < DR; ++j) {
-            const int t = gi * DR + j;
-            lds_barrier();
-            sh[(j + 2) % DR].to_lds(smem + ((j + 2) % NSLOT) * SLOT, hw);
-            sh[(j + 2) % DR].load(blk(t + 2 + DR), hw);
-            if (t > 0) out(t - 1);
-        }
-    }
-#pragma unroll 1
-    for (int t = nfull * DR; t < nsteps; ++t) {           // fewer than DR steps left: one block at a time
-        lds_barrier();
-        Share<T, NI, NM, NT> tmp;
-        tmp.load(blk(t + 2), hw);
-        if (t > 0) out(t - 1);
-        tmp.to_lds(smem + ((t + 2) % NSLOT) * SLOT, hw);
-    }
-    lds_barrier();
-    out(nsteps - 1);
-}
-
-// LDS of a scan workgroup: the three operand slots, then (with memory waves) two outboxes.  What an outbox holds:
-//   OUT_O      forward pass: the workgroup's 16 x (16 NWC) piece of the output rows, padded by 16 bytes a row
-//              against bank conflicts;
-//   OUT_STATE  forward scan of the backward pass: the workgroup's part of the chunk's state checkpoint,
-//              [K/32][NWC] tile pairs (1 KiB a pair for 2-byte elements).  v_new is not checkpointed: the
-//              chunk_grad kernel rebuilds it from this checkpoint, w and u;
-//   OUT_GRAD   reverse scan: the same for dS, followed by [NWC] tile pairs of dv_new.
-//   OUT_SUM    summary of a time segment: no outbox, the record is written at the end
+// What a scan leaves:
+//   OUT_O      forward pass: the output rows;
+//   OUT_STATE  forward scan of the backward pass: the chunk's state checkpoint, [K/32][V/16] tile pairs.  v_new is not
+//              checkpointed: the chunk_grad kernel rebuilds it from this checkpoint, w and u;
+//   OUT_GRAD   reverse scan: the same for dS, and tile pairs of dv_new;
+//   OUT_SUM    summary of a time segment: the record, written at the end
 enum ScanOut { OUT_O, OUT_STATE, OUT_GRAD, OUT_SUM };
-template <typename T, int K, int V, int NWC, int SLOT_, ScanOut OUT> struct ScanLds {
-    static constexpr int ES = sizeof(T), NM = ScanCfg<T, K, V, NWC>::NM, SLOT = SLOT_;
-    static constexpr int OROW = 16 * NWC * ES + 16;
-    static constexpr int OB_HC = (K / 32) * NWC * PAIR * ES;
-    static constexpr int OB = OUT == OUT_SUM ? 0 : OUT == OUT_O ? CH * OROW : OUT == OUT_STATE ? OB_HC : OB_HC + NWC * PAIR * ES;
-    static constexpr int BYTES = NSLOT * SLOT + (NM ? 2 * OB : 0);
-};
+constexpr int SCAN_TARGET_WORKGROUPS = 256;               // compute units of the device
 
 // ---- time segments -------------------------------------------------------------------------------------------
 // Few (sequence, head) pairs leave most of the device idle while each of them walks its chunks one after the other, at
@@ -259,15 +159,10 @@ template <typename T, int K, int V, int NWC, ScanOut OUT>
 __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem, int n, int seg, int split) {
     constexpr bool WRITE_O = OUT == OUT_O, SUM = OUT == OUT_SUM;
     typedef ScanCfg<T, K, V, NWC> C;
-    constexpr int KT = K / 16, KT2 = KT / 2, VT = V / 16, NM = C::NM, ES = sizeof(T);
+    constexpr int KT = K / 16, KT2 = KT / 2, VT = V / 16;
     constexpr BlkF B = blk_fwd(K, sizeof(T), WRITE_O);
-    constexpr bool PIPE = C::pipelined(WRITE_O), SPREAD = C::SPREAD;
-    constexpr bool PIPE_UPD = PIPE && C::early_update_reads(WRITE_O);
-    constexpr int NIB = B.SIZE / 1024, SLOT = B.SIZE + C::OWN_FWD, NI = SLOT / 1024;
-    constexpr bool OWN_LDS = C::OWN_FWD > 0;
-    typedef ScanLds<T, K, V, NWC, SLOT, OUT> L;
-    constexpr int OROW = L::OROW, OB_HC = L::OB_HC, OB = L::OB;
-    char* const outbox = smem + NSLOT * SLOT;
+    constexpr bool PIPE = C::pipelined(WRITE_O), PIPE_UPD = PIPE && C::early_update_reads();
+    constexpr int SLOT = B.SIZE, NI = SLOT / 1024;
 
     const int h = blockIdx.x;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -291,49 +186,9 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
         const int64_t chw = chw0 + min(c0 + t, last);
         // (the forward pass's blocks are B.SIZE apart; those the backward pass reads may be a forward pass's, further apart)
         const char* b = reinterpret_cast<const char*>(p.ws.W) + chw * (WRITE_O ? B.SIZE : p.ws.sa_stride);
-        if constexpr (OWN_LDS)
-            return BlockFwd<NIB, C::OWN_UT, C::OWN_VTT>{b, reinterpret_cast<const char*>(p.ws.UT + (chw * VT + own0) * PAIR),
-                                                        reinterpret_cast<const char*>(p.ws.VTT + (chw * VT + own0) * TILE)};
-        else
-            return BlockOne{b};
+        return BlockOne{b};
     };
 
-    if (NM && wv >= NWC) {
-        if (nchunks <= 0) return;
-        const int hw = wv - NWC;
-        memory_wave<T, NI, NM ? NM : 1, NM ? C::DR_SHARE : NSLOT, SLOT, 0>(smem, nchunks, hw, blk, [&](int t) __attribute__((always_inline)) {
-            if (SUM) return;
-            const int cid = c0 + t;
-            const char* ob = outbox + (t & 1) * OB;
-            if (WRITE_O) {
-                // rows of o: 16-byte pieces, LPR lanes a row
-                constexpr int LPR = 16 * NWC * ES / 16, RPI = 64 / LPR;
-                const int64_t tok0 = bos + (int64_t)t * CH;
-                const int len = (int)min((int64_t)CH, eos - tok0);
-#pragma unroll
-                for (int r0 = hw * RPI; r0 < CH; r0 += (NM ? NM : 1) * RPI) {
-                    const int r = r0 + l / LPR, e = (l % LPR) * 16;
-                    if (r < len) {                        // also keeps lanes beyond the 16 rows inside the outbox
-                        const i32x4 x = *reinterpret_cast<const i32x4*>(ob + r * OROW + e);
-                        *reinterpret_cast<i32x4*>(reinterpret_cast<char*>(p.o + ((tok0 + r) * H + h) * V + 16 * vt0) + e) = x;
-                    }
-                }
-            } else {
-                char* hc = reinterpret_cast<char*>(p.ws.HC + (chw0 + cid) * (K * V) + vt0 * PAIR);
-                constexpr int NP = OB / 1024;
-#pragma unroll
-                for (int j = 0; j < (NP + (NM ? NM : 1) - 1) / (NM ? NM : 1); ++j) {
-                    const int i = hw + j * (NM ? NM : 1);
-                    if (i < NP)
-                        *reinterpret_cast<i32x4*>(hc + ((i / NWC) * VT + i % NWC) * 1024 + l * 16) =
-                            *reinterpret_cast<const i32x4*>(ob + i * 1024 + l * 16);
-                }
-            }
-        });
-        return;
-    }
-
-    // ---- computing wave
     const int vt = vt0 + wv;
     // state block: lane (g,c) reg i of tile kt = S[16kt + 4g + i][16vt + c]
     f32x4 S[KT];
@@ -348,13 +203,11 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
 #pragma unroll
             for (int i = 0; i < 4; ++i) S[kt][i] = p.h0[soff + (int64_t)(16 * kt + 4 * g + i) * V];
     }
-    struct Own { Frag<T> ut[2], vtt; };                   // the tiles only this wave reads (from LDS where they travel with the block)
+    struct Own { Frag<T> ut[2], vtt; };                   // the tiles only this wave reads
     auto load_own = [&](Own& o, int t) __attribute__((always_inline)) {
-        if constexpr (!OWN_LDS) {
-            const int64_t chw = chw0 + min(c0 + t, last);
-            ld_pair(p.ws.UT + (chw * VT + own0 + wv % VT) * PAIR, o.ut[0], o.ut[1]);
-            o.vtt = ld_tile(p.ws.VTT + (chw * VT + own0 + wv % VT) * TILE);
-        }
+        const int64_t chw = chw0 + min(c0 + t, last);
+        ld_pair(p.ws.UT + (chw * VT + own0 + wv % VT) * PAIR, o.ut[0], o.ut[1]);
+        o.vtt = ld_tile(p.ws.VTT + (chw * VT + own0 + wv % VT) * TILE);
     };
 
     Frag<T> w[2][KT];                                     // phase-1 operands; when pipelined, read a step ahead
@@ -368,17 +221,12 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
         for (int kp = 0; kp < KT2; ++kp) read_w(slot, kp);
     };
 
-    // one chunk: shared operands from `slot`, the phase-1 operands of the next chunk from `slot_next`, results
-    // that go to global memory into the outbox `ob` (when there are memory waves)
-    auto step = [&](const char* slot, const char* slot_next, char* ob, Own own, int t) __attribute__((always_inline)) {
+    // one chunk: shared operands from `slot`, the phase-1 operands of the next chunk from `slot_next`
+    auto step = [&](const char* slot, const char* slot_next, Own own, int t) __attribute__((always_inline)) {
         const int cid = c0 + t;
         const int64_t chw = chw0 + cid;
         const int64_t tok0 = bos + (int64_t)t * CH;
         const int len = (int)min((int64_t)CH, eos - tok0);
-        if constexpr (OWN_LDS) {
-            ld_pair(reinterpret_cast<const T*>(slot + B.SIZE) + wv * PAIR, own.ut[0], own.ut[1]);
-            own.vtt = ld_tile(reinterpret_cast<const T*>(slot + B.SIZE + C::OWN_UT) + wv * TILE);
-        }
         if (SUM && trans) { own.ut[0] = zero_frag<T>(); own.ut[1] = zero_frag<T>(); own.vtt = zero_frag<T>(); }
         const T* sBGT = reinterpret_cast<const T*>(slot + B.BGT);
         const T* sKGT = reinterpret_cast<const T*>(slot + B.KGT);
@@ -396,77 +244,60 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
             egl[2 * kp + 1] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (2 * kp + 1) + 4 * g);
         };
         if (WRITE_O) {
-            if (PIPE && !SPREAD) {
-#pragma unroll
-                for (int kp = 0; kp < KT2; ++kp) read_qg(kp);
-            }
             ld_pair(reinterpret_cast<const T*>(slot + B.AQB), aqb[0], aqb[1]);
             aqk = ld_tile(reinterpret_cast<const T*>(slot + B.AQK));
         }
-        if (PIPE_UPD && !SPREAD) {
-#pragma unroll
-            for (int kp = 0; kp < KT2; ++kp) read_upd(kp);
-        }
-        if (PIPE && !SPREAD) __builtin_amdgcn_sched_barrier(0);   // the reads above stay above the products below
         Frag<T> sb[KT];
         // v_new^T (rows value, inner token) = u^T + S^T w^T; what is read on the way is used a group of products later or after
         f32x4 vn[2] = {to_f32(own.ut[0]), to_f32(own.ut[1])};
 #pragma unroll
         for (int kp = 0; kp < KT2; ++kp) {
-            if (PIPE && SPREAD && WRITE_O) read_qg(kp);
-            if (PIPE_UPD && SPREAD && !WRITE_O) read_upd(kp);
+            if (PIPE && WRITE_O) read_qg(kp);
+            if (PIPE_UPD && !WRITE_O) read_upd(kp);
             if (!PIPE) read_w(slot, kp);
-            if (PIPE && SPREAD) __builtin_amdgcn_sched_barrier(0);
+            if (PIPE) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int kt = 2 * kp; kt < 2 * kp + 2; ++kt) {
                 sb[kt] = to_frag<T>(S[kt]);
                 vn[0] = mm(sb[kt], w[0][kt], vn[0]);
                 vn[1] = mm(sb[kt], w[1][kt], vn[1]);
             }
-            if (PIPE && SPREAD) __builtin_amdgcn_sched_barrier(0);
+            if (PIPE) __builtin_amdgcn_sched_barrier(0);
         }
         f32x4 o = zero4();
         if (WRITE_O) {
             // o (rows token, inner value) = qg S + A_qk v + sum_s A_qb^s v_new_s; the first two terms here
 #pragma unroll
             for (int kp = 0; kp < KT2; ++kp) {
-                if (PIPE_UPD && SPREAD) read_upd(kp);
+                if (PIPE_UPD) read_upd(kp);
                 if (!PIPE) read_qg(kp);
-                if (PIPE && SPREAD) __builtin_amdgcn_sched_barrier(0);
+                if (PIPE) __builtin_amdgcn_sched_barrier(0);
                 o = mm(qg[2 * kp], sb[2 * kp], o);
                 o = mm(qg[2 * kp + 1], sb[2 * kp + 1], o);
-                if (PIPE && SPREAD) __builtin_amdgcn_sched_barrier(0);
+                if (PIPE) __builtin_amdgcn_sched_barrier(0);
             }
             o = mm(aqk, own.vtt, o);
         }
         if (PIPE) __builtin_amdgcn_sched_barrier(0);
-        if (PIPE && !SPREAD) {
-            read_w_all(slot_next);                        // the products above have taken their operands already
-            __builtin_amdgcn_sched_barrier(0);
-        }
         const Frag<T> vnb[2] = {to_frag<T>(vn[0]), to_frag<T>(vn[1])};
         if (OUT == OUT_STATE) {
             // checkpoint of the entering state, as the fragments held here (tile pairs, 16 bytes per lane, whole
             // cache lines): the chunk_grad kernel turns them the way it needs them
-            T* hc = NM ? reinterpret_cast<T*>(ob) + wv * PAIR : p.ws.HC + chw * (K * V) + vt * PAIR;
-            constexpr int HSTR = (NM ? NWC : VT) * PAIR;  // elements between the pairs of consecutive channel tiles
+            T* hc = p.ws.HC + chw * (K * V) + vt * PAIR;
+            constexpr int HSTR = VT * PAIR;               // elements between the pairs of consecutive channel tiles
 #pragma unroll
             for (int kp = 0; kp < KT2; ++kp) st_pair2(hc + kp * HSTR, sb[2 * kp], sb[2 * kp + 1]);
         }
         if (WRITE_O) {
             o = mm(aqb[0], vnb[0], o);
             o = mm(aqb[1], vnb[1], o);
-            if (NM) st_frag(reinterpret_cast<T*>(ob + c * OROW) + 16 * wv + 4 * g, to_frag<T>(o));
-            else if (c < len) st_frag(p.o + ((tok0 + c) * H + h) * V + 16 * vt + 4 * g, to_frag<T>(o));
-            // the output leaves for the outbox before the state update below, not after it: the barrier that ends the step
-            // waits for this LDS write, and behind the update's products the wait is free
-            if (NM && PIPE) __builtin_amdgcn_sched_barrier(0);
+            if (c < len) st_frag(p.o + ((tok0 + c) * H + h) * V + 16 * vt + 4 * g, to_frag<T>(o));
         }
         // S <- exp(g_last) S + kg^T v + sum_s bg_s^T v_new_s
 #pragma unroll
         for (int kp = 0; kp < KT2; ++kp) {
             if (!PIPE_UPD) read_upd(kp);
-            if (PIPE && SPREAD) {                             // (those of phase 1, whose products have taken them already)
+            if (PIPE) {                             // (those of phase 1, whose products have taken them already)
                 read_w(slot_next, kp);
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -478,47 +309,43 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
                 x = mm(vnb[1], bgt[1][kt], x);
                 S[kt] = x;
             }
-            if (PIPE && SPREAD) __builtin_amdgcn_sched_barrier(0);
+            if (PIPE) __builtin_amdgcn_sched_barrier(0);
         }
     };
 
     if (nchunks > 0) {
-        constexpr int DRO = C::DR_OWN, DRS = NM ? 0 : C::DR_SHARE;   // without memory waves both rings are one
+        constexpr int DR = C::DR;
         int done = 0;
-        if constexpr (DRO > 0) {
-            Share<T, NI, NWC> sh[DRS ? DRS : 1];
-            Own own[DRO];
+        if constexpr (DR > 0) {
+            Share<T, NI, NWC> sh[DR];
+            Own own[DR];
 #pragma unroll
-            for (int d = 0; d < DRO; ++d) {
-                if (DRS) sh[DRS ? d : 0].load(blk(d), wv);
+            for (int d = 0; d < DR; ++d) {
+                sh[d].load(blk(d), wv);
                 load_own(own[d], d);
             }
-            if (DRS) {
-                sh[0].to_lds(smem, wv);
-                sh[DRS ? 1 : 0].to_lds(smem + SLOT, wv);
-                sh[0].load(blk(DRS), wv);
-                sh[DRS ? 1 : 0].load(blk(DRS + 1), wv);
-            }
+            sh[0].to_lds(smem, wv);
+            sh[1].to_lds(smem + SLOT, wv);
+            sh[0].load(blk(DR), wv);
+            sh[1].load(blk(DR + 1), wv);
             lds_barrier();
             if (PIPE) read_w_all(smem);
-            const int nfull = nchunks / DRO;
+            const int nfull = nchunks / DR;
 #pragma unroll 1
             for (int gi = 0; gi < nfull; ++gi) {
 #pragma unroll
-                for (int j = 0; j < DRO; ++j) {            // DRO is a multiple of NSLOT: step gi*DRO+j uses slot j % 3
-                    const int t = gi * DRO + j;
+                for (int j = 0; j < DR; ++j) {            // DR is a multiple of NSLOT: step gi*DR+j uses slot j % 3
+                    const int t = gi * DR + j;
                     lds_barrier();
-                    if (DRS) {
-                        sh[DRS ? (j + 2) % DRO : 0].to_lds(smem + ((j + 2) % NSLOT) * SLOT, wv);
-                        sh[DRS ? (j + 2) % DRO : 0].load(blk(t + 2 + DRS), wv);
-                    }
-                    step(smem + (j % NSLOT) * SLOT, smem + ((j + 1) % NSLOT) * SLOT, outbox + (t & 1) * OB, own[j], t);
+                    sh[(j + 2) % DR].to_lds(smem + ((j + 2) % NSLOT) * SLOT, wv);
+                    sh[(j + 2) % DR].load(blk(t + 2 + DR), wv);
+                    step(smem + (j % NSLOT) * SLOT, smem + ((j + 1) % NSLOT) * SLOT, own[j], t);
                     // refilled only after the last use: a register that is loaded while its old value is still
                     // live needs a copy, and the copy would wait for the load just issued
-                    load_own(own[j], t + DRO);
+                    load_own(own[j], t + DR);
                 }
             }
-            done = nfull * DRO;
+            done = nfull * DR;
         } else {
             Share<T, NI, NWC> tmp;
             tmp.load(blk(0), wv);
@@ -536,15 +363,14 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
             for (int t = done; t < nchunks; ++t) {
                 lds_barrier();
                 Share<T, NI, NWC> tmp;
-                if (!NM) tmp.load(blk(t + 2), wv);
+                tmp.load(blk(t + 2), wv);
                 Own nxt;
                 load_own(nxt, t + 1);
-                step(smem + (t % NSLOT) * SLOT, smem + ((t + 1) % NSLOT) * SLOT, outbox + (t & 1) * OB, cur, t);
-                if (!NM) tmp.to_lds(smem + ((t + 2) % NSLOT) * SLOT, wv);
+                step(smem + (t % NSLOT) * SLOT, smem + ((t + 1) % NSLOT) * SLOT, cur, t);
+                tmp.to_lds(smem + ((t + 2) % NSLOT) * SLOT, wv);
                 cur = nxt;
             }
         }
-        if (NM) lds_barrier();                            // hands the last outbox to the memory waves
     }
     if (SUM) {
         store_record<T, K>(S, p.seg.loc, p.seg.tr, rec, V, vt, trans);
@@ -562,17 +388,13 @@ template <typename T, int K, int V, int NWC, ScanOut OUT>
 __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem, int n, int seg, int split) {
     constexpr bool SUM = OUT == OUT_SUM;
     typedef ScanCfg<T, K, V, NWC> C;
-    constexpr int KT = K / 16, KT2 = KT / 2, VT = V / 16, NM = C::NM, ES = sizeof(T);
+    constexpr int KT = K / 16, KT2 = KT / 2, VT = V / 16;
     // LDS slot: [BG | WT] (BGT and W of the forward-scan block, transposed on their way in) | EGL | QGT | AQBT
     constexpr SlotB B = slot_bwd(K, sizeof(T));
     constexpr int SBWD = blk_bwd(K, sizeof(T)).SIZE, NT = B.NIF;
     const int SFWD = p.ws.sa_stride;
-    constexpr bool PIPE = C::pipelined(false), SPREAD = C::SPREAD;
-    constexpr bool PIPE_UPD = PIPE && C::early_update_reads(false);
+    constexpr bool PIPE = C::pipelined(false), PIPE_UPD = PIPE && C::early_update_reads();
     constexpr int NI = B.SIZE / 1024, SLOT = B.SIZE;
-    typedef ScanLds<T, K, V, NWC, SLOT, OUT> L;
-    constexpr int OB_HC = L::OB_HC, OB = L::OB;
-    char* const outbox = smem + NSLOT * SLOT;
 
     const int h = blockIdx.x;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -593,28 +415,6 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
         const int64_t slot = chw0 + max(first - t, c0);
         return BlockTwo<T, K>{reinterpret_cast<const char*>(p.ws.W) + slot * SFWD, reinterpret_cast<const char*>(p.ws.QGT) + slot * SBWD};
     };
-
-    if (NM && wv >= NWC) {
-        if (nchunks <= 0) return;
-        const int hw = wv - NWC;
-        memory_wave<T, NI, NM ? NM : 1, NM ? C::DR_SHARE : NSLOT, SLOT, NT>(smem, nchunks, hw, blk, [&](int t) __attribute__((always_inline)) {
-            if (SUM) return;
-            const int cid = first - t;
-            const char* ob = outbox + (t & 1) * OB;
-            char* hc = reinterpret_cast<char*>(p.ws.DHC + (chw0 + cid) * (K * V) + vt0 * PAIR);
-            char* vn = reinterpret_cast<char*>(p.ws.DVN + (chw0 + cid) * (2 * CH * V) + vt0 * PAIR);
-            constexpr int NP = OB / 1024, NPH = OB_HC / 1024;
-#pragma unroll
-            for (int j = 0; j < (NP + (NM ? NM : 1) - 1) / (NM ? NM : 1); ++j) {
-                const int i = hw + j * (NM ? NM : 1);
-                if (i < NP) {
-                    char* dst = i < NPH ? hc + ((i / NWC) * VT + i % NWC) * 1024 : vn + (i - NPH) * 1024;
-                    *reinterpret_cast<i32x4*>(dst + l * 16) = *reinterpret_cast<const i32x4*>(ob + i * 1024 + l * 16);
-                }
-            }
-        });
-        return;
-    }
 
     const int vt = vt0 + wv;
     f32x4 dS[KT];   // lane (g,c) reg i of tile kt = dS[16kt + 4g + i][16vt + c]
@@ -650,7 +450,7 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
         for (int kp = 0; kp < KT2; ++kp) read_bg(slot, kp);
     };
 
-    auto step = [&](const char* slot, const char* slot_next, char* ob, Frag<T> don, int t) __attribute__((always_inline)) {
+    auto step = [&](const char* slot, const char* slot_next, Frag<T> don, int t) __attribute__((always_inline)) {
         const int cid = first - t;
         const int64_t chw = chw0 + cid;
         const T* sWT = reinterpret_cast<const T*>(slot + B.W);
@@ -665,12 +465,7 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
             egl[2 * kp] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (2 * kp) + 4 * g);
             egl[2 * kp + 1] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (2 * kp + 1) + 4 * g);
         };
-        if (PIPE_UPD && !SPREAD) {
-#pragma unroll
-            for (int kp = 0; kp < KT2; ++kp) read_upd(kp);
-        }
         if (!PIPE) ld_pair(reinterpret_cast<const T*>(slot + B.AQBT), aq[0], aq[1]);
-        else if (!SPREAD) __builtin_amdgcn_sched_barrier(0);
         Frag<T> dsb[KT];
         const int len = (int)min((int64_t)CH, eos - (bos + (int64_t)(cid - c0) * CH));
         if (c >= len || trans) don = zero_frag<T>();
@@ -681,28 +476,23 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
         dvn[1] = mm(doT, aq[1], zero4());
 #pragma unroll
         for (int kp = 0; kp < KT2; ++kp) {
-            if (PIPE_UPD && SPREAD) read_upd(kp);
+            if (PIPE_UPD) read_upd(kp);
             if (!PIPE) read_bg(slot, kp);
-            if (PIPE && SPREAD) __builtin_amdgcn_sched_barrier(0);
+            if (PIPE) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int kt = 2 * kp; kt < 2 * kp + 2; ++kt) {
                 dsb[kt] = to_frag<T>(dS[kt]);
                 dvn[0] = mm(dsb[kt], bg[0][kt], dvn[0]);
                 dvn[1] = mm(dsb[kt], bg[1][kt], dvn[1]);
             }
-            if (PIPE && SPREAD) __builtin_amdgcn_sched_barrier(0);
-        }
-        if (PIPE && !SPREAD) {
-            __builtin_amdgcn_sched_barrier(0);
-            read_p1_all(slot_next);
-            __builtin_amdgcn_sched_barrier(0);
+            if (PIPE) __builtin_amdgcn_sched_barrier(0);
         }
         const Frag<T> dvb[2] = {to_frag<T>(dvn[0]), to_frag<T>(dvn[1])};
         // gradient of the state leaving the chunk and of v_new, as the fragments held here (tile pairs)
         if constexpr (!SUM) {
-        T* dhc = NM ? reinterpret_cast<T*>(ob) + wv * PAIR : p.ws.DHC + chw * (K * V) + vt * PAIR;
-        T* dvp = NM ? reinterpret_cast<T*>(ob + OB_HC) + wv * PAIR : p.ws.DVN + chw * (2 * CH * V) + vt * PAIR;
-        constexpr int HSTR = (NM ? NWC : VT) * PAIR;
+        T* dhc = p.ws.DHC + chw * (K * V) + vt * PAIR;
+        T* dvp = p.ws.DVN + chw * (2 * CH * V) + vt * PAIR;
+        constexpr int HSTR = VT * PAIR;
 #pragma unroll
         for (int kp = 0; kp < KT2; ++kp) st_pair2(dhc + kp * HSTR, dsb[2 * kp], dsb[2 * kp + 1]);
         st_pair2(dvp, dvb[0], dvb[1]);
@@ -711,7 +501,7 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
 #pragma unroll
         for (int kp = 0; kp < KT2; ++kp) {
             if (!PIPE_UPD) read_upd(kp);
-            if (PIPE && SPREAD) {                             // (those of phase 1, whose products have taken them already)
+            if (PIPE) {                             // (those of phase 1, whose products have taken them already)
                 if (kp == 0) ld_pair(reinterpret_cast<const T*>(slot_next + B.AQBT), aq[0], aq[1]);
                 read_bg(slot_next, kp);
                 __builtin_amdgcn_sched_barrier(0);
@@ -724,45 +514,41 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
                 x = mm(dvb[1], wt[1][kt], x);
                 dS[kt] = x;
             }
-            if (PIPE && SPREAD) __builtin_amdgcn_sched_barrier(0);
+            if (PIPE) __builtin_amdgcn_sched_barrier(0);
         }
     };
 
     if (nchunks > 0) {
-        constexpr int DRO = C::DR_OWN, DRS = NM ? 0 : C::DR_SHARE;
+        constexpr int DR = C::DR;
         int done = 0;
-        if constexpr (DRO > 0) {
-            Share<T, NI, NWC, NT> sh[DRS ? DRS : 1];
-            Frag<T> own[DRO];
+        if constexpr (DR > 0) {
+            Share<T, NI, NWC, NT> sh[DR];
+            Frag<T> own[DR];
 #pragma unroll
-            for (int d = 0; d < DRO; ++d) {
-                if (DRS) sh[DRS ? d : 0].load(blk(d), wv);
+            for (int d = 0; d < DR; ++d) {
+                sh[d].load(blk(d), wv);
                 load_own(own[d], d);
             }
-            if (DRS) {
-                sh[0].to_lds(smem, wv);
-                sh[DRS ? 1 : 0].to_lds(smem + SLOT, wv);
-                sh[0].load(blk(DRS), wv);
-                sh[DRS ? 1 : 0].load(blk(DRS + 1), wv);
-            }
+            sh[0].to_lds(smem, wv);
+            sh[1].to_lds(smem + SLOT, wv);
+            sh[0].load(blk(DR), wv);
+            sh[1].load(blk(DR + 1), wv);
             lds_barrier();
             if (PIPE) read_p1_all(smem);
-            const int nfull = nchunks / DRO;
+            const int nfull = nchunks / DR;
 #pragma unroll 1
             for (int gi = 0; gi < nfull; ++gi) {
 #pragma unroll
-                for (int j = 0; j < DRO; ++j) {
-                    const int t = gi * DRO + j;
+                for (int j = 0; j < DR; ++j) {
+                    const int t = gi * DR + j;
                     lds_barrier();
-                    if (DRS) {
-                        sh[DRS ? (j + 2) % DRO : 0].to_lds(smem + ((j + 2) % NSLOT) * SLOT, wv);
-                        sh[DRS ? (j + 2) % DRO : 0].load(blk(t + 2 + DRS), wv);
-                    }
-                    step(smem + (j % NSLOT) * SLOT, smem + ((j + 1) % NSLOT) * SLOT, outbox + (t & 1) * OB, own[j], t);
-                    load_own(own[j], t + DRO);             // after the last use of the old value: no copy, no wait
+                    sh[(j + 2) % DR].to_lds(smem + ((j + 2) % NSLOT) * SLOT, wv);
+                    sh[(j + 2) % DR].load(blk(t + 2 + DR), wv);
+                    step(smem + (j % NSLOT) * SLOT, smem + ((j + 1) % NSLOT) * SLOT, own[j], t);
+                    load_own(own[j], t + DR);             // after the last use of the old value: no copy, no wait
                 }
             }
-            done = nfull * DRO;
+            done = nfull * DR;
         } else {
             Share<T, NI, NWC, NT> tmp;
             tmp.load(blk(0), wv);
@@ -779,15 +565,14 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
             for (int t = done; t < nchunks; ++t) {
                 lds_barrier();
                 Share<T, NI, NWC, NT> tmp;
-                if (!NM) tmp.load(blk(t + 2), wv);
+                tmp.load(blk(t + 2), wv);
                 Frag<T> nxt;
                 load_own(nxt, t + 1);
-                step(smem + (t % NSLOT) * SLOT, smem + ((t + 1) % NSLOT) * SLOT, outbox + (t & 1) * OB, cur, t);
-                if (!NM) tmp.to_lds(smem + ((t + 2) % NSLOT) * SLOT, wv);
+                step(smem + (t % NSLOT) * SLOT, smem + ((t + 1) % NSLOT) * SLOT, cur, t);
+                tmp.to_lds(smem + ((t + 2) % NSLOT) * SLOT, wv);
                 cur = nxt;
             }
         }
-        if (NM) lds_barrier();
     }
     if (SUM) {
         store_record<T, K>(dS, p.seg.rloc, p.seg.rtr, rec, V, vt, trans);
@@ -809,21 +594,21 @@ __device__ __forceinline__ int scan_sequence(const SeqTab& st, int z) { return s
 template <typename T, int K, int V, int NWC, bool WRITE_O>
 __global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_fwd_kernel(ChunkArgs<T> p) {
     constexpr ScanOut OUT = WRITE_O ? OUT_O : OUT_STATE;
-    __shared__ __attribute__((aligned(16))) char smem[ScanLds<T, K, V, NWC, blk_fwd(K, sizeof(T), WRITE_O).SIZE + ScanCfg<T, K, V, NWC>::OWN_FWD, OUT>::BYTES];
+    __shared__ __attribute__((aligned(16))) char smem[NSLOT * blk_fwd(K, sizeof(T), WRITE_O).SIZE];
     const int z = blockIdx.z / p.seg.nseg, seg = blockIdx.z % p.seg.nseg;
     scan_fwd_body<T, K, V, NWC, OUT>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
 }
 template <typename T, int K, int V, int NWC>
 __global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_bwd_kernel(ChunkArgs<T> p) {
-    __shared__ __attribute__((aligned(16))) char smem[ScanLds<T, K, V, NWC, slot_bwd(K, sizeof(T)).SIZE, OUT_GRAD>::BYTES];
+    __shared__ __attribute__((aligned(16))) char smem[NSLOT * slot_bwd(K, sizeof(T)).SIZE];
     const int z = blockIdx.z / p.seg.nseg, seg = blockIdx.z % p.seg.nseg;
     scan_bwd_body<T, K, V, NWC, OUT_GRAD>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
 }
 // Both scans of the backward pass in one launch: they depend on the prep kernel only, not on each other.
 template <typename T, int K, int V, int NWC>
 __global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_pair_kernel(ChunkArgs<T> p) {
-    constexpr int NF = ScanLds<T, K, V, NWC, blk_fwd(K, sizeof(T), false).SIZE + ScanCfg<T, K, V, NWC>::OWN_FWD, OUT_STATE>::BYTES;
-    constexpr int NB = ScanLds<T, K, V, NWC, slot_bwd(K, sizeof(T)).SIZE, OUT_GRAD>::BYTES;
+    constexpr int NF = NSLOT * blk_fwd(K, sizeof(T), false).SIZE;
+    constexpr int NB = NSLOT * slot_bwd(K, sizeof(T)).SIZE;
     constexpr int SPLIT = ScanCfg<T, K, V, NWC>::SPLIT;
     __shared__ __attribute__((aligned(16))) char smem[NF > NB ? NF : NB];
     const int z = blockIdx.z / p.seg.nseg, seg = blockIdx.z % p.seg.nseg;
@@ -835,8 +620,8 @@ __global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_pair_ke
 // last, in reverse those behind the first.
 template <typename T, int K, int V, int NWC, bool BOTH>
 __global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_sum_kernel(ChunkArgs<T> p) {
-    constexpr int NF = ScanLds<T, K, V, NWC, blk_fwd(K, sizeof(T), false).SIZE + ScanCfg<T, K, V, NWC>::OWN_FWD, OUT_SUM>::BYTES;
-    constexpr int NB = ScanLds<T, K, V, NWC, slot_bwd(K, sizeof(T)).SIZE, OUT_SUM>::BYTES;
+    constexpr int NF = NSLOT * blk_fwd(K, sizeof(T), false).SIZE;
+    constexpr int NB = NSLOT * slot_bwd(K, sizeof(T)).SIZE;
     constexpr int SPLIT = ScanCfg<T, K, V, NWC>::SPLIT, COLS = (V + K) / 16 / NWC;
     __shared__ __attribute__((aligned(16))) char smem[BOTH && NB > NF ? NB : NF];
     const int z = blockIdx.z / (p.seg.nseg - 1), seg = blockIdx.z % (p.seg.nseg - 1);
@@ -933,10 +718,7 @@ static hipError_t launch_scan_nwc(const ChunkArgs<T>& a, ScanKind kind, hipStrea
     typedef ScanCfg<T, K, V, NWC> C;
     dim3 grid(a.H, C::SPLIT * (kind == SCAN_PAIR ? 2 : 1), a.st.N * a.seg.nseg), block(C::THREADS);
     switch (kind) {
-        case SCAN_FWD_O:
-            if constexpr (sizeof(T) == 4) hipLaunchKernelGGL((scan_fwd_kernel<T, K, V, NWC, true>), grid, block, 0, stream, a);
-            else return hipErrorInvalidValue;             // scan_out.cuh
-            break;
+        case SCAN_FWD_O: hipLaunchKernelGGL((scan_fwd_kernel<T, K, V, NWC, true>), grid, block, 0, stream, a); break;
         case SCAN_FWD: hipLaunchKernelGGL((scan_fwd_kernel<T, K, V, NWC, false>), grid, block, 0, stream, a); break;
         case SCAN_BWD: hipLaunchKernelGGL((scan_bwd_kernel<T, K, V, NWC>), grid, block, 0, stream, a); break;
         case SCAN_PAIR: hipLaunchKernelGGL((scan_pair_kernel<T, K, V, NWC>), grid, block, 0, stream, a); break;
@@ -944,22 +726,9 @@ static hipError_t launch_scan_nwc(const ChunkArgs<T>& a, ScanKind kind, hipStrea
     return hipGetLastError();
 }
 
-// Workgroups per head: as many as keep the whole launch within the compute units of the device (one workgroup per
-// unit: what a split buys is memory throughput), 2-byte inputs only.
-constexpr int SCAN_TARGET_WORKGROUPS = 256;
 template <typename T, int K, int V>
 hipError_t launch_scan_shape(const ChunkArgs<T>& a, ScanKind kind, hipStream_t stream) {
-    constexpr int VT = V / 16;
-    if constexpr (sizeof(T) == 2) {
-        const int lanes = a.H * a.st.N * a.seg.nseg * (kind == SCAN_PAIR ? 2 : 1);
-        if (lanes * 4 <= SCAN_TARGET_WORKGROUPS) return launch_scan_nwc<T, K, V, VT / 4>(a, kind, stream);
-        // eight computing waves leave no room for memory waves: V = 128 is always split at least in two
-        if (lanes * 2 <= SCAN_TARGET_WORKGROUPS || VT == 8) return launch_scan_nwc<T, K, V, VT / 2>(a, kind, stream);
-        if constexpr (VT == 8) return hipErrorInvalidValue;   // not reached
-        else return launch_scan_nwc<T, K, V, VT>(a, kind, stream);
-    } else {
-        return launch_scan_nwc<T, K, V, VT>(a, kind, stream);
-    }
+    return launch_scan_nwc<T, K, V, V / 16>(a, kind, stream);
 }
 
 template <typename T, int K, int V>
@@ -968,8 +737,7 @@ hipError_t launch_scan_segments_shape(const ChunkArgs<T>& a, bool both, hipStrea
     typedef ScanCfg<T, K, V, NWC> C;
     dim3 grid(a.H, (V + K) / 16 / NWC * (both ? 2 : 1), a.st.N * (a.seg.nseg - 1)), block(C::THREADS);
     if (both) hipLaunchKernelGGL((scan_sum_kernel<T, K, V, NWC, true>), grid, block, 0, stream, a);
-    else if constexpr (sizeof(T) == 4) hipLaunchKernelGGL((scan_sum_kernel<T, K, V, NWC, false>), grid, block, 0, stream, a);
-    else return hipErrorInvalidValue;                     // scan_out.cuh
+    else hipLaunchKernelGGL((scan_sum_kernel<T, K, V, NWC, false>), grid, block, 0, stream, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((scan_chain_kernel<T, K, V>), dim3(a.H, V / 16 * (both ? 2 : 1), a.st.N), dim3(64 * (K / 16)), 0, stream, a);

@@ -1,9 +1,10 @@
 // The forward pass's scan for 2-byte elements: the state recurrence and the output o (HRDPLR/fwd_triton.py:808-1095), and the
-// records of time segments in the forward direction.  (4-byte elements and the scans of the backward pass: scan_impl.cuh.)  Computing
+// records of time segments in the forward direction; without the output, the backward pass's forward scan.  (The reverse one:
+// scan_grad.cuh; 4-byte elements: scan_impl.cuh.)  Computing
 // waves hold a 16-column block of the fp32 state for the whole sequence; those of NWC blocks and NM waves that move data make a workgroup.
 //
 // A sequence is a chain of steps, and up to some 32 heads in flight the time is the number of steps of the longest sequence times
-// the time of one, whatever the traffic (0.69 us at K = V = 128 in the form of scan_impl.cuh, with 4 heads as with 32).  What a step costs
+// the time of one, whatever the traffic (0.69 us at K = V = 128 in the form it had, that of scan_impl.cuh with four more waves that moved data, with 4 heads as with 32).  What a step costs
 // is the instructions of a wave that has its SIMD to itself, some five cycles each, the latencies of the chain through the state (product ->
 // conversion -> product -> exchange -> product), and what waits at its barrier.  So:
 //  * products in twos (mm2), those with one product a sum first, one settle; b^T is stored with the two ranks of a channel tile side by
@@ -25,24 +26,25 @@
 
 namespace hdla {
 
-template <int K, int V, int NWC, bool SUM> struct OutCfg {
+template <int K, int V, int NWC, ScanOut OUT> struct OutCfg {
+    static constexpr bool WITH_O = OUT == OUT_O;
     static constexpr int VT = V / 16, SPLIT = VT / NWC, KT = K / 16;
     static constexpr BlkF B = blk_fwd(K, 2, true);
-    // 1-KiB pieces of a chunk's block that the scan needs (records: without q's and the scores')
-    static constexpr int NI = (SUM ? B.EGL + 1024 : B.SIZE) / 1024, SLOT = NI * 1024;
+    // 1-KiB pieces of a chunk's block that the scan needs (without o: without q's and the scores')
+    static constexpr int NI = (WITH_O ? B.SIZE : B.EGL + 1024) / 1024, SLOT = NI * 1024;
     // computing waves of a column block, each holding KH channel tiles of the state
     static constexpr int PARTS = K / 64, KH = KT / PARTS, NC = NWC * PARTS;
-    static constexpr int NL = 2, NM = NL + 2;             // waves that load, with the one that forms u and the one that copies the output out
+    static constexpr int NL = 2, NM = NL + 1 + WITH_O;    // waves that load, with the one that forms u and the one that copies the output out
     static constexpr int CNT = (NI + NL - 1) / NL;        // loads of a wave per chunk (the last pieces may be fetched twice)
     static constexpr int THREADS = 64 * (NC + NM);
-    static constexpr int OROW = 16 * NWC * 2 + 16, OB = SUM ? 0 : CH * OROW;   // output rows of a step, padded; two of them
+    static constexpr int OROW = 16 * NWC * 2 + 16, OB = WITH_O ? CH * OROW : 0;   // output rows of a step, padded; two of them
     static constexpr int UB = NWC * 1536;                 // u^T (a pair) and v^T (a tile) of the column blocks; two chunks' of them
     // what the waves of a column block hand each other: two tiles each, and from the second one its part of the output; two steps' of it
-    static constexpr int XP = (SUM ? 4 : 5) * 1024, XB = PARTS > 1 ? NWC * XP : 0;
+    static constexpr int XP = (WITH_O ? 5 : 4) * 1024, XB = PARTS > 1 ? NWC * XP : 0;
     static constexpr int REST = 2 * (OB + UB + XB);
     // as many slots as LDS holds, or as half of it does where that is enough (two workgroups on a compute unit)
     static constexpr int ROOM = (4 * SLOT + REST <= 80 * 1024 ? 80 : 160) * 1024 - REST;
-    static constexpr int SLOTS = ROOM / SLOT < 8 ? ROOM / SLOT : 8;
+    static constexpr int MOST = 62 / CNT + 1 < 8 ? 62 / CNT + 1 : 8, SLOTS = ROOM / SLOT < MOST ? ROOM / SLOT : MOST;
     static_assert(SLOTS >= 3 && (SLOTS - 1) * CNT < 63, "a chunk to read, the next one, and one on its way; the memory counter's range");
     static constexpr int OUTBOX = SLOTS * SLOT, UBUF = OUTBOX + 2 * OB, XBUF = UBUF + 2 * UB, BYTES = XBUF + 2 * XB;
 };
@@ -54,12 +56,15 @@ template <int N> __device__ __forceinline__ void wait_loads() {
     asm volatile("" ::: "memory");
 }
 
-// KEPT: on a workspace that the backward pass will read (PREP_KEEP): u and v^T are there, and b^T's pairs are of two channel tiles, as the
-// scans of the backward pass take them.  The same products in the same order: the same bits.
-template <int K, int V, int NWC, bool SUM, bool KEPT>
+// OUT_O: with the output; OUT_STATE: the forward scan of the backward pass, which leaves the state that enters each chunk; OUT_SUM:
+// records of segments.
+// KEPT: on a workspace of the backward pass (or that it will read, PREP_KEEP): u and v^T are there, and b^T's pairs are of two channel
+// tiles, as the reverse scan takes them.  The same products in the same order: the same bits.
+template <int K, int V, int NWC, ScanOut OUT, bool KEPT>
 __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* smem, int n, int seg, int split) {
-    typedef OutCfg<K, V, NWC, SUM> C;
+    typedef OutCfg<K, V, NWC, OUT> C;
     typedef bf16 T;
+    constexpr bool WITH_O = OUT == OUT_O, SUM = OUT == OUT_SUM;
     constexpr int KT = C::KT, KT2 = KT / 2, SLOTS = C::SLOTS, SLOT = C::SLOT, PARTS = C::PARTS, KH = C::KH, KH2 = KH / 2;
     constexpr BlkF B = C::B;
     const int h = blockIdx.x;
@@ -84,11 +89,12 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
         if (nchunks <= 0) return;
         const int hw = wv - C::NC;
         if (hw < C::NL) {
-            const char* const blk = reinterpret_cast<const char*>(p.ws.W) + chw0 * B.SIZE + l * 16;
+            const int stride = KEPT ? p.ws.sa_stride : B.SIZE;
+            const char* const blk = reinterpret_cast<const char*>(p.ws.W) + chw0 * stride + l * 16;
             int slot = 0;
             auto load = [&](int t) __attribute__((always_inline)) {
                 // past the end: the last chunk again, never looked at
-                const char* const bt = blk + (int64_t)min(t, last) * B.SIZE;
+                const char* const bt = blk + (int64_t)min(t, last) * stride;
 #pragma unroll
                 for (int j = 0; j < C::CNT; ++j) {
                     const int i = min(hw + j * C::NL, C::NI - 1);
@@ -106,7 +112,7 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
                 __builtin_amdgcn_s_barrier();
                 load(t + SLOTS);                          // where chunk t was
             }
-            if (!SUM) __builtin_amdgcn_s_barrier();
+            if (WITH_O) __builtin_amdgcn_s_barrier();
             wait_loads<0>();                              // nothing may arrive in LDS that is no longer this workgroup's
         } else if (hw == C::NL) {
             // v^T and u = Tm (A_ak v) of the workgroup's column blocks, a chunk ahead, with the roundings of the kernel that prepared the
@@ -122,8 +128,9 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
                 if constexpr (KEPT) {
 #pragma unroll
                     for (int j = 0; j < NWC; ++j) {
-                        o.ut[j] = *reinterpret_cast<const i32x4*>(p.ws.UT + ((chw0 + t) * (V / 16) + vt0 + j) * PAIR + 8 * l);
-                        o.v[j] = ld_tile(p.ws.VTT + ((chw0 + t) * (V / 16) + vt0 + j) * TILE);
+                        const int64_t at = (chw0 + t) * (V / 16) + (trans ? 0 : vt0 + j);
+                        o.ut[j] = *reinterpret_cast<const i32x4*>(p.ws.UT + at * PAIR + 8 * l);
+                        o.v[j] = ld_tile(p.ws.VTT + at * TILE);
                     }
                     return o;
                 }
@@ -145,8 +152,8 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
                 if constexpr (KEPT) {
 #pragma unroll
                     for (int j = 0; j < NWC; ++j) {
-                        *reinterpret_cast<i32x4*>(ub + j * (3 * TILE) + 8 * l) = o.ut[j];
-                        st_tile(ub + j * (3 * TILE) + PAIR, o.v[j]);
+                        *reinterpret_cast<i32x4*>(ub + j * (3 * TILE) + 8 * l) = trans ? i32x4{0, 0, 0, 0} : o.ut[j];
+                        st_tile(ub + j * (3 * TILE) + PAIR, trans ? zero_frag<T>() : o.v[j]);
                     }
                     return;
                 }
@@ -188,13 +195,12 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
 #pragma unroll
             for (int j = 0; j < UD - 1; ++j)
                 if (t0 + j < nchunks) step(t0 + j, own[(j + 1) % UD]);
-            if (!SUM) lds_barrier();
-        } else {
+            if (WITH_O) lds_barrier();
+        } else if constexpr (WITH_O) {
             __builtin_amdgcn_s_barrier();
             for (int t = 0; t <= nchunks; ++t) {
-                if (t == nchunks && SUM) break;
                 lds_barrier();
-                if (SUM || t == 0) continue;
+                if (t == 0) continue;
                 // rows of o: 16-byte pieces, LPR lanes a row
                 constexpr int LPR = 2 * NWC, RPI = 64 / LPR;
                 const int64_t tok0 = bos + (int64_t)(t - 1) * CH;
@@ -238,7 +244,7 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
         constexpr int part = decltype(part_)::value, kt0 = part * KH;
         constexpr bool first = part == 0, from_u = part == PARTS - 1;   // the wave with the output, and the one that starts v_new from u
         // A chunk's operands, read as soon as the chunk before has been through with their registers: half a step and more before they are used
-        Frag<T> w[2][KH], qg[SUM ? 1 : KH], kgt[KH], bgt[2][KH], aqk, aqb[2], ut[2], vtt;
+        Frag<T> w[2][KH], qg[WITH_O ? KH : 1], kgt[KH], bgt[2][KH], aqk, aqb[2], ut[2], vtt;
         f32x4 egl[KH];
         // (the lane's offset is all of an address that the wave holds in vector registers: the rest is the slot's and immediate)
         const uint32_t lo = 16 * l, ge = 16 * g;
@@ -260,23 +266,24 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
             }
 #pragma unroll
             for (int kp = 0; kp < KH2; ++kp) {
-                if constexpr (!SUM) pair_at(so, B.QG + (part * KH2 + kp) * 1024, qg[2 * kp], qg[2 * kp + 1]);
+                if constexpr (WITH_O) pair_at(so, B.QG + (part * KH2 + kp) * 1024, qg[2 * kp], qg[2 * kp + 1]);
                 pair_at(so, B.KGT + (part * KH2 + kp) * 1024, kgt[2 * kp], kgt[2 * kp + 1]);
             }
 #pragma unroll
             for (int k = 0; k < KH; ++k) egl[k] = *reinterpret_cast<const f32x4*>(smem + so + ge + B.EGL + 64 * (kt0 + k));
-            if constexpr (!SUM && first) aqk.v = *reinterpret_cast<const s16x4*>(smem + so + lo / 2 + B.AQK);
+            if constexpr (WITH_O && first) aqk.v = *reinterpret_cast<const s16x4*>(smem + so + lo / 2 + B.AQK);
         };
         auto read_rest = [&](uint32_t so) __attribute__((always_inline)) {
 #pragma unroll
             for (int k = 0; k < KH; ++k) {
                 if constexpr (!KEPT) pair_at(so, B.BGT + (kt0 + k) * 1024, bgt[0][k], bgt[1][k]);
-                else if (k % 2 == 0) {
-                    pair_at(so, B.BGT + (kt0 + k) * 512, bgt[0][k], bgt[0][k + 1]);
-                    pair_at(so, B.BGT + (KT + kt0 + k) * 512, bgt[1][k], bgt[1][k + 1]);
+                else {                                    // half a pair each, into the place that the product wants it in
+                    const int at = B.BGT + (kt0 + k) / 2 * 1024 + (k & 1) * 8;
+                    bgt[0][k].v = *reinterpret_cast<const s16x4*>(smem + so + lo + at);
+                    bgt[1][k].v = *reinterpret_cast<const s16x4*>(smem + so + lo + at + KT2 * 1024);
                 }
             }
-            if constexpr (!SUM && first) pair_at(so, B.AQB, aqb[0], aqb[1]);
+            if constexpr (WITH_O && first) pair_at(so, B.AQB, aqb[0], aqb[1]);
         };
         // the column block's area: the parts of the first wave, then those of the second
         char* const xcol = smem + C::XBUF + col * C::XP + l * 16;
@@ -300,20 +307,27 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
                 vn[0] = mm2(sb[2 * kp], sb[2 * kp + 1], w[0][2 * kp], w[0][2 * kp + 1], vn[0]);
                 vn[1] = mm2(sb[2 * kp], sb[2 * kp + 1], w[1][2 * kp], w[1][2 * kp + 1], vn[1]);
             }
-            if constexpr (!SUM) {
+            if constexpr (WITH_O) {
 #pragma unroll
                 for (int kp = 0; kp < KH2; ++kp) o = mm2(qg[2 * kp], qg[2 * kp + 1], sb[2 * kp], sb[2 * kp + 1], o);
+            }
+            if constexpr (OUT == OUT_STATE) {
+                // checkpoint of the entering state, as the fragments held here (tile pairs, 16 bytes per lane, whole cache lines): the
+                // chunk_grad kernel turns them the way it needs them
+                T* const hc = p.ws.HC + (chw0 + t) * (K * V) + (part * KH2 * (V / 16) + vt) * PAIR;
+#pragma unroll
+                for (int kp = 0; kp < KH2; ++kp) st_pair2(hc + kp * (V / 16) * PAIR, sb[2 * kp], sb[2 * kp + 1]);
             }
             // ---- what is one product a sum: the chunk's own part of the state, A_qk v
             f32x4 x[KH + 1];
 #pragma unroll
             for (int k = 0; k < KH; ++k) x[k] = mm(vtt, kgt[k], S[k] * egl[k]);
             x[KH] = zero4();
-            if constexpr (!SUM && first) x[KH] = mm(aqk, vtt, x[KH]);
+            if constexpr (WITH_O && first) x[KH] = mm(aqk, vtt, x[KH]);
             if constexpr (PARTS > 1) {
                 *reinterpret_cast<f32x4*>(xt + part * 2048) = vn[0];
                 *reinterpret_cast<f32x4*>(xt + part * 2048 + 1024) = vn[1];
-                if constexpr (!SUM && !first) *reinterpret_cast<f32x4*>(xt + 4096) = o;
+                if constexpr (WITH_O && !first) *reinterpret_cast<f32x4*>(xt + 4096) = o;
             }
             // the parts are there; so are chunk t + 1 and its u, and chunk t has been read by all
             lds_barrier();
@@ -321,7 +335,7 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
             if constexpr (PARTS > 1) {
                 ov[0] = *reinterpret_cast<const f32x4*>(xt + (1 - part) * 2048);
                 ov[1] = *reinterpret_cast<const f32x4*>(xt + (1 - part) * 2048 + 1024);
-                if constexpr (!SUM && first) oo = *reinterpret_cast<const f32x4*>(xt + 4096);
+                if constexpr (WITH_O && first) oo = *reinterpret_cast<const f32x4*>(xt + 4096);
             }
             __builtin_amdgcn_sched_barrier(0);            // (before the reads of the next chunk: they are what is waited for)
             read_u(t + 1);
@@ -336,16 +350,16 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
             // ---- S <- exp(g_last) S + kg^T v + sum_s bg_s^T v_new_s
 #pragma unroll
             for (int k = 0; k < KH; ++k) S[k] = mm2(vnb[0], vnb[1], bgt[0][k], bgt[1][k], x[k]);
-            if constexpr (!SUM && first) {
+            if constexpr (WITH_O && first) {
                 // o (rows token, inner value) = A_qk v + qg S + sum_s A_qb^s v_new_s
                 if constexpr (PARTS > 1) o += oo;
                 o = mm2(aqb[0], aqb[1], vnb[0], vnb[1], o + x[KH]);
             }
             __builtin_amdgcn_sched_barrier(0);
             read_rest(so);
-            if constexpr (!SUM && first) st_frag(reinterpret_cast<T*>(smem + C::OUTBOX + (t & 1) * C::OB + c * C::OROW) + 16 * col + 4 * g, to_frag<T>(o));
+            if constexpr (WITH_O && first) st_frag(reinterpret_cast<T*>(smem + C::OUTBOX + (t & 1) * C::OB + c * C::OROW) + 16 * col + 4 * g, to_frag<T>(o));
         }
-        if (!SUM) lds_barrier();                          // hands over the last output
+        if (WITH_O) lds_barrier();                          // hands over the last output
     };
     if (nchunks > 0) {
         if (PARTS == 1 || part == 0) walk(std::integral_constant<int, 0>());
@@ -376,22 +390,22 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
 
 // grid = (H, SPLIT, N * segments), as the other scans' (scan_impl.cuh)
 template <int K, int V, int NWC, bool KEPT>
-__global__ __launch_bounds__((OutCfg<K, V, NWC, false>::THREADS)) void scan_out_kernel(ChunkArgs<bf16> p) {
-    __shared__ __attribute__((aligned(16))) char smem[OutCfg<K, V, NWC, false>::BYTES];
+__global__ __launch_bounds__((OutCfg<K, V, NWC, OUT_O>::THREADS)) void scan_out_kernel(ChunkArgs<bf16> p) {
+    __shared__ __attribute__((aligned(16))) char smem[OutCfg<K, V, NWC, OUT_O>::BYTES];
     const int z = blockIdx.z / p.seg.nseg, seg = blockIdx.z % p.seg.nseg;
-    scan_out_body<K, V, NWC, false, KEPT>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
+    scan_out_body<K, V, NWC, OUT_O, KEPT>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
 }
 // the segments' records in the forward direction: grid = (H, (V + K) / 16 / NWC, N * (segments - 1))
 template <int K, int V, int NWC>
-__global__ __launch_bounds__((OutCfg<K, V, NWC, true>::THREADS)) void scan_out_sum_kernel(ChunkArgs<bf16> p) {
-    __shared__ __attribute__((aligned(16))) char smem[OutCfg<K, V, NWC, true>::BYTES];
+__global__ __launch_bounds__((OutCfg<K, V, NWC, OUT_SUM>::THREADS)) void scan_out_sum_kernel(ChunkArgs<bf16> p) {
+    __shared__ __attribute__((aligned(16))) char smem[OutCfg<K, V, NWC, OUT_SUM>::BYTES];
     const int z = blockIdx.z / (p.seg.nseg - 1), seg = blockIdx.z % (p.seg.nseg - 1);
-    if (seg == 0 && (int)blockIdx.y >= OutCfg<K, V, NWC, true>::SPLIT) return;   // starts from h0: nobody asks for its transition
-    scan_out_body<K, V, NWC, true, false>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
+    if (seg == 0 && (int)blockIdx.y >= OutCfg<K, V, NWC, OUT_SUM>::SPLIT) return;   // starts from h0: nobody asks for its transition
+    scan_out_body<K, V, NWC, OUT_SUM, false>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
 }
 
 template <int K, int V, int NWC> static hipError_t launch_scan_out_nwc(const ChunkArgs<bf16>& a, bool kept, hipStream_t stream) {
-    typedef OutCfg<K, V, NWC, false> C;
+    typedef OutCfg<K, V, NWC, OUT_O> C;
     const dim3 grid(a.H, C::SPLIT, a.st.N * a.seg.nseg), block(C::THREADS);
     if (kept) hipLaunchKernelGGL((scan_out_kernel<K, V, NWC, true>), grid, block, 0, stream, a);
     else hipLaunchKernelGGL((scan_out_kernel<K, V, NWC, false>), grid, block, 0, stream, a);
@@ -410,7 +424,7 @@ template <int K, int V> hipError_t launch_scan_out_shape(const ChunkArgs<bf16>& 
 // the segments' records, chained into what enters the segments
 template <int K, int V> hipError_t launch_scan_out_segments_shape(const ChunkArgs<bf16>& a, hipStream_t stream) {
     constexpr int NWC = 4;
-    typedef OutCfg<K, V, NWC, true> C;
+    typedef OutCfg<K, V, NWC, OUT_SUM> C;
     hipLaunchKernelGGL((scan_out_sum_kernel<K, V, NWC>), dim3(a.H, (V + K) / 16 / NWC, a.st.N * (a.seg.nseg - 1)), dim3(C::THREADS), 0, stream, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
