@@ -5,14 +5,14 @@
 // or 128 is bound by what it writes (M x d, three times).  As two BLAS calls and an elementwise kernel it took
 // 14.6 + 9.1 + 10.1 us at M = 8192, d = 1024, and in a decode step three launches of 4.5 us and 40 us of host time.
 // layer_down: their input gradients, dx0 [M, D] = dY [M, d] W [d, D], with dY = dlog_f sigmoid(-f) formed on the way in for
-// the first (before: 12 + 12 us and a pass of its own for dY, 10.7 us).
+// the first (as BLAS calls 12 + 12 us and a pass of its own for dY, 10.7 us).
 // rows_gemm: y [M, N] = x [M, K] W [N, K]^T for at most 64 rows, i.e. the large projections of a decode step: a stream of W,
 // all of the chip's workgroups on it, where the BLAS call costs 20 us of host time and 6 to 13 us (16 x 6416 x 2048; here 5 to 9).
 //
 // bf16 in and out, fp32 accumulation.  Operands are read 16 bytes a lane; the eight elements are two fragments whose inner
-// index is permuted the same way on both sides (elements 8j..8j+3 and 8j+4..8j+7, see ld_two_tiles in skinny.hip), which a
+// index is permuted the same way on both sides (elements 8j..8j+3 and 8j+4..8j+7), which a
 // sum over that index does not notice.
-#include "hdla_common.cuh"
+#include "row_tile.cuh"
 #include "../../include/hdla_hip.h"
 
 namespace hdla {
@@ -26,9 +26,8 @@ __device__ __forceinline__ TwoTiles ld16(const bf16* p) {
     return t;
 }
 // column 8g + i (tile a) and 8g + 4 + i (tile b) of a 32-column block, row c: eight consecutive elements of a row
-__device__ __forceinline__ void st16(bf16* p, f32x4 a, f32x4 b) {
-    const Frag<bf16> fa = to_frag<bf16>(a), fb = to_frag<bf16>(b);
-    *reinterpret_cast<s16x8*>(p) = __builtin_shufflevector(fa.v, fb.v, 0, 1, 2, 3, 4, 5, 6, 7);
+__device__ __forceinline__ s16x8 pack16(f32x4 a, f32x4 b) {
+    return __builtin_shufflevector(to_frag<bf16>(a).v, to_frag<bf16>(b).v, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 // row of a 32-row block that lane c of a fragment holds, for tile a (+ 4 for tile b)
 __device__ __forceinline__ int row8(int c) { return 8 * (c >> 2) + (c & 3); }
@@ -45,56 +44,89 @@ struct UpArgs {
     long long ldx;
     int M, d;
 };
-// A wave per 16 MT rows and 32 NB columns; blockIdx.y: decay or gate.  Every wave reads its 64 rows of W (8 or 16 KiB) from L2:
-// with one row tile a wave that was 134 MB next to 50 MB of results, 28 us (8192 x 1024), with four 21.
+// A wave per 16 MT rows and 32 NB columns; blockIdx.y: decay or gate.  Every wave reads its rows of W (8 or 16 KiB) from L2:
+// with one row tile a wave that was 134 MB next to 50 MB of results, 28 us (8192 x 1024), with four 21.  x0, W and (NB = 2) the results
+// change lanes in LDS (row_tile.cuh), one after the other in the same place: 21 -> 16.
 template <int D, int MT, int NB>
 __global__ __launch_bounds__(256) void layer_up_kernel(UpArgs p) {
     constexpr int KB = D / 32;
+    typedef RowTile<D> TI;
+    typedef RowTile<64> TO;
+    constexpr int XR = 16 * MT / TI::RPR, WR = 32 * NB / TI::RPR, BYTES = (MT > 2 * NB ? 16 * MT : 32 * NB) * TI::ROW;
+    static_assert(BYTES >= 16 * TO::ROW, "a row tile's results fit as well");
+    __shared__ __attribute__((aligned(16))) char sm[4 * BYTES];
     const int l = lane_id(), g = l >> 4, c = l & 15, which = blockIdx.y;
-    const long long unit = (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const long long unit = (long long)blockIdx.x * (blockDim.x >> 6) + wv;
     const int cbs = p.d / (32 * NB);
     const long long r0 = unit / cbs * (16 * MT);
     const int n0 = (int)(unit % cbs) * (32 * NB);
     if (r0 >= p.M) return;
-    const bf16* w = p.w[which] + (long long)(n0 + row8(c)) * D + 8 * g;
+    char* const tile = sm + wv * BYTES;
+    s16x8 x[XR], w[WR];
+#pragma unroll
+    for (int j = 0; j < XR; ++j) x[j] = *reinterpret_cast<const s16x8*>(p.x0[which] + min(r0 + TI::row(j, l), (long long)p.M - 1) * p.ldx + TI::col(l));
+#pragma unroll
+    for (int j = 0; j < WR; ++j) w[j] = *reinterpret_cast<const s16x8*>(p.w[which] + (long long)(n0 + TI::row(j, l)) * D + TI::col(l));
     TwoTiles xf[MT][KB], wf[NB][2][KB];
+#pragma unroll
+    for (int j = 0; j < XR; ++j) TI::put(tile, j, l, x[j]);
+    wave_lds_fence();
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int k = 0; k < KB; ++k) xf[m][k] = ld16(p.x0[which] + min(r0 + 16 * m + c, (long long)p.M - 1) * p.ldx + 8 * g + 32 * k);
+        for (int k = 0; k < KB; ++k) TI::rows(tile, 16 * m + c, k, l, xf[m][k].a, xf[m][k].b);
+    wave_lds_fence();
+#pragma unroll
+    for (int j = 0; j < WR; ++j) TI::put(tile, j, l, w[j]);
+    wave_lds_fence();
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int k = 0; k < KB; ++k) wf[b][h][k] = ld16(w + (32 * b + 4 * h) * D + 32 * k);
+            for (int k = 0; k < KB; ++k) TI::rows(tile, 32 * b + row8(c) + 4 * h, k, l, wf[b][h][k].a, wf[b][h][k].b);
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int m = 0; m < MT; ++m) {
+        const long long m0 = r0 + 16 * m;
+        f32x4 acc[NB][2];
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            f32x4 acc[2] = {zero4(), zero4()};
+        for (int b = 0; b < NB; ++b)
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
+            for (int h = 0; h < 2; ++h) {
+                acc[b][h] = zero4();
 #pragma unroll
-                for (int k = 0; k < KB; ++k) {
-                    acc[h] = mm(xf[m][k].a, wf[b][h][k].a, acc[h]);
-                    acc[h] = mm(xf[m][k].b, wf[b][h][k].b, acc[h]);
-                }
-            if (r0 + 16 * m + c >= p.M) continue;
-            const long long out = (r0 + 16 * m + c) * p.d + n0 + 8 * g + 32 * b;
-            if (which == 1) {
-                st16(p.gate + out, acc[0], acc[1]);
-            } else {
-                if (p.f) st16(p.f + out, acc[0], acc[1]);
+                for (int k = 0; k < KB; ++k) acc[b][h] = mm2(xf[m][k].a, xf[m][k].b, wf[b][h][k].a, wf[b][h][k].b, acc[b][h]);
+            }
+        // lane (g, c): row c, columns 32 b + 8 g + 0..7
+        auto store = [&](bf16* out) __attribute__((always_inline)) {
+            if constexpr (NB == 2) {
+                wave_lds_fence();
+#pragma unroll
+                for (int b = 0; b < NB; ++b) *reinterpret_cast<s16x8*>(tile + TO::place(c, 4 * b + g)) = pack16(acc[b][0], acc[b][1]);
+                wave_lds_fence();
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    if (m0 + TO::row(j, l) < p.M) *reinterpret_cast<s16x8*>(out + (m0 + TO::row(j, l)) * p.d + n0 + TO::col(l)) = TO::get(tile, j, l);
+            } else if (m0 + c < p.M) {
+                *reinterpret_cast<s16x8*>(out + (m0 + c) * p.d + n0 + 8 * g) = pack16(acc[0][0], acc[0][1]);
+            }
+        };
+        if (which == 1) {
+            store(p.gate);
+        } else {
+            if (p.f) store(p.f);
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    const f32x4 r = to_f32(to_frag<bf16>(acc[h]));         // f as the stored tensor has it
+                    const f32x4 r = to_f32(to_frag<bf16>(acc[b][h]));      // f as the stored tensor has it
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) acc[h][i] = logsig(r[i]);
+                    for (int i = 0; i < 4; ++i) acc[b][h][i] = logsig(r[i]);
                 }
-                st16(p.log_f + out, acc[0], acc[1]);
-            }
+            store(p.log_f);
         }
+    }
 }
 
 struct DownArgs {
@@ -103,77 +135,84 @@ struct DownArgs {
     long long ldx;
     int M, d;
 };
-// A workgroup per 16 MT rows; its four waves share out the columns of dY and add up through LDS; blockIdx.y: decay or gate.
-// W has the contraction index outermost: its tiles are turned by a product with the identity, once for MT row tiles.
+// A workgroup per 16 MT rows; its four waves share out the columns of dY, 64 (a cache line of each row) at a time, and add up through
+// LDS; blockIdx.y: decay or gate.  W has the contraction index outermost: its rows go to LDS as they come and the transposing LDS read
+// takes its tiles from there; dY changes lanes in LDS as well (row_tile.cuh).  8192 x 1024, D = 64: lanes of a request in fragment order
+// and products with the identity for W's tiles 18.3 us, this 16.3.
 template <int D, int MT>
 __global__ __launch_bounds__(256) void layer_down_kernel(DownArgs p) {
-    constexpr int DB = D / 32;
-    __shared__ f32x4 red[3][MT * 2 * DB][64];
-    const int wv = threadIdx.x >> 6, l = lane_id(), g = l >> 4, c = l & 15, which = blockIdx.y;
+    constexpr int NT = D / 16;
+    typedef RowTile<64> TY;
+    typedef RowTile<D> TW;
+    constexpr int YR = 16 * MT / TY::RPR, WR = 64 / TW::RPR, BYTES = 16 * MT * TY::ROW + 64 * TW::ROW;
+    static_assert(BYTES >= MT * NT * 1024, "a wave's sums fit where its tiles were");
+    __shared__ __attribute__((aligned(16))) char sm[4 * BYTES];
+    const int l = lane_id(), g = l >> 4, c = l & 15, which = blockIdx.y;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const long long r0 = (long long)blockIdx.x * (16 * MT);
-    const Frag<bf16> id = ident_frag<bf16>();
-    f32x4 acc[MT][2 * DB];
+    char* const ty = sm + wv * BYTES;
+    char* const tw = ty + 16 * MT * TY::ROW;
+    f32x4 acc[MT][NT];
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int b = 0; b < 2 * DB; ++b) acc[m][b] = zero4();
-    const bf16* dy[MT];
-    const bf16* fr[MT];
+        for (int b = 0; b < NT; ++b) acc[m][b] = zero4();
+    struct In { s16x8 y[YR], f[YR], w[WR]; };
+    long long yo[YR];                                     // rows past the end: the last one again, computed and not stored
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        const long long row = min(r0 + 16 * m + c, (long long)p.M - 1);   // rows past the end: computed, not stored
-        dy[m] = p.dy[which] + row * p.d + 8 * g;
-        fr[m] = p.f + row * p.d + 8 * g;
-    }
-#pragma unroll 2
-    for (int n0 = 32 * wv; n0 < p.d; n0 += 128) {
-        TwoTiles y[MT], ff[MT], wt[2][DB];
+    for (int j = 0; j < YR; ++j) yo[j] = min(r0 + TY::row(j, l), (long long)p.M - 1) * p.d + TY::col(l);
+    auto request = [&](int n0) __attribute__((always_inline)) {
+        In in;
+        const bf16 *const y0 = p.dy[which] + n0, *const f0 = p.f + n0, *const w0 = p.w[which] + (long long)n0 * D;
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            y[m] = ld16(dy[m] + n0);
-            if (which == 0) ff[m] = ld16(fr[m] + n0);
+        for (int j = 0; j < YR; ++j) {
+            in.y[j] = *reinterpret_cast<const s16x8*>(y0 + yo[j]);
+            if (which == 0) in.f[j] = *reinterpret_cast<const s16x8*>(f0 + yo[j]);
         }
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int b = 0; b < DB; ++b) wt[h][b] = ld16(p.w[which] + (long long)(n0 + row8(c) + 4 * h) * D + 32 * b + 8 * g);
+        for (int j = 0; j < WR; ++j) in.w[j] = *reinterpret_cast<const s16x8*>(w0 + TW::row(j, l) * D + TW::col(l));
+        return in;
+    };
+    // the next columns on their way while some are worked on (D = 64: the other's registers are all taken)
+    constexpr bool AHEAD = D == 64;
+    int n0 = 64 * wv;
+    In next;
+    if (AHEAD && n0 < p.d) next = request(n0);
+    for (; n0 < p.d; n0 += 256) {
+        In in;
+        if constexpr (AHEAD) in = next;
+        else in = request(n0);
+        if (AHEAD && n0 + 256 < p.d) next = request(n0 + 256);
         if (which == 0) {
 #pragma unroll
-            for (int m = 0; m < MT; ++m) {
-                // df = dlog_f sigmoid(-f), rounded as the stored gradient would be
-                auto one = [](Frag<bf16>& d, Frag<bf16> f) __attribute__((always_inline)) {
-                    f32x4 x = to_f32(d);
-                    const f32x4 z = to_f32(f);
-                    float e[4], s[4];
+            for (int j = 0; j < YR; ++j) in.y[j] = times_sigmoid_neg(in.y[j], in.f[j]);
+        }
+        wave_lds_fence();                                 // (the reads of the columns before)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) e[i] = __expf(z[i]);
-                    sigmoid_of_exp<4>(e, s);
+        for (int j = 0; j < YR; ++j) TY::put(ty, j, l, in.y[j]);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) x[i] *= s[i];
-                    d = to_frag<bf16>(x);
-                };
-                one(y[m].a, ff[m].a);
-                one(y[m].b, ff[m].b);
+        for (int j = 0; j < WR; ++j) TW::put(tw, j, l, in.w[j]);
+        wave_lds_fence();
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            TwoTiles y[MT];
+#pragma unroll
+            for (int m = 0; m < MT; ++m) TY::rows(ty, 16 * m + c, k, l, y[m].a, y[m].b);
+#pragma unroll
+            for (int b = 0; b < NT; ++b) {
+                const Frag<bf16> wa = TW::columns(tw, 32 * k, 8, b, l), wb = TW::columns(tw, 32 * k + 4, 8, b, l);
+#pragma unroll
+                for (int m = 0; m < MT; ++m) acc[m][b] = mm2(y[m].a, y[m].b, wa, wb, acc[m][b]);
             }
         }
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int b = 0; b < DB; ++b) {
-                const Frag<bf16> ta = transpose(wt[h][b].a, id), tb = transpose(wt[h][b].b, id);
-#pragma unroll
-                for (int m = 0; m < MT; ++m) {
-                    const Frag<bf16> x = h == 0 ? y[m].a : y[m].b;
-                    acc[m][2 * b] = mm(x, ta, acc[m][2 * b]);
-                    acc[m][2 * b + 1] = mm(x, tb, acc[m][2 * b + 1]);
-                }
-            }
     }
+    __syncthreads();                                      // the sums lie where the waves' tiles were
+    f32x4* const red = reinterpret_cast<f32x4*>(sm);
     if (wv) {
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
-            for (int b = 0; b < 2 * DB; ++b) red[wv - 1][m * 2 * DB + b][l] = acc[m][b];
+            for (int b = 0; b < NT; ++b) red[((wv - 1) * MT * NT + m * NT + b) * 64 + l] = acc[m][b];
     }
     __syncthreads();
     if (wv) return;
@@ -181,14 +220,11 @@ __global__ __launch_bounds__(256) void layer_down_kernel(DownArgs p) {
     for (int m = 0; m < MT; ++m) {
         if (r0 + 16 * m + c >= p.M) continue;
 #pragma unroll
-        for (int b = 0; b < DB; ++b) {
-            f32x4 s[2];
+        for (int b = 0; b < NT; ++b) {
+            f32x4 s = acc[m][b];
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int i = m * 2 * DB + 2 * b + h;
-                s[h] = acc[m][2 * b + h] + red[0][i][l] + red[1][i][l] + red[2][i][l];
-            }
-            st16(p.dx[which] + (r0 + 16 * m + c) * p.ldx + 32 * b + 8 * g, s[0], s[1]);
+            for (int i = 0; i < 3; ++i) s += red[(i * MT * NT + m * NT + b) * 64 + l];
+            st_frag(p.dx[which] + (r0 + 16 * m + c) * p.ldx + 16 * b + 4 * g, to_frag<bf16>(s));
         }
     }
 }
@@ -206,12 +242,6 @@ __global__ __launch_bounds__(256) void layer_down_kernel(DownArgs p) {
 // UNR: a wave's whole share of K up to 2048 (16 rows) in one or two goes; twice as many is no faster (16 x 6416 x 2048 5.0,
 // 64 x 6416 x 2048 7.6 -> 8.7) and asks twice for K = 512 what is there once (1 -> 2 blocks a wave too many, 2.5 -> 3.0 for 32 rows).
 constexpr int RW = 8;                                     // waves
-// a wave's LDS writes before its reads of what its other lanes wrote, and the other way round: the hardware keeps the order
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-}
 template <int MT, int RT, int UNR>
 __global__ __launch_bounds__(64 * RW) void rows_gemm_kernel(const bf16* __restrict__ x, long long ldx, const bf16* __restrict__ w, long long ldw,
                                                             bf16* __restrict__ y, long long ldy, int M, int N, int K) {

@@ -4,28 +4,15 @@
 // Linear(embed_dim -> head_dim) followed by Linear(head_dim -> embed_dim), HRDPLR/hdla_custom.py:117-121,151-155; in the
 // reference a BLAS call inside autograd).  The output is tiny (K x N) and the contraction runs over all rows, so a
 // BLAS kernel tiled over the output has 16 workgroups to work with; here the rows are split as well: a workgroup owns
-// 32 columns of dY and one range of rows, its four wavefronts take every fourth 16-row tile of that range (16 bytes a
-// lane from dY and from X0), add their sums through LDS, and leave a fp32 partial result; a second small kernel adds
-// the partial results of the row ranges in a fixed order.
+// 16 KA columns of dY and one range of rows, its WW wavefronts take every WW'th 32-row tile of that range, add their sums through
+// LDS, and leave a fp32 partial result; a second small kernel adds the partial results of the row ranges in a fixed order.
 //
-// The contraction index (the row) must be the inner index of both MFMA operands, and both are stored with the row
-// outermost, so each 16 x 16 tile is transposed on its way in by one product with the identity (exact in bf16).
-#include "hdla_common.cuh"
+// The contraction index (the row) must be the inner index of both MFMA operands, and both are stored with the row outermost: tiles of
+// 32 rows go through LDS as they come (RowTile) and the transposing LDS read takes them from there.
+#include "row_tile.cuh"
 #include "../../include/hdla_hip.h"
 
 namespace hdla {
-
-// Two 16 x 16 tiles from one 16-byte load per lane: lane (g, c) reads elements 8g .. 8g+7 of row c of a 16 x 32 block;
-// the first four are the fragment of tile A, the last four of tile B, where tile A holds the block's columns
-// 8j + 0..3 and tile B the columns 8j + 4..7 (j = 0..3).  Element e = 0..15 of a tile's column index is therefore
-// column 8 (e / 4) + e % 4 (+ 4 for tile B) of the block.
-__device__ __forceinline__ void ld_two_tiles(const bf16* p, bool ok, Frag<bf16>& a, Frag<bf16>& b) {
-    s16x8 x = *reinterpret_cast<const s16x8*>(p);
-    const s16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
-    x = ok ? x : z;
-    a.v = __builtin_shufflevector(x, x, 0, 1, 2, 3);
-    b.v = __builtin_shufflevector(x, x, 4, 5, 6, 7);
-}
 
 // One product, or the two of the layer (blockIdx.z).  With F given the gradient is that of logsigmoid(F): dY sigmoid(-F),
 // rounded to bf16 as a stored gradient would be (forming it here saves a pass over it: 10.7 us of 8192 x 1024).
@@ -35,80 +22,93 @@ struct WgradArgs {
     long long ldy, ldx;
     int M, K, rows_per;
 };
-template <int N>
-__global__ __launch_bounds__(256) void skinny_wgrad_kernel(WgradArgs p) {
+// Measured, both products of the layer, 8192 rows, K = 1024, N = 64 (three 16.8 MB tensors read: 10.2 us at copy rate), without the sums of
+// the partial results: 25.2 us with the lanes of a request in fragment order (row_tile.cuh), tiles turned by products with the identity and
+// 32 columns a workgroup; 17.5 like this.
+template <int N, int KA, int WW>
+__global__ __launch_bounds__(64 * WW) void skinny_wgrad_kernel(WgradArgs p) {
     const int which = blockIdx.z;
     const bf16* __restrict__ dY = p.dY[which];
     const bf16* __restrict__ F = p.F[which];
     const bf16* __restrict__ X0 = p.X0[which];
-    float* __restrict__ part = p.part[which];
-    const long long ldy = p.ldy, ldx = p.ldx;
-    const int M = p.M, K = p.K, rows_per = p.rows_per;
-    constexpr int ZP = N / 32;                                 // 32-column blocks of X0
-    __shared__ f32x4 red[3][2 * 2 * ZP][64];
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-    const int k0 = blockIdx.x * 32, s = blockIdx.y;
-    const long long rbeg = (long long)s * rows_per;
-    const long long rend = rbeg + rows_per < M ? rbeg + rows_per : M;
-    const Frag<bf16> id = ident_frag<bf16>();
-    f32x4 acc[2][2 * ZP];                                      // [tile of dY's 32 columns][tile of X0's columns]
+    constexpr int NB = N / 16;
+    typedef RowTile<16 * KA> TY;
+    typedef RowTile<N> TX;
+    constexpr int RY = 32 / TY::RPR, RX = 32 / TX::RPR;        // requests of a tile of 32 rows
+    constexpr int TILES = 32 * (TY::ROW + TX::ROW), SUMS = KA * NB * 1024;   // bytes a wave
+    constexpr int BYTES = WW * (TILES > SUMS ? TILES : SUMS);
+    static_assert(KA * NB % WW == 0, "whole tiles a wavefront");
+    __shared__ __attribute__((aligned(16))) char sm[BYTES];
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane_id(), g = l >> 4, c = l & 15;
+    char* const ty = sm + wv * TILES;
+    char* const tx = ty + 32 * TY::ROW;
+    const int k0 = blockIdx.x * (16 * KA), s = blockIdx.y;
+    const long long rbeg = (long long)s * p.rows_per;
+    const long long rend = rbeg + p.rows_per < p.M ? rbeg + p.rows_per : p.M;
+    f32x4 acc[KA][NB];                                         // [tile of dY's columns][tile of X0's columns]
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int a = 0; a < KA; ++a)
 #pragma unroll
-        for (int b = 0; b < 2 * ZP; ++b) acc[a][b] = zero4();
-    // the four wavefronts take every fourth 16-row tile of the range
-#pragma unroll 4
-    for (long long r0 = rbeg + 16 * w; r0 < rend; r0 += 64) {
-        const bool ok = r0 + c < rend;
-        const long long row = ok ? r0 + c : rbeg;              // a readable row on every lane
-        Frag<bf16> x[2], z[2 * ZP];
-        ld_two_tiles(dY + row * ldy + k0 + 8 * g, ok, x[0], x[1]);
+        for (int b = 0; b < NB; ++b) acc[a][b] = zero4();
+    // a tile's rows as they come; rows past the range: its last one again, zeros where used
+    struct In { s16x8 y[RY], f[RY], x[RX]; };
+    auto request = [&](long long r0) __attribute__((always_inline)) {
+        In in;
 #pragma unroll
-        for (int b = 0; b < ZP; ++b) ld_two_tiles(X0 + row * ldx + 32 * b + 8 * g, ok, z[2 * b], z[2 * b + 1]);
+        for (int j = 0; j < RY; ++j) {
+            const long long at = min(r0 + TY::row(j, l), rend - 1) * p.ldy + k0 + TY::col(l);
+            in.y[j] = *reinterpret_cast<const s16x8*>(dY + at);
+            if (F) in.f[j] = *reinterpret_cast<const s16x8*>(F + at);
+        }
+#pragma unroll
+        for (int j = 0; j < RX; ++j) in.x[j] = *reinterpret_cast<const s16x8*>(X0 + min(r0 + TX::row(j, l), rend - 1) * p.ldx + TX::col(l));
+        return in;
+    };
+    long long r0 = rbeg + 32 * wv;
+    In next;
+    if (r0 < rend) next = request(r0);
+    for (; r0 < rend; r0 += 32 * WW) {
+        In in = next;
+        if (r0 + 32 * WW < rend) next = request(r0 + 32 * WW);   // (the next tile's on their way while this one is worked on)
+        const s16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+        const int live = (int)(rend - r0 < 32 ? rend - r0 : 32);
         if (F) {
-            Frag<bf16> f[2];
-            ld_two_tiles(F + row * ldy + k0 + 8 * g, ok, f[0], f[1]);
 #pragma unroll
-            for (int a = 0; a < 2; ++a) {
-                f32x4 d = to_f32(x[a]);
-                const f32x4 t = to_f32(f[a]);
-                float e[4], s[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) e[i] = __expf(t[i]);
-                sigmoid_of_exp<4>(e, s);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) d[i] *= s[i];
-                x[a] = to_frag<bf16>(d);
-            }
+            for (int j = 0; j < RY; ++j) in.y[j] = times_sigmoid_neg(in.y[j], in.f[j]);
         }
-        // transposed tiles: rows = columns of the block, inner index = row of the range
-        x[0] = transpose(x[0], id);
-        x[1] = transpose(x[1], id);
+        wave_lds_fence();                                      // (the reads of the tile before)
 #pragma unroll
-        for (int b = 0; b < 2 * ZP; ++b) {
-            const Frag<bf16> zt = transpose(z[b], id);
-            acc[0][b] = mm(x[0], zt, acc[0][b]);
-            acc[1][b] = mm(x[1], zt, acc[1][b]);
+        for (int j = 0; j < RY; ++j) TY::put(ty, j, l, TY::row(j, l) < live ? in.y[j] : zero);
+#pragma unroll
+        for (int j = 0; j < RX; ++j) TX::put(tx, j, l, TX::row(j, l) < live ? in.x[j] : zero);
+        wave_lds_fence();
+        Frag<bf16> y[KA][2];
+#pragma unroll
+        for (int a = 0; a < KA; ++a)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) y[a][h] = TY::columns(ty, 16 * h, 4, a, l);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const Frag<bf16> x0 = TX::columns(tx, 0, 4, b, l), x1 = TX::columns(tx, 16, 4, b, l);
+#pragma unroll
+            for (int a = 0; a < KA; ++a) acc[a][b] = mm2(y[a][0], y[a][1], x0, x1, acc[a][b]);
         }
     }
-    if (w) {
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2 * ZP; ++b) red[w - 1][a * 2 * ZP + b][lane] = acc[a][b];
-    }
+    // the wavefronts' sums: each adds up its share of the tiles
+    f32x4* const red = reinterpret_cast<f32x4*>(sm);
     __syncthreads();
-    if (w) return;
-    // lane (g, c) register i of acc[a][b]: dY column k0 + 8 (c / 4) + c % 4 + 4 a,
-    //                                      X0 column 32 (b / 2) + 8 g + 4 (b % 2) + i
-    const int krow = k0 + 8 * (c >> 2) + (c & 3);
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int i = 0; i < KA * NB; ++i) red[(wv * KA * NB + i) * 64 + l] = acc[i / NB][i % NB];
+    __syncthreads();
 #pragma unroll
-        for (int b = 0; b < 2 * ZP; ++b) {
-            const f32x4 v = acc[a][b] + red[0][a * 2 * ZP + b][lane] + red[1][a * 2 * ZP + b][lane] + red[2][a * 2 * ZP + b][lane];
-            *reinterpret_cast<f32x4*>(part + ((long long)s * K + krow + 4 * a) * N + 32 * (b >> 1) + 8 * g + 4 * (b & 1)) = v;
-        }
+    for (int j = 0; j < KA * NB / WW; ++j) {
+        const int i = wv * (KA * NB / WW) + j, a = i / NB, b = i % NB;
+        f32x4 sum = red[i * 64 + l];
+#pragma unroll
+        for (int w = 1; w < WW; ++w) sum += red[(w * KA * NB + i) * 64 + l];
+        // lane (g, c) register e: dY column k0 + 16 a + c, X0 column 16 b + 4 g + e
+        *reinterpret_cast<f32x4*>(p.part[which] + ((long long)s * p.K + k0 + 16 * a + c) * N + 16 * b + 4 * g) = sum;
+    }
 }
 
 // dW = sum over the row ranges of their partial results, eight outputs a thread
@@ -133,16 +133,16 @@ __global__ __launch_bounds__(256) void skinny_wgrad_sum_kernel(const float* __re
 }
 
 // row ranges: enough workgroups for the chip (and, when there are many rows, several per CU, about 1024 rows each, so
-// that enough loads are in flight to cover the latency of HBM), whole 16-row tiles each
+// that enough loads are in flight to cover the latency of HBM), whole 32-row tiles each
 static int wgrad_split(long long M, int K, int& rows_per) {
     const int kb = K / 32;
     long long S = (256 + kb - 1) / kb;
     const long long by_rows = M / 1024, most = (2048 + kb - 1) / kb;
     if (by_rows > S) S = by_rows < most ? by_rows : most;
-    const long long tiles = (M + 15) / 16;
+    const long long tiles = (M + 31) / 32;
     if (S > tiles) S = tiles;
     if (S < 1) S = 1;
-    rows_per = (int)(((tiles + S - 1) / S) * 16);
+    rows_per = (int)(((tiles + S - 1) / S) * 32);
     return (int)((M + rows_per - 1) / rows_per);
 }
 
@@ -152,9 +152,14 @@ using namespace hdla;
 
 // `count` products (1 or 2), then the sums of their partial results
 static int wgrad_launch(const WgradArgs& a, int N, int S, int count, bf16* dW0, bf16* dW1, hipStream_t s) {
-    const dim3 grid(a.K / 32, S, count), block(256);
-    if (N == 64) hipLaunchKernelGGL((skinny_wgrad_kernel<64>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((skinny_wgrad_kernel<128>), grid, block, 0, s, a);
+    const dim3 block(256);
+    // Columns of dY and wavefronts a workgroup.  Many rows, N = 64: whole cache lines of dY and half of the reads of X0; few rows leave
+    // some of eight wavefronts without any.  Both products and their sums, us, 32 columns and 4 wavefronts / 64 and 8: 8192 x 1024
+    // 26.9 / 22.8, 3000 x 1024 14.7 / 14.7, 1000 x 512 9.1 / 13.8.  N = 128 has no registers for 64 columns; with 8 wavefronts, so one
+    // workgroup a compute unit, 8192 x 2048 takes 61.8, with 4 52.0.
+    if (N == 64 && a.M >= 2048) hipLaunchKernelGGL((skinny_wgrad_kernel<64, 4, 8>), dim3(a.K / 64, S, count), dim3(512), 0, s, a);
+    else if (N == 64) hipLaunchKernelGGL((skinny_wgrad_kernel<64, 2, 4>), dim3(a.K / 32, S, count), block, 0, s, a);
+    else hipLaunchKernelGGL((skinny_wgrad_kernel<128, 2, 4>), dim3(a.K / 32, S, count), block, 0, s, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
     const long long kn = (long long)a.K * N;

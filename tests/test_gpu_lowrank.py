@@ -49,6 +49,12 @@ def test_low_rank_pair(rows, d, D):
     assert lib.hdla_layer_up_fwd(ctypes.byref(_lib.HdlaUpDims(rows, d, 96, ld, cf, cg)), P(y), P(wf), P(wg), None, P(lf), P(gate), st) == -2
 
 
+@pytest.mark.parametrize("rows,d,D", [(2047, 128, 64), (2048, 384, 64), (2079, 256, 64), (5000, 640, 64), (31, 128, 128), (33, 384, 64), (4129, 384, 128)])
+def test_low_rank_pair_at_the_lines(rows, d, D):
+    """Where a dispatch goes another way (rows), and with tiles of 32 rows and of 64 columns that are not all there."""
+    test_low_rank_pair(rows, d, D)
+
+
 @pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
 @pytest.mark.parametrize("N,K", [(20, 32), (16, 160), (200, 1056), (1040, 2048)])
 def test_rows_gemm(M, N, K):
