@@ -58,6 +58,9 @@ __device__ __forceinline__ void seg_range(const SeqTab& st, int n, int nseg, int
     seg_range(c0, c1, nseg, seg, s0, s1);
 }
 
+// Columns 16 j + 4 g .. + 3 of row c of a chunk's G, in elements from its start: pieces of eight columns, the 16 rows of a piece side by side
+__device__ __forceinline__ int gw_at(int j, int g, int c) { return (j >> 1) * PAIR + ((2 * (j & 1) + (g >> 1)) * 16 + c) * 8 + 4 * (g & 1); }
+
 // LDS of a fused workgroup (byte offsets): per producer pair one slot = [operands | outbox | solver scratch], then the flags
 template <typename T, int K, int V, int MODE> struct FusedLds {
     static constexpr int ES = sizeof(T), TB = TILE * ES, KT = K / 16, VT = V / 16;
@@ -206,19 +209,20 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
                     if (r < len) *reinterpret_cast<i32x4*>(reinterpret_cast<char*>(p.o + ((tok0 + r) * H + h) * V) + e) = x;
                 }
             } else {
-                constexpr int LPO = V * 4 / 16, RPO = 64 / LPO;
-                char* ol = reinterpret_cast<char*>(a.ol + chw * (CH * V));
+                // in the order in which fixup_kernel takes them: 1-KiB pieces, lane (g, c) has columns 16 j + 4 g .. + 3 of o's row c, and
+                // columns 32 j + 8 g .. + 7 of G's
+                const int g = l >> 4, c = l & 15;
+                char* ol = reinterpret_cast<char*>(a.ol + chw * (CH * V)) + 16 * l;
 #pragma unroll
-                for (int r0 = 0; r0 < NR; r0 += RPO) {
-                    const int r = rb + r0 + l / LPO, e = (l % LPO) * 16;
-                    *reinterpret_cast<i32x4*>(ol + r * (V * 4) + e) = *reinterpret_cast<const i32x4*>(slot + L::OBOX + r * L::OROW + e);
+                for (int i = 0; i < V / 16 * NR / CH; ++i) {
+                    const int j = rb * (V / 16) / CH + i;
+                    *reinterpret_cast<i32x4*>(ol + j * 1024) = *reinterpret_cast<const i32x4*>(slot + L::OBOX + c * L::OROW + 64 * j + 16 * g);
                 }
-                constexpr int LPG = K * (int)sizeof(T) / 16, RPG = 64 / LPG;
-                char* gw = reinterpret_cast<char*>(a.gw + chw * (CH * K));
+                char* gw = reinterpret_cast<char*>(a.gw + chw * (CH * K)) + 16 * l;
 #pragma unroll
-                for (int r0 = 0; r0 < NR; r0 += RPG) {
-                    const int r = rb + r0 + l / LPG, e = (l % LPG) * 16;
-                    *reinterpret_cast<i32x4*>(gw + r * (K * (int)sizeof(T)) + e) = *reinterpret_cast<const i32x4*>(slot + L::GBOX + r * L::GROW + e);
+                for (int i = 0; i < K / 32 * NR / CH; ++i) {
+                    const int j = rb * (K / 32) / CH + i;
+                    *reinterpret_cast<i32x4*>(gw + j * 1024) = *reinterpret_cast<const i32x4*>(slot + L::GBOX + c * L::GROW + 64 * j + 16 * g);
                 }
             }
         }
@@ -1047,7 +1051,7 @@ __device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* 
             G = mm2(aqb[0], aqb[1], vpb[0], vpb[1], G);
             const Frag<T> Gf = to_frag<T>(G);             // rows token, inner k' (the block's columns)
             if (FWD) st_frag(reinterpret_cast<T*>(smem + pp * L::SLOT + L::GBOX + c * L::GROW) + 16 * wv + 4 * g, Gf);
-            else st_frag(a.gw + (chw * CH + c) * K + 16 * wv + 4 * g, Gf);
+            else st_frag(a.gw + chw * (CH * K) + gw_at(wv, g, c), Gf);
 #pragma unroll
             for (int kt = 0; kt < KT; ++kt) M[kt] = mm2(vpb[0], vpb[1], bgt[0][kt], bgt[1][kt], M[kt] * egl[kt]);
         }
@@ -1117,7 +1121,7 @@ __device__ __forceinline__ void fused_consumer_ckpt(const FusedArgs<T>& a, char*
     }
     const Frag<T> ident = ident_frag<T>();
     // rows token, inner k' (the block's columns), requested a chunk ahead
-    const T* gw = a.gw + ((int64_t)h * p.st.nch + s0) * (CH * K) + c * K + 16 * wv + 4 * g;
+    const T* gw = a.gw + ((int64_t)h * p.st.nch + s0) * (CH * K) + gw_at(wv, g, c);
     Frag<T> gn = zero_frag<T>();
     if (later) gn = ld_frag(gw);
 
@@ -1409,7 +1413,9 @@ __global__ __launch_bounds__(64 * (V / 16 + 2 * FNP)) void fused_kernel(FusedArg
 // whole, are loaded a quarter by each wave and shared through LDS as split operands; wave j chains column block j of
 // the state (the blocks are independent); FIXUP_PARTS workgroups share the chunks of a segment, each repeating the
 // chain, so that a workgroup's share of the chunks is in flight from the start as well.
-constexpr int FIXUP_PARTS = 2;                            // workgroups that share one segment's chunks (measured: 1, 2, 4 -> 17.1, 16.8, 18.8 us)
+// The local outputs and G lie in memory as the waves take them (copy_out): 16.1 -> 12.8 us for 4 x 2048 tokens of 16 heads in four segments,
+// where requests for 16 rows had met 16 cache lines each; those two read and o written are 9 at copy rate.
+constexpr int FIXUP_PARTS = 2;                            // workgroups that share one segment's chunks (measured: 1, 2, 4 -> 12.8, 12.8, 16.0 us)
 constexpr int FIXUP_STAGE = 3;                            // chain steps whose records are in LDS at a time
 template <typename T, int K, int V>
 __global__ __launch_bounds__(256) void fixup_kernel(FusedArgs<T> a) {
@@ -1450,12 +1456,12 @@ __global__ __launch_bounds__(256) void fixup_kernel(FusedArgs<T> a) {
         for (int b = 0; b < NB; ++b) {
             const int cid = min(first + 4 * b, s1 - 1);   // past the end: the last chunk again, never used
             const int64_t chw = (int64_t)h * p.st.nch + cid;
-            const T* gw = a.gw + chw * (CH * K) + c * K + 4 * g;
-            const float* ol = a.ol + chw * (CH * V) + c * V + 4 * g;
+            const T* gw = a.gw + chw * (CH * K);
+            const float* ol = a.ol + chw * (CH * V) + 4 * l;
 #pragma unroll
-            for (int kt = 0; kt < KT; ++kt) G[b][kt] = ld_frag(gw + 16 * kt);
+            for (int kp = 0; kp < KT / 2; ++kp) ld_pair(gw + kp * PAIR, G[b][2 * kp], G[b][2 * kp + 1]);
 #pragma unroll
-            for (int j = 0; j < VT; ++j) OLr[b][j] = *reinterpret_cast<const f32x4*>(ol + 16 * j);
+            for (int j = 0; j < VT; ++j) OLr[b][j] = *reinterpret_cast<const f32x4*>(ol + j * TILE);
         }
     };
     const bool outputs = target < a.nseg && a.ol != nullptr;
@@ -1561,7 +1567,11 @@ __global__ __launch_bounds__(256) void fixup_kernel(FusedArgs<T> a) {
 #pragma unroll
     for (int j = 0; j < VT; ++j)
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt) Sb[j][kt] = ld_tile(sS + (j * KT + kt) * TILE);
+        for (int kt = 0; kt < KT; ++kt) {
+            // the channels that G's fragment kt has on this lane: 32 (kt / 2) + 8 g + 4 (kt % 2) .. + 3
+            const int ch = 8 * g + 4 * (kt & 1);
+            Sb[j][kt].v = *reinterpret_cast<const s16x4*>(sS + (j * KT + (kt & ~1) + ch / 16) * TILE + 4 * (ch % 16 / 4 * 16 + c));
+        }
     char* const st = stage[wv];
     for (int first = s0 + wv; first < s1; first += 4 * NB) {
 #pragma unroll

@@ -21,10 +21,10 @@ struct FusedArgs {
     float* rseg;           // [N][H][nseg][K*V]
     const float* sin;      // [N][H][nseg][K*V]  states entering the segments (read by FUSED_CKPT)
     float* sin_out;        // the same record, written by fixup_kernel (nullable)
-    float* ol;             // [H][nch][16][V] fp32  local outputs of segments > 0 (forward pass); null: fixup_kernel only chains
+    float* ol;             // [H][nch][V/16] fp32 tiles  local outputs of segments > 0 (forward pass); null: fixup_kernel only chains
     // the record (with c.ws.TM and c.ws.STRONG): written by FUSED_FWD and FUSED_SUM, read by FUSED_CKPT and FUSED_REV
     float* mt;             // [N][H][nseg][K*K]     transposed transitions of segments > 0 (nullable)
-    T* gw;                 // [H][nch][16][K]       G of segments > 0 (the forward pass's fixup_kernel needs it as well)
+    T* gw;                 // [H][nch][K/8][16][8]  G of segments > 0 (the forward pass's fixup_kernel needs it as well)
     T* aq;                 // [H][nch][2][2 tiles]  A_ak, A_qb
     int* err;              // set nonzero by a wave whose bounded wait ran out
 };
