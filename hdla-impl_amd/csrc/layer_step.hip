@@ -17,16 +17,19 @@
 
 namespace hdla {
 
+// what becomes of o: it is stored as it is, gated and normalised, or gated in fp32 with its head's part of the sum of squares
+enum StepNorm { NORM_NOT, NORM_HERE, NORM_LATER };
 struct StepArgs {
     const bf16 *y, *log_f;                // [rows, ldy]; [rows, H, D] (not UP)
     bf16* gate;                           // [rows, H, D]: read, or (UP, null if nobody wants it) written
     const bf16 *wf, *wg;                  // UP: [H D, D] x 2, of the decay and of the gate
     const void* weight;                   // [H, D] of the norm, or null
     const float* h0;                      // [N, H, D, D], or null
-    bf16* o;                              // [rows, H, D]
+    bf16* o;                              // [rows, H, D] (not where the norm is left to the projection)
+    float *gated, *sums;                  // NORM_LATER: [rows, H, D] o sigmoid(gate), [rows, H] sums of squares
     float* ht;                            // [N, H, D, D], or null
     int T, H, ldy, cq, ck, cv, cb, cf, cg;
-    int norm_q, norm_k, norm_v, w_f32, norm, gate_pre;         // norm: o gated and normalised, else as it is
+    int norm_q, norm_k, norm_v, w_f32, norm, gate_pre;
     float beta_scale, eps_d, scale, cn, inv_e, eps;
 };
 
@@ -93,7 +96,7 @@ __global__ __launch_bounds__(4 * D, 4) void layer_step_kernel(StepArgs p) {
 #pragma unroll
     for (int i = 0; i < WPR; ++i) {
         const int at = h * D + WPR * lane + i;
-        w[i] = !p.norm || !p.weight ? 1.f : p.w_f32 ? static_cast<const float*>(p.weight)[at] : bf2f(static_cast<const bf16*>(p.weight)[at].x);
+        w[i] = p.norm != NORM_HERE || !p.weight ? 1.f : p.w_f32 ? static_cast<const float*>(p.weight)[at] : bf2f(static_cast<const bf16*>(p.weight)[at].x);
     }
     // UP: 16 lanes a row of the weights, D / 16 elements a lane, D / 4 rows at a time
     constexpr int EL = D / 16;
@@ -222,13 +225,21 @@ __global__ __launch_bounds__(4 * D, 4) void layer_step_kernel(StepArgs p) {
                 for (int k = 0; k < NW; ++k) o[i] += red[k][2][WPR * lane + i];
                 o[i] = as_bf16(o[i]);
                 gs[i] = step_sigmoid(UP ? up[1][WPR * lane + i] : bf2f((uint16_t)(now.gate >> (16 * i))));
-                if (p.norm && p.gate_pre) o[i] *= gs[i];
-                sum += o[i] * o[i];
+                if (p.norm == NORM_HERE && p.gate_pre) o[i] *= gs[i];
+                const float x = p.norm == NORM_LATER && p.gate_pre ? o[i] * gs[i] : o[i];
+                sum += x * x;
+            }
+            if (p.norm == NORM_LATER) {
+                sum = wave_sum(sum);
+                if (lane == 0) p.sums[t * p.H + h] = sum;
+#pragma unroll
+                for (int i = 0; i < WPR; ++i) p.gated[(t * p.H + h) * D + WPR * lane + i] = o[i] * gs[i];
+                continue;
             }
             const float rs = p.cn / sqrtf(wave_sum(sum) * p.inv_e + p.eps);
 #pragma unroll
             for (int i = 0; i < WPR; ++i) {
-                if (p.norm) {
+                if (p.norm == NORM_HERE) {
                     o[i] = o[i] * rs * w[i];
                     if (!p.gate_pre) o[i] *= gs[i];
                 }
@@ -251,7 +262,7 @@ using namespace hdla;
 
 extern "C" int hdla_layer_step(const hdla_pre_dims* pre, const hdla_up_dims* up, const hdla_norm_dims* norm, int32_t T, const void* y,
                                const void* wf, const void* wg, const void* log_f, void* gate, const void* weight, const float* h0, void* o,
-                               float* ht, void* stream) {
+                               float* gated, float* ht, void* stream) {
     if (!pre) return HDLA_ERR_NULL;
     if (pre->dtype != HDLA_BF16) return HDLA_ERR_DTYPE;
     const long long rows = pre->rows, H = pre->H, D = pre->D;
@@ -266,12 +277,13 @@ extern "C" int hdla_layer_step(const hdla_pre_dims* pre, const hdla_up_dims* up,
     }
     if (norm) {
         if (norm->dtype != HDLA_BF16 || (weight && norm->weight_dtype != HDLA_BF16 && norm->weight_dtype != HDLA_FP32)) return HDLA_ERR_DTYPE;
-        if (norm->rows != rows || norm->G != H || norm->E != D || (norm->gate_pos != 1 && norm->gate_pos != 2) || !(norm->eps >= 0.f))
+        if (norm->rows != rows || norm->G != (gated ? 1 : H) || norm->E != (gated ? H * D : D) || (norm->gate_pos != 1 && norm->gate_pos != 2) || !(norm->eps >= 0.f))
             return HDLA_ERR_SHAPE;
     }
+    if (gated && !norm) return HDLA_ERR_NULL;
     if (rows == 0) return HDLA_OK;
-    if (!y || !o || (up ? !wf || !wg : !log_f || (norm && !gate))) return HDLA_ERR_NULL;
-    for (const void* p : {y, wf, wg, log_f, (const void*)gate, weight, (const void*)h0, (const void*)o, (const void*)ht})
+    if (!y || (!o && !gated) || (up ? !wf || !wg : !log_f || (norm && !gate))) return HDLA_ERR_NULL;
+    for (const void* p : {y, wf, wg, log_f, (const void*)gate, weight, (const void*)h0, (const void*)o, (const void*)gated, (const void*)ht})
         if (!step_al(p)) return HDLA_ERR_ALIGN;
     StepArgs a{};
     a.y = static_cast<const bf16*>(y); a.log_f = static_cast<const bf16*>(log_f); a.gate = static_cast<bf16*>(gate);
@@ -282,7 +294,8 @@ extern "C" int hdla_layer_step(const hdla_pre_dims* pre, const hdla_up_dims* up,
     a.norm_q = pre->norm_q; a.norm_k = pre->norm_k; a.norm_v = pre->norm_v;
     a.beta_scale = pre->beta_scale; a.eps_d = pre->eps * (float)D; a.scale = 1.f;
     if (norm) {
-        a.norm = 1; a.w_f32 = norm->weight_dtype == HDLA_FP32; a.gate_pre = norm->gate_pos == 1;
+        a.norm = gated ? NORM_LATER : NORM_HERE; a.gated = gated; a.sums = gated + rows * H * D;
+        a.w_f32 = norm->weight_dtype == HDLA_FP32; a.gate_pre = norm->gate_pos == 1;
         a.cn = norm->c / sqrtf((float)norm->E); a.inv_e = 1.f / (float)norm->E; a.eps = norm->eps;
     }
     const dim3 grid((unsigned)(rows / T * H)), block((unsigned)(4 * D));

@@ -242,9 +242,19 @@ __global__ __launch_bounds__(256) void layer_down_kernel(DownArgs p) {
 // UNR: a wave's whole share of K up to 2048 (16 rows) in one or two goes; twice as many is no faster (16 x 6416 x 2048 5.0,
 // 64 x 6416 x 2048 7.6 -> 8.7) and asks twice for K = 512 what is there once (1 -> 2 blocks a wave too many, 2.5 -> 3.0 for 32 rows).
 constexpr int RW = 8;                                     // waves
-template <int MT, int RT, int UNR>
+// NORM (one row tile): x is formed on the way in, x = gated c / sqrt(K) / sqrt(sum of the row's parts / K + eps) weight, rounded to bf16
+// as the norm's output is: one launch less, and no pass over a few rows that is all latency (16 x 2048 x 2048: norm 4.1 and product 4.4
+// -> 7.6 us).
+struct NormIn {
+    const float *gated, *sums;            // [M, K], [M, parts]
+    const void* weight;                   // [K] or null
+    int parts, w_f32;
+    float cn, inv_e, eps;
+};
+template <int MT, int RT, int UNR, bool NORM>
 __global__ __launch_bounds__(64 * RW) void rows_gemm_kernel(const bf16* __restrict__ x, long long ldx, const bf16* __restrict__ w, long long ldw,
-                                                            bf16* __restrict__ y, long long ldy, int M, int N, int K) {
+                                                            bf16* __restrict__ y, long long ldy, int M, int N, int K, NormIn nrm) {
+    static_assert(!NORM || MT == 1, "one row tile");
     constexpr int TURN = RT + MT, SUMS = RT * MT;         // KiB a wave: to change lanes in, of sums
     static_assert(SUMS <= RW, "a wave per tile of the result");
     __shared__ __attribute__((aligned(16))) char sm[RW * (TURN > SUMS ? TURN : SUMS) * 1024];
@@ -252,11 +262,32 @@ __global__ __launch_bounds__(64 * RW) void rows_gemm_kernel(const bf16* __restri
     const int n0 = blockIdx.x * (16 * RT), row = l >> 2, piece = l & 3;
     // row r's pieces p lie at 4 r + (p ^ r / 4): 16 lanes of either order meet each bank once
     char* const put = sm + wv * (TURN * 1024) + ((4 * row + (piece ^ (row >> 2))) << 4);
+    char* const put_half = sm + wv * (TURN * 1024) + 64 * row + 8 * (piece & 1);
     const char* const get = sm + wv * (TURN * 1024) + ((4 * c + (g ^ (c >> 2))) << 4);
     const bf16* from[TURN];                               // rows past the end: read again, not stored
 #pragma unroll
     for (int i = 0; i < TURN; ++i)
         from[i] = (i < RT ? w + (long long)min(n0 + 16 * i + row, N - 1) * ldw : x + (long long)min(16 * (i - RT) + row, M - 1) * ldx) + 8 * piece;
+    float rs = 0.f;
+    // (of gated, twice the bytes, a lane has four columns in each half of the block: requests of 64 bytes a row here too)
+    const float* const gated = NORM ? nrm.gated + (long long)min(row, M - 1) * K + 4 * piece : nullptr;
+    bool scaled = false;
+    // the row's scale, four lanes a row as everywhere here; behind the first blocks' requests, and all of its own at once
+    auto scale_row = [&]() __attribute__((always_inline)) {
+        const float* const sums = nrm.sums + (long long)min(row, M - 1) * nrm.parts;
+        float ss = 0.f;
+        for (int h0 = 0; h0 < nrm.parts; h0 += 32) {
+            float v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = sums[min(h0 + 4 * i + piece, nrm.parts - 1)];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) ss += h0 + 4 * i + piece < nrm.parts ? v[i] : 0.f;
+        }
+        ss += __shfl_xor(ss, 1);
+        ss += __shfl_xor(ss, 2);
+        rs = nrm.cn / sqrtf(ss * nrm.inv_e + nrm.eps);
+        scaled = true;
+    };
     const int nb = K / 32, per = (nb + RW - 1) / RW, end = min(nb, (wv + 1) * per);
     f32x4 acc[RT][MT];
 #pragma unroll
@@ -266,17 +297,39 @@ __global__ __launch_bounds__(64 * RW) void rows_gemm_kernel(const bf16* __restri
     // (no branch around a block's products: its requests would be moved behind it)
     auto blocks = [&](int b0, bool whole) __attribute__((always_inline)) {
         s16x8 in[UNR][TURN];
+        f32x4 gx[NORM ? UNR : 1][2], wx[NORM ? UNR : 1][2];
 #pragma unroll
-        for (int u = 0; u < UNR; ++u)
+        for (int u = 0; u < UNR; ++u) {
+            const int at = 32 * (whole ? b0 + u : min(b0 + u, end - 1));
 #pragma unroll
-            for (int i = 0; i < TURN; ++i) in[u][i] = *reinterpret_cast<const s16x8*>(from[i] + 32 * (whole ? b0 + u : min(b0 + u, end - 1)));
+            for (int i = 0; i < (NORM ? RT : TURN); ++i) in[u][i] = *reinterpret_cast<const s16x8*>(from[i] + at);
+            if constexpr (NORM) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) gx[u][i] = *reinterpret_cast<const f32x4*>(gated + at + 16 * i);
+                if (!nrm.weight) {
+                    wx[u][0] = wx[u][1] = f32x4{1.f, 1.f, 1.f, 1.f};
+                } else if (nrm.w_f32) {
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) wx[u][i] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(nrm.weight) + at + 16 * i + 4 * piece);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) wx[u][i] = to_f32(ld_frag(static_cast<const bf16*>(nrm.weight) + at + 16 * i + 4 * piece));
+                }
+            }
+        }
         __builtin_amdgcn_sched_barrier(0);                // all of them requested before the first is waited for
+        if (NORM && !scaled) scale_row();
 #pragma unroll
         for (int u = 0; u < UNR; ++u) {
             const s16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
             wave_lds_fence();                             // (the reads of the block before)
 #pragma unroll
-            for (int i = 0; i < TURN; ++i) *reinterpret_cast<s16x8*>(put + 1024 * i) = whole || b0 + u < end ? in[u][i] : zero;
+            for (int i = 0; i < (NORM ? RT : TURN); ++i) *reinterpret_cast<s16x8*>(put + 1024 * i) = whole || b0 + u < end ? in[u][i] : zero;
+            if constexpr (NORM) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    *reinterpret_cast<s16x4*>(put_half + 1024 * RT + (((piece >> 1) + 2 * i) ^ (row >> 2)) * 16) = to_frag<bf16>(gx[u][i] * rs * wx[u][i]).v;
+            }
             wave_lds_fence();
             TwoTiles t[TURN];
 #pragma unroll
@@ -451,7 +504,7 @@ extern "C" int hdla_rows_gemm(int32_t M, int32_t N, int32_t K, const void* x, in
     const bool two = M > 16 && N > 16 * 256;
     const dim3 grid((N + (two ? 31 : 15)) / (two ? 32 : 16)), block(64 * RW);
 #define HDLA_ROWS(MT, RT, UNR) \
-    hipLaunchKernelGGL((rows_gemm_kernel<MT, RT, UNR>), grid, block, 0, s, xp, (long long)ldx, wp, (long long)ldw, yp, (long long)ldy, M, N, K)
+    hipLaunchKernelGGL((rows_gemm_kernel<MT, RT, UNR, false>), grid, block, 0, s, xp, (long long)ldx, wp, (long long)ldw, yp, (long long)ldy, M, N, K, NormIn{})
     if (M <= 16 && K <= 64 * RW) HDLA_ROWS(1, 1, 2);
     else if (M <= 16) HDLA_ROWS(1, 1, 4);
     else if (M <= 32 && !two && K <= 64 * RW) HDLA_ROWS(2, 1, 2);
@@ -460,5 +513,26 @@ extern "C" int hdla_rows_gemm(int32_t M, int32_t N, int32_t K, const void* x, in
     else if (!two) HDLA_ROWS(4, 1, 2);
     else HDLA_ROWS(4, 2, 2);
 #undef HDLA_ROWS
+    return (int)hipGetLastError();
+}
+
+extern "C" int hdla_rows_gemm_norm(int32_t M, int32_t N, int32_t K, const float* gated, int32_t parts, const hdla_norm_dims* norm, const void* weight,
+                                   const void* w, int64_t ldw, void* y, int64_t ldy, void* stream) {
+    if (!norm) return HDLA_ERR_NULL;
+    if (norm->dtype != HDLA_BF16 || (weight && norm->weight_dtype != HDLA_BF16 && norm->weight_dtype != HDLA_FP32)) return HDLA_ERR_DTYPE;
+    if (M < 0 || M > 16 || N < 1 || K < 32 || K % 32 || parts < 1 || norm->rows != M || norm->G != 1 || norm->E != K || !(norm->eps >= 0.f)) return HDLA_ERR_SHAPE;
+    if (M == 0) return HDLA_OK;
+    if (ldw < K || ldy < N) return HDLA_ERR_SHAPE;
+    if (!gated || !w || !y) return HDLA_ERR_NULL;
+    if (!lr_al(gated, 16) || !lr_al(weight, 16) || !lr_al(w, 16) || !lr_al(y, 8) || ldw % 8 || ldy % 4) return HDLA_ERR_ALIGN;
+    const NormIn nrm{gated, gated + (int64_t)M * K, weight, parts, norm->weight_dtype == HDLA_FP32, norm->c / sqrtf((float)K), 1.f / (float)K, norm->eps};
+    const dim3 grid((N + 15) / 16), block(64 * RW);
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    const bf16* wp = static_cast<const bf16*>(w);
+    bf16* yp = static_cast<bf16*>(y);
+    if (K <= 64 * RW)
+        hipLaunchKernelGGL((rows_gemm_kernel<1, 1, 2, true>), grid, block, 0, s, nullptr, 0LL, wp, (long long)ldw, yp, (long long)ldy, M, N, K, nrm);
+    else
+        hipLaunchKernelGGL((rows_gemm_kernel<1, 1, 4, true>), grid, block, 0, s, nullptr, 0LL, wp, (long long)ldw, yp, (long long)ldy, M, N, K, nrm);
     return (int)hipGetLastError();
 }

@@ -43,7 +43,7 @@ struct Api {
     HDLA_FN(recurrent_fwd); HDLA_FN(param_recurrent_fwd); HDLA_FN(normalize_fwd); HDLA_FN(normalize_bwd);
     HDLA_FN(normalize_workspace_bytes); HDLA_FN(layer_pre_fwd); HDLA_FN(layer_pre_bwd); HDLA_FN(layer_up_fwd); HDLA_FN(layer_down);
     HDLA_FN(layer_up_wgrad); HDLA_FN(layer_up_wgrad_workspace_bytes); HDLA_FN(rows_gemm); HDLA_FN(sum_partials); HDLA_FN(stack_rows);
-    HDLA_FN(layer_step);
+    HDLA_FN(layer_step); HDLA_FN(rows_gemm_norm);
 #undef HDLA_FN
 } api;
 PyObject* error_class = nullptr;                 // _lib.HdlaError
@@ -580,26 +580,31 @@ struct LayerFwd { Tensor x, w, y, f, g, o, n, out, ht, boundary; ChunkIn op; hdl
 
 // A few tokens: what is between the projections in one to three launches, without the tensors that the steps would hand on.  (Many
 // tokens are better off with what does not depend on the state done for all of them at once.)  One token after a cached state, us a
-// call, as six launches and eleven tensors -> as this (batch x channels, heads): 1 x 512, 8 37.8 -> 23.9, 16 x 2048, 16 36.9 -> 25.2,
+// call, as six launches and eleven tensors -> as this (batch x channels, heads): 1 x 512, 8 37.8 -> 19.7, 16 x 2048, 16 36.9 -> 24.3,
 // 25 x 4096, 32 67.7 -> 54.5, 256 x 1024, 16 71 -> 57, 256 x 4096, 32 281 -> 249.  The low-rank products in the same launch or in
-// one before it: 23.9 / 26.8, 25.2 / 27.0, 54.5 / 55.9, 57 / 60, 249 / 252; the other way round only at 256 x 2048, 32: 85.3 / 84.5.
+// one before it (and the norm in one of its own): 23.9 / 26.8, 25.2 / 27.0, 54.5 / 55.9, 57 / 60, 249 / 252; the other way round only at 256 x 2048, 32: 85.3 / 84.5.
 void layer_step(const Tensor* P, const LayerCfg& f, const LayerCols& L, const hdla_pre_dims& pd, int64_t T, const Tensor& h0, bool want_ht,
                 LayerFwd& r) {
     const int64_t rows = pd.rows, N = rows / T;
     void* const s = stream_of(r.x);
     const auto opt = r.x.options();
     const bool in_step = T == 1, norm_in_step = f.groups == L.H;
-    r.n = at::empty({rows, L.d}, opt);
+    // A norm over all channels of at most 16 rows: formed where the projection reads it, by every workgroup of the projection for itself.
+    // A launch less, which the host is glad of, but what the workgroups read grows with the square of the channels.  us a call, in a launch
+    // of its own / here: 1 x 512 24.1 / 19.7, 16 x 1024 24.9 / 19.7, 3 x 2048 24.5 / 21.9, 16 x 2048 25.2 / 24.3, 1 x 4096 39.3 / 41.2.
+    const bool later = !norm_in_step && f.groups == 1 && rows <= 16 && L.d <= 2048, own_norm = !norm_in_step && !later;
+    if (!later) r.n = at::empty({rows, L.d}, opt);
     const hdla_up_dims ud = up_dims(L, rows);
-    const hdla_norm_dims nd = norm_dims(r.n, P[8], f.gate_pos, f.c, f.eps, f.groups);
-    const int64_t parts = (norm_in_step ? 0 : 2) + (in_step ? 0 : norm_in_step ? 2 : 1);     // gate, o, log_f as far as they are handed on
+    const hdla_norm_dims nd = norm_dims(r.x, P[8], f.gate_pos, f.c, f.eps, f.groups);
+    // gate, o, log_f and the gated o (fp32) with its sums, as far as they are handed on
+    const int64_t one = rows * L.d, parts = (own_norm ? 2 : 0) + (in_step ? 0 : own_norm ? 1 : 2);
     Tensor between;
-    if (parts) between = at::empty({parts, rows * L.d}, opt);
+    if (parts || later) between = at::empty({parts * one + (later ? 2 * (one + rows * L.H) : 0)}, opt);
     char* room = static_cast<char*>(ptr(between));
     void *gate = nullptr, *o = ptr(r.n), *log_f = nullptr;
-    const auto take = [&] { void* const p = room; room += rows * L.d * 2; return p; };
-    if (!norm_in_step) o = take();
-    if (!norm_in_step || !in_step) gate = take();
+    const auto take = [&] { void* const p = room; room += one * 2; return p; };
+    if (own_norm) o = take();
+    if (own_norm || !in_step) gate = take();
     if (!in_step) {
         log_f = take();
         check(api.layer_up_fwd(&ud, ptr(r.y), ptr(P[6]), ptr(P[7]), nullptr, log_f, gate, s), "hdla_layer_up_fwd");
@@ -607,10 +612,19 @@ void layer_step(const Tensor* P, const LayerCfg& f, const LayerCols& L, const hd
     Tensor state;
     if (h0.defined()) state = h0.to(at::kFloat).contiguous();
     if (want_ht) r.ht = at::empty({N, L.H, L.D, L.D}, opt.dtype(at::kFloat));
-    check(api.layer_step(&pd, in_step ? &ud : nullptr, norm_in_step ? &nd : nullptr, (int32_t)T, ptr(r.y), in_step ? ptr(P[6]) : nullptr,
-                         in_step ? ptr(P[7]) : nullptr, log_f, gate, norm_in_step ? ptr(P[8]) : nullptr, fptr(state), o, fptr(r.ht), s),
+    float* const gated = later ? reinterpret_cast<float*>(room) : nullptr;
+    check(api.layer_step(&pd, in_step ? &ud : nullptr, own_norm ? nullptr : &nd, (int32_t)T, ptr(r.y), in_step ? ptr(P[6]) : nullptr,
+                         in_step ? ptr(P[7]) : nullptr, log_f, gate, norm_in_step ? ptr(P[8]) : nullptr, fptr(state), o, gated, fptr(r.ht), s),
           "hdla_layer_step");
-    if (!norm_in_step) check(api.normalize_fwd(&nd, o, ptr(P[8]), gate, ptr(r.n), s), "hdla_normalize_fwd");
+    if (later) {
+        const Tensor &w = P[9];
+        r.out = at::empty({rows, L.d}, opt);
+        check(api.rows_gemm_norm((int32_t)rows, (int32_t)L.d, (int32_t)L.d, gated, (int32_t)L.H, &nd, ptr(P[8]), ptr(w), w.stride(0), ptr(r.out),
+                                 r.out.stride(0), s), "hdla_rows_gemm_norm");
+        return;
+    }
+    if (own_norm) check(api.normalize_fwd(&nd, o, ptr(P[8]), gate, ptr(r.n), s), "hdla_normalize_fwd");
+    r.out = project(r.n, P[9]);
 }
 
 // params: wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo; r.w gathered; keep: a backward pass follows
@@ -623,7 +637,7 @@ void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, const T
     const hdla_pre_dims pd = pre_dims(L, f, rows);
     if (!chunked && T < RECURRENT_BELOW) {
         layer_step(P, f, L, pd, T, h0, want_ht, r);
-        r.out = project(r.n, P[9]).view({B, T, d});
+        r.out = r.out.view({B, T, d});
         return;
     }
     ChunkIn& in = r.op;
@@ -877,6 +891,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HDLA_FN(recurrent_fwd) HDLA_FN(param_recurrent_fwd) HDLA_FN(normalize_fwd) HDLA_FN(normalize_bwd)
     HDLA_FN(normalize_workspace_bytes) HDLA_FN(layer_pre_fwd) HDLA_FN(layer_pre_bwd) HDLA_FN(layer_up_fwd) HDLA_FN(layer_down)
     HDLA_FN(layer_up_wgrad) HDLA_FN(layer_up_wgrad_workspace_bytes) HDLA_FN(rows_gemm) HDLA_FN(sum_partials) HDLA_FN(stack_rows) HDLA_FN(layer_step)
+    HDLA_FN(rows_gemm_norm)
 #undef HDLA_FN
     Py_INCREF(a[1]);
     Py_XDECREF(error_class);

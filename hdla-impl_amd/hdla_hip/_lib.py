@@ -148,7 +148,9 @@ def load():
     lib.hdla_layer_up_wgrad_workspace_bytes.restype = ctypes.c_size_t
     lib.hdla_layer_up_wgrad_workspace_bytes.argtypes = [UF]
     lib.hdla_layer_step.restype = ctypes.c_int
-    lib.hdla_layer_step.argtypes = [PF, UF, NF, ctypes.c_int32] + [P] * 10
+    lib.hdla_layer_step.argtypes = [PF, UF, NF, ctypes.c_int32] + [P] * 11
+    lib.hdla_rows_gemm_norm.restype = ctypes.c_int
+    lib.hdla_rows_gemm_norm.argtypes = [ctypes.c_int32] * 3 + [P, ctypes.c_int32, NF, P, P, ctypes.c_int64, P, ctypes.c_int64, P]
     lib.hdla_rows_gemm.restype = ctypes.c_int
     lib.hdla_rows_gemm.argtypes = [ctypes.c_int32] * 3 + [P, ctypes.c_int64, P, ctypes.c_int64, P, ctypes.c_int64, P]
     lib.hdla_sum_partials.restype = ctypes.c_int

@@ -344,16 +344,24 @@ size_t hdla_layer_up_wgrad_workspace_bytes(const hdla_up_dims* dims);
  * norm given (one group a head: G = H, E = D, with a gate): hdla_normalize_fwd as well, o is the normalised and gated output and
  * weight its weight [H D] or NULL.
  * up given (T = 1): hdla_layer_up_fwd as well, wf and wg are its weights; log_f is not used and gate, unless NULL, written.
- * Without it log_f and (with norm) gate [rows, H, D] are inputs. */
+ * Without it log_f and (with norm) gate [rows, H, D] are inputs.
+ * gated given: the norm is over all channels (norm: G = 1, E = H D) and left to hdla_rows_gemm_norm.  gated [rows H D + rows H] receives
+ * o sigmoid(gate) and then each head's part of the row's sum of squares (of the gated o, or with gate_pos 2 of o itself); o and weight
+ * are not used. */
 int hdla_layer_step(const hdla_pre_dims* pre, const hdla_up_dims* up, const hdla_norm_dims* norm, int32_t T, const void* y,
                     const void* wf, const void* wg, const void* log_f, void* gate, const void* weight, const float* h0, void* o,
-                    float* ht, void* stream);
+                    float* gated, float* ht, void* stream);
 
 /* y [M, N] = x [M, K] w [N, K]^T in bf16 for M <= 64 rows and K a multiple of 32 (the large projections of a decode step;
  * nn.Linear without bias).  ldx, ldw: row strides in elements, multiples of 8; ldy: a multiple of 4; x, w 16-byte, y 8-byte
  * aligned. */
 int hdla_rows_gemm(int32_t M, int32_t N, int32_t K, const void* x, int64_t ldx, const void* w, int64_t ldw, void* y,
                    int64_t ldy, void* stream);
+
+/* hdla_rows_gemm for M <= 16 rows whose x is the norm of what hdla_layer_step left in gated (`parts` sums a row): x = gated c / sqrt(K) /
+ * sqrt(sum / K + eps) * weight [K], rounded to bf16 (weight NULL: ones).  gated and weight 16-byte aligned. */
+int hdla_rows_gemm_norm(int32_t M, int32_t N, int32_t K, const float* gated, int32_t parts, const hdla_norm_dims* norm, const void* weight,
+                        const void* w, int64_t ldw, void* y, int64_t ldy, void* stream);
 
 /* Measurement aid; it has no counterpart in the reference.  One launch of a kernel that reads `n_read` (0..3)
  * buffers and writes `n_write` (0..2) buffers of `bytes` bytes each (a multiple of 16; every pointer 16-byte

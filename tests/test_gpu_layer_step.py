@@ -58,7 +58,7 @@ def test_layer_step(D, N, T, H, norm_q, norm_v, gate_pos, weight, state):
         o, ht, g = torch.full((rows + 1, H, D), 7., device=DEV, dtype=torch.bfloat16), torch.empty_like(rht), new(rows, H, D)
         assert lib.hdla_layer_step(ref(pre), ref(up) if with_up else None, ref(nd) if norm else None, T, P(y), P(wf) if with_up else None,
                                    P(wg) if with_up else None, None if with_up else P(log_f), P(g) if with_up else P(gate), P(w) if norm else None,
-                                   P(h0), P(o), P(ht) if want_ht else None, st) == 0
+                                   P(h0), P(o), None, P(ht) if want_ht else None, st) == 0
         assert bool((o[rows:] == 7.).all())
         assert _rel(o[:rows], rn if norm else ro) <= tol
         assert not want_ht or _rel(ht, rht) <= tol
@@ -71,14 +71,45 @@ def test_layer_step(D, N, T, H, norm_q, norm_v, gate_pos, weight, state):
     if T == 1:
         run(True, True)
         run(False, True)
-    bad = lambda pre, up, nd, T, y=P(y): lib.hdla_layer_step(pre, up, nd, T, y, P(wf), P(wg), P(log_f), P(gate), None, None, P(ro), None, st)
+    bad = lambda pre, up, nd, T, y=P(y): lib.hdla_layer_step(pre, up, nd, T, y, P(wf), P(wg), P(log_f), P(gate), None, None, P(ro), None, None, st)
     assert bad(ref(pre), None, None, 0) == -2 and bad(ref(pre), None, None, rows + 1) == -2 and bad(ref(pre), ref(up), None, 2) == -2
     assert bad(ref(pre), None, ref(_lib.HdlaNormDims(rows, 2 * H, D // 2, _lib.dtype_code(torch.bfloat16), _lib.dtype_code(torch.bfloat16), 1, 1., 1e-5)), T) == -2
     assert bad(ref(pre), None, None, T, None) != 0 and bad(ref(pre), None, None, T, ctypes.c_void_p(y.data_ptr() + 2)) != 0
 
 
+@pytest.mark.parametrize("gate_pos", [1, 2])
+@pytest.mark.parametrize("D,rows,T,H,N,weight", [(64, 1, 1, 2, 20, "bf16"), (64, 16, 1, 9, 200, "fp32"), (128, 5, 1, 16, 2048, "bf16"), (64, 14, 7, 4, 16, None),
+                                                (128, 16, 2, 4, 100, "bf16")])
+def test_norm_left_to_the_projection(D, rows, T, H, N, weight, gate_pos):
+    """hdla_layer_step with `gated`, then hdla_rows_gemm_norm, against step, norm and product."""
+    lib, st, ref = _lib.load(), _lib.current_stream(DEV), ctypes.byref
+    d = H * D
+    ld = (3 * d + H + 7) // 8 * 8
+    y, log_f, gate, w = _rn(1, rows, ld).bfloat16(), -_rn(2, rows, d).abs().bfloat16(), _rn(3, rows, d).bfloat16(), _rn(4, N, d).bfloat16()
+    wn = None if weight is None else (1. + .1 * _rn(5, d)).to(torch.bfloat16 if weight == "bf16" else torch.float32)
+    h0 = _rn(6, rows // T, H, D, D)
+    bf = _lib.dtype_code(torch.bfloat16)
+    pre = _lib.HdlaPreDims(rows, H, D, bf, ld, 0, d, 2 * d, 3 * d, 0, 1, 0, 1.0, 1e-5, 0)
+    nd = _lib.HdlaNormDims(rows, 1, d, bf, _lib.dtype_code(torch.float32 if weight == "fp32" else torch.bfloat16), gate_pos, d ** .5, 1e-5)
+    o, n = torch.empty(rows, d, device=DEV, dtype=torch.bfloat16), torch.empty(rows, d, device=DEV, dtype=torch.bfloat16)
+    step = lambda norm, out, gated: lib.hdla_layer_step(ref(pre), None, norm, T, P(y), None, None, P(log_f), P(gate), None, P(h0), out, gated, None, st)
+    assert step(None, P(o), None) == 0
+    assert lib.hdla_normalize_fwd(ref(nd), P(o), P(wn), P(gate), P(n), st) == 0
+    want = n.double() @ w.double().t()
+    gated = torch.full((rows * (d + H) + 4,), 7., device=DEV)
+    assert step(ref(nd), None, P(gated)) == 0
+    assert bool((gated[rows * (d + H):] == 7.).all())
+    out = torch.full((rows + 1, N + 4), 7., device=DEV, dtype=torch.bfloat16)
+    run = lambda M, K=d, nd=nd: lib.hdla_rows_gemm_norm(M, N, K, P(gated), H, ref(nd), P(wn), P(w), d, P(out), N + 4, st)
+    assert run(rows) == 0
+    # one rounding of the result: at most 2^-8 of each (a third of that in the mean of many, but N = 20 are few)
+    assert _rel(out[:rows, :N], want) <= 2 ** -8
+    assert bool((out[rows:] == 7.).all() and (out[:, N:] == 7.).all())
+    assert run(17) == -2 and run(rows, d - 32) == -2 and step(None, None, P(gated)) != 0
+
+
 @pytest.mark.parametrize("norm", ["rmsnorm", "grouprmsnorm"])
-@pytest.mark.parametrize("B,T,H", [(3, 1, 4), (65, 1, 2), (2, 8, 4), (2, 9, 4)])
+@pytest.mark.parametrize("B,T,H", [(3, 1, 4), (17, 1, 4), (65, 1, 2), (2, 8, 4), (3, 8, 4), (2, 9, 4), (2, 1, 34)])
 def test_layer_routes(B, T, H, norm):
     """Both sides of the lines that the native call chooses by (tokens, rows, the norm's groups) next to the layer's Python
     code, and replays of a captured step."""
