@@ -57,6 +57,12 @@ def interface_bytes(kernel, pass_, K, V, es, gs, frac_seg=0.0):
     HC = DHC = K * V * es
     DVN = 32 * V * es
     inputs = 2 * 16 * K * es + 16 * K * gs + 2 * 32 * K * es + 16 * V * es          # q,k,gk,a,b,v
+    if pass_ == 0 and es == 2:          # (2-byte elements: u is formed in the scan, from three tile pairs the prep kernel leaves, and v)
+        TMF, VR = 1536 * es, 16 * V * es
+        if kernel == "prep":
+            return inputs - VR + W + KGT + BGT + EGL + QG + AQK + AQB + TMF
+        if kernel == "scan_fwd":
+            return W + KGT + BGT + EGL + QG + AQK + AQB + TMF + VR + 16 * V * es
     if kernel == "prep":
         out = W + UT + KGT + BGT + VTT + EGL + ((QG + AQK + AQB) if pass_ == 0 else (AQBT + QGT + TM))
         return inputs + out
@@ -170,16 +176,19 @@ def measured_traffic(workload, kernel_key, K, V):
             if fused_mode is not None and k.startswith("fused_kernel<") and targs[2:] == [str(K), str(V), fused_mode, "false"]:
                 return rec["hbm_bytes_per_launch"]
             continue
+        # scan_out<K, V, NWC, KEPT> (the forward pass's scan), scan_grad<K, V, NWC> (both of the backward pass)
+        if name in ("scan_fwd", "scan_pair"):
+            if k.startswith("scan_out_kernel<" if name == "scan_fwd" else "scan_grad_kernel<") and targs[:2] == [str(K), str(V)] and \
+                    targs[3:] != ["true"]:
+                return rec["hbm_bytes_per_launch"]
+            continue
         if not k.startswith(name + "_kernel<"):
             continue
-        # prep<T, GKF32, K, V, MODE (0 forward, 1 backward, 2 kept forward), HD>, scan_fwd<T, K, V, NWC, WRITE_O>, scan_pair<T, K, V, NWC>,
-        # chunk_grad<T, GKF32, K, V, HD>, recurrent<T, K, V, BV, HD>
+        # prep<T, GKF32, K, V, MODE (0 forward, 1 backward, 2 kept forward), HD>, chunk_grad<T, GKF32, K, V, HD>, recurrent<T, K, V, BV, HD>
         kv = targs[2:4] if name in ("prep", "chunk_grad") else targs[1:3]
         if kv != [str(K), str(V)]:
             continue
         if name == "prep" and (targs[4] != ("1" if pass_ == "bwd" else "0") or targs[5:] == ["true"]):
-            continue
-        if name == "scan_fwd" and (targs[4] == "true") != (pass_ == "fwd"):
             continue
         if name in ("chunk_grad", "recurrent") and targs[4:] == ["true"]:
             continue
