@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-#define HDLA_VERSION 204
+#define HDLA_VERSION 205
 
 enum { HDLA_BF16 = 0, HDLA_FP32 = 1 };
 
@@ -68,9 +68,10 @@ enum {
  * split over workgroups.  HDLA_ROUTE_FUSED (bf16 inputs, K = V = 64): the preparation runs inside the scan kernels'
  * workgroups and reaches the scan through LDS; a sequence is cut into `segments` time segments whose affine maps are
  * chained afterwards, so that few (sequence, head) pairs still fill the device.  HDLA_ROUTE_AUTO takes the fused route
- * where it is built, except for few short sequences (at most 64 pairs of a sequence and a head, at most 31 chunks a sequence on
- * average, in a backward pass at least 6, no segments asked for), where the classic kernels are through sooner, unless a call is given
- * a boundary or record buffer (hdla_record_bytes is 0 where the backward pass takes the classic kernels).  Both routes compute the same function; they differ in rounding only where segments > 1. */
+ * where it is built, except for few short sequences (at most 64 pairs of a sequence and a head, at most 31 chunks a
+ * sequence on average, in a backward pass at least 6, no segments asked for), where the classic kernels are through
+ * sooner, unless a call is given a boundary or record buffer (hdla_record_bytes is 0 where the backward pass takes the
+ * classic kernels).  Both routes compute the same function; they differ in rounding only where segments > 1. */
 enum { HDLA_ROUTE_AUTO = 0, HDLA_ROUTE_CLASSIC = 1, HDLA_ROUTE_FUSED = 2 };
 #define HDLA_FUSED_ABORTED 0x48444c00
 
