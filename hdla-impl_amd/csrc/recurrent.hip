@@ -10,6 +10,21 @@
 // (a^T S and q^T S) run as in-lane partial sums, two cross-lane butterfly steps and one LDS exchange between
 // the four wavefronts.
 //
+// What bounds it: the state's way from and to HBM (256 sequences of 32 heads, K = V = 128, one token: 1.09 GB), and where the state is
+// in a cache the chain of a token: its values, the LDS fill, two reductions.
+//   - A token's values are requested before the previous token's arithmetic, the first token's before the state: requests complete in
+//     order, so behind the state they would be waited for as long.  Requested at the token's begin (and converted beside the
+//     load) it was, in us: 4 sequences of 8 heads, 128 x 128, 16 tokens 34.6 -> 30.2; 8 of 16, 64 x 64, 8 tokens 15.4 -> 13.3;
+//     16 of 16, 128 x 128, one token 7.9 -> 7.5.
+//   - The column blocks of a head are neighbours in launch order: they are in flight together and memory sees whole rows.  As the second
+//     dimension of the grid they ran thousands of workgroups apart: 256 sequences of 32 heads 211 -> 186, 128 105 -> 92, 64 51 -> 47,
+//     24 of 16 heads 8.8 -> 7.9.  Below 256 workgroups the order it had is kept: there the blocks of a head meet in the
+//     same L2 where the number of heads is a multiple of 8, and the token's values are what is waited for (4 of 16 heads with beta
+//     5.2 against 5.5).  The blocks of a head on one XCD on large grids: 195 to 199 for the 186.
+//   - One branch around the state's loads, not one each: 108 instead of 94 registers a lane at K = 128, four waves a SIMD instead of
+//     five, and still 186 instead of 192 (without the branch) at 256 sequences; held to five waves it spills.  All 128 columns in one
+//     workgroup: 196.
+//
 // HD mode (p.beta given) forms the rank terms of the HDLA layer per token from (beta, k, gk) instead of reading
 // them (HRDPLR/hdla_custom.py:19-43): with f = exp(gk) and s = sum_c k_c^2 f_c,
 //     a_1 = -beta k,  a_2 = beta k (beta s - f),  b_1 = f k,  b_2 = k,
@@ -19,13 +34,19 @@
 
 namespace hdla {
 
-__device__ __forceinline__ float ld_as_float(const bf16* p) { return bf2f(p->x); }
-__device__ __forceinline__ float ld_as_float(const float* p) { return *p; }
+__device__ __forceinline__ float as_float(bf16 x) { return bf2f(x.x); }
+__device__ __forceinline__ float as_float(float x) { return x; }
 __device__ __forceinline__ float round_as(const bf16*, float x) { return bf2f(f2bf(x)); }
 __device__ __forceinline__ float round_as(const float*, float x) { return x; }
-__device__ __forceinline__ float ld_gk1(const void* base, int64_t off, int is_f32) {
-    return is_f32 ? reinterpret_cast<const float*>(base)[off] : bf2f(reinterpret_cast<const bf16*>(base)[off].x);
-}
+
+// A token's values for one thread (channel tid, value column tid) as they lie in memory: converted where they are used.  A conversion
+// beside a load is a wait for it in the conditional block that the load stands in.
+template <typename T, bool HD>
+struct TokenValues {
+    T q, k, v, b0;       // b0: beta with HD
+    T a0, a1, b1;        // without HD
+    uint32_t gk;         // the bits, fp32's or in the low half bf16's
+};
 
 template <typename T, int K, int V, int BV, bool HD>
 __global__ __launch_bounds__(256) void recurrent_kernel(RecurrentArgs<T> p) {
@@ -37,7 +58,9 @@ __global__ __launch_bounds__(256) void recurrent_kernel(RecurrentArgs<T> p) {
     __shared__ float sq[K], sk[K], seg[K], sa[2][K], sb[2][K], sv[BV];
     __shared__ float red[4][3][BV];
 
-    const int nh = blockIdx.x, vb = blockIdx.y;
+    constexpr int NV = V / BV;
+    const bool apart = NV > 1 && gridDim.y > 1;
+    const int nh = apart ? blockIdx.x : blockIdx.x / NV, vb = apart ? blockIdx.y : blockIdx.x % NV;
     const int n = nh / p.H, h = nh - n * p.H;
     const int H = p.H;
     const int tid = threadIdx.x, cg = tid % CG, rg = tid / CG, wave = tid >> 6, lane = tid & 63;
@@ -46,53 +69,70 @@ __global__ __launch_bounds__(256) void recurrent_kernel(RecurrentArgs<T> p) {
     else { bos = (int64_t)n * p.T_; eos = bos + p.T_; }
     const int len = (int)(eos - bos);
 
+    auto request = [&](int64_t t) __attribute__((always_inline)) {
+        TokenValues<T, HD> x{};
+        if (tid < K) {
+            const int64_t off = (t * H + h) * K + tid;
+            x.q = p.q[off];
+            x.k = p.k[off];
+            x.gk = p.gk_f32 ? reinterpret_cast<const uint32_t*>(p.gk)[off] : reinterpret_cast<const uint16_t*>(p.gk)[off];
+            if constexpr (HD) {
+                x.b0 = p.beta[t * H + h];
+            } else {
+                const int64_t off0 = ((t * RANK + 0) * H + h) * K + tid, off1 = ((t * RANK + 1) * H + h) * K + tid;
+                x.a0 = p.a[off0];
+                x.a1 = p.a[off1];
+                x.b0 = p.b[off0];
+                x.b1 = p.b[off1];
+            }
+        }
+        if (tid < BV) x.v = p.v[(t * H + h) * V + vb * BV + tid];
+        return x;
+    };
+    TokenValues<T, HD> raw{};
+    if (len > 0) raw = request(p.reverse ? eos - 1 : bos);
     const int64_t sbase = (int64_t)nh * K * V + vb * BV + 4 * cg;
     f32x4 S[RPT];
+    if (p.h0) {
 #pragma unroll
-    for (int j = 0; j < RPT; ++j)
-        S[j] = p.h0 ? __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p.h0 + sbase + (int64_t)(rg + RG * j) * V)) : zero4();
+        for (int j = 0; j < RPT; ++j) S[j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p.h0 + sbase + (int64_t)(rg + RG * j) * V));
+    } else {
+#pragma unroll
+        for (int j = 0; j < RPT; ++j) S[j] = zero4();
+    }
 
     for (int step = 0; step < len; ++step) {
         const int64_t t = p.reverse ? (eos - 1 - step) : (bos + step);
         __syncthreads();
+        const float kk = as_float(raw.k), f = exp_t<T>(p.gk_f32 ? __builtin_bit_cast(float, raw.gk) : bf2f((uint16_t)raw.gk));
         if constexpr (HD) {
-            const int64_t off = (t * H + h) * K + tid;
-            float kk = 0.f, f = 0.f;
-            if (tid < K) {
-                kk = ld_as_float(p.k + off);
-                f = exp_t<T>(ld_gk1(p.gk, off, p.gk_f32));
-                sq[tid] = ld_as_float(p.q + off) * p.scale;
-            }
-            float part = kk * kk * f;
+            float part = tid < K ? kk * kk * f : 0.f;
 #pragma unroll
             for (int o = 1; o < 64; o <<= 1) part += __shfl_xor(part, o);
             if (lane == 0) red[wave][0][0] = part;
             __syncthreads();
-            if (tid < K) {
+        }
+        if (tid < K) {
+            sq[tid] = as_float(raw.q) * p.scale;
+            sk[tid] = kk;
+            seg[tid] = f;
+            if constexpr (HD) {
                 const float s = red[0][0][0] + red[1][0][0] + red[2][0][0] + red[3][0][0];
-                const float beta = ld_as_float(p.beta + t * H + h);
-                sk[tid] = kk;
-                seg[tid] = f;
+                const float beta = as_float(raw.b0);
                 sa[0][tid] = round_as(p.k, -beta * kk);
                 sa[1][tid] = round_as(p.k, (beta * s - f) * beta * kk);
                 sb[0][tid] = round_as(p.k, f * kk);
                 sb[1][tid] = kk;
-            }
-        } else {
-            for (int idx = tid; idx < K; idx += 256) {
-                const int64_t off = (t * H + h) * K + idx;
-                const int64_t off0 = ((t * RANK + 0) * H + h) * K + idx, off1 = ((t * RANK + 1) * H + h) * K + idx;
-                sq[idx] = ld_as_float(p.q + off) * p.scale;
-                sk[idx] = ld_as_float(p.k + off);
-                seg[idx] = exp_t<T>(ld_gk1(p.gk, off, p.gk_f32));
-                sa[0][idx] = ld_as_float(p.a + off0);
-                sa[1][idx] = ld_as_float(p.a + off1);
-                sb[0][idx] = ld_as_float(p.b + off0);
-                sb[1][idx] = ld_as_float(p.b + off1);
+            } else {
+                sa[0][tid] = as_float(raw.a0);
+                sa[1][tid] = as_float(raw.a1);
+                sb[0][tid] = as_float(raw.b0);
+                sb[1][tid] = as_float(raw.b1);
             }
         }
-        if (tid < BV) sv[tid] = ld_as_float(p.v + (t * H + h) * V + vb * BV + tid);
+        if (tid < BV) sv[tid] = as_float(raw.v);
         __syncthreads();
+        if (step + 1 < len) raw = request(p.reverse ? t - 1 : t + 1);
 
         // a_r^T S over the block's rows
         f32x4 p0 = zero4(), p1 = zero4();
@@ -148,7 +188,11 @@ __global__ __launch_bounds__(256) void recurrent_kernel(RecurrentArgs<T> p) {
 template <typename T, int K, int V>
 static hipError_t launch_recurrent_kv(const RecurrentArgs<T>& a, hipStream_t stream) {
     constexpr int BV = 64;
-    dim3 grid(a.N * a.H, V / BV), block(256);
+    // A head's column blocks next to each other in launch order, except on grids that do not give every CU a workgroup (and where
+    // the grid would reach 2^32 threads).  See above.
+    const int64_t blocks = (int64_t)a.N * a.H * (V / BV);
+    const bool apart = blocks < 256 || blocks >= (1 << 24);
+    dim3 grid = apart ? dim3(a.N * a.H, V / BV) : dim3((unsigned)blocks), block(256);
     if (a.beta) hipLaunchKernelGGL((recurrent_kernel<T, K, V, BV, true>), grid, block, 0, stream, a);
     else hipLaunchKernelGGL((recurrent_kernel<T, K, V, BV, false>), grid, block, 0, stream, a);
     return hipGetLastError();
