@@ -56,9 +56,12 @@ bool few_short_sequences(const hdla_dims* d, int least = SHORT_MIN_CHUNKS) {
     const long long chunks = ((d->T + CHUNK - 1) / CHUNK) / (d->cu_seqlens ? std::max(d->N, 1) : 1);
     return (long long)d->N * d->H <= SHORT_MAX_LANES && chunks >= least && chunks <= SHORT_MAX_CHUNKS;
 }
-// (The forward pass alone costs the same on both routes below six chunks; it takes the classic kernels there too, so that a prompt cut into
-// pieces comes out in the bits of the whole one.)
-int short_least(int pass) { return pass == HDLA_PASS_FWD ? 1 : SHORT_MIN_CHUNKS; }
+// The forward pass alone only where the fused route would cut a sequence into segments: below, its workgroup walks the whole
+// sequence and a prompt cut into pieces at chunk boundaries comes out in the bits of the whole one, which a line among these lengths would
+// end; and up to four chunks, one round in one launch, it is the sooner one.  Measured, us on the device, fused / classic:
+// 12 lanes of 2 chunks 8.6/10.4, 4 10.1/11.4, 8 16.8/13.4, 15 28.9/16.7, 30 34/24; 64 lanes of 2 8.8/11.3, 8 17.2/16.6, 15 29/23, 30 38/31.
+constexpr int SHORT_MIN_CHUNKS_FWD = 2 * FUSED_MIN_SEGMENT_CHUNKS;
+int short_least(int pass) { return pass == HDLA_PASS_FWD ? SHORT_MIN_CHUNKS_FWD : SHORT_MIN_CHUNKS; }
 // whether the plain entry points take the fused route for these dimensions; HDLA_ROUTE_FUSED on another shape is an error.
 // with_boundary: a boundary (or record) buffer is given: then it is the fused route's.
 int pick_route(const hdla_dims* d, int pass, bool with_boundary, bool& fused) {

@@ -69,8 +69,8 @@ enum {
  * workgroups and reaches the scan through LDS; a sequence is cut into `segments` time segments whose affine maps are
  * chained afterwards, so that few (sequence, head) pairs still fill the device.  HDLA_ROUTE_AUTO takes the fused route
  * where it is built, except for few short sequences (at most 64 pairs of a sequence and a head, at most 31 chunks a
- * sequence on average, in a backward pass at least 6, no segments asked for), where the classic kernels are through
- * sooner, unless a call is given a boundary or record buffer (hdla_record_bytes is 0 where the backward pass takes the
+ * sequence on average, at least 16 in a forward and 6 in a backward pass, no segments asked for), where the classic
+ * kernels are through sooner, unless a call is given a boundary or record buffer (hdla_record_bytes is 0 where the backward pass takes the
  * classic kernels).  Both routes compute the same function; they differ in rounding only where segments > 1. */
 enum { HDLA_ROUTE_AUTO = 0, HDLA_ROUTE_CLASSIC = 1, HDLA_ROUTE_FUSED = 2 };
 #define HDLA_FUSED_ABORTED 0x48444c00

@@ -57,3 +57,26 @@ def test_the_same_results_as_on_the_fused_route(form, gk_dtype, B, T, H, cu, sta
         assert x.dtype == y.dtype and torch.isfinite(x.float()).all(), i
         # both are within 5e-3 (outputs) and 1e-2 (gradients) of exact arithmetic, and share most of their roundings
         assert O.rel_l2(x, y) <= 6e-3, (i, O.rel_l2(x, y))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H", [(1, 3), (4, 16)])
+@pytest.mark.parametrize("T,route", [(16, "fused"), (33, "fused"), (80, "fused"), (240, "fused"), (241, "classic"), (496, "classic"), (497, "fused")])
+def test_the_forward_pass_alone(B, H, T, route, monkeypatch):
+    """Which route a forward pass is on shows in its bits; below 16 chunks they are also those of the prompt in pieces."""
+    inp = make_inputs(970 + T, B, T, H, 64, 64, gk_div=4.0)
+    leaves = [t.bfloat16().to(DEV) for t in (inp.q, inp.k, inp.v, inp.a, inp.b, inp.gk)]
+
+    def run(h0, first=0, last=T):
+        part = [t[:, first * (t.shape[1] // T):last * (t.shape[1] // T)].contiguous() for t in leaves]      # (a, b: two rows a token)
+        return chunk_hrdplr_delta_rule(*part, 2, scale=0.7, initial_state=h0, output_final_state=True)
+
+    with torch.no_grad():
+        o, ht = run(inp.h0.to(DEV))
+        if 16 < T <= 240:
+            o_1, h = run(inp.h0.to(DEV), 0, 16)
+            o_2, h = run(h, 16)
+            assert torch.equal(o, torch.cat([o_1, o_2], 1)) and torch.equal(ht, h)
+        monkeypatch.setenv("HDLA_HIP_ROUTE", route)
+        o_r, ht_r = run(inp.h0.to(DEV))
+    assert torch.equal(o, o_r) and torch.equal(ht, ht_r)
