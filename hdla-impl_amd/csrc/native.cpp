@@ -578,8 +578,8 @@ Tensor project(const Tensor& x, const Tensor& w) {
 // everything between x and the output; what the backward pass needs of it
 struct LayerFwd { Tensor x, w, y, f, g, o, n, out, ht, boundary; ChunkIn op; hdla_dims dims; };
 
-// A few tokens: what is between the projections in one to three launches, without the tensors that the steps would hand on.  (Many
-// tokens are better off with what does not depend on the state done for all of them at once.)  One token after a cached state, us a
+// A few tokens: what is between the projections in one to three launches, without the tensors that the steps would hand on (see
+// in_few_launches).  One token after a cached state, us a
 // call, as six launches and eleven tensors -> as this (batch x channels, heads): 1 x 512, 8 37.8 -> 19.7, 16 x 2048, 16 36.9 -> 24.3,
 // 25 x 4096, 32 67.7 -> 54.5, 256 x 1024, 16 71 -> 57, 256 x 4096, 32 281 -> 249.  The low-rank products in the same launch or in
 // one before it (and the norm in one of its own): 23.9 / 26.8, 25.2 / 27.0, 54.5 / 55.9, 57 / 60, 249 / 252; the other way round only at 256 x 2048, 32: 85.3 / 84.5.
@@ -591,7 +591,8 @@ void layer_step(const Tensor* P, const LayerCfg& f, const LayerCols& L, const hd
     const bool in_step = T == 1, norm_in_step = f.groups == L.H;
     // A norm over all channels of at most 16 rows: formed where the projection reads it, by every workgroup of the projection for itself.
     // A launch less, which the host is glad of, but what the workgroups read grows with the square of the channels.  us a call, in a launch
-    // of its own / here: 1 x 512 24.1 / 19.7, 16 x 1024 24.9 / 19.7, 3 x 2048 24.5 / 21.9, 16 x 2048 25.2 / 24.3, 1 x 4096 39.3 / 41.2.
+    // of its own / here: 1 x 512 24.1 / 19.7, 16 x 1024 24.9 / 19.7, 3 x 2048 24.5 / 21.9, 16 x 2048 25.2 / 24.3; wider ones on the
+    // device: 3 x 2560, 40 23.4 / 24.6 (the host 25.3 / 24.7), 3 x 3072, 48 26.6 / 28.6, 3 x 3584, 28 33.1 / 35.3, 1 x 4096, 32 39.2 / 41.8.
     const bool later = !norm_in_step && f.groups == 1 && rows <= 16 && L.d <= 2048, own_norm = !norm_in_step && !later;
     if (!later) r.n = at::empty({rows, L.d}, opt);
     const hdla_up_dims ud = up_dims(L, rows);
@@ -627,6 +628,17 @@ void layer_step(const Tensor* P, const LayerCfg& f, const LayerCols& L, const hd
     r.out = project(r.n, P[9]);
 }
 
+// Whether layer_step takes the tokens of a token-serial call.  It works a head's tokens off one after the other; with several tokens of
+// many sequences the steps are the faster, which do what does not depend on the state for all tokens at once.  One token: always.  us on the device, steps / here
+// (sequences x tokens, channels, heads).  With the norm in layer_step's launch: 256 x 2 4096, 32 304/300; 48 x 8 1024, 16 56/52; 128 x 6 74.7/72.7;
+// 128 x 8 84/84; 256 x 8 134/139; 64 x 3 2048, 16 74/71; 48 x 8 95/101; 256 x 8 315/371; 24 x 8 4096, 32 127/128; 64 x 8 217/232; 256 x 8 698/815.  With it in a
+// launch of its own: 64 x 3 1024, 16 44.7/41.7; 48 x 8 56.7/57.8 (the host 72/61); 128 x 8 84/89; 24 x 8 2048, 32 63.0/64.4; 64 x 8 95/99; 16 x 8 4096, 32 96/97;
+// 64 x 8 217/240; 256 x 8 695/809; 256 x 2 2048, 16 150/155.
+bool in_few_launches(int64_t rows, int64_t T, int64_t d, bool norm_in_step) {
+    if (T == 1 || (T == 2 && norm_in_step)) return true;
+    return rows * d <= (norm_in_step ? 3 << 18 : 3 << 17);
+}
+
 // params: wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo; r.w gathered; keep: a backward pass follows
 void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, const Tensor& h0, bool want_ht, bool chunked, bool keep, LayerFwd& r) {
     const int64_t B = x3.size(0), T = x3.size(1), d = x3.size(2), rows = B * T;
@@ -635,7 +647,7 @@ void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, const T
     r.x = x3.contiguous().view({rows, d});
     r.y = project(r.x, r.w);
     const hdla_pre_dims pd = pre_dims(L, f, rows);
-    if (!chunked && T < RECURRENT_BELOW) {
+    if (!chunked && T < RECURRENT_BELOW && in_few_launches(rows, T, d, f.groups == f.H)) {
         layer_step(P, f, L, pd, T, h0, want_ht, r);
         r.out = r.out.view({B, T, d});
         return;

@@ -147,3 +147,36 @@ def test_layer_routes(B, T, H, norm):
             g.replay()
             torch.cuda.synchronize()
             assert torch.equal(c, want) and torch.equal(sc, ws)
+
+
+@pytest.mark.parametrize("norm", ["rmsnorm", "grouprmsnorm"])
+@pytest.mark.parametrize("B,T,H,few", [(192, 1, 32, (True, True)), (192, 2, 16, (True, True)), (193, 2, 16, (True, False)),
+                                       (192, 8, 4, (True, True)), (193, 8, 4, (True, False)), (192, 8, 8, (True, False)), (193, 8, 8, (False, False))])
+def test_several_tokens_of_many_sequences(B, T, H, few, norm):
+    """Both sides of the line by which the native call takes several tokens of many sequences in few launches or as steps (few: with the norm
+    in the same launch, in one of its own): which of the two runs shows in the tensors it holds, and both agree with the Python code."""
+    from hdla_hip.layer import HDLA_Custom, RecurrentCache
+    torch.manual_seed(4)
+    d = 64 * H
+    with torch.device("cuda"):
+        m = HDLA_Custom(d, H, token_mixer_init_type=2, rescale_type=0, token_mixer_norm_type=norm).to(torch.bfloat16).eval()
+    x, s0 = _rn(9, B, T, d).bfloat16(), _rn(10, B, H, 64, 64)
+
+    def step():
+        cache = RecurrentCache()
+        cache.update(recurrent_state=[s0], layer_idx=0, offset=T)
+        return m(x, past_key_values=cache, use_cache=True)[0], cache[0]["recurrent_state"][0]
+
+    with torch.no_grad():
+        step()                                                  # (the weights gathered, the BLAS library's workspace there)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        at = torch.cuda.memory_allocated()
+        a, sa = step()
+        # beside the new state: y (three d and up to one more) and the output both ways; the steps hold q, k, v, the decay, the gate, o and the
+        # norm's result at once, the few launches the gate, o and the decay at the most
+        held = (torch.cuda.max_memory_allocated() - at - sa.numel() * 4) / (B * T * d * 2)
+        assert (held < 10.) == few[norm == "rmsnorm"], held
+        m._forward_native = lambda *_: None
+        b, sb = step()
+        assert _rel(a, b) <= 5e-3 and _rel(sa, sb) <= 5e-3      # (as above)
