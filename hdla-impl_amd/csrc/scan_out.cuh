@@ -412,12 +412,13 @@ template <int K, int V, int NWC> static hipError_t launch_scan_out_nwc(const Chu
     return hipGetLastError();
 }
 // Column blocks a workgroup: as few as give each workgroup a compute unit of its own (every workgroup fetches the chunks' blocks for
-// itself).  K = V = 128, 128 heads, 2 and 4 blocks: 193 and 146 us; 64 heads: 101 and 114.
+// itself).  A forward pass, us, two blocks and one, 128 chunks in one segment: K = V = 128, 1 lane 82 and 73, 16 lanes 102 and 96, 32 lanes 135 and
+// 127; K = 64, V = 128, 8 lanes 71 and 59, 32 lanes 88 and 79; of 16 chunks K = V = 128 22.3 and 20.8.  The scan alone, two and four: K = V = 128,
+// 128 heads 193 and 146, 64 heads 101 and 114.
 template <int K, int V> hipError_t launch_scan_out_shape(const ChunkArgs<bf16>& a, bool kept, hipStream_t stream) {
     constexpr int VT = V / 16;
     const int lanes = a.H * a.st.N * a.seg.nseg;
-    if constexpr (VT == 4)
-        if (lanes * 4 <= SCAN_TARGET_WORKGROUPS) return launch_scan_out_nwc<K, V, 1>(a, kept, stream);
+    if (lanes * VT <= SCAN_TARGET_WORKGROUPS) return launch_scan_out_nwc<K, V, 1>(a, kept, stream);
     if (lanes * (VT / 2) <= SCAN_TARGET_WORKGROUPS) return launch_scan_out_nwc<K, V, 2>(a, kept, stream);
     return launch_scan_out_nwc<K, V, 4>(a, kept, stream);
 }

@@ -31,7 +31,7 @@ def test_few_chunks(K, V, T, monkeypatch):
 
 
 @pytest.mark.parametrize("K,V", [(64, 64), (64, 128), (128, 64), (128, 128)])
-@pytest.mark.parametrize("H", [3, 65, 129])
+@pytest.mark.parametrize("H", [3, 32, 33, 64, 65, 129])
 def test_column_blocks_of_a_workgroup(K, V, H, monkeypatch):
     monkeypatch.setenv("HDLA_HIP_ROUTE", "classic")
     _check(make_inputs(600 + H, 1, 100, H, K, V, gk_div=4.0), [0, H // 2, H - 1])
