@@ -651,8 +651,15 @@ int hdla_chunk_fwd(const hdla_dims* dims, const void* q, const void* k, const vo
 
 int hdla_chunk_fwd_static(const hdla_dims* dims, const void* q, const void* k, const void* v, const void* a,
                           const void* b, const void* gk, const float* h0, void* o, float* ht, void* stream) {
-    const size_t need = hdla_workspace_bytes(dims, 0);
+    size_t need = hdla_workspace_bytes(dims, 0);
     if (need == 0) { const int rc = check_dims(dims); return rc ? rc : HDLA_ERR_SHAPE; }
+    // the records of the scans' segments are what a call can do without
+    hdla_dims whole = *dims;
+    if (need > (size_t)HDLA_STATIC_WORKSPACE_BYTES && dims->segments == 0 && !fused_shape(dims)) {
+        whole.segments = 1;
+        dims = &whole;
+        need = hdla_workspace_bytes(dims, 0);
+    }
     if (need > (size_t)HDLA_STATIC_WORKSPACE_BYTES) return HDLA_ERR_STATIC_LIMIT;
     int err = 0;
     void* ws = static_scratch(&err);

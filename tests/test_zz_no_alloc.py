@@ -56,6 +56,18 @@ def test_two_calls_in_a_row_match_the_workspace_entry_point(dtype):
         assert torch.equal(o_s, o_w) and torch.equal(ht_s, ht_w)
 
 
+def test_a_call_whose_scans_would_be_cut_into_segments():
+    """Near the limit a call goes without the segments' records, rather than being refused for them."""
+    dims, t, h0, _ = _case(34, 1, 8160, 4, 128, 128, torch.bfloat16)
+    whole = _lib.make_dims(1, 8160, 4, 128, 128, 2, 1, torch.bfloat16, torch.bfloat16, 0.5, None, segments=1)
+    need = lambda d: _lib.load().hdla_workspace_bytes(ctypes.byref(d), 0)
+    assert need(whole) <= STATIC_BYTES < need(dims)
+    rc_s, o_s, ht_s = _call(True, dims, t, h0, with_ws=False)
+    rc_w, o_w, ht_w = _call(False, whole, t, h0, with_ws=True)
+    assert rc_s == 0 and rc_w == 0
+    assert torch.isfinite(o_w.float()).all() and torch.equal(o_s, o_w) and torch.equal(ht_s, ht_w)
+
+
 def test_size_limit_and_argument_errors():
     lib = _lib.load()
     dims, t, h0, _ = _case(33, 8, 2048, 16, 64, 64, torch.bfloat16)      # 117 MB of workspace or more: beyond the array
