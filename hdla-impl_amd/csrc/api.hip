@@ -87,31 +87,49 @@ int fused_segments(const hdla_dims* d) {
 }
 
 // ---- time segments of the stand-alone scans (scan_impl.cuh, scan_out.cuh, scan_grad.cuh): where a whole sequence per workgroup would leave most of the
-// device idle.  A launch for the segments' records, one that chains them (together 10 us at the least), then the scans on
-// shorter sequences: twice the steps, of which nseg run at once.  Measured (us, forward / backward pass, one segment ->
-// as many as chosen here): fp32, K=V=64, 16 lanes of 63 chunks 156/224 -> 69/157 (8); fp32, K=V=128, 4 lanes of 125
-// chunks 812/896 -> 142/278 (16); bf16, K=V=128, 16 lanes of 313 chunks 293/546 -> 192/546 (8 and 1); bf16, K=128 V=64,
-// 8 lanes of 500 chunks 377/509 -> 154/352 (16 and 8).
+// device idle.  A launch for the segments' records, one that chains them, then the scans on shorter sequences: twice the steps,
+// of which nseg run at once.
 constexpr int SCAN_MAX_SEGMENTS = 32;
 // Records (lanes x segments) of a segment count asked for: a record is a state and a matrix of K x K, a few of them per pass, and
 // a sequence's segments share a grid dimension with the sequences (65535).  The device is full long before this many.
 constexpr long long SCAN_MAX_RECORDS = 4096;
+// 2-byte elements: the time of a pass's scans (us), from the launches a number of segments makes.  A step takes what its chain of
+// products does, which grows with K, until the lanes in flight read more than comes in meanwhile; so does one of the records' launch, which
+// has the transitions' columns beside the state's; then there are these two launches, and the records chained one behind the other.
+// Fitted to passes of 32 to 400 chunks and 1 to 32 lanes, K, V in {64, 128}, each in 1, 4, 8, 16 and 32 segments (216 shapes): the choice costs
+// 0.2 % (forward) and 0.6 % (backward pass) more than the best of these, 6 and 9 % at the most.  A least length for every number of lanes, 13 chunks forward and 7
+// backward, cost 3.8 and 5.4 %, 40 and 27 % at the most.  us, forward / backward pass in one segment -> in 4 -> in 8 (* the choice), K = V = 128:
+// 2 lanes of 97 chunks 61/68 -> 57/65 -> 49*/58*, 8 lanes of 64 50*/70* -> 52/78 -> 50/84, 16 lanes of 97 77*/162* -> 77/190 -> 87/206,
+// 24 lanes of 97 84*/241* -> 113/270 -> 118/293, 8 lanes of 313 175/336 -> 144/297 -> 110*/292*.
+struct ScanTime { double step, step_k, load, rec, rec_k, rec_load, launches, chain, chain_k; int most; };   // most: lanes x segments
+constexpr ScanTime SCAN_TIME_FWD{0.18, 0.13, 0.0024, 0.37, 0.12, 0.0015, 6.5, 0.04, 0.73, 128},
+    SCAN_TIME_BWD{0.26, 0.20, 0.0042, 0.29, 0.16, 0.0054, 21., 0.37, 0.49, 64};
+double scan_time(const ScanTime& t, const hdla_dims* d, double lanes, long long chunks, int nseg) {
+    const double k = d->K / 64., v = d->V / 64., steps = (double)((chunks + nseg - 1) / nseg);
+    const double walk = steps * std::max(t.step + t.step_k * k, t.load * lanes * nseg * k * v);
+    if (nseg == 1) return walk;
+    return walk + steps * std::max(t.rec + t.rec_k * k, t.rec_load * lanes * (nseg - 1) * k * (k + v)) + t.launches + nseg * (t.chain + t.chain_k * k);
+}
 int scan_segments(const hdla_dims* d, bool bwd) {
     if (d->route != HDLA_ROUTE_AUTO) return 1;
     const long long lanes = (long long)d->N * d->H;
     if (d->segments > 0) return (int)std::max(1LL, std::min<long long>({d->segments, SCAN_MAX_SEGMENTS, SCAN_MAX_RECORDS / lanes}));
-    const bool f32 = d->in_dtype == HDLA_FP32;
     const long long chunks = ((d->T + CHUNK - 1) / CHUNK) / (d->cu_seqlens ? d->N : 1);
-    // lanes x segments: beyond 128 the records' launch needs more than one round on the device.  The backward scans of
-    // 2-byte inputs are bound by their traffic from a dozen lanes on, and the reverse records come on top: fewer there.
-    if (bwd && !f32 && lanes > 8) return 1;
-    const long long most = bwd && !f32 ? 64 : 128;
-    // chunks a segment: a step takes 2-4 us with fp32 products, about 0.7 with bf16, 0.55 in the forward pass's scan (K = V = 128, 16 lanes of
-    // 97 chunks: 57 us in 8 segments, 52 in 4, 55 whole)
-    const long long least = f32 ? 4 : bwd ? 7 : 13;
     int nseg = 1;
-    while (nseg * 2 <= SCAN_MAX_SEGMENTS && lanes * nseg * 2 <= most && chunks / (nseg * 2) >= least) nseg *= 2;
-    return nseg >= 4 ? nseg : 1;                          // two segments only make up for the second walk
+    if (d->in_dtype != HDLA_FP32) {
+        const ScanTime& t = bwd ? SCAN_TIME_BWD : SCAN_TIME_FWD;
+        double best = scan_time(t, d, (double)lanes, chunks, 1);
+        for (int n = 4; n <= SCAN_MAX_SEGMENTS && lanes * n <= t.most; n *= 2) {      // (two only make up for the second walk)
+            const double x = scan_time(t, d, (double)lanes, chunks, n);
+            if (x < best) { best = x; nseg = n; }
+        }
+        return nseg;
+    }
+    // 4-byte elements: a step takes 2-4 us; beyond 128 lanes x segments the records' launch needs more than one round on the
+    // device.  us, forward / backward pass, one segment -> as many as chosen here: K = V = 64, 16 lanes of 63 chunks 148/216 ->
+    // 72/152 (8); K = V = 128, 4 lanes of 125 chunks 816/894 -> 155/282 (16).
+    while (nseg * 2 <= SCAN_MAX_SEGMENTS && lanes * nseg * 2 <= 128 && chunks / (nseg * 2) >= 4) nseg *= 2;
+    return nseg >= 4 ? nseg : 1;
 }
 
 struct FusedLayout {
