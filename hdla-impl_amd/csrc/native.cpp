@@ -15,8 +15,10 @@
 #include <ATen/ATen.h>
 #include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/Event.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/VirtualGuardImpl.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <dlfcn.h>
@@ -534,9 +536,9 @@ struct LayerCols {
 };
 constexpr int64_t PAD_FROM_ROWS = 1024;
 
-// the concatenated projection weight [ld, d]; rows behind the last projection are zero
-Tensor gather_weights(const Tensor* w, const LayerCols& L) {       // wq, wk, wv, wf0, wg0, wbeta
-    const Tensor out = at::empty({L.ld, L.d}, w[0].options());
+// the concatenated projection weight [ld, d], in `out` if there is one; rows behind the last projection are zero
+Tensor gather_weights(const Tensor* w, const LayerCols& L, Tensor out = Tensor()) {       // wq, wk, wv, wf0, wg0, wbeta
+    if (!out.defined()) out = at::empty({L.ld, L.d}, w[0].options());
     const void* parts[6];
     int64_t rows[6];
     std::vector<Tensor> whole(6);                                  // (a parameter may be a view at any address)
@@ -787,10 +789,77 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     }
 };
 
+// What evaluation mode knows of a concatenated weight that it keeps between calls without gradients.
+struct Kept {
+    struct Part { const void* p; uint64_t v; } of[7];              // the parameters it was formed from, and its width
+    c10::Event ready;                                              // behind the launch that formed it
+    c10::Stream made, home;                                        // the stream of that launch, and the one the memory is from
+    bool complete = false;                                         // `ready` is known to have passed
+    bool captured = false;                                         // a captured graph reads it: it stays where it is
+    bool stale = false;                                            // to be formed anew all the same
+};
+constexpr const char* KEPT = "hdla_hip.kept";
+Kept* kept_at(PyObject* list, Py_ssize_t slot) {
+    PyObject* const o = PyList_GET_ITEM(list, slot);
+    return PyCapsule_IsValid(o, KEPT) ? static_cast<Kept*>(PyCapsule_GetPointer(o, KEPT)) : nullptr;
+}
+PyObject* kept_capsule(Kept&& k) {
+    Kept* const p = new Kept(std::move(k));
+    PyObject* const o = PyCapsule_New(p, KEPT, [](PyObject* c) { delete static_cast<Kept*>(PyCapsule_GetPointer(c, KEPT)); });
+    if (!o) delete p;
+    return o;
+}
+// of the current device
+bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
+// an event that a capture has no part in may be asked for while one is under way, if the thread says that it knows
+bool has_passed(const c10::Event& e) {
+    const c10::hip::HIPStreamCaptureModeGuard relaxed(hipStreamCaptureModeRelaxed);
+    return e.query();
+}
+// Makes the stream `here` read or write behind the launch that formed the weight.  A graph under capture can only take one that is
+// complete: what the replay waits for is not known here.
+bool wait_for(Kept& k, const c10::Stream& here, bool under_capture) {
+    if (k.complete || (here == k.made && !under_capture)) return true;
+    k.complete = has_passed(k.ready);
+    if (!k.complete && !under_capture) k.ready.block(here);
+    return k.complete || !under_capture;
+}
+
+// forget(cache) -> the cache to go on with: what a captured graph reads stays there, to be formed anew in its place by the next call
+PyObject* py_forget(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 1 || !PyList_CheckExact(a[0]) || PyList_GET_SIZE(a[0]) != 4) { PyErr_SetString(PyExc_TypeError, "forget(cache)"); return nullptr; }
+    PyObject* const out = PyList_New(4);
+    if (!out) return nullptr;
+    for (Py_ssize_t i = 0; i < 4; ++i) { Py_INCREF(Py_None); PyList_SET_ITEM(out, i, Py_None); }
+    for (Py_ssize_t slot = 0; slot < 4; slot += 2) {
+        Kept* const k = kept_at(a[0], slot);
+        if (!k || !k->captured) continue;
+        k->stale = true;
+        for (Py_ssize_t i = slot; i < slot + 2; ++i) {
+            PyObject* const o = PyList_GET_ITEM(a[0], i);
+            Py_INCREF(o);
+            PyList_SetItem(out, i, o);
+        }
+    }
+    return out;
+}
+// passed(event handle) -> whether a torch event has passed; also while a capture is under way
+PyObject* py_passed(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 1) { PyErr_SetString(PyExc_TypeError, "passed(event)"); return nullptr; }
+    void* const e = PyLong_AsVoidPtr(a[0]);
+    if (PyErr_Occurred()) return nullptr;
+    return guarded([&]() -> PyObject* {
+        const c10::hip::HIPStreamCaptureModeGuard relaxed(hipStreamCaptureModeRelaxed);
+        const hipError_t rc = hipEventQuery(static_cast<hipEvent_t>(e));
+        if (rc != hipSuccess) (void)hipGetLastError();
+        return PyBool_FromLong(rc == hipSuccess);
+    });
+}
+
 // layer(x, (wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo), initial_state, want_state, mode, cache,
 //       H, groups, norm_q, norm_v, beta_scale, c, eps, gate_pos) -> (output, state) or None
 // mode: 0 chunked with gradients and from RECURRENT_BELOW tokens on, else token-serial; 1 chunked; 2 token-serial
-// cache: a list [key, weight] x 2 that keeps the concatenated weight, narrow and padded, between calls without gradients, or None
+// cache: a list [Kept, weight] x 2 that keeps the concatenated weight, narrow and padded, between calls without gradients, or None
 PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 14 || !api.strerror || !is_tensor(a[0]) || !PyTuple_CheckExact(a[1]) || PyTuple_GET_SIZE(a[1]) != 10) return none();
     const Tensor& x = unpack(a[0]);
@@ -851,36 +920,61 @@ PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
         }
         LayerFwd r;
         const LayerCols L(d, f.H, B * T >= PAD_FROM_ROWS);
+        const at::DeviceGuard guard(dev);
         // the weight of the last call, as long as the parameters are the ones it was built from, unmodified
         // (each width has its own place: a captured graph of decode steps goes on reading the one while long calls use the other)
         const bool cached = PyList_CheckExact(a[5]) && PyList_GET_SIZE(a[5]) == 4;
         const Py_ssize_t slot = B * T >= PAD_FROM_ROWS ? 2 : 0;
-        struct { const void* p; uint64_t v; } key[7];
+        Kept::Part of[7];
+        const c10::Stream here = c10::impl::VirtualGuardImpl(c10::DeviceType::CUDA).getStream(dev);
+        bool built = true, fill = false;                          // fill: in the place that a captured graph reads
         if (cached) {
-            for (int i = 0; i < 6; ++i) key[i] = {P[i].data_ptr(), (uint64_t)P[i]._version()};
-            key[6] = {nullptr, (uint64_t)L.ld};
-            PyObject *old_key = PyList_GET_ITEM(a[5], slot), *old = PyList_GET_ITEM(a[5], slot + 1);
-            if (PyBytes_CheckExact(old_key) && PyBytes_GET_SIZE(old_key) == (Py_ssize_t)sizeof key &&
-                !memcmp(PyBytes_AS_STRING(old_key), key, sizeof key) && is_tensor(old)) r.w = unpack(old);
+            for (int i = 0; i < 6; ++i) of[i] = {P[i].data_ptr(), (uint64_t)P[i]._version()};
+            of[6] = {nullptr, (uint64_t)L.ld};
+            Kept* const k = kept_at(a[5], slot);
+            PyObject* const old = PyList_GET_ITEM(a[5], slot + 1);
+            if (k && is_tensor(old)) {
+                const Tensor& w = unpack(old);
+                const bool under_capture = (!k->complete || !k->captured) && capturing();
+                if (!k->stale && !memcmp(k->of, of, sizeof of)) {
+                    built = !wait_for(*k, here, under_capture);
+                    if (!built) {
+                        k->captured = k->captured || under_capture;
+                        if (here != k->home && !under_capture) w.record_stream(here);
+                        r.w = w;
+                    }
+                } else if (k->captured && w.device() == dev && same_sizes(w, {L.ld, L.d}) && !capturing()) {
+                    fill = wait_for(*k, here, false);            // (one launch that forms it behind the other)
+                    if (here != k->home) w.record_stream(here);
+                    r.w = w;
+                }
+            }
         }
-        const bool built = !r.w.defined();
-        bool keep = false;
+        std::optional<c10::Event> ready;
         unlocked([&] {
-            const at::DeviceGuard guard(dev);
             if (built) {
-                r.w = gather_weights(P, L);
+                r.w = gather_weights(P, L, r.w);
                 // (one gathered under capture is not there before the graph is replayed, and belongs to it)
-                keep = cached && c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None;
+                if (cached && !capturing()) {
+                    ready.emplace(c10::DeviceType::CUDA);
+                    ready->record(here);
+                }
             }
             layer_forward(x, P, f, h0, want, chunked, false, r);
         });
-        if (keep && PyList_GET_SIZE(a[5]) == 4) {
+        if (ready && PyList_GET_SIZE(a[5]) == 4) {
             // (key and weight one behind the other, with the lock held: another thread sees both or neither)
-            PyObject* const k = PyBytes_FromStringAndSize(reinterpret_cast<const char*>(key), sizeof key);
-            if (!k) return nullptr;
+            const Kept* const now = kept_at(a[5], slot);
+            const bool taken = now && now->captured && is_tensor(PyList_GET_ITEM(a[5], slot + 1));
+            if (taken && !fill && unpack(PyList_GET_ITEM(a[5], slot + 1)).device() == dev) return pair(r.out, r.ht);    // captured meanwhile
+            Kept k{{}, std::move(*ready), here, fill && taken ? now->home : here};
+            memcpy(k.of, of, sizeof of);
+            k.captured = fill;
+            PyObject* const key = kept_capsule(std::move(k));
+            if (!key) return nullptr;
             PyObject* const w = THPVariable_Wrap(r.w);
-            if (!w) { Py_DECREF(k); return nullptr; }
-            PyList_SetItem(a[5], slot, k);
+            if (!w) { Py_DECREF(key); return nullptr; }
+            PyList_SetItem(a[5], slot, key);
             PyList_SetItem(a[5], slot + 1, w);
         }
         return pair(r.out, r.ht);
@@ -918,7 +1012,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
 #define HDLA_DEF(name, fn) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(fn)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     HDLA_DEF("bind", py_bind), HDLA_DEF("chunk", py_chunk), HDLA_DEF("chunk_hdla", py_chunk_hdla), HDLA_DEF("recurrent", py_recurrent),
-    HDLA_DEF("recurrent_hdla", py_recurrent_hdla), HDLA_DEF("normalize", py_normalize), HDLA_DEF("layer", py_layer), {nullptr, nullptr, 0, nullptr}};
+    HDLA_DEF("recurrent_hdla", py_recurrent_hdla), HDLA_DEF("normalize", py_normalize), HDLA_DEF("layer", py_layer), HDLA_DEF("forget", py_forget), HDLA_DEF("passed", py_passed), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

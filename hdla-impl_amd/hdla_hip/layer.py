@@ -78,6 +78,35 @@ class RecurrentCache:
         return self.states[layer_idx]
 
 
+class _Kept:
+    """A concatenated weight (and bias) that evaluation mode keeps: what it was formed from, where, and whether a captured graph reads it."""
+
+    def __init__(self, key, w, b, captured=False):
+        self.key, self.w, self.b, self.captured = key, w, b, captured
+        self.made = self.ready = None
+
+    def formed_on(self, stream):
+        self.made, self.ready = stream, torch.cuda.Event()
+        self.ready.record(stream)
+        self.used_on(stream)
+
+    def used_on(self, stream):
+        """Memory of another stream's is not given back before what is on this one has run."""
+        for t in (self.w, self.b):
+            if t is not None:
+                t.record_stream(stream)
+
+    def wait_for(self, stream, capturing) -> bool:
+        """Makes `stream` wait for the weight.  Under capture it has to be there: what the replay waits for is not known here."""
+        if self.ready is None or (stream == self.made and not capturing):
+            return True
+        if _lib.native().passed(self.ready.cuda_event):
+            self.ready = None
+        elif not capturing:
+            stream.wait_event(self.ready)
+        return self.ready is None or not capturing
+
+
 class HDLA_Custom(nn.Module):
     """S[t] = (I - beta k k^T) Diag(f) (I - beta k k^T) S[t-1] + k v^T,  o[t] = S[t]^T q[t]   (hdla_custom.py:46-62,270-288)."""
 
@@ -197,38 +226,83 @@ class HDLA_Custom(nn.Module):
         concatenation is rebuilt per call (and is part of the graph).  In evaluation mode without gradients it is built
         once and reused: it is rebuilt when a parameter is replaced or modified in place (tracked by its version
         counter), on ``.train()`` / ``.eval()``, ``.to()`` and ``load_state_dict``, and by ``reset_cache()`` -- which
-        is what code that writes through ``param.data`` (untracked) has to call."""
+        is what code that writes through ``param.data`` (untracked) has to call.
+
+        Calls on another stream than the one that built it wait for it.  A captured graph that reads it keeps reading the same
+        memory: rebuilt, by the next call outside a capture, it is rebuilt in its place, and only ``reset_cache()`` or the end of the module
+        gives it back."""
         ps = [m.weight for m in heads] + ([m.bias for m in heads] if heads[0].bias is not None else [])
         if self.training or (torch.is_grad_enabled() and any(p.requires_grad for p in ps)):
             w = torch.cat([m.weight for m in heads], dim=0)
             return w, (torch.cat([m.bias for m in heads], dim=0) if heads[0].bias is not None else None)
-        key = tuple((p.data_ptr(), p._version, p.dtype, p.device) for p in ps)
-        if getattr(self, "_gathered_key", None) != key:
-            with torch.no_grad():
-                w = torch.cat([m.weight for m in heads], dim=0)
-                b = torch.cat([m.bias for m in heads], dim=0) if heads[0].bias is not None else None
-            if w.is_cuda:
-                with torch.cuda.device(w.device):
-                    if torch.cuda.is_current_stream_capturing():           # not there before the graph is replayed
-                        return w, b
-            self._gathered_key, self._gathered_val = key, (w, b)
-        return self._gathered_val
+        key, kept = tuple((p.data_ptr(), p._version, p.dtype, p.device) for p in ps), getattr(self, "_kept", None)
+        if not ps[0].is_cuda:
+            if kept is None or kept.key != key:
+                kept = self._kept = _Kept(key, *self._concatenated(heads))
+            return kept.w, kept.b
+        with torch.cuda.device(ps[0].device):
+            capturing, here = torch.cuda.is_current_stream_capturing(), torch.cuda.current_stream()
+            if kept is not None and kept.key == key and kept.wait_for(here, capturing):
+                kept.captured = kept.captured or capturing
+                if not capturing:
+                    kept.used_on(here)
+                return kept.w, kept.b
+            if capturing:                                                      # not there before the graph is replayed
+                return self._concatenated(heads)
+            like = lambda x, m: x is None or (x.dtype, x.device) == (m.dtype, m.device)
+            if kept is not None and kept.captured and like(kept.w, ps[0]) and like(kept.b, ps[-1]):
+                kept.wait_for(here, False)                                     # formed anew in its place
+                kept.used_on(here)
+                with torch.inference_mode(kept.w.is_inference()):
+                    self._concatenated(heads, kept.w, kept.b)
+                new = _Kept(key, kept.w, kept.b, True)
+            else:
+                new = _Kept(key, *self._concatenated(heads))
+            new.formed_on(here)
+            self._kept = new
+        return new.w, new.b
+
+    @staticmethod
+    def _concatenated(heads, w=None, b=None):
+        with torch.no_grad():
+            w = torch.cat([m.weight for m in heads], dim=0, out=w)
+            if heads[0].bias is not None:
+                b = torch.cat([m.bias for m in heads], dim=0, out=b)
+        return w, b
 
     def reset_cache(self):
-        """Forget the concatenated projection weight of evaluation mode (a captured graph that reads it must be captured anew)."""
-        self._gathered_key = self._gathered_val = None
-        self._native_cache = [None] * 4
+        """Forget the concatenated projection weight of evaluation mode, also where a captured graph reads it: that must be captured
+        anew."""
+        self._kept, self._native_cache = None, [None] * 4
+
+    def _form_anew(self):
+        """The next call forms the concatenated weight of evaluation mode anew: where a captured graph reads it, in its place."""
+        kept, native = getattr(self, "_kept", None), self._native_cache
+        if kept is not None:
+            if kept.captured:
+                kept.key = None
+            else:
+                self._kept = None
+        self._native_cache = [None] * 4 if native is None or native == [None] * 4 else _lib.native().forget(native)
+
+    def __getstate__(self):
+        """A copy forms its own weight."""
+        state = self.__dict__.copy()
+        state.pop("_kept", None)
+        if state.get("_native_cache") is not None:
+            state["_native_cache"] = [None] * 4
+        return state
 
     def train(self, mode: bool = True):
-        self.reset_cache()
+        self._form_anew()
         return super().train(mode)
 
     def _apply(self, fn, *args, **kwargs):
-        self.reset_cache()
+        self._form_anew()
         return super()._apply(fn, *args, **kwargs)
 
     def _load_from_state_dict(self, *args, **kwargs):
-        self.reset_cache()
+        self._form_anew()
         return super()._load_from_state_dict(*args, **kwargs)
 
     def _up(self, lin: nn.Linear, x0: torch.Tensor) -> torch.Tensor:
