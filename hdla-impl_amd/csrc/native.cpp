@@ -83,26 +83,34 @@ inline int dtype_code(at::ScalarType t) { return t == at::kBFloat16 ? HDLA_BF16 
 inline bool native_dtype(at::ScalarType t) { return t == at::kBFloat16 || t == at::kFloat; }
 inline Tensor bytes_like(const Tensor& t, size_t n) { return at::empty({(int64_t)n}, t.options().dtype(at::kByte)); }
 
-// the package's environment switches, read on every call like the Python code does
+// The package's environment switches, read on every call like the Python code does, and once: while the interpreter lock is held, under
+// which os.environ writes them.
+const char* env(const char* name) {
+    if (!PyGILState_Check()) throw std::logic_error("the environment is read with the interpreter lock held");
+    return getenv(name);
+}
 bool env_is(const char* name, std::initializer_list<const char*> values, bool unset) {
-    const char* v = getenv(name);
+    const char* v = env(name);
     if (!v) return unset;
     for (const char* x : values) if (!strcmp(v, x)) return true;
     return false;
 }
 bool keep_forward_default() { return !env_is("HDLA_HIP_KEEP_FORWARD", {"", "0", "false", "False"}, true); }
-bool keep_boundaries_default() { return env_is("HDLA_HIP_INPUTS_ONLY", {"", "0", "false", "False"}, true); }
+// launch plan and record of a chunked call
+struct Plan { int32_t route, segments; bool record; };
 // false: the Python code has to look at it (another spelling, a number that is none)
-bool route_and_segments(hdla_dims& d) {
-    const char* r = getenv("HDLA_HIP_ROUTE");
-    if (!r || !*r || !strcmp(r, "auto")) d.route = HDLA_ROUTE_AUTO;
-    else if (!strcmp(r, "classic")) d.route = HDLA_ROUTE_CLASSIC;
-    else if (!strcmp(r, "fused")) d.route = HDLA_ROUTE_FUSED;
+bool read_plan(Plan& p) {
+    const char* r = env("HDLA_HIP_ROUTE");
+    if (!r || !*r || !strcmp(r, "auto")) p.route = HDLA_ROUTE_AUTO;
+    else if (!strcmp(r, "classic")) p.route = HDLA_ROUTE_CLASSIC;
+    else if (!strcmp(r, "fused")) p.route = HDLA_ROUTE_FUSED;
     else return false;
-    const char* s = getenv("HDLA_HIP_SEGMENTS");
-    if (!s) { d.segments = 0; return true; }
+    p.record = env_is("HDLA_HIP_INPUTS_ONLY", {"", "0", "false", "False"}, true);
+    p.segments = 0;
+    const char* s = env("HDLA_HIP_SEGMENTS");
+    if (!s) return true;
     char* end = nullptr;
-    d.segments = (int32_t)strtol(s, &end, 10);
+    p.segments = (int32_t)strtol(s, &end, 10);
     return *s && !*end;
 }
 
@@ -112,8 +120,9 @@ struct ChunkIn {
     Tensor q, k, v, a, b, beta, gk, h0, cu;
 };
 
-bool chunk_dims(const ChunkIn& x, double scale, hdla_dims& d) {
+void chunk_dims(const ChunkIn& x, double scale, const Plan& p, hdla_dims& d) {
     d = hdla_dims{};
+    d.route = p.route; d.segments = p.segments;
     d.B = (int32_t)x.q.size(0); d.T = (int32_t)x.q.size(1); d.H = (int32_t)x.q.size(2); d.K = (int32_t)x.q.size(3);
     d.V = (int32_t)x.v.size(3); d.R = 2;
     d.N = x.cu.defined() ? (int32_t)(x.cu.numel() - 1) : d.B;
@@ -121,15 +130,13 @@ bool chunk_dims(const ChunkIn& x, double scale, hdla_dims& d) {
     d.gk_dtype = dtype_code(x.gk.scalar_type());
     d.scale = (float)scale;
     d.cu_seqlens = x.cu.defined() ? x.cu.data_ptr<int64_t>() : nullptr;
-    return route_and_segments(d);
 }
 
 // The launch plan of a backward pass is that of its forward pass, whatever the environment says by then: the record is laid out by it.
-void keep_plan(AutogradContext* ctx, const hdla_dims& d) { ctx->saved_data["plan"] = std::vector<int64_t>{d.route, d.segments}; }
-void kept_plan(AutogradContext* ctx, hdla_dims& d) {
-    const auto plan = ctx->saved_data["plan"].toIntVector();
-    d.route = (int32_t)plan[0];
-    d.segments = (int32_t)plan[1];
+void keep_plan(AutogradContext* ctx, const Plan& p) { ctx->saved_data["plan"] = std::vector<int64_t>{p.route, p.segments}; }
+Plan kept_plan(AutogradContext* ctx) {
+    const auto p = ctx->saved_data["plan"].toIntVector();
+    return {(int32_t)p[0], (int32_t)p[1], false};
 }
 
 // with_record: of a backward pass that is given the forward pass's record
@@ -156,14 +163,15 @@ void chunk_forward(const ChunkIn& x, const hdla_dims& d, bool want_ht, bool want
 // has one, the record for the backward pass are saved; everything else is recomputed).
 struct ChunkFn : torch::autograd::Function<ChunkFn> {
     static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Maybe& a, const Maybe& b,
-                                 const Maybe& beta, const Tensor& gk, const Maybe& h0, const Maybe& cu, double scale, bool want_ht) {
+                                 const Maybe& beta, const Tensor& gk, const Maybe& h0, const Maybe& cu, double scale, bool want_ht,
+                                 const Plan& plan) {
         ChunkIn x{q, k, v, value(a), value(b), value(beta), gk, value(h0), value(cu)};
         if (h0) x.h0 = h0->to(at::kFloat).contiguous();
         hdla_dims d;
-        chunk_dims(x, scale, d);
-        keep_plan(ctx, d);
+        chunk_dims(x, scale, plan, d);
+        keep_plan(ctx, plan);
         Tensor o, ht, boundary;
-        chunk_forward(x, d, want_ht, keep_boundaries_default(), o, ht, boundary);
+        chunk_forward(x, d, want_ht, plan.record, o, ht, boundary);
         ctx->save_for_backward({q, k, v, x.a, x.b, x.beta, gk, value(h0), x.cu, boundary});
         ctx->saved_data["scale"] = scale;
         ctx->set_materialize_grads(false);
@@ -179,8 +187,7 @@ struct ChunkFn : torch::autograd::Function<ChunkFn> {
         const at::DeviceGuard guard(x.q.device());
         if (x.h0.defined()) x.h0 = x.h0.to(at::kFloat).contiguous();
         hdla_dims d;
-        chunk_dims(x, ctx->saved_data["scale"].toDouble(), d);
-        kept_plan(ctx, d);
+        chunk_dims(x, ctx->saved_data["scale"].toDouble(), kept_plan(ctx), d);
         const Tensor d_o = grads[0].defined() ? grads[0].to(x.v.scalar_type()).contiguous() : at::zeros_like(x.v);
         Tensor dht;
         if (grads.size() > 1 && grads[1].defined()) dht = grads[1].to(at::kFloat).contiguous();
@@ -195,7 +202,7 @@ struct ChunkFn : torch::autograd::Function<ChunkFn> {
                               boundary.defined() ? (size_t)boundary.numel() : 0, ptr(ws), (size_t)ws.numel(), stream_of(x.q)),
               "hdla_chunk_bwd_b");
         if (dh0.defined()) dh0 = dh0.to(s[7].scalar_type());
-        return {dq, dk, dv, da, db, dbeta, dgk, dh0, Tensor(), Tensor(), Tensor()};
+        return {dq, dk, dv, da, db, dbeta, dgk, dh0, Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };
 
@@ -334,15 +341,18 @@ PyObject* run_chunk(ChunkIn& x, PyObject* pscale, PyObject* pwant, PyObject* pke
     if (pkeep == Py_None ? keep_forward_default() : (!truth(pkeep, keep) || keep)) return none();
     if (pscale == Py_None) scale = std::pow((double)x.q.size(3), -0.5);
     else if (!number(pscale, scale)) return none();
-    hdla_dims d;
+    Plan plan;
+    if (!read_plan(plan)) return none();
     return guarded([&]() -> PyObject* {
-        if (!chunk_dims(x, scale, d)) return none();
+        hdla_dims d;
+        chunk_dims(x, scale, plan, d);
         Tensor o, ht;
         unlocked([&] {
             const at::DeviceGuard guard(x.q.device());
             make_contiguous(x);
             if (any_grad(x)) {
-                const auto r = ChunkFn::apply(x.q, x.k, x.v, maybe(x.a), maybe(x.b), maybe(x.beta), x.gk, maybe(x.h0), maybe(x.cu), scale, want);
+                const auto r = ChunkFn::apply(x.q, x.k, x.v, maybe(x.a), maybe(x.b), maybe(x.beta), x.gk, maybe(x.h0), maybe(x.cu), scale, want,
+                                              plan);
                 o = r[0];
                 if (want) ht = r[1];
                 return;
@@ -381,9 +391,11 @@ PyObject* run_recurrent(ChunkIn& x, PyObject* pscale, PyObject* pwant, PyObject*
     if (any_grad(x) || !truth(pwant, want) || !truth(preverse, reverse)) return none();
     if (pscale == Py_None) scale = std::pow((double)x.q.size(3), -0.5);
     else if (!number(pscale, scale)) return none();
-    hdla_dims d;
+    Plan plan;
+    if (!read_plan(plan)) return none();
     return guarded([&]() -> PyObject* {
-        if (!chunk_dims(x, scale, d)) return none();
+        hdla_dims d;
+        chunk_dims(x, scale, plan, d);
         Tensor o, ht;
         unlocked([&] {
             const at::DeviceGuard guard(x.q.device());
@@ -642,7 +654,8 @@ bool in_few_launches(int64_t rows, int64_t T, int64_t d, bool norm_in_step) {
 }
 
 // params: wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo; r.w gathered; keep: a backward pass follows
-void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, const Tensor& h0, bool want_ht, bool chunked, bool keep, LayerFwd& r) {
+void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, const Plan& plan, const Tensor& h0, bool want_ht, bool chunked, bool keep,
+                   LayerFwd& r) {
     const int64_t B = x3.size(0), T = x3.size(1), d = x3.size(2), rows = B * T;
     const LayerCols L(d, f.H, r.w.size(0) != LayerCols(d, f.H, false).ld);
     const auto opt = x3.options();
@@ -666,9 +679,9 @@ void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, const T
     check(api.layer_up_fwd(&ud, ptr(r.y), ptr(P[6]), ptr(P[7]), ptr(r.f), ptr(in.gk), ptr(r.g), s), "hdla_layer_up_fwd");
     if (h0.defined()) in.h0 = h0.to(at::kFloat).contiguous();
     hdla_dims& cd = r.dims;
-    chunk_dims(in, 1.0, cd);
+    chunk_dims(in, 1.0, plan, cd);
     if (chunked) {
-        chunk_forward(in, cd, want_ht, keep && keep_boundaries_default(), r.o, r.ht, r.boundary);
+        chunk_forward(in, cd, want_ht, keep && plan.record, r.o, r.ht, r.boundary);
     } else {
         r.o = at::empty_like(in.v);
         if (want_ht) r.ht = at::empty({cd.N, cd.H, cd.K, cd.V}, opt.dtype(at::kFloat));
@@ -696,12 +709,12 @@ Tensor weight_grad(const Tensor& dy, const Tensor& x) {
 struct LayerFn : torch::autograd::Function<LayerFn> {
     static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& wq, const Tensor& wk, const Tensor& wv, const Tensor& wf0,
                                  const Tensor& wg0, const Tensor& wbeta, const Tensor& wf1, const Tensor& wg1, const Tensor& wnorm,
-                                 const Tensor& wo, const Maybe& h0, const LayerCfg& f, bool want_ht) {
+                                 const Tensor& wo, const Maybe& h0, const LayerCfg& f, bool want_ht, const Plan& plan) {
         const Tensor P[10] = {wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo};
         LayerFwd r;
         r.w = gather_weights(P, LayerCols(x.size(2), f.H, x.size(0) * x.size(1) >= PAD_FROM_ROWS));
-        layer_forward(x, P, f, value(h0), want_ht, true, true, r);
-        keep_plan(ctx, r.dims);
+        layer_forward(x, P, f, plan, value(h0), want_ht, true, true, r);
+        keep_plan(ctx, plan);
         ctx->save_for_backward({r.x, r.w, r.y, r.f, r.g, r.o, r.n, r.boundary, r.op.q, r.op.k, r.op.v, r.op.beta, r.op.gk, value(h0), wf1, wg1,
                                 wnorm, wo});
         ctx->saved_data["c"] = std::vector<double>{f.beta_scale, f.c, f.eps};
@@ -729,7 +742,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
         void* const stream = stream_of(x);
         const auto opt = x.options();
         const auto need = [&](size_t i) { return ctx->needs_input_grad(i); };
-        variable_list out(14);
+        variable_list out(15);
 
         // output projection and gated norm
         const Tensor dout = grads[0].defined() ? grads[0].to(at::kBFloat16).contiguous().view({rows, d}) : at::zeros({rows, d}, opt);
@@ -754,8 +767,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
             Tensor dht;
             if (grads.size() > 1 && grads[1].defined()) dht = grads[1].to(at::kFloat).contiguous();
             hdla_dims cd;
-            chunk_dims(in, 1.0, cd);
-            kept_plan(ctx, cd);
+            chunk_dims(in, 1.0, kept_plan(ctx), cd);
             const Tensor ws = workspace(cd, HDLA_PASS_BWD, x, boundary.defined());
             check(api.chunk_bwd_b(&cd, ptr(q), ptr(k), ptr(v), nullptr, nullptr, ptr(beta), ptr(gk), fptr(in.h0), ptr(d_o), fptr(dht), ptr(dq),
                                   ptr(dk), ptr(dv), nullptr, nullptr, ptr(dbeta), ptr(dgk), fptr(dh0), ptr(boundary),
@@ -905,14 +917,14 @@ PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const bool chunked = mode == 1 || (mode == 0 && ((c10::GradMode::is_enabled() && op_grad) || T >= RECURRENT_BELOW));
     if (grad && !chunked) return none();                         // gradients behind the token-serial operator: as the Python code has it
     if (keep_forward_default() && grad) return none();
-    hdla_dims probe{};
-    if (!route_and_segments(probe)) return none();
+    Plan plan;
+    if (!read_plan(plan)) return none();
     return guarded([&]() -> PyObject* {
         Tensor out, ht;
         if (grad) {
             unlocked([&] {
                 const at::DeviceGuard guard(dev);
-                const auto r = LayerFn::apply(x, P[0], P[1], P[2], P[3], P[4], P[5], P[6], P[7], P[8], P[9], maybe(h0), f, want);
+                const auto r = LayerFn::apply(x, P[0], P[1], P[2], P[3], P[4], P[5], P[6], P[7], P[8], P[9], maybe(h0), f, want, plan);
                 out = r[0];
                 if (want) ht = r[1];
             });
@@ -960,7 +972,7 @@ PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
                     ready->record(here);
                 }
             }
-            layer_forward(x, P, f, h0, want, chunked, false, r);
+            layer_forward(x, P, f, plan, h0, want, chunked, false, r);
         });
         if (ready && PyList_GET_SIZE(a[5]) == 4) {
             // (key and weight one behind the other, with the lock held: another thread sees both or neither)

@@ -406,3 +406,12 @@ def test_cu_seqlens_on_the_cpu_is_validated_before_any_launch():
         _lib.check_cu_seqlens(torch.tensor([[0, 10]]), 10)
     with pytest.raises(ValueError):
         _lib.check_cu_seqlens(torch.tensor([0]), 0)
+
+
+def test_native_code_reads_the_environment_in_one_place_with_the_lock_held():
+    """os.environ writes the environment under the interpreter lock, and the C library may move it then."""
+    text = open(os.path.join(os.path.dirname(_lib.__file__), os.pardir, "csrc", "native.cpp")).read()
+    at = [m.start() for m in re.finditer(r"\bgetenv\(", text)]
+    assert len(at) == 1
+    body = text[text.rindex("\n}\n", 0, at[0]):at[0]]
+    assert "if (!PyGILState_Check()) throw" in body
