@@ -13,29 +13,68 @@ from hdla_hip import _lib
 
 OBJDUMP = shutil.which("llvm-objdump", path=os.pathsep.join(["/opt/rocm/llvm/bin", os.environ.get("PATH", "")]))
 WAIT = 6            # wait states below which a pair is reported; 5 were enough where it was measured
-MFMA = re.compile(r"v_mfma_f32_16x16x(16|32)_bf16 v\[(\d+):(\d+)\], \S+ \S+ (?:v\[(\d+):(\d+)\]|\S+)")
+MFMA = re.compile(r"v_mfma_f32_16x16x(16|32)_bf16 ([va])\[(\d+):(\d+)\], \S+ \S+ (?:([va])\[(\d+):(\d+)\]|\S+)")
+LABEL = re.compile(r"<(\w+)>:")
+BRANCH = re.compile(r"(s_c?branch\w*) (\w+)")
 
 
 def pairs_too_close(lines):
-    """(line number, text) of products whose accumulator a product of the other shape wrote less than WAIT wait states before."""
-    found, recent, now = [], [], 0
+    """(line number, text) of products whose accumulator a product of the other shape may have written less than WAIT wait states
+    before, along any way through the branches of one function's listing (labels `<L0>:`)."""
+    code, labels = [], {}                                   # (line number, text, wait states), label -> index of what is behind it
     for no, ln in enumerate(lines):
         ln = ln.split("//")[0].strip()
-        if not ln or ln.endswith(":"):
-            continue
-        now += 1
-        m = re.match(r"s_nop (\d+|0x[0-9a-f]+)", ln)
+        m = LABEL.match(ln)
         if m:
-            now += int(m[1], 0)
-        m = MFMA.match(ln)
-        if not m:
-            continue
-        if m[4]:
-            c0, c1 = int(m[4]), int(m[5])
-            if any(now - at <= WAIT and shape != m[1] and d0 <= c1 and c0 <= d1 for at, shape, d0, d1 in recent):
-                found.append((no, ln))
-        recent = [r for r in recent if now - r[0] <= WAIT] + [(now, m[1], int(m[2]), int(m[3]))]
-    return found
+            labels[m[1]] = len(code)
+        elif ln:
+            m = re.match(r"s_nop (\d+|0x[0-9a-f]+)", ln)
+            code.append((no, ln, 1 + (int(m[1], 0) if m else 0)))
+    # what is in flight before an instruction: (shape, register file, first, last) -> wait states since, on the shortest way there
+    before, todo, found = {0: {}}, [0], set()
+    while todo:
+        i = todo.pop()
+        state = before[i]
+        while i < len(code):
+            no, ln, cost = code[i]
+            state = {r: age + cost for r, age in state.items() if age + cost <= WAIT}
+            m = MFMA.match(ln)
+            if m:
+                if m[5] and any(r[0] != m[1] and r[1] == m[5] and r[2] <= int(m[7]) and int(m[6]) <= r[3] for r in state):
+                    found.add((no, ln))
+                state[m[1], m[2], int(m[3]), int(m[4])] = 0
+            m = BRANCH.match(ln)
+            to = [labels[m[2]]] if m and m[2] in labels else []
+            assert not m or to, "a branch without its label: " + ln
+            if not (m and m[1] == "s_branch") and not ln.startswith("s_endpgm"):
+                to.append(i + 1)
+            go = None
+            for j in to:
+                old = before.get(j)
+                new = dict(state) if old is None else {r: min(state.get(r, WAIT), old.get(r, WAIT)) for r in state.keys() | old.keys()}
+                if old is not None and new == old:
+                    continue
+                before[j] = new
+                if j == i + 1:
+                    go = new
+                else:
+                    todo.append(j)
+            if go is None:
+                break
+            i, state = i + 1, go
+    return sorted(found)
+
+
+def functions(lines):
+    """The listing's functions: their lines behind the name."""
+    out = []
+    for ln in lines:
+        m = LABEL.match(ln.strip())
+        if m and not re.fullmatch(r"L\d+", m[1]):
+            out.append([])
+        elif out:
+            out[-1].append(ln)
+    return out
 
 
 def code_objects(path):
@@ -59,6 +98,14 @@ def test_the_check_finds_a_planted_pair():
     assert pairs_too_close([x32 + "0", "s_nop 1", x16 + "v[4:7]"])
     assert not pairs_too_close([x16 + "0", "s_nop 7", x32 + "v[0:3]"])
     assert not pairs_too_close([x16 + "0", x16 + "v[0:3]", x32 + "v[4:7]"])
+    # round a loop, into a branch and over one; and in accumulation registers
+    assert pairs_too_close(["<L0>:", x32 + "v[0:3]", *["s_nop 7"] * 2, x16 + "0", "s_cbranch_scc1 L0", "s_endpgm"])
+    assert not pairs_too_close(["<L0>:", x32 + "v[0:3]", *["s_nop 7"] * 2, x16 + "0", "s_nop 5", "s_cbranch_scc1 L0", "s_endpgm"])
+    assert pairs_too_close([x16 + "0", "s_cbranch_scc0 L3", *["v_mov_b32 v30, v31"] * 9, "<L3>:", x32 + "v[0:3]", "s_endpgm"])
+    assert not pairs_too_close([x16 + "0", "s_branch L4", "<L3>:", x32 + "v[0:3]", "s_endpgm", "<L4>:", *["s_nop 7"], "s_branch L3"])
+    a16, a32 = x16.replace("v[0:3]", "a[0:3]"), x32.replace("v[4:7]", "a[4:7]")
+    assert pairs_too_close([a16 + "0", a32 + "a[0:3]"]) and pairs_too_close([a32 + "0", x16 + "a[4:7]"])
+    assert not pairs_too_close([a16 + "0", x32 + "v[0:3]"])
 
 
 @pytest.mark.skipif(OBJDUMP is None, reason="no llvm-objdump")
@@ -70,9 +117,11 @@ def test_no_accumulator_changes_product_shape_without_a_wait(tmp_path):
     for i, code in enumerate(code_objects(path)):
         f = tmp_path / ("%d.o" % i)
         f.write_bytes(code)
-        text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", "--no-leading-addr", str(f)], check=True, capture_output=True, text=True).stdout
-        lines = text.splitlines()
-        seen += sum("16x16x32_bf16" in ln for ln in lines)
-        bad += [(i, no, ln) for no, ln in pairs_too_close(lines)]
+        text = subprocess.run([OBJDUMP, "-d", "--symbolize-operands", "--no-show-raw-insn", "--no-leading-addr", str(f)], check=True, capture_output=True,
+                              text=True).stdout
+        seen += text.count("16x16x32_bf16")
+        for lines in functions(text.splitlines()):
+            if any("16x16x32_bf16" in ln for ln in lines):
+                bad += [(i, no, ln) for no, ln in pairs_too_close(lines)]
     assert seen > 0, "no 16x16x32 product found: the disassembly was not read"
     assert not bad, bad[:5]
