@@ -180,3 +180,111 @@ def test_several_tokens_of_many_sequences(B, T, H, few, norm):
         m._forward_native = lambda *_: None
         b, sb = step()
         assert _rel(a, b) <= 5e-3 and _rel(sa, sb) <= 5e-3      # (as above)
+
+
+# ---- against float64, without the library's other kernels ----------------------------------------------------------------
+def _exact(y, wf, wg, w, h0, N, T, H, D, cols, norm_q, norm_v, gate_pos, groups, log_f=None, gate=None):
+    """What lies between the projections, in float64 and rounded nowhere: (o as the norm leaves it, final state)."""
+    from oracle import hrdplr_oracle as O
+    from oracle import normalize_oracle as NO
+    y = y.double()
+    take = lambda c, n: y[:, c:c + n]
+    head = lambda t: t.reshape(N, T, H, D)
+    silu = lambda x: x * torch.sigmoid(x)
+    q, k, v = (head(silu(take(cols[i], H * D))) for i in "qkv")
+    q, k, v = NO.l2_norm(q) if norm_q else q, NO.l2_norm(k), NO.l2_norm(v) if norm_v else v
+    beta = 2.0 * torch.sigmoid(take(cols["b"], H)).reshape(N, T, H, 1)
+    if log_f is None:
+        log_f, gate = torch.nn.functional.logsigmoid(take(cols["f"], D) @ wf.double().t()), take(cols["g"], D) @ wg.double().t()
+    log_f, gate = head(log_f.double()), gate.double().reshape(N, T, H * D)
+    a, b = O.parameterize_a_b(beta, k, log_f)
+    o, S = O.recurrence(q, k, v, a, b, log_f, 1.0, h0.double())
+    pos = "pre" if gate_pos == 1 else "post"
+    return NO.normalize(o.reshape(N, T, H * D), w, gate, gate_pos=pos, c=(H * D // groups) ** .5, eps=1e-5, num_groups=groups), S
+
+
+def _operands(seed, N, T, H, D):
+    rows, d = N * T, H * D
+    cols = dict(q=0, k=d, v=2 * d, f=3 * d, g=3 * d + D, b=3 * d + 2 * D)
+    y = _rn(seed, rows, (cols["b"] + H + 7) // 8 * 8).bfloat16()
+    wf, wg = (_rn(seed + 1, d, D) * .2).bfloat16(), (_rn(seed + 2, d, D) * .2).bfloat16()
+    w, h0 = 1. + .1 * _rn(seed + 3, d), _rn(seed + 4, N, H, D, D)
+    log_f, gate = -_rn(seed + 5, rows, d).abs().bfloat16(), _rn(seed + 6, rows, d).bfloat16()
+    return cols, y, wf, wg, w, h0, log_f, gate
+
+
+def _step(cols, y, wf, wg, w, h0, log_f, gate, N, T, H, D, norm_q, norm_v, gate_pos, groups, later=False):
+    """The launch (T = 1: with the low-rank products), and the norm of its own where that is over all channels, or (later) the projection that
+    forms it, with the identity for its weight."""
+    lib, st, ref, bf, rows, d = _lib.load(), _lib.current_stream(DEV), ctypes.byref, _lib.dtype_code(torch.bfloat16), N * T, H * D
+    pre = _lib.HdlaPreDims(rows, H, D, bf, y.shape[1], cols["q"], cols["k"], cols["v"], cols["b"], norm_q, 1, norm_v, 2.0, 1e-5, 0)
+    up = _lib.HdlaUpDims(rows, d, D, y.shape[1], cols["f"], cols["g"]) if T == 1 else None
+    nd = _lib.HdlaNormDims(rows, groups, d // groups, bf, _lib.dtype_code(torch.float32), gate_pos, (d // groups) ** .5, 1e-5)
+    o, n, ht = torch.empty(rows, d, device=DEV, dtype=torch.bfloat16), torch.empty(rows, d, device=DEV, dtype=torch.bfloat16), torch.empty_like(h0)
+    g = torch.empty_like(gate) if T == 1 else gate
+    here = groups == H
+    if later:
+        gated, eye = torch.empty(rows * (d + H), device=DEV), torch.eye(d, device=DEV).bfloat16()
+        assert lib.hdla_layer_step(ref(pre), ref(up) if up else None, ref(nd), T, P(y), P(wf) if up else None, P(wg) if up else None,
+                                   None if up else P(log_f), P(g), None, P(h0), None, P(gated), P(ht), st) == 0
+        assert lib.hdla_rows_gemm_norm(rows, d, d, P(gated), H, ref(nd), P(w), P(eye), d, P(n), d, st) == 0
+        return n, ht
+    assert lib.hdla_layer_step(ref(pre), ref(up) if up else None, ref(nd) if here else None, T, P(y), P(wf) if up else None, P(wg) if up else None,
+                               None if up else P(log_f), P(g), P(w) if here else None, P(h0), P(o), None, P(ht), st) == 0
+    if here:
+        return o, ht
+    assert lib.hdla_normalize_fwd(ref(nd), P(o), P(w), P(g), P(n), st) == 0
+    return n, ht
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("N,T,H,norm_q,norm_v,gate_pos,all_channels", [(1, 1, 2, True, False, 1, False), (5, 1, 4, False, True, 2, True), (3, 2, 3, True, True, 2, False),
+                                                                      (2, 8, 4, True, False, 1, True)])
+def test_layer_step_against_float64(D, N, T, H, norm_q, norm_v, gate_pos, all_channels):
+    ops, groups = _operands(50 + T, N, T, H, D), 1 if all_channels else H
+    cols, y, wf, wg, w, h0, log_f, gate = ops
+    more = {} if T == 1 else dict(log_f=log_f, gate=gate)
+    o_r, ht_r = _exact(y.cpu(), wf.cpu(), wg.cpu(), w.cpu(), h0.cpu(), N, T, H, D, cols, norm_q, norm_v, gate_pos, groups, **{k: t.cpu() for k, t in more.items()})
+    # On the way to o: q, k, v, beta, f, its logarithm, the gate, the two rank terms, o and the result are rounded to 8 bits, 2^-9 / sqrt(3) of
+    # each in the mean: sqrt(11) of that; the state sees the first nine.  Twice it for sums in which parts of the terms cancel
+    rms = 2 ** -9 / 3 ** .5
+    for later in ([False, True] if all_channels else [False]):
+        o, ht = _step(*ops, N, T, H, D, norm_q, norm_v, gate_pos, groups, later)
+        assert _rel(o.view(N, T, -1).cpu(), o_r) <= 2 * 11 ** .5 * rms and _rel(ht.cpu(), ht_r) <= 2 * 3 * rms
+
+
+LOWEST = -3.3895313892515355e38                              # of bf16
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("T", [1, 3])
+@pytest.mark.parametrize("norm", ["head", "all channels", "later"])
+@pytest.mark.parametrize("where,value", [("q", float("nan")), ("k", float("nan")), ("v", float("nan")), ("b", float("nan")), ("f", float("nan")), ("g", float("nan")),
+                                         ("S", float("nan")), ("v", float("inf")), ("S", float("inf")), ("S", -float("inf")), ("b", float("inf")), ("b", -float("inf")),
+                                         ("b", LOWEST), ("q", LOWEST), ("k", LOWEST), ("f", LOWEST), ("g", LOWEST), ("g", float("inf"))])
+def test_layer_step_on_values_that_are_none(D, T, norm, where, value):
+    """A NaN, an infinity or the lowest number in one head (or one token's inner activations) of one sequence: what it reaches in float64
+    arithmetic is what it reaches here, and nothing else; the other sequences keep their bits."""
+    N, H = 3, 4
+    groups, later = H if norm == "head" else 1, norm == "later"
+    cols, y, wf, wg, w, h0, log_f, gate = _operands(70, N, T, H, D)
+    clean = _step(cols, y, wf, wg, w, h0, log_f, gate, N, T, H, D, True, False, 1, groups, later)
+    row = T                                                  # the first token of the second sequence
+    if where == "S":
+        h0[1, 2, 5, 7] = value
+    elif T > 1 and where in "fg":                            # formed before this launch
+        (log_f if where == "f" else gate)[row, 2 * D + 9] = value
+    else:
+        y[row, cols[where] + (2 if where == "b" else 9 if where in "fg" else 2 * D + 9)] = value
+    o, ht = _step(cols, y, wf, wg, w, h0, log_f, gate, N, T, H, D, True, False, 1, groups, later)
+    more = {} if T == 1 else dict(log_f=log_f.cpu(), gate=gate.cpu())
+    o_r, ht_r = _exact(y.cpu(), wf.cpu(), wg.cpu(), w.cpu(), h0.cpu(), N, T, H, D, cols, True, False, 1, groups, **more)
+    if later:
+        o_r = o_r @ torch.eye(H * D, dtype=torch.float64)
+    o, o_0 = (t.view(N, T, -1).cpu() for t in (o, clean[0]))
+    for other in (0, 2):
+        assert torch.equal(o[other], o_0[other]) and torch.equal(ht[other], clean[1][other])
+    for got, want in ((o[1], o_r[1]), (ht[1].cpu(), ht_r[1])):
+        ok = torch.isfinite(want)
+        assert torch.equal(torch.isfinite(got), ok)
+        assert not ok.any() or _rel(got[ok], want[ok]) <= 2e-2

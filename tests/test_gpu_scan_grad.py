@@ -53,3 +53,37 @@ def test_packed_sequences(K, V, segments, monkeypatch):
     monkeypatch.setenv("HDLA_HIP_SEGMENTS", str(segments))
     cu = torch.tensor([0, 5, 5, 101, 117, 300])
     _check(make_inputs(1800, 1, 300, 2, K, V, gk_div=4.0, n_states=5), [0, 1], cu=cu)
+
+
+@pytest.mark.parametrize("K,V,segments", [(64, 64, 1), (64, 128, 1), (128, 64, 1), (128, 128, 1), (64, 128, 4), (128, 64, 4), (128, 128, 4)])
+@pytest.mark.parametrize("where,value", [("do", float("nan")), ("do", float("inf")), ("dht", float("nan")), ("v", float("nan"))])
+def test_a_value_that_is_none_stays_with_its_head(K, V, segments, where, value, monkeypatch):
+    """In chunk 9 of one head, or in its final state's gradient: the other heads and sequences keep their gradients' bits, and what comes
+    behind a gradient does as well."""
+    if segments == 1:
+        monkeypatch.setenv("HDLA_HIP_ROUTE", "classic")
+    monkeypatch.setenv("HDLA_HIP_SEGMENTS", str(segments))
+    T = 330
+    inp = make_inputs(1850, 2, T, 3, K, V, gk_div=8.0)
+    t = [x.bfloat16().to(DEV) for x in (inp.q, inp.k, inp.v, inp.a, inp.b, inp.gk)] + [inp.h0.to(DEV)]
+    do, dht = inp.do.bfloat16().to(DEV), inp.dht.to(DEV)
+
+    def run():
+        x = [y.clone().requires_grad_() for y in t]
+        return torch.autograd.grad(chunk_hrdplr_delta_rule(*x[:6], 2, scale=0.9, initial_state=x[6], output_final_state=True), x, [do, dht])
+
+    clean = run()
+    if where == "dht":
+        dht[1, 2, 3, 5] = value
+    else:
+        (do if where == "do" else t[2])[1, 150, 2, 5] = value
+    for i, (g, g_0) in enumerate(zip(run(), clean)):
+        if i == 6:
+            assert torch.equal(g[0], g_0[0]) and torch.equal(g[1, :2], g_0[1, :2])
+            assert where == "v" or not torch.isfinite(g[1, 2]).all()
+            continue
+        r = g.shape[1] // T
+        bad = torch.zeros(2, T * r, 3, dtype=torch.bool)
+        bad[1, :(160 * r if where == "do" else None), 2] = True
+        assert torch.equal(g[~bad], g_0[~bad]), i
+        assert where == "v" or i == 0 or not torch.isfinite(g[1, :144 * r, 2].float()).all(), i

@@ -51,3 +51,29 @@ def test_packed_sequences(K, V, segments, monkeypatch):
     cu = torch.tensor([0, 5, 5, 101, 117, 300])
     inp = make_inputs(800, 1, 300, 2, K, V, gk_div=4.0, n_states=5)
     _check(inp, [0, 1], cu=cu)
+
+
+@pytest.mark.parametrize("K,V,segments", [(64, 64, 1), (64, 128, 1), (128, 64, 1), (128, 128, 1), (64, 128, 4), (128, 64, 4), (128, 128, 4)])
+@pytest.mark.parametrize("where,value", [("q", float("nan")), ("k", float("nan")), ("v", float("nan")), ("v", float("inf")), ("gk", float("nan")), ("h0", float("nan")),
+                                         ("h0", -float("inf"))])
+def test_a_value_that_is_none_stays_with_its_head(K, V, segments, where, value, monkeypatch):
+    """In chunk 9 of one head, or its initial state: the other heads and sequences and the chunks before it keep their bits."""
+    if segments == 1:
+        monkeypatch.setenv("HDLA_HIP_ROUTE", "classic")
+    monkeypatch.setenv("HDLA_HIP_SEGMENTS", str(segments))
+    inp = make_inputs(850, 2, 330, 3, K, V, gk_div=8.0)
+    t = [x.bfloat16().to(DEV) for x in (inp.q, inp.k, inp.v, inp.a, inp.b, inp.gk)] + [inp.h0.to(DEV)]
+    run = lambda: chunk_hrdplr_delta_rule(*t[:6], 2, scale=0.9, initial_state=t[6], output_final_state=True)
+    with torch.no_grad():
+        o_0, ht_0 = run()
+        if where == "h0":
+            t[6][1, 2, 3, 5] = value
+        else:
+            t[{"q": 0, "k": 1, "v": 2, "gk": 5}[where]][1, 150, 2, 5] = value
+        o, ht = run()
+    bad = torch.zeros(2, 330, 3, dtype=torch.bool)
+    bad[1, 0 if where == "h0" else 144:, 2] = True
+    assert torch.equal(o[~bad], o_0[~bad]) and torch.equal(ht[0], ht_0[0]) and torch.equal(ht[1, :2], ht_0[1, :2])
+    hit = o[1, 160:, 2] if where != "q" else o[1, 150, 2]
+    assert not torch.isfinite(hit.float()).all()
+    assert torch.isfinite(ht[1, 2]).all() == (where == "q")
