@@ -42,5 +42,11 @@ def test_bounds(K, V, bwd, most):
                 continue
             n = _segments(K, V, lanes, chunks, bwd)[0]          # (of many lanes more are taken for fewer)
             assert n in (1, 4, 8, 16, 32) and (n == 1 or lanes * n <= most) and (chunks > 17 or n == 1)
-    # packed sequences: the average length counts
-    assert _segments(K, V, 4, 128, bwd, N=4) == _segments(K, V, 4, 128, bwd)
+
+
+def test_packed_sequences_are_expected_to_be_of_unequal_lengths():
+    """Two sequences of 8 heads: a longest one of 1.6 times the average makes segments worth their launches (1.10)."""
+    assert _segments(128, 64, 16, 66, False) == [1] and _segments(128, 64, 16, 66, False, N=2)[0] > 1
+    for lanes, chunks in ((2, 97), (8, 313), (64, 1000), (2, 1)):
+        for bwd in (False, True):
+            assert _segments(128, 128, lanes, chunks, bwd, N=2)[0] >= _segments(128, 128, lanes, chunks, bwd)[0]
