@@ -12,18 +12,19 @@
 //
 // What bounds it: the state's way from and to HBM (256 sequences of 32 heads, K = V = 128, one token: 1.09 GB), and where the state is
 // in a cache the chain of a token: its values, the LDS fill, two reductions.
+// Figures: us a call on the device, calls in a row in one process; the largest one's depends on where its two states of 0.5 GB lie
+// (193 to 196 with one pair of buffers, 186 with fresh outputs from a graph's pool, 202 for a launch that waits for the last one).
 //   - A token's values are requested before the previous token's arithmetic, the first token's before the state: requests complete in
-//     order, so behind the state they would be waited for as long.  Requested at the token's begin (and converted beside the
-//     load) it was, in us: 4 sequences of 8 heads, 128 x 128, 16 tokens 34.6 -> 30.2; 8 of 16, 64 x 64, 8 tokens 15.4 -> 13.3;
-//     16 of 16, 128 x 128, one token 7.9 -> 7.5.
+//     order, so behind the state they would be waited for as long.
 //   - The column blocks of a head are neighbours in launch order: they are in flight together and memory sees whole rows.  As the second
-//     dimension of the grid they ran thousands of workgroups apart: 256 sequences of 32 heads 211 -> 186, 128 105 -> 92, 64 51 -> 47,
-//     24 of 16 heads 8.8 -> 7.9.  Below 256 workgroups the order it had is kept: there the blocks of a head meet in the
-//     same L2 where the number of heads is a multiple of 8, and the token's values are what is waited for (4 of 16 heads with beta
-//     5.2 against 5.5).  The blocks of a head on one XCD on large grids: 195 to 199 for the 186.
-//   - One branch around the state's loads, not one each: 108 instead of 94 registers a lane at K = 128, four waves a SIMD instead of
-//     five, and still 186 instead of 192 (without the branch) at 256 sequences; held to five waves it spills.  All 128 columns in one
-//     workgroup: 196.
+//     dimension of the grid they ran thousands of workgroups apart.  Below 256 workgroups that order is kept: there the blocks of a head meet
+//     in the same L2 where the number of heads is a multiple of 8, and the token's values are what is waited for (4 sequences of 16 heads with
+//     beta 5.2 against 5.5).
+//     Both together, against values requested at the token's begin and blocks apart: 256 sequences of 32 heads, 128 x 128, one token 199.6 -> 193.2
+//     (204 -> 186 with fresh outputs), 128 of 32 104.2 -> 91.7, 64 of 32 51.7 -> 46.0, 24 of 16 9.5 -> 8.2, 16 of 16 7.5 -> 7.0; 4 of 8, 16 tokens
+//     34.1 -> 29.8; 8 of 16, 64 x 64, 8 tokens 15.1 -> 12.9; 4 of 16, 128 x 128, one token 4.9 -> 5.1 (a graph's replay).
+//   - Tried, where this form took the 186: the blocks of a head on one XCD 195 to 199; no branch around the state's loads instead of one
+//     (94 registers a lane at K = 128 and five waves a SIMD, not 108 and four) 192; all 128 columns in one workgroup 196.  Held to five waves it spills.
 //
 // HD mode (p.beta given) forms the rank terms of the HDLA layer per token from (beta, k, gk) instead of reading
 // them (HRDPLR/hdla_custom.py:19-43): with f = exp(gk) and s = sum_c k_c^2 f_c,
