@@ -134,7 +134,8 @@ int hdla_chunk_fwd(const hdla_dims* dims, const void* q, const void* k, const vo
  * hipMalloc.  It has no counterpart in the reference.  Same arguments and results as hdla_chunk_fwd without the
  * workspace: the kernels use an array of HDLA_STATIC_WORKSPACE_BYTES bytes that is part of the library's device
  * code (every GPU the library runs on holds it until the process ends); the call allocates and frees nothing.
- * A shape whose hdla_workspace_bytes(dims, 0) exceeds that size is refused with HDLA_ERR_STATIC_LIMIT (K = V = 64,
+ * Near that size a call goes without the records of time segments that the library would have chosen (segments 1: results equal to
+ * rounding).  A shape whose hdla_workspace_bytes(dims, 0) exceeds it even so is refused with HDLA_ERR_STATIC_LIMIT (K = V = 64,
  * bf16, classic route: up to 3855 (16-token chunk, head) pairs, e.g. one sequence of 3840 tokens with 16 heads).  All calls on
  * one GPU share the array: calls that may overlap on one GPU (different streams, different threads) race; calls
  * on one stream are safe.  The array's device address is looked up on the first call on each device; make that
