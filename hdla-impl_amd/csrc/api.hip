@@ -104,28 +104,32 @@ constexpr long long SCAN_MAX_RECORDS = 4096;
 struct ScanTime { double step, step_k, load, rec, rec_k, rec_load, launches, chain, chain_k; int most; };   // most: lanes x segments
 constexpr ScanTime SCAN_TIME_FWD{0.18, 0.13, 0.0024, 0.37, 0.12, 0.0015, 6.5, 0.04, 0.73, 128},
     SCAN_TIME_BWD{0.26, 0.20, 0.0042, 0.29, 0.16, 0.0054, 21., 0.37, 0.49, 64};
+// The backward pass that is given the forward one's transitions: the records' launch has the reverse direction's state columns only.
+constexpr ScanTime SCAN_TIME_BWD_KEPT{0.26, 0.20, 0.0042, 0.61, 0.37, 0.0030, 0.5, -0.19, 2.07, 128};
 // chunks: of a sequence on average; longest: of the longest one, whose chain of steps the launch waits for.
 double scan_time(const ScanTime& t, const hdla_dims* d, double lanes, long long chunks, long long longest, int nseg) {
-    const double k = d->K / 64., v = d->V / 64.;
+    const double k = d->K / 64., v = d->V / 64., columns = &t == &SCAN_TIME_BWD_KEPT ? v : k + v;
     const double steps = (double)((chunks + nseg - 1) / nseg), chain = (double)((longest + nseg - 1) / nseg);
     const double walk = std::max(chain * (t.step + t.step_k * k), steps * t.load * lanes * nseg * k * v);
     if (nseg == 1) return walk;
-    return walk + std::max(chain * (t.rec + t.rec_k * k), steps * t.rec_load * lanes * (nseg - 1) * k * (k + v)) + t.launches +
+    return walk + std::max(chain * (t.rec + t.rec_k * k), steps * t.rec_load * lanes * (nseg - 1) * k * columns) + t.launches +
            nseg * (t.chain + t.chain_k * k);
 }
 // The lengths of packed sequences are on the device: the longest one is taken for 1.6 times the average.  128 batches of 2 to 12 sequences
 // of random lengths, forward / backward pass over the best of the five: 5.7 / 3.3 % on average (1.0: 6.4 / 3.5, 2.5: 6.4 / 3.5; a least length as
 // above: 6.3 / 4.2).
 constexpr double PACKED_LONGEST = 1.6;
+long long average_chunks(const hdla_dims* d) { return ((d->T + CHUNK - 1) / CHUNK) / (d->cu_seqlens ? d->N : 1); }
+long long longest_chunks(const hdla_dims* d) { return d->cu_seqlens && d->N > 1 ? (long long)(average_chunks(d) * PACKED_LONGEST) : average_chunks(d); }
 int scan_segments(const hdla_dims* d, bool bwd) {
     if (d->route != HDLA_ROUTE_AUTO) return 1;
     const long long lanes = (long long)d->N * d->H;
     if (d->segments > 0) return (int)std::max(1LL, std::min<long long>({d->segments, SCAN_MAX_SEGMENTS, SCAN_MAX_RECORDS / lanes}));
-    const long long chunks = ((d->T + CHUNK - 1) / CHUNK) / (d->cu_seqlens ? d->N : 1);
+    const long long chunks = average_chunks(d);
     int nseg = 1;
     if (d->in_dtype != HDLA_FP32) {
         const ScanTime& t = bwd ? SCAN_TIME_BWD : SCAN_TIME_FWD;
-        const long long longest = d->cu_seqlens && d->N > 1 ? (long long)(chunks * PACKED_LONGEST) : chunks;
+        const long long longest = longest_chunks(d);
         double best = scan_time(t, d, (double)lanes, chunks, longest, 1);
         for (int n = 4; n <= SCAN_MAX_SEGMENTS && lanes * n <= t.most; n *= 2) {      // (two only make up for the second walk)
             const double x = scan_time(t, d, (double)lanes, chunks, longest, n);
@@ -138,6 +142,42 @@ int scan_segments(const hdla_dims* d, bool bwd) {
     // 72/152 (8); K = V = 128, 4 lanes of 125 chunks 816/894 -> 155/282 (16).
     while (nseg * 2 <= SCAN_MAX_SEGMENTS && lanes * nseg * 2 <= 128 && chunks / (nseg * 2) >= 4) nseg *= 2;
     return nseg >= 4 ? nseg : 1;
+}
+
+// Segments of the passes that keep and are given a forward pass's workspace: as many as asked for (hdla_keep_plan's choice), one where
+// nothing is said.
+int kept_segments(const hdla_dims* d) { return d->segments > 0 ? scan_segments(d, false) : 1; }
+
+// What a training call keeps of its forward pass where nothing else is said: all that the prep kernel forms, which the backward pass would form
+// again (1.6 times the inputs' bytes at K = V = 64), and the records of the segments, if it is little beside the 288 GB of the device.  us on the device,
+// a training step that keeps the inputs -> this: 1 x 256 tokens, 2 heads, K = V = 64 43 -> 37; 2 x 1537 tokens, 8 heads, K = V = 128 214 -> 185;
+// 4 x 1000 tokens, 16 heads 430 -> 393; 4 x 500, 8 heads 127 -> 107; fp32, 2 x 1003 tokens, 8 heads, K = V = 64 227 -> 190.
+constexpr size_t KEEP_MOST = (size_t)256 << 20;
+// Segments of the two passes of such a call (return, bwd).  The backward pass takes the forward one's, whose entering states and transitions are there,
+// or none.  2-byte elements: by the time of both; over passes of 16 to 313 chunks and 1 to 32 lanes, K, V in {64, 128}, 143 shapes in 1 to 32 segments,
+// 0.3 % over the best on average, 6 % at the most (each pass's own choice: 1.0 and 12 %).  4-byte elements: as scan_segments; at K = 128 four segments
+// from eight chunks on (us, 16 lanes of 8 chunks 166 -> 140).
+int kept_plan_segments(const hdla_dims* d, int32_t& bwd) {
+    bwd = 1;
+    if (d->route != HDLA_ROUTE_AUTO) return 1;
+    if (d->segments > 0) return bwd = scan_segments(d, false);
+    const long long lanes = (long long)d->N * d->H, chunks = average_chunks(d), longest = longest_chunks(d);
+    if (d->in_dtype == HDLA_FP32) {
+        const int n = scan_segments(d, false);
+        return bwd = n == 1 && d->K == 128 && chunks >= 8 && lanes <= 32 ? 4 : n;
+    }
+    if (fused_shape(d)) return 1;
+    int fwd = 1;
+    double best = 0;
+    for (int n = 1; n == 1 || (n <= SCAN_MAX_SEGMENTS && lanes * n <= SCAN_TIME_BWD_KEPT.most); n = n == 1 ? 4 : 2 * n) {
+        const double f = scan_time(SCAN_TIME_FWD, d, (double)lanes, chunks, longest, n);
+        for (int b = 1;; b = n) {
+            const double x = f + scan_time(SCAN_TIME_BWD_KEPT, d, (double)lanes, chunks, longest, b);
+            if ((n == 1 && b == 1) || x < best) { best = x; fwd = n; bwd = b; }
+            if (b == n) break;
+        }
+    }
+    return fwd;
 }
 
 struct FusedLayout {
@@ -265,11 +305,12 @@ int make_layout(const hdla_dims* d, int pass, WsLayout& L, int& nch) {
         L.CHUNK_OFF = take((size_t)(2 * d->N + 1) * 4);          // chunk_off [N+1], then order [N]
         L.CHUNK_SEQ = take((size_t)(nch > 0 ? nch : 1) * 4);
     }
-    const int nseg = pass == HDLA_PASS_FWD || pass == HDLA_PASS_BWD ? scan_segments(d, pass == HDLA_PASS_BWD) : 1;
+    const int nseg = pass == HDLA_PASS_FWD || pass == HDLA_PASS_BWD ? scan_segments(d, pass == HDLA_PASS_BWD) : kept_segments(d);
     if (nseg > 1) {
         const size_t recs = (size_t)d->N * d->H * nseg, state = recs * K * V * 4, matrix = recs * K * K * 4;
-        L.SEG_LOC = take(state); L.SEG_TR = take(matrix); L.SEG_IN = take(state);
+        if (prep_out) { L.SEG_LOC = take(state); L.SEG_TR = take(matrix); L.SEG_IN = take(state); }
         if (pass == HDLA_PASS_BWD) { L.SEG_RLOC = take(state); L.SEG_RTR = take(matrix); L.SEG_RIN = take(state); }
+        if (pass == HDLA_PASS_BWD_KEPT) { L.SEG_RLOC = take(state); L.SEG_RIN = take(state); }
     }
     L.total = off > 0 ? off : 256;
     return HDLA_OK;
@@ -349,13 +390,21 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
     a.beta = static_cast<const T*>(beta); a.dbeta = static_cast<T*>(dbeta);
     bind_ws(a, d, LP, prep_ws, LS, pass == HDLA_PASS_BWD_KEPT ? workspace : prep_ws, nch);
     a.seg = SegRec{1, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-    const int nseg = on_kept ? 1 : scan_segments(d, !fwd);
+    const int nseg = on_kept ? kept_segments(d) : scan_segments(d, !fwd);
     if (nseg > 1) {
-        const auto at = [&](size_t o) { return reinterpret_cast<float*>(static_cast<char*>(workspace) + o); };
-        a.seg = SegRec{nseg, at(LP.SEG_LOC), at(LP.SEG_TR), at(LP.SEG_IN), at(LP.SEG_RLOC), at(LP.SEG_RTR), at(LP.SEG_RIN)};
+        const auto at = [](void* base, size_t o) { return reinterpret_cast<float*>(static_cast<char*>(base) + o); };
+        a.seg = SegRec{nseg, at(prep_ws, LP.SEG_LOC), at(prep_ws, LP.SEG_TR), at(prep_ws, LP.SEG_IN), nullptr, nullptr, nullptr};
+        if (!fwd) { a.seg.rloc = at(workspace, LS.SEG_RLOC); a.seg.rin = at(workspace, LS.SEG_RIN); }
+        if (pass == HDLA_PASS_BWD) a.seg.rtr = at(workspace, LS.SEG_RTR);
     }
     hipError_t e;
-    if (pass == HDLA_PASS_BWD_KEPT) stages &= ~HDLA_STAGE_PREP;    // the forward pass has run it
+    if (pass == HDLA_PASS_BWD_KEPT) {
+        stages &= ~HDLA_STAGE_PREP;                                // the forward pass has run it
+        if (d->cu_seqlens) {
+            e = launch_clear_uncovered(d->cu_seqlens, d->N, d->T, packed_outputs(d, a), stream);
+            if (e != hipSuccess) return (int)e;
+        }
+    }
     if (d->cu_seqlens && (stages & HDLA_STAGE_PREP)) {
         char* base = static_cast<char*>(prep_ws);
         e = launch_chunk_table(d->cu_seqlens, d->N, d->T, nch, reinterpret_cast<int32_t*>(base + LP.CHUNK_OFF),
@@ -367,7 +416,8 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
         if (e != hipSuccess) return (int)e;
     }
     if (a.seg.nseg > 1 && (stages & HDLA_STAGE_CHAIN)) {
-        e = launch_scan_segments<T>(a, d->K, d->V, !fwd, stream);
+        const SegStart what = pass == HDLA_PASS_FWD ? SEG_FWD : pass == HDLA_PASS_FWD_KEEP ? SEG_FWD_KEPT : pass == HDLA_PASS_BWD ? SEG_BWD : SEG_BWD_KEPT;
+        e = launch_scan_segments<T>(a, d->K, d->V, what, stream);
         if (e != hipSuccess) return (int)e;
     }
     // the two scans of the backward pass are independent of each other: one launch when both are asked for
@@ -579,6 +629,19 @@ size_t hdla_record_workspace_bytes(const hdla_dims* dims) {
     FusedLayout L;
     if (!hdla_record_bytes(dims)) return hdla_workspace_bytes(dims, HDLA_PASS_BWD);
     return make_fused_layout(dims, PASS_BWD_RECORD, L) ? 0 : L.total;
+}
+
+size_t hdla_keep_plan(const hdla_dims* dims, int32_t* fwd_segments, int32_t* bwd_segments) {
+    bool fused_fwd, fused_bwd;
+    if (!fwd_segments || !bwd_segments || check_dims(dims) || dims->T < 1) return 0;
+    if (pick_route(dims, HDLA_PASS_FWD, false, fused_fwd) || pick_route(dims, HDLA_PASS_BWD, false, fused_bwd) || fused_fwd || fused_bwd) return 0;
+    hdla_dims d = *dims;
+    WsLayout L;
+    int nch;
+    d.segments = kept_plan_segments(dims, *bwd_segments);
+    *fwd_segments = d.segments;
+    if (make_layout(&d, HDLA_PASS_FWD_KEEP, L, nch) || L.total > KEEP_MOST) return 0;
+    return L.total;
 }
 
 int hdla_workspace_layout(const hdla_dims* dims, int pass, hdla_ws_layout* out) {

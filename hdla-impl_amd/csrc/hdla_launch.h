@@ -16,6 +16,8 @@ struct PackedOut {
 };
 hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int32_t* chunk_off, int32_t* chunk_seq, const PackedOut& out,
                               hipStream_t stream);
+// only what clears the rows that belong to no sequence
+hipError_t launch_clear_uncovered(const int64_t* cu, int N, int T, const PackedOut& out, hipStream_t stream);
 
 // K, V in {64, 128}; returns hipErrorInvalidValue for any other pair.
 // mode: 0 = for the forward pass, 1 = for the backward pass, 2 = forward pass whose workspace the backward pass will use
@@ -27,8 +29,14 @@ template <typename T> hipError_t launch_scan_out(const ChunkArgs<T>& a, int K, i
 template <typename T> hipError_t launch_scan_bwd(const ChunkArgs<T>& a, int K, int V, hipStream_t stream);
 // both in one launch
 template <typename T> hipError_t launch_scan_pair(const ChunkArgs<T>& a, int K, int V, hipStream_t stream);
-// several time segments per sequence: what the scans above start their segments from (both: of the backward pass; else of launch_scan_out)
-template <typename T> hipError_t launch_scan_segments(const ChunkArgs<T>& a, int K, int V, bool both, hipStream_t stream);
+// several time segments per sequence: what the scans above start their segments from
+enum SegStart {
+    SEG_FWD,          // of launch_scan_out, after launch_prep of mode 0
+    SEG_FWD_KEPT,     // the same after mode 2
+    SEG_BWD,          // of the two scans of the backward pass, after mode 1
+    SEG_BWD_KEPT      // the reverse scan's alone, on the states and transitions that SEG_FWD_KEPT left (seg.rtr is not there)
+};
+template <typename T> hipError_t launch_scan_segments(const ChunkArgs<T>& a, int K, int V, SegStart what, hipStream_t stream);
 template <typename T> hipError_t launch_chunk_grad(const ChunkArgs<T>& a, int K, int V, hipStream_t stream);
 template <typename T> hipError_t launch_recurrent(const RecurrentArgs<T>& a, int K, int V, hipStream_t stream);
 

@@ -42,6 +42,7 @@ using torch::autograd::variable_list;
 struct Api {
 #define HDLA_FN(name) decltype(&hdla_##name) name
     HDLA_FN(strerror); HDLA_FN(workspace_bytes); HDLA_FN(record_bytes); HDLA_FN(record_workspace_bytes); HDLA_FN(chunk_fwd_b); HDLA_FN(chunk_bwd_b);
+    HDLA_FN(keep_plan); HDLA_FN(chunk_fwd_keep); HDLA_FN(chunk_bwd_kept);
     HDLA_FN(recurrent_fwd); HDLA_FN(param_recurrent_fwd); HDLA_FN(normalize_fwd); HDLA_FN(normalize_bwd);
     HDLA_FN(normalize_workspace_bytes); HDLA_FN(layer_pre_fwd); HDLA_FN(layer_pre_bwd); HDLA_FN(layer_up_fwd); HDLA_FN(layer_down);
     HDLA_FN(layer_up_wgrad); HDLA_FN(layer_up_wgrad_workspace_bytes); HDLA_FN(rows_gemm); HDLA_FN(sum_partials); HDLA_FN(stack_rows);
@@ -96,8 +97,9 @@ bool env_is(const char* name, std::initializer_list<const char*> values, bool un
     return false;
 }
 bool keep_forward_default() { return !env_is("HDLA_HIP_KEEP_FORWARD", {"", "0", "false", "False"}, true); }
-// launch plan and record of a chunked call
-struct Plan { int32_t route, segments; bool record; };
+bool keep_forward_unsaid() { return env("HDLA_HIP_KEEP_FORWARD") == nullptr; }
+// launch plan of a chunked call, and what its backward pass may be given: the record, and where the route has none the forward pass's workspace
+struct Plan { int32_t route, segments; bool record, keep; };
 // false: the Python code has to look at it (another spelling, a number that is none)
 bool read_plan(Plan& p) {
     const char* r = env("HDLA_HIP_ROUTE");
@@ -106,6 +108,7 @@ bool read_plan(Plan& p) {
     else if (!strcmp(r, "fused")) p.route = HDLA_ROUTE_FUSED;
     else return false;
     p.record = env_is("HDLA_HIP_INPUTS_ONLY", {"", "0", "false", "False"}, true);
+    p.keep = false;
     p.segments = 0;
     const char* s = env("HDLA_HIP_SEGMENTS");
     if (!s) return true;
@@ -132,11 +135,11 @@ void chunk_dims(const ChunkIn& x, double scale, const Plan& p, hdla_dims& d) {
     d.cu_seqlens = x.cu.defined() ? x.cu.data_ptr<int64_t>() : nullptr;
 }
 
-// The launch plan of a backward pass is that of its forward pass, whatever the environment says by then: the record is laid out by it.
-void keep_plan(AutogradContext* ctx, const Plan& p) { ctx->saved_data["plan"] = std::vector<int64_t>{p.route, p.segments}; }
-Plan kept_plan(AutogradContext* ctx) {
+// The launch plan of a backward pass is that of its forward pass, whatever the environment says by then: what that left is laid out by it.
+void save_plan(AutogradContext* ctx, const Plan& p) { ctx->saved_data["plan"] = std::vector<int64_t>{p.route, p.segments, p.keep}; }
+Plan saved_plan(AutogradContext* ctx) {
     const auto p = ctx->saved_data["plan"].toIntVector();
-    return {(int32_t)p[0], (int32_t)p[1], false};
+    return {(int32_t)p[0], (int32_t)p[1], false, p[2] != 0};
 }
 
 // with_record: of a backward pass that is given the forward pass's record
@@ -148,15 +151,46 @@ Tensor workspace(const hdla_dims& d, int pass, const Tensor& like, bool with_rec
     return bytes_like(like, n);
 }
 
-void chunk_forward(const ChunkIn& x, const hdla_dims& d, bool want_ht, bool want_boundary, Tensor& o, Tensor& ht, Tensor& boundary) {
+// left: what the backward pass is given (undefined: the inputs are all); plan: the one that pass is to run with
+void chunk_forward(const ChunkIn& x, const hdla_dims& d, bool want_ht, Plan* plan, Tensor& o, Tensor& ht, Tensor& left) {
     const auto f32 = x.q.options().dtype(at::kFloat);
     o = at::empty_like(x.v);
     if (want_ht) ht = at::empty({d.N, d.H, d.K, d.V}, f32);
-    const size_t nb = want_boundary ? api.record_bytes(&d) : 0;
-    if (nb) boundary = bytes_like(x.q, nb);
+    const size_t nb = plan && plan->record ? api.record_bytes(&d) : 0;
+    if (plan && plan->keep) {
+        hdla_dims k = d;
+        int32_t for_bwd = 0;
+        const size_t n = plan->record && !nb ? api.keep_plan(&d, &k.segments, &for_bwd) : 0;
+        plan->keep = n > 0;
+        if (n) {
+            left = bytes_like(x.q, n);
+            plan->segments = for_bwd;
+            check(api.chunk_fwd_keep(&k, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.beta), ptr(x.gk), fptr(x.h0), ptr(o), fptr(ht),
+                                     ptr(left), n, stream_of(x.q)), "hdla_chunk_fwd_keep");
+            return;
+        }
+    }
+    if (nb) left = bytes_like(x.q, nb);
     const Tensor ws = workspace(d, HDLA_PASS_FWD, x.q);
     check(api.chunk_fwd_b(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.beta), ptr(x.gk), fptr(x.h0), ptr(o), fptr(ht),
-                          ptr(boundary), nb, ptr(ws), (size_t)ws.numel(), stream_of(x.q)), "hdla_chunk_fwd_b");
+                          ptr(left), nb, ptr(ws), (size_t)ws.numel(), stream_of(x.q)), "hdla_chunk_fwd_b");
+}
+
+struct ChunkGrads { Tensor q, k, v, a, b, beta, gk, h0; };      // of what is defined
+Tensor backward_workspace(const hdla_dims& d, const Plan& plan, const Tensor& like, const Tensor& left) {
+    return plan.keep ? workspace(d, HDLA_PASS_BWD_KEPT, like) : workspace(d, HDLA_PASS_BWD, like, left.defined());
+}
+void chunk_backward(const ChunkIn& x, const hdla_dims& d, const Plan& plan, const Tensor& d_o, const Tensor& dht, const Tensor& left, const Tensor& ws,
+                    const ChunkGrads& g) {
+    if (plan.keep) {
+        check(api.chunk_bwd_kept(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.beta), ptr(x.gk), fptr(x.h0), ptr(d_o), fptr(dht),
+                                 ptr(g.q), ptr(g.k), ptr(g.v), ptr(g.a), ptr(g.b), ptr(g.beta), ptr(g.gk), fptr(g.h0), ptr(left),
+                                 (size_t)left.numel(), ptr(ws), (size_t)ws.numel(), stream_of(x.q)), "hdla_chunk_bwd_kept");
+        return;
+    }
+    check(api.chunk_bwd_b(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.beta), ptr(x.gk), fptr(x.h0), ptr(d_o), fptr(dht),
+                          ptr(g.q), ptr(g.k), ptr(g.v), ptr(g.a), ptr(g.b), ptr(g.beta), ptr(g.gk), fptr(g.h0), ptr(left),
+                          left.defined() ? (size_t)left.numel() : 0, ptr(ws), (size_t)ws.numel(), stream_of(x.q)), "hdla_chunk_bwd_b");
 }
 
 // The autograd node: the contract of ChunkDPLRDeltaRuleFunction and ChunkHDLAFunction (the inputs and, where the route
@@ -164,15 +198,15 @@ void chunk_forward(const ChunkIn& x, const hdla_dims& d, bool want_ht, bool want
 struct ChunkFn : torch::autograd::Function<ChunkFn> {
     static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Maybe& a, const Maybe& b,
                                  const Maybe& beta, const Tensor& gk, const Maybe& h0, const Maybe& cu, double scale, bool want_ht,
-                                 const Plan& plan) {
+                                 Plan plan) {
         ChunkIn x{q, k, v, value(a), value(b), value(beta), gk, value(h0), value(cu)};
         if (h0) x.h0 = h0->to(at::kFloat).contiguous();
         hdla_dims d;
         chunk_dims(x, scale, plan, d);
-        keep_plan(ctx, plan);
-        Tensor o, ht, boundary;
-        chunk_forward(x, d, want_ht, plan.record, o, ht, boundary);
-        ctx->save_for_backward({q, k, v, x.a, x.b, x.beta, gk, value(h0), x.cu, boundary});
+        Tensor o, ht, left;
+        chunk_forward(x, d, want_ht, &plan, o, ht, left);
+        save_plan(ctx, plan);
+        ctx->save_for_backward({q, k, v, x.a, x.b, x.beta, gk, value(h0), x.cu, left});
         ctx->saved_data["scale"] = scale;
         ctx->set_materialize_grads(false);
         return want_ht ? variable_list{o, ht} : variable_list{o};
@@ -183,26 +217,23 @@ struct ChunkFn : torch::autograd::Function<ChunkFn> {
     static variable_list gradients(AutogradContext* ctx, const variable_list& grads) {
         const auto s = ctx->get_saved_variables();
         ChunkIn x{s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7], s[8]};
-        const Tensor& boundary = s[9];
         const at::DeviceGuard guard(x.q.device());
         if (x.h0.defined()) x.h0 = x.h0.to(at::kFloat).contiguous();
+        const Plan plan = saved_plan(ctx);
         hdla_dims d;
-        chunk_dims(x, ctx->saved_data["scale"].toDouble(), kept_plan(ctx), d);
+        chunk_dims(x, ctx->saved_data["scale"].toDouble(), plan, d);
         const Tensor d_o = grads[0].defined() ? grads[0].to(x.v.scalar_type()).contiguous() : at::zeros_like(x.v);
         Tensor dht;
         if (grads.size() > 1 && grads[1].defined()) dht = grads[1].to(at::kFloat).contiguous();
-        const Tensor ws = workspace(d, HDLA_PASS_BWD, x.q, boundary.defined());
-        const Tensor dq = at::empty_like(x.q), dk = at::empty_like(x.k), dv = at::empty_like(x.v), dgk = at::empty_like(x.gk);
-        Tensor da, db, dbeta, dh0;
-        if (x.beta.defined()) dbeta = at::empty_like(x.beta);
-        else { da = at::empty_like(x.a); db = at::empty_like(x.b); }
-        if (x.h0.defined()) dh0 = at::empty_like(x.h0);
-        check(api.chunk_bwd_b(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.beta), ptr(x.gk), fptr(x.h0), ptr(d_o), fptr(dht),
-                              ptr(dq), ptr(dk), ptr(dv), ptr(da), ptr(db), ptr(dbeta), ptr(dgk), fptr(dh0), ptr(boundary),
-                              boundary.defined() ? (size_t)boundary.numel() : 0, ptr(ws), (size_t)ws.numel(), stream_of(x.q)),
-              "hdla_chunk_bwd_b");
-        if (dh0.defined()) dh0 = dh0.to(s[7].scalar_type());
-        return {dq, dk, dv, da, db, dbeta, dgk, dh0, Tensor(), Tensor(), Tensor(), Tensor()};
+        const Tensor ws = backward_workspace(d, plan, x.q, s[9]);
+        ChunkGrads r;
+        r.q = at::empty_like(x.q); r.k = at::empty_like(x.k); r.v = at::empty_like(x.v); r.gk = at::empty_like(x.gk);
+        if (x.beta.defined()) r.beta = at::empty_like(x.beta);
+        else { r.a = at::empty_like(x.a); r.b = at::empty_like(x.b); }
+        if (x.h0.defined()) r.h0 = at::empty_like(x.h0);
+        chunk_backward(x, d, plan, d_o, dht, s[9], ws, r);
+        if (r.h0.defined()) r.h0 = r.h0.to(s[7].scalar_type());
+        return {r.q, r.k, r.v, r.a, r.b, r.beta, r.gk, r.h0, Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };
 
@@ -343,6 +374,7 @@ PyObject* run_chunk(ChunkIn& x, PyObject* pscale, PyObject* pwant, PyObject* pke
     else if (!number(pscale, scale)) return none();
     Plan plan;
     if (!read_plan(plan)) return none();
+    plan.keep = pkeep == Py_None && keep_forward_unsaid();
     return guarded([&]() -> PyObject* {
         hdla_dims d;
         chunk_dims(x, scale, plan, d);
@@ -358,8 +390,8 @@ PyObject* run_chunk(ChunkIn& x, PyObject* pscale, PyObject* pwant, PyObject* pke
                 return;
             }
             if (x.h0.defined()) x.h0 = x.h0.to(at::kFloat).contiguous();
-            Tensor boundary;
-            chunk_forward(x, d, want, false, o, ht, boundary);
+            Tensor left;
+            chunk_forward(x, d, want, nullptr, o, ht, left);
         });
         return pair(o, ht);
     });
@@ -590,7 +622,7 @@ Tensor project(const Tensor& x, const Tensor& w) {
     return y;
 }
 // everything between x and the output; what the backward pass needs of it
-struct LayerFwd { Tensor x, w, y, f, g, o, n, out, ht, boundary; ChunkIn op; hdla_dims dims; };
+struct LayerFwd { Tensor x, w, y, f, g, o, n, out, ht, left; ChunkIn op; hdla_dims dims; };
 
 // A few tokens: what is between the projections in one to three launches, without the tensors that the steps would hand on (see
 // in_few_launches).  One token after a cached state, us a
@@ -653,8 +685,8 @@ bool in_few_launches(int64_t rows, int64_t T, int64_t d, bool norm_in_step) {
     return rows * d <= (norm_in_step ? 3 << 18 : 3 << 17);
 }
 
-// params: wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo; r.w gathered; keep: a backward pass follows
-void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, const Plan& plan, const Tensor& h0, bool want_ht, bool chunked, bool keep,
+// params: wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo; r.w gathered; keep: a backward pass follows (which plan is for then)
+void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, Plan& plan, const Tensor& h0, bool want_ht, bool chunked, bool keep,
                    LayerFwd& r) {
     const int64_t B = x3.size(0), T = x3.size(1), d = x3.size(2), rows = B * T;
     const LayerCols L(d, f.H, r.w.size(0) != LayerCols(d, f.H, false).ld);
@@ -681,7 +713,7 @@ void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, const P
     hdla_dims& cd = r.dims;
     chunk_dims(in, 1.0, plan, cd);
     if (chunked) {
-        chunk_forward(in, cd, want_ht, keep && plan.record, r.o, r.ht, r.boundary);
+        chunk_forward(in, cd, want_ht, keep ? &plan : nullptr, r.o, r.ht, r.left);
     } else {
         r.o = at::empty_like(in.v);
         if (want_ht) r.ht = at::empty({cd.N, cd.H, cd.K, cd.V}, opt.dtype(at::kFloat));
@@ -709,13 +741,13 @@ Tensor weight_grad(const Tensor& dy, const Tensor& x) {
 struct LayerFn : torch::autograd::Function<LayerFn> {
     static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& wq, const Tensor& wk, const Tensor& wv, const Tensor& wf0,
                                  const Tensor& wg0, const Tensor& wbeta, const Tensor& wf1, const Tensor& wg1, const Tensor& wnorm,
-                                 const Tensor& wo, const Maybe& h0, const LayerCfg& f, bool want_ht, const Plan& plan) {
+                                 const Tensor& wo, const Maybe& h0, const LayerCfg& f, bool want_ht, Plan plan) {
         const Tensor P[10] = {wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo};
         LayerFwd r;
         r.w = gather_weights(P, LayerCols(x.size(2), f.H, x.size(0) * x.size(1) >= PAD_FROM_ROWS));
         layer_forward(x, P, f, plan, value(h0), want_ht, true, true, r);
-        keep_plan(ctx, plan);
-        ctx->save_for_backward({r.x, r.w, r.y, r.f, r.g, r.o, r.n, r.boundary, r.op.q, r.op.k, r.op.v, r.op.beta, r.op.gk, value(h0), wf1, wg1,
+        save_plan(ctx, plan);
+        ctx->save_for_backward({r.x, r.w, r.y, r.f, r.g, r.o, r.n, r.left, r.op.q, r.op.k, r.op.v, r.op.beta, r.op.gk, value(h0), wf1, wg1,
                                 wnorm, wo});
         ctx->saved_data["c"] = std::vector<double>{f.beta_scale, f.c, f.eps};
         ctx->saved_data["i"] = std::vector<int64_t>{f.H, f.groups, f.norm_q, f.norm_v, f.gate_pos, x.size(0), x.size(1)};
@@ -730,7 +762,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
         // state to this thread, and torch's products below would come out in the region's type where kernels read bf16.
         const c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::DispatchKey::AutocastCUDA);
         const auto s = ctx->get_saved_variables();
-        const Tensor &x = s[0], &w = s[1], &y = s[2], &f = s[3], &g = s[4], &o = s[5], &n = s[6], &boundary = s[7];
+        const Tensor &x = s[0], &w = s[1], &y = s[2], &f = s[3], &g = s[4], &o = s[5], &n = s[6], &left = s[7];
         const Tensor &q = s[8], &k = s[9], &v = s[10], &beta = s[11], &gk = s[12], &h0 = s[13], &wf1 = s[14], &wg1 = s[15], &wnorm = s[16],
                      &wo = s[17];
         const at::DeviceGuard guard(x.device());
@@ -767,11 +799,9 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
             Tensor dht;
             if (grads.size() > 1 && grads[1].defined()) dht = grads[1].to(at::kFloat).contiguous();
             hdla_dims cd;
-            chunk_dims(in, 1.0, kept_plan(ctx), cd);
-            const Tensor ws = workspace(cd, HDLA_PASS_BWD, x, boundary.defined());
-            check(api.chunk_bwd_b(&cd, ptr(q), ptr(k), ptr(v), nullptr, nullptr, ptr(beta), ptr(gk), fptr(in.h0), ptr(d_o), fptr(dht), ptr(dq),
-                                  ptr(dk), ptr(dv), nullptr, nullptr, ptr(dbeta), ptr(dgk), fptr(dh0), ptr(boundary),
-                                  boundary.defined() ? (size_t)boundary.numel() : 0, ptr(ws), (size_t)ws.numel(), stream), "hdla_chunk_bwd_b");
+            const Plan plan = saved_plan(ctx);
+            chunk_dims(in, 1.0, plan, cd);
+            chunk_backward(in, cd, plan, d_o, dht, left, backward_workspace(cd, plan, x, left), ChunkGrads{dq, dk, dv, Tensor(), Tensor(), dbeta, dgk, dh0});
             if (dh0.defined()) out[11] = dh0.to(h0.scalar_type());
         }
 
@@ -919,6 +949,7 @@ PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (keep_forward_default() && grad) return none();
     Plan plan;
     if (!read_plan(plan)) return none();
+    plan.keep = keep_forward_unsaid();
     return guarded([&]() -> PyObject* {
         Tensor out, ht;
         if (grad) {
@@ -1006,6 +1037,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
         return nullptr;                                                                                            \
     }
     HDLA_FN(strerror) HDLA_FN(workspace_bytes) HDLA_FN(record_bytes) HDLA_FN(record_workspace_bytes) HDLA_FN(chunk_fwd_b) HDLA_FN(chunk_bwd_b)
+    HDLA_FN(keep_plan) HDLA_FN(chunk_fwd_keep) HDLA_FN(chunk_bwd_kept)
     HDLA_FN(recurrent_fwd) HDLA_FN(param_recurrent_fwd) HDLA_FN(normalize_fwd) HDLA_FN(normalize_bwd)
     HDLA_FN(normalize_workspace_bytes) HDLA_FN(layer_pre_fwd) HDLA_FN(layer_pre_bwd) HDLA_FN(layer_up_fwd) HDLA_FN(layer_down)
     HDLA_FN(layer_up_wgrad) HDLA_FN(layer_up_wgrad_workspace_bytes) HDLA_FN(rows_gemm) HDLA_FN(sum_partials) HDLA_FN(stack_rows) HDLA_FN(layer_step)

@@ -452,6 +452,19 @@ __device__ __forceinline__ void clear_bytes(char* p, long long n, long long i, l
         if (head + body + 2 * i < n) *reinterpret_cast<uint16_t*>(p + head + body + 2 * i) = 0;
     }
 }
+// (all threads of `groups` workgroups, of which this is the one numbered `group`)
+__device__ __forceinline__ void clear_uncovered(const int64_t* cu, int N, int T, const PackedOut& out, int group, int groups, int t) {
+    const ClearRange r = uncovered(cu, N, T, t);
+    const long long count = (long long)groups * TABLE_THREADS, i = (long long)group * TABLE_THREADS + t;
+    for (int b = 0; b < out.n; ++b) {
+        char* const p = static_cast<char*>(out.p[b]);
+        clear_bytes(p, r.lo * out.row[b], i, count);
+        clear_bytes(p + r.hi * out.row[b], (T - r.hi) * out.row[b], i, count);
+    }
+}
+__global__ __launch_bounds__(TABLE_THREADS) void clear_uncovered_kernel(const int64_t* cu, int N, int T, PackedOut out) {
+    clear_uncovered(cu, N, T, out, blockIdx.x, gridDim.x, threadIdx.x);
+}
 __global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const int64_t* cu, int N, int T, int nch, int32_t* chunk_off,
                                                                           int32_t* chunk_seq, int rankers, PackedOut out) {
     constexpr int LONG_SEQ = 64, LONG_LIST = 512;
@@ -466,14 +479,7 @@ __global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const 
     };
     int32_t* order = chunk_off + N + 1;
     if ((int)blockIdx.x > rankers) {
-        const ClearRange r = uncovered(cu, N, T, t);
-        const long long count = (long long)((int)gridDim.x - 1 - rankers) * TABLE_THREADS;
-        const long long i = (long long)((int)blockIdx.x - 1 - rankers) * TABLE_THREADS + t;
-        for (int b = 0; b < out.n; ++b) {
-            char* const p = static_cast<char*>(out.p[b]);
-            clear_bytes(p, r.lo * out.row[b], i, count);
-            clear_bytes(p + r.hi * out.row[b], (T - r.hi) * out.row[b], i, count);
-        }
+        clear_uncovered(cu, N, T, out, (int)blockIdx.x - 1 - rankers, (int)gridDim.x - 1 - rankers, t);
         return;
     }
     if (blockIdx.x > 0) {
@@ -570,15 +576,23 @@ hipError_t launch_prep(const ChunkArgs<T>& a, int K, int V, int mode, hipStream_
 template hipError_t launch_prep<bf16>(const ChunkArgs<bf16>&, int, int, int, hipStream_t);
 template hipError_t launch_prep<float>(const ChunkArgs<float>&, int, int, int, hipStream_t);
 
-hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int32_t* chunk_off, int32_t* chunk_seq, const PackedOut& out,
-                              hipStream_t stream) {
-    const int rankers = N <= ORDER_MAX_N ? (N + TABLE_THREADS - 1) / TABLE_THREADS : 0;
-    // workgroups that look for rows to clear: one for every 16 KiB they might have to write, as many as fill the device, and fewer
-    // where each has a long table to read first
+// workgroups that look for rows to clear: one for every 16 KiB they might have to write, as many as fill the device, and fewer
+// where each has a long table to read first
+static int clearing_workgroups(int N, int T, const PackedOut& out) {
     long long bytes = 0;
     for (int b = 0; b < out.n; ++b) bytes += out.row[b] * T;
     const long long most = max(32, min(512, (1 << 20) / N));
-    const int clearers = (int)min((bytes + 16383) / 16384, most);
+    return (int)min((bytes + 16383) / 16384, most);
+}
+hipError_t launch_clear_uncovered(const int64_t* cu, int N, int T, const PackedOut& out, hipStream_t stream) {
+    const int clearers = clearing_workgroups(N, T, out);
+    if (clearers == 0) return hipSuccess;
+    hipLaunchKernelGGL(clear_uncovered_kernel, dim3(clearers), dim3(TABLE_THREADS), 0, stream, cu, N, T, out);
+    return hipGetLastError();
+}
+hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int32_t* chunk_off, int32_t* chunk_seq, const PackedOut& out,
+                              hipStream_t stream) {
+    const int rankers = N <= ORDER_MAX_N ? (N + TABLE_THREADS - 1) / TABLE_THREADS : 0, clearers = clearing_workgroups(N, T, out);
     hipLaunchKernelGGL(build_chunk_table_kernel, dim3(1 + rankers + clearers), dim3(TABLE_THREADS), 0, stream, cu, N, T, nch, chunk_off, chunk_seq,
                        rankers, out);
     return hipGetLastError();

@@ -44,23 +44,23 @@ hipError_t launch_scan_pair(const ChunkArgs<T>& a, int K, int V, hipStream_t str
     return launch_scan<T>(a, K, V, SCAN_PAIR, stream);
 }
 template <typename T>
-hipError_t launch_scan_segments(const ChunkArgs<T>& a, int K, int V, bool both, hipStream_t stream) {
+hipError_t launch_scan_segments(const ChunkArgs<T>& a, int K, int V, SegStart what, hipStream_t stream) {
     if constexpr (sizeof(T) == 2) {
-        if (K == 64 && V == 64) return both ? launch_scan_grad_segments_shape<64, 64>(a, stream) : launch_scan_out_segments_shape<64, 64>(a, stream);
-        if (K == 128 && V == 128) return both ? launch_scan_grad_segments_shape<128, 128>(a, stream) : launch_scan_out_segments_shape<128, 128>(a, stream);
-        if (K == 64 && V == 128) return both ? launch_scan_grad_segments_shape<64, 128>(a, stream) : launch_scan_out_segments_shape<64, 128>(a, stream);
-        if (K == 128 && V == 64) return both ? launch_scan_grad_segments_shape<128, 64>(a, stream) : launch_scan_out_segments_shape<128, 64>(a, stream);
+        if (K == 64 && V == 64) return what == SEG_FWD ? launch_scan_out_segments_shape<64, 64>(a, stream) : launch_scan_grad_segments_shape<64, 64>(a, what, stream);
+        if (K == 128 && V == 128) return what == SEG_FWD ? launch_scan_out_segments_shape<128, 128>(a, stream) : launch_scan_grad_segments_shape<128, 128>(a, what, stream);
+        if (K == 64 && V == 128) return what == SEG_FWD ? launch_scan_out_segments_shape<64, 128>(a, stream) : launch_scan_grad_segments_shape<64, 128>(a, what, stream);
+        if (K == 128 && V == 64) return what == SEG_FWD ? launch_scan_out_segments_shape<128, 64>(a, stream) : launch_scan_grad_segments_shape<128, 64>(a, what, stream);
         return hipErrorInvalidValue;
     } else {
-        if (K == 64 && V == 64) return launch_scan_segments_shape<T, 64, 64>(a, both, stream);
-        if (K == 128 && V == 128) return launch_scan_segments_shape<T, 128, 128>(a, both, stream);
-        if (K == 64 && V == 128) return launch_scan_segments_shape<T, 64, 128>(a, both, stream);
-        if (K == 128 && V == 64) return launch_scan_segments_shape<T, 128, 64>(a, both, stream);
+        if (K == 64 && V == 64) return launch_scan_segments_shape<T, 64, 64>(a, what, stream);
+        if (K == 128 && V == 128) return launch_scan_segments_shape<T, 128, 128>(a, what, stream);
+        if (K == 64 && V == 128) return launch_scan_segments_shape<T, 64, 128>(a, what, stream);
+        if (K == 128 && V == 64) return launch_scan_segments_shape<T, 128, 64>(a, what, stream);
         return hipErrorInvalidValue;
     }
 }
-template hipError_t launch_scan_segments<bf16>(const ChunkArgs<bf16>&, int, int, bool, hipStream_t);
-template hipError_t launch_scan_segments<float>(const ChunkArgs<float>&, int, int, bool, hipStream_t);
+template hipError_t launch_scan_segments<bf16>(const ChunkArgs<bf16>&, int, int, SegStart, hipStream_t);
+template hipError_t launch_scan_segments<float>(const ChunkArgs<float>&, int, int, SegStart, hipStream_t);
 template hipError_t launch_scan_fwd<bf16>(const ChunkArgs<bf16>&, int, int, hipStream_t);
 template hipError_t launch_scan_fwd<float>(const ChunkArgs<float>&, int, int, hipStream_t);
 template hipError_t launch_scan_out<bf16>(const ChunkArgs<bf16>&, int, int, bool, hipStream_t);

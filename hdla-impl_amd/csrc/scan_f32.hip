@@ -3,11 +3,11 @@
 
 namespace hdla {
 template hipError_t launch_scan_shape<float, 64, 64>(const ChunkArgs<float>&, ScanKind, hipStream_t);
-template hipError_t launch_scan_segments_shape<float, 64, 64>(const ChunkArgs<float>&, bool, hipStream_t);
+template hipError_t launch_scan_segments_shape<float, 64, 64>(const ChunkArgs<float>&, SegStart, hipStream_t);
 template hipError_t launch_scan_shape<float, 64, 128>(const ChunkArgs<float>&, ScanKind, hipStream_t);
-template hipError_t launch_scan_segments_shape<float, 64, 128>(const ChunkArgs<float>&, bool, hipStream_t);
+template hipError_t launch_scan_segments_shape<float, 64, 128>(const ChunkArgs<float>&, SegStart, hipStream_t);
 template hipError_t launch_scan_shape<float, 128, 64>(const ChunkArgs<float>&, ScanKind, hipStream_t);
-template hipError_t launch_scan_segments_shape<float, 128, 64>(const ChunkArgs<float>&, bool, hipStream_t);
+template hipError_t launch_scan_segments_shape<float, 128, 64>(const ChunkArgs<float>&, SegStart, hipStream_t);
 template hipError_t launch_scan_shape<float, 128, 128>(const ChunkArgs<float>&, ScanKind, hipStream_t);
-template hipError_t launch_scan_segments_shape<float, 128, 128>(const ChunkArgs<float>&, bool, hipStream_t);
+template hipError_t launch_scan_segments_shape<float, 128, 128>(const ChunkArgs<float>&, SegStart, hipStream_t);
 }  // namespace hdla

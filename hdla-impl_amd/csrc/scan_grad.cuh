@@ -323,18 +323,17 @@ __global__ __launch_bounds__((RevCfg<K, V, NWC, false>::THREADS)) void scan_grad
     if (y < R::SPLIT) scan_out_body<K, V, NWC, OUT_STATE, true>(p, smem, n, seg, y);
     else scan_rev_body<K, V, NWC, false>(p, smem, n, seg, y - R::SPLIT);
 }
-// the segments' records: grid = (H, 2 (V + K) / 16 / NWC, N * (segments - 1)); forward the segments before the last, in reverse those
-// behind the first
+// the segments' records on a workspace of the backward pass (or that it will read): grid and first_y as scan_sum_kernel's
 template <int K, int V, int NWC>
-__global__ __launch_bounds__((RevCfg<K, V, NWC, true>::THREADS)) void scan_grad_sum_kernel(ChunkArgs<bf16> p) {
+__global__ __launch_bounds__((RevCfg<K, V, NWC, true>::THREADS)) void scan_grad_sum_kernel(ChunkArgs<bf16> p, int first_y) {
     typedef OutCfg<K, V, NWC, OUT_SUM> F;
     typedef RevCfg<K, V, NWC, true> R;
     static_assert(F::THREADS == R::THREADS, "one launch");
     constexpr int COLS = (V + K) / 16 / NWC;
     __shared__ __attribute__((aligned(16))) char smem[F::BYTES > R::BYTES ? F::BYTES : R::BYTES];
     const int z = blockIdx.z / (p.seg.nseg - 1), seg = blockIdx.z % (p.seg.nseg - 1);
-    const int n = scan_sequence(p.st, z), split = blockIdx.y % COLS;
-    if ((int)blockIdx.y < COLS) {
+    const int n = scan_sequence(p.st, z), y = blockIdx.y + first_y, split = y % COLS;
+    if (y < COLS) {
         if (seg == 0 && split >= R::SPLIT) return;        // starts from h0: nobody asks for its transition
         scan_out_body<K, V, NWC, OUT_SUM, true>(p, smem, n, seg, split);
     } else {
@@ -358,14 +357,13 @@ template <int K, int V> hipError_t launch_scan_grad_shape(const ChunkArgs<bf16>&
     if (lanes * (VT / 2) <= SCAN_TARGET_WORKGROUPS) return launch_scan_grad_nwc<K, V, 2>(a, kind, stream);
     return launch_scan_grad_nwc<K, V, 4>(a, kind, stream);
 }
-template <int K, int V> hipError_t launch_scan_grad_segments_shape(const ChunkArgs<bf16>& a, hipStream_t stream) {
+template <int K, int V> hipError_t launch_scan_grad_segments_shape(const ChunkArgs<bf16>& a, SegStart what, hipStream_t stream) {
     constexpr int NWC = 4;
     typedef RevCfg<K, V, NWC, true> C;
-    hipLaunchKernelGGL((scan_grad_sum_kernel<K, V, NWC>), dim3(a.H, 2 * (V + K) / 16 / NWC, a.st.N * (a.seg.nseg - 1)), dim3(C::THREADS), 0, stream, a);
+    hipLaunchKernelGGL((scan_grad_sum_kernel<K, V, NWC>), dim3(a.H, sum_splits<K, V, NWC>(what), a.st.N * (a.seg.nseg - 1)), dim3(C::THREADS), 0,
+                       stream, a, sum_first<K, V, NWC>(what));
     const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((scan_chain_kernel<bf16, K, V>), dim3(a.H, V / 16 * 2, a.st.N), dim3(64 * (K / 16)), 0, stream, a);
-    return hipGetLastError();
+    return e == hipSuccess ? launch_scan_chain<bf16, K, V>(a, what, stream) : e;
 }
 
 }  // namespace hdla

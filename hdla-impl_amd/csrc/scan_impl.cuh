@@ -617,16 +617,17 @@ __global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_pair_ke
     else scan_bwd_body<T, K, V, NWC, OUT_GRAD>(p, smem, n, seg, blockIdx.y - SPLIT);
 }
 // The segments' records: grid = (H, directions * (V + K) / 16 / NWC, N * (segments - 1)); forward the segments before the
-// last, in reverse those behind the first.
+// last, in reverse those behind the first.  first_y: blockIdx.y counts from there on (SEG_BWD_KEPT: the reverse direction's V / 16 / NWC, which
+// leave out the transitions' columns).
 template <typename T, int K, int V, int NWC, bool BOTH>
-__global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_sum_kernel(ChunkArgs<T> p) {
+__global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_sum_kernel(ChunkArgs<T> p, int first_y) {
     constexpr int NF = NSLOT * blk_fwd(K, sizeof(T), false).SIZE;
     constexpr int NB = NSLOT * slot_bwd(K, sizeof(T)).SIZE;
     constexpr int SPLIT = ScanCfg<T, K, V, NWC>::SPLIT, COLS = (V + K) / 16 / NWC;
     __shared__ __attribute__((aligned(16))) char smem[BOTH && NB > NF ? NB : NF];
     const int z = blockIdx.z / (p.seg.nseg - 1), seg = blockIdx.z % (p.seg.nseg - 1);
-    const int n = scan_sequence(p.st, z), split = blockIdx.y % COLS;
-    if (!BOTH || (int)blockIdx.y < COLS) {
+    const int n = scan_sequence(p.st, z), y = blockIdx.y + first_y, split = y % COLS;
+    if (!BOTH || y < COLS) {
         if (seg == 0 && split >= SPLIT) return;           // starts from h0: nobody asks for its transition
         scan_fwd_body<T, K, V, NWC, OUT_SUM>(p, smem, n, seg, split);
     } else {
@@ -635,7 +636,9 @@ __global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_sum_ker
     }
 }
 // The records chained into what enters the segments, X <- M_s X + X_loc(s) from the segment that starts the sequence (or, in
-// reverse, ends it): grid = (H, directions * V/16, N), one wave per 16 rows of the state's column block.  A chain of
+// reverse, ends it): grid = (H, directions * V/16, N), one wave per 16 rows of the state's column block; blockIdx.y counts from first_y on.
+// Without transitions of its own (rtr) the reverse chain takes the forward ones turned: what the state's gradient meets on its way
+// back through a segment is the transpose of what the state met on its way there.  A chain of
 // dependent steps, so a step is kept short: the wave's rows of the next transition matrix are requested a step ahead, the
 // waves exchange their rows through LDS (split operands: the error of fp32 products), one barrier a step.
 // With 4-byte elements the sums are 64-bit (v_mfma_f64_16x16x4_f64): in fp32 a chain step rounds a state K / 4 times more than the
@@ -646,16 +649,16 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 template <typename T> struct ChainState { typedef Split<T> shared; };
 template <> struct ChainState<float> { typedef f64x4 shared; };
 template <typename T, int K, int V>
-__global__ __launch_bounds__(64 * (K / 16)) void scan_chain_kernel(ChunkArgs<T> p) {
+__global__ __launch_bounds__(64 * (K / 16)) void scan_chain_kernel(ChunkArgs<T> p, int first_y) {
     constexpr int KT = K / 16, VT = V / 16;
     constexpr bool WIDE = sizeof(T) == 4;
     typedef typename ChainState<T>::shared Shared;
     __shared__ __attribute__((aligned(16))) Shared sx[2][KT][64];
-    const int h = blockIdx.x, vt = blockIdx.y % VT, n = blockIdx.z, nseg = p.seg.nseg;
-    const bool rev = blockIdx.y >= VT;
+    const int y = blockIdx.y + first_y, h = blockIdx.x, vt = y % VT, n = blockIdx.z, nseg = p.seg.nseg;
+    const bool rev = y >= VT, turned = rev && !p.seg.rtr;
     const int kt = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane_id();
     const float* const loc = rev ? p.seg.rloc : p.seg.loc;
-    const float* const tr = rev ? p.seg.rtr : p.seg.tr;
+    const float* const tr = rev && !turned ? p.seg.rtr : p.seg.tr;
     float* const in = rev ? p.seg.rin : p.seg.in;
     const int64_t rec0 = ((int64_t)n * p.H + h) * nseg;
     // step i handles the i-th segment from the start of the chain
@@ -664,9 +667,18 @@ __global__ __launch_bounds__(64 * (K / 16)) void scan_chain_kernel(ChunkArgs<T> 
     // Register i of lane (g, c) of a 64-bit result is row g + 4 i of the product: the rows of the transition matrix are handed over
     // in the order in which that is row 4 g + i, as everywhere else.
     const int row = WIDE ? (l & 48) + 4 * (l & 3) + ((l >> 2) & 3) : l;
+    // (lane (g, c) of a turned tile: column c of rows 4 g .. 4 g + 3, element c % 4 of the lanes (c / 4, 4 g + i))
+    const int col = (16 * ((row & 15) >> 2) + 4 * (row >> 4)) * 4 + (row & 3);
     auto request = [&](int i, f32x4 (&m)[KT], f32x4& a) __attribute__((always_inline)) {
         i = min(i, nseg - 2);                             // past the end: never used
         a = *reinterpret_cast<const f32x4*>(loc + rec(i) * (K * V) + own);
+        if (turned) {
+#pragma unroll
+            for (int ki = 0; ki < KT; ++ki)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) m[ki][e] = tr[rec(i) * (K * K) + (ki * KT + kt) * TILE + col + 4 * e];
+            return;
+        }
 #pragma unroll
         for (int ki = 0; ki < KT; ++ki) m[ki] = *reinterpret_cast<const f32x4*>(tr + rec(i) * (K * K) + (kt * KT + ki) * TILE + 4 * row);
     };
@@ -732,16 +744,24 @@ hipError_t launch_scan_shape(const ChunkArgs<T>& a, ScanKind kind, hipStream_t s
 }
 
 template <typename T, int K, int V>
-hipError_t launch_scan_segments_shape(const ChunkArgs<T>& a, bool both, hipStream_t stream) {
+static hipError_t launch_scan_chain(const ChunkArgs<T>& a, SegStart what, hipStream_t stream) {
+    hipLaunchKernelGGL((scan_chain_kernel<T, K, V>), dim3(a.H, V / 16 * (what == SEG_BWD ? 2 : 1), a.st.N), dim3(64 * (K / 16)), 0, stream, a,
+                       what == SEG_BWD_KEPT ? V / 16 : 0);
+    return hipGetLastError();
+}
+// workgroups of a (sequence, head, segment) in the launch of the segments' records, and the first of them
+template <int K, int V, int NWC> static int sum_splits(SegStart what) { return what == SEG_BWD_KEPT ? V / 16 / NWC : (V + K) / 16 / NWC * (what == SEG_BWD ? 2 : 1); }
+template <int K, int V, int NWC> static int sum_first(SegStart what) { return what == SEG_BWD_KEPT ? (V + K) / 16 / NWC : 0; }
+template <typename T, int K, int V>
+hipError_t launch_scan_segments_shape(const ChunkArgs<T>& a, SegStart what, hipStream_t stream) {
     constexpr int NWC = 4;                                // column blocks per workgroup: each fetches the chunks' operands once for them
     typedef ScanCfg<T, K, V, NWC> C;
-    dim3 grid(a.H, (V + K) / 16 / NWC * (both ? 2 : 1), a.st.N * (a.seg.nseg - 1)), block(C::THREADS);
-    if (both) hipLaunchKernelGGL((scan_sum_kernel<T, K, V, NWC, true>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((scan_sum_kernel<T, K, V, NWC, false>), grid, block, 0, stream, a);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((scan_chain_kernel<T, K, V>), dim3(a.H, V / 16 * (both ? 2 : 1), a.st.N), dim3(64 * (K / 16)), 0, stream, a);
-    return hipGetLastError();
+    const dim3 grid(a.H, sum_splits<K, V, NWC>(what), a.st.N * (a.seg.nseg - 1)), block(C::THREADS);
+    const int first = sum_first<K, V, NWC>(what);
+    if (what == SEG_BWD || what == SEG_BWD_KEPT) hipLaunchKernelGGL((scan_sum_kernel<T, K, V, NWC, true>), grid, block, 0, stream, a, first);
+    else hipLaunchKernelGGL((scan_sum_kernel<T, K, V, NWC, false>), grid, block, 0, stream, a, first);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? launch_scan_chain<T, K, V>(a, what, stream) : e;
 }
 
 }  // namespace hdla

@@ -428,9 +428,7 @@ template <int K, int V> hipError_t launch_scan_out_segments_shape(const ChunkArg
     typedef OutCfg<K, V, NWC, OUT_SUM> C;
     hipLaunchKernelGGL((scan_out_sum_kernel<K, V, NWC>), dim3(a.H, (V + K) / 16 / NWC, a.st.N * (a.seg.nseg - 1)), dim3(C::THREADS), 0, stream, a);
     const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((scan_chain_kernel<bf16, K, V>), dim3(a.H, V / 16, a.st.N), dim3(64 * (K / 16)), 0, stream, a);
-    return hipGetLastError();
+    return e == hipSuccess ? launch_scan_chain<bf16, K, V>(a, SEG_FWD, stream) : e;
 }
 
 }  // namespace hdla

@@ -5,12 +5,12 @@ The library is the only compute path: if it cannot be loaded every operator rais
 import ctypes
 import os
 import warnings
-from typing import Optional
+from typing import Optional, Tuple
 
 import torch
 
 HDLA_BF16, HDLA_FP32 = 0, 1
-HDLA_VERSION = 205          # the header this binding was written against (struct layouts, entry points)
+HDLA_VERSION = 206          # the header this binding was written against (struct layouts, entry points)
 ROUTE_AUTO, ROUTE_CLASSIC, ROUTE_FUSED = 0, 1, 2
 _ROUTES = {"": ROUTE_AUTO, "auto": ROUTE_AUTO, "classic": ROUTE_CLASSIC, "fused": ROUTE_FUSED}
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -105,6 +105,8 @@ def load():
     lib.hdla_chunk_fwd_b.argtypes = [F] + [P] * 10 + [P, ctypes.c_size_t, P, ctypes.c_size_t, P]
     lib.hdla_chunk_bwd_b.restype = ctypes.c_int
     lib.hdla_chunk_bwd_b.argtypes = [F] + [P] * 18 + [P, ctypes.c_size_t, P, ctypes.c_size_t, P]
+    lib.hdla_keep_plan.restype = ctypes.c_size_t
+    lib.hdla_keep_plan.argtypes = [F, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)]
     lib.hdla_chunk_fwd_keep.restype = ctypes.c_int
     lib.hdla_chunk_fwd_keep.argtypes = [F] + [P] * 10 + [P, ctypes.c_size_t, P]
     lib.hdla_chunk_bwd_kept.restype = ctypes.c_int
@@ -253,6 +255,14 @@ def record(dims: HdlaDims, device) -> Optional[torch.Tensor]:
     return torch.empty(n, dtype=torch.uint8, device=device) if n else None
 
 
+def keep_plan(dims: HdlaDims) -> Tuple[int, int, int]:
+    """What the library suggests a training call keep of its forward pass where the route has no record: bytes (0: nothing), and the
+    segments for hdla_chunk_fwd_keep and hdla_chunk_bwd_kept."""
+    fwd, bwd = ctypes.c_int32(0), ctypes.c_int32(0)
+    n = load().hdla_keep_plan(ctypes.byref(dims), ctypes.byref(fwd), ctypes.byref(bwd))
+    return n, fwd.value, bwd.value
+
+
 def check_cu_seqlens(cu_seqlens: torch.Tensor, T: int) -> None:
     """Validate a packed-sequence table that is still on the CPU (free: no device synchronisation): it must start at
     0, end at T and never decrease.  A table that already lives on the GPU is not read back; the kernels force its
@@ -271,11 +281,12 @@ def check_cu_seqlens(cu_seqlens: torch.Tensor, T: int) -> None:
 PASS_FWD, PASS_BWD, PASS_FWD_KEEP, PASS_BWD_KEPT = 0, 1, 2, 3
 
 
-def keep_forward_default() -> bool:
+def keep_forward_default() -> Optional[bool]:
     """Whether the chunked operators keep the forward pass's per-chunk intermediates for the backward pass when the
-    caller does not say (``keep_forward=None``): environment variable HDLA_HIP_KEEP_FORWARD=1.  Off by default: the
-    reference keeps only the inputs between the passes (HRDPLR/hrdplr.py:137) and so does this library unless asked."""
-    return os.environ.get("HDLA_HIP_KEEP_FORWARD", "0") not in ("", "0", "false", "False")
+    caller does not say (``keep_forward=None``): environment variable HDLA_HIP_KEEP_FORWARD=1 or 0.  Where that does not say
+    either (None), the library keeps them where they are small (``keep_plan``), unless HDLA_HIP_INPUTS_ONLY=1."""
+    v = os.environ.get("HDLA_HIP_KEEP_FORWARD")
+    return None if v is None else v not in ("", "0", "false", "False")
 
 
 def current_stream(device) -> ctypes.c_void_p:

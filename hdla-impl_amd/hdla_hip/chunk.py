@@ -69,17 +69,17 @@ def _dims(q, v, gk, scale, cu_seqlens, n_seq, plan=(None, None)):
 
 
 def chunk_hrdplr_fwd(q, k, v, a, b, gk, scale, initial_state, output_final_state, cu_seqlens=None, keep=False,
-                     beta=None, want_boundary=False):
+                     beta=None, want_boundary=False, plan=(None, None)):
     """Forward launch sequence (HRDPLR/hrdplr.py:25-99) on native shapes: returns (o, final_state), with ``keep`` also
     the workspace the backward pass can run on instead of recomputing it (``hdla_chunk_fwd_keep``), with
     ``want_boundary`` also the record for the backward pass (None where the route has none).
-    With ``beta`` a and b are formed in the kernels (they may be None)."""
+    With ``beta`` a and b are formed in the kernels (they may be None).  ``plan``: route and segments (None: the environment's)."""
     lib = _lib.load()
     B, T, H, K = q.shape
     V = v.shape[-1]
     N = B if cu_seqlens is None else cu_seqlens.numel() - 1
     with torch.cuda.device(q.device):
-        dims = _dims(q, v, gk, scale, cu_seqlens, N)
+        dims = _dims(q, v, gk, scale, cu_seqlens, N, plan)
         o = torch.empty_like(v)
         ht = torch.empty(N, H, K, V, dtype=torch.float32, device=q.device) if output_final_state else None
         if keep:
@@ -101,8 +101,19 @@ def chunk_hrdplr_fwd(q, k, v, a, b, gk, scale, initial_state, output_final_state
     return o, ht
 
 
+def keep_plan(q, v, gk, scale, cu_seqlens):
+    """The plans (route, segments) of a forward pass that keeps its workspace and of the backward pass on it, where the library
+    suggests to keep it; None where it does not."""
+    dims = _dims(q, v, gk, scale, cu_seqlens, q.shape[0] if cu_seqlens is None else cu_seqlens.numel() - 1)
+    n, fwd, bwd = _lib.keep_plan(dims)
+    return ((dims.route, fwd), (dims.route, bwd)) if n and not _lib.load().hdla_record_bytes(ctypes.byref(dims)) else None
+
+
+ONE_SEGMENT = (_lib.ROUTE_AUTO, 1)                        # keep_forward=True: results are those of the classic kernels on whole sequences
+
+
 def chunk_hrdplr_bwd_kept(q, k, v, a, b, gk, scale, initial_state, do, dht, kept, cu_seqlens=None, want_dh0=True,
-                          beta=None):
+                          beta=None, plan=ONE_SEGMENT):
     """Backward launch sequence on the workspace a forward pass kept (``hdla_chunk_bwd_kept``): the per-chunk
     intermediates are read there, not recomputed.  Returns (dq, dk, dv, da, db, dgk, dh0), or with ``beta``
     (dq, dk, dv, dbeta, dgk, dh0)."""
@@ -110,11 +121,10 @@ def chunk_hrdplr_bwd_kept(q, k, v, a, b, gk, scale, initial_state, do, dht, kept
     B, T, H, K = q.shape
     V = v.shape[-1]
     N = B if cu_seqlens is None else cu_seqlens.numel() - 1
+    new = torch.empty_like
     with torch.cuda.device(q.device):
-        dims = _dims(q, v, gk, scale, cu_seqlens, N)
+        dims = _dims(q, v, gk, scale, cu_seqlens, N, plan)
         ws = _lib.workspace(dims, _lib.PASS_BWD_KEPT, q.device)
-        # rows outside every sequence of a packed batch stay unwritten: they must not carry garbage upstream
-        new = torch.zeros_like if cu_seqlens is not None else torch.empty_like
         dq, dk, dv, dgk = new(q), new(k), new(v), new(gk)
         da = db = dbeta = None
         if beta is None:
@@ -179,18 +189,22 @@ class ChunkDPLRDeltaRuleFunction(torch.autograd.Function):
         # keep_forward (off unless asked for): the per-chunk intermediates of this pass stay alive on ctx until the
         # backward pass, which then does not recompute them; only when a gradient can be asked for at all
         ctx.kept = None
-        boundary = None
+        boundary, ctx.plan, ctx.on_kept = None, (_lib.default_route(), _lib.default_segments()), False
         if keep_forward and any(ctx.needs_input_grad):
-            o, final_state, ctx.kept = chunk_hrdplr_fwd(q, k, v, a, b, gk, scale, h0, output_final_state, cu_seqlens, keep=True)
+            o, final_state, ctx.kept = chunk_hrdplr_fwd(q, k, v, a, b, gk, scale, h0, output_final_state, cu_seqlens, keep=True,
+                                                        plan=ONE_SEGMENT)
+            ctx.plan = ONE_SEGMENT
         elif any(ctx.needs_input_grad) and _lib.keep_boundaries_default():
+            plans = keep_plan(q, v, gk, scale, cu_seqlens) if keep_forward is None else None
+            if plans:
+                ctx.on_kept, ctx.plan = True, plans[1]
             o, final_state, boundary = chunk_hrdplr_fwd(q, k, v, a, b, gk, scale, h0, output_final_state, cu_seqlens,
-                                                        want_boundary=True)
+                                                        keep=ctx.on_kept, want_boundary=True, plan=plans[0] if plans else ctx.plan)
         else:
             o, final_state = chunk_hrdplr_fwd(q, k, v, a, b, gk, scale, h0, output_final_state, cu_seqlens)
-        # the inputs (hrdplr.py:137) and, where the route has one, the forward pass's record (37 % of the inputs' bytes;
-        # HDLA_HIP_INPUTS_ONLY=1: strictly the inputs)
+        # the inputs (hrdplr.py:137) and, where the route has one, the forward pass's record (37 % of the inputs' bytes), or its
+        # workspace where that is small (HDLA_HIP_INPUTS_ONLY=1: strictly the inputs)
         ctx.save_for_backward(q, k, v, a, b, gk, initial_state, cu_seqlens, boundary)
-        ctx.plan = _lib.default_route(), _lib.default_segments()
         ctx.scale = scale
         ctx.chunk_size = chunk_size
         ctx.output_final_state = output_final_state
@@ -209,9 +223,10 @@ class ChunkDPLRDeltaRuleFunction(torch.autograd.Function):
         if dht is not None:
             dht = dht.to(torch.float32).contiguous()
         h0 = None if initial_state is None else initial_state.to(torch.float32).contiguous()
-        if ctx.kept is not None:
-            dq, dk, dv, da, db, dgk, dh0 = chunk_hrdplr_bwd_kept(q, k, v, a, b, gk, ctx.scale, h0, do, dht, ctx.kept,
-                                                                 cu_seqlens, want_dh0=initial_state is not None)
+        if ctx.kept is not None or ctx.on_kept:
+            dq, dk, dv, da, db, dgk, dh0 = chunk_hrdplr_bwd_kept(q, k, v, a, b, gk, ctx.scale, h0, do, dht,
+                                                                 boundary if ctx.on_kept else ctx.kept, cu_seqlens,
+                                                                 want_dh0=initial_state is not None, plan=ctx.plan)
         else:
             dq, dk, dv, da, db, dgk, dh0 = chunk_hrdplr_bwd(q, k, v, a, b, gk, ctx.scale, h0, do, dht, cu_seqlens,
                                                             want_dh0=initial_state is not None, boundary=boundary,
@@ -247,8 +262,10 @@ def chunk_hrdplr_delta_rule(
 
     ``keep_forward`` (keyword-only, not in the reference): True keeps the forward pass's per-chunk intermediates alive
     until the backward pass (about 1.6 times the bytes of q, k, v, a, b, gk together), which then skips recomputing
-    them; False (and None without HDLA_HIP_KEEP_FORWARD=1 in the environment) is the reference's behaviour: only the
-    inputs are kept (hrdplr.py:137) and the backward pass recomputes (:161-198).  Results agree to rounding.
+    them; False is closest to the reference's behaviour, where only the inputs are kept (hrdplr.py:137) and the backward pass
+    recomputes (:161-198): here the fused route's record is kept beside them.  None (and HDLA_HIP_KEEP_FORWARD unset): kept
+    where that is at most 256 MiB and the route has no record.  HDLA_HIP_INPUTS_ONLY=1: strictly the inputs, unless True.
+    Results agree to rounding.
     """
     out = _lib.native().chunk(q, k, v, a, b, gk, RANK_AB, scale, initial_state, output_final_state, head_first, chunk_size,
                               cu_seqlens, keep_forward)

@@ -21,8 +21,8 @@ import torch
 import torch.nn.functional as F
 
 from . import _lib
-from .chunk import (_dims, _native_dim, _pad_last, _require_gpu, chunk_hrdplr_bwd, chunk_hrdplr_bwd_kept,
-                    chunk_hrdplr_fwd)
+from .chunk import (ONE_SEGMENT, _dims, _native_dim, _pad_last, _require_gpu, chunk_hrdplr_bwd, chunk_hrdplr_bwd_kept,
+                    chunk_hrdplr_fwd, keep_plan)
 from .utils import autocast_custom_bwd, autocast_custom_fwd, contiguous
 
 
@@ -40,9 +40,9 @@ def parameterize_a_b(beta: torch.Tensor, k: torch.Tensor, log_f: torch.Tensor) -
     return a, b
 
 
-def _fwd(q, k, v, beta, gk, scale, initial_state, output_final_state, cu_seqlens, want_boundary=False):
+def _fwd(q, k, v, beta, gk, scale, initial_state, output_final_state, cu_seqlens, want_boundary=False, keep=False, plan=(None, None)):
     return chunk_hrdplr_fwd(q, k, v, None, None, gk, scale, initial_state, output_final_state, cu_seqlens, beta=beta,
-                            want_boundary=want_boundary)
+                            want_boundary=want_boundary, keep=keep, plan=plan)
 
 
 def _bwd(q, k, v, beta, gk, scale, initial_state, do, dht, cu_seqlens, want_dh0, boundary=None, plan=(None, None)):
@@ -60,16 +60,19 @@ class ChunkHDLAFunction(torch.autograd.Function):
     def forward(ctx, q, k, v, beta, gk, scale, initial_state, output_final_state, cu_seqlens=None, keep_forward=False):
         h0 = None if initial_state is None else initial_state.to(torch.float32).contiguous()
         ctx.kept = None
-        boundary = None
+        boundary, ctx.plan, ctx.on_kept = None, (_lib.default_route(), _lib.default_segments()), False
         if keep_forward and any(ctx.needs_input_grad):     # see ChunkDPLRDeltaRuleFunction.forward
-            o, final_state, ctx.kept = chunk_hrdplr_fwd(q, k, v, None, None, gk, scale, h0, output_final_state, cu_seqlens,
-                                                        keep=True, beta=beta)
+            o, final_state, ctx.kept = _fwd(q, k, v, beta, gk, scale, h0, output_final_state, cu_seqlens, keep=True, plan=ONE_SEGMENT)
+            ctx.plan = ONE_SEGMENT
         elif any(ctx.needs_input_grad) and _lib.keep_boundaries_default():
-            o, final_state, boundary = _fwd(q, k, v, beta, gk, scale, h0, output_final_state, cu_seqlens, want_boundary=True)
+            plans = keep_plan(q, v, gk, scale, cu_seqlens) if keep_forward is None else None
+            if plans:
+                ctx.on_kept, ctx.plan = True, plans[1]
+            o, final_state, boundary = _fwd(q, k, v, beta, gk, scale, h0, output_final_state, cu_seqlens, want_boundary=True,
+                                            keep=ctx.on_kept, plan=plans[0] if plans else ctx.plan)
         else:
             o, final_state = _fwd(q, k, v, beta, gk, scale, h0, output_final_state, cu_seqlens)
         ctx.save_for_backward(q, k, v, beta, gk, initial_state, cu_seqlens, boundary)
-        ctx.plan = _lib.default_route(), _lib.default_segments()
         ctx.scale = scale
         return o.to(q.dtype), final_state
 
@@ -84,9 +87,10 @@ class ChunkHDLAFunction(torch.autograd.Function):
         if dht is not None:
             dht = dht.to(torch.float32).contiguous()
         h0 = None if initial_state is None else initial_state.to(torch.float32).contiguous()
-        if ctx.kept is not None:
-            dq, dk, dv, dbeta, dgk, dh0 = chunk_hrdplr_bwd_kept(q, k, v, None, None, gk, ctx.scale, h0, do, dht, ctx.kept,
-                                                                cu_seqlens, want_dh0=initial_state is not None, beta=beta)
+        if ctx.kept is not None or ctx.on_kept:
+            dq, dk, dv, dbeta, dgk, dh0 = chunk_hrdplr_bwd_kept(q, k, v, None, None, gk, ctx.scale, h0, do, dht,
+                                                                boundary if ctx.on_kept else ctx.kept, cu_seqlens,
+                                                                want_dh0=initial_state is not None, beta=beta, plan=ctx.plan)
         else:
             dq, dk, dv, dbeta, dgk, dh0 = _bwd(q, k, v, beta, gk, ctx.scale, h0, do, dht, cu_seqlens,
                                                want_dh0=initial_state is not None, boundary=boundary, plan=ctx.plan)

@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-#define HDLA_VERSION 205
+#define HDLA_VERSION 206
 
 enum { HDLA_BF16 = 0, HDLA_FP32 = 1 };
 
@@ -171,6 +171,10 @@ int hdla_chunk_bwd(const hdla_dims* dims, const void* q, const void* k, const vo
 size_t hdla_boundary_bytes(const hdla_dims* dims);
 size_t hdla_record_bytes(const hdla_dims* dims);
 size_t hdla_record_workspace_bytes(const hdla_dims* dims);
+/* What a training call on the classic kernels may hand from the forward to the backward pass instead of having it formed again: bytes of the
+ * buffer for hdla_chunk_fwd_keep and hdla_chunk_bwd_kept that the library suggests to keep, and the `segments` to give the one and the other in
+ * dims; 0 where it suggests none (the fused route has its record; a buffer of more than 256 MiB; no tokens). */
+size_t hdla_keep_plan(const hdla_dims* dims, int32_t* fwd_segments, int32_t* bwd_segments);
 int hdla_chunk_fwd_b(const hdla_dims* dims, const void* q, const void* k, const void* v, const void* a, const void* b,
                      const void* beta, const void* gk, const float* h0, void* o, float* ht, void* boundary,
                      size_t boundary_bytes, void* workspace, size_t workspace_bytes, void* stream);
@@ -203,7 +207,10 @@ int hdla_param_chunk_bwd(const hdla_dims* dims, const void* q, const void* k, co
  * keeps only the inputs between the passes and recomputes (ctx.save_for_backward at HRDPLR/hrdplr.py:137, recompute at
  * :161-198); these two trade that for about 1.6x the inputs' bytes of extra memory held between the passes.  `kept` is
  * only read by the backward call (it can be used again); `workspace` is scratch of
- * hdla_workspace_bytes(dims, HDLA_PASS_BWD_KEPT) bytes.  Same dims, inputs and stream ordering as the forward call. */
+ * hdla_workspace_bytes(dims, HDLA_PASS_BWD_KEPT) bytes.  Same dims, inputs and stream ordering as the forward call.
+ * Time segments: one where dims->segments is 0, otherwise (HDLA_ROUTE_AUTO) as many as it says; the states that enter them and their transitions
+ * are part of `kept`.  The backward call takes the forward call's number, whose records it then reads, or 1.  Rows of a packed batch that
+ * belong to no sequence are cleared in the gradients, as in hdla_chunk_bwd. */
 int hdla_chunk_fwd_keep(const hdla_dims* dims, const void* q, const void* k, const void* v, const void* a,
                         const void* b, const void* beta, const void* gk, const float* h0, void* o, float* ht,
                         void* kept, size_t kept_bytes, void* stream);

@@ -1,0 +1,176 @@
+"""What a training call keeps of its forward pass where nothing is said about it (hdla_keep_plan): where the library suggests it (on the CPU), and
+that a backward pass on it is the one that recomputes: whole sequences bit for bit, in time segments, whose reverse chain takes the forward
+pass's transitions turned, within the rounding of the element type."""
+import ctypes
+
+import pytest
+import torch
+
+import hdla_hip.chunk as CK
+from hdla_hip import _lib, chunk_hdla_delta_rule, chunk_hrdplr_delta_rule
+from hdla_hip.layer import HDLA_Custom
+from hdla_hip.synthetic import make_inputs
+from oracle import hrdplr_oracle as O
+
+DEV = "cuda"
+
+
+def _plan(T, lanes, K=128, V=128, dtype=torch.bfloat16, cu=None, **kw):
+    d = _lib.make_dims(1, T, lanes, K, V, 2, 1, dtype, dtype, 1.0, None, **kw)
+    if cu:
+        d.N, d.cu_seqlens = cu, 256                             # never read on the host
+    return _lib.keep_plan(d)
+
+
+def test_where_it_is_suggested():
+    n, fwd, bwd = _plan(1537, 16)
+    assert 0 < n <= 256 << 20 and (fwd, bwd) == (1, 1)
+    assert _plan(16384, 16)[0] == 0                             # more than 256 MiB
+    assert _plan(2048, 64, K=64, V=64)[0] == 0                  # the fused route has its record
+    assert _plan(256, 2, K=64, V=64)[1:] == (1, 1)              # few short sequences: the classic kernels
+    assert _plan(96, 2, K=64, V=64)[0] == 0                     # (their backward pass only)
+    assert _plan(0, 4)[0] == 0 and _plan(64, 4, K=96)[0] == 0
+    # as many segments as were asked for in both passes; none on the classic route
+    assert _plan(600, 4, segments=3)[1:] == (3, 3) and _plan(600, 4, route=_lib.ROUTE_CLASSIC)[1:] == (1, 1)
+    d = _lib.make_dims(1, 600, 4, 128, 128, 2, 1, torch.bfloat16, torch.bfloat16, 1.0, None, segments=3)
+    size = lambda p: _lib.load().hdla_workspace_bytes(ctypes.byref(d), p)
+    assert _lib.keep_plan(d)[0] == size(_lib.PASS_FWD_KEEP)
+    d.segments = 1
+    assert size(_lib.PASS_FWD_KEEP) < _plan(600, 4, segments=3)[0]
+
+
+# the fastest of 1 to 32 segments, forward and backward pass together, with the next one's time over it
+@pytest.mark.parametrize("K,V,lanes,chunks,dtype,want", [
+    (128, 128, 1, 313, torch.bfloat16, (16, 8)), (128, 128, 8, 128, torch.bfloat16, (8, 8)), (128, 128, 16, 16, torch.bfloat16, (1, 1)),
+    (64, 128, 2, 200, torch.bfloat16, (16, 16)), (64, 64, 16, 63, torch.float32, (8, 8)), (128, 128, 16, 8, torch.float32, (4, 4)),
+    (64, 64, 1, 8, torch.float32, (1, 1))])
+def test_segments(K, V, lanes, chunks, dtype, want):
+    fwd, bwd = _plan(16 * chunks, lanes, K, V, dtype)[1:]
+    assert bwd in (1, fwd)
+    assert fwd == want[0] and bwd == want[1] or (dtype == torch.bfloat16 and chunks == 313 and fwd in (8, 16) and bwd == fwd)
+
+
+CASES = [(2, 100, 2, 64, 64, None), (1, 70, 3, 128, 128, None), (1, 300, 2, 64, 128, (0, 37, 37, 200, 300)), (1, 330, 2, 128, 64, None),
+         (1, 260, 3, 128, 128, (0, 5, 101, 117, 260))]
+
+
+def _leaves(form, B, T, H, K, V, cu, dtype, gk_div=4.0):
+    inp = make_inputs(2100 + T, B, T, H, K, V, gk_div=gk_div, n_states=B if cu is None else len(cu) - 1)
+    k = torch.nn.functional.normalize(inp.k, dim=-1)
+    beta = 2.0 * torch.rand(B, T, H, 1, generator=torch.Generator().manual_seed(5))
+    x = [inp.q, k, inp.v] + ([inp.a, inp.b] if form == "ab" else [beta]) + [inp.gk]
+    return [t.to(dtype) for t in x] + [inp.h0], inp.do.to(dtype), inp.dht
+
+
+def _grads(form, leaves, do, dht, cu, keep):
+    op = (lambda *a, **kw: chunk_hrdplr_delta_rule(*a, 2, **kw)) if form == "ab" else chunk_hdla_delta_rule
+    o, ht = op(*leaves[:-1], scale=0.7, initial_state=leaves[-1], output_final_state=True, cu_seqlens=cu, keep_forward=keep)
+    return [o.detach(), ht.detach(), *torch.autograd.grad([o, ht], leaves, [do, dht])]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("form", ["ab", "beta"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,T,H,K,V,cu", CASES)
+@pytest.mark.parametrize("segments", [1, 2, 3, 5])
+def test_the_gradients_of_a_pass_that_recomputes(B, T, H, K, V, cu, dtype, form, native, segments, monkeypatch):
+    if K == V == 64 and dtype == torch.bfloat16:
+        if segments > 1:
+            pytest.skip("the fused route's")
+        T = 256                                                 # few short sequences
+    if not native:
+        monkeypatch.setattr(_lib, "_native", _lib._NoNative())
+    x, do, dht = _leaves(form, B, T, H, K, V, cu, dtype)
+    x, do, dht = [t.to(DEV).requires_grad_() for t in x], do.to(DEV), dht.to(DEV)
+    table = None if cu is None else torch.tensor(cu, device=DEV)
+    if segments > 1 or dtype == torch.float32 or K != 64 or V != 64:
+        monkeypatch.setenv("HDLA_HIP_SEGMENTS", str(segments))
+    before = torch.cuda.memory_allocated()
+    got, again = _grads(form, x, do, dht, table, None), _grads(form, x, do, dht, table, False)
+    for i, (a, b) in enumerate(zip(got, again)):
+        if i < 2 or segments == 1:
+            assert torch.equal(a, b), i
+        else:
+            # a transition formed on the way there and one formed on the way back, each of operands rounded to the element type
+            assert torch.isfinite(a.float()).all() and O.rel_l2(a, b) <= (2e-3 if dtype == torch.bfloat16 else 2e-7), (i, O.rel_l2(a, b))
+    if segments == 3 and native:                                # against the float64 recurrence
+        ref = [t.detach().cpu().double().requires_grad_() for t in x]
+        ab = list(O.parameterize_a_b(ref[3], ref[1], ref[4])) if form == "beta" else ref[3:5]
+        o, ht = O.recurrence(*ref[:3], *ab, ref[-2], 0.7, ref[-1], cu_seqlens=None if cu is None else torch.tensor(cu))
+        want = [o.detach(), ht.detach(), *torch.autograd.grad([o, ht], ref, [do.cpu().double(), dht.cpu().double()])]
+        errs = [O.rel_l2(a, b) for a, b in zip(got, want)]
+        assert max(errs) <= (1e-2 if dtype == torch.bfloat16 else 1e-5), errs
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("native", [True, False])
+def test_it_is_kept_and_given_back(native, monkeypatch):
+    if not native:
+        monkeypatch.setattr(_lib, "_native", _lib._NoNative())
+    x, do, dht = _leaves("ab", 1, 400, 4, 128, 128, None, torch.bfloat16)
+    x, do = [t.to(DEV).requires_grad_() for t in x], do.to(DEV)
+    run = lambda keep=None: chunk_hrdplr_delta_rule(*x[:-1], 2, scale=0.7, initial_state=x[-1], keep_forward=keep)[0]
+
+    def held(keep=None):
+        torch.cuda.synchronize()
+        at = torch.cuda.memory_allocated()
+        o = run(keep)
+        n = torch.cuda.memory_allocated() - at - o.numel() * 2
+        torch.autograd.grad(o, x, do, retain_graph=True)
+        assert torch.cuda.memory_allocated() - at - o.numel() * 2 == n
+        del o
+        assert torch.cuda.memory_allocated() == at
+        return n
+
+    want = _plan(400, 4)[0]
+    assert want <= held() <= want + (1 << 16)
+    assert held(False) < 1 << 16
+    for name, value in (("HDLA_HIP_INPUTS_ONLY", "1"), ("HDLA_HIP_KEEP_FORWARD", "0")):
+        with monkeypatch.context() as c:
+            c.setenv(name, value)
+            assert held() < 1 << 16
+    # the plan is the forward pass's, whatever the environment says by the backward pass
+    monkeypatch.setenv("HDLA_HIP_SEGMENTS", "4")
+    ref = torch.autograd.grad(run(), x, do)
+    for env in ({"HDLA_HIP_SEGMENTS": "2"}, {"HDLA_HIP_ROUTE": "classic"}, {"HDLA_HIP_INPUTS_ONLY": "1"}, {"HDLA_HIP_KEEP_FORWARD": "0"}):
+        o = run()
+        with monkeypatch.context() as c:
+            for name, value in env.items():
+                c.setenv(name, value)
+            assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(o, x, do), ref)), env
+
+
+@pytest.mark.gpu
+def test_rows_of_no_sequence():
+    """A packed batch padded at both ends: the kept pass clears the gradients' rows that no sequence has."""
+    cu = torch.tensor([3, 40, 150], device=DEV)
+    x, do, _ = _leaves("ab", 1, 170, 2, 128, 128, (0, 85, 170), torch.bfloat16)
+    x, do = [t.to(DEV).requires_grad_() for t in x], do.to(DEV)
+    dirty = [torch.full_like(t, float("nan")) for t in x[:6]]    # what the allocator hands out next
+    del dirty
+    o = chunk_hrdplr_delta_rule(*x[:-1], 2, scale=0.7, initial_state=x[-1], cu_seqlens=cu)[0]
+    for i, g in enumerate(torch.autograd.grad(o, x, do)[:6]):
+        r = g.shape[1] // 170
+        assert not g[:, :3 * r].any() and not g[:, 150 * r:].any() and torch.isfinite(g.float()).all(), i
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,H,T", [(256, 4, 256), (512, 4, 300)])
+def test_the_layer(d, H, T, monkeypatch):
+    torch.manual_seed(3)
+    m = HDLA_Custom(d, H, token_mixer_init_type=2, rescale_type=0).to(DEV).bfloat16().train()
+    x, do = torch.randn(1, T, d, device=DEV).bfloat16().requires_grad_(), torch.randn(1, T, d, device=DEV).bfloat16()
+    run = lambda: torch.autograd.grad(m(x)[0], [x, *m.parameters()], do)
+    got = run()
+    monkeypatch.setenv("HDLA_HIP_INPUTS_ONLY", "1")
+    assert all(torch.equal(a, b) for a, b in zip(got, run()))
+
+
+@pytest.mark.gpu
+def test_a_buffer_of_another_plan_is_refused():
+    x, do, dht = [t if isinstance(t, list) else t.to(DEV) for t in _leaves("ab", 1, 200, 2, 128, 128, None, torch.float32)]
+    q, k, v, a, b, gk, h0 = [t.to(DEV) for t in x]
+    _, _, kept = CK.chunk_hrdplr_fwd(q, k, v, a, b, gk, 0.7, h0, True, keep=True, plan=(_lib.ROUTE_AUTO, 1))
+    with pytest.raises(_lib.HdlaError, match="-5"):
+        CK.chunk_hrdplr_bwd_kept(q, k, v, a, b, gk, 0.7, h0, do, dht, kept, plan=(_lib.ROUTE_AUTO, 4))
