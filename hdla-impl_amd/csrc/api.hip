@@ -309,6 +309,7 @@ int make_layout(const hdla_dims* d, int pass, WsLayout& L, int& nch) {
     if (nseg > 1) {
         const size_t recs = (size_t)d->N * d->H * nseg, state = recs * K * V * 4, matrix = recs * K * K * 4;
         if (prep_out) { L.SEG_LOC = take(state); L.SEG_TR = take(matrix); L.SEG_IN = take(state); }
+        if (pass == HDLA_PASS_FWD_KEEP) L.SEG_RTR = take(matrix);
         if (pass == HDLA_PASS_BWD) { L.SEG_RLOC = take(state); L.SEG_RTR = take(matrix); L.SEG_RIN = take(state); }
         if (pass == HDLA_PASS_BWD_KEPT) { L.SEG_RLOC = take(state); L.SEG_RIN = take(state); }
     }
@@ -389,13 +390,13 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
     a.da = static_cast<T*>(da); a.db = static_cast<T*>(db); a.dgk = dgk;
     a.beta = static_cast<const T*>(beta); a.dbeta = static_cast<T*>(dbeta);
     bind_ws(a, d, LP, prep_ws, LS, pass == HDLA_PASS_BWD_KEPT ? workspace : prep_ws, nch);
-    a.seg = SegRec{1, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+    a.seg = SegRec{1, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
     const int nseg = on_kept ? kept_segments(d) : scan_segments(d, !fwd);
     if (nseg > 1) {
         const auto at = [](void* base, size_t o) { return reinterpret_cast<float*>(static_cast<char*>(base) + o); };
-        a.seg = SegRec{nseg, at(prep_ws, LP.SEG_LOC), at(prep_ws, LP.SEG_TR), at(prep_ws, LP.SEG_IN), nullptr, nullptr, nullptr};
-        if (!fwd) { a.seg.rloc = at(workspace, LS.SEG_RLOC); a.seg.rin = at(workspace, LS.SEG_RIN); }
-        if (pass == HDLA_PASS_BWD) a.seg.rtr = at(workspace, LS.SEG_RTR);
+        a.seg = SegRec{nseg, at(prep_ws, LP.SEG_LOC), at(prep_ws, LP.SEG_TR), at(prep_ws, LP.SEG_IN), nullptr, nullptr, nullptr, nullptr};
+        if (!fwd) { a.seg.rloc = at(workspace, LS.SEG_RLOC); a.seg.rtr = at(prep_ws, LP.SEG_RTR); a.seg.rin = at(workspace, LS.SEG_RIN); }
+        if (pass == HDLA_PASS_FWD_KEEP) a.seg.turned = at(prep_ws, LP.SEG_RTR);
     }
     hipError_t e;
     if (pass == HDLA_PASS_BWD_KEPT) {

@@ -121,9 +121,10 @@ constexpr int SCAN_TARGET_WORKGROUPS = 256;               // compute units of th
 // nseg times as many of them at once (scan_segments in api.hip says when).
 //
 // At the end of a segment: column block j of the state, or (trans) of the transition matrix X, whose tile (kt, j) is kept
-// with rows k, inner k', which is how the chain takes it.
+// with rows k, inner k', which is how the chain takes it.  turned: where the backward pass will find its own, or null: what the state's gradient
+// meets on its way back through a segment is the transpose of what the state met on its way there.
 template <typename T, int K>
-__device__ __forceinline__ void store_record(const f32x4 (&S)[K / 16], float* loc, float* tr, int64_t rec, int V, int j, bool trans) {
+__device__ __forceinline__ void store_record(const f32x4 (&S)[K / 16], float* loc, float* tr, float* turned, int64_t rec, int V, int j, bool trans) {
     constexpr int KT = K / 16;
     if (trans) {
         const Frag<float> ident = ident_frag<float>();
@@ -133,6 +134,10 @@ __device__ __forceinline__ void store_record(const f32x4 (&S)[K / 16], float* lo
             f.v = S[kt];
             f = transpose(f, ident);                      // exact: fp32 products with ones and zeros
             *reinterpret_cast<f32x4*>(tr + rec * (K * K) + (kt * KT + j) * TILE + 4 * lane_id()) = f.v;
+        }
+        if (turned) {
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt) *reinterpret_cast<f32x4*>(turned + rec * (K * K) + (j * KT + kt) * TILE + 4 * lane_id()) = S[kt];
         }
     } else {
 #pragma unroll
@@ -373,7 +378,7 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
         }
     }
     if (SUM) {
-        store_record<T, K>(S, p.seg.loc, p.seg.tr, rec, V, vt, trans);
+        store_record<T, K>(S, p.seg.loc, p.seg.tr, p.seg.turned, rec, V, vt, trans);
     } else if (p.ht && seg == p.seg.nseg - 1) {
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
@@ -575,7 +580,7 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
         }
     }
     if (SUM) {
-        store_record<T, K>(dS, p.seg.rloc, p.seg.rtr, rec, V, vt, trans);
+        store_record<T, K>(dS, p.seg.rloc, p.seg.rtr, nullptr, rec, V, vt, trans);
     } else if (p.dh0 && seg == 0) {
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
@@ -636,9 +641,7 @@ __global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_sum_ker
     }
 }
 // The records chained into what enters the segments, X <- M_s X + X_loc(s) from the segment that starts the sequence (or, in
-// reverse, ends it): grid = (H, directions * V/16, N), one wave per 16 rows of the state's column block; blockIdx.y counts from first_y on.
-// Without transitions of its own (rtr) the reverse chain takes the forward ones turned: what the state's gradient meets on its way
-// back through a segment is the transpose of what the state met on its way there.  A chain of
+// reverse, ends it): grid = (H, directions * V/16, N), one wave per 16 rows of the state's column block; blockIdx.y counts from first_y on.  A chain of
 // dependent steps, so a step is kept short: the wave's rows of the next transition matrix are requested a step ahead, the
 // waves exchange their rows through LDS (split operands: the error of fp32 products), one barrier a step.
 // With 4-byte elements the sums are 64-bit (v_mfma_f64_16x16x4_f64): in fp32 a chain step rounds a state K / 4 times more than the
@@ -655,10 +658,10 @@ __global__ __launch_bounds__(64 * (K / 16)) void scan_chain_kernel(ChunkArgs<T> 
     typedef typename ChainState<T>::shared Shared;
     __shared__ __attribute__((aligned(16))) Shared sx[2][KT][64];
     const int y = blockIdx.y + first_y, h = blockIdx.x, vt = y % VT, n = blockIdx.z, nseg = p.seg.nseg;
-    const bool rev = y >= VT, turned = rev && !p.seg.rtr;
+    const bool rev = y >= VT;
     const int kt = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane_id();
     const float* const loc = rev ? p.seg.rloc : p.seg.loc;
-    const float* const tr = rev && !turned ? p.seg.rtr : p.seg.tr;
+    const float* const tr = rev ? p.seg.rtr : p.seg.tr;
     float* const in = rev ? p.seg.rin : p.seg.in;
     const int64_t rec0 = ((int64_t)n * p.H + h) * nseg;
     // step i handles the i-th segment from the start of the chain
@@ -667,18 +670,9 @@ __global__ __launch_bounds__(64 * (K / 16)) void scan_chain_kernel(ChunkArgs<T> 
     // Register i of lane (g, c) of a 64-bit result is row g + 4 i of the product: the rows of the transition matrix are handed over
     // in the order in which that is row 4 g + i, as everywhere else.
     const int row = WIDE ? (l & 48) + 4 * (l & 3) + ((l >> 2) & 3) : l;
-    // (lane (g, c) of a turned tile: column c of rows 4 g .. 4 g + 3, element c % 4 of the lanes (c / 4, 4 g + i))
-    const int col = (16 * ((row & 15) >> 2) + 4 * (row >> 4)) * 4 + (row & 3);
     auto request = [&](int i, f32x4 (&m)[KT], f32x4& a) __attribute__((always_inline)) {
         i = min(i, nseg - 2);                             // past the end: never used
         a = *reinterpret_cast<const f32x4*>(loc + rec(i) * (K * V) + own);
-        if (turned) {
-#pragma unroll
-            for (int ki = 0; ki < KT; ++ki)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) m[ki][e] = tr[rec(i) * (K * K) + (ki * KT + kt) * TILE + col + 4 * e];
-            return;
-        }
 #pragma unroll
         for (int ki = 0; ki < KT; ++ki) m[ki] = *reinterpret_cast<const f32x4*>(tr + rec(i) * (K * K) + (kt * KT + ki) * TILE + 4 * row);
     };

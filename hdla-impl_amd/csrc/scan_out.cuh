@@ -376,6 +376,7 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
                 f.v = S[k];
                 f = transpose(f, identf);                 // exact: fp32 products with ones and zeros
                 *reinterpret_cast<f32x4*>(p.seg.tr + rec * (K * K) + (kt * KT + vt) * TILE + 4 * l) = f.v;
+                if (p.seg.turned) *reinterpret_cast<f32x4*>(p.seg.turned + rec * (K * K) + (vt * KT + kt) * TILE + 4 * l) = S[k];
             } else {
                 *reinterpret_cast<f32x4*>(p.seg.loc + rec * (K * V) + (vt * KT + kt) * TILE + 4 * l) = S[k];
             }
