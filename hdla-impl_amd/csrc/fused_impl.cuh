@@ -396,7 +396,7 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
             Frag<T> rq, rk, ra[2], rb[2];
             operands(j, g4, rq, rk, ra, rb);
             if (HD) __builtin_amdgcn_sched_barrier(0);
-            const TileDecay e(g4, c);
+            const TileDecay<T> e(g4, c);
             strong |= e.strong;
             egi[j] = e.egi;
             edn[j] = e.edn;

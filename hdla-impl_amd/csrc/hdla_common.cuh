@@ -74,6 +74,8 @@ __device__ __forceinline__ f32x4 to_f32(Frag<float> a) { return a.v; }
 // out of the loop and kept in registers across it.
 __device__ __forceinline__ void pin(Frag<bf16>& x) { asm volatile("" : "+v"(x.v)); }
 __device__ __forceinline__ void pin(f32x4& x) { asm volatile("" : "+v"(x)); }
+__device__ __forceinline__ void hold(Frag<bf16>& x) { pin(x); }
+__device__ __forceinline__ void hold(Frag<float>& x) { pin(x.v); }
 __device__ __forceinline__ void pin(Frag<float>&) {}     // fp32 operands are used as they are: nothing to hoist
 
 // The value of x is not needed any more; x is left with whatever its registers hold (no instruction).  For what is refilled under a
@@ -482,17 +484,6 @@ __device__ __forceinline__ float sum_groups(float x) {
 constexpr float SAFE_RANGE = 70.f;
 constexpr float PASS_CLAMP = 20.f;
 
-template <int N> __device__ __forceinline__ bool strong_decay(const f32x4 (&gi)[N], const f32x4 (&ge)[N]) {
-    float big = 0.f;
-#pragma unroll
-    for (int kt = 0; kt < N; ++kt) {
-        const f32x4 m = bcast16<MID>(gi[kt]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) big = fmaxf(big, fmaxf(fabsf(gi[kt][i] - m[i]), fabsf(ge[kt][i] - m[i])));
-    }
-    return __any(big > SAFE_RANGE) != 0;                 // the same answer on every lane of the wave
-}
-
 // ---- the same factors in base 2 (2-byte element types) --------------------------------------------------------------
 // A channel tile needs e^{gi-m}, e^{m-gi}, e^{ge-m} for its scores and e^{gi}, e^{ge}, e^{gl-gi}, e^{gl} for the gated copies.
 // An exponential is 16 cycles of a SIMD (a quarter-rate instruction) and a multiplication before it; but ge of a token is
@@ -521,7 +512,8 @@ __device__ __forceinline__ f32x4 prev_token(f32x4 x, f32x4 first) {
         r[i] = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(first[i]), __float_as_int(x[i]), 0x111, 0xf, 0xf, false));   // row_shr:1
     return r;
 }
-struct TileDecay {
+template <typename T> struct TileDecay;
+template <> struct TileDecay<bf16> {
     f32x4 eq, ek, ea;                                     // e^{gi-m}, e^{m-gi}, e^{ge-m}
     f32x4 egi, ege, edn, egl;                             // e^{gi}, e^{ge}, e^{gl-gi}, e^{gl}
     bool strong;                                          // a factor beyond the safe range (the same on every lane)
@@ -549,6 +541,26 @@ struct TileDecay {
         const f32x4 one = {1.f, 1.f, 1.f, 1.f};
         ege = prev_token(egi, one);
         egl = bcast16<CH - 1>(egi);
+    }
+};
+// 4-byte element types: every factor an exponential of its own.  With a token's exclusive ones taken from the token before it, the outputs of
+// 2000 tokens of 8 heads were 0.1 % further from a float64 evaluation (standard error 0.01 %); with products more so.
+template <> struct TileDecay<float> {
+    f32x4 eq, ek, ea, egi, ege, edn, egl;
+    bool strong;
+    __device__ __forceinline__ TileDecay(f32x4 g4, int) {
+        const f32x4 gi = scan16_incl(g4), ge = gi - g4, m = bcast16<MID>(gi), gl = bcast16<CH - 1>(gi);
+        eq = exp4<float>(gi - m);
+        ek = exp4<float>(m - gi);
+        ea = exp4<float>(ge - m);
+        egi = exp4<float>(gi);
+        ege = exp4<float>(ge);
+        edn = exp4<float>(gl - gi);
+        egl = bcast16<CH - 1>(egi);
+        float big = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) big = fmaxf(big, fmaxf(fabsf(gi[i] - m[i]), fabsf(ge[i] - m[i])));
+        strong = __any(!(big <= SAFE_RANGE)) != 0;
     }
 };
 

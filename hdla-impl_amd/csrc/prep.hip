@@ -21,8 +21,15 @@ constexpr int LDP = 36;   // padded row length of the 32x32 LDS matrices (keeps 
 // output); PREP_BWD: what the two scans of the backward pass and the chunk_grad kernels read; PREP_KEEP: both, for a
 // forward pass whose workspace the backward pass will use instead of running this kernel again.
 enum PrepMode { PREP_FWD = 0, PREP_BWD = 1, PREP_KEEP = 2 };
+// Waves a SIMD: what the registers of a wave allow.  Three of 2-byte elements (with fp32 decays beside plain a, b: two): a tile's factors, operands
+// and gated copies are done with before the next one's begin, the copies that need nothing else leave at once, and (I - A_ab)^-1 lies where the
+// parts of the score tiles were (20 KB of LDS a workgroup of two waves instead of 37).  Three exponentials a tile instead of seven (TileDecay).
+// Measured, us, before (all copies formed behind (I - A_ab)^-1 from inputs and decays kept for that, 216 registers) -> after: K = V = 128, 16384
+// tokens of 16 heads, forward / backward mode 190 / 237 -> 176 / 222, which is 5.7 TB/s of their traffic; with the HDLA parameterisation 5003 tokens
+// of 16 heads 62 -> 52, 3074 tokens of 8 heads, both modes in one, 26 -> 23.  4-byte elements, 1008 chunks and heads (a wave a SIMD): the same.
+template <typename T, bool GKF32, bool HD> constexpr int prep_waves() { return sizeof(T) == 2 && (HD || !GKF32) ? 3 : 2; }
 template <typename T, bool GKF32, int K, int V, int MODE, bool HD>
-__global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void prep_kernel(ChunkArgs<T> p) {
+__global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T, GKF32, HD>(), prep_waves<T, GKF32, HD>()))) void prep_kernel(ChunkArgs<T> p) {
     constexpr bool BWD = MODE == PREP_BWD;                // neither the output's score tiles nor qg are needed
     constexpr bool WB = MODE != PREP_FWD;                 // the backward pass's extras are
     // the forward pass's scan of 2-byte elements forms u itself and takes the ranks of b^T side by side (scan_out.cuh): v is not read
@@ -31,14 +38,19 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void 
     constexpr int KTW = 4, VT = V / 16, VTW = VT / NWP, KT2 = K / 32;
     constexpr int SAS = blk_fwd(K, sizeof(T), !BWD).SIZE / (int)sizeof(T);   // elements between (chunk, head) slots
     constexpr int SBS = blk_bwd(K, sizeof(T)).SIZE / (int)sizeof(T);
-    __shared__ __attribute__((aligned(16))) float sNw[NWP][32 * LDP];   // A_ab, rank-major (one copy per wave)
-    __shared__ __attribute__((aligned(16))) float sTw[NWP][32 * LDP];   // (I - A_ab)^-1
     constexpr int NPART = BWD ? 8 : 9;                                    // score tiles that are summed over the waves
-    __shared__ __attribute__((aligned(16))) float sPart[NWP > 1 ? NWP * NPART * 256 : 4];
+    // Per wave: A_ab, rank-major, and (I - A_ab)^-1.  A wave's matrices lie where the other wave's parts of the score tiles were, which it
+    // has then read and nobody else does.
+    constexpr int MAT = 32 * LDP;
+    static_assert(NPART * 256 <= 2 * MAT, "");
+    __shared__ __attribute__((aligned(16))) float sMat[NWP][2 * MAT];
+    __shared__ __attribute__((aligned(16))) char sRows[NWP][ROWS_SCRATCH];   // rows on their way to fragments
+    __shared__ float sSum[NWP * CH];
     __shared__ int sStrong[NWP];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    float* const sN = sNw[w];
-    float* const sT = sTw[w];
+    float* const sN = sMat[w];
+    float* const sT = sN + MAT;
+    char* const scratch = sRows[w];
     const int kt0 = w * KTW, vt0 = w * VTW;                              // first own channel tile / value tile
 
     // Which of the two indices runs fastest over the workgroups decides which rows of the [token][head][channel]
@@ -58,148 +70,178 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void 
     const int64_t chw = (int64_t)h * p.st.nch + cid;                // chunk-head slot in the workspace
     const float scale = p.scale;
 
-    // ---- phase A: cumulative decays and the score tiles (rows i, inner j) -----------------------------------
-    f32x4 gi[KTW], ge[KTW];
+    // ---- phase A: decays, the score tiles (rows i, inner j) and the gated copies --------------------------------
     f32x4 aqk = zero4(), aqb[2] = {zero4(), zero4()}, aak[2] = {zero4(), zero4()};
     f32x4 aab[2][2] = {{zero4(), zero4()}, {zero4(), zero4()}};
-    // the inputs of the chunk stay in registers (as loaded) for the second use in phase C: the working set of the
-    // resident waves is larger than the L2, so a second load would come from HBM again
-    Frag<T> rq[KTW], rk[KTW], ra[2][KTW], rb[2][KTW];       // own channel tiles; index kt below is local, kt0 + kt global
-    // us, a fragment's lanes loading for themselves -> TileLoad: K=V=128 bf16, 16384 tokens of 16 heads, forward / backward mode
-    // 248 / 253 -> 236 / 239; with the HDLA parameterisation, where a wave also read the other one's channels of k and gk for s,
-    // 5003 tokens of 16 heads 85 -> 72.  What is left is the traffic: 70 KB a chunk and head, 239 us at a large copy's rate.
+    const Frag<T> ident = ident_frag<T>();
+    Frag<T> ag[2][KTW];                                    // of the own channel tiles; index kt below is local, kt0 + kt global
     typedef std::conditional_t<GKF32, float, bf16> G;
     typedef TileLoad<T, 2> Load;
     typedef TileLoad<G, 2> LoadG;
-    char* const scratch = reinterpret_cast<char*>(sT);               // free until phase B
-    static_assert(ROWS_SCRATCH <= sizeof(sTw[0]), "");
     const T* const qrow = p.q + (cp.tok0 * H + h) * K + 16 * kt0;
     const T* const krow = p.k + (cp.tok0 * H + h) * K + 16 * kt0;
     const G* const grow = reinterpret_cast<const G*>(p.gk) + (cp.tok0 * H + h) * K + 16 * kt0;
     const T* const arow = HD ? nullptr : p.a + (cp.tok0 * RANK * H + h) * K + 16 * kt0;
     const T* const brow = HD ? nullptr : p.b + (cp.tok0 * RANK * H + h) * K + 16 * kt0;
     const T* const vrow = p.v + (cp.tok0 * H + h) * V + 16 * vt0;
-    // v is used last (phase D) but requested first: the barriers in between would otherwise keep its loads, and a
-    // full round trip to HBM, behind everything else
-    Frag<T> rv[VTW];
-    Load lv[VTW / 2];
-    if (!SCAN_U)
+    // two channel tiles of a token: log-decay, q, k, a, b, requested and as fragments
+    struct Request { Load q, k, a[2], b[2]; LoadG g; };
+    struct Inputs { f32x4 g; Frag<T> q, k, a[2], b[2]; };
+    auto request = [&](int kp, Request& x) __attribute__((always_inline)) {
+        x.g.load(grow + 32 * kp, H * K, cp.len, l);
+        x.k.load(krow + 32 * kp, H * K, cp.len, l);
+        x.q.load(qrow + 32 * kp, H * K, cp.len, l);
+        if (!HD) {
 #pragma unroll
-    for (int vp = 0; vp < VTW / 2; ++vp) lv[vp].load(vrow + 32 * vp, H * V, cp.len, l);
+            for (int r = 0; r < 2; ++r) {
+                x.a[r].load(arow + r * H * K + 32 * kp, RANK * H * K, cp.len, l);
+                x.b[r].load(brow + r * H * K + 32 * kp, RANK * H * K, cp.len, l);
+            }
+        }
+    };
+    // (both pairs at once: each takes half of the rows' cache lines, and with the second one requested when the first had been used, and three
+    // waves a SIMD, the lines had left the L2: 190 -> 208 us for 16384 tokens of 16 heads, K = V = 128; this way 176)
+    Request req[KTW / 2];
+#pragma unroll
+    for (int kp = 0; kp < KTW / 2; ++kp) request(kp, req[kp]);
+    __builtin_amdgcn_sched_barrier(0);
     // HDLA parameterisation: a_1 = -beta k, a_2 = beta k (beta s - f), b_1 = f k, b_2 = k with f = exp(gk) and
     // s = sum over ALL channels of k^2 f (two waves exchange their channels' parts)
     float beta_t = 0.f, s_t = 0.f;
     if (HD) beta_t = rowok ? ld_elem(p.beta + tok * H + h) : 0.f;
     f32x4 gks[HD ? KTW : 1];
+    Frag<T> ks[HD ? KTW : 1];
     if (HD) {
 #pragma unroll
         for (int kp = 0; kp < KTW / 2; ++kp) {
-            LoadG lg;
-            Load lk;
-            lg.load(grow + 32 * kp, H * K, cp.len, l);
-            lk.load(krow + 32 * kp, H * K, cp.len, l);
             Frag<G> fg[2];
             Frag<T> f[2];
-            lg.tiles(scratch, cp.len, l, fg);
-            lk.tiles(scratch, cp.len, l, f);
+            req[kp].g.tiles(scratch, cp.len, l, fg);
+            req[kp].k.tiles(scratch, cp.len, l, f);
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
                 const int kt = 2 * kp + e;
                 gks[kt] = to_f32(fg[e]);
-                rk[kt] = f[e];
+                ks[kt] = f[e];
                 const f32x4 k4 = to_f32(f[e]), kf = k4 * k4 * exp4<T>(gks[kt]);
                 s_t += kf[0] + kf[1] + kf[2] + kf[3];
             }
         }
-        s_t += __shfl_xor(s_t, 16);
-        s_t += __shfl_xor(s_t, 32);
-        if (NWP > 1) {                                    // sPart is free until the score tiles are summed
-            if (g == 0) sPart[w * CH + c] = s_t;
+        s_t = sum_groups(s_t);
+        if (NWP > 1) {
+            if (g == 0) sSum[w * CH + c] = s_t;
             __syncthreads();
             s_t = 0.f;
 #pragma unroll
-            for (int ww = 0; ww < NWP; ++ww) s_t += sPart[ww * CH + c];
-            __syncthreads();
+            for (int ww = 0; ww < NWP; ++ww) s_t += sSum[ww * CH + c];
         }
     }
-#pragma unroll
-    for (int kp = 0; kp < KTW / 2; ++kp) {
-        Load lq, lk, la[2], lb[2];
-        LoadG lg;
-        Frag<T> fq[2], fk[2], fa[2][2], fb[2][2];
+    // held: with the HDLA parameterisation k and the decays are there already, from the sum
+    auto inputs = [&](int kp, const Request& x, Inputs (&in)[2], bool held) __attribute__((always_inline)) {
+        Frag<T> f[2];
         Frag<G> fg[2];
-        lq.load(qrow + 32 * kp, H * K, cp.len, l);
+        if (!HD || !held) {
+            x.g.tiles(scratch, cp.len, l, fg);
+            x.k.tiles(scratch, cp.len, l, f);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) { in[e].g = to_f32(fg[e]); in[e].k = f[e]; }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 2; ++e) { in[e].g = gks[HD ? 2 * kp + e : 0]; in[e].k = ks[HD ? 2 * kp + e : 0]; }
+        }
+        x.q.tiles(scratch, cp.len, l, f);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) in[e].q = f[e];
         if (!HD) {
-            lg.load(grow + 32 * kp, H * K, cp.len, l);
-            lk.load(krow + 32 * kp, H * K, cp.len, l);
 #pragma unroll
             for (int r = 0; r < 2; ++r) {
-                la[r].load(arow + r * H * K + 32 * kp, RANK * H * K, cp.len, l);
-                lb[r].load(brow + r * H * K + 32 * kp, RANK * H * K, cp.len, l);
-            }
-            lg.tiles(scratch, cp.len, l, fg);
-            lk.tiles(scratch, cp.len, l, fk);
-        }
-        lq.tiles(scratch, cp.len, l, fq);
-        if (!HD) {
+                x.a[r].tiles(scratch, cp.len, l, f);
 #pragma unroll
-            for (int r = 0; r < 2; ++r) { la[r].tiles(scratch, cp.len, l, fa[r]); lb[r].tiles(scratch, cp.len, l, fb[r]); }
+                for (int e = 0; e < 2; ++e) in[e].a[r] = f[e];
+                x.b[r].tiles(scratch, cp.len, l, f);
+#pragma unroll
+                for (int e = 0; e < 2; ++e) in[e].b[r] = f[e];
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const f32x4 kk = to_f32(in[e].k), f4 = exp4<T>(in[e].g);
+                in[e].a[0] = to_frag<T>(kk * (-beta_t));
+                in[e].a[1] = to_frag<T>(kk * ((beta_t * s_t - f4) * beta_t));
+                in[e].b[0] = to_frag<T>(f4 * kk);
+                in[e].b[1] = in[e].k;
+            }
         }
+    };
+    // 2-byte elements: one tile's factors and operands at a time, for the registers
+    constexpr bool TIGHT = sizeof(T) == 2;
+    bool strong = false;
+#pragma unroll
+    for (int kp = 0; kp < KTW / 2; ++kp) {
+        Inputs in[2];
+        inputs(kp, req[kp], in, true);
+        Frag<T> kgT[2], bgT[2][2], qg[2];                  // [..][tile of the stored pair]
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             const int kt = 2 * kp + e;
-            const f32x4 g4 = HD ? gks[HD ? kt : 0] : to_f32(fg[e]);
-            rq[kt] = fq[e];
-            if (HD) {
-                const f32x4 kk = to_f32(rk[kt]), f4 = exp4<T>(g4);
-                ra[0][kt] = to_frag<T>(kk * (-beta_t));
-                ra[1][kt] = to_frag<T>(kk * ((beta_t * s_t - f4) * beta_t));
-                rb[0][kt] = to_frag<T>(f4 * kk);
-                rb[1][kt] = rk[kt];
-            } else {
-                rk[kt] = fk[e];
-#pragma unroll
-                for (int r = 0; r < 2; ++r) { ra[r][kt] = fa[r][e]; rb[r][kt] = fb[r][e]; }
-            }
-            gi[kt] = scan16_incl(g4);
-            ge[kt] = gi[kt] - g4;
             // Every score is a dense product of operands decayed relative to the middle of the chunk: exp(gi_i - gi_j) =
             // exp(gi_i - m) exp(m - gi_j) with m = gi of token MID.  That is done here for every chunk, tile by tile as the
             // inputs arrive; it is only valid while the exponents stay within +-SAFE_RANGE, which is checked afterwards.
-            const f32x4 m = bcast16<MID>(gi[kt]);
-            const f32x4 eq = exp4<T>(gi[kt] - m), ek = exp4<T>(m - gi[kt]), ea = exp4<T>(ge[kt] - m);
-            const f32x4 q4 = to_f32(rq[kt]), k4 = to_f32(rk[kt]);
-            const f32x4 a0 = to_f32(ra[0][kt]), a1 = to_f32(ra[1][kt]), b0 = to_f32(rb[0][kt]), b1 = to_f32(rb[1][kt]);
-            Split<T> qh, kh, ah[2], bh[2];
-            split(q4 * eq * scale, qh);
-            split(k4 * ek, kh);
-            split(a0 * ea, ah[0]);
-            split(a1 * ea, ah[1]);
-            split(b0 * ek, bh[0]);
-            split(b1 * ek, bh[1]);
-            aqk = mm_split(qh, kh, aqk);
+            const TileDecay<T> d(in[e].g, c);
+            strong |= d.strong;
+            qg[e] = to_frag<T>(to_f32(in[e].q) * d.egi * scale);
+            kgT[e] = transpose(to_frag<T>(to_f32(in[e].k) * d.edn), ident);
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                aqb[s] = mm_split(qh, bh[s], aqb[s]);
-                aak[s] = mm_split(ah[s], kh, aak[s]);
-#pragma unroll
-                for (int r = 0; r < 2; ++r) aab[r][s] = mm_split(ah[r], bh[s], aab[r][s]);
+            for (int r = 0; r < 2; ++r) {
+                ag[r][kt] = to_frag<T>(to_f32(in[e].a[r]) * d.ege);
+                if (TIGHT) hold(ag[r][kt]);                          // formed here, not where it is used: that would keep a and its factors instead
+                bgT[r][e] = transpose(to_frag<T>(to_f32(in[e].b[r]) * d.edn), ident);
             }
-        }
-    }
-    if (!SCAN_U)
+            // (the same from all tokens' lanes: without a branch in the way of the scheduler)
+            *reinterpret_cast<f32x4*>(p.ws.EGL + chw * (SAS * (int)sizeof(T) / 4) + 16 * (kt0 + kt) + 4 * g) = d.egl;
+            if (TIGHT) __builtin_amdgcn_sched_barrier(0);
+            // (pin(): converted to fp32 again rather than held so from above)
+            if (!HD) {
+                pin(in[e].q); pin(in[e].k);
 #pragma unroll
-    for (int vp = 0; vp < VTW / 2; ++vp) {
-        Frag<T> f[2];
-        lv[vp].tiles(scratch, cp.len, l, f);
-        rv[2 * vp] = f[0];
-        rv[2 * vp + 1] = f[1];
+                for (int r = 0; r < 2; ++r) { pin(in[e].a[r]); pin(in[e].b[r]); }
+            }
+            Split<T> kh, bh[2];
+            split(to_f32(in[e].k) * d.ek, kh);
+            split(to_f32(in[e].b[0]) * d.ek, bh[0]);
+            split(to_f32(in[e].b[1]) * d.ek, bh[1]);
+            {
+                Split<T> qh;
+                split(to_f32(in[e].q) * d.eq * scale, qh);
+                aqk = mm_split(qh, kh, aqk);
+#pragma unroll
+                for (int s = 0; s < 2; ++s) aqb[s] = mm_split(qh, bh[s], aqb[s]);
+            }
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                if (TIGHT) __builtin_amdgcn_sched_barrier(0);
+                Split<T> ah;
+                split(to_f32(in[e].a[r]) * d.ea, ah);
+                aak[r] = mm_split(ah, kh, aak[r]);
+#pragma unroll
+                for (int s = 0; s < 2; ++s) aab[r][s] = mm_split(ah, bh[s], aab[r][s]);
+            }
+            if (TIGHT) __builtin_amdgcn_sched_barrier(0);
+        }
+        const int pair = kt0 / 2 + kp;
+        st_pair2(p.ws.KGT + chw * SAS + pair * PAIR, kgT[0], kgT[1]);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            if (SCAN_U) st_pair2(p.ws.BGT + chw * SAS + (2 * pair + s) * PAIR, bgT[0][s], bgT[1][s]);   // (s: the tile of the pair)
+            else st_pair2(p.ws.BGT + chw * SAS + (s * KT2 + pair) * PAIR, bgT[s][0], bgT[s][1]);
+        }
+        if (!BWD) st_pair2(p.ws.QG + chw * SAS + pair * PAIR, qg[0], qg[1]);
+        if (WB) st_pair2(p.ws.QGT + chw * SBS + pair * PAIR, transpose(qg[0], ident), transpose(qg[1], ident));
     }
     // Each wave decides for its own channels (the parts of the score tiles add up whichever way they were formed); the
     // backward pass records the decision per (chunk, head) for the chunk_grad kernels.  Where a channel decays too
     // strongly for the single centre, what was accumulated above may hold infinities: it is thrown away and the tiles
-    // are formed again by passes whose exponents cannot overflow (see DecayPass).
-    const bool strong = strong_decay(gi, ge);
+    // are formed again, from inputs read again, by passes whose exponents cannot overflow (see DecayPass).
     if (WB && l == 0) {
         if (NWP == 1) p.ws.STRONG[chw] = strong;
         else sStrong[w] = strong;
@@ -210,53 +252,61 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void 
         for (int s = 0; s < 2; ++s) {
             aqb[s] = zero4(); aak[s] = zero4(); aab[0][s] = zero4(); aab[1][s] = zero4();
         }
+        // this path is rare and must not cost the common one registers: one tile and one operand at a time
 #pragma unroll 1
         for (int ps = 0; ps < DecayPass::COUNT; ++ps) {
             const DecayPass dp(ps, c);
+#pragma unroll 1
+            for (int kp = 0; kp < KTW / 2; ++kp) {
+                Request x;
+                Inputs in[2];
+                request(kp, x);
+                inputs(kp, x, in, false);
 #pragma unroll
-            for (int kt = 0; kt < KTW; ++kt) {
-                f32x4 eq, ek, ea;
-                dp.factors<T>(gi[kt], ge[kt], eq, ek, ea);
-                // the same products as above, one operand at a time with the scheduler kept from interleaving them: this
-                // path is rare and must not cost the common one registers
-                // (pin(): the conversions of the inputs do not depend on the pass, and hoisted out of the pass loop they
-                // would all be live across it)
-                pin(rk[kt]); pin(rq[kt]); pin(ra[0][kt]); pin(ra[1][kt]); pin(rb[0][kt]); pin(rb[1][kt]);
-                Split<T> qh, kh, bh[2];
-                split(to_f32(rk[kt]) * ek, kh);
-                split(to_f32(rq[kt]) * eq * scale, qh);
-                aqk = mm_split(qh, kh, aqk);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    split(to_f32(rb[s][kt]) * ek, bh[s]);
-                    aqb[s] = mm_split(qh, bh[s], aqb[s]);
+                for (int e = 0; e < 2; ++e) {
+                    const f32x4 gi = scan16_incl(in[e].g);
+                    f32x4 eq, ek, ea;
+                    dp.factors<T>(gi, gi - in[e].g, eq, ek, ea);
+                    Split<T> qh, kh, bh[2];
+                    split(to_f32(in[e].k) * ek, kh);
+                    split(to_f32(in[e].q) * eq * scale, qh);
+                    aqk = mm_split(qh, kh, aqk);
                     __builtin_amdgcn_sched_barrier(0);
-                }
 #pragma unroll
-                for (int r = 0; r < 2; ++r) {
-                    Split<T> ah;
-                    split(to_f32(ra[r][kt]) * ea, ah);
-                    aak[r] = mm_split(ah, kh, aak[r]);
-                    aab[r][0] = mm_split(ah, bh[0], aab[r][0]);
-                    aab[r][1] = mm_split(ah, bh[1], aab[r][1]);
-                    __builtin_amdgcn_sched_barrier(0);
+                    for (int s = 0; s < 2; ++s) {
+                        split(to_f32(in[e].b[s]) * ek, bh[s]);
+                        aqb[s] = mm_split(qh, bh[s], aqb[s]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+#pragma unroll
+                    for (int r = 0; r < 2; ++r) {
+                        Split<T> ah;
+                        split(to_f32(in[e].a[r]) * ea, ah);
+                        aak[r] = mm_split(ah, kh, aak[r]);
+                        aab[r][0] = mm_split(ah, bh[0], aab[r][0]);
+                        aab[r][1] = mm_split(ah, bh[1], aab[r][1]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
                 }
             }
         }
     }
+    // v is used last (phase D) but requested here: the barriers in between would otherwise keep its loads, and a
+    // full round trip to HBM, behind everything else
+    Load lv[VTW / 2];
+    if (!SCAN_U)
+#pragma unroll
+    for (int vp = 0; vp < VTW / 2; ++vp) lv[vp].load(vrow + 32 * vp, H * V, cp.len, l);
     if (NWP > 1) {
         // sums over all channels: every wave leaves its parts in LDS and adds the others'
         f32x4* const tiles[9] = {&aak[0], &aak[1], &aab[0][0], &aab[0][1], &aab[1][0], &aab[1][1],
                                  &aqb[0], &aqb[1], &aqk};
 #pragma unroll
-        for (int i = 0; i < NPART; ++i) *reinterpret_cast<f32x4*>(&sPart[((w * NPART + i) * 64 + l) * 4]) = *tiles[i];
+        for (int i = 0; i < NPART; ++i) *reinterpret_cast<f32x4*>(&sMat[NWP - 1 - w][(i * 64 + l) * 4]) = *tiles[i];
         __syncthreads();
+        static_assert(NWP <= 2, "the other wave");
 #pragma unroll
-        for (int ww = 1; ww < NWP; ++ww)
-#pragma unroll
-            for (int i = 0; i < NPART; ++i)
-                *tiles[i] += *reinterpret_cast<const f32x4*>(&sPart[((((w + ww) % NWP) * NPART + i) * 64 + l) * 4]);
+        for (int i = 0; i < NPART; ++i) *tiles[i] += *reinterpret_cast<const f32x4*>(&sMat[w][(i * 64 + l) * 4]);
         if (WB && w == 0 && l == 0) {
             int any = 0;
 #pragma unroll
@@ -280,8 +330,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void 
         if (BWD || WB) {
             // the other orientation is the rounded tile turned (a product with the identity: exact), in every mode, so
             // that a backward pass finds the same bytes whether it recomputes them or reads what a forward pass kept
-            const Frag<T> id = ident_frag<T>();
-            st_pair2(p.ws.AQBT + chw * SBS, transpose(to_frag<T>(aqb[0]), id), transpose(to_frag<T>(aqb[1]), id));
+            st_pair2(p.ws.AQBT + chw * SBS, transpose(to_frag<T>(aqb[0]), ident), transpose(to_frag<T>(aqb[1]), ident));
         }
     }
 #pragma unroll
@@ -349,7 +398,6 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void 
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2)
             tm[s][s2] = to_frag<T>(*reinterpret_cast<const f32x4*>(&sT[(16 * s + c) * LDP + 16 * s2 + 4 * g]));
-    const Frag<T> ident = ident_frag<T>();
     if (WB && w == NWP - 1) {
         // for the chunk_grad kernel: the four blocks transposed, as fragments (two tile pairs), ready to load
         T* tmw = p.ws.TM + chw * 1024;
@@ -357,42 +405,18 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void 
         for (int s = 0; s < 2; ++s) st_pair2(tmw + s * PAIR, transpose(tm[s][0], ident), transpose(tm[s][1], ident));
     }
 
-    // ---- phase C: w = Tm ag and the gated copies, two channel tiles (one stored pair) at a time -----------------
+    // ---- phase C: w = Tm ag, two channel tiles (one stored pair) at a time ---------------------------------------
 #pragma unroll
-    for (int kpl = 0; kpl < KTW / 2; ++kpl) {
-        const int kp = kt0 / 2 + kpl;                         // stored pair
-        Frag<T> fw[2][2], fkgT[2], fbgT[2][2], fqg[2], fqgT[2];   // [..][tile of the pair]
+    for (int kp = 0; kp < KTW / 2; ++kp) {
+        Frag<T> fw[2][2];                                     // [..][tile of the pair]
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-            const int kt = 2 * kpl + e;
-            const f32x4 gl = bcast16<CH - 1>(gi[kt]);
-            const f32x4 egi = exp4<T>(gi[kt]), ege = exp4<T>(ge[kt]), edn = exp4<T>(gl - gi[kt]);
-            const Frag<T> agT[2] = {transpose(to_frag<T>(to_f32(ra[0][kt]) * ege), ident),
-                                    transpose(to_frag<T>(to_f32(ra[1][kt]) * ege), ident)};
+            const Frag<T> agT[2] = {transpose(ag[0][2 * kp + e], ident), transpose(ag[1][2 * kp + e], ident)};
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                fw[s][e] = to_frag<T>(mm2(tm[s][0], tm[s][1], agT[0], agT[1], zero4()));
-            }
-            fqg[e] = to_frag<T>(to_f32(rq[kt]) * egi * scale);
-            const Frag<T> kg = to_frag<T>(to_f32(rk[kt]) * edn);
-            fkgT[e] = transpose(kg, ident);
-            fbgT[0][e] = transpose(to_frag<T>(to_f32(rb[0][kt]) * edn), ident);
-            fbgT[1][e] = transpose(to_frag<T>(to_f32(rb[1][kt]) * edn), ident);
-            if (WB) fqgT[e] = transpose(fqg[e], ident);
-            if (c == 0) {
-                const f32x4 egl = exp4<T>(gl);
-                *reinterpret_cast<f32x4*>(p.ws.EGL + chw * (SAS * (int)sizeof(T) / 4) + 16 * (kt0 + kt) + 4 * g) = egl;
-            }
+            for (int s = 0; s < 2; ++s) fw[s][e] = to_frag<T>(mm2(tm[s][0], tm[s][1], agT[0], agT[1], zero4()));
         }
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            st_pair2(p.ws.W + chw * SAS + (s * KT2 + kp) * PAIR, fw[s][0], fw[s][1]);
-            if (SCAN_U) st_pair2(p.ws.BGT + chw * SAS + (2 * kp + s) * PAIR, fbgT[0][s], fbgT[1][s]);   // (s: the tile of the pair)
-            else st_pair2(p.ws.BGT + chw * SAS + (s * KT2 + kp) * PAIR, fbgT[s][0], fbgT[s][1]);
-        }
-        st_pair2(p.ws.KGT + chw * SAS + kp * PAIR, fkgT[0], fkgT[1]);
-        if (!BWD) st_pair2(p.ws.QG + chw * SAS + kp * PAIR, fqg[0], fqg[1]);
-        if (WB) st_pair2(p.ws.QGT + chw * SBS + kp * PAIR, fqgT[0], fqgT[1]);
+        for (int s = 0; s < 2; ++s) st_pair2(p.ws.W + chw * SAS + (s * KT2 + kt0 / 2 + kp) * PAIR, fw[s][0], fw[s][1]);
     }
 
     // ---- phase D: u = Tm (A_ak v), kept transposed (rows value, inner token) ---------------------------------
@@ -406,10 +430,12 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(2, 2))) void 
         }
         return;
     }
+    Frag<T> rv[2];
 #pragma unroll
     for (int vl = 0; vl < VTW; ++vl) {
         const int vt = vt0 + vl;
-        const Frag<T> vT = transpose(rv[vl], ident);
+        if (vl % 2 == 0) lv[vl / 2].tiles(scratch, cp.len, l, rv);
+        const Frag<T> vT = transpose(rv[vl % 2], ident);
         st_tile(p.ws.VTT + (chw * VT + vt) * TILE, vT);
         const Frag<T> mT[2] = {to_frag<T>(mm(vT, aakf[0], zero4())), to_frag<T>(mm(vT, aakf[1], zero4()))};
         Frag<T> fu[2];
