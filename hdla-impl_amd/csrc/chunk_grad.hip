@@ -19,6 +19,16 @@
 // chunk would hold the whole chunk in registers, at one wave per SIMD, and nothing would overlap its arithmetic
 // with the memory round trips of its neighbours; four waves on a quarter each leave room for two or three
 // workgroups per compute unit.
+//
+// What bounds it: the chain of a chunk's dependent steps at the two or three workgroups a compute unit holds.  The time per
+// (chunk, head) is the same whether its inputs are in the last-level cache or not (K = V = 64: 13.5 ns, 128: 32), and no unit
+// is saturated (vector issue 56 %, address unit 56 %, LDS 36 %, matrix cores 26 % of the time).  So what shortens the chain
+// counts, and what merely saves instructions gave nothing: products requested in the order of their use; three
+// exponentials a channel tile instead of seven; do, v and the score gradients turned by the transposing LDS read instead
+// of a product and a second store each; sum S dS as the diagonal of a product.  Together, bf16, a/b form, before -> after:
+// K = V = 64: 1024 (chunk, head) 22.3 -> 21.4 us, 8192 118.6 -> 116.0, 16384 221.6 -> 214.9; K = V = 128: 1024 41.9 -> 39.8,
+// 16384 537 -> 524.  A fixed grid whose workgroups loop over the pairs was slower (114.7 -> 118.7; 519 -> 552), and so were
+// one 32-deep product in place of two 16-deep ones where tiles pair up (a few registers more, spilled).
 #include "hdla_common.cuh"
 #include "hdla_launch.h"
 
@@ -33,9 +43,10 @@ template <typename T, int K, int V> struct CgLds {
     static constexpr int VP = V + 16 / ES;
     static constexpr int TOK = 0, TOK_B = 6 * CH * VP * ES;
     // first, per wave: its part of A_qk^T, A_ak^T (2 ranks), fp32 tiles in fragment order (read between barriers 1
-    // and 2); later the nine score-gradient tiles, as fragments and as fragments of their transposes (written
-    // between barriers 2 and 3)
-    static constexpr int SCORE = TOK + TOK_B, SCORE_B = NW * 3 * 1024, FIN = SCORE, FIN_B = 18 * TILE * ES;
+    // and 2); later the nine score-gradient tiles, as fragments (4-byte elements: and as fragments of their transposes;
+    // 2-byte ones are turned by the transposing LDS read), written between barriers 2 and 3
+    static constexpr bool TURN = ES == 2;
+    static constexpr int SCORE = TOK + TOK_B, SCORE_B = NW * 3 * 1024, FIN = SCORE, FIN_B = (TURN ? 9 : 18) * TILE * ES;
     // kg of every channel tile (fragments), for dv
     static constexpr int KG = SCORE + (SCORE_B > FIN_B ? SCORE_B : FIN_B), KG_B = (K / 16) * TILE * ES;
     // first: the parts of the nine tiles (fp32), summed in two rounds through NW/2 slots; later, for 2-byte elements: the rows of the seven
@@ -58,7 +69,6 @@ template <typename T, int K, int V> struct CgLds {
 template <typename T, bool GKF32, int K, int V, bool HD> constexpr int cg_waves(bool highest) {
     const bool small = sizeof(T) * K * V <= 2 * 64 * 64;
     if (sizeof(T) != 2) return highest ? 2 : 1;
-    if (HD && GKF32 && small) return 2;                   // fp32 decay next to 2-byte inputs: four more registers a tile
     return small ? 3 : 2;
 }
 

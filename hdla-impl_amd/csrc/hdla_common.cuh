@@ -233,6 +233,17 @@ __device__ __forceinline__ void st_pair2(float* pair, Frag<float> f0, Frag<float
     *reinterpret_cast<f32x4*>(pair + 8 * lane_id() + 4) = f1.v;
 }
 
+// lane (g, c)'s four elements of column c of a tile: of 16 lanes, lane s names the piece with row group s % 4 of row 4 g + s / 4, and lane c
+// gets element c % 4 of the pieces c / 4 + 4 i
+__device__ __forceinline__ Frag<bf16> ld_turned(const char* p) {
+    Frag<bf16> f;
+    f.v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
+    return f;
+}
+
+// where lane l's piece of a tile in fragment order is, in bytes, for the tile turned
+__device__ __forceinline__ int turned_tile(int l) { return (16 * (l & 3) + (l >> 4) * 4 + ((l >> 2) & 3)) * 8; }
+
 // ---- rows of a tensor into fragments, through LDS -----------------------------------------------------------
 // The lanes of a fragment run over the rows first.  Loaded straight from a row-major tensor an instruction touches 64
 // separate pieces of 8 bytes, and the vector cache's address unit takes them one by one: the fused kernels' waves spent
@@ -517,8 +528,8 @@ template <> struct TileDecay<bf16> {
     f32x4 eq, ek, ea;                                     // e^{gi-m}, e^{m-gi}, e^{ge-m}
     f32x4 egi, ege, edn, egl;                             // e^{gi}, e^{ge}, e^{gl-gi}, e^{gl}
     bool strong;                                          // a factor beyond the safe range (the same on every lane)
-    // g4: log-decay of the lane's token and channels; c: the token
-    __device__ __forceinline__ TileDecay(f32x4 g4, int c) {
+    // g4: log-decay of the lane's token and channels; c: the token; check: whether the tile may be a strong one
+    __device__ __forceinline__ TileDecay(f32x4 g4, int c, bool check = true) {
         const f32x4 gi = scan16_incl(g4 * LOG2E), m = bcast16<MID>(gi);
         eq = exp2_4(gi - m);
         ek = exp2_4(m - gi);
@@ -530,7 +541,7 @@ template <> struct TileDecay<bf16> {
         float big = 0.f;
 #pragma unroll
         for (int i = 0; i < 4; ++i) big = fmaxf(fmaxf(big, em[i]), fmaxf(eq[i], ek[i]));
-        strong = __any(!(big <= SAFE_FACTOR)) != 0;
+        strong = check && __any(!(big <= SAFE_FACTOR)) != 0;
         ea = prev_token(eq, em);
         egi = eq * bcast16<1>(em);
         edn = ek * bcast16<CH - 1>(eq);
@@ -548,7 +559,7 @@ template <> struct TileDecay<bf16> {
 template <> struct TileDecay<float> {
     f32x4 eq, ek, ea, egi, ege, edn, egl;
     bool strong;
-    __device__ __forceinline__ TileDecay(f32x4 g4, int) {
+    __device__ __forceinline__ TileDecay(f32x4 g4, int, bool check = true) {
         const f32x4 gi = scan16_incl(g4), ge = gi - g4, m = bcast16<MID>(gi), gl = bcast16<CH - 1>(gi);
         eq = exp4<float>(gi - m);
         ek = exp4<float>(m - gi);
@@ -560,7 +571,7 @@ template <> struct TileDecay<float> {
         float big = 0.f;
 #pragma unroll
         for (int i = 0; i < 4; ++i) big = fmaxf(big, fmaxf(fabsf(gi[i] - m[i]), fabsf(ge[i] - m[i])));
-        strong = __any(!(big <= SAFE_RANGE)) != 0;
+        strong = check && __any(!(big <= SAFE_RANGE)) != 0;
     }
 };
 

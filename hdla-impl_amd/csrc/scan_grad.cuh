@@ -39,14 +39,6 @@ template <int K, int V, int NWC, bool SUM> struct RevCfg {
     static constexpr int DBUF = SLOTS * SLOT, XBUF = DBUF + 2 * DB, BYTES = XBUF + 2 * XB;
 };
 
-// lane (g, c)'s four elements of column c of a tile: of 16 lanes, lane s names the piece with row group s % 4 of row 4 g + s / 4, and lane c
-// gets element c % 4 of the pieces c / 4 + 4 i
-__device__ __forceinline__ Frag<bf16> ld_turned(const char* p) {
-    Frag<bf16> f;
-    f.v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
-    return f;
-}
-
 // Step t handles chunk c1 - 1 - t.
 template <int K, int V, int NWC, bool SUM>
 __device__ __forceinline__ void scan_rev_body(const ChunkArgs<bf16>& p, char* smem, int n, int seg, int split) {
