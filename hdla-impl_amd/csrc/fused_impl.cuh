@@ -6,8 +6,9 @@
 // Work division.  A workgroup owns one (sequence, head, time segment): the chunks of a sequence are cut into `nseg`
 // consecutive segments so that few (sequence, head) pairs still fill the device.  It has
 //   * FNP = 4 pairs of producer waves.  Pair p prepares the chunks p, p+4, ... of the segment and leaves the operands in
-//     LDS slot p.  The two waves of a pair take two of the four channel tiles and half of the value tiles each; one of
-//     them (the pair's lead) also adds up the two waves' parts of the score tiles and solves for (I - A_ab)^-1;
+//     LDS slot p.  The two waves of a pair take two of the four channel tiles each.  What comes after their parts of the
+//     score tiles is shared out by what the longer chain leaves room for: one of them (the pair's lead) adds up A_ab and
+//     solves for (I - A_ab)^-1; the other one adds up the other score tiles, has v to itself (A_ak v, then u) and copies out;
 //   * V/16 consumer waves.  Consumer j owns column block j of the fp32 state for the whole segment, in registers, and
 //     walks the chunks in order, exactly as the stand-alone scan kernels do.
 // A segment other than the first does not know the state that enters it.  The state leaving a chunk is affine in the
@@ -35,6 +36,17 @@
 // Waiting is polling with s_sleep; every wait is bounded (FUSED_SPIN_LIMIT polls), and a wave that runs into the bound
 // raises an abort flag that ends every other wave's waits as well and is reported through FusedArgs::err, so the grid
 // always drains.  There are no workgroup barriers after the first.
+//
+// What bounds the forward kernel: the producers' instructions.  A pair takes 13 k cycles a chunk, four pairs 3.3 k, the
+// consumers 1.3 k; the two producer waves of a SIMD and its consumer issue vector instructions 70 to 80 % of the time, and
+// requesting the inputs earlier gains nothing.  Two things had cost a tenth of it on top.  The lead did everything on its
+// own while the other wave waited for the inverse: 4 of 15 k cycles.  And a SIMD prefers its older wave: pairs 0 and 1 ran a
+// whole round ahead of pairs 2 and 3, whose chunks the consumers needed first, until they stood still for want of a slot;
+// with the waves that are past the scores, so nearer to the hand-over, preferred (s_setprio), the pairs take turns.
+// us for a forward pass, before -> the work shared out -> and the priority: 4 x 2048 tokens of 16 heads 76.2 -> 74.0 -> 71.6 (a
+// and b formed here 77.6 -> 74.4 -> 70.6), 8 x 1024 70.6 -> 67.3 -> 64.1, 16 x 512 of 32 heads 116.5 -> 110.7 -> 101, 1 x 16384 154 ->
+// 149 -> 140, 2 x 777 of 8 heads 33.8 -> 32.5 -> 30.6.  Priority for the consumers as well: 72.8; a third level for the solve: the
+// same; and in fused_replay, which is bound by its traffic: the same or 5 % more.
 #pragma once
 #include "hdla_common.cuh"
 #include "fused_shapes.h"
@@ -152,10 +164,10 @@ template <typename T> __device__ __forceinline__ Frag<T> ident_of(int g, int c) 
 
 // ---- producers -----------------------------------------------------------------------------------------------------
 // Everything of a chunk that does not depend on the state, by a PAIR of waves, into LDS slot `pp`.  Wave `half` of the
-// pair takes the channel tiles 2 half, 2 half + 1 (one stored tile pair of every operand) and half of the value tiles.
-// The score tiles are sums over all channels: the other wave hands its parts to the pair's `lead` wave through LDS, the
-// lead solves the (small) triangular system and hands (I - A_ab)^-1 and A_ak back, and each forms w and u for its own
-// tiles.  The formulas are the stand-alone prep kernel's (prep.hip); what differs from its one-wave form is the order
+// pair takes the channel tiles 2 half, 2 half + 1 (one stored tile pair of every operand).  The score tiles are sums over
+// all channels: each wave hands the other its parts of some through LDS.  The pair's `lead` wave finishes A_ab, solves the
+// (small) triangular system and hands (I - A_ab)^-1 back; meanwhile the other wave finishes A_qk, A_qb and A_ak, forms A_ak v
+// and copies out the chunk before; each forms w for its own tiles, the other wave u.  The formulas are the stand-alone prep kernel's (prep.hip); what differs from its one-wave form is the order
 // in which the two halves of a score tile's sum over channels are added.
 //
 // One wave per chunk (the first form of this kernel) took 19,000 cycles a chunk, most of them waiting for its own
@@ -166,7 +178,7 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
     typedef FusedLds<T, K, V, MODE> L;
     constexpr bool FWD = MODE == FUSED_FWD;
     static_assert(L::SOLVES, "the backward pass's kernels read what this producer solves for (fused_replay)");
-    constexpr int KT = K / 16, VT = V / 16, KT2 = KT / 2, KH = 2, VH = VT / 2;
+    constexpr int KT = K / 16, VT = V / 16, KT2 = KT / 2, KH = 2;
     constexpr BlkF BF = L::BF;
     const ChunkArgs<T>& p = a.c;
     char* slot = smem + pp * L::SLOT;
@@ -176,13 +188,13 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
     T* sPub;
     int* const flags = reinterpret_cast<int*>(smem + L::FLAGS);
     int* const f_ready = flags + pp, * const f_consumed = flags + 4 + pp, * const f_abort = flags + 8;
-    int* const f_part = flags + 12 + pp, * const f_inv = flags + 16 + pp, * const f_strong = flags + 20 + pp;
+    int* const f_part = flags + 12 + pp, * const f_inv = flags + 16 + pp, * const f_strong = flags + 20 + pp, * const f_rest = flags + 28 + pp;
     const bool lead = half == (pp >> 1);                  // spreads the leads over the SIMDs
     int l = lane_id(), g = l >> 4, c = l & 15;
     const int H = p.H;
     const float scale = p.scale;
     const int nst = s1 - s0;
-    const int kt0 = half * KH, vt0 = half * VH;
+    const int kt0 = half * KH;
     int64_t bos, eos;
     seq_bounds(p.st, n, bos, eos);
     int c0, c1;
@@ -233,7 +245,7 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
     // With the HDLA parameterisation the sum over ALL channels of k^2 f is needed: the other half's k and gk come along.
     // In parts, by what three waves per SIMD have registers for: 0 beside the score tiles, 1 when those are done with; v (2)
     // only behind the scores of its own chunk; the decays once more (3) where the strong-decay passes want them.
-    i32x4 xq, xk, xa[2], xb[2], xv, xok;
+    i32x4 xq, xk, xa[2], xb[2], xv[2], xok;
     typename GkRaw<T, GKF32>::rows xg, xog;
     T nbeta;
     char* const sX = lead ? smem + L::ROWS + pp * ROWS_SCRATCH : smem + pp * L::SLOT + L::SOLVE + 32 * FLDP * 4;
@@ -249,7 +261,8 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
         const uint32_t row = (uint32_t)min(ll >> 2, max(len, 1) - 1), last = (uint32_t)(max(len, 1) - 1), piece = 16 * (ll & 3);
         constexpr uint32_t ES = sizeof(T), GS = GKF32 ? 4 : 2;
         if (part == 2) {
-            xv = *reinterpret_cast<const i32x4*>(at(p.v + (tok0 * H + h) * V, (row * (uint32_t)(H * V) + 16 * vt0) * ES + piece));
+#pragma unroll
+            for (int j = 0; j < 2; ++j) xv[j] = *reinterpret_cast<const i32x4*>(at(p.v + (tok0 * H + h) * V, (row * (uint32_t)(H * V) + 32 * j) * ES + piece));
             return;
         }
         const uint32_t qo = (row * (uint32_t)(H * K) + 16 * kt0) * ES + piece, ao = (row * (uint32_t)(RANK * H * K) + 16 * kt0) * ES + piece;
@@ -286,15 +299,11 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
     // their old values stay in registers through the whole chunk)
     auto forget_first = [&]() __attribute__((always_inline)) { GkRaw<T, GKF32>::drop(xg); forget(xk); forget(xb[0]); forget(xb[1]); };
     auto forget_rest = [&]() __attribute__((always_inline)) { GkRaw<T, GKF32>::drop(xog); forget(xok); forget(xq); forget(xa[0]); forget(xa[1]); };
-    auto gave_up = [&]() __attribute__((always_inline)) {
-        if (l == 0) *a.err = FUSED_ABORTED + 1;
-        forget_first();
-        forget_rest();
-        forget(xv);
-    };
-
+    // A wait that gave up (see wait_ge) ends the loop, not the chunk: with the abort flag up no later wait takes time, what the chunk's steps
+    // then make of LDS is thrown away, no address depends on it, and the steps stay one straight piece of code for the register allocation.
+    bool alive = true;
     int it = 0, prev_cid = -1;
-    for (int t = pp; t < nst; t += FNP, ++it) {
+    for (int t = pp; t < nst && alive; t += FNP, ++it) {
         const int cid = s0 + t;
         const int64_t tok0 = bos + (int64_t)(cid - c0) * CH;
         const int len = (int)min((int64_t)CH, eos - tok0);
@@ -473,81 +482,94 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
                 }
             }
         }
-        // ---- the other wave's parts travel to the lead ------------------------------------------------------------------
-        // tile order in the scratch: A_ab (4), A_ak (2), A_qb (2), A_qk (where the outputs are formed)
-        constexpr int NPART = FWD ? 9 : 8;
-        if (!lead) {
-            f32x4* const tiles[9] = {&aab[0][0], &aab[0][1], &aab[1][0], &aab[1][1], &aak[0], &aak[1],
-                                     &aqb[0], &aqb[1], &aqk};
+        __builtin_amdgcn_s_setprio(1);                    // nearer to the hand-over than a wave that forms scores (see the top of the file)
+        // ---- what both waves do with their own channel tiles ------------------------------------------------------------
+        auto gated = [&]() __attribute__((always_inline)) {
+            // gated copies (prep.hip, phase C), each to its half of the stored pair
 #pragma unroll
-            for (int i = 0; i < NPART; ++i) *reinterpret_cast<f32x4*>(sP + (i * 64 + l) * 4) = *tiles[i];
-            if (l == 0) *f_strong = strong;
-            signal_set(f_part, it + 1);
-        }
-
-        request(t, 2);
-        __builtin_amdgcn_sched_barrier(0);
-        // ---- the slot: wait until the consumers have left the chunk it held ---------------------------------------------
-        if (!wait_ge(f_consumed, VT * it, f_abort)) { gave_up(); return; }
-        __builtin_amdgcn_sched_barrier(0);
-        // ---- gated copies of the own channel tiles (prep.hip, phase C), each to its half of the stored pair --------------
-#pragma unroll
-        for (int j = 0; j < KH; ++j) {
-            pin(nq[j]); pin(nk[j]);                       // converted again, not kept converted from above
-            if (HD) pin(ng[j]);
-            else { pin(na[0][j]); pin(na[1][j]); pin(nb[0][j]); pin(nb[1][j]); }
-            Frag<T> rq, rk, ra[2], rb[2];
-            operands(j, HD ? GkRaw<T, GKF32>::value(ng[j]) : zero4(), rq, rk, ra, rb);
-            const f32x4 one = {1.f, 1.f, 1.f, 1.f}, ege = prev_token(egi[j], one), egl = bcast16<CH - 1>(egi[j]);
-            st_pair2(sWW + (j * KT2 + half) * PAIR, transpose(to_frag<T>(to_f32(ra[0]) * ege), ident),
-                     transpose(to_frag<T>(to_f32(ra[1]) * ege), ident));
-            const Frag<T> fqg = to_frag<T>(to_f32(rq) * egi[j] * scale);
-            const Frag<T> fbg[2] = {to_frag<T>(to_f32(rb[0]) * edn[j]), to_frag<T>(to_f32(rb[1]) * edn[j])};
-            st_pair(reinterpret_cast<T*>(slot + BF.KGT) + half * PAIR, j, transpose(to_frag<T>(to_f32(rk) * edn[j]), ident));
-            st_pair2(reinterpret_cast<T*>(slot + BF.BGT) + (kt0 + j) * PAIR, transpose(fbg[0], ident), transpose(fbg[1], ident));
-            st_pair(reinterpret_cast<T*>(slot + BF.QG) + half * PAIR, j, fqg);
-            if (c == 0) *reinterpret_cast<f32x4*>(slot + BF.EGL + (16 * (kt0 + j) + 4 * g) * 4) = egl;
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        Frag<T> vT[VH];
-        rows_to_tiles(slot + L::UT + vt0 * PAIR * (int)sizeof(T), l, xv, vT[0], vT[1]);   // (where u of these tiles goes later)
-#pragma unroll
-        for (int j = 0; j < VH; ++j) {
-            if (len < CH) mask(vT[j], rowok);
-            vT[j] = transpose(vT[j], ident);
-            st_frag(reinterpret_cast<T*>(slot + L::VTT) + (vt0 + j) * TILE + 4 * l, vT[j]);
-        }
-        // the inputs are used up: the next chunk's may come
-        __builtin_amdgcn_sched_barrier(0);
-        forget_first();
-        if (t + FNP < nst) request(t + FNP, 0);
-        __builtin_amdgcn_sched_barrier(0);
-
-        // ---- the lead: whole score tiles, (I - A_ab)^-1 by forward substitution (prep.hip, phase B) ---------------------
-        Frag<T> tm[2][2], aakf[2];
-        if (lead) {
-            if (!wait_ge(f_part, it + 1, f_abort)) { gave_up(); return; }
-            f32x4* const tiles[9] = {&aab[0][0], &aab[0][1], &aab[1][0], &aab[1][1], &aak[0], &aak[1],
-                                     &aqb[0], &aqb[1], &aqk};
-            // the lower channel tiles' part first, as a single wave adds them
-#pragma unroll
-            for (int i = 0; i < NPART; ++i) {
-                const f32x4 o = *reinterpret_cast<const f32x4*>(sP + (i * 64 + l) * 4);
-                *tiles[i] = half == 0 ? *tiles[i] + o : o + *tiles[i];
+            for (int j = 0; j < KH; ++j) {
+                pin(nq[j]); pin(nk[j]);                       // converted again, not kept converted from above
+                if (HD) pin(ng[j]);
+                else { pin(na[0][j]); pin(na[1][j]); pin(nb[0][j]); pin(nb[1][j]); }
+                Frag<T> rq, rk, ra[2], rb[2];
+                operands(j, HD ? GkRaw<T, GKF32>::value(ng[j]) : zero4(), rq, rk, ra, rb);
+                const f32x4 one = {1.f, 1.f, 1.f, 1.f}, ege = prev_token(egi[j], one), egl = bcast16<CH - 1>(egi[j]);
+                st_pair2(sWW + (j * KT2 + half) * PAIR, transpose(to_frag<T>(to_f32(ra[0]) * ege), ident),
+                         transpose(to_frag<T>(to_f32(ra[1]) * ege), ident));
+                const Frag<T> fqg = to_frag<T>(to_f32(rq) * egi[j] * scale);
+                const Frag<T> fbg[2] = {to_frag<T>(to_f32(rb[0]) * edn[j]), to_frag<T>(to_f32(rb[1]) * edn[j])};
+                st_pair(reinterpret_cast<T*>(slot + BF.KGT) + half * PAIR, j, transpose(to_frag<T>(to_f32(rk) * edn[j]), ident));
+                st_pair2(reinterpret_cast<T*>(slot + BF.BGT) + (kt0 + j) * PAIR, transpose(fbg[0], ident), transpose(fbg[1], ident));
+                st_pair(reinterpret_cast<T*>(slot + BF.QG) + half * PAIR, j, fqg);
+                if (c == 0) *reinterpret_cast<f32x4*>(slot + BF.EGL + (16 * (kt0 + j) + 4 * g) * 4) = egl;
+                __builtin_amdgcn_sched_barrier(0);
             }
-            if (p.ws.TM && l == 0) p.ws.STRONG[chw] = (strong || *f_strong != 0) ? 1 : 0;
-            // causal masks: lane (g,c) reg i is entry (row c, inner 4g+i)
+        };
+        // the inputs are used up: the next chunk's may come
+        auto next_first = [&]() __attribute__((always_inline)) {
+            __builtin_amdgcn_sched_barrier(0);
+            forget_first();
+            if (t + FNP < nst) request(t + FNP, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto next_rest = [&]() __attribute__((always_inline)) {
+            __builtin_amdgcn_sched_barrier(0);
+            forget_rest();
+            if (t + FNP < nst) request(t + FNP, 1);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto form_w = [&](const Frag<T> (&tm)[2][2]) __attribute__((always_inline)) {
+            // w = Tm ag, in place of ag^T
+            {
+                Frag<T> agT[2][2], fw[2][2];
+                ld_pair(sWW + half * PAIR, agT[0][0], agT[1][0]);
+                ld_pair(sWW + (KT2 + half) * PAIR, agT[0][1], agT[1][1]);
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+#pragma unroll
+                    for (int s = 0; s < 2; ++s) {
+                        fw[s][e] = to_frag<T>(mm2(tm[s][0], tm[s][1], agT[0][e], agT[1][e], zero4()));
+                    }
+#pragma unroll
+                for (int s = 0; s < 2; ++s) st_pair2(sWW + (s * KT2 + half) * PAIR, fw[s][0], fw[s][1]);
+            }
+        };
+        // causal masks: lane (g,c) reg i is entry (row c, inner 4g+i)
+        auto below = [&](f32x4& x, bool diag) __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int j = 4 * g + i;
-                const bool le = j <= c, lt = j < c;
-                if (!le) { aqk[i] = 0.f; aqb[0][i] = 0.f; aqb[1][i] = 0.f; }
-                if (!lt) { aak[0][i] = 0.f; aak[1][i] = 0.f; aab[0][0][i] = 0.f; aab[0][1][i] = 0.f; aab[1][0][i] = 0.f; aab[1][1][i] = 0.f; }
+                if (!(diag ? j <= c : j < c)) x[i] = 0.f;
             }
-            if (FWD) st_frag(reinterpret_cast<T*>(slot + BF.AQK) + 4 * l, to_frag<T>(aqk));
-            st_pair2(reinterpret_cast<T*>(slot + BF.AQB), to_frag<T>(aqb[0]), to_frag<T>(aqb[1]));
-            aakf[0] = to_frag<T>(aak[0]);
-            aakf[1] = to_frag<T>(aak[1]);
+        };
+        // Each wave leaves the other its parts of the score tiles that the other one finishes: the lead has A_ab, the other wave the
+        // rest, whose parts lie in the slot where that wave itself writes later (u's place and, the fifth, A_ak's).
+        constexpr int NPART = FWD ? 5 : 4;
+        static_assert(VT == 4, "four tiles in u's place");
+        auto part_at = [&](int i) __attribute__((always_inline)) { return reinterpret_cast<f32x4*>(slot + (i < 4 ? L::UT + i * 1024 : L::AKB) + 16 * l); };
+        f32x4* const rest[5] = {&aak[0], &aak[1], &aqb[0], &aqb[1], &aqk};
+        if (lead) {
+            // the slot: wait until the consumers have left the chunk it held
+            __builtin_amdgcn_sched_barrier(0);
+            alive &= wait_ge(f_consumed, VT * it, f_abort);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < NPART; ++i) *part_at(i) = *rest[i];
+            signal_set(f_rest, it + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            gated();
+            next_first();
+            // ---- whole A_ab, (I - A_ab)^-1 by forward substitution (prep.hip, phase B) -----------------------------------
+            Frag<T> tm[2][2];
+            alive &= wait_ge(f_part, it + 1, f_abort);
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    aab[r][s] += *reinterpret_cast<const f32x4*>(sP + ((2 * r + s) * 64 + l) * 4);
+                    below(aab[r][s], false);
+                }
+            if (p.ws.TM && l == 0) p.ws.STRONG[chw] = (strong || *f_strong != 0) ? 1 : 0;
             // (all of the other wave's parts have been read: the scratch may be written)
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -616,60 +638,87 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
 #pragma unroll
                 for (int s2 = 0; s2 < 2; ++s2)
                     tm[s][s2] = to_frag<T>(*reinterpret_cast<const f32x4*>(&sT[(16 * s + c) * FLDP + 16 * s2 + 4 * g]));
-            // for the other wave: the inverse's four blocks and A_ak as operand tiles (in A_ab's bytes, which are used up)
+            // for the other wave: the inverse's four blocks as operand tiles (in A_ab's bytes, which are used up)
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int s = 0; s < 2; ++s) st_pair2(sPub + s * PAIR, tm[s][0], tm[s][1]);
-            st_pair2(sPub + 2 * PAIR, aakf[0], aakf[1]);
             if (p.ws.TM) {
                 // the record goes out from the consumers, which have no loads to wait for: a store issued here would stand
                 // behind the next chunk's loads in this wave's in-order memory counter
                 T* tmw = reinterpret_cast<T*>(slot + L::TMB);
 #pragma unroll
                 for (int s = 0; s < 2; ++s) st_pair2(tmw + s * PAIR, transpose(tm[s][0], ident), transpose(tm[s][1], ident));
-                st_pair2(reinterpret_cast<T*>(slot + L::AKB), aakf[0], aakf[1]);
             }
             signal_set(f_inv, it + 1);
+            next_rest();
+            form_w(tm);
         } else {
-            // while the lead solves: the rows the consumers left in the outbox for the chunk the slot held (they write the
+            f32x4* const parts[4] = {&aab[0][0], &aab[0][1], &aab[1][0], &aab[1][1]};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) *reinterpret_cast<f32x4*>(sP + (i * 64 + l) * 4) = *parts[i];
+            if (l == 0) *f_strong = strong;
+            signal_set(f_part, it + 1);
+            request(t, 2);
+            __builtin_amdgcn_sched_barrier(0);
+            alive &= wait_ge(f_consumed, VT * it, f_abort);
+            __builtin_amdgcn_sched_barrier(0);
+            // the other score tiles, whole
+            alive &= wait_ge(f_rest, it + 1, f_abort);
+#pragma unroll
+            for (int i = 0; i < NPART; ++i) {
+                *rest[i] += *part_at(i);
+                below(*rest[i], i >= 2);
+            }
+            if (FWD) st_frag(reinterpret_cast<T*>(slot + BF.AQK) + 4 * l, to_frag<T>(aqk));
+            st_pair2(reinterpret_cast<T*>(slot + BF.AQB), to_frag<T>(aqb[0]), to_frag<T>(aqb[1]));
+            const Frag<T> aakf[2] = {to_frag<T>(aak[0]), to_frag<T>(aak[1])};
+            if (p.ws.TM) st_pair2(reinterpret_cast<T*>(slot + L::AKB), aakf[0], aakf[1]);
+            __builtin_amdgcn_sched_barrier(0);
+            gated();
+            // v, turned, of all value tiles
+            char* const sV = slot + L::VTT;
+            static_assert(ROWS_SCRATCH <= VT * TILE * (int)sizeof(T), "");
+            Frag<T> vT[VT];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) rows_to_tiles(sV, l, xv[j], vT[2 * j], vT[2 * j + 1]);
+#pragma unroll
+            for (int j = 0; j < VT; ++j) {
+                if (len < CH) mask(vT[j], rowok);
+                vT[j] = transpose(vT[j], ident);
+                st_frag(reinterpret_cast<T*>(sV) + j * TILE + 4 * l, vT[j]);
+            }
+            next_first();
+            // ---- while the lead solves: A_ak v, and the rows the consumers left in the outbox for the chunk the slot held (they write the
             // outbox again only after both signals at the end)
+            Frag<T> mT[VT][2];
+#pragma unroll
+            for (int j = 0; j < VT; ++j)
+#pragma unroll
+                for (int r = 0; r < 2; ++r) mT[j][r] = to_frag<T>(mm(vT[j], aakf[r], zero4()));
+            __builtin_amdgcn_sched_barrier(0);
             if (it > 0) copy_out(prev_cid, 0, std::integral_constant<int, CH>());
-            if (!wait_ge(f_inv, it + 1, f_abort)) { gave_up(); return; }
+            alive &= wait_ge(f_inv, it + 1, f_abort);
+            Frag<T> tm[2][2];
 #pragma unroll
             for (int s = 0; s < 2; ++s) ld_pair(sPub + s * PAIR, tm[s][0], tm[s][1]);
-            ld_pair(sPub + 2 * PAIR, aakf[0], aakf[1]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        forget_rest();
-        if (t + FNP < nst) request(t + FNP, 1);
-        __builtin_amdgcn_sched_barrier(0);
-        // ---- w = Tm ag for the own channel tiles, in place of ag^T -------------------------------------------------------
-        {
-            Frag<T> agT[2][2], fw[2][2];
-            ld_pair(sWW + half * PAIR, agT[0][0], agT[1][0]);
-            ld_pair(sWW + (KT2 + half) * PAIR, agT[0][1], agT[1][1]);
+            next_rest();
+            form_w(tm);
+            // ---- u = Tm (A_ak v), transposed (prep.hip, phase D) ---------------------------------------------------------
 #pragma unroll
-            for (int e = 0; e < 2; ++e)
+            for (int j = 0; j < VT; ++j) {
+                Frag<T> fu[2];
 #pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    fw[s][e] = to_frag<T>(mm2(tm[s][0], tm[s][1], agT[0][e], agT[1][e], zero4()));
-                }
-#pragma unroll
-            for (int s = 0; s < 2; ++s) st_pair2(sWW + (s * KT2 + half) * PAIR, fw[s][0], fw[s][1]);
-        }
-        // ---- u = Tm (A_ak v) for the own value tiles, transposed (prep.hip, phase D) ------------------------------------
-#pragma unroll
-        for (int j = 0; j < VH; ++j) {
-            const Frag<T> mT[2] = {to_frag<T>(mm(vT[j], aakf[0], zero4())), to_frag<T>(mm(vT[j], aakf[1], zero4()))};
-            Frag<T> fu[2];
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                fu[s] = to_frag<T>(mm2(mT[0], mT[1], tm[s][0], tm[s][1], zero4()));
+                for (int s = 0; s < 2; ++s) fu[s] = to_frag<T>(mm2(mT[j][0], mT[j][1], tm[s][0], tm[s][1], zero4()));
+                st_pair2(reinterpret_cast<T*>(slot + L::UT) + j * PAIR, fu[0], fu[1]);
             }
-            st_pair2(reinterpret_cast<T*>(slot + L::UT) + (vt0 + j) * PAIR, fu[0], fu[1]);
         }
         signal_add(f_ready);
+        __builtin_amdgcn_s_setprio(0);
         prev_cid = cid;
+    }
+    if (!alive) {
+        if (l == 0) *a.err = FUSED_ABORTED + 1;
+        return;
     }
     // the last chunk's rows, half by each wave
     if (FWD && it > 0) {
@@ -960,6 +1009,7 @@ __device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* 
 #pragma unroll
             for (int i = 0; i < 4; ++i) S[kt][i] = p.h0[soff + (int64_t)(16 * kt + 4 * g + i) * V];
     }
+
 
     for (int t = 0; t < nst; ++t) {
         const int pp = t & (FNP - 1), it = t / FNP;
