@@ -408,7 +408,7 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
     }
     if (d->cu_seqlens && (stages & HDLA_STAGE_PREP)) {
         char* base = static_cast<char*>(prep_ws);
-        e = launch_chunk_table(d->cu_seqlens, d->N, d->T, nch, reinterpret_cast<int32_t*>(base + LP.CHUNK_OFF),
+        e = launch_chunk_table(d->cu_seqlens, d->N, d->T, nch, d->H, d->in_dtype == HDLA_FP32 ? 0 : d->V, reinterpret_cast<int32_t*>(base + LP.CHUNK_OFF),
                                reinterpret_cast<int32_t*>(base + LP.CHUNK_SEQ), packed_outputs(d, a), stream);
         if (e != hipSuccess) return (int)e;
     }
@@ -501,7 +501,7 @@ int run_fused(const hdla_dims* d, bool fwd, const void* q, const void* k, const 
     f.err = reinterpret_cast<int*>(base + L.ERR);
     hipError_t e;
     if (d->cu_seqlens && (stages & HDLA_STAGE_PREP)) {
-        e = launch_chunk_table(d->cu_seqlens, d->N, d->T, L.nch, reinterpret_cast<int32_t*>(base + L.CHUNK_OFF),
+        e = launch_chunk_table(d->cu_seqlens, d->N, d->T, L.nch, d->H, 0, reinterpret_cast<int32_t*>(base + L.CHUNK_OFF),
                                reinterpret_cast<int32_t*>(base + L.CHUNK_SEQ), packed_outputs(d, a), stream);
         if (e != hipSuccess) return (int)e;
     }

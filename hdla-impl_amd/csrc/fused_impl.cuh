@@ -1434,7 +1434,7 @@ __global__ __launch_bounds__(64 * (V / 16 + 2 * FNP)) void fused_kernel(FusedArg
     typedef FusedLds<T, K, V, MODE> L;
     __shared__ __attribute__((aligned(16))) char smem[L::BYTES];
     const int h = blockIdx.x, seg = blockIdx.y;
-    const int n = a.c.st.cu ? a.c.st.order[blockIdx.z] : (int)blockIdx.z;
+    const int n = scan_sequence(a.c.st, blockIdx.z);
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int s0, s1;
     seg_range(a.c.st, n, a.nseg, seg, s0, s1);
@@ -1477,7 +1477,7 @@ __global__ __launch_bounds__(256) void fixup_kernel(FusedArgs<T> a) {
     __shared__ __attribute__((aligned(16))) T sM[FIXUP_STAGE][2][KT * KT * TILE];   // transition records, hi and lo halves
     const ChunkArgs<T>& p = a.c;
     const int h = blockIdx.x;
-    const int n = p.st.cu ? p.st.order[blockIdx.z] : (int)blockIdx.z;
+    const int n = scan_sequence(p.st, blockIdx.z);
     const int ty = (int)blockIdx.y / FIXUP_PARTS, part = (int)blockIdx.y % FIXUP_PARTS;
     const int target = ty == 0 ? a.nseg : ty;                            // chain segments 0 .. target-1
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

@@ -387,6 +387,8 @@ __device__ __forceinline__ bool locate_chunk(const SeqTab& st, int cid, ChunkPos
     return cp.len > 0;
 }
 
+// the z-th sequence in the order in which workgroups start: packed ones from the longest down (all that `order` is read with, but for scan_share)
+__device__ __forceinline__ int scan_sequence(const SeqTab& st, int z) { return st.cu ? st.order[z] & ORDER_SEQ : z; }
 // chunk range [c0, c1) of sequence n (n: the same on every lane)
 __device__ __forceinline__ void seq_chunks(const SeqTab& st, int n, int& c0, int& c1) {
     if (st.cu == nullptr) { c0 = n * st.NT; c1 = c0 + st.NT; }

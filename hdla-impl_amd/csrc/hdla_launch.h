@@ -14,8 +14,9 @@ struct PackedOut {
     int n;
     void add(void* q, long long b) { if (q) { p[n] = q; row[n++] = b; } }
 };
-hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int32_t* chunk_off, int32_t* chunk_seq, const PackedOut& out,
-                              hipStream_t stream);
+// (V: of the 2-byte stand-alone scans, which share the device by the sequences' lengths; 0 for the other kernels)
+hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int H, int V, int32_t* chunk_off, int32_t* chunk_seq,
+                              const PackedOut& out, hipStream_t stream);
 // only what clears the rows that belong to no sequence
 hipError_t launch_clear_uncovered(const int64_t* cu, int N, int T, const PackedOut& out, hipStream_t stream);
 

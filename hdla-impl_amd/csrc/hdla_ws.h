@@ -20,10 +20,17 @@ struct SeqTab {
     const int64_t* cu;        // nullable
     const int32_t* chunk_off; // valid when cu != nullptr
     const int32_t* chunk_seq; // valid when cu != nullptr: sequence of each chunk
-    const int32_t* order;     // valid when cu != nullptr: int32[N], the sequences from the one with the most chunks down
+    const int32_t* order;     // valid when cu != nullptr: int32[N], the sequences from the one with the most chunks down (see ORDER_SEQ)
     int T, NT, N;
     int nch;                  // chunk slots the workspace is laid out for (an upper bound with cu_seqlens)
 };
+
+// Few packed sequences of unequal length share the device by their lengths: build_chunk_table_kernel leaves beside each entry of `order`, for
+// the forward pass's scan and for the backward pass's two, how many column blocks a workgroup of that sequence has: 4 >> code.
+constexpr int SHARE_MAX_N = 32, ORDER_SEQ = 0x0fffffff, ORDER_OUT = 28, ORDER_GRAD = 30;
+// workgroups of a head (and direction) that the device holds at once, one a compute unit, and as many as a shared launch has at the most
+constexpr int share_slots(int H, int directions) { return 256 / (H * directions) > 1 ? 256 / (H * directions) : 1; }
+constexpr int share_most(int H, int directions, int N, int V) { return N * (V / 64) + share_slots(H, directions); }
 
 // Operands of the state scans that all value-column blocks of a (chunk, head) share are kept in ONE contiguous
 // block per (chunk, head), so that a workgroup can copy a block into LDS with a few whole-kilobyte loads.

@@ -491,8 +491,58 @@ __device__ __forceinline__ void clear_uncovered(const int64_t* cu, int N, int T,
 __global__ __launch_bounds__(TABLE_THREADS) void clear_uncovered_kernel(const int64_t* cu, int N, int T, PackedOut out) {
     clear_uncovered(cu, N, T, out, blockIdx.x, gridDim.x, threadIdx.x);
 }
-__global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const int64_t* cu, int N, int T, int nch, int32_t* chunk_off,
-                                                                          int32_t* chunk_seq, int rankers, PackedOut out) {
+// How wide the workgroups of each sequence are in the scans of the backward and the forward pass.  A workgroup of fewer column blocks takes a shorter
+// step, but more workgroups read a chunk's block.  Unequal lengths want unequal widths: a launch ends with its longest sequence, which walks its last
+// steps on a device that the others have left.  Candidates: every length in every width as the time that no sequence may exceed where a
+// narrower workgroup helps it; of these the one whose longest walk, or whose work spread over the slots, is least.  (Column blocks never meet: the
+// results have the same bits in every width.)  Times of a step of 4, 2 and
+// 1 blocks, 10 ns, one sequence of 16 heads alone on the device, K = V = 128: forward 81, 60, 58, both scans 105, 87, 78 (K = 64: 42, 35, 34; 59,
+// 51, 45); the choice needs their ratios only.
+constexpr float SHARE_STEP[2][3] = {{81.f, 60.f, 58.f}, {105.f, 87.f, 78.f}}, SHARE_PROLOGUE = 6.f;
+// More workgroups than slots leave gaps behind them.  Over 1500 random batches of 2 to 14 sequences, the choice against the best of its candidates with the
+// workgroups dealt out one by one: 0.3 % on average, 12 % at the most (without the factor 0.8 and 41 %; one width for all 17 and 40 %).
+constexpr float SHARE_PACKING = 1.15f;
+struct ShareLds {
+    float steps[SHARE_MAX_N];                             // of the sequences from the longest down, and which they are
+    int seq[SHARE_MAX_N];
+    unsigned long long best[2];
+};
+__device__ __forceinline__ int share_code(int pass, float steps, float limit) {
+    return steps * SHARE_STEP[pass][0] <= limit ? 0 : steps * SHARE_STEP[pass][1] <= limit ? 1 : 2;
+}
+// (all threads; returns the bits that go beside order[t])
+__device__ __forceinline__ int share_device(ShareLds& sh, int N, int H, int V, int t) {
+    if (t < 2) sh.best[t] = ~0ull;
+    __syncthreads();
+    auto limit = [&](int pass, int i) { return sh.steps[i / 3] * SHARE_STEP[pass][i % 3]; };
+    for (int i = t; i < 6 * N; i += TABLE_THREADS) {
+        const int pass = i >= 3 * N, cand = pass ? i - 3 * N : i;
+        const float x = limit(pass, cand);
+        float chain = 0.f, work = 0.f;
+        int groups = 0;
+        for (int j = 0; j < N; ++j) {
+            const int code = share_code(pass, sh.steps[j], x), g = (V / 64) << code;
+            const float time = sh.steps[j] * SHARE_STEP[pass][code];
+            chain = max(chain, time);
+            work += time * (float)g;
+            groups += g;
+        }
+        if (groups <= share_most(H, 1 + pass, N, V)) {
+            const int slots = share_slots(H, 1 + pass);
+            const float cost = groups <= slots ? chain : max(chain, SHARE_PACKING * work / (float)slots);
+            atomicMin(&sh.best[pass], (unsigned long long)__float_as_uint(cost) << 32 | (unsigned)cand);
+        }
+    }
+    __syncthreads();
+    int codes = 0;
+    if (t < N) {
+        codes = share_code(0, sh.steps[t], limit(0, (int)(unsigned)sh.best[0])) << ORDER_OUT;
+        codes |= (int)((unsigned)share_code(1, sh.steps[t], limit(1, (int)(unsigned)sh.best[1])) << ORDER_GRAD);
+    }
+    return codes;
+}
+__global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const int64_t* cu, int N, int T, int nch, int H, int V,
+                                                                          int32_t* chunk_off, int32_t* chunk_seq, int rankers, PackedOut out) {
     constexpr int LONG_SEQ = 64, LONG_LIST = 512;
     __shared__ long long strip[2][TABLE_THREADS];
     __shared__ __attribute__((aligned(16))) int32_t len[ORDER_MAX_N];
@@ -516,7 +566,8 @@ __global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const 
         for (int n = t; n < ORDER_MAX_N; n += TABLE_THREADS) len[n] = n < N ? (int)min(chunks_of(n), (long long)0x7fffffff) : -1;
         __syncthreads();
         const int n = ((int)blockIdx.x - 1) * TABLE_THREADS + t;
-        if (n >= N) return;
+        const bool shared = V > 0 && N > 1 && N <= SHARE_MAX_N;
+        if (n >= N && !shared) return;
         const int mine = len[n];
         int r = 0;
         for (int m = 0; m < N; m += 4) {
@@ -524,7 +575,17 @@ __global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const 
 #pragma unroll
             for (int j = 0; j < 4; ++j) r += (lm[j] > mine || (lm[j] == mine && m + j < n)) ? 1 : 0;
         }
-        order[r] = n;
+        if (!shared) {
+            order[r] = n;
+            return;
+        }
+        __shared__ ShareLds sh;
+        if (n < N) {
+            sh.steps[r] = (float)mine + SHARE_PROLOGUE;
+            sh.seq[r] = n;
+        }
+        const int codes = share_device(sh, N, H, V, t);
+        if (t < N) order[t] = sh.seq[t] | codes;
         return;
     }
     // chunk_off = exclusive prefix sum of the sequences' chunk counts: every thread sums a strip of consecutive
@@ -616,11 +677,11 @@ hipError_t launch_clear_uncovered(const int64_t* cu, int N, int T, const PackedO
     hipLaunchKernelGGL(clear_uncovered_kernel, dim3(clearers), dim3(TABLE_THREADS), 0, stream, cu, N, T, out);
     return hipGetLastError();
 }
-hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int32_t* chunk_off, int32_t* chunk_seq, const PackedOut& out,
-                              hipStream_t stream) {
+hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int H, int V, int32_t* chunk_off, int32_t* chunk_seq,
+                              const PackedOut& out, hipStream_t stream) {
     const int rankers = N <= ORDER_MAX_N ? (N + TABLE_THREADS - 1) / TABLE_THREADS : 0, clearers = clearing_workgroups(N, T, out);
-    hipLaunchKernelGGL(build_chunk_table_kernel, dim3(1 + rankers + clearers), dim3(TABLE_THREADS), 0, stream, cu, N, T, nch, chunk_off, chunk_seq,
-                       rankers, out);
+    hipLaunchKernelGGL(build_chunk_table_kernel, dim3(1 + rankers + clearers), dim3(TABLE_THREADS), 0, stream, cu, N, T, nch, H, V, chunk_off,
+                       chunk_seq, rankers, out);
     return hipGetLastError();
 }
 

@@ -302,6 +302,9 @@ __device__ __forceinline__ void scan_rev_body(const ChunkArgs<bf16>& p, char* sm
     }
 }
 
+template <int K, int V, int NWC> constexpr int grad_lds() {
+    return OutCfg<K, V, NWC, OUT_STATE>::BYTES > RevCfg<K, V, NWC, false>::BYTES ? OutCfg<K, V, NWC, OUT_STATE>::BYTES : RevCfg<K, V, NWC, false>::BYTES;
+}
 // grid = (H, directions * SPLIT, N * segments), as scan_impl.cuh's; blockIdx.y counts from the forward scan's splits on, or (first_dir 1) from
 // the reverse one's
 template <int K, int V, int NWC>
@@ -309,11 +312,29 @@ __global__ __launch_bounds__((RevCfg<K, V, NWC, false>::THREADS)) void scan_grad
     typedef OutCfg<K, V, NWC, OUT_STATE> F;
     typedef RevCfg<K, V, NWC, false> R;
     static_assert(F::THREADS == R::THREADS, "one launch");
-    __shared__ __attribute__((aligned(16))) char smem[F::BYTES > R::BYTES ? F::BYTES : R::BYTES];
+    __shared__ __attribute__((aligned(16))) char smem[grad_lds<K, V, NWC>()];
     const int z = blockIdx.z / p.seg.nseg, seg = blockIdx.z % p.seg.nseg;
     const int n = scan_sequence(p.st, z), y = blockIdx.y + first_dir * R::SPLIT;
     if (y < R::SPLIT) scan_out_body<K, V, NWC, OUT_STATE, true>(p, smem, n, seg, y);
     else scan_rev_body<K, V, NWC, false>(p, smem, n, seg, y - R::SPLIT);
+}
+// packed sequences that share the device by their lengths, as scan_out_share_kernel; the two directions in turn
+template <int K, int V>
+__global__ __launch_bounds__((RevCfg<K, V, 4, false>::THREADS)) void scan_grad_share_kernel(ChunkArgs<bf16> p) {
+    constexpr int B1 = grad_lds<K, V, 1>(), B2 = grad_lds<K, V, 2>(), B4 = grad_lds<K, V, 4>();
+    __shared__ __attribute__((aligned(16))) char smem[B4 > B2 ? (B4 > B1 ? B4 : B1) : B2 > B1 ? B2 : B1];
+    int n, code, split;
+    if (!scan_share<V>(p.st, blockIdx.y >> 1, ORDER_GRAD, n, code, split)) return;
+    const bool rev = blockIdx.y & 1;
+    auto walk = [&](auto nwc) __attribute__((always_inline)) {
+        constexpr int NWC = decltype(nwc)::value;
+        if ((int)threadIdx.x >= RevCfg<K, V, NWC, false>::THREADS) return;
+        if (rev) scan_rev_body<K, V, NWC, false>(p, smem, n, 0, split);
+        else scan_out_body<K, V, NWC, OUT_STATE, true>(p, smem, n, 0, split);
+    };
+    if (code == 0) walk(std::integral_constant<int, 4>());
+    else if (code == 1) walk(std::integral_constant<int, 2>());
+    else walk(std::integral_constant<int, 1>());
 }
 // the segments' records on a workspace of the backward pass (or that it will read): grid and first_y as scan_sum_kernel's
 template <int K, int V, int NWC>
@@ -346,6 +367,11 @@ template <int K, int V> hipError_t launch_scan_grad_shape(const ChunkArgs<bf16>&
     constexpr int VT = V / 16;
     const int lanes = a.H * a.st.N * a.seg.nseg * (kind == SCAN_PAIR ? 2 : 1);
     if (lanes * VT <= SCAN_TARGET_WORKGROUPS) return launch_scan_grad_nwc<K, V, 1>(a, kind, stream);
+    if (kind == SCAN_PAIR && scan_shares(a.st, a.seg.nseg)) {
+        hipLaunchKernelGGL((scan_grad_share_kernel<K, V>), dim3(a.H, 2 * share_most(a.H, 2, a.st.N, V)), dim3(RevCfg<K, V, 4, false>::THREADS), 0,
+                           stream, a);
+        return hipGetLastError();
+    }
     if (lanes * (VT / 2) <= SCAN_TARGET_WORKGROUPS) return launch_scan_grad_nwc<K, V, 2>(a, kind, stream);
     return launch_scan_grad_nwc<K, V, 4>(a, kind, stream);
 }

@@ -595,7 +595,28 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
 // the workgroups of one (sequence, head) are H apart, which puts them on the same XCD (and its L2, where they share the
 // chunk blocks) when H is a multiple of 8, and when the launch has more workgroups than the device holds at once, the long
 // sequences, which decide when the launch ends, start first and the short ones fill in behind them.
-__device__ __forceinline__ int scan_sequence(const SeqTab& st, int z) { return st.cu ? st.order[z] : z; }
+// Where the sequences share the device by their lengths: sequence, width and column blocks of the unit-th workgroup of a head.  False: there are
+// fewer.  The longest sequence's come first.
+template <int V> __device__ __forceinline__ bool scan_share(const SeqTab& st, int unit, int shift, int& n, int& code, int& split) {
+    static_assert(SHARE_MAX_N <= 64, "a lane a sequence");
+    const int l = lane_id();
+    const uint32_t e = l < st.N ? (uint32_t)st.order[l] : 0u;
+    const int own = l < st.N ? (V / 64) << (e >> shift & 3) : 0;
+    int end = own;
+#pragma unroll
+    for (int d = 1; d < SHARE_MAX_N; d <<= 1) {
+        const int x = __shfl_up(end, d);
+        end += l >= d ? x : 0;
+    }
+    const int r = __builtin_popcountll(__ballot(l < st.N && end <= unit));
+    if (r >= st.N) return false;
+    const uint32_t er = __builtin_amdgcn_readlane(e, r);
+    n = (int)(er & ORDER_SEQ);
+    code = (int)(er >> shift & 3);
+    split = unit - __builtin_amdgcn_readlane(end - own, r);
+    return true;
+}
+inline bool scan_shares(const SeqTab& st, int nseg) { return st.cu && st.N > 1 && st.N <= SHARE_MAX_N && nseg == 1; }
 template <typename T, int K, int V, int NWC, bool WRITE_O>
 __global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_fwd_kernel(ChunkArgs<T> p) {
     constexpr ScanOut OUT = WRITE_O ? OUT_O : OUT_STATE;

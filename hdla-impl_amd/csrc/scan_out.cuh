@@ -396,6 +396,24 @@ __global__ __launch_bounds__((OutCfg<K, V, NWC, OUT_O>::THREADS)) void scan_out_
     const int z = blockIdx.z / p.seg.nseg, seg = blockIdx.z % p.seg.nseg;
     scan_out_body<K, V, NWC, OUT_O, KEPT>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
 }
+// Packed sequences that share the device by their lengths (see share_device, prep.hip): grid = (H, workgroups of a head).  Waves that a narrow
+// workgroup has no use for end at once; barriers are among those that are left.  Measured, us, one width for all -> this, K = V = 128, 16 heads: forward
+// pass of 1731 + 37 + 2204 + 1031 tokens 136 -> 131 (the scan 81 -> 72), of 9000 in 6 sequences, the longest 3700, 298 -> 262, of 6000 in 12 of
+// similar lengths 137.7 -> 138.0; 12000 in 12, 8 heads 209 -> 186; training steps of 6000 in 6 748 -> 683, of 1500 in 7, 12 heads 174 -> 153, of
+// 16384 in 4 1726 -> 1705 (its two scans are at their traffic, 2.2 GB in 520 us, in every width).  Where one block a workgroup for all fits the device,
+// that is faster still and stays.  Beyond 32 sequences the device is full with the widest workgroups for all but the last few steps.
+template <int K, int V, bool KEPT>
+__global__ __launch_bounds__((OutCfg<K, V, 4, OUT_O>::THREADS)) void scan_out_share_kernel(ChunkArgs<bf16> p) {
+    typedef OutCfg<K, V, 4, OUT_O> C4;
+    typedef OutCfg<K, V, 2, OUT_O> C2;
+    typedef OutCfg<K, V, 1, OUT_O> C1;
+    __shared__ __attribute__((aligned(16))) char smem[C4::BYTES > C2::BYTES ? (C4::BYTES > C1::BYTES ? C4::BYTES : C1::BYTES) : C2::BYTES > C1::BYTES ? C2::BYTES : C1::BYTES];
+    int n, code, split;
+    if (!scan_share<V>(p.st, blockIdx.y, ORDER_OUT, n, code, split)) return;
+    if (code == 0) scan_out_body<K, V, 4, OUT_O, KEPT>(p, smem, n, 0, split);
+    else if (code == 1) { if ((int)threadIdx.x < C2::THREADS) scan_out_body<K, V, 2, OUT_O, KEPT>(p, smem, n, 0, split); }
+    else if ((int)threadIdx.x < C1::THREADS) scan_out_body<K, V, 1, OUT_O, KEPT>(p, smem, n, 0, split);
+}
 // the segments' records in the forward direction: grid = (H, (V + K) / 16 / NWC, N * (segments - 1))
 template <int K, int V, int NWC>
 __global__ __launch_bounds__((OutCfg<K, V, NWC, OUT_SUM>::THREADS)) void scan_out_sum_kernel(ChunkArgs<bf16> p) {
@@ -420,6 +438,12 @@ template <int K, int V> hipError_t launch_scan_out_shape(const ChunkArgs<bf16>& 
     constexpr int VT = V / 16;
     const int lanes = a.H * a.st.N * a.seg.nseg;
     if (lanes * VT <= SCAN_TARGET_WORKGROUPS) return launch_scan_out_nwc<K, V, 1>(a, kept, stream);
+    if (scan_shares(a.st, a.seg.nseg)) {
+        const dim3 grid(a.H, share_most(a.H, 1, a.st.N, V)), block(OutCfg<K, V, 4, OUT_O>::THREADS);
+        if (kept) hipLaunchKernelGGL((scan_out_share_kernel<K, V, true>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((scan_out_share_kernel<K, V, false>), grid, block, 0, stream, a);
+        return hipGetLastError();
+    }
     if (lanes * (VT / 2) <= SCAN_TARGET_WORKGROUPS) return launch_scan_out_nwc<K, V, 2>(a, kept, stream);
     return launch_scan_out_nwc<K, V, 4>(a, kept, stream);
 }
