@@ -454,7 +454,7 @@ template <int SRC> __device__ __forceinline__ f32x4 bcast16(f32x4 x) {
     f32x4 r;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-        r[i] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x[i]), 0x150 + SRC, 0xf, 0xf, false));
+        r[i] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x[i]), 0x150 + SRC, 0xf, 0xf, true));
     return r;
 }
 // value held by the lane 32 positions away (v_permlane32_swap exchanges the two halves of the wave)
@@ -547,6 +547,10 @@ template <> struct TileDecay<bf16> {
         ea = prev_token(eq, em);
         egi = eq * bcast16<1>(em);
         edn = ek * bcast16<CH - 1>(eq);
+        if (check) {                                      // formed here, where the lane moves are part of the products, and not behind the branch
+            pin(egi);
+            pin(edn);
+        }
         if (strong) {
             egi = exp2_4(gi);
             edn = exp2_4(bcast16<CH - 1>(gi) - gi);
