@@ -72,10 +72,53 @@ template <typename T, bool GKF32, int K, int V, bool HD> constexpr int cg_waves(
     return small ? 3 : 2;
 }
 
-// The common kernel: one workgroup per (chunk, head); pairs flagged for the strong-decay route are left alone.
 template <typename T, bool GKF32, int K, int V, bool HD>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(cg_waves<T, GKF32, K, V, HD>(false), cg_waves<T, GKF32, K, V, HD>(true)))) void chunk_grad_kernel(ChunkArgs<T> p) {
+__device__ __forceinline__ void chunk_grad_strong_pair(const ChunkArgs<T>& p, int cid, int h, char* smem) {
+#define CG_STRONG 1
+#include "chunk_grad_body.inc"
+#undef CG_STRONG
+}
+
+// The common pairs, one workgroup per (chunk, head), which leave the flagged ones alone; and behind them, or in a launch of their own, what looks for
+// the flagged pairs and works them off.  They are rare (a channel must lose more than e^-70 within eight tokens), so this is a small number of
+// workgroups that each look through their share of the flags (one read per thread and round) and work off what they find one pair after the other.
+// CG_ALL: one launch, where the three passes of a flagged pair do with the registers that the common pairs' occupancy leaves a wave (4-byte elements).
+// CG_COMMON and CG_FLAGGED: elsewhere (up to 138 registers too many) the flagged pairs have all registers of a wave per SIMD, the common ones, at the
+// limit of their occupancy, pay nothing for them, and when nothing is flagged, which is the rule, their launch costs its start-up and one round of flag
+// reads, 4 to 5 us.  fp32, training step of 2 x 1003 tokens, 8 heads, K = V = 64, two launches -> one: 185.6 -> 181.5 us;
+// 838 tokens, 12 heads, K = V = 128 382 -> 377; beta form, 900 tokens, 8 heads 141.6 -> 138.6; 2 x 2000 tokens, 16 heads 547 both.
+enum CgPairs { CG_COMMON, CG_FLAGGED, CG_ALL };
+constexpr int CG_STRONG_GRID = 256;
+template <typename T, bool GKF32, int K, int V, bool HD, CgPairs WHAT>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WHAT == CG_FLAGGED ? 1 : cg_waves<T, GKF32, K, V, HD>(false),
+                                                                         WHAT == CG_FLAGGED ? 1 : cg_waves<T, GKF32, K, V, HD>(true))))
+void chunk_grad_kernel(ChunkArgs<T> p) {
     __shared__ __attribute__((aligned(16))) char smem[CgLds<T, K, V>::BYTES];
+    const int total = p.H * p.st.nch;
+    if (WHAT != CG_COMMON && (WHAT == CG_FLAGGED || (int)blockIdx.x >= total)) {
+        __shared__ unsigned long long sMask[NW];
+        constexpr int nth = 64 * NW;
+        const int group = (int)blockIdx.x - (WHAT == CG_ALL ? total : 0), groups = (int)gridDim.x - (WHAT == CG_ALL ? total : 0);
+        const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        for (int base = group; base < total; base += groups * nth) {               // uniform over the workgroup
+            const int mine = base + (int)threadIdx.x * groups;
+            const unsigned long long m = __ballot(mine < total && p.ws.STRONG[mine] != 0);
+            if (lane_id() == 0) sMask[w] = m;
+            __syncthreads();
+            for (int ww = 0; ww < NW; ++ww) {
+                unsigned long long todo = sMask[ww];                               // uniform: the same word for all
+                while (todo) {
+                    const int t = 64 * ww + __builtin_ctzll(todo);
+                    todo &= todo - 1;
+                    const int chw = base + t * groups;
+                    chunk_grad_strong_pair<T, GKF32, K, V, HD>(p, chw % p.st.nch, chw / p.st.nch, smem);
+                    __syncthreads();                                               // the next pair reuses the staging areas
+                }
+            }
+            __syncthreads();
+        }
+        return;
+    }
     // Which of the two indices runs fastest over the workgroups decides which rows of the [token][head][channel]
     // tensors the workgroups resident at one time touch.  Measured: with rows of 4 KiB and more, neighbouring
     // workgroups should be the heads of one chunk (together they read whole rows; chunk-fastest, all of them would
@@ -90,57 +133,20 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(cg_wave
 }
 
 template <typename T, bool GKF32, int K, int V, bool HD>
-__device__ __forceinline__ void chunk_grad_strong_pair(const ChunkArgs<T>& p, int cid, int h, char* smem) {
-#define CG_STRONG 1
-#include "chunk_grad_body.inc"
-#undef CG_STRONG
-}
-
-// The kernel for the flagged pairs.  They are rare (a channel must lose more than e^-70 within eight tokens), so this
-// is a small fixed grid whose workgroups each look through their share of the flags (one read per thread and round)
-// and work off what they find one pair after the other, at one wave per SIMD with all the registers the three passes
-// want; when nothing is flagged, which is the rule, the launch costs its start-up and one round of flag reads.  The
-// common kernel sits at the register limit of three workgroups per compute unit and pays nothing for this one.
-constexpr int CG_STRONG_GRID = 256;
-template <typename T, bool GKF32, int K, int V, bool HD>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1))) void chunk_grad_strong_kernel(ChunkArgs<T> p) {
-    __shared__ __attribute__((aligned(16))) char smem[CgLds<T, K, V>::BYTES];
-    __shared__ unsigned long long sMask[NW];
-    const int total = p.H * p.st.nch, nth = 64 * NW;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    for (int base = blockIdx.x; base < total; base += (int)gridDim.x * nth) {      // uniform over the workgroup
-        const int mine = base + (int)threadIdx.x * (int)gridDim.x;
-        const unsigned long long m = __ballot(mine < total && p.ws.STRONG[mine] != 0);
-        if (lane_id() == 0) sMask[w] = m;
-        __syncthreads();
-        for (int ww = 0; ww < NW; ++ww) {
-            unsigned long long todo = sMask[ww];                                   // uniform: the same word for all
-            while (todo) {
-                const int t = 64 * ww + __builtin_ctzll(todo);
-                todo &= todo - 1;
-                const int chw = base + t * (int)gridDim.x;
-                chunk_grad_strong_pair<T, GKF32, K, V, HD>(p, chw % p.st.nch, chw / p.st.nch, smem);
-                __syncthreads();                                                   // the next pair reuses the staging areas
-            }
-        }
-        __syncthreads();
-    }
-}
-
-template <typename T, int K, int V, bool HD>
-static hipError_t launch_chunk_grad_kv(const ChunkArgs<T>& a, hipStream_t stream) {
-    dim3 grid(a.st.nch * a.H), block(64 * NW);
-    constexpr bool kAlwaysF32 = sizeof(T) == 4;
-    const int total = a.st.nch * a.H;
-    dim3 sgrid(total < CG_STRONG_GRID ? total : CG_STRONG_GRID);
-    if (kAlwaysF32 || a.gk_f32) {
-        hipLaunchKernelGGL((chunk_grad_kernel<T, true, K, V, HD>), grid, block, 0, stream, a);
-        hipLaunchKernelGGL((chunk_grad_strong_kernel<T, true, K, V, HD>), sgrid, block, 0, stream, a);
+static hipError_t launch_chunk_grad_gk(const ChunkArgs<T>& a, hipStream_t stream) {
+    const int total = a.st.nch * a.H, strong = total < CG_STRONG_GRID ? total : CG_STRONG_GRID;
+    if constexpr (sizeof(T) == 4) {
+        hipLaunchKernelGGL((chunk_grad_kernel<T, GKF32, K, V, HD, CG_ALL>), dim3(total + strong), dim3(64 * NW), 0, stream, a);
     } else {
-        hipLaunchKernelGGL((chunk_grad_kernel<T, kAlwaysF32, K, V, HD>), grid, block, 0, stream, a);
-        hipLaunchKernelGGL((chunk_grad_strong_kernel<T, kAlwaysF32, K, V, HD>), sgrid, block, 0, stream, a);
+        hipLaunchKernelGGL((chunk_grad_kernel<T, GKF32, K, V, HD, CG_COMMON>), dim3(total), dim3(64 * NW), 0, stream, a);
+        hipLaunchKernelGGL((chunk_grad_kernel<T, GKF32, K, V, HD, CG_FLAGGED>), dim3(strong), dim3(64 * NW), 0, stream, a);
     }
     return hipGetLastError();
+}
+template <typename T, int K, int V, bool HD>
+static hipError_t launch_chunk_grad_kv(const ChunkArgs<T>& a, hipStream_t stream) {
+    constexpr bool kAlwaysF32 = sizeof(T) == 4;
+    return kAlwaysF32 || a.gk_f32 ? launch_chunk_grad_gk<T, true, K, V, HD>(a, stream) : launch_chunk_grad_gk<T, kAlwaysF32, K, V, HD>(a, stream);
 }
 
 template <typename T, bool HD>
