@@ -46,6 +46,7 @@ struct Api {
     HDLA_FN(recurrent_fwd); HDLA_FN(param_recurrent_fwd); HDLA_FN(normalize_fwd); HDLA_FN(normalize_bwd);
     HDLA_FN(normalize_workspace_bytes); HDLA_FN(layer_pre_fwd); HDLA_FN(layer_pre_bwd); HDLA_FN(layer_up_fwd); HDLA_FN(layer_down);
     HDLA_FN(layer_up_wgrad); HDLA_FN(layer_up_wgrad_workspace_bytes); HDLA_FN(rows_gemm); HDLA_FN(sum_partials); HDLA_FN(stack_rows);
+    HDLA_FN(weight_grad); HDLA_FN(weight_grad_workspace_bytes);
     HDLA_FN(layer_step); HDLA_FN(rows_gemm_norm);
 #undef HDLA_FN
 } api;
@@ -725,10 +726,21 @@ void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, Plan& p
     r.out = project(r.n, P[9]).view({B, T, d});
 }
 
-// dW [n, k] = dY [rows, n]^T X [rows, k].  An output of few tiles would leave most of the chip idle (1024 x 1024 over 8192
-// rows: 54 us): the rows are split over a batch of products whose fp32 results one kernel adds (28 + 4 us).
+// dW [n, k] = dY [rows, n]^T X [rows, k].  Up to one round of whole 128 x 128 tiles on the device by the library's own kernel (us
+// within a training step: 8192 rows, 3328 x 1024 102 -> 82, 1024 x 1024 33 -> 30; 4000 rows, 2048 x 2048 56 -> 44; 1500 rows, 3328 x 1024 30 -> 17; but
+// 4000 rows, 6656 x 2048, 832 tiles: 128 and 147).  Others: an output of few tiles would leave most of the chip idle (1024 x 1024 over 8192 rows: 54 us), so the rows are split over a batch
+// of products whose fp32 results one kernel adds (28 + 4 us).
 Tensor weight_grad(const Tensor& dy, const Tensor& x) {
     const int64_t rows = dy.size(0), n = dy.size(1), k = x.size(1);
+    if (rows > 0 && rows <= 0x7fff0000 && n > 0 && k > 0 && n % 128 == 0 && k % 128 == 0 && n / 128 * (k / 128) <= 256 && dy.stride(1) == 1 &&
+        x.stride(1) == 1 && dy.stride(0) >= n && x.stride(0) >= k && dy.stride(0) % 8 == 0 && x.stride(0) % 8 == 0 && !off_grid(dy) && !off_grid(x)) {
+        const Tensor dw = at::empty({n, k}, dy.options());
+        const size_t nws = api.weight_grad_workspace_bytes(rows, (int32_t)n, (int32_t)k);
+        const Tensor ws = nws ? bytes_like(x, nws) : Tensor();
+        check(api.weight_grad(rows, (int32_t)n, (int32_t)k, ptr(dy), dy.stride(0), ptr(x), x.stride(0), ptr(dw), ptr(ws), nws, stream_of(dy)),
+              "hdla_weight_grad");
+        return dw;
+    }
     const int64_t tiles = ((n + 127) / 128) * ((k + 127) / 128);
     int64_t S = 1;
     while (S < 8 && tiles * S * 2 <= 256 && rows % (S * 2) == 0 && rows / (S * 2) >= 1024) S *= 2;
@@ -1041,6 +1053,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HDLA_FN(recurrent_fwd) HDLA_FN(param_recurrent_fwd) HDLA_FN(normalize_fwd) HDLA_FN(normalize_bwd)
     HDLA_FN(normalize_workspace_bytes) HDLA_FN(layer_pre_fwd) HDLA_FN(layer_pre_bwd) HDLA_FN(layer_up_fwd) HDLA_FN(layer_down)
     HDLA_FN(layer_up_wgrad) HDLA_FN(layer_up_wgrad_workspace_bytes) HDLA_FN(rows_gemm) HDLA_FN(sum_partials) HDLA_FN(stack_rows) HDLA_FN(layer_step)
+    HDLA_FN(weight_grad) HDLA_FN(weight_grad_workspace_bytes)
     HDLA_FN(rows_gemm_norm)
 #undef HDLA_FN
     Py_INCREF(a[1]);

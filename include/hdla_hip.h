@@ -322,6 +322,12 @@ size_t hdla_skinny_wgrad_workspace_bytes(int dtype, int64_t M, int32_t N, int32_
 /* out [n] (bf16) = sum of `count` consecutive fp32 partial results part [count][n], added in order; n a multiple of 8,
  * both 16-byte aligned: the second half of a product whose contraction was split. */
 int hdla_sum_partials(const float* part, int32_t count, int64_t n, void* out, void* stream);
+/* dW [N, K] = dY [M, N]^T X [M, K], bf16, rows of dY and X ldy and ldx elements apart (multiples of 8), dW contiguous, all 16-byte aligned; N and K multiples
+ * of 128, M >= 1.  Where the result has few tiles the rows are shared out and the fp32 partial results, in `workspace`
+ * (hdla_weight_grad_workspace_bytes() bytes, 16-byte aligned), are added in a fixed order. */
+size_t hdla_weight_grad_workspace_bytes(int64_t M, int32_t N, int32_t K);
+int hdla_weight_grad(int64_t M, int32_t N, int32_t K, const void* dY, int64_t ldy, const void* X, int64_t ldx, void* dW, void* workspace,
+                     size_t workspace_bytes, void* stream);
 /* out [total_rows, width] (2-byte elements) = the rows of parts[0 .. count) one part behind the other, parts[m] being [rows[m], width],
  * then zeros; count <= 8, width a multiple of 8, everything contiguous and 16-byte aligned.  parts and rows are host arrays. */
 int hdla_stack_rows(const void* const* parts, const int64_t* rows, int32_t count, int64_t width, void* out, int64_t total_rows, void* stream);
