@@ -2,6 +2,7 @@
 that a backward pass on it is the one that recomputes: whole sequences bit for bit, in time segments, whose reverse chain takes the forward
 pass's transitions turned, within the rounding of the element type."""
 import ctypes
+import time
 
 import pytest
 import torch
@@ -112,15 +113,22 @@ def test_it_is_kept_and_given_back(native, monkeypatch):
     x, do = [t.to(DEV).requires_grad_() for t in x], do.to(DEV)
     run = lambda keep=None: chunk_hrdplr_delta_rule(*x[:-1], 2, scale=0.7, initial_state=x[-1], keep_forward=keep)[0]
 
+    def becomes(want, what):                                    # (the engine's thread lets go of its last tensors a moment after the call has returned)
+        for _ in range(1000):
+            if what() == want:
+                return True
+            time.sleep(1e-3)
+        return False
+
     def held(keep=None):
         torch.cuda.synchronize()
         at = torch.cuda.memory_allocated()
         o = run(keep)
         n = torch.cuda.memory_allocated() - at - o.numel() * 2
         torch.autograd.grad(o, x, do, retain_graph=True)
-        assert torch.cuda.memory_allocated() - at - o.numel() * 2 == n
+        assert becomes(n, lambda: torch.cuda.memory_allocated() - at - o.numel() * 2)
         del o
-        assert torch.cuda.memory_allocated() == at
+        assert becomes(at, torch.cuda.memory_allocated)
         return n
 
     want = _plan(400, 4)[0]
