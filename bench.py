@@ -176,21 +176,22 @@ def measured_traffic(workload, kernel_key, K, V):
             if fused_mode is not None and k.startswith("fused_kernel<") and targs[2:] == [str(K), str(V), fused_mode, "false"]:
                 return rec["hbm_bytes_per_launch"]
             continue
-        # scan_out<K, V, NWC, KEPT> (the forward pass's scan), scan_grad<K, V, NWC> (both of the backward pass)
+        # scan_out<K, V, NWC, KEPT> (the forward pass's scan), scan_grad<K, V, NWC> (both of the backward pass); of packed sequences that share
+        # the device by their lengths scan_out_share<K, V, KEPT> and scan_grad_share<K, V>
         if name in ("scan_fwd", "scan_pair"):
-            if k.startswith("scan_out_kernel<" if name == "scan_fwd" else "scan_grad_kernel<") and targs[:2] == [str(K), str(V)] and \
-                    targs[3:] != ["true"]:
+            if k.startswith(("scan_out_kernel<", "scan_out_share_kernel<") if name == "scan_fwd" else ("scan_grad_kernel<", "scan_grad_share_kernel<")) and \
+                    targs[:2] == [str(K), str(V)] and targs[-1] != "true":
                 return rec["hbm_bytes_per_launch"]
             continue
         if not k.startswith(name + "_kernel<"):
             continue
-        # prep<T, GKF32, K, V, MODE (0 forward, 1 backward, 2 kept forward), HD>, chunk_grad<T, GKF32, K, V, HD>, recurrent<T, K, V, BV, HD>
+        # prep<T, GKF32, K, V, MODE (0 forward, 1 backward, 2 kept forward), HD>, chunk_grad<T, GKF32, K, V, HD, pairs (0 the common ones)>, recurrent<T, K, V, BV, HD>
         kv = targs[2:4] if name in ("prep", "chunk_grad") else targs[1:3]
         if kv != [str(K), str(V)]:
             continue
         if name == "prep" and (targs[4] != ("1" if pass_ == "bwd" else "0") or targs[5:] == ["true"]):
             continue
-        if name in ("chunk_grad", "recurrent") and targs[4:] == ["true"]:
+        if name in ("chunk_grad", "recurrent") and (targs[4:5] == ["true"] or targs[5:6] not in ([], ["0"], ["(hdla::CgPairs)0"])):
             continue
         return rec["hbm_bytes_per_launch"]
     return None
