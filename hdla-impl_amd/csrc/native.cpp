@@ -43,7 +43,7 @@ struct Api {
 #define HDLA_FN(name) decltype(&hdla_##name) name
     HDLA_FN(strerror); HDLA_FN(workspace_bytes); HDLA_FN(record_bytes); HDLA_FN(record_workspace_bytes); HDLA_FN(chunk_fwd_b); HDLA_FN(chunk_bwd_b);
     HDLA_FN(keep_plan); HDLA_FN(chunk_fwd_keep); HDLA_FN(chunk_bwd_kept);
-    HDLA_FN(recurrent_fwd); HDLA_FN(param_recurrent_fwd); HDLA_FN(normalize_fwd); HDLA_FN(normalize_bwd);
+    HDLA_FN(recurrent_fwd); HDLA_FN(param_recurrent_fwd); HDLA_FN(normalize_fwd); HDLA_FN(normalize_bwd_as);
     HDLA_FN(normalize_workspace_bytes); HDLA_FN(layer_pre_fwd); HDLA_FN(layer_pre_bwd); HDLA_FN(layer_up_fwd); HDLA_FN(layer_down);
     HDLA_FN(layer_up_wgrad); HDLA_FN(layer_up_wgrad_workspace_bytes); HDLA_FN(rows_gemm); HDLA_FN(sum_partials); HDLA_FN(stack_rows);
     HDLA_FN(weight_grad); HDLA_FN(weight_grad_workspace_bytes);
@@ -505,13 +505,12 @@ struct NormFn : torch::autograd::Function<NormFn> {
         if (gate.defined()) dgate = at::empty_like(x);
         size_t nws = 0;
         if (w.defined()) {
-            dw = at::empty({x.size(-1)}, x.options().dtype(at::kFloat));
+            dw = at::empty(w.sizes(), w.options());
             nws = api.normalize_workspace_bytes(&d);
             ws = bytes_like(x, nws < 16 ? 16 : nws);
         }
-        check(api.normalize_bwd(&d, ptr(x), ptr(w), ptr(gate), ptr(d_o), ptr(dx), ptr(dgate), fptr(dw), ptr(ws), nws, stream_of(x)),
-              "hdla_normalize_bwd");
-        if (dw.defined()) dw = dw.to(w.scalar_type()).reshape(w.sizes());
+        check(api.normalize_bwd_as(&d, ptr(x), ptr(w), ptr(gate), ptr(d_o), ptr(dx), ptr(dgate), ptr(dw), ptr(ws), nws, stream_of(x)),
+              "hdla_normalize_bwd_as");
         return {dx, dw, dgate, Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };
@@ -793,15 +792,15 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
         if (need(10)) out[10] = weight_grad(dout, n);
         const Tensor dn = at::mm(dout, wo);
         const Tensor o2 = o.view({rows, d}), d_o = at::empty({rows, d}, opt), dgate = at::empty({rows, d}, opt);
-        Tensor dwn = at::empty({d}, opt.dtype(at::kFloat));
+        const Tensor dwn = at::empty(wnorm.sizes(), wnorm.options());
         {
             const hdla_norm_dims nd = norm_dims(o2, wnorm, cfg.gate_pos, cfg.c, cfg.eps, cfg.groups);
             const size_t nws = api.normalize_workspace_bytes(&nd);
             const Tensor ws = bytes_like(x, nws < 16 ? 16 : nws);
-            check(api.normalize_bwd(&nd, ptr(o2), ptr(wnorm), ptr(g), ptr(dn), ptr(d_o), ptr(dgate), fptr(dwn), ptr(ws), nws, stream),
-                  "hdla_normalize_bwd");
+            check(api.normalize_bwd_as(&nd, ptr(o2), ptr(wnorm), ptr(g), ptr(dn), ptr(d_o), ptr(dgate), ptr(dwn), ptr(ws), nws, stream),
+                  "hdla_normalize_bwd_as");
         }
-        if (need(9)) out[9] = dwn.to(wnorm.scalar_type()).view(wnorm.sizes());
+        if (need(9)) out[9] = dwn;
 
         // the operator
         Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), dbeta = at::empty_like(beta), dgk = at::empty_like(gk), dh0;
@@ -1050,7 +1049,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     HDLA_FN(strerror) HDLA_FN(workspace_bytes) HDLA_FN(record_bytes) HDLA_FN(record_workspace_bytes) HDLA_FN(chunk_fwd_b) HDLA_FN(chunk_bwd_b)
     HDLA_FN(keep_plan) HDLA_FN(chunk_fwd_keep) HDLA_FN(chunk_bwd_kept)
-    HDLA_FN(recurrent_fwd) HDLA_FN(param_recurrent_fwd) HDLA_FN(normalize_fwd) HDLA_FN(normalize_bwd)
+    HDLA_FN(recurrent_fwd) HDLA_FN(param_recurrent_fwd) HDLA_FN(normalize_fwd) HDLA_FN(normalize_bwd_as)
     HDLA_FN(normalize_workspace_bytes) HDLA_FN(layer_pre_fwd) HDLA_FN(layer_pre_bwd) HDLA_FN(layer_up_fwd) HDLA_FN(layer_down)
     HDLA_FN(layer_up_wgrad) HDLA_FN(layer_up_wgrad_workspace_bytes) HDLA_FN(rows_gemm) HDLA_FN(sum_partials) HDLA_FN(stack_rows) HDLA_FN(layer_step)
     HDLA_FN(weight_grad) HDLA_FN(weight_grad_workspace_bytes)

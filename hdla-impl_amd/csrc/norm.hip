@@ -357,8 +357,10 @@ __global__ __launch_bounds__(256) void normalize_bwd_kernel(NormArgs p) {
 }
 
 // dw[g*E + e] = sum of the partial rows idx = g, g + G, g + 2G, ... ; one workgroup per 16 columns: 4 lanes of four
-// columns each, 64 row phases, summed through LDS in a fixed order.
-__global__ __launch_bounds__(256) void normalize_dw_kernel(const float* __restrict__ partial, float* __restrict__ dw,
+// columns each, 64 row phases, summed through LDS in a fixed order.  dw in 32 bits or (O: bf16) in the weight's own 16, rounded once (as a launch of its
+// own that was 4.8 us of a training step of the layer).
+template <typename O>
+__global__ __launch_bounds__(256) void normalize_dw_kernel(const float* __restrict__ partial, O* __restrict__ dw,
                                                            long long nrow, int G, int E) {
     __shared__ f32x4 red[64][4];
     const int cq = threadIdx.x & 3, rl = threadIdx.x >> 2;
@@ -377,7 +379,8 @@ __global__ __launch_bounds__(256) void normalize_dw_kernel(const float* __restri
         f32x4 s = red[0][cq];
 #pragma unroll
         for (int r = 1; r < 64; ++r) s += red[r][cq];
-        *reinterpret_cast<f32x4*>(dw + col) = s;
+        if constexpr (sizeof(O) == 4) *reinterpret_cast<f32x4*>(dw + col) = s;
+        else st_frag(dw + col, to_frag<bf16>(s));
     }
 }
 
@@ -488,9 +491,8 @@ extern "C" int hdla_normalize_fwd(const hdla_norm_dims* dims, const void* x, con
     return e == hipSuccess ? HDLA_OK : (int)e;
 }
 
-extern "C" int hdla_normalize_bwd(const hdla_norm_dims* dims, const void* x, const void* weight, const void* gate,
-                                  const void* d_o, void* dx, void* dgate, float* dw, void* workspace,
-                                  size_t workspace_bytes, void* stream) {
+static int normalize_bwd(const hdla_norm_dims* dims, const void* x, const void* weight, const void* gate, const void* d_o, void* dx, void* dgate, void* dw,
+                         bool dw_f32, void* workspace, size_t workspace_bytes, void* stream) {
     NormCfg c;
     const int rc = norm_config(dims, true, c);
     if (rc) return rc;
@@ -510,10 +512,21 @@ extern "C" int hdla_normalize_bwd(const hdla_norm_dims* dims, const void* x, con
     }
     if (weight) {
         const long long D = (long long)dims->G * dims->E;
-        hipLaunchKernelGGL(normalize_dw_kernel, dim3((unsigned)((D + 15) / 16)), dim3(256), 0, s, a.partial, dw,
-                           dims->rows > 0 ? c.partial_rows() : 0LL, dims->G, dims->E);
+        const dim3 grid((unsigned)((D + 15) / 16));
+        const long long rows = dims->rows > 0 ? c.partial_rows() : 0LL;
+        if (dw_f32) hipLaunchKernelGGL((normalize_dw_kernel<float>), grid, dim3(256), 0, s, a.partial, static_cast<float*>(dw), rows, dims->G, dims->E);
+        else hipLaunchKernelGGL((normalize_dw_kernel<bf16>), grid, dim3(256), 0, s, a.partial, static_cast<bf16*>(dw), rows, dims->G, dims->E);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return (int)e;
     }
     return HDLA_OK;
+}
+extern "C" int hdla_normalize_bwd(const hdla_norm_dims* dims, const void* x, const void* weight, const void* gate,
+                                  const void* d_o, void* dx, void* dgate, float* dw, void* workspace,
+                                  size_t workspace_bytes, void* stream) {
+    return normalize_bwd(dims, x, weight, gate, d_o, dx, dgate, dw, true, workspace, workspace_bytes, stream);
+}
+extern "C" int hdla_normalize_bwd_as(const hdla_norm_dims* dims, const void* x, const void* weight, const void* gate, const void* d_o, void* dx,
+                                     void* dgate, void* dw, void* workspace, size_t workspace_bytes, void* stream) {
+    return normalize_bwd(dims, x, weight, gate, d_o, dx, dgate, dw, !dims || dims->weight_dtype == HDLA_FP32, workspace, workspace_bytes, stream);
 }

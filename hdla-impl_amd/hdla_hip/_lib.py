@@ -126,6 +126,8 @@ def load():
     lib.hdla_normalize_fwd.argtypes = [NF] + [P] * 5
     lib.hdla_normalize_bwd.restype = ctypes.c_int
     lib.hdla_normalize_bwd.argtypes = [NF] + [P] * 8 + [ctypes.c_size_t, P]
+    lib.hdla_normalize_bwd_as.restype = ctypes.c_int
+    lib.hdla_normalize_bwd_as.argtypes = [NF] + [P] * 8 + [ctypes.c_size_t, P]
     PF = ctypes.POINTER(HdlaPreDims)
     lib.hdla_layer_pre_fwd.restype = ctypes.c_int
     lib.hdla_layer_pre_fwd.argtypes = [PF] + [P] * 6

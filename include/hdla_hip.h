@@ -282,6 +282,9 @@ int hdla_normalize_fwd(const hdla_norm_dims* dims, const void* x, const void* we
 int hdla_normalize_bwd(const hdla_norm_dims* dims, const void* x, const void* weight, const void* gate,
                        const void* d_o, void* dx, void* dgate, float* dw, void* workspace, size_t workspace_bytes,
                        void* stream);
+/* The same with dw [G*E] in the weight's type, rounded once. */
+int hdla_normalize_bwd_as(const hdla_norm_dims* dims, const void* x, const void* weight, const void* gate, const void* d_o, void* dx, void* dgate,
+                          void* dw, void* workspace, size_t workspace_bytes, void* stream);
 size_t hdla_normalize_workspace_bytes(const hdla_norm_dims* dims);
 
 /* What the HDLA layer does between its projections and the operator, one pass per direction
