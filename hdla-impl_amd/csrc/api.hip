@@ -153,30 +153,19 @@ int kept_segments(const hdla_dims* d) { return d->segments > 0 ? scan_segments(d
 // a training step that keeps the inputs -> this: 1 x 256 tokens, 2 heads, K = V = 64 43 -> 37; 2 x 1537 tokens, 8 heads, K = V = 128 214 -> 185;
 // 4 x 1000 tokens, 16 heads 430 -> 393; 4 x 500, 8 heads 127 -> 107; fp32, 2 x 1003 tokens, 8 heads, K = V = 64 227 -> 190.
 constexpr size_t KEEP_MOST = (size_t)256 << 20;
-// Segments of the two passes of such a call (return, bwd).  The backward pass takes the forward one's, whose entering states and transitions are there,
-// or none.  2-byte elements: by the time of both; over passes of 16 to 313 chunks and 1 to 32 lanes, K, V in {64, 128}, 143 shapes in 1 to 32 segments,
-// 0.3 % over the best on average, 6 % at the most (each pass's own choice: 1.0 and 12 %).  4-byte elements: as scan_segments; at K = 128 four segments
-// from eight chunks on (us, 16 lanes of 8 chunks 166 -> 140).
+// Segments of the two passes of such a call (return, bwd).  The forward pass has those it has without gradients, and so the same bits (what recomputes a
+// part of a model runs one pass without and one with them); the backward pass takes these, whose entering states and transitions are there,
+// or, with 2-byte elements, none where that is the sooner by more than the times above are off by.  us, a training step in one segment -> in four forward and
+// one backward -> four -> eight in both passes (* the choice), K = V = 128: 16 lanes of 200 chunks 402 -> 392 -> 384* -> 386, 16 of 313 654 -> 608 ->
+// 571* -> 560, 12 of 128 207 -> 204 -> 217* -> 219; 16 of 97 in one, four, eight 182* -> 211 -> 214.  (Eight in both for the second, and for 4-byte elements at K = 128 four from
+// 8 chunks on, 166 -> 137 for 16 lanes of 8, would need a forward pass in other segments than without gradients.)
 int kept_plan_segments(const hdla_dims* d, int32_t& bwd) {
-    bwd = 1;
-    if (d->route != HDLA_ROUTE_AUTO) return 1;
-    if (d->segments > 0) return bwd = scan_segments(d, false);
-    const long long lanes = (long long)d->N * d->H, chunks = average_chunks(d), longest = longest_chunks(d);
-    if (d->in_dtype == HDLA_FP32) {
-        const int n = scan_segments(d, false);
-        return bwd = n == 1 && d->K == 128 && chunks >= 8 && lanes <= 32 ? 4 : n;
-    }
-    if (fused_shape(d)) return 1;
-    int fwd = 1;
-    double best = 0;
-    for (int n = 1; n == 1 || (n <= SCAN_MAX_SEGMENTS && lanes * n <= SCAN_TIME_BWD_KEPT.most); n = n == 1 ? 4 : 2 * n) {
-        const double f = scan_time(SCAN_TIME_FWD, d, (double)lanes, chunks, longest, n);
-        for (int b = 1;; b = n) {
-            const double x = f + scan_time(SCAN_TIME_BWD_KEPT, d, (double)lanes, chunks, longest, b);
-            if ((n == 1 && b == 1) || x < best) { best = x; fwd = n; bwd = b; }
-            if (b == n) break;
-        }
-    }
+    const int fwd = bwd = scan_segments(d, false);
+    if (fwd == 1 || d->segments > 0 || d->in_dtype == HDLA_FP32) return fwd;
+    const double lanes = (double)d->N * d->H;
+    const long long chunks = average_chunks(d), longest = longest_chunks(d);
+    const auto time = [&](int n) { return scan_time(SCAN_TIME_BWD_KEPT, d, lanes, chunks, longest, n); };
+    if (time(1) < 0.95 * time(fwd)) bwd = 1;
     return fwd;
 }
 

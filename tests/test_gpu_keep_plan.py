@@ -40,15 +40,34 @@ def test_where_it_is_suggested():
     assert size(_lib.PASS_FWD_KEEP) < _plan(600, 4, segments=3)[0]
 
 
-# the fastest of 1 to 32 segments, forward and backward pass together, with the next one's time over it
+# the forward pass's segments, and the faster of these and one for the backward pass
 @pytest.mark.parametrize("K,V,lanes,chunks,dtype,want", [
-    (128, 128, 1, 313, torch.bfloat16, (16, 8)), (128, 128, 8, 128, torch.bfloat16, (8, 8)), (128, 128, 16, 16, torch.bfloat16, (1, 1)),
-    (64, 128, 2, 200, torch.bfloat16, (16, 16)), (64, 64, 16, 63, torch.float32, (8, 8)), (128, 128, 16, 8, torch.float32, (4, 4)),
-    (64, 64, 1, 8, torch.float32, (1, 1))])
+    (128, 128, 1, 313, torch.bfloat16, (16, 16)), (128, 128, 8, 128, torch.bfloat16, (8, 8)), (128, 128, 16, 16, torch.bfloat16, (1, 1)),
+    (128, 128, 16, 200, torch.bfloat16, (4, 4)), (64, 128, 2, 200, torch.bfloat16, (16, 16)), (64, 64, 16, 63, torch.float32, (8, 8)),
+    (128, 128, 16, 8, torch.float32, (1, 1)), (64, 64, 1, 8, torch.float32, (1, 1))])
 def test_segments(K, V, lanes, chunks, dtype, want):
-    fwd, bwd = _plan(16 * chunks, lanes, K, V, dtype)[1:]
-    assert bwd in (1, fwd)
-    assert fwd == want[0] and bwd == want[1] or (dtype == torch.bfloat16 and chunks == 313 and fwd in (8, 16) and bwd == fwd)
+    assert _plan(16 * chunks, lanes, K, V, dtype)[1:] == want
+
+
+def test_the_forward_pass_runs_in_the_segments_it_has_without_gradients():
+    """Read off the workspace, which holds the segments' records."""
+    for dtype in (torch.bfloat16, torch.float32):
+        for K, V in ((64, 64), (64, 128), (128, 64), (128, 128)):
+            for lanes in (1, 2, 3, 5, 8, 12, 16, 33, 64, 200):
+                for chunks in (1, 4, 8, 12, 15, 16, 31, 64, 97, 128, 200, 313, 500):
+                    for cu in (None, 2):
+                        n, fwd, bwd = _plan(16 * chunks * (cu or 1), lanes, K, V, dtype, cu)
+                        if not n:
+                            continue
+                        assert bwd in (1, fwd)
+                        if dtype == torch.bfloat16 and K == V == 64:
+                            assert fwd == 1                     # (asked for, segments are the fused route's)
+                            continue
+                        d = _lib.make_dims(1, 16 * chunks * (cu or 1), lanes, K, V, 2, cu or 1, dtype, dtype, 1.0, None)
+                        d.cu_seqlens = 256 if cu else None
+                        size = lambda: _lib.load().hdla_workspace_bytes(ctypes.byref(d), _lib.PASS_FWD)
+                        own, d.segments = size(), fwd
+                        assert size() == own, (dtype, K, V, lanes, chunks, cu)
 
 
 CASES = [(2, 100, 2, 64, 64, None), (1, 70, 3, 128, 128, None), (1, 300, 2, 64, 128, (0, 37, 37, 200, 300)), (1, 330, 2, 128, 64, None),
@@ -102,6 +121,24 @@ def test_the_gradients_of_a_pass_that_recomputes(B, T, H, K, V, cu, dtype, form,
         want = [o.detach(), ht.detach(), *torch.autograd.grad([o, ht], ref, [do.cpu().double(), dht.cpu().double()])]
         errs = [O.rel_l2(a, b) for a, b in zip(got, want)]
         assert max(errs) <= (1e-2 if dtype == torch.bfloat16 else 1e-5), errs
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("T,H,K,V,cu,dtype", [(3200, 16, 128, 128, None, torch.bfloat16), (3200, 1, 128, 128, None, torch.bfloat16),
+                                              (2048, 4, 64, 128, None, torch.bfloat16), (3300, 3, 128, 64, (0, 1900, 1917, 3300), torch.bfloat16),
+                                              (128, 16, 128, 128, None, torch.float32), (250, 2, 128, 64, None, torch.float32)])
+def test_outputs_with_and_without_gradients(T, H, K, V, cu, dtype, native, monkeypatch):
+    """The same bits, as a recomputation that replaces a pass without gradients expects them."""
+    if not native:
+        monkeypatch.setattr(_lib, "_native", _lib._NoNative())
+    x, _, _ = _leaves("ab", 1, T, H, K, V, cu, dtype, gk_div=64.0)      # (so little decay that every segment hears of the first)
+    x = [t.to(DEV) for t in x]
+    table = None if cu is None else torch.tensor(cu, device=DEV)
+    run = lambda: chunk_hrdplr_delta_rule(*x[:-1], 2, scale=0.7, initial_state=x[-1], output_final_state=True, cu_seqlens=table)
+    plain = run()
+    x[0].requires_grad_()
+    assert all(torch.equal(a, b) for a, b in zip(run(), plain))
 
 
 @pytest.mark.gpu
