@@ -385,7 +385,9 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
         const auto at = [](void* base, size_t o) { return reinterpret_cast<float*>(static_cast<char*>(base) + o); };
         a.seg = SegRec{nseg, at(prep_ws, LP.SEG_LOC), at(prep_ws, LP.SEG_TR), at(prep_ws, LP.SEG_IN), nullptr, nullptr, nullptr, nullptr};
         if (!fwd) { a.seg.rloc = at(workspace, LS.SEG_RLOC); a.seg.rtr = at(prep_ws, LP.SEG_RTR); a.seg.rin = at(workspace, LS.SEG_RIN); }
-        if (pass == HDLA_PASS_FWD_KEEP) a.seg.turned = at(prep_ws, LP.SEG_RTR);
+        // (a backward pass that is told its number of segments: the transitions as one on a kept workspace meets them, so that its bits do not depend on
+        // whether there was room to keep one)
+        if (pass == HDLA_PASS_FWD_KEEP || (pass == HDLA_PASS_BWD && d->segments > 0)) a.seg.turned = at(prep_ws, LP.SEG_RTR);
     }
     hipError_t e;
     if (pass == HDLA_PASS_BWD_KEPT) {

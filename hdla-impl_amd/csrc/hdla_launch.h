@@ -34,7 +34,7 @@ template <typename T> hipError_t launch_scan_pair(const ChunkArgs<T>& a, int K, 
 enum SegStart {
     SEG_FWD,          // of launch_scan_out, after launch_prep of mode 0
     SEG_FWD_KEPT,     // the same after mode 2
-    SEG_BWD,          // of the two scans of the backward pass, after mode 1
+    SEG_BWD,          // of the two scans of the backward pass, after mode 1 (with seg.turned: rtr as SEG_FWD_KEPT leaves it)
     SEG_BWD_KEPT      // the reverse scan's alone, on the states and transitions that SEG_FWD_KEPT left
 };
 template <typename T> hipError_t launch_scan_segments(const ChunkArgs<T>& a, int K, int V, SegStart what, hipStream_t stream);

@@ -129,7 +129,9 @@ struct SegRec {
     float *loc, *tr, *in;     // [V/16][K/16] state the segment leaves when it starts from zero (the first: from h0);
                               // [K/16][K/16] its transition matrix; [V/16][K/16] the state that enters it
     float *rloc, *rtr, *rin;  // the same for the state gradient, from the right (the last: from dht)
-    float* turned;            // of a forward pass whose workspace the backward pass will use: where that finds its rtr (null: it forms its own)
+    float* turned;            // where the forward direction's records leave rtr, the transitions the other way round (null: they don't; the reverse
+                              // direction's records form their own): in a forward pass whose workspace the backward pass will use, and in a
+                              // backward pass that is told its number of segments
 };
 
 template <typename T>

@@ -378,7 +378,7 @@ template <int K, int V> hipError_t launch_scan_grad_shape(const ChunkArgs<bf16>&
 template <int K, int V> hipError_t launch_scan_grad_segments_shape(const ChunkArgs<bf16>& a, SegStart what, hipStream_t stream) {
     constexpr int NWC = 4;
     typedef RevCfg<K, V, NWC, true> C;
-    hipLaunchKernelGGL((scan_grad_sum_kernel<K, V, NWC>), dim3(a.H, sum_splits<K, V, NWC>(what), a.st.N * (a.seg.nseg - 1)), dim3(C::THREADS), 0,
+    hipLaunchKernelGGL((scan_grad_sum_kernel<K, V, NWC>), dim3(a.H, sum_splits<K, V, NWC>(what, a.seg.turned), a.st.N * (a.seg.nseg - 1)), dim3(C::THREADS), 0,
                        stream, a, sum_first<K, V, NWC>(what));
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? launch_scan_chain<bf16, K, V>(a, what, stream) : e;

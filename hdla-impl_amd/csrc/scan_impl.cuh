@@ -644,7 +644,7 @@ __global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_pair_ke
 }
 // The segments' records: grid = (H, directions * (V + K) / 16 / NWC, N * (segments - 1)); forward the segments before the
 // last, in reverse those behind the first.  first_y: blockIdx.y counts from there on (SEG_BWD_KEPT: the reverse direction's V / 16 / NWC, which
-// leave out the transitions' columns).
+// leave out the transitions' columns; see sum_splits).
 template <typename T, int K, int V, int NWC, bool BOTH>
 __global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_sum_kernel(ChunkArgs<T> p, int first_y) {
     constexpr int NF = NSLOT * blk_fwd(K, sizeof(T), false).SIZE;
@@ -764,14 +764,18 @@ static hipError_t launch_scan_chain(const ChunkArgs<T>& a, SegStart what, hipStr
                        what == SEG_BWD_KEPT ? V / 16 : 0);
     return hipGetLastError();
 }
-// workgroups of a (sequence, head, segment) in the launch of the segments' records, and the first of them
-template <int K, int V, int NWC> static int sum_splits(SegStart what) { return what == SEG_BWD_KEPT ? V / 16 / NWC : (V + K) / 16 / NWC * (what == SEG_BWD ? 2 : 1); }
+// workgroups of a (sequence, head, segment) in the launch of the segments' records, and the first of them.  With `turned` the forward direction's
+// leave the reverse one's transitions, whose columns, the last ones of the launch, are then not asked for.
+template <int K, int V, int NWC> static int sum_splits(SegStart what, bool turned) {
+    constexpr int state = V / 16 / NWC, all = (V + K) / 16 / NWC;
+    return what == SEG_BWD_KEPT ? state : what != SEG_BWD ? all : turned ? all + state : 2 * all;
+}
 template <int K, int V, int NWC> static int sum_first(SegStart what) { return what == SEG_BWD_KEPT ? (V + K) / 16 / NWC : 0; }
 template <typename T, int K, int V>
 hipError_t launch_scan_segments_shape(const ChunkArgs<T>& a, SegStart what, hipStream_t stream) {
     constexpr int NWC = 4;                                // column blocks per workgroup: each fetches the chunks' operands once for them
     typedef ScanCfg<T, K, V, NWC> C;
-    const dim3 grid(a.H, sum_splits<K, V, NWC>(what), a.st.N * (a.seg.nseg - 1)), block(C::THREADS);
+    const dim3 grid(a.H, sum_splits<K, V, NWC>(what, a.seg.turned), a.st.N * (a.seg.nseg - 1)), block(C::THREADS);
     const int first = sum_first<K, V, NWC>(what);
     if (what == SEG_BWD || what == SEG_BWD_KEPT) hipLaunchKernelGGL((scan_sum_kernel<T, K, V, NWC, true>), grid, block, 0, stream, a, first);
     else hipLaunchKernelGGL((scan_sum_kernel<T, K, V, NWC, false>), grid, block, 0, stream, a, first);

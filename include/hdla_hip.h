@@ -84,7 +84,8 @@ typedef struct hdla_dims {
     const int64_t* cu_seqlens; /* DEVICE int64[N+1] cumulative sequence starts on the T axis, or NULL */
     int32_t route;             /* HDLA_ROUTE_*; 0 = the library chooses */
     int32_t segments;          /* time segments per sequence; 0 = the library chooses.  Fused route: at most 64.  Scans of the
-                                * classic kernels under HDLA_ROUTE_AUTO: at most 32, and 4096 over all sequences and heads */
+                                * classic kernels under HDLA_ROUTE_AUTO: at most 32, and 4096 over all sequences and heads; told a number,
+                                * hdla_chunk_bwd has the bits of hdla_chunk_bwd_kept on a workspace kept with it */
 } hdla_dims;
 
 /* Byte offsets of the named intermediates inside the workspace (0 = not part of this pass); for tests and

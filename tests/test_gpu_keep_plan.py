@@ -1,6 +1,5 @@
 """What a training call keeps of its forward pass where nothing is said about it (hdla_keep_plan): where the library suggests it (on the CPU), and
-that a backward pass on it is the one that recomputes: whole sequences bit for bit, in time segments, whose reverse chain takes the forward
-pass's transitions turned, within the rounding of the element type."""
+that a backward pass on it is the one that recomputes in as many time segments, bit for bit."""
 import ctypes
 import time
 
@@ -106,14 +105,9 @@ def test_the_gradients_of_a_pass_that_recomputes(B, T, H, K, V, cu, dtype, form,
     table = None if cu is None else torch.tensor(cu, device=DEV)
     if segments > 1 or dtype == torch.float32 or K != 64 or V != 64:
         monkeypatch.setenv("HDLA_HIP_SEGMENTS", str(segments))
-    before = torch.cuda.memory_allocated()
     got, again = _grads(form, x, do, dht, table, None), _grads(form, x, do, dht, table, False)
     for i, (a, b) in enumerate(zip(got, again)):
-        if i < 2 or segments == 1:
-            assert torch.equal(a, b), i
-        else:
-            # a transition formed on the way there and one formed on the way back, each of operands rounded to the element type
-            assert torch.isfinite(a.float()).all() and O.rel_l2(a, b) <= (2e-3 if dtype == torch.bfloat16 else 2e-7), (i, O.rel_l2(a, b))
+        assert torch.equal(a, b), (i, O.rel_l2(a, b))
     if segments == 3 and native:                                # against the float64 recurrence
         ref = [t.detach().cpu().double().requires_grad_() for t in x]
         ab = list(O.parameterize_a_b(ref[3], ref[1], ref[4])) if form == "beta" else ref[3:5]
