@@ -149,8 +149,10 @@ int scan_segments(const hdla_dims* d, bool bwd) {
 int kept_segments(const hdla_dims* d) { return d->segments > 0 ? scan_segments(d, false) : 1; }
 
 // What a training call keeps of its forward pass where nothing else is said: all that the prep kernel forms, which the backward pass would form
-// again (1.6 times the inputs' bytes at K = V = 64), and the records of the segments, if it is little beside the 288 GB of the device.  us on the device,
-// a training step that keeps the inputs -> this: 1 x 256 tokens, 2 heads, K = V = 64 43 -> 37; 2 x 1537 tokens, 8 heads, K = V = 128 214 -> 185;
+// again (1.6 times the inputs' bytes at K = V = 64), and the records of the segments; of one call this much, 0.1 % of the device's memory (what all of them hold,
+// the caller bounds: native.cpp, kept_room).  With its scratch a call's backward pass
+// then has 5 % more than one that recomputes has, median of 839 shapes, 41 % at the most, where the forward pass alone is in segments.  us on the device, a training step
+// that keeps the inputs -> this: 1 x 256 tokens, 2 heads, K = V = 64 43 -> 37; 2 x 1537 tokens, 8 heads, K = V = 128 214 -> 185;
 // 4 x 1000 tokens, 16 heads 430 -> 393; 4 x 500, 8 heads 127 -> 107; fp32, 2 x 1003 tokens, 8 heads, K = V = 64 227 -> 190.
 constexpr size_t KEEP_MOST = (size_t)256 << 20;
 // Segments of the two passes of such a call (return, bwd).  The forward pass has those it has without gradients, and so the same bits (what recomputes a

@@ -4,7 +4,9 @@ The library is the only compute path: if it cannot be loaded every operator rais
 """
 import ctypes
 import os
+import threading
 import warnings
+import weakref
 from typing import Optional, Tuple
 
 import torch
@@ -169,6 +171,9 @@ def load():
     return lib
 
 
+KEPT_MOST, KEPT_CALLS = 1 << 30, 256             # as in csrc/native.cpp
+
+
 class _NoNative:
     """What stands in for the native host path where that cannot be loaded: nothing is its case."""
 
@@ -179,6 +184,29 @@ class _NoNative:
 
     def forget(self, cache):
         return [None] * 4
+
+    def __init__(self):
+        self._held, self._coming, self._lock = {}, {}, threading.Lock()
+
+    def kept_room(self, like, n):
+        """Room for a forward workspace that a call holds for its backward pass unasked, or None: KEPT_MOST bytes a device and KEPT_CALLS calls
+        over all whose backward pass is still to come, and what the allocator has (csrc/native.cpp, kept_room)."""
+        dev, t = like.device.index, None
+        with self._lock:
+            held = self._held[dev] = [h for h in self._held.get(dev, ()) if h[0]() is not None]
+            if sum(h[1] for h in held) + self._coming.get(dev, 0) + n > KEPT_MOST or len(held) >= KEPT_CALLS:
+                return None
+            self._coming[dev] = self._coming.get(dev, 0) + n
+        try:
+            t = torch.empty(n, dtype=torch.uint8, device=like.device)
+        except torch.OutOfMemoryError:
+            pass
+        finally:
+            with self._lock:
+                self._coming[dev] -= n
+                if t is not None:
+                    self._held[dev].append((weakref.ref(t), n))
+        return t
 
 
 def native():
@@ -290,7 +318,8 @@ PASS_FWD, PASS_BWD, PASS_FWD_KEEP, PASS_BWD_KEPT = 0, 1, 2, 3
 def keep_forward_default() -> Optional[bool]:
     """Whether the chunked operators keep the forward pass's per-chunk intermediates for the backward pass when the
     caller does not say (``keep_forward=None``): environment variable HDLA_HIP_KEEP_FORWARD=1 or 0.  Where that does not say
-    either (None), the library keeps them where they are small (``keep_plan``), unless HDLA_HIP_INPUTS_ONLY=1."""
+    either (None), the library keeps them where they are small (``keep_plan``) and there is room (``kept_room``), unless
+    HDLA_HIP_INPUTS_ONLY=1."""
     v = os.environ.get("HDLA_HIP_KEEP_FORWARD")
     return None if v is None else v not in ("", "0", "false", "False")
 

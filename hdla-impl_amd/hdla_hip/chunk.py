@@ -71,7 +71,7 @@ def _dims(q, v, gk, scale, cu_seqlens, n_seq, plan=(None, None)):
 def chunk_hrdplr_fwd(q, k, v, a, b, gk, scale, initial_state, output_final_state, cu_seqlens=None, keep=False,
                      beta=None, want_boundary=False, plan=(None, None)):
     """Forward launch sequence (HRDPLR/hrdplr.py:25-99) on native shapes: returns (o, final_state), with ``keep`` also
-    the workspace the backward pass can run on instead of recomputing it (``hdla_chunk_fwd_keep``), with
+    the workspace the backward pass can run on instead of recomputing it (``hdla_chunk_fwd_keep``; ``keep``: True, or the buffer), with
     ``want_boundary`` also the record for the backward pass (None where the route has none).
     With ``beta`` a and b are formed in the kernels (they may be None).  ``plan``: route and segments (None: the environment's)."""
     lib = _lib.load()
@@ -82,8 +82,8 @@ def chunk_hrdplr_fwd(q, k, v, a, b, gk, scale, initial_state, output_final_state
         dims = _dims(q, v, gk, scale, cu_seqlens, N, plan)
         o = torch.empty_like(v)
         ht = torch.empty(N, H, K, V, dtype=torch.float32, device=q.device) if output_final_state else None
-        if keep:
-            ws = _lib.workspace(dims, _lib.PASS_FWD_KEEP, q.device)
+        if keep is not False:
+            ws = _lib.workspace(dims, _lib.PASS_FWD_KEEP, q.device) if keep is True else keep
             rc = lib.hdla_chunk_fwd_keep(ctypes.byref(dims), _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(a),
                                          _lib.ptr(b), _lib.ptr(beta), _lib.ptr(gk), _lib.ptr(initial_state), _lib.ptr(o),
                                          _lib.ptr(ht), _lib.ptr(ws), ws.numel(), _lib.current_stream(q.device))
@@ -102,11 +102,15 @@ def chunk_hrdplr_fwd(q, k, v, a, b, gk, scale, initial_state, output_final_state
 
 
 def keep_plan(q, v, gk, scale, cu_seqlens):
-    """The plans (route, segments) of a forward pass that keeps its workspace and of the backward pass on it, where the library
-    suggests to keep it; None where it does not."""
+    """Where the library suggests that a training call keep its forward pass's workspace: the plans (route, segments) of that pass and of the
+    backward pass, which is the same whether there was room to keep it, and the buffer, or False where there was none.  None where
+    the library does not suggest it."""
     dims = _dims(q, v, gk, scale, cu_seqlens, q.shape[0] if cu_seqlens is None else cu_seqlens.numel() - 1)
     n, fwd, bwd = _lib.keep_plan(dims)
-    return ((dims.route, fwd), (dims.route, bwd)) if n and not _lib.load().hdla_record_bytes(ctypes.byref(dims)) else None
+    if not n or _lib.load().hdla_record_bytes(ctypes.byref(dims)):
+        return None
+    room = _lib.native().kept_room(q, n)
+    return (dims.route, fwd), (_lib.ROUTE_CLASSIC if bwd == 1 else dims.route, bwd), False if room is None else room
 
 
 ONE_SEGMENT = (_lib.ROUTE_AUTO, 1)                        # keep_forward=True: results are those of the classic kernels on whole sequences
@@ -196,10 +200,12 @@ class ChunkDPLRDeltaRuleFunction(torch.autograd.Function):
             ctx.plan = ONE_SEGMENT
         elif any(ctx.needs_input_grad) and _lib.keep_boundaries_default():
             plans = keep_plan(q, v, gk, scale, cu_seqlens) if keep_forward is None else None
+            own, room = ctx.plan, False
             if plans:
-                ctx.on_kept, ctx.plan = True, plans[1]
+                ctx.plan, room = plans[1:]
+                ctx.on_kept = room is not False
             o, final_state, boundary = chunk_hrdplr_fwd(q, k, v, a, b, gk, scale, h0, output_final_state, cu_seqlens,
-                                                        keep=ctx.on_kept, want_boundary=True, plan=plans[0] if plans else ctx.plan)
+                                                        keep=room, want_boundary=True, plan=plans[0] if ctx.on_kept else own)
         else:
             o, final_state = chunk_hrdplr_fwd(q, k, v, a, b, gk, scale, h0, output_final_state, cu_seqlens)
         # the inputs (hrdplr.py:137) and, where the route has one, the forward pass's record (37 % of the inputs' bytes), or its
@@ -264,8 +270,9 @@ def chunk_hrdplr_delta_rule(
     until the backward pass (about 1.6 times the bytes of q, k, v, a, b, gk together), which then skips recomputing
     them; False is closest to the reference's behaviour, where only the inputs are kept (hrdplr.py:137) and the backward pass
     recomputes (:161-198): here the fused route's record is kept beside them.  None (and HDLA_HIP_KEEP_FORWARD unset): kept
-    where that is at most 256 MiB and the route has no record.  HDLA_HIP_INPUTS_ONLY=1: strictly the inputs, unless True.
-    Results agree to rounding.
+    where that is at most 256 MiB and the route has no record, and only as long as all calls whose backward pass is still to come hold
+    at most 1 GiB a device that way; beyond, and where the memory cannot be had, the same bits are recomputed.
+    HDLA_HIP_INPUTS_ONLY=1: strictly the inputs, unless True.  Results agree to rounding.
     """
     out = _lib.native().chunk(q, k, v, a, b, gk, RANK_AB, scale, initial_state, output_final_state, head_first, chunk_size,
                               cu_seqlens, keep_forward)

@@ -66,10 +66,12 @@ class ChunkHDLAFunction(torch.autograd.Function):
             ctx.plan = ONE_SEGMENT
         elif any(ctx.needs_input_grad) and _lib.keep_boundaries_default():
             plans = keep_plan(q, v, gk, scale, cu_seqlens) if keep_forward is None else None
+            own, room = ctx.plan, False
             if plans:
-                ctx.on_kept, ctx.plan = True, plans[1]
+                ctx.plan, room = plans[1:]
+                ctx.on_kept = room is not False
             o, final_state, boundary = _fwd(q, k, v, beta, gk, scale, h0, output_final_state, cu_seqlens, want_boundary=True,
-                                            keep=ctx.on_kept, plan=plans[0] if plans else ctx.plan)
+                                            keep=room, plan=plans[0] if ctx.on_kept else own)
         else:
             o, final_state = _fwd(q, k, v, beta, gk, scale, h0, output_final_state, cu_seqlens)
         ctx.save_for_backward(q, k, v, beta, gk, initial_state, cu_seqlens, boundary)

@@ -174,7 +174,10 @@ size_t hdla_record_bytes(const hdla_dims* dims);
 size_t hdla_record_workspace_bytes(const hdla_dims* dims);
 /* What a training call on the classic kernels may hand from the forward to the backward pass instead of having it formed again: bytes of the
  * buffer for hdla_chunk_fwd_keep and hdla_chunk_bwd_kept that the library suggests to keep, and the `segments` to give the one and the other in
- * dims; 0 where it suggests none (the fused route has its record; a buffer of more than 256 MiB; no tokens). */
+ * dims; 0 where it suggests none (the fused route has its record; a buffer of more than 256 MiB; no tokens).  The suggestion is for one call: a
+ * program with many calls between a forward and its backward pass holds as many buffers, and bounds what they come to (the Python package: 1 GiB and
+ * 256 calls a device).  A backward pass without the buffer, hdla_chunk_bwd_b with bwd_segments in dims (and, where that is 1, HDLA_ROUTE_CLASSIC), has the same
+ * bits. */
 size_t hdla_keep_plan(const hdla_dims* dims, int32_t* fwd_segments, int32_t* bwd_segments);
 int hdla_chunk_fwd_b(const hdla_dims* dims, const void* q, const void* k, const void* v, const void* a, const void* b,
                      const void* beta, const void* gk, const float* h0, void* o, float* ht, void* boundary,

@@ -1,6 +1,7 @@
 """What a training call keeps of its forward pass where nothing is said about it (hdla_keep_plan): where the library suggests it (on the CPU), and
 that a backward pass on it is the one that recomputes in as many time segments, bit for bit."""
 import ctypes
+import gc
 import time
 
 import pytest
@@ -178,6 +179,107 @@ def test_it_is_kept_and_given_back(native, monkeypatch):
             for name, value in env.items():
                 c.setenv(name, value)
             assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(o, x, do), ref)), env
+
+
+def test_the_account_of_the_python_code(monkeypatch):
+    """On the CPU: what a call holds is on it until its backward pass is through, also behind torch's saved tensors."""
+    monkeypatch.setattr(_lib, "KEPT_MOST", 1000)
+    acc, like = _lib._NoNative(), torch.empty(1)
+
+    class Keep(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x, n):
+            room = acc.kept_room(like, n)
+            ctx.got = room is not None
+            ctx.save_for_backward(x, room)
+            return x * 2
+
+        @staticmethod
+        def backward(ctx, g):
+            ctx.saved_tensors
+            return g * 2, None
+
+    x = torch.ones(3, requires_grad=True)
+    got = lambda y: y.grad_fn.got
+    a, b, c = Keep.apply(x, 400), Keep.apply(x, 600), Keep.apply(x, 1)
+    gc.collect()
+    d = Keep.apply(x, 1)
+    assert [got(y) for y in (a, b, c, d)] == [True, True, False, False]
+    torch.autograd.grad(a.sum(), x)                              # (the graph's end lets go of its saved tensors)
+    e, f = Keep.apply(x, 300), Keep.apply(x, 200)
+    assert got(e) and not got(f)
+    del b, e
+    fresh = lambda: [got(Keep.apply(x, 1000)) for _ in range(2)]
+    assert fresh() == [True, True]
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.clone(), lambda t: t):
+        h = Keep.apply(x, 1000)
+    assert got(h) and fresh() == [True, True]                    # (the hook's copy is not on it)
+    many = [Keep.apply(x, 1) for _ in range(_lib.KEPT_CALLS + 1)]
+    assert [got(y) for y in many] == [True] * _lib.KEPT_CALLS + [False]
+    del many
+    monkeypatch.setattr(torch, "empty", lambda *a, **kw: (_ for _ in ()).throw(torch.OutOfMemoryError()))
+    assert acc.kept_room(like, 900) is None and acc._coming == {None: 0}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("native", [True, False])
+def test_calls_whose_backward_pass_is_to_come_hold_a_gibibyte_at_most(native, monkeypatch):
+    if not native:
+        monkeypatch.setattr(_lib, "_native", _lib._NoNative())
+    T, H, D = 5008, 16, 128
+    each = _plan(T, H)[0]
+    most = (1 << 30) // each
+    assert 2 < most < 8
+    x, do, _ = _leaves("ab", 1, T, H, D, D, None, torch.bfloat16, gk_div=64.0)
+    x, do = [t.to(DEV).requires_grad_() for t in x], do.to(DEV)
+    run = lambda: chunk_hrdplr_delta_rule(*x[:-1], 2, scale=0.7, initial_state=x[-1])[0]
+    gc.collect()
+    torch.cuda.synchronize()
+    held, outs = [], []
+    for _ in range(most + 2):
+        at = torch.cuda.memory_allocated()
+        outs.append(run())
+        held.append(torch.cuda.memory_allocated() - at - outs[-1].numel() * 2 >= each)
+    assert held == [True] * most + [False] * 2
+    first = torch.autograd.grad(outs[0], x, do)
+    for o in outs[1:]:                                           # kept or not: the same bits
+        assert torch.equal(o, outs[0]) and all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(o, x, do), first))
+    del o, outs
+    for _ in range(1000):
+        at = torch.cuda.memory_allocated()
+        o = run()
+        if torch.cuda.memory_allocated() - at >= each:
+            return
+        del o
+        time.sleep(1e-3)
+    assert False, "nothing was given back"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("native", [True, False])
+def test_where_the_buffer_cannot_be_had(native, monkeypatch):
+    """A limit of torch's allocator between what the call needs and what it would keep: it runs, and so does its backward pass later."""
+    if not native:
+        monkeypatch.setattr(_lib, "_native", _lib._NoNative())
+    T, H, D = 5008, 16, 128
+    each = _plan(T, H)[0]
+    x, do, _ = _leaves("ab", 1, T, H, D, D, None, torch.bfloat16, gk_div=64.0)
+    x, do = [t.to(DEV).requires_grad_() for t in x], do.to(DEV)
+    run = lambda: chunk_hrdplr_delta_rule(*x[:-1], 2, scale=0.7, initial_state=x[-1])[0]
+    want = torch.autograd.grad(run(), x, do)
+    gc.collect()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    d = _lib.make_dims(1, T, H, D, D, 2, 1, torch.bfloat16, torch.bfloat16, 1.0, None)
+    need = _lib.load().hdla_workspace_bytes(ctypes.byref(d), _lib.PASS_FWD) + 2 * T * H * D
+    room = need + (24 << 20)                                     # (the allocator's blocks of 2 and 20 MiB)
+    assert room < each
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + room) / torch.cuda.get_device_properties(0).total_memory)
+        o = run()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(o, x, do), want))
 
 
 @pytest.mark.gpu
