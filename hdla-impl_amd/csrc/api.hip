@@ -369,6 +369,8 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
         rc = make_layout(d, pass, LS, nch);
         if (rc) return rc;
         if (bad_ws(workspace, workspace_bytes, LS.total)) return HDLA_ERR_WORKSPACE;
+        // (the records lie where their number puts them: another number's buffer, which another size shows, would be read wrongly)
+        if (kept_segments(d) > 1 && kept_bytes != LP.total) return HDLA_ERR_WORKSPACE;
     }
     ChunkArgs<T> a{};
     a.q = static_cast<const T*>(q); a.k = static_cast<const T*>(k); a.v = static_cast<const T*>(v);
@@ -579,7 +581,7 @@ const char* hdla_strerror(int code) {
         case HDLA_ERR_SHAPE: return "unsupported shape (need K,V in {64,128}, or 256 as well for the token-serial entry points; B,H,N >= 1, T >= 0, H,N <= 65535, chunks x heads < 2^31)";
         case HDLA_ERR_RANK: return "only rank R = 2 is supported";
         case HDLA_ERR_DTYPE: return "unsupported dtype (in_dtype bf16|fp32; gk fp32, or bf16 with bf16 inputs)";
-        case HDLA_ERR_WORKSPACE: return "workspace is NULL, not 256-byte aligned, or smaller than hdla_workspace_bytes()";
+        case HDLA_ERR_WORKSPACE: return "workspace is NULL, not 256-byte aligned, smaller than hdla_workspace_bytes(), or kept with another number of segments";
         case HDLA_ERR_ALIGN: return "tensor pointers must be 16-byte aligned";
         case HDLA_ERR_SEQ: return "cu_seqlens needs B == 1; without it N must equal B";
         case HDLA_ERR_ROUTE: return "route must be HDLA_ROUTE_AUTO, _CLASSIC or _FUSED (the fused route: bf16 inputs, K = V = 64) and segments >= 0";

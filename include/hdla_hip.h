@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-#define HDLA_VERSION 206
+#define HDLA_VERSION 207
 
 enum { HDLA_BF16 = 0, HDLA_FP32 = 1 };
 
@@ -213,7 +213,8 @@ int hdla_param_chunk_bwd(const hdla_dims* dims, const void* q, const void* k, co
  * only read by the backward call (it can be used again); `workspace` is scratch of
  * hdla_workspace_bytes(dims, HDLA_PASS_BWD_KEPT) bytes.  Same dims, inputs and stream ordering as the forward call.
  * Time segments: one where dims->segments is 0, otherwise (HDLA_ROUTE_AUTO) as many as it says; the states that enter them and their transitions
- * are part of `kept`.  The backward call takes the forward call's number, whose records it then reads, or 1.  Rows of a packed batch that
+ * are part of `kept`.  The backward call takes the forward call's number, whose records it then reads (kept_bytes must be exactly
+ * hdla_workspace_bytes(dims, HDLA_PASS_FWD_KEEP), which tells one number from another), or 1.  Rows of a packed batch that
  * belong to no sequence are cleared in the gradients, as in hdla_chunk_bwd. */
 int hdla_chunk_fwd_keep(const hdla_dims* dims, const void* q, const void* k, const void* v, const void* a,
                         const void* b, const void* beta, const void* gk, const float* h0, void* o, float* ht,

@@ -312,6 +312,13 @@ def test_the_layer(d, H, T, monkeypatch):
 def test_a_buffer_of_another_plan_is_refused():
     x, do, dht = [t if isinstance(t, list) else t.to(DEV) for t in _leaves("ab", 1, 200, 2, 128, 128, None, torch.float32)]
     q, k, v, a, b, gk, h0 = [t.to(DEV) for t in x]
-    _, _, kept = CK.chunk_hrdplr_fwd(q, k, v, a, b, gk, 0.7, h0, True, keep=True, plan=(_lib.ROUTE_AUTO, 1))
-    with pytest.raises(_lib.HdlaError, match="-5"):
-        CK.chunk_hrdplr_bwd_kept(q, k, v, a, b, gk, 0.7, h0, do, dht, kept, plan=(_lib.ROUTE_AUTO, 4))
+    plan = lambda n: (_lib.ROUTE_AUTO, n)
+    kept = {n: CK.chunk_hrdplr_fwd(q, k, v, a, b, gk, 0.7, h0, True, keep=True, plan=plan(n))[2] for n in (1, 4, 8)}
+    bwd = lambda n, buffer: CK.chunk_hrdplr_bwd_kept(q, k, v, a, b, gk, 0.7, h0, do, dht, buffer, plan=plan(n))
+    # too few records, too many, and a longer buffer that may be either; one segment reads none of them
+    for n, buffer in ((4, kept[1]), (8, kept[4]), (4, kept[8]), (4, torch.cat([kept[4], kept[4]]))):
+        with pytest.raises(_lib.HdlaError, match="-5"):
+            bwd(n, buffer)
+    for n in (4, 8):
+        bwd(n, kept[n])
+        assert all(torch.equal(s, t) for s, t in zip(bwd(1, kept[n]), bwd(1, kept[1])))
