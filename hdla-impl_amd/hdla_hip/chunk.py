@@ -113,11 +113,14 @@ def keep_plan(q, v, gk, scale, cu_seqlens):
     return (dims.route, fwd), (_lib.ROUTE_CLASSIC if bwd == 1 else dims.route, bwd), False if room is None else room
 
 
-ONE_SEGMENT = (_lib.ROUTE_AUTO, 1)                        # keep_forward=True: results are those of the classic kernels on whole sequences
+def one_segment(plan):
+    """keep_forward=True: results are those of the classic kernels on whole sequences, whatever number of segments is asked for; a route or
+    number that the library refuses stays so."""
+    return plan[0], min(plan[1], 1)
 
 
 def chunk_hrdplr_bwd_kept(q, k, v, a, b, gk, scale, initial_state, do, dht, kept, cu_seqlens=None, want_dh0=True,
-                          beta=None, plan=ONE_SEGMENT):
+                          beta=None, plan=(None, 1)):
     """Backward launch sequence on the workspace a forward pass kept (``hdla_chunk_bwd_kept``): the per-chunk
     intermediates are read there, not recomputed.  Returns (dq, dk, dv, da, db, dgk, dh0), or with ``beta``
     (dq, dk, dv, dbeta, dgk, dh0)."""
@@ -195,9 +198,9 @@ class ChunkDPLRDeltaRuleFunction(torch.autograd.Function):
         ctx.kept = None
         boundary, ctx.plan, ctx.on_kept = None, (_lib.default_route(), _lib.default_segments()), False
         if keep_forward and any(ctx.needs_input_grad):
+            ctx.plan = one_segment(ctx.plan)
             o, final_state, ctx.kept = chunk_hrdplr_fwd(q, k, v, a, b, gk, scale, h0, output_final_state, cu_seqlens, keep=True,
-                                                        plan=ONE_SEGMENT)
-            ctx.plan = ONE_SEGMENT
+                                                        plan=ctx.plan)
         elif any(ctx.needs_input_grad) and _lib.keep_boundaries_default():
             plans = keep_plan(q, v, gk, scale, cu_seqlens) if keep_forward is None else None
             own, room = ctx.plan, False

@@ -21,8 +21,8 @@ import torch
 import torch.nn.functional as F
 
 from . import _lib
-from .chunk import (ONE_SEGMENT, _dims, _native_dim, _pad_last, _require_gpu, chunk_hrdplr_bwd, chunk_hrdplr_bwd_kept,
-                    chunk_hrdplr_fwd, keep_plan)
+from .chunk import (_dims, _native_dim, _pad_last, _require_gpu, chunk_hrdplr_bwd, chunk_hrdplr_bwd_kept, chunk_hrdplr_fwd, keep_plan,
+                    one_segment)
 from .utils import autocast_custom_bwd, autocast_custom_fwd, contiguous
 
 
@@ -62,8 +62,8 @@ class ChunkHDLAFunction(torch.autograd.Function):
         ctx.kept = None
         boundary, ctx.plan, ctx.on_kept = None, (_lib.default_route(), _lib.default_segments()), False
         if keep_forward and any(ctx.needs_input_grad):     # see ChunkDPLRDeltaRuleFunction.forward
-            o, final_state, ctx.kept = _fwd(q, k, v, beta, gk, scale, h0, output_final_state, cu_seqlens, keep=True, plan=ONE_SEGMENT)
-            ctx.plan = ONE_SEGMENT
+            ctx.plan = one_segment(ctx.plan)
+            o, final_state, ctx.kept = _fwd(q, k, v, beta, gk, scale, h0, output_final_state, cu_seqlens, keep=True, plan=ctx.plan)
         elif any(ctx.needs_input_grad) and _lib.keep_boundaries_default():
             plans = keep_plan(q, v, gk, scale, cu_seqlens) if keep_forward is None else None
             own, room = ctx.plan, False

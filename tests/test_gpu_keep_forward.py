@@ -124,6 +124,21 @@ def test_parameterised_operator_kept_route(dtype):
     assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
 
 
+@pytest.mark.parametrize("env", [("HDLA_HIP_ROUTE", "fused"), ("HDLA_HIP_SEGMENTS", "-1")])
+@pytest.mark.parametrize("keep", [True, False, None])
+@pytest.mark.parametrize("form", ["ab", "beta"])
+def test_a_refused_plan_is_refused_with_and_without_keeping(env, keep, form, monkeypatch):
+    inp = make_inputs(604, 1, 40, 2, 128, 128)
+    q, k, v, a, b, gk = [t.bfloat16().to(DEV).requires_grad_() for t in (inp.q, inp.k, inp.v, inp.a, inp.b, inp.gk)]
+    beta = torch.ones(1, 40, 2, 1, device=DEV, dtype=torch.bfloat16)
+    monkeypatch.setenv(*env)
+    with pytest.raises(_lib.HdlaError):
+        if form == "ab":
+            chunk_hrdplr_delta_rule(q, k, v, a, b, gk, 2, keep_forward=keep)
+        else:
+            chunk_hdla_delta_rule(q, k, v, beta, gk, keep_forward=keep)
+
+
 def test_config2_full_size_kept_route_matches_the_recomputing_route():
     inp = make_config(2)
     kept = _run(inp, torch.bfloat16, 1.0, True)
