@@ -403,7 +403,10 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
     }
     if (d->cu_seqlens && (stages & HDLA_STAGE_PREP)) {
         char* base = static_cast<char*>(prep_ws);
-        e = launch_chunk_table(d->cu_seqlens, d->N, d->T, nch, d->H, d->in_dtype == HDLA_FP32 ? 0 : d->V, reinterpret_cast<int32_t*>(base + LP.CHUNK_OFF),
+        // whether one of the scans on this table is shared out by the sequences' lengths (a kept one: of either pass, the backward one's in as many segments
+        // or one)
+        const bool shares = sizeof(T) == 2 && scan_shares(d->cu_seqlens, d->N, d->H, d->V, pass == HDLA_PASS_FWD_KEEP ? 1 : nseg, pass == HDLA_PASS_FWD ? 1 : 2);
+        e = launch_chunk_table(d->cu_seqlens, d->N, d->T, nch, d->H, shares ? d->V : 0, reinterpret_cast<int32_t*>(base + LP.CHUNK_OFF),
                                reinterpret_cast<int32_t*>(base + LP.CHUNK_SEQ), packed_outputs(d, a), stream);
         if (e != hipSuccess) return (int)e;
     }

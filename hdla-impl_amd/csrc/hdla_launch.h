@@ -14,7 +14,7 @@ struct PackedOut {
     int n;
     void add(void* q, long long b) { if (q) { p[n] = q; row[n++] = b; } }
 };
-// (V: of the 2-byte stand-alone scans, which share the device by the sequences' lengths; 0 for the other kernels)
+// (V: where a scan on the table is shared out by the sequences' lengths (scan_shares); else 0, and `order` holds no widths)
 hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int H, int V, int32_t* chunk_off, int32_t* chunk_seq,
                               const PackedOut& out, hipStream_t stream);
 // only what clears the rows that belong to no sequence

@@ -31,6 +31,11 @@ constexpr int SHARE_MAX_N = 32, ORDER_SEQ = 0x0fffffff, ORDER_OUT = 28, ORDER_GR
 // workgroups of a head (and direction) that the device holds at once, one a compute unit, and as many as a shared launch has at the most
 constexpr int share_slots(int H, int directions) { return 256 / (H * directions) > 1 ? 256 / (H * directions) : 1; }
 constexpr int share_most(int H, int directions, int N, int V) { return N * (V / 64) + share_slots(H, directions); }
+// whether a launch of the 2-byte scans is shared out so: whole sequences, and not where the narrowest workgroups fit the device.  The table kernel, which
+// everything else waits for, chooses the widths only then: that takes it 1 us for 8 sequences, 5 for 30.
+inline bool scan_shares(const int64_t* cu, int N, int H, int V, int nseg, int directions) {
+    return cu && N > 1 && N <= SHARE_MAX_N && nseg == 1 && (long long)H * N * directions * (V / 16) > 256;
+}
 
 // Operands of the state scans that all value-column blocks of a (chunk, head) share are kept in ONE contiguous
 // block per (chunk, head), so that a workgroup can copy a block into LDS with a few whole-kilobyte loads.

@@ -367,7 +367,7 @@ template <int K, int V> hipError_t launch_scan_grad_shape(const ChunkArgs<bf16>&
     constexpr int VT = V / 16;
     const int lanes = a.H * a.st.N * a.seg.nseg * (kind == SCAN_PAIR ? 2 : 1);
     if (lanes * VT <= SCAN_TARGET_WORKGROUPS) return launch_scan_grad_nwc<K, V, 1>(a, kind, stream);
-    if (kind == SCAN_PAIR && scan_shares(a.st, a.seg.nseg)) {
+    if (kind == SCAN_PAIR && scan_shares(a.st.cu, a.st.N, a.H, V, a.seg.nseg, 2)) {
         hipLaunchKernelGGL((scan_grad_share_kernel<K, V>), dim3(a.H, 2 * share_most(a.H, 2, a.st.N, V)), dim3(RevCfg<K, V, 4, false>::THREADS), 0,
                            stream, a);
         return hipGetLastError();

@@ -616,7 +616,6 @@ template <int V> __device__ __forceinline__ bool scan_share(const SeqTab& st, in
     split = unit - __builtin_amdgcn_readlane(end - own, r);
     return true;
 }
-inline bool scan_shares(const SeqTab& st, int nseg) { return st.cu && st.N > 1 && st.N <= SHARE_MAX_N && nseg == 1; }
 template <typename T, int K, int V, int NWC, bool WRITE_O>
 __global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_fwd_kernel(ChunkArgs<T> p) {
     constexpr ScanOut OUT = WRITE_O ? OUT_O : OUT_STATE;

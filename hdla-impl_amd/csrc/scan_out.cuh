@@ -438,7 +438,7 @@ template <int K, int V> hipError_t launch_scan_out_shape(const ChunkArgs<bf16>& 
     constexpr int VT = V / 16;
     const int lanes = a.H * a.st.N * a.seg.nseg;
     if (lanes * VT <= SCAN_TARGET_WORKGROUPS) return launch_scan_out_nwc<K, V, 1>(a, kept, stream);
-    if (scan_shares(a.st, a.seg.nseg)) {
+    if (scan_shares(a.st.cu, a.st.N, a.H, V, a.seg.nseg, 1)) {
         const dim3 grid(a.H, share_most(a.H, 1, a.st.N, V)), block(OutCfg<K, V, 4, OUT_O>::THREADS);
         if (kept) hipLaunchKernelGGL((scan_out_share_kernel<K, V, true>), grid, block, 0, stream, a);
         else hipLaunchKernelGGL((scan_out_share_kernel<K, V, false>), grid, block, 0, stream, a);

@@ -1,10 +1,13 @@
 """Few packed sequences whose workgroups in the scans are as wide as their lengths make them (scan_out_share_kernel, scan_grad_share_kernel): every
 width in one launch, empty sequences, more workgroups than the device holds, the first count of sequences that is too many.  Column
 blocks do not meet in a scan, so outputs and gradients have the bits of a call for each sequence by itself."""
+import ctypes
+
 import pytest
 import torch
 
-from hdla_hip import chunk_hrdplr_delta_rule
+import hdla_hip.chunk as CK
+from hdla_hip import _lib, chunk_hrdplr_delta_rule
 from hdla_hip.synthetic import make_inputs
 
 pytestmark = pytest.mark.gpu
@@ -53,3 +56,26 @@ def test_the_bits_of_each_sequence_by_itself(K, V, H, lens, keep, monkeypatch):
         parts = [cut(whole[0], 1), whole[1][n:n + 1]] + [cut(t, k) for t, k in zip(whole[2:8], r)] + [whole[8][n:n + 1]]
         for i, (a, b) in enumerate(zip(parts, alone)):
             assert torch.equal(a, b), (n, i)
+
+
+# (H, segments) of three sequences at V = 128: the scan of the forward pass in workgroups of one column block fits the device up to 10 heads, the two
+# of the backward pass up to 5
+@pytest.mark.parametrize("H,segments,widths", [(5, 1, {"fwd": False, "bwd": False, "keep": False}), (6, 1, {"fwd": False, "bwd": True, "keep": True}),
+                                               (11, 1, {"fwd": True, "bwd": True, "keep": True}), (11, 4, {"fwd": False, "bwd": False, "keep": True})])
+def test_widths_are_chosen_where_a_scan_asks_for_them(H, segments, widths):
+    lens, K, V = [400, 130, 60], 64, 128
+    T, N, plan = sum(lens), len(lens), (_lib.ROUTE_AUTO, segments)
+    cu = torch.tensor([0] + lens, device=DEV).cumsum(0)
+    inp = make_inputs(2101, 1, T, H, K, V, gk_div=4.0, n_states=N)
+    x = [t.bfloat16().to(DEV) for t in (inp.q, inp.k, inp.v, inp.a, inp.b, inp.gk)] + [0.9, inp.h0.to(DEV)]
+    dims = CK._dims(x[0], x[2], x[5], 0.9, cu, N, plan)
+    ws = {"keep": CK.chunk_hrdplr_fwd(*x, True, cu, keep=True, plan=plan)[2],
+          "bwd": CK.chunk_hrdplr_bwd(*x, inp.do.bfloat16().to(DEV), inp.dht.to(DEV), cu, keep_workspace=True, plan=plan)[7],
+          "fwd": _lib.workspace(dims, _lib.PASS_FWD, x[0].device)}
+    P, o = _lib.ptr, torch.empty_like(x[2])
+    assert _lib.load().hdla_chunk_fwd_b(ctypes.byref(dims), *[P(t) for t in x[:5]], None, P(x[5]), P(x[7]), P(o), None, None, 0, P(ws["fwd"]),
+                                        ws["fwd"].numel(), _lib.current_stream(x[0].device)) == 0
+    for name, p in (("fwd", _lib.PASS_FWD), ("bwd", _lib.PASS_BWD), ("keep", _lib.PASS_FWD_KEEP)):
+        at = _lib.workspace_layout(dims, p)["CHUNK_OFF"] + 4 * (N + 1)
+        order = ws[name][at:at + 4 * N].view(torch.int32).tolist()
+        assert [e & 0x0fffffff for e in order] == [0, 1, 2] and any(e >> 28 for e in order) == widths[name], (name, order)
