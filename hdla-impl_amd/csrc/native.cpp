@@ -13,6 +13,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/SavedTensorHooks.h>
 #include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/Event.h>
@@ -158,7 +159,8 @@ Tensor workspace(const hdla_dims& d, int pass, const Tensor& like, bool with_rec
 // Forward workspaces that calls hold for their backward passes because the library suggests it (hdla_keep_plan), and nobody asked: as much as KEPT_MOST
 // a device over all calls whose backward pass is still to come, 0.4 % of its memory, so that a stack of layers that trains within the device's memory
 // without them does so with them, and that of KEPT_CALLS calls, a microsecond to look through.  A call that finds no room, there or with the allocator,
-// keeps its inputs and recomputes, the same bits.  us a training step with room / without / with keep_forward=False: fp32, 2 x 1003 tokens, 8 heads,
+// keeps its inputs and recomputes, the same bits.  So does one under saved-tensor hooks: what these see of a call must not depend on the room that
+// others leave (a checkpointed part that is run again has to save what it saved the first time), nor grow what they move or count.  us a training step with room / without / with keep_forward=False: fp32, 2 x 1003 tokens, 8 heads,
 // K = V = 64 181 / 218 / 224; 2 x 1537 tokens, 8 heads, K = V = 128 195 / 212 / 215; 4 x 1000, 16 heads 379 / 408 / 410.
 constexpr int64_t KEPT_MOST = (int64_t)1 << 30;
 constexpr size_t KEPT_CALLS = 256;
@@ -186,7 +188,7 @@ constexpr int KEPT_DEVICES = 64;
 Tensor kept_room(const Tensor& like, int64_t n) {
     static KeptRoom* const rooms = new KeptRoom[KEPT_DEVICES];    // (never destroyed: tensors may outlive this library's statics)
     const int dev = like.device().index();
-    if (dev < 0 || dev >= KEPT_DEVICES || !rooms[dev].take(n)) return Tensor();
+    if (dev < 0 || dev >= KEPT_DEVICES || !at::SavedTensorDefaultHooks::get_tls_state().stack.empty() || !rooms[dev].take(n)) return Tensor();
     Tensor t;
     try {
         t = bytes_like(like, (size_t)n);

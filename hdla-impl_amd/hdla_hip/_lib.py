@@ -190,8 +190,11 @@ class _NoNative:
 
     def kept_room(self, like, n):
         """Room for a forward workspace that a call holds for its backward pass unasked, or None: KEPT_MOST bytes a device and KEPT_CALLS calls
-        over all whose backward pass is still to come, and what the allocator has (csrc/native.cpp, kept_room)."""
+        over all whose backward pass is still to come, and what the allocator has; none under saved-tensor hooks (csrc/native.cpp,
+        kept_room)."""
         dev, t = like.device.index, None
+        if torch._C._autograd._top_saved_tensors_default_hooks(False) is not None:
+            return None
         with self._lock:
             held = self._held[dev] = [h for h in self._held.get(dev, ()) if h[0]() is not None]
             if sum(h[1] for h in held) + self._coming.get(dev, 0) + n > KEPT_MOST or len(held) >= KEPT_CALLS:

@@ -211,9 +211,9 @@ def test_the_account_of_the_python_code(monkeypatch):
     del b, e
     fresh = lambda: [got(Keep.apply(x, 1000)) for _ in range(2)]
     assert fresh() == [True, True]
-    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.clone(), lambda t: t):
-        h = Keep.apply(x, 1000)
-    assert got(h) and fresh() == [True, True]                    # (the hook's copy is not on it)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t):
+        assert fresh() == [False, False]
+    assert fresh() == [True, True]
     many = [Keep.apply(x, 1) for _ in range(_lib.KEPT_CALLS + 1)]
     assert [got(y) for y in many] == [True] * _lib.KEPT_CALLS + [False]
     del many
@@ -253,6 +253,27 @@ def test_calls_whose_backward_pass_is_to_come_hold_a_gibibyte_at_most(native, mo
         del o
         time.sleep(1e-3)
     assert False, "nothing was given back"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("full", ["first", "again"])
+def test_a_checkpointed_call_saves_the_same_when_it_is_run_again(full, native, monkeypatch):
+    """With the room taken by other calls in one of its two forward passes."""
+    from torch.utils.checkpoint import checkpoint
+    if not native:
+        monkeypatch.setattr(_lib, "_native", _lib._NoNative())
+    T, H, D = 5008, 16, 128
+    x, do, _ = _leaves("ab", 1, T, H, D, D, None, torch.bfloat16)
+    x, do = [t.to(DEV).requires_grad_() for t in x], do.to(DEV)
+    run = lambda *x: chunk_hrdplr_delta_rule(*x[:-1], 2, scale=0.7, initial_state=x[-1])[0]
+    want = torch.autograd.grad(run(*x), x, do)
+    fill = lambda: [run(*x) for _ in range((1 << 30) // _plan(T, H)[0] + 1)]
+    others = fill() if full == "first" else None
+    o = checkpoint(run, *x, use_reentrant=False)
+    others = fill() if full == "again" else None
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(o, x, do), want))
+    del others
 
 
 @pytest.mark.gpu
