@@ -304,17 +304,29 @@ def test_where_the_buffer_cannot_be_had(native, monkeypatch):
 
 
 @pytest.mark.gpu
-def test_rows_of_no_sequence():
-    """A packed batch padded at both ends: the kept pass clears the gradients' rows that no sequence has."""
-    cu = torch.tensor([3, 40, 150], device=DEV)
-    x, do, _ = _leaves("ab", 1, 170, 2, 128, 128, (0, 85, 170), torch.bfloat16)
-    x, do = [t.to(DEV).requires_grad_() for t in x], do.to(DEV)
-    dirty = [torch.full_like(t, float("nan")) for t in x[:6]]    # what the allocator hands out next
-    del dirty
-    o = chunk_hrdplr_delta_rule(*x[:-1], 2, scale=0.7, initial_state=x[-1], cu_seqlens=cu)[0]
-    for i, g in enumerate(torch.autograd.grad(o, x, do)[:6]):
-        r = g.shape[1] // 170
-        assert not g[:, :3 * r].any() and not g[:, 150 * r:].any() and torch.isfinite(g.float()).all(), i
+@pytest.mark.parametrize("segments", [1, 3])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("form", ["ab", "beta"])
+def test_rows_of_no_sequence(form, dtype, segments):
+    """A packed batch padded at both ends: the kept pass clears the gradients' rows that no sequence has, whatever they held."""
+    T, H, K, V = 170, 2, 128, 64
+    cu, plan, P = torch.tensor([3, 40, 150], device=DEV), (_lib.ROUTE_AUTO, segments), _lib.ptr
+    x, do, dht = _leaves(form, 1, T, H, K, V, (0, 85, 170), dtype)
+    x, do, dht = [t.to(DEV) for t in x], do.to(DEV), dht.to(DEV)
+    q, k, v, gk, h0 = x[0], x[1], x[2], x[-2], x[-1]
+    a, b, beta = (*x[3:5], None) if form == "ab" else (None, None, x[3])
+    kept = CK.chunk_hrdplr_fwd(q, k, v, a, b, gk, 0.7, h0, True, cu, keep=True, beta=beta, plan=plan)[2]
+    dims = CK._dims(q, v, gk, 0.7, cu, 2, plan)
+    ws = _lib.workspace(dims, _lib.PASS_BWD_KEPT, q.device)
+    da, db, dbeta = [None if t is None else torch.full_like(t, float("nan")) for t in (a, b, beta)]
+    dq, dk, dv, dgk, dh0 = [torch.full_like(t, float("nan")) for t in (q, k, v, gk, h0)]
+    assert _lib.load().hdla_chunk_bwd_kept(ctypes.byref(dims), P(q), P(k), P(v), P(a), P(b), P(beta), P(gk), P(h0), P(do), P(dht), P(dq), P(dk), P(dv),
+                                           P(da), P(db), P(dbeta), P(dgk), P(dh0), P(kept), kept.numel(), P(ws), ws.numel(),
+                                           _lib.current_stream(q.device)) == 0
+    for i, g in enumerate(t for t in (dq, dk, dv, dgk, da, db, dbeta) if t is not None):
+        r = g.shape[1] // T
+        assert torch.isfinite(g.float()).all() and not g[:, :3 * r].any() and not g[:, 150 * r:].any() and g[:, 3 * r:150 * r].any(), i
+    assert torch.isfinite(dh0).all()
 
 
 @pytest.mark.gpu

@@ -43,12 +43,26 @@ def test_many_tiles_and_refusals():
     assert lib.hdla_weight_grad(2048, 128, 128, P(dy), 128, P(x), 128, P(dw), None, 0, st) == -5
 
 
+@pytest.mark.parametrize("M", [65, 1025, 1030, 2200, 5000])
+@pytest.mark.parametrize("N,K", [(128, 128), (256, 384)])
+def test_every_row_counts_once(M, N, K):
+    """Small whole numbers, most of them zero, whose sums bf16 holds: the bits, at rows that fill neither the last stage nor the last share."""
+    g = torch.Generator().manual_seed(M)
+    dy = (torch.randint(-1, 2, (M, N), generator=g) * (torch.rand(M, N, generator=g) < 0.1)).bfloat16().to(DEV)
+    x = (torch.randint(-1, 2, (M, K), generator=g) * (torch.rand(M, K, generator=g) < 0.1)).bfloat16().to(DEV)
+    dy[-1], x[-1] = 1, 1                                           # (the row that those past the end are read from)
+    want = dy.double().t() @ x.double()
+    assert want.abs().max() <= 256
+    assert torch.equal(_call(dy, x, N, K)[0].double(), want)
+
+
+@pytest.mark.parametrize("M", [100, 1025, 2200])                  # one share; the last one's last stage of one row; several stages
 @pytest.mark.parametrize("value", [float("nan"), float("inf"), -3.3895313892515355e38])
-def test_a_value_that_is_none_stays_in_its_row(value):
+def test_a_value_that_is_none_stays_in_its_row(value, M):
     g = torch.Generator().manual_seed(2)
-    dy, x = torch.randn(100, 256, generator=g).bfloat16().to(DEV), torch.rand(100, 128, generator=g).bfloat16().to(DEV) + 0.5
+    dy, x = torch.randn(M, 256, generator=g).bfloat16().to(DEV), torch.rand(M, 128, generator=g).bfloat16().to(DEV) + 0.5
     clean = _call(dy, x, 256, 128)[0]
-    dy[99, 77] = value                                             # (in the last row, which the rows past the end are read from)
+    dy[M - 1, 77] = value                                          # (in the last row, which the rows past the end are read from)
     dw = _call(dy, x, 256, 128)[0]
     rest = torch.arange(256, device=DEV) != 77
     assert torch.equal(dw[rest], clean[rest])
