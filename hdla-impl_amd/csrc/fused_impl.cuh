@@ -92,7 +92,8 @@ template <typename T, int K, int V, int MODE> struct FusedLds {
     static constexpr int SOLVE = GBOX + (FWD ? CH * GROW : 0);
     static constexpr int SLOT = SOLVE + (SOLVES ? 2 * 32 * FLDP * 4 : 0);
     // int ready[4], consumed[4], abort, -, -, -, part[4], inv[4], strong[4] (per producer pair; see fused_producer), then
-    // two counters of the reverse kernel's consumers (records staged, records used: fused_consumer_rev)
+    // two counters of the reverse kernel's consumers (words 24 and 25; records staged, records used: fused_consumer_rev), -, -, and rest[4]
+    // (fused_producer): all 32 words
     static constexpr int FLAGS = FNP * SLOT;
     // reverse kernel: transition records of the segments to the right, as split operands, for the consumers' chain
     // (CHAIN_STAGE records of K x K at a time: every consumer wave needs them whole, each loads a quarter)
@@ -182,8 +183,8 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
     constexpr BlkF BF = L::BF;
     const ChunkArgs<T>& p = a.c;
     char* slot = smem + pp * L::SLOT;
-    // the pair's scratch: first the other wave's parts of the nine score tiles (fp32, 9 KiB); then, in the same bytes,
-    // A_ab and its inverse for the solve; then the inverse and A_ak as operand tiles for the other wave
+    // the pair's scratch: first the other wave's parts of A_ab's four tiles (fp32, 4 KiB); then, in the same bytes,
+    // A_ab and its inverse for the solve; then the inverse as operand tiles for the other wave
     float *sP, *sN, *sT;
     T* sPub;
     int* const flags = reinterpret_cast<int*>(smem + L::FLAGS);
@@ -1009,7 +1010,6 @@ __device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* 
 #pragma unroll
             for (int i = 0; i < 4; ++i) S[kt][i] = p.h0[soff + (int64_t)(16 * kt + 4 * g + i) * V];
     }
-
 
     for (int t = 0; t < nst; ++t) {
         const int pp = t & (FNP - 1), it = t / FNP;

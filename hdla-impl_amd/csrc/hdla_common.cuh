@@ -244,6 +244,20 @@ __device__ __forceinline__ Frag<bf16> ld_turned(const char* p) {
 // where lane l's piece of a tile in fragment order is, in bytes, for the tile turned
 __device__ __forceinline__ int turned_tile(int l) { return (16 * (l & 3) + (l >> 4) * 4 + ((l >> 2) & 3)) * 8; }
 
+// workgroup barrier that orders LDS accesses only: global loads issued before it may still be outstanding
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// all but the last n of this wave's memory accesses are complete
+template <int N> __device__ __forceinline__ void wait_loads() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0f70);
+    asm volatile("" ::: "memory");
+}
+
 // ---- rows of a tensor into fragments, through LDS -----------------------------------------------------------
 // The lanes of a fragment run over the rows first.  Loaded straight from a row-major tensor an instruction touches 64
 // separate pieces of 8 bytes, and the vector cache's address unit takes them one by one: the fused kernels' waves spent
@@ -503,10 +517,10 @@ constexpr float PASS_CLAMP = 20.f;
 // gi of the token before it, and the second group is the first times e^{m} and e^{gl-m}: three exponentials and lane moves
 // in place of seven.  Products of two factors of the safe range stay inside that of fp32; a tile beyond it (its scores
 // take the strong-decay route) forms the second group directly.  A product carries one rounding of 2^-24 more than an exponential,
-// and the backward kernels form their factors directly: beside operands of 8 bits neither is seen.  Errors against a float64
-// evaluation, mean of 12 training steps of 4 x 512 tokens, 16 heads, relative to those with every factor an exponential of its own:
-// 1.0000 (outputs), 0.9999 to 1.0002 (final state, gradients), standard errors up to 0.0002; the products save 1.3 us of a training
-// step of 4 x 2048 tokens and 0.3 us of a forward pass.
+// which beside operands of 8 bits is not seen.  All kernels take their factors so: fused producers, prep, chunk_grad.  Errors against a float64
+// evaluation, relative to a build with every factor an exponential of its own, mean of 10 training steps of 2 x 256 tokens, outputs, final state and all
+// gradients: K = V = 64, 8 heads (fused) 0.9997 to 1.0001, K = V = 128, 4 heads (classic) 0.9995 to 1.0000, with sixteen times the decay 0.9999 to 1.0001;
+// standard errors up to 0.0004.  The products save 1.3 us of a training step of 4 x 2048 tokens and 0.3 us of a forward pass.
 // Measured on 8192 tokens x 16 heads, K = V = 64 (with the producers' reordering in the fused kernels that came with it):
 // forward 75.2 -> 73.8 us, checkpoints 78.6 -> 76.1, reverse 70.7 -> 69.0.
 constexpr float LOG2E = 1.44269504088896340736f;

@@ -779,7 +779,9 @@ void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, Plan& p
 
 // dW [n, k] = dY [rows, n]^T X [rows, k].  Up to one round of whole 128 x 128 tiles on the device by the library's own kernel (us
 // within a training step: 8192 rows, 3328 x 1024 102 -> 82, 1024 x 1024 33 -> 30; 4000 rows, 2048 x 2048 56 -> 44; 1500 rows, 3328 x 1024 30 -> 17; but
-// 4000 rows, 6656 x 2048, 832 tiles: 128 and 147).  Others: an output of few tiles would leave most of the chip idle (1024 x 1024 over 8192 rows: 54 us), so the rows are split over a batch
+// 4000 rows, 6656 x 2048, 832 tiles: 128 and 147).  The line: one call behind the other, 16 to 8192 rows, 2 to 256 tiles are all faster (4096 rows, 256 tiles
+// 44 -> 38), but a second round of workgroups for a few tiles costs what it gains: 288 tiles, 1000 / 2048 / 4096 / 8192 rows 27 -> 23, 33 -> 35, 59 -> 62,
+// 114 -> 115; 512 tiles 29 -> 30, 39 -> 43, 68 -> 75, 130 -> 135.  Others: an output of few tiles would leave most of the chip idle (1024 x 1024 over 8192 rows: 54 us), so the rows are split over a batch
 // of products whose fp32 results one kernel adds (28 + 4 us).
 Tensor weight_grad(const Tensor& dy, const Tensor& x) {
     const int64_t rows = dy.size(0), n = dy.size(1), k = x.size(1);

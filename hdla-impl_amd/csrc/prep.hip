@@ -497,7 +497,8 @@ __global__ __launch_bounds__(TABLE_THREADS) void clear_uncovered_kernel(const in
 // narrower workgroup helps it; of these the one whose longest walk, or whose work spread over the slots, is least.  (Column blocks never meet: the
 // results have the same bits in every width.)  Times of a step of 4, 2 and
 // 1 blocks, 10 ns, one sequence of 16 heads alone on the device, K = V = 128: forward 81, 60, 58, both scans 105, 87, 78 (K = 64: 42, 35, 34; 59,
-// 51, 45); the choice needs their ratios only.
+// 51, 45); the choice needs their ratios only, and with K = 128's it is at K = 64 as good as with its own (1203 random batches: 0.4 and 0.3 % over the best
+// of its candidates on average, 14 and 13 % at the most).
 constexpr float SHARE_STEP[2][3] = {{81.f, 60.f, 58.f}, {105.f, 87.f, 78.f}}, SHARE_PROLOGUE = 6.f;
 // More workgroups than slots leave gaps behind them.  Over 1500 random batches of 2 to 14 sequences, the choice against the best of its candidates with the
 // workgroups dealt out one by one: 0.3 % on average, 12 % at the most (without the factor 0.8 and 41 %; one width for all 17 and 40 %).

@@ -25,13 +25,6 @@
 
 namespace hdla {
 
-// workgroup barrier that orders LDS accesses only: global loads issued before it may still be outstanding
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 constexpr int NSLOT = 3;
 
 template <typename T, int K, int V, int NWC> struct ScanCfg {

@@ -49,13 +49,6 @@ template <int K, int V, int NWC, ScanOut OUT> struct OutCfg {
     static constexpr int OUTBOX = SLOTS * SLOT, UBUF = OUTBOX + 2 * OB, XBUF = UBUF + 2 * UB, BYTES = XBUF + 2 * XB;
 };
 
-// all but the last n of this wave's memory accesses are complete
-template <int N> __device__ __forceinline__ void wait_loads() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0f70);
-    asm volatile("" ::: "memory");
-}
-
 // OUT_O: with the output; OUT_STATE: the forward scan of the backward pass, which leaves the state that enters each chunk; OUT_SUM:
 // records of segments.
 // KEPT: on a workspace of the backward pass (or that it will read, PREP_KEEP): u and v^T are there, and b^T's pairs are of two channel

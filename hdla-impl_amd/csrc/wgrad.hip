@@ -36,16 +36,6 @@ constexpr int WG_OPERAND = WG_ROWS * WG_TILE * 2, WG_STAGE = 2 * WG_OPERAND;
 constexpr int WG_LOADS = WG_STAGE / 1024 / WG_LOADERS;
 static_assert(WG_SLOTS * WG_STAGE <= 160 * 1024 && (WG_SLOTS - 1) * WG_LOADS < 63, "what LDS holds; the memory counter's range");
 
-template <int N> __device__ __forceinline__ void wait_loads_but() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0f70);
-    asm volatile("" ::: "memory");
-}
-__device__ __forceinline__ void wg_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 __device__ __forceinline__ int wg_turn(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
 
 __global__ __launch_bounds__(64 * (WG_LOADERS + WG_COMPUTE)) void weight_grad_kernel(WeightGradArgs p) {
@@ -88,17 +78,17 @@ __global__ __launch_bounds__(64 * (WG_LOADERS + WG_COMPUTE)) void weight_grad_ke
         };
 #pragma unroll
         for (int t = 0; t < WG_SLOTS; ++t) load(min(t, stages - 1));
-        wait_loads_but<(WG_SLOTS - 1) * WG_LOADS>();
+        wait_loads<(WG_SLOTS - 1) * WG_LOADS>();
         if (whole == 0) clear(0);
-        wg_barrier();
+        lds_barrier();
         for (int t = 0; t + 1 < stages; ++t) {
-            wait_loads_but<(WG_SLOTS - 2) * WG_LOADS>();          // stage t + 1
+            wait_loads<(WG_SLOTS - 2) * WG_LOADS>();          // stage t + 1
             if (t + 1 >= whole) clear(t + 1);
-            wg_barrier();
+            lds_barrier();
             load(min(t + WG_SLOTS, stages - 1));                  // where stage t was
         }
-        wait_loads_but<0>();                                      // nothing may arrive where the sums go
-        wg_barrier();
+        wait_loads<0>();                                      // nothing may arrive where the sums go
+        lds_barrier();
         return;
     }
 
@@ -139,12 +129,12 @@ __global__ __launch_bounds__(64 * (WG_LOADERS + WG_COMPUTE)) void weight_grad_ke
             for (int j = 0; j < 4; ++j) acc[i][j] = mm2(f.n[i][0], f.n[i][1], f.k[j][0], f.k[j][1], acc[i][j]);
     };
     Frags f[2];
-    wg_barrier();
+    lds_barrier();
     read(0, f[0]);
     int slot = 0;
     auto stage = [&](const Frags& now, Frags& next) __attribute__((always_inline)) {
         slot = slot + 1 == WG_SLOTS ? 0 : slot + 1;
-        wg_barrier();                                             // the next stage is there; this one has been read by all
+        lds_barrier();                                             // the next stage is there; this one has been read by all
         read(slot, next);
         __builtin_amdgcn_sched_barrier(0);
         multiply(now);
@@ -156,13 +146,13 @@ __global__ __launch_bounds__(64 * (WG_LOADERS + WG_COMPUTE)) void weight_grad_ke
     }
     stage(f[0], f[1]);
     multiply(f[1]);
-    wg_barrier();
+    lds_barrier();
     f32x4* const sums = reinterpret_cast<f32x4*>(smem) + (wv & 3) * 1024 + l;
     if (half) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) sums[i * 64] = acc[i / 4][i % 4];
     }
-    wg_barrier();
+    lds_barrier();
     if (half) return;
     const long long first = (long long)(n0 + 64 * nq) * p.K + k0 + 64 * kq;
 #pragma unroll
