@@ -278,6 +278,27 @@ def test_a_checkpointed_call_saves_the_same_when_it_is_run_again(full, native, m
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("form", ["ab", "beta"])
+@pytest.mark.parametrize("T,H,K,V,cu,dtype,plan", [
+    (1024, 4, 128, 64, None, torch.bfloat16, (8, 1)), (2048, 8, 128, 128, None, torch.bfloat16, (8, 8)), (700, 12, 128, 128, None, torch.bfloat16, (1, 1)),
+    (3000, 2, 128, 64, (0, 1700, 3000), torch.bfloat16, (8, 8)), (256, 2, 64, 64, None, torch.bfloat16, (1, 1)),
+    (500, 6, 64, 64, None, torch.float32, (8, 8)), (250, 16, 128, 128, None, torch.float32, (4, 4)), (200, 16, 128, 128, None, torch.float32, (1, 1))])
+def test_the_librarys_own_plan_kept_and_not(T, H, K, V, cu, dtype, plan, form, native, monkeypatch):
+    """Nothing is kept under saved-tensor hooks: what is computed is the same, whichever segments the library chooses."""
+    if not native:
+        monkeypatch.setattr(_lib, "_native", _lib._NoNative())
+    assert _plan(T, H, K, V, dtype, None if cu is None else len(cu) - 1)[1:] == plan
+    x, do, dht = _leaves(form, 1, T, H, K, V, cu, dtype, gk_div=64.0)
+    x, do, dht = [t.to(DEV).requires_grad_() for t in x], do.to(DEV), dht.to(DEV)
+    table = None if cu is None else torch.tensor(cu, device=DEV)
+    got, saved = _grads(form, x, do, dht, table, None), []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: saved.append(t.dtype) or t, lambda t: t):
+        again = _grads(form, x, do, dht, table, None)
+    assert torch.uint8 not in saved and all(torch.equal(a, b) for a, b in zip(got, again))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("native", [True, False])
 def test_where_the_buffer_cannot_be_had(native, monkeypatch):
     """A limit of torch's allocator between what the call needs and what it would keep: it runs, and so does its backward pass later."""
     if not native:
