@@ -219,7 +219,7 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
                 for (int r0 = 0; r0 < NR; r0 += RPI) {
                     const int r = rb + r0 + l / LPR, e = (l % LPR) * 16;
                     const i32x4 x = *reinterpret_cast<const i32x4*>(slot + L::OBOX + r * L::OROW + e);
-                    if (r < len) *reinterpret_cast<i32x4*>(reinterpret_cast<char*>(p.o + ((tok0 + r) * H + h) * V) + e) = x;
+                    if (r < len) st_past(reinterpret_cast<i32x4*>(reinterpret_cast<char*>(p.o + ((tok0 + r) * H + h) * V) + e), x);
                 }
             } else {
                 // in the order in which fixup_kernel takes them: 1-KiB pieces, lane (g, c) has columns 16 j + 4 g .. + 3 of o's row c, and
@@ -1226,7 +1226,7 @@ __device__ __forceinline__ void fused_consumer_ckpt(const FusedArgs<T>& a, char*
         const Frag<T> vnb[2] = {to_frag<T>(vn[0]), to_frag<T>(vn[1])};
         T* hc = p.ws.HC + chw * (K * V) + vt * PAIR;
 #pragma unroll
-        for (int kp = 0; kp < KT2; ++kp) st_pair2(hc + kp * (VT * PAIR), sb[2 * kp], sb[2 * kp + 1]);
+        for (int kp = 0; kp < KT2; ++kp) st_pair2_past(hc + kp * (VT * PAIR), sb[2 * kp], sb[2 * kp + 1]);
         if (W_GLOBAL) {
             static_assert(2 * KT2 == VT, "one pair of w per consumer");
             st_pair2(p.ws.UT + (chw * VT + vt) * PAIR, ut[0], ut[1]);
@@ -1413,8 +1413,8 @@ __device__ __forceinline__ void fused_consumer_rev(const FusedArgs<T>& a, char* 
         T* dhc = p.ws.DHC + chw * (K * V) + vt * PAIR;
         T* dvp = p.ws.DVN + chw * (2 * CH * V) + vt * PAIR;
 #pragma unroll
-        for (int kp = 0; kp < KT2; ++kp) st_pair2(dhc + kp * (VT * PAIR), dsb[2 * kp], dsb[2 * kp + 1]);
-        st_pair2(dvp, dvb[0], dvb[1]);
+        for (int kp = 0; kp < KT2; ++kp) st_pair2_past(dhc + kp * (VT * PAIR), dsb[2 * kp], dsb[2 * kp + 1]);
+        st_pair2_past(dvp, dvb[0], dvb[1]);
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) dS[kt] = mm2(dvb[0], dvb[1], wt[0][kt], wt[1][kt], x[2 + kt]);
         signal_add(&flags[4 + pp]);
@@ -1643,7 +1643,7 @@ __global__ __launch_bounds__(256) void fixup_kernel(FusedArgs<T> a) {
                 for (int r0 = 0; r0 < CH; r0 += RPI) {
                     const int r = r0 + l / LPR, e = (l % LPR) * 16;
                     const i32x4 x = *reinterpret_cast<const i32x4*>(st + r * OROW + e);
-                    if (r < len) *reinterpret_cast<i32x4*>(reinterpret_cast<char*>(p.o + ((tok0 + r) * H + h) * V) + e) = x;
+                    if (r < len) st_past(reinterpret_cast<i32x4*>(reinterpret_cast<char*>(p.o + ((tok0 + r) * H + h) * V) + e), x);
                 }
             }
         }

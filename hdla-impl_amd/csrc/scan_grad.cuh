@@ -241,7 +241,7 @@ __device__ __forceinline__ void scan_rev_body(const ChunkArgs<bf16>& p, char* sm
             if constexpr (!SUM) {
                 T* const dhc = p.ws.DHC + chw * (K * V) + (part * KH2 * VT + vt) * PAIR;
 #pragma unroll
-                for (int kp = 0; kp < KH2; ++kp) st_pair2(dhc + kp * VT * PAIR, dsb[2 * kp], dsb[2 * kp + 1]);
+                for (int kp = 0; kp < KH2; ++kp) st_pair2_past(dhc + kp * VT * PAIR, dsb[2 * kp], dsb[2 * kp + 1]);
             }
             // ---- what is one product a sum: the chunk's own part of the state's gradient
             f32x4 x[KH];
@@ -271,7 +271,7 @@ __device__ __forceinline__ void scan_rev_body(const ChunkArgs<bf16>& p, char* sm
             // ---- dS <- exp(g_last) dS + qg^T do + sum_s w_s^T dv_new_s
 #pragma unroll
             for (int k = 0; k < KH; ++k) dS[k] = mm2(dvb[0], dvb[1], wt[0][k], wt[1][k], x[k]);
-            if constexpr (!SUM && first) st_pair2(p.ws.DVN + chw * (2 * CH * V) + vt * PAIR, dvb[0], dvb[1]);
+            if constexpr (!SUM && first) st_pair2_past(p.ws.DVN + chw * (2 * CH * V) + vt * PAIR, dvb[0], dvb[1]);
             __builtin_amdgcn_sched_barrier(0);
             read_rest(so);
         }

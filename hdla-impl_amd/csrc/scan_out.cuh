@@ -204,7 +204,7 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
                     const int r = r0 + l / LPR, e = (l % LPR) * 16;
                     if (r < len) {
                         const i32x4 x = *reinterpret_cast<const i32x4*>(ob + r * C::OROW + e);
-                        *reinterpret_cast<i32x4*>(reinterpret_cast<char*>(p.o + ((tok0 + r) * H + h) * V + 16 * vt0) + e) = x;
+                        st_past(reinterpret_cast<i32x4*>(reinterpret_cast<char*>(p.o + ((tok0 + r) * H + h) * V + 16 * vt0) + e), x);
                     }
                 }
             }
@@ -309,7 +309,7 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
                 // chunk_grad kernel turns them the way it needs them
                 T* const hc = p.ws.HC + (chw0 + t) * (K * V) + (part * KH2 * (V / 16) + vt) * PAIR;
 #pragma unroll
-                for (int kp = 0; kp < KH2; ++kp) st_pair2(hc + kp * (V / 16) * PAIR, sb[2 * kp], sb[2 * kp + 1]);
+                for (int kp = 0; kp < KH2; ++kp) st_pair2_past(hc + kp * (V / 16) * PAIR, sb[2 * kp], sb[2 * kp + 1]);
             }
             // ---- what is one product a sum: the chunk's own part of the state, A_qk v
             f32x4 x[KH + 1];
