@@ -44,7 +44,8 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
     constexpr int MAT = 32 * LDP;
     static_assert(NPART * 256 <= 2 * MAT, "");
     __shared__ __attribute__((aligned(16))) float sMat[NWP][2 * MAT];
-    __shared__ __attribute__((aligned(16))) char sRows[NWP][ROWS_SCRATCH];   // rows on their way to fragments
+    // rows on their way to fragments; 4-byte elements: tiles that are turned
+    __shared__ __attribute__((aligned(16))) char sRows[NWP][sizeof(T) == 4 ? TURN_SCRATCH : ROWS_SCRATCH];
     __shared__ float sSum[NWP * CH];
     __shared__ int sStrong[NWP];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -190,12 +191,12 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
             const TileDecay<T> d(in[e].g, c);
             strong |= d.strong;
             qg[e] = to_frag<T>(to_f32(in[e].q) * d.egi * scale);
-            kgT[e] = transpose(to_frag<T>(to_f32(in[e].k) * d.edn), ident);
+            kgT[e] = turn(to_frag<T>(to_f32(in[e].k) * d.edn), ident, scratch);
 #pragma unroll
             for (int r = 0; r < 2; ++r) {
                 ag[r][kt] = to_frag<T>(to_f32(in[e].a[r]) * d.ege);
                 if (TIGHT) hold(ag[r][kt]);                          // formed here, not where it is used: that would keep a and its factors instead
-                bgT[r][e] = transpose(to_frag<T>(to_f32(in[e].b[r]) * d.edn), ident);
+                bgT[r][e] = turn(to_frag<T>(to_f32(in[e].b[r]) * d.edn), ident, scratch);
             }
             // (the same from all tokens' lanes: without a branch in the way of the scheduler)
             *reinterpret_cast<f32x4*>(p.ws.EGL + chw * (SAS * (int)sizeof(T) / 4) + 16 * (kt0 + kt) + 4 * g) = d.egl;
@@ -236,7 +237,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
             else st_pair2(p.ws.BGT + chw * SAS + (s * KT2 + pair) * PAIR, bgT[s][0], bgT[s][1]);
         }
         if (!BWD) st_pair2(p.ws.QG + chw * SAS + pair * PAIR, qg[0], qg[1]);
-        if (WB) st_pair2(p.ws.QGT + chw * SBS + pair * PAIR, transpose(qg[0], ident), transpose(qg[1], ident));
+        if (WB) st_pair2(p.ws.QGT + chw * SBS + pair * PAIR, turn(qg[0], ident, scratch), turn(qg[1], ident, scratch));
     }
     // Each wave decides for its own channels (the parts of the score tiles add up whichever way they were formed); the
     // backward pass records the decision per (chunk, head) for the chunk_grad kernels.  Where a channel decays too
@@ -330,7 +331,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
         if (BWD || WB) {
             // the other orientation is the rounded tile turned (a product with the identity: exact), in every mode, so
             // that a backward pass finds the same bytes whether it recomputes them or reads what a forward pass kept
-            st_pair2(p.ws.AQBT + chw * SBS, transpose(to_frag<T>(aqb[0]), ident), transpose(to_frag<T>(aqb[1]), ident));
+            st_pair2(p.ws.AQBT + chw * SBS, turn(to_frag<T>(aqb[0]), ident, scratch), turn(to_frag<T>(aqb[1]), ident, scratch));
         }
     }
 #pragma unroll
@@ -402,7 +403,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
         // for the chunk_grad kernel: the four blocks transposed, as fragments (two tile pairs), ready to load
         T* tmw = p.ws.TM + chw * 1024;
 #pragma unroll
-        for (int s = 0; s < 2; ++s) st_pair2(tmw + s * PAIR, transpose(tm[s][0], ident), transpose(tm[s][1], ident));
+        for (int s = 0; s < 2; ++s) st_pair2(tmw + s * PAIR, turn(tm[s][0], ident, scratch), turn(tm[s][1], ident, scratch));
     }
 
     // ---- phase C: w = Tm ag, two channel tiles (one stored pair) at a time ---------------------------------------
@@ -411,7 +412,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
         Frag<T> fw[2][2];                                     // [..][tile of the pair]
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-            const Frag<T> agT[2] = {transpose(ag[0][2 * kp + e], ident), transpose(ag[1][2 * kp + e], ident)};
+            const Frag<T> agT[2] = {turn(ag[0][2 * kp + e], ident, scratch), turn(ag[1][2 * kp + e], ident, scratch)};
 #pragma unroll
             for (int s = 0; s < 2; ++s) fw[s][e] = to_frag<T>(mm2(tm[s][0], tm[s][1], agT[0], agT[1], zero4()));
         }
@@ -435,7 +436,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
     for (int vl = 0; vl < VTW; ++vl) {
         const int vt = vt0 + vl;
         if (vl % 2 == 0) lv[vl / 2].tiles(scratch, cp.len, l, rv);
-        const Frag<T> vT = transpose(rv[vl % 2], ident);
+        const Frag<T> vT = turn(rv[vl % 2], ident, scratch);
         st_tile(p.ws.VTT + (chw * VT + vt) * TILE, vT);
         const Frag<T> mT[2] = {to_frag<T>(mm(vT, aakf[0], zero4())), to_frag<T>(mm(vT, aakf[1], zero4()))};
         Frag<T> fu[2];
