@@ -175,6 +175,7 @@ __device__ __forceinline__ void scan_rev_body(const ChunkArgs<bf16>& p, char* sm
     }
     auto walk = [&](auto part_) __attribute__((always_inline)) {
         constexpr int part = decltype(part_)::value, kt0 = part * KH;
+        constexpr bool ALONE = NWC == 1 && PARTS > 1;
         constexpr bool first = part == 0, from_do = part == PARTS - 1;   // the wave that stores dv_new, and the one that starts it from do
         Frag<T> bg[2][KH], wt[2][KH], qgt[KH], doT;
         f32x4 egl[KH], e[2];
@@ -251,6 +252,7 @@ __device__ __forceinline__ void scan_rev_body(const ChunkArgs<bf16>& p, char* sm
                 *reinterpret_cast<f32x4*>(xt + part * 2048) = dvn[0];
                 *reinterpret_cast<f32x4*>(xt + part * 2048 + 1024) = dvn[1];
             }
+            if constexpr (ALONE) __builtin_amdgcn_sched_barrier(0);       // (x in front of the barrier, as in scan_out.cuh)
             // the parts are there; so are step t + 1's block and do, and step t's has been read by all
             lds_barrier();
             f32x4 ov[2];
@@ -262,7 +264,7 @@ __device__ __forceinline__ void scan_rev_body(const ChunkArgs<bf16>& p, char* sm
             read_do(t + 1);
             read_first(so);
             __builtin_amdgcn_sched_barrier(0);
-            settle<T>(x);
+            if constexpr (!ALONE) settle<T>(x);
             if constexpr (PARTS > 1) {
                 dvn[0] += ov[0];
                 dvn[1] += ov[1];

@@ -16,7 +16,7 @@
 //    of v (in the computing waves it cost 0.14 us a step: a chain of five dependent products).  The kernel that prepares the
 //    chunks does not read v and writes 3 KB instead of u and v^T, 12 KB of its 70 a chunk and head at K = V = 128: 236 -> 192 us for 16384
 //    tokens of 16 heads.  The products and roundings are the ones it had.
-// Measured, us, before -> after, 2048 tokens a sequence: K = V = 128, 16 heads 88 -> 73, 32 heads 92 -> 79, 64 heads 105 -> 101, 128 heads
+// Measured, us, before -> after (when it was built), 2048 tokens a sequence: K = V = 128, 16 heads 88 -> 73, 32 heads 92 -> 79, 64 heads 105 -> 101, 128 heads
 // 167 -> 146; K = 64, V = 128, 128 heads 116 -> 98; K = 128, V = 64, 32 heads 87 -> 72.  From 48 heads on a step waits for its loads: 82 us
 // of the 101 where they never leave the L2, 70 without them; touching the blocks' lines 12 chunks ahead made it 105.
 #pragma once
@@ -235,6 +235,12 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
     // The walk, compiled for each part by itself: a wave alone on its SIMD pays some five cycles for every instruction, branches more
     auto walk = [&](auto part_) __attribute__((always_inline)) {
         constexpr int part = decltype(part_)::value, kt0 = part * KH;
+        // Two waves of one column block: each has its SIMD to itself, and a step is its chain of latencies: 960 cycles, of them 200 until the parts are on
+        // their way into LDS, 140 to the barrier, 270 until v_new is there, 350 for the products.  Left to itself the compiler put the products of x and of
+        // o before those that the next step waits for.  Measured, us for the scan, before -> after, the same bits: K = V = 128, 97 chunks, 16 heads 44.3 -> 41.6,
+        // 44, 8 heads 22.3 -> 21.2; K = 128, V = 64, 63 chunks, 16 heads 30.0 -> 28.3; both backward scans 45 -> 43, 22.9 -> 20.4, 30.5 -> 29.3.  With two blocks,
+        // or at K = 64, it was the same time.  Four waves a block (a channel tile pair each) took 47: the parts of four have to be read and added.
+        constexpr bool ALONE = NWC == 1 && PARTS > 1;
         constexpr bool first = part == 0, from_u = part == PARTS - 1;   // the wave with the output, and the one that starts v_new from u
         // A chunk's operands, read as soon as the chunk before has been through with their registers: half a step and more before they are used
         Frag<T> w[2][KH], qg[WITH_O ? KH : 1], kgt[KH], bgt[2][KH], aqk, aqb[2], ut[2], vtt;
@@ -322,6 +328,9 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
                 *reinterpret_cast<f32x4*>(xt + part * 2048 + 1024) = vn[1];
                 if constexpr (WITH_O && !first) *reinterpret_cast<f32x4*>(xt + 4096) = o;
             }
+            // (alone on its SIMD, a wave has the products of x issued in front of the barrier, while the parts are on their way into LDS, and those of S in
+            // front of o's: see ALONE)
+            if constexpr (ALONE) __builtin_amdgcn_sched_barrier(0);
             // the parts are there; so are chunk t + 1 and its u, and chunk t has been read by all
             lds_barrier();
             f32x4 ov[2], oo;
@@ -334,7 +343,7 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
             read_u(t + 1);
             read_first(so);
             __builtin_amdgcn_sched_barrier(0);
-            settle<T>(x);
+            if constexpr (!ALONE) settle<T>(x);
             if constexpr (PARTS > 1) {
                 vn[0] += ov[0];
                 vn[1] += ov[1];
@@ -343,6 +352,7 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
             // ---- S <- exp(g_last) S + kg^T v + sum_s bg_s^T v_new_s
 #pragma unroll
             for (int k = 0; k < KH; ++k) S[k] = mm2(vnb[0], vnb[1], bgt[0][k], bgt[1][k], x[k]);
+            if constexpr (ALONE) __builtin_amdgcn_sched_barrier(0);
             if constexpr (WITH_O && first) {
                 // o (rows token, inner value) = A_qk v + qg S + sum_s A_qb^s v_new_s
                 if constexpr (PARTS > 1) o += oo;
