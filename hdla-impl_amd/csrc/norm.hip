@@ -49,10 +49,8 @@ template <> struct Piece<bf16> {
         }
     }
     static __device__ __forceinline__ void st(void* base, long long elem, const float (&f)[8]) {
-        u32x4 r;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) r[i] = (uint32_t)f2bf(f[2 * i]) | ((uint32_t)f2bf(f[2 * i + 1]) << 16);
-        __builtin_nontemporal_store(r, reinterpret_cast<u32x4*>(static_cast<bf16*>(base) + elem));
+        const s16x4 lo = to_frag<bf16>(f32x4{f[0], f[1], f[2], f[3]}).v, hi = to_frag<bf16>(f32x4{f[4], f[5], f[6], f[7]}).v;
+        __builtin_nontemporal_store(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7), reinterpret_cast<s16x8*>(static_cast<bf16*>(base) + elem));
     }
 };
 template <> struct Piece<float> {
@@ -128,7 +126,15 @@ struct NormLane {
 // the workgroup makes the same calls.
 __device__ __forceinline__ void group_sum(const NormLane& L, float& a, float& b, float* sred, int& buf) {
     const int width = L.wg_row ? 64 : L.lpr;
-    for (int o = 1; o < width; o <<= 1) { a += __shfl_xor(a, o); b += __shfl_xor(b, o); }
+    // butterflies on the vector ALU: within 16 lanes by DPP (the mirrors meet sums that are the same on four, or eight, neighbours), beyond by swaps
+    // of rows of lanes.  The sums are those of __shfl_xor, which goes through LDS; us, that -> this: 8192 x 1024 bf16 11.7 + 21.3 -> 11.2 + 20.4,
+    // 65536 x 4096 364 + 621 -> 350 + 605.
+    if (width > 1) { a += dpp0<0xB1>(a); b += dpp0<0xB1>(b); }
+    if (width > 2) { a += dpp0<0x4E>(a); b += dpp0<0x4E>(b); }
+    if (width > 4) { a += dpp0<0x141>(a); b += dpp0<0x141>(b); }
+    if (width > 8) { a += dpp0<0x140>(a); b += dpp0<0x140>(b); }
+    if (width > 16) { a += xor16(a); b += xor16(b); }
+    if (width > 32) { a += xor32(a); b += xor32(b); }
     if (L.wg_row) {
         float* s = sred + buf * 8;
         if ((threadIdx.x & 63) == 0) { s[2 * (threadIdx.x >> 6)] = a; s[2 * (threadIdx.x >> 6) + 1] = b; }
@@ -257,7 +263,25 @@ __global__ __launch_bounds__(256) void normalize_bwd_kernel(NormArgs p) {
 #pragma unroll
         for (int j = 0; j < N; ++j) dw[i][j] = 0.f;
     }
+    // A workgroup that shares its groups meets four times as many as a wavefront would: the weight gradient's sums of FOLD of them are added to those of
+    // the ones before in the lane's own place in LDS, so that no sum is longer than it was (fp32 20000 x 1024, error 1.93e-7; one sum of 20: 2.06e-7).
+    constexpr int FOLD = 4;
+    __shared__ float sdw[NV * N * 256];
+    int folded = 0, met = 0;
     for (long long sg = L.wave; sg < p.nsg; sg += L.nwave) {
+        if (has_w && L.wg_row && met == FOLD) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+#pragma unroll
+                for (int j = 0; j < N; ++j) {
+                    float* const at = sdw + (i * N + j) * 256 + threadIdx.x;
+                    *at = folded ? *at + dw[i][j] : dw[i][j];
+                    dw[i][j] = 0.f;
+                }
+            folded = 1;
+            met = 0;
+        }
+        ++met;
         const long long slot = sg * L.rpw + L.rw;
         const bool live = slot < p.nslot;
         if (!AHEAD) request(sg);
@@ -315,10 +339,16 @@ __global__ __launch_bounds__(256) void normalize_bwd_kernel(NormArgs p) {
         }
     }
     if (has_w) {
+        if (folded) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+#pragma unroll
+                for (int j = 0; j < N; ++j) dw[i][j] += sdw[(i * N + j) * 256 + threadIdx.x];
+        }
         long long prow = L.wave * L.rpw + L.rw;
         if (p.wg_reduce) {
             // lane by lane the four wavefronts hold the same columns: waves 2, 3 hand over to 0, 1, then 1 to 0
-            __shared__ float swg[2 * NV * N * 64];
+            float* const swg = sdw;                       // [2][NV * N][64]
             const int wl = threadIdx.x >> 6, lane = threadIdx.x & 63;
 #pragma unroll
             for (int round = 0; round < 2; ++round) {
@@ -393,6 +423,10 @@ struct NormCfg {
 
 static long long gcd_ll(long long a, long long b) { while (b) { const long long t = a % b; a = b; b = t; } return a; }
 
+// The backward kernel of 2-byte elements with two pieces a lane: its registers leave room for three workgroups a compute unit, and a fourth on all of them
+// would come in a round of its own.  us, 1024 workgroups -> as many as are resident, evenly filled: 20000 x 1024 43.0 -> 38.8, 65536 x 4096 548 -> 516.
+// (The forward kernel, and 4-byte elements, were the same or slower so.)
+constexpr long long NORM_RESIDENT = 3 * 256;
 static int norm_config(const hdla_norm_dims* d, bool bwd, NormCfg& c) {
     if (!d) return HDLA_ERR_NULL;
     if (d->dtype != HDLA_BF16 && d->dtype != HDLA_FP32) return HDLA_ERR_DTYPE;
@@ -405,9 +439,10 @@ static int norm_config(const hdla_norm_dims* d, bool bwd, NormCfg& c) {
     if (pieces > 256 * 8) return HDLA_ERR_SHAPE;                // a group lives in one workgroup's registers
     if (d->rows > (1LL << 40) / d->G) return HDLA_ERR_SHAPE;
     c.nslot = d->rows * d->G;
-    // long groups always, and groups of at least 128 pieces when there are too few of them to fill the chip one
-    // wavefront each (a decode step: a few hundred rows)
-    c.wg_row = pieces > 64 * 8 || (pieces >= 128 && c.nslot <= 2048);
+    // groups of more than two pieces a lane, whose wavefronts would have the registers of few, and of two when there are too few of them
+    // to fill the chip one wavefront each (a decode step: a few hundred rows).  us, both passes, one wavefront a group -> four: bf16 65536 x 4096 1000 -> 838,
+    // 10000 x 4096 202 -> 135, 20000 x 2048 130 -> 122; fp32 5000 x 2048 81 -> 68, 20000 x 1024 124 -> 115, 30000 x 2048 362 both.
+    c.wg_row = pieces > 64 * 2 || (pieces >= 128 && c.nslot <= 2048);
     if (c.wg_row) {
         // one group per workgroup pass, 256 lanes across it
         c.nv = 1;
@@ -431,6 +466,10 @@ static int norm_config(const hdla_norm_dims* d, bool bwd, NormCfg& c) {
     long long nwg = (c.nsg + owners * per_wave - 1) / (owners * per_wave);
     if (nwg < 1) nwg = 1;
     if (nwg > cap) nwg = cap;
+    if (bwd && d->dtype == HDLA_BF16 && c.nv == 2 && nwg > NORM_RESIDENT) {
+        const long long passes = (c.nsg + owners * NORM_RESIDENT - 1) / (owners * NORM_RESIDENT);
+        nwg = (c.nsg + owners * passes - 1) / (owners * passes);
+    }
     const long long m = d->G / gcd_ll(d->G, owners * c.rpw);
     if (m > 65536) return HDLA_ERR_SHAPE;
     c.nwg = (nwg + m - 1) / m * m;
