@@ -258,6 +258,12 @@ __device__ __forceinline__ void st_pair2(float* pair, Frag<float> f0, Frag<float
 // 191 -> 183.  Not so: what prep leaves (packed prefill of 5003 tokens 121 -> 132), local outputs and G of the fused forward kernel (fixup 12 -> 15), the
 // checkpoints' loads, which two waves make each (chunk_grad at K = V = 128 520 -> 655), the inputs' last loads (nothing at K = 64, 1696 -> 1714).
 template <typename X> __device__ __forceinline__ void st_past(X* p, X x) { __builtin_nontemporal_store(x, p); }
+// The other side of a branch beside st_past: the compiler makes one store of the two otherwise, and that an ordinary one.
+template <typename X> __device__ __forceinline__ void st_near(X* p, X x) {
+    __builtin_amdgcn_sched_barrier(0);
+    *p = x;
+    __builtin_amdgcn_sched_barrier(0);
+}
 __device__ __forceinline__ void st_pair2_past(bf16* pair, Frag<bf16> f0, Frag<bf16> f1) {
     st_past(reinterpret_cast<s16x8*>(pair + 8 * lane_id()), __builtin_shufflevector(f0.v, f1.v, 0, 1, 2, 3, 4, 5, 6, 7));
 }

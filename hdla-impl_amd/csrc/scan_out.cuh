@@ -190,6 +190,10 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
                 if (t0 + j < nchunks) step(t0 + j, own[(j + 1) % UD]);
             if (WITH_O) lds_barrier();
         } else if constexpr (WITH_O) {
+            // Outputs past the caches from 4 MiB a call on, an XCD's L2: below, the blocks' parts of a line meet there, and the kernel's end does not wait
+            // for memory.  Calls in us, past -> near: 2 x 28 and 2 x 100 tokens of 12 heads, K = V = 128, 13.6 -> 13.1 and 18.6 -> 18.2; 2 x 1537 of 8
+            // 63.7 -> 63.7; 2 x 2000 of 16 95 -> 104.
+            const bool past = (int64_t)p.st.nch * H * (CH * V * 2) >= (4 << 20);
             __builtin_amdgcn_s_barrier();
             for (int t = 0; t <= nchunks; ++t) {
                 lds_barrier();
@@ -204,7 +208,9 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
                     const int r = r0 + l / LPR, e = (l % LPR) * 16;
                     if (r < len) {
                         const i32x4 x = *reinterpret_cast<const i32x4*>(ob + r * C::OROW + e);
-                        st_past(reinterpret_cast<i32x4*>(reinterpret_cast<char*>(p.o + ((tok0 + r) * H + h) * V + 16 * vt0) + e), x);
+                        i32x4* const to = reinterpret_cast<i32x4*>(reinterpret_cast<char*>(p.o + ((tok0 + r) * H + h) * V + 16 * vt0) + e);
+                        if (past) st_past(to, x);
+                        else st_near(to, x);
                     }
                 }
             }
