@@ -367,8 +367,7 @@ __device__ __forceinline__ void fused_producer(const FusedArgs<T>& a, char* smem
                 const f32x4 kf = k4 * k4 * exp4<T>(g4) + kx * kx * exp4<T>(gx);
                 s_t += kf[0] + kf[1] + kf[2] + kf[3];
             }
-            s_t += __shfl_xor(s_t, 16);
-            s_t += __shfl_xor(s_t, 32);
+            s_t = sum_groups(s_t);
         }
         // the operands of channel tile j as the products take them: as loaded, or (HDLA parameterisation) formed from k,
         // gk, beta and s
@@ -878,8 +877,7 @@ __device__ __forceinline__ void fused_replay(const FusedArgs<T>& a, char* smem, 
                 const f32x4 kf = k4 * k4 * exp4<T>(g4) + kx * kx * exp4<T>(gx);
                 s_t += kf[0] + kf[1] + kf[2] + kf[3];
             }
-            s_t += __shfl_xor(s_t, 16);
-            s_t += __shfl_xor(s_t, 32);
+            s_t = sum_groups(s_t);
         }
         // ---- gated copies of the own channel tiles (prep.hip, phase C) ---------------------------------------------------
         Frag<T> agT[2][KH], fb[2][KH], fx[KH];            // fb, fx: bg^T, kg^T (checkpoint kernel); bg, qg^T (reverse kernel)

@@ -526,6 +526,37 @@ __device__ __forceinline__ float xor16(float x) {
     auto r = __builtin_amdgcn_permlane16_swap(xi, xi, false, false);     // r[0] rows: x0 x0 x2 x2, r[1]: x1 x1 x3 x3
     return __int_as_float((lane_id() & 16) ? r[0] : r[1]);
 }
+// Sums over the `width` lanes (1 to 64, a power of two, the same on all) of a lane's neighbourhood, on all of them: a butterfly on the vector ALU, within 16
+// lanes by DPP (the mirrors meet sums that are the same on four, or eight, neighbours), beyond by swaps of rows of lanes.  Additions and
+// order are those of a butterfly of __shfl_xor, and so are the bits; that one goes through LDS, at some 60 cycles a stage.
+template <int N> __device__ __forceinline__ void sum_lanes(float (&x)[N], int width) {
+    auto stage = [&](auto other) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) x[i] += other(x[i]);
+    };
+    if (width > 1) stage([](float v) __attribute__((always_inline)) { return dpp0<0xB1>(v); });     // quad_perm:[1,0,3,2]
+    if (width > 2) stage([](float v) __attribute__((always_inline)) { return dpp0<0x4E>(v); });     // quad_perm:[2,3,0,1]
+    if (width > 4) stage([](float v) __attribute__((always_inline)) { return dpp0<0x141>(v); });    // row_half_mirror
+    if (width > 8) stage([](float v) __attribute__((always_inline)) { return dpp0<0x140>(v); });    // row_mirror
+    if (width > 16) stage([](float v) __attribute__((always_inline)) { return xor16(v); });
+    if (width > 32) stage([](float v) __attribute__((always_inline)) { return xor32(v); });
+}
+__device__ __forceinline__ float sum_lanes(float x, int width) {
+    float v[1] = {x};
+    sum_lanes<1>(v, width);
+    return v[0];
+}
+
+// Sums over the lanes that lie CG (16 or 32) apart, on all of them
+template <int CG> __device__ __forceinline__ void sum_rows(f32x4& x) {
+    static_assert(CG == 16 || CG == 32, "rows or halves of a wavefront");
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (CG == 16) x[i] += xor16(x[i]);
+        x[i] += xor32(x[i]);
+    }
+}
+
 // sum over the four lanes c, c+16, c+32, c+48, on all of them
 __device__ __forceinline__ float sum_groups(float x) {
     x += xor16(x);

@@ -40,10 +40,8 @@ template <> struct PrePiece<bf16> {
         }
     }
     static __device__ __forceinline__ void st(void* base, long long elem, const float (&f)[8]) {
-        pre_u32x4 r;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) r[i] = (uint32_t)f2bf(f[2 * i]) | ((uint32_t)f2bf(f[2 * i + 1]) << 16);
-        *reinterpret_cast<pre_u32x4*>(static_cast<bf16*>(base) + elem) = r;
+        const s16x4 lo = to_frag<bf16>(f32x4{f[0], f[1], f[2], f[3]}).v, hi = to_frag<bf16>(f32x4{f[4], f[5], f[6], f[7]}).v;
+        *reinterpret_cast<s16x8*>(static_cast<bf16*>(base) + elem) = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     }
 };
 template <> struct PrePiece<float> {
@@ -104,7 +102,9 @@ __global__ __launch_bounds__(256) void layer_pre_fwd_kernel(PreArgs p) {
         float sq = 0.f, sk = 0.f, sv = 0.f;
 #pragma unroll
         for (int j = 0; j < N; ++j) { sq += q[j] * q[j]; sk += k[j] * k[j]; sv += v[j] * v[j]; }
-        for (int o = 1; o < lpr; o <<= 1) { sq += __shfl_xor(sq, o); sk += __shfl_xor(sk, o); sv += __shfl_xor(sv, o); }
+        float ss[3] = {sq, sk, sv};
+        sum_lanes<3>(ss, lpr);
+        sq = ss[0]; sk = ss[1]; sv = ss[2];
         const float iq = p.norm_q ? 1.f / sqrtf(sq + p.eps_d) : 1.f;
         const float ik = p.norm_k ? 1.f / sqrtf(sk + p.eps_d) : 1.f;
         const float iv = p.norm_v ? 1.f / sqrtf(sv + p.eps_d) : 1.f;
@@ -133,7 +133,9 @@ __device__ __forceinline__ void pre_bwd_one(float (&x)[N], float (&g)[N], bool n
         float su = 0.f, sd = 0.f;
 #pragma unroll
         for (int j = 0; j < N; ++j) { su += u[j] * u[j]; sd += u[j] * g[j]; }
-        for (int o = 1; o < lpr; o <<= 1) { su += __shfl_xor(su, o); sd += __shfl_xor(sd, o); }
+        float both[2] = {su, sd};
+        sum_lanes<2>(both, lpr);
+        su = both[0]; sd = both[1];
         const float inv = 1.f / sqrtf(su + eps_d);
         const float proj = sd * inv * inv;                 // sum(o * do) / |.|: with o = u inv, du = inv (do - o sum(o do))
 #pragma unroll

@@ -39,11 +39,7 @@ __device__ __forceinline__ float step_sigmoid(float x) {
     return s[0];
 }
 __device__ __forceinline__ float as_bf16(float x) { return bf2f(f2bf(x)); }
-__device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) x += __shfl_xor(x, o);
-    return x;
-}
+__device__ __forceinline__ float wave_sum(float x) { return sum_lanes(x, 64); }
 
 // the sum over 16 lanes side by side, on all of them
 __device__ __forceinline__ float row_sum(float x) {
@@ -183,11 +179,8 @@ __global__ __launch_bounds__(4 * D, 4) void layer_step_kernel(StepArgs p) {
             p0 += S[j] * sa[0][row];
             p1 += S[j] * sa[1][row];
         }
-#pragma unroll
-        for (int off = CG; off < 64; off <<= 1) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) { p0[i] += __shfl_xor(p0[i], off); p1[i] += __shfl_xor(p1[i], off); }
-        }
+        sum_rows<CG>(p0);
+        sum_rows<CG>(p1);
         if (lane < CG) {
             *reinterpret_cast<f32x4*>(&red[wave][0][4 * cg]) = p0;
             *reinterpret_cast<f32x4*>(&red[wave][1][4 * cg]) = p1;
@@ -207,11 +200,7 @@ __global__ __launch_bounds__(4 * D, 4) void layer_step_kernel(StepArgs p) {
             S[j] = S[j] * sf[row] + u0 * sb[row] + u1 * sk[row] + v4 * sk[row];
             po += S[j] * sq[row];
         }
-#pragma unroll
-        for (int off = CG; off < 64; off <<= 1) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) po[i] += __shfl_xor(po[i], off);
-        }
+        sum_rows<CG>(po);
         if (lane < CG) *reinterpret_cast<f32x4*>(&red[wave][2][4 * cg]) = po;
         __syncthreads();
         // o of the head, its gate and norm, by one wavefront (the others go on: what it reads here is written again behind the

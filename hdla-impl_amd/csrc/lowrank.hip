@@ -283,8 +283,7 @@ __global__ __launch_bounds__(64 * RW) void rows_gemm_kernel(const bf16* __restri
 #pragma unroll
             for (int i = 0; i < 8; ++i) ss += h0 + 4 * i + piece < nrm.parts ? v[i] : 0.f;
         }
-        ss += __shfl_xor(ss, 1);
-        ss += __shfl_xor(ss, 2);
+        ss = sum_lanes(ss, 4);
         rs = nrm.cn / sqrtf(ss * nrm.inv_e + nrm.eps);
         scaled = true;
     };

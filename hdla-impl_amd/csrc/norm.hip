@@ -126,15 +126,11 @@ struct NormLane {
 // the workgroup makes the same calls.
 __device__ __forceinline__ void group_sum(const NormLane& L, float& a, float& b, float* sred, int& buf) {
     const int width = L.wg_row ? 64 : L.lpr;
-    // butterflies on the vector ALU: within 16 lanes by DPP (the mirrors meet sums that are the same on four, or eight, neighbours), beyond by swaps
-    // of rows of lanes.  The sums are those of __shfl_xor, which goes through LDS; us, that -> this: 8192 x 1024 bf16 11.7 + 21.3 -> 11.2 + 20.4,
-    // 65536 x 4096 364 + 621 -> 350 + 605.
-    if (width > 1) { a += dpp0<0xB1>(a); b += dpp0<0xB1>(b); }
-    if (width > 2) { a += dpp0<0x4E>(a); b += dpp0<0x4E>(b); }
-    if (width > 4) { a += dpp0<0x141>(a); b += dpp0<0x141>(b); }
-    if (width > 8) { a += dpp0<0x140>(a); b += dpp0<0x140>(b); }
-    if (width > 16) { a += xor16(a); b += xor16(b); }
-    if (width > 32) { a += xor32(a); b += xor32(b); }
+    // (us, by __shfl_xor -> this: 8192 x 1024 bf16 11.7 + 21.3 -> 11.2 + 20.4, 65536 x 4096 364 + 621 -> 350 + 605)
+    float both[2] = {a, b};
+    sum_lanes<2>(both, width);
+    a = both[0];
+    b = both[1];
     if (L.wg_row) {
         float* s = sred + buf * 8;
         if ((threadIdx.x & 63) == 0) { s[2 * (threadIdx.x >> 6)] = a; s[2 * (threadIdx.x >> 6) + 1] = b; }

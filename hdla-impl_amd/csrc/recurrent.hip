@@ -107,9 +107,7 @@ __global__ __launch_bounds__(256) void recurrent_kernel(RecurrentArgs<T> p) {
         __syncthreads();
         const float kk = as_float(raw.k), f = exp_t<T>(p.gk_f32 ? __builtin_bit_cast(float, raw.gk) : bf2f((uint16_t)raw.gk));
         if constexpr (HD) {
-            float part = tid < K ? kk * kk * f : 0.f;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) part += __shfl_xor(part, o);
+            const float part = sum_lanes(tid < K ? kk * kk * f : 0.f, 64);
             if (lane == 0) red[wave][0][0] = part;
             __syncthreads();
         }
@@ -143,11 +141,8 @@ __global__ __launch_bounds__(256) void recurrent_kernel(RecurrentArgs<T> p) {
             p0 += S[j] * sa[0][row];
             p1 += S[j] * sa[1][row];
         }
-#pragma unroll
-        for (int off = CG; off < 64; off <<= 1) {
-#pragma unroll
-            for (int x = 0; x < 4; ++x) { p0[x] += __shfl_xor(p0[x], off); p1[x] += __shfl_xor(p1[x], off); }
-        }
+        sum_rows<CG>(p0);
+        sum_rows<CG>(p1);
         if (lane < CG) {
             *reinterpret_cast<f32x4*>(&red[wave][0][4 * cg]) = p0;
             *reinterpret_cast<f32x4*>(&red[wave][1][4 * cg]) = p1;
@@ -167,11 +162,7 @@ __global__ __launch_bounds__(256) void recurrent_kernel(RecurrentArgs<T> p) {
             S[j] = S[j] * seg[row] + u0 * sb[0][row] + u1 * sb[1][row] + v4 * sk[row];
             po += S[j] * sq[row];
         }
-#pragma unroll
-        for (int off = CG; off < 64; off <<= 1) {
-#pragma unroll
-            for (int x = 0; x < 4; ++x) po[x] += __shfl_xor(po[x], off);
-        }
+        sum_rows<CG>(po);
         if (lane < CG) *reinterpret_cast<f32x4*>(&red[wave][2][4 * cg]) = po;
         __syncthreads();
         if (tid < BV) {
