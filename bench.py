@@ -63,6 +63,12 @@ def interface_bytes(kernel, pass_, K, V, es, gs, frac_seg=0.0):
             return inputs - VR + W + KGT + BGT + EGL + QG + AQK + AQB + TMF
         if kernel == "scan_fwd":
             return W + KGT + BGT + EGL + QG + AQK + AQB + TMF + VR + 16 * V * es
+    if es == 2:                         # (the backward pass's forward scan too: from TM, a tile pair of A_ak and v; chunk_grad rebuilds u)
+        AAK, VR = 512 * es, 16 * V * es
+        if kernel == "prep":
+            return inputs - VR + W + KGT + BGT + EGL + AQBT + QGT + TM + AAK
+        if kernel == "scan_fwd":
+            return W + KGT + BGT + EGL + TM + AAK + VR + HC
     if kernel == "prep":
         out = W + UT + KGT + BGT + VTT + EGL + ((QG + AQK + AQB) if pass_ == 0 else (AQBT + QGT + TM))
         return inputs + out

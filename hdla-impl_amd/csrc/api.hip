@@ -275,8 +275,11 @@ int make_layout(const hdla_dims* d, int pass, WsLayout& L, int& nch) {
         if (pass == HDLA_PASS_FWD && es == 2) {
             L.TM = take(chw * 1536 * es);                         // the scan forms u itself (scan_out.cuh)
         } else {
+            // (2-byte elements: the scans form u and v^T themselves.  chunk_grad may read u; v^T is there, and u, for whoever names the classic route
+            // and looks at a backward pass's buffers.  A kept forward pass's layout does not depend on the route.)
             L.UT = take(chw * 2 * V * 16 * es);
-            L.VTT = take(chw * V * 16 * es);
+            if (es == 4 || (pass == HDLA_PASS_BWD && d->route == HDLA_ROUTE_CLASSIC)) L.VTT = take(chw * V * 16 * es);
+            if (es == 2) L.AAK = take(chw * 512 * es);
         }
     }
     if (bwd_parts) {
@@ -315,7 +318,8 @@ template <typename T>
 void bind_ws(ChunkArgs<T>& a, const hdla_dims* d, const WsLayout& LP, void* prep_ws, const WsLayout& LS, void* scan_ws, int nch) {
     char* base = static_cast<char*>(prep_ws);
     auto at = [&](size_t o) { return reinterpret_cast<T*>(base + o); };
-    a.ws.W = at(LP.W); a.ws.UT = at(LP.UT); a.ws.KGT = at(LP.KGT); a.ws.BGT = at(LP.BGT); a.ws.VTT = at(LP.VTT);
+    a.ws.W = at(LP.W); a.ws.UT = at(LP.UT); a.ws.KGT = at(LP.KGT); a.ws.BGT = at(LP.BGT);
+    a.ws.VTT = LP.VTT ? at(LP.VTT) : nullptr; a.ws.AAK = at(LP.AAK);
     a.ws.QG = at(LP.QG); a.ws.AQK = at(LP.AQK); a.ws.AQB = at(LP.AQB);
     a.ws.AQBT = at(LP.AQBT); a.ws.QGT = at(LP.QGT);
     a.ws.EGL = reinterpret_cast<float*>(base + LP.EGL);

@@ -96,6 +96,7 @@ struct WsLayout {
     size_t KGT;    // tiles  [K/16]      F(kg^T)       rows channel, inner token
     size_t BGT;    // tiles  [2][K/16]   F(bg_s^T)     rows channel, inner token
     size_t VTT;    // tiles  [V/16]      F(v^T)        rows value, inner token
+    size_t AAK;    // tiles  [2]         F(A_ak^s)     rows i, inner j: 2-byte elements, where the scan forms u from it, TM and v
     size_t EGL;    // fp32   [K]         exp(g_last)
     // forward pass only
     size_t QG;     // tiles  [K/16]      F(qg)         rows token, inner channel
@@ -121,6 +122,7 @@ struct WsLayout {
 template <typename T>
 struct Ws {
     T *W, *UT, *KGT, *BGT, *VTT, *QG, *AQK, *AQB, *AQBT, *QGT, *HC, *DHC, *DVN;
+    T* AAK;                   // VTT: null where nobody asks for u and v^T that the scans of 2-byte elements form themselves
     float *EGL;
     T* TM;
     int32_t* STRONG;

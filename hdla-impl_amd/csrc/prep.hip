@@ -34,6 +34,10 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
     constexpr bool WB = MODE != PREP_FWD;                 // the backward pass's extras are
     // the forward pass's scan of 2-byte elements forms u itself and takes the ranks of b^T side by side (scan_out.cuh): v is not read
     constexpr bool SCAN_U = MODE == PREP_FWD && sizeof(T) == 2;
+    // The other scans of 2-byte elements form u too, from (I - A_ab)^-1, A_ak and v; u is written where chunk_grad reads it (its REBUILD_U), or where the
+    // caller has named the classic route, whose buffers can be looked at (VTT is given).  This mode at K = V = 128, 16384 tokens of 16 heads, us: 221 -> 178,
+    // for 12 KB not written and v not read of 85 a chunk and head.
+    constexpr bool WRITE_U = sizeof(T) == 4 || HD || GKF32;
     constexpr int NWP = K / 64;                       // waves per (chunk, head)
     constexpr int KTW = 4, VT = V / 16, VTW = VT / NWP, KT2 = K / 32;
     constexpr int SAS = blk_fwd(K, sizeof(T), !BWD).SIZE / (int)sizeof(T);   // elements between (chunk, head) slots
@@ -295,7 +299,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
     // v is used last (phase D) but requested here: the barriers in between would otherwise keep its loads, and a
     // full round trip to HBM, behind everything else
     Load lv[VTW / 2];
-    if (!SCAN_U)
+    if (!SCAN_U && WRITE_U)
 #pragma unroll
     for (int vp = 0; vp < VTW / 2; ++vp) lv[vp].load(vrow + 32 * vp, H * V, cp.len, l);
     if (NWP > 1) {
@@ -431,13 +435,20 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
         }
         return;
     }
+    if (sizeof(T) == 2 && w == NWP - 1) st_pair2(p.ws.AAK + chw * PAIR, aakf[0], aakf[1]);
+    const bool vtt = sizeof(T) == 4 || p.ws.VTT;
+    if (!WRITE_U) {
+        if (!vtt) return;
+#pragma unroll
+        for (int vp = 0; vp < VTW / 2; ++vp) lv[vp].load(vrow + 32 * vp, H * V, cp.len, l);
+    }
     Frag<T> rv[2];
 #pragma unroll
     for (int vl = 0; vl < VTW; ++vl) {
         const int vt = vt0 + vl;
         if (vl % 2 == 0) lv[vl / 2].tiles(scratch, cp.len, l, rv);
         const Frag<T> vT = turn(rv[vl % 2], ident, scratch);
-        st_tile(p.ws.VTT + (chw * VT + vt) * TILE, vT);
+        if (vtt) st_tile(p.ws.VTT + (chw * VT + vt) * TILE, vT);
         const Frag<T> mT[2] = {to_frag<T>(mm(vT, aakf[0], zero4())), to_frag<T>(mm(vT, aakf[1], zero4()))};
         Frag<T> fu[2];
 #pragma unroll

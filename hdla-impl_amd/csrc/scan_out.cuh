@@ -15,7 +15,8 @@
 //  * u = Tm (A_ak v) is formed here by a wave of its own, a chunk ahead, from the chunk's (I - A_ab)^-1 and A_ak and the workgroup's columns
 //    of v (in the computing waves it cost 0.14 us a step: a chain of five dependent products).  The kernel that prepares the
 //    chunks does not read v and writes 3 KB instead of u and v^T, 12 KB of its 70 a chunk and head at K = V = 128: 236 -> 192 us for 16384
-//    tokens of 16 heads.  The products and roundings are the ones it had.
+//    tokens of 16 heads.  The products and roundings are the ones it had.  On the backward pass's workspace likewise, where that wave turns (I - A_ab)^-1 first
+//    (chunk_grad wants it the other way round): a training step of 16384 tokens of 16 heads 1700 -> 1649 us, of 2 x 1537 of 8 187 -> 182.
 // Measured, us, before -> after (when it was built), 2048 tokens a sequence: K = V = 128, 16 heads 88 -> 73, 32 heads 92 -> 79, 64 heads 105 -> 101, 128 heads
 // 167 -> 146; K = 64, V = 128, 128 heads 116 -> 98; K = 128, V = 64, 32 heads 87 -> 72.  From 48 heads on a step waits for its loads: 82 us
 // of the 101 where they never leave the L2, 70 without them; touching the blocks' lines 12 chunks ahead made it 105.
@@ -51,8 +52,8 @@ template <int K, int V, int NWC, ScanOut OUT> struct OutCfg {
 
 // OUT_O: with the output; OUT_STATE: the forward scan of the backward pass, which leaves the state that enters each chunk; OUT_SUM:
 // records of segments.
-// KEPT: on a workspace of the backward pass (or that it will read, PREP_KEEP): u and v^T are there, and b^T's pairs are of two channel
-// tiles, as the reverse scan takes them.  The same products in the same order: the same bits.
+// KEPT: on a workspace of the backward pass (or that it will read, PREP_KEEP): (I - A_ab)^-1 is there turned, as chunk_grad takes it, A_ak in a place of its
+// own, and b^T's pairs are of two channel tiles, as the reverse scan takes them.  The same products in the same order: the same bits.
 template <int K, int V, int NWC, ScanOut OUT, bool KEPT>
 __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* smem, int n, int seg, int split) {
     typedef OutCfg<K, V, NWC, OUT> C;
@@ -111,24 +112,19 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
             // v^T and u = Tm (A_ak v) of the workgroup's column blocks, a chunk ahead, with the roundings of the kernel that prepared the
             // chunk in u's place.  The operands come through registers, UD chunks ahead.
             constexpr int UD = 3;
-            struct Own { i32x4 tm[3], ut[KEPT ? NWC : 1]; Frag<T> v[NWC]; };
+            struct Own { i32x4 tm[3]; Frag<T> v[NWC]; };
             const Frag<T> ident = ident_frag<T>();
             auto request = [&](int t) __attribute__((always_inline)) {
                 t = min(t, last);
                 const int64_t tok0 = bos + (int64_t)t * CH;
                 const int len = (int)min((int64_t)CH, eos - tok0);
                 Own o;
-                if constexpr (KEPT) {
 #pragma unroll
-                    for (int j = 0; j < NWC; ++j) {
-                        const int64_t at = (chw0 + t) * (V / 16) + (trans ? 0 : vt0 + j);
-                        o.ut[j] = *reinterpret_cast<const i32x4*>(p.ws.UT + at * PAIR + 8 * l);
-                        o.v[j] = ld_tile(p.ws.VTT + at * TILE);
-                    }
-                    return o;
+                for (int i = 0; i < 3; ++i) {
+                    const T* const from = !KEPT ? p.ws.TM + (chw0 + t) * (3 * PAIR) + i * PAIR : i < 2 ? p.ws.TM + (chw0 + t) * (2 * PAIR) + i * PAIR
+                                                                                                       : p.ws.AAK + (chw0 + t) * PAIR;
+                    o.tm[i] = *reinterpret_cast<const i32x4*>(from + 8 * l);
                 }
-#pragma unroll
-                for (int i = 0; i < 3; ++i) o.tm[i] = *reinterpret_cast<const i32x4*>(p.ws.TM + (chw0 + t) * (3 * PAIR) + i * PAIR + 8 * l);
 #pragma unroll
                 for (int j = 0; j < NWC; ++j)
                     o.v[j] = ld_frag(p.v + ((tok0 + min(c, len - 1)) * H + h) * V + 16 * (trans ? 0 : vt0 + j) + 4 * g);
@@ -142,18 +138,16 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
             auto form = [&](int t, const Own& o) __attribute__((always_inline)) {
                 const int len = (int)min((int64_t)CH, eos - (bos + (int64_t)min(t, last) * CH));
                 T* const ub = reinterpret_cast<T*>(smem + C::UBUF + (t & 1) * C::UB);
-                if constexpr (KEPT) {
-#pragma unroll
-                    for (int j = 0; j < NWC; ++j) {
-                        *reinterpret_cast<i32x4*>(ub + j * (3 * TILE) + 8 * l) = trans ? i32x4{0, 0, 0, 0} : o.ut[j];
-                        st_tile(ub + j * (3 * TILE) + PAIR, trans ? zero_frag<T>() : o.v[j]);
-                    }
-                    return;
-                }
                 Frag<T> tm[2][2], aak[2], vT[NWC], mT[NWC][2];
                 pair(o.tm[0], tm[0][0], tm[0][1]);
                 pair(o.tm[1], tm[1][0], tm[1][1]);
                 pair(o.tm[2], aak[0], aak[1]);
+                if constexpr (KEPT) {
+#pragma unroll
+                    for (int s = 0; s < 2; ++s)
+#pragma unroll
+                        for (int r = 0; r < 2; ++r) tm[s][r] = transpose(tm[s][r], ident);
+                }
 #pragma unroll
                 for (int j = 0; j < NWC; ++j) vT[j] = transpose((c >= len || trans) ? zero_frag<T>() : o.v[j], ident);
 #pragma unroll
