@@ -173,7 +173,7 @@ int kept_plan_segments(const hdla_dims* d, int32_t& bwd) {
 
 struct FusedLayout {
     size_t OL, GW, SLOC, MSEG, RSEG, SIN, ERR;                 // fused kernels' own
-    size_t HC, DHC, DVN, TM, UT, W, STRONG;                    // what chunk_grad reads (backward pass)
+    size_t HC, DHC, DVN, TM, UT, W, SUM, STRONG;               // what chunk_grad reads (backward pass; UT and W beside fp32 decays)
     size_t MT, AQ;                                             // and the rest of the record
     size_t CHUNK_OFF, CHUNK_SEQ;
     size_t total;
@@ -215,8 +215,8 @@ int make_fused_layout(const hdla_dims* d, int pass, FusedLayout& L) {
         L.HC = take(chw * K * V * es);
         L.DHC = take(chw * K * V * es);
         L.DVN = take(chw * 2 * 16 * V * es);
-        L.UT = take(chw * 2 * V * 16 * es);
-        L.W = take(chw * 2 * K * 16 * es);
+        if (d->gk_dtype == HDLA_FP32) { L.UT = take(chw * 2 * V * 16 * es); L.W = take(chw * 2 * K * 16 * es); }
+        L.SUM = take(chw * 64);
     }
     if (d->cu_seqlens) {
         L.CHUNK_OFF = take((size_t)(2 * d->N + 1) * 4);
@@ -275,11 +275,12 @@ int make_layout(const hdla_dims* d, int pass, WsLayout& L, int& nch) {
         if (pass == HDLA_PASS_FWD && es == 2) {
             L.TM = take(chw * 1536 * es);                         // the scan forms u itself (scan_out.cuh)
         } else {
-            // (2-byte elements: the scans form u and v^T themselves.  chunk_grad may read u; v^T is there, and u, for whoever names the classic route
-            // and looks at a backward pass's buffers.  A kept forward pass's layout does not depend on the route.)
-            L.UT = take(chw * 2 * V * 16 * es);
-            if (es == 4 || (pass == HDLA_PASS_BWD && d->route == HDLA_ROUTE_CLASSIC)) L.VTT = take(chw * V * 16 * es);
-            if (es == 2) L.AAK = take(chw * 512 * es);
+            // (2-byte elements: the scans form u and v^T themselves.  chunk_grad reads u beside fp32 decays; v^T is there, and u, for whoever names the classic
+            // route and looks at a backward pass's buffers.  A kept forward pass's layout does not depend on the route.)
+            const bool shown = pass == HDLA_PASS_BWD && d->route == HDLA_ROUTE_CLASSIC;
+            if (d->gk_dtype == HDLA_FP32 || shown || pass == HDLA_PASS_FWD_KEEP) L.UT = take(chw * 2 * V * 16 * es);
+            if (es == 4 || shown) L.VTT = take(chw * V * 16 * es);
+            if (es == 2) { L.AAK = take(chw * 512 * es); L.SUM = take(chw * 64); }
         }
     }
     if (bwd_parts) {
@@ -319,7 +320,8 @@ void bind_ws(ChunkArgs<T>& a, const hdla_dims* d, const WsLayout& LP, void* prep
     char* base = static_cast<char*>(prep_ws);
     auto at = [&](size_t o) { return reinterpret_cast<T*>(base + o); };
     a.ws.W = at(LP.W); a.ws.UT = at(LP.UT); a.ws.KGT = at(LP.KGT); a.ws.BGT = at(LP.BGT);
-    a.ws.VTT = LP.VTT ? at(LP.VTT) : nullptr; a.ws.AAK = at(LP.AAK);
+    a.ws.VTT = LP.VTT ? at(LP.VTT) : nullptr; a.ws.AAK = at(LP.AAK); a.ws.aak_stride = 512;
+    a.ws.SUM = reinterpret_cast<float*>(base + LP.SUM);
     a.ws.QG = at(LP.QG); a.ws.AQK = at(LP.AQK); a.ws.AQB = at(LP.AQB);
     a.ws.AQBT = at(LP.AQBT); a.ws.QGT = at(LP.QGT);
     a.ws.EGL = reinterpret_cast<float*>(base + LP.EGL);
@@ -491,6 +493,8 @@ int run_fused(const hdla_dims* d, bool fwd, const void* q, const void* k, const 
         f.aq = reinterpret_cast<T*>(base + L.AQ);
         f.mt = reinterpret_cast<float*>(base + L.MT);
     }
+    a.ws.AAK = f.aq; a.ws.aak_stride = 1024;                       // (of the record's pairs, the first)
+    a.ws.SUM = reinterpret_cast<float*>(base + L.SUM);
     a.ws.sa_stride = 2 * d->K * 16 * 2;                            // chunk_grad's view of w: [2][K/16] tiles per slot
     a.st.cu = d->cu_seqlens;
     a.st.chunk_off = d->cu_seqlens ? reinterpret_cast<const int32_t*>(base + L.CHUNK_OFF) : nullptr;

@@ -878,6 +878,7 @@ __device__ __forceinline__ void fused_replay(const FusedArgs<T>& a, char* smem, 
                 s_t += kf[0] + kf[1] + kf[2] + kf[3];
             }
             s_t = sum_groups(s_t);
+            if (!REV && half == 0 && g == 0) p.ws.SUM[((int64_t)h * p.st.nch + cid) * CH + c] = s_t;
         }
         // ---- gated copies of the own channel tiles (prep.hip, phase C) ---------------------------------------------------
         Frag<T> agT[2][KH], fb[2][KH], fx[KH];            // fb, fx: bg^T, kg^T (checkpoint kernel); bg, qg^T (reverse kernel)
@@ -1136,7 +1137,8 @@ __device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* 
 // ---- consumers, checkpoint kernel ------------------------------------------------------------------------------------
 // The state walk of the forward direction from the true entering state, leaving the state entering every chunk for
 // chunk_grad, and R from the record's G.
-// W_GLOBAL: chunk_grad reads u and w from the workspace where it cannot rebuild them (chunk_grad_body.inc: REBUILD_W)
+// W_GLOBAL: chunk_grad reads u and w from the workspace where it cannot rebuild them (chunk_grad_body.inc: REBUILD_W).  (With the HDLA
+// parameterisation it rebuilds them too, from the sums over channels that the producers leave.)
 template <typename T, int K, int V, bool W_GLOBAL>
 __device__ __forceinline__ void fused_consumer_ckpt(const FusedArgs<T>& a, char* smem, int n, int h, int seg, int s0, int s1, int wv) {
     typedef FusedLds<T, K, V, FUSED_CKPT> L;
@@ -1443,7 +1445,7 @@ __global__ __launch_bounds__(64 * (V / 16 + 2 * FNP)) void fused_kernel(FusedArg
     __syncthreads();
     if (wv < V / 16) {
         if constexpr (MODE == FUSED_REV) fused_consumer_rev<T, K, V>(a, smem, n, h, seg, s0, s1, wv);
-        else if constexpr (MODE == FUSED_CKPT) fused_consumer_ckpt<T, K, V, HD || GKF32>(a, smem, n, h, seg, s0, s1, wv);
+        else if constexpr (MODE == FUSED_CKPT) fused_consumer_ckpt<T, K, V, GKF32>(a, smem, n, h, seg, s0, s1, wv);
         else fused_consumer_fwd<T, K, V, MODE>(a, smem, n, h, seg, s0, s1, wv);
     } else {
         const int pp = (wv - V / 16) >> 1, half = (wv - V / 16) & 1;

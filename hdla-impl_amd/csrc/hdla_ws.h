@@ -97,6 +97,7 @@ struct WsLayout {
     size_t BGT;    // tiles  [2][K/16]   F(bg_s^T)     rows channel, inner token
     size_t VTT;    // tiles  [V/16]      F(v^T)        rows value, inner token
     size_t AAK;    // tiles  [2]         F(A_ak^s)     rows i, inner j: 2-byte elements, where the scan forms u from it, TM and v
+    size_t SUM;    // fp32   [16]        HDLA parameterisation: sum over the channels of k^2 exp(gk), for chunk_grad's REBUILD_W
     size_t EGL;    // fp32   [K]         exp(g_last)
     // forward pass only
     size_t QG;     // tiles  [K/16]      F(qg)         rows token, inner channel
@@ -122,11 +123,13 @@ struct WsLayout {
 template <typename T>
 struct Ws {
     T *W, *UT, *KGT, *BGT, *VTT, *QG, *AQK, *AQB, *AQBT, *QGT, *HC, *DHC, *DVN;
+    float* SUM;
     T* AAK;                   // VTT: null where nobody asks for u and v^T that the scans of 2-byte elements form themselves
     float *EGL;
     T* TM;
     int32_t* STRONG;
     int sa_stride;            // bytes between the forward-scan blocks of consecutive (chunk, head) slots
+    int aak_stride;           // elements between their tile pairs of A_ak
 };
 
 // Time segments of the stand-alone scans (scan_impl.cuh, scan_out.cuh, scan_grad.cuh): records per (sequence, head, segment), fp32 tiles in fragment

@@ -37,7 +37,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
     // The other scans of 2-byte elements form u too, from (I - A_ab)^-1, A_ak and v; u is written where chunk_grad reads it (its REBUILD_U), or where the
     // caller has named the classic route, whose buffers can be looked at (VTT is given).  This mode at K = V = 128, 16384 tokens of 16 heads, us: 221 -> 178,
     // for 12 KB not written and v not read of 85 a chunk and head.
-    constexpr bool WRITE_U = sizeof(T) == 4 || HD || GKF32;
+    constexpr bool WRITE_U = sizeof(T) == 4 || GKF32;
     constexpr int NWP = K / 64;                       // waves per (chunk, head)
     constexpr int KTW = 4, VT = V / 16, VTW = VT / NWP, KT2 = K / 32;
     constexpr int SAS = blk_fwd(K, sizeof(T), !BWD).SIZE / (int)sizeof(T);   // elements between (chunk, head) slots
@@ -140,6 +140,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
 #pragma unroll
             for (int ww = 0; ww < NWP; ++ww) s_t += sSum[ww * CH + c];
         }
+        if (WB && sizeof(T) == 2 && w == 0 && g == 0) p.ws.SUM[chw * CH + c] = s_t;
     }
     // held: with the HDLA parameterisation k and the decays are there already, from the sum
     auto inputs = [&](int kp, const Request& x, Inputs (&in)[2], bool held) __attribute__((always_inline)) {

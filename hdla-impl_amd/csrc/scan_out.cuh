@@ -16,7 +16,7 @@
 //    of v (in the computing waves it cost 0.14 us a step: a chain of five dependent products).  The kernel that prepares the
 //    chunks does not read v and writes 3 KB instead of u and v^T, 12 KB of its 70 a chunk and head at K = V = 128: 236 -> 192 us for 16384
 //    tokens of 16 heads.  The products and roundings are the ones it had.  On the backward pass's workspace likewise, where that wave turns (I - A_ab)^-1 first
-//    (chunk_grad wants it the other way round): a training step of 16384 tokens of 16 heads 1700 -> 1649 us, of 2 x 1537 of 8 187 -> 182.
+//    (chunk_grad wants it the other way round): a training step of 16384 tokens of 16 heads 1700 -> 1649 us, of 2 x 1537 of 8 191 -> 182.
 // Measured, us, before -> after (when it was built), 2048 tokens a sequence: K = V = 128, 16 heads 88 -> 73, 32 heads 92 -> 79, 64 heads 105 -> 101, 128 heads
 // 167 -> 146; K = 64, V = 128, 128 heads 116 -> 98; K = 128, V = 64, 32 heads 87 -> 72.  From 48 heads on a step waits for its loads: 82 us
 // of the 101 where they never leave the L2, 70 without them; touching the blocks' lines 12 chunks ahead made it 105.

@@ -95,11 +95,10 @@ typedef struct hdla_dims {
  * [H][nch][...].  W, BGT, KGT, QG, AQB, AQK, EGL are parts of one block per (head, chunk) slot: the value given
  * is the offset for slot 0 and consecutive slots are SA_STRIDE bytes apart; likewise QGT, AQBT
  * with SB_STRIDE.  On the fused route the scans' operands never reach the workspace: only TM, HC, DHC, DVN, STRONG
- * (and W, UT where chunk_grad reads them instead of rebuilding them: the hdla_param_ forms, fp32 decays beside bf16
- * inputs) are written, in the backward pass.  In a forward pass on bf16 inputs (HDLA_PASS_FWD, classic route) the scan forms u
+ * (and W, UT where chunk_grad reads them instead of rebuilding them: fp32 decays beside bf16 inputs) are written, in the backward pass.  In a forward pass on bf16 inputs (HDLA_PASS_FWD, classic route) the scan forms u
  * itself: there is no UT and no VTT, TM holds three tile pairs a slot, the blocks of (I - A_ab)^-1 (not transposed: rows i, inner j) and
  * the two ranks of A_ak, and the tile pairs of BGT are the two ranks of a channel tile.  The other passes' scans of bf16 inputs form u themselves
- * as well: there is VTT, and UT is filled, in a backward pass under HDLA_ROUTE_CLASSIC only (UT also where chunk_grad reads it, as above). */
+ * as well: there is VTT, and UT is filled, in a backward pass under HDLA_ROUTE_CLASSIC only (UT also beside fp32 decays). */
 typedef struct hdla_ws_layout {
     int64_t nch;               /* chunk slots per head */
     int64_t W, UT, KGT, BGT, VTT, EGL, QG, AQK, AQB, AQBT, QGT, TM, HC, DHC, DVN;
