@@ -407,18 +407,22 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
             if (e != hipSuccess) return (int)e;
         }
     }
-    if (d->cu_seqlens && (stages & HDLA_STAGE_PREP)) {
-        char* base = static_cast<char*>(prep_ws);
+    if (stages & HDLA_STAGE_PREP) {
         // whether one of the scans on this table is shared out by the sequences' lengths (a kept one: of either pass, the backward one's in as many segments
         // or one)
         const bool shares = sizeof(T) == 2 && scan_shares(d->cu_seqlens, d->N, d->H, d->V, pass == HDLA_PASS_FWD_KEEP ? 1 : nseg, pass == HDLA_PASS_FWD ? 1 : 2);
-        e = launch_chunk_table(d->cu_seqlens, d->N, d->T, nch, d->H, shares ? d->V : 0, reinterpret_cast<int32_t*>(base + LP.CHUNK_OFF),
-                               reinterpret_cast<int32_t*>(base + LP.CHUNK_SEQ), packed_outputs(d, a), stream);
-        if (e != hipSuccess) return (int)e;
-    }
-    if (nch > 0 && (stages & HDLA_STAGE_PREP)) {
-        e = launch_prep<T>(a, d->K, d->V, pass == HDLA_PASS_FWD ? 0 : pass == HDLA_PASS_BWD ? 1 : 2, stream);
-        if (e != hipSuccess) return (int)e;
+        const int share_V = shares ? d->V : 0;
+        const PackedOut out = packed_outputs(d, a);
+        const bool made = prep_makes_table(d->cu_seqlens, d->N, d->H, nch);
+        if (d->cu_seqlens && !made) {
+            e = launch_chunk_table(d->cu_seqlens, d->N, d->T, nch, d->H, share_V, const_cast<int32_t*>(a.st.chunk_off), const_cast<int32_t*>(a.st.chunk_seq),
+                                   out, stream);
+            if (e != hipSuccess) return (int)e;
+        }
+        if (nch > 0) {
+            e = launch_prep<T>(a, d->K, d->V, pass == HDLA_PASS_FWD ? 0 : pass == HDLA_PASS_BWD ? 1 : 2, made ? &out : nullptr, share_V, stream);
+            if (e != hipSuccess) return (int)e;
+        }
     }
     if (a.seg.nseg > 1 && (stages & HDLA_STAGE_CHAIN)) {
         const SegStart what = pass == HDLA_PASS_FWD ? SEG_FWD : pass == HDLA_PASS_FWD_KEEP ? SEG_FWD_KEPT : pass == HDLA_PASS_BWD ? SEG_BWD : SEG_BWD_KEPT;

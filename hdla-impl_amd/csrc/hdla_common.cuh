@@ -442,6 +442,45 @@ __device__ __forceinline__ bool locate_chunk(const SeqTab& st, int cid, ChunkPos
     return cp.len > 0;
 }
 
+// The same without a table, for at most FEW_SEQS packed sequences: a wave reads the bounds of all of them, a sequence a lane, and adds up their chunks.
+// One round of loads, where the table is three of them one after the other.
+constexpr int FEW_SEQS = 64;
+struct FewSeqs {
+    int64_t bos, eos;  // of lane n's sequence
+    int chunks, end;   // its chunks, and where they end: their sum so far, no more than `nch` (sums of larger ones may not fit)
+};
+template <int CTRL, int ROWS> __device__ __forceinline__ int add_lanes(int x, int most) {
+    return min(x + __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false), most);
+}
+__device__ __forceinline__ FewSeqs few_seqs(const int64_t* cu, int N, int T, int nch) {
+    FewSeqs f;
+    const int n = lane_id();
+    packed_bounds(cu, min(n, N - 1), T, f.bos, f.eos);
+    f.chunks = n < N ? (int)((f.eos - f.bos + CH - 1) / CH) : 0;
+    f.end = min(f.chunks, nch);
+    f.end = add_lanes<0x111, 0xf>(f.end, nch);    // row_shr:1
+    f.end = add_lanes<0x112, 0xf>(f.end, nch);
+    f.end = add_lanes<0x114, 0xf>(f.end, nch);
+    f.end = add_lanes<0x118, 0xf>(f.end, nch);
+    f.end = add_lanes<0x142, 0xa>(f.end, nch);    // row_bcast:15, into the second and the fourth row of lanes
+    f.end = add_lanes<0x143, 0xc>(f.end, nch);    // row_bcast:31, into the third and the fourth
+    return f;
+}
+__device__ __forceinline__ int of_lane(int x, int n) { return __builtin_amdgcn_readlane(x, n); }
+__device__ __forceinline__ int64_t of_lane(int64_t x, int n) {
+    return (int64_t)(((uint64_t)(uint32_t)of_lane((int)((uint64_t)x >> 32), n) << 32) | (uint32_t)of_lane((int)(uint32_t)x, n));
+}
+// (cid: the same on every lane; all lanes)
+__device__ __forceinline__ bool locate_few(const SeqTab& st, int cid, ChunkPos& cp) {
+    const FewSeqs f = few_seqs(st.cu, st.N, st.T, st.nch);
+    if (cid >= of_lane(f.end, 63)) return false;
+    cp.n = __builtin_popcountll(__ballot(f.end <= cid));
+    const int c0 = cp.n ? of_lane(f.end, cp.n - 1) : 0;
+    cp.tok0 = of_lane(f.bos, cp.n) + (int64_t)(cid - c0) * CH;
+    cp.len = (int)min((int64_t)CH, of_lane(f.eos, cp.n) - cp.tok0);
+    return cp.len > 0;
+}
+
 // the z-th sequence in the order in which workgroups start: packed ones from the longest down (all that `order` is read with, but for scan_share)
 __device__ __forceinline__ int scan_sequence(const SeqTab& st, int z) { return st.cu ? st.order[z] & ORDER_SEQ : z; }
 // chunk range [c0, c1) of sequence n (n: the same on every lane)

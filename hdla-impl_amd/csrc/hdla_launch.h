@@ -22,7 +22,9 @@ hipError_t launch_clear_uncovered(const int64_t* cu, int N, int T, const PackedO
 
 // K, V in {64, 128}; returns hipErrorInvalidValue for any other pair.
 // mode: 0 = for the forward pass, 1 = for the backward pass, 2 = forward pass whose workspace the backward pass will use
-template <typename T> hipError_t launch_prep(const ChunkArgs<T>& a, int K, int V, int mode, hipStream_t stream);
+// out: with it the launch leaves the chunk table too and does launch_chunk_table's other work (prep_makes_table says whether it can); share_V as V there
+inline bool prep_makes_table(const int64_t* cu, int N, int H, int nch) { return cu && N <= 64 /* FEW_SEQS */ && nch > 0 && (long long)H * nch < 0x7ffff000LL; }
+template <typename T> hipError_t launch_prep(const ChunkArgs<T>& a, int K, int V, int mode, const PackedOut* out, int share_V, hipStream_t stream);
 // the two scans of the backward pass
 template <typename T> hipError_t launch_scan_fwd(const ChunkArgs<T>& a, int K, int V, hipStream_t stream);
 // the scan of the forward pass, with the output (kept: after launch_prep of mode 2, otherwise of mode 0)

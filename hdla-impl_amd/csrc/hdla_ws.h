@@ -14,7 +14,7 @@ struct bf16 { uint16_t x; };  // storage type tag for bf16 tensors (raw bits)
 
 // Tokens live on one flattened axis of B*T rows.  Without cu_seqlens sequence n covers rows [n*T, (n+1)*T) and
 // has NT = ceil(T/16) chunks; with cu_seqlens (device int64[N+1], batch 1) sequence n covers [cu[n], cu[n+1])
-// and its chunks are numbered from chunk_off[n] (device int32[N+1], built by build_chunk_table_kernel, which leaves
+// and its chunks are numbered from chunk_off[n] (device int32[N+1], built by build_chunk_table_kernel or prep_kernel, which leave
 // the int32[N] `order` right behind it).
 struct SeqTab {
     const int64_t* cu;        // nullable
@@ -25,14 +25,14 @@ struct SeqTab {
     int nch;                  // chunk slots the workspace is laid out for (an upper bound with cu_seqlens)
 };
 
-// Few packed sequences of unequal length share the device by their lengths: build_chunk_table_kernel leaves beside each entry of `order`, for
+// Few packed sequences of unequal length share the device by their lengths: beside each entry of `order` lies, for
 // the forward pass's scan and for the backward pass's two, how many column blocks a workgroup of that sequence has: 4 >> code.
 constexpr int SHARE_MAX_N = 32, ORDER_SEQ = 0x0fffffff, ORDER_OUT = 28, ORDER_GRAD = 30;
 // workgroups of a head (and direction) that the device holds at once, one a compute unit, and as many as a shared launch has at the most
 constexpr int share_slots(int H, int directions) { return 256 / (H * directions) > 1 ? 256 / (H * directions) : 1; }
 constexpr int share_most(int H, int directions, int N, int V) { return N * (V / 64) + share_slots(H, directions); }
-// whether a launch of the 2-byte scans is shared out so: whole sequences, and not where the narrowest workgroups fit the device.  The table kernel, which
-// everything else waits for, chooses the widths only then: that takes it 1 us for 8 sequences, 5 for 30.
+// whether a launch of the 2-byte scans is shared out so: whole sequences, and not where the narrowest workgroups fit the device.  The widths are
+// chosen only then: that takes 1 us for 8 sequences, 5 for 30, which a short prep_kernel does not hide.
 inline bool scan_shares(const int64_t* cu, int N, int H, int V, int nseg, int directions) {
     return cu && N > 1 && N <= SHARE_MAX_N && nseg == 1 && (long long)H * N * directions * (V / 16) > 256;
 }

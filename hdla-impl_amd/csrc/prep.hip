@@ -13,7 +13,231 @@
 #include "hdla_common.cuh"
 #include "hdla_launch.h"
 
+#include <algorithm>
+
 namespace hdla {
+
+// ---- chunk table for packed variable-length batches ----------------------------------------------------------
+constexpr int ORDER_MAX_N = 2048;      // beyond this many sequences they are taken as they come (ranking is quadratic)
+constexpr int TABLE_THREADS = 256;
+// More than FEW_SEQS sequences (fewer: few_table): workgroup 0 builds the table; with at most ORDER_MAX_N sequences, workgroups 1 .. ceil(N / 256) rank the sequences by
+// their chunk counts, one sequence a thread (they form the counts from cu themselves, so they wait for nobody).
+// The workgroups behind them clear the rows of the outputs that belong to no sequence.  Each looks the table over for itself
+// and, where it is a partition of the T tokens, is done: all of them together are in the shadow of workgroup 0 (clearing the
+// outputs for every call took 88 of 2050 us of a training step on 16384 tokens, H = 16, K = V = 128).  A table that does not
+// decrease leaves out only what lies before its first and behind its last entry (a batch padded at its end); one that does may
+// leave out anything, and the outputs are cleared whole.
+// Measured, 16384 tokens of 16 heads, K = V = 128, the last 200 in no sequence, forward and backward pass: 1.79 ms (a full batch 1.94);
+// with all outputs cleared by workgroup 0, two bytes a lane, 21.6.
+struct ClearRange { long long lo, hi; };                  // tokens [0, lo) and [hi, T)
+__device__ __forceinline__ ClearRange uncovered(const int64_t* cu, int N, int T, int t, int threads) {
+    int decreases = 0;
+    for (int n = t; n < N; n += threads) decreases |= cu[n + 1] < cu[n];
+    ClearRange r;
+    r.lo = min(max(cu[0], (int64_t)0), (int64_t)T);
+    r.hi = min(max(cu[N], (int64_t)r.lo), (int64_t)T);
+    if (__syncthreads_or(decreases)) r.lo = r.hi = T;
+    return r;
+}
+// n bytes at p (both multiples of 2) become zero, 16 bytes a store between the first and the last multiple of 16; i of `count` threads
+__device__ __forceinline__ void clear_bytes(char* p, long long n, long long i, long long count) {
+    const long long head = min((long long)(-reinterpret_cast<uintptr_t>(p) & 15), n), body = (n - head) & ~15LL;
+    for (long long e = 16 * i; e < body; e += 16 * count) *reinterpret_cast<i32x4*>(p + head + e) = i32x4{0, 0, 0, 0};
+    if (i < 8) {
+        if (2 * i < head) *reinterpret_cast<uint16_t*>(p + 2 * i) = 0;
+        if (head + body + 2 * i < n) *reinterpret_cast<uint16_t*>(p + head + body + 2 * i) = 0;
+    }
+}
+// (all threads of `groups` workgroups, of which this is the one numbered `group`)
+__device__ __forceinline__ void clear_uncovered(const int64_t* cu, int N, int T, const PackedOut& out, int group, int groups, int t, int threads) {
+    const ClearRange r = uncovered(cu, N, T, t, threads);
+    const long long count = (long long)groups * threads, i = (long long)group * threads + t;
+    for (int b = 0; b < out.n; ++b) {
+        char* const p = static_cast<char*>(out.p[b]);
+        clear_bytes(p, r.lo * out.row[b], i, count);
+        clear_bytes(p + r.hi * out.row[b], (T - r.hi) * out.row[b], i, count);
+    }
+}
+__global__ __launch_bounds__(TABLE_THREADS) void clear_uncovered_kernel(const int64_t* cu, int N, int T, PackedOut out) {
+    clear_uncovered(cu, N, T, out, blockIdx.x, gridDim.x, threadIdx.x, TABLE_THREADS);
+}
+// How wide the workgroups of each sequence are in the scans of the backward and the forward pass.  A workgroup of fewer column blocks takes a shorter
+// step, but more workgroups read a chunk's block.  Unequal lengths want unequal widths: a launch ends with its longest sequence, which walks its last
+// steps on a device that the others have left.  Candidates: every length in every width as the time that no sequence may exceed where a
+// narrower workgroup helps it; of these the one whose longest walk, or whose work spread over the slots, is least.  (Column blocks never meet: the
+// results have the same bits in every width.)  Times of a step of 4, 2 and
+// 1 blocks, 10 ns, one sequence of 16 heads alone on the device, K = V = 128: forward 81, 60, 58, both scans 105, 87, 78 (K = 64: 42, 35, 34; 59,
+// 51, 45); the choice needs their ratios only, and with K = 128's it is at K = 64 as good as with its own (1203 random batches: 0.4 and 0.3 % over the best
+// of its candidates on average, 14 and 13 % at the most).
+constexpr float SHARE_STEP[2][3] = {{81.f, 60.f, 58.f}, {105.f, 87.f, 78.f}}, SHARE_PROLOGUE = 6.f;
+// More workgroups than slots leave gaps behind them.  Over 1500 random batches of 2 to 14 sequences, the choice against the best of its candidates with the
+// workgroups dealt out one by one: 0.3 % on average, 12 % at the most (without the factor 0.8 and 41 %; one width for all 17 and 40 %).
+constexpr float SHARE_PACKING = 1.15f;
+struct ShareLds {
+    float steps[SHARE_MAX_N];                             // of the sequences from the longest down, and which they are
+    int seq[SHARE_MAX_N];
+    unsigned long long best[2];
+};
+__device__ __forceinline__ int share_code(int pass, float steps, float limit) {
+    return steps * SHARE_STEP[pass][0] <= limit ? 0 : steps * SHARE_STEP[pass][1] <= limit ? 1 : 2;
+}
+// (all threads; returns the bits that go beside order[t])
+__device__ __forceinline__ int share_device(ShareLds& sh, int N, int H, int V, int t, int threads) {
+    if (t < 2) sh.best[t] = ~0ull;
+    __syncthreads();
+    auto limit = [&](int pass, int i) { return sh.steps[i / 3] * SHARE_STEP[pass][i % 3]; };
+    for (int i = t; i < 6 * N; i += threads) {
+        const int pass = i >= 3 * N, cand = pass ? i - 3 * N : i;
+        const float x = limit(pass, cand);
+        float chain = 0.f, work = 0.f;
+        int groups = 0;
+        for (int j = 0; j < N; ++j) {
+            const int code = share_code(pass, sh.steps[j], x), g = (V / 64) << code;
+            const float time = sh.steps[j] * SHARE_STEP[pass][code];
+            chain = max(chain, time);
+            work += time * (float)g;
+            groups += g;
+        }
+        if (groups <= share_most(H, 1 + pass, N, V)) {
+            const int slots = share_slots(H, 1 + pass);
+            const float cost = groups <= slots ? chain : max(chain, SHARE_PACKING * work / (float)slots);
+            atomicMin(&sh.best[pass], (unsigned long long)__float_as_uint(cost) << 32 | (unsigned)cand);
+        }
+    }
+    __syncthreads();
+    int codes = 0;
+    if (t < N) {
+        codes = share_code(0, sh.steps[t], limit(0, (int)(unsigned)sh.best[0])) << ORDER_OUT;
+        codes |= (int)((unsigned)share_code(1, sh.steps[t], limit(1, (int)(unsigned)sh.best[1])) << ORDER_GRAD);
+    }
+    return codes;
+}
+// A table of at most FEW_SEQS sequences, in registers: work 0 writes chunk_off and chunk_seq, work 1 ranks the sequences (V: as in
+// launch_chunk_table).  All threads of a workgroup, at least a wave, each wave for itself but for the widths.
+__device__ __forceinline__ void few_table(int work, const int64_t* cu, int N, int T, int nch, int H, int V, int32_t* chunk_off, int32_t* chunk_seq,
+                                          ShareLds& sh, int t, int threads) {
+    const FewSeqs f = few_seqs(cu, N, T, nch);
+    if (work == 0) {
+        if (t < N) chunk_off[t + 1] = f.end;
+        if (t == 0) chunk_off[0] = 0;
+        for (int n = 0, c0 = 0; n < N; ++n) {
+            const int c1 = of_lane(f.end, n);
+            for (int cid = c0 + t; cid < c1; cid += threads) chunk_seq[cid] = n;
+            c0 = c1;
+        }
+        return;
+    }
+    int32_t* const order = chunk_off + N + 1;
+    const int n = lane_id();
+    int r = 0;
+    for (int m = 0; m < N; ++m) {
+        const int other = of_lane(f.chunks, m);
+        r += other > f.chunks || (other == f.chunks && m < n) ? 1 : 0;
+    }
+    if (V == 0 || N == 1 || N > SHARE_MAX_N) {
+        if (t < N) order[r] = n;
+        return;
+    }
+    if (t < N) {
+        sh.steps[r] = (float)f.chunks + SHARE_PROLOGUE;
+        sh.seq[r] = n;
+    }
+    const int codes = share_device(sh, N, H, V, t, threads);
+    if (t < N) order[t] = sh.seq[t] | codes;
+}
+__global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const int64_t* cu, int N, int T, int nch, int H, int V,
+                                                                          int32_t* chunk_off, int32_t* chunk_seq, int rankers, PackedOut out) {
+    constexpr int LONG_SEQ = 64, LONG_LIST = 512;
+    __shared__ long long strip[2][TABLE_THREADS];
+    __shared__ __attribute__((aligned(16))) int32_t len[ORDER_MAX_N];
+    __shared__ int n_long, long_seq[LONG_LIST], long_c0[LONG_LIST], long_c1[LONG_LIST];
+    const int t = threadIdx.x;
+    auto chunks_of = [&](int n) {
+        int64_t bos, eos;
+        packed_bounds(cu, n, T, bos, eos);
+        return (long long)((eos - bos + CH - 1) / CH);
+    };
+    int32_t* order = chunk_off + N + 1;
+    if ((int)blockIdx.x > rankers) {
+        clear_uncovered(cu, N, T, out, (int)blockIdx.x - 1 - rankers, (int)gridDim.x - 1 - rankers, t, TABLE_THREADS);
+        return;
+    }
+    __shared__ ShareLds sh;
+    if (N <= FEW_SEQS) {
+        few_table(blockIdx.x, cu, N, T, nch, H, V, chunk_off, chunk_seq, sh, t, TABLE_THREADS);
+        return;
+    }
+    if (blockIdx.x > 0) {
+        // order[r] = the sequence with the r-th most chunks (ties by index): the scans start their workgroups in this
+        // order, so that when there are more workgroups than compute units the long sequences are not the ones that
+        // wait.  All counts go to LDS (entries past N hold -1 and rank behind everything); a thread reads them four at
+        // a time against its own.
+        for (int n = t; n < ORDER_MAX_N; n += TABLE_THREADS) len[n] = n < N ? (int)min(chunks_of(n), (long long)0x7fffffff) : -1;
+        __syncthreads();
+        const int n = ((int)blockIdx.x - 1) * TABLE_THREADS + t;
+        if (n >= N) return;
+        const int mine = len[n];
+        int r = 0;
+        for (int m = 0; m < N; m += 4) {
+            const i32x4 lm = *reinterpret_cast<const i32x4*>(&len[m]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) r += (lm[j] > mine || (lm[j] == mine && m + j < n)) ? 1 : 0;
+        }
+        order[r] = n;
+        return;
+    }
+    // chunk_off = exclusive prefix sum of the sequences' chunk counts: every thread sums a strip of consecutive
+    // sequences, the strip sums are scanned in LDS, and the strips are walked a second time.
+    const int per = (N + TABLE_THREADS - 1) / TABLE_THREADS;
+    const int n0 = min(t * per, N), n1 = min(n0 + per, N);
+    long long own = 0;
+#pragma unroll 8
+    for (int n = n0; n < n1; ++n) own += chunks_of(n);
+    strip[0][t] = own;
+    if (t == 0) n_long = 0;
+    __syncthreads();
+    int cur = 0;
+    for (int d = 1; d < TABLE_THREADS; d <<= 1) {         // inclusive scan, one doubling step per round
+        strip[cur ^ 1][t] = strip[cur][t] + (t >= d ? strip[cur][t - d] : 0);
+        cur ^= 1;
+        __syncthreads();
+    }
+    // chunk_off, and chunk_seq: a thread writes the entries of its own strip's sequences; sequences of more than
+    // LONG_SEQ chunks are put on a list and written by the whole workgroup afterwards (a thread that finds the list
+    // full writes its own).  Offsets never go beyond the slots the workspace has (cannot happen for a non-decreasing
+    // table that ends at T).
+    long long acc = strip[cur][t] - own;
+    for (int n = n0; n < n1; ++n) {
+        const long long nx = acc + chunks_of(n);
+        const int c0 = (int)min(acc, (long long)nch), c1 = (int)min(nx, (long long)nch);
+        acc = nx;
+        chunk_off[n] = c0;
+        int slot = LONG_LIST;
+        if (c1 - c0 > LONG_SEQ) slot = atomicAdd(&n_long, 1);
+        if (slot < LONG_LIST) { long_seq[slot] = n; long_c0[slot] = c0; long_c1[slot] = c1; }
+        else for (int cid = c0; cid < c1; ++cid) chunk_seq[cid] = n;
+    }
+    if (t == 0) chunk_off[N] = (int)min(strip[cur][TABLE_THREADS - 1], (long long)nch);
+    __syncthreads();
+    const int nl = min(n_long, LONG_LIST);
+    for (int i = 0; i < nl; ++i)
+        for (int cid = long_c0[i] + t; cid < long_c1[i]; cid += TABLE_THREADS) chunk_seq[cid] = long_seq[i];
+    if (N > ORDER_MAX_N)                                  // too many to rank: as they come
+        for (int n = t; n < N; n += TABLE_THREADS) order[n] = n;
+}
+
+// The table as the work of prep_kernel's last workgroups, where a wave has a lane for each sequence: a launch of 4 to 8 us less that everything waited
+// for, and prep_kernel's other workgroups find their chunks by themselves (locate_few).  us, forward passes, table first -> this: 90 tokens in 4 sequences,
+// 4 heads 15.8 -> 13.0; 520 in 8, 8 heads, K = V = 128 27.5 -> 23.2; 3000 in 12, 16 heads, K = 64, V = 128 54.3 -> 47.4, in 30, K = V = 128 98.6 -> 91.8;
+// 5003 in 4 130.7 -> 127.0; fp32, 700 in 4 61.6 -> 57.1; training step of 16384 in 4 1649 -> 1634.  The fused route, whose first kernel walks
+// sequences, has the table first, in registers too: 2500 tokens in 5, 16 heads 52.0 -> 50.1.  FEW_CLEARERS: a workgroup a compute unit, beside prep's own.
+struct FewTable {
+    int32_t *chunk_off, *chunk_seq;       // null: the table is there
+    int V;
+    PackedOut out;
+};
+static_assert(FEW_SEQS == 64 && SHARE_MAX_N <= FEW_SEQS, "a lane each (prep_makes_table)");
+constexpr int FEW_CLEARERS = 256;
 
 constexpr int LDP = 36;   // padded row length of the 32x32 LDS matrices (keeps 16-byte row alignment)
 
@@ -29,7 +253,7 @@ enum PrepMode { PREP_FWD = 0, PREP_BWD = 1, PREP_KEEP = 2 };
 // of 16 heads 62 -> 52, 3074 tokens of 8 heads, both modes in one, 26 -> 23.  4-byte elements, 1008 chunks and heads (a wave a SIMD): the same.
 template <typename T, bool GKF32, bool HD> constexpr int prep_waves() { return sizeof(T) == 2 && (HD || !GKF32) ? 3 : 2; }
 template <typename T, bool GKF32, int K, int V, int MODE, bool HD>
-__global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T, GKF32, HD>(), prep_waves<T, GKF32, HD>()))) void prep_kernel(ChunkArgs<T> p) {
+__global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T, GKF32, HD>(), prep_waves<T, GKF32, HD>()))) void prep_kernel(ChunkArgs<T> p, FewTable few) {
     constexpr bool BWD = MODE == PREP_BWD;                // neither the output's score tiles nor qg are needed
     constexpr bool WB = MODE != PREP_FWD;                 // the backward pass's extras are
     // the forward pass's scan of 2-byte elements forms u itself and takes the ranks of b^T side by side (scan_out.cuh): v is not read
@@ -64,10 +288,17 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
     // touch the same few hundred bytes of every row, a fraction of the HBM channels); with shorter rows the chunks
     // of one head, whose workspace records are contiguous.
     const bool head_fastest = (uint32_t)(p.H * K) * sizeof(T) >= 4096;
+    if (few.chunk_off && (int)blockIdx.x >= p.H * p.st.nch) {
+        const int work = (int)blockIdx.x - p.H * p.st.nch, rest = (int)gridDim.x - p.H * p.st.nch - 2;
+        if (work < 2)
+            few_table(work, p.st.cu, p.st.N, p.st.T, p.st.nch, p.H, few.V, few.chunk_off, few.chunk_seq, *reinterpret_cast<ShareLds*>(sMat), threadIdx.x, K);
+        else clear_uncovered(p.st.cu, p.st.N, p.st.T, few.out, work - 2, rest, threadIdx.x, K);
+        return;
+    }
     const int cid = head_fastest ? blockIdx.x / p.H : blockIdx.x % p.st.nch;
     const int h = head_fastest ? blockIdx.x % p.H : blockIdx.x / p.st.nch;
     ChunkPos cp;
-    if (!locate_chunk(p.st, cid, cp)) return;
+    if (!(few.chunk_off ? locate_few(p.st, cid, cp) : locate_chunk(p.st, cid, cp))) return;
     const int l = lane_id(), g = l >> 4, c = l & 15;
     const int H = p.H;
     const bool rowok = c < cp.len;
@@ -460,194 +691,21 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
     }
 }
 
-// ---- chunk table for packed variable-length batches ----------------------------------------------------------
-constexpr int ORDER_MAX_N = 2048;      // beyond this many sequences they are taken as they come (ranking is quadratic)
-constexpr int TABLE_THREADS = 256;
-// Workgroup 0 builds the table; with at most ORDER_MAX_N sequences, workgroups 1 .. ceil(N / 256) rank the sequences by
-// their chunk counts, one sequence a thread (they form the counts from cu themselves, so they wait for nobody).
-// The workgroups behind them clear the rows of the outputs that belong to no sequence.  Each looks the table over for itself
-// and, where it is a partition of the T tokens, is done: all of them together are in the shadow of workgroup 0 (clearing the
-// outputs for every call took 88 of 2050 us of a training step on 16384 tokens, H = 16, K = V = 128).  A table that does not
-// decrease leaves out only what lies before its first and behind its last entry (a batch padded at its end); one that does may
-// leave out anything, and the outputs are cleared whole.
-// Measured, 16384 tokens of 16 heads, K = V = 128, the last 200 in no sequence, forward and backward pass: 1.79 ms (a full batch 1.94);
-// with all outputs cleared by workgroup 0, two bytes a lane, 21.6.
-struct ClearRange { long long lo, hi; };                  // tokens [0, lo) and [hi, T)
-__device__ __forceinline__ ClearRange uncovered(const int64_t* cu, int N, int T, int t) {
-    int decreases = 0;
-    for (int n = t; n < N; n += TABLE_THREADS) decreases |= cu[n + 1] < cu[n];
-    ClearRange r;
-    r.lo = min(max(cu[0], (int64_t)0), (int64_t)T);
-    r.hi = min(max(cu[N], (int64_t)r.lo), (int64_t)T);
-    if (__syncthreads_or(decreases)) r.lo = r.hi = T;
-    return r;
+// workgroups that look for rows to clear: one for every 16 KiB they might have to write, as many as fill the device, and fewer
+// where each has a long table to read first
+static int clearing_workgroups(int N, int T, const PackedOut& out) {
+    long long bytes = 0;
+    for (int b = 0; b < out.n; ++b) bytes += out.row[b] * T;
+    const long long most = max(32, min(512, (1 << 20) / N));
+    return (int)min((bytes + 16383) / 16384, most);
 }
-// n bytes at p (both multiples of 2) become zero, 16 bytes a store between the first and the last multiple of 16; i of `count` threads
-__device__ __forceinline__ void clear_bytes(char* p, long long n, long long i, long long count) {
-    const long long head = min((long long)(-reinterpret_cast<uintptr_t>(p) & 15), n), body = (n - head) & ~15LL;
-    for (long long e = 16 * i; e < body; e += 16 * count) *reinterpret_cast<i32x4*>(p + head + e) = i32x4{0, 0, 0, 0};
-    if (i < 8) {
-        if (2 * i < head) *reinterpret_cast<uint16_t*>(p + 2 * i) = 0;
-        if (head + body + 2 * i < n) *reinterpret_cast<uint16_t*>(p + head + body + 2 * i) = 0;
-    }
-}
-// (all threads of `groups` workgroups, of which this is the one numbered `group`)
-__device__ __forceinline__ void clear_uncovered(const int64_t* cu, int N, int T, const PackedOut& out, int group, int groups, int t) {
-    const ClearRange r = uncovered(cu, N, T, t);
-    const long long count = (long long)groups * TABLE_THREADS, i = (long long)group * TABLE_THREADS + t;
-    for (int b = 0; b < out.n; ++b) {
-        char* const p = static_cast<char*>(out.p[b]);
-        clear_bytes(p, r.lo * out.row[b], i, count);
-        clear_bytes(p + r.hi * out.row[b], (T - r.hi) * out.row[b], i, count);
-    }
-}
-__global__ __launch_bounds__(TABLE_THREADS) void clear_uncovered_kernel(const int64_t* cu, int N, int T, PackedOut out) {
-    clear_uncovered(cu, N, T, out, blockIdx.x, gridDim.x, threadIdx.x);
-}
-// How wide the workgroups of each sequence are in the scans of the backward and the forward pass.  A workgroup of fewer column blocks takes a shorter
-// step, but more workgroups read a chunk's block.  Unequal lengths want unequal widths: a launch ends with its longest sequence, which walks its last
-// steps on a device that the others have left.  Candidates: every length in every width as the time that no sequence may exceed where a
-// narrower workgroup helps it; of these the one whose longest walk, or whose work spread over the slots, is least.  (Column blocks never meet: the
-// results have the same bits in every width.)  Times of a step of 4, 2 and
-// 1 blocks, 10 ns, one sequence of 16 heads alone on the device, K = V = 128: forward 81, 60, 58, both scans 105, 87, 78 (K = 64: 42, 35, 34; 59,
-// 51, 45); the choice needs their ratios only, and with K = 128's it is at K = 64 as good as with its own (1203 random batches: 0.4 and 0.3 % over the best
-// of its candidates on average, 14 and 13 % at the most).
-constexpr float SHARE_STEP[2][3] = {{81.f, 60.f, 58.f}, {105.f, 87.f, 78.f}}, SHARE_PROLOGUE = 6.f;
-// More workgroups than slots leave gaps behind them.  Over 1500 random batches of 2 to 14 sequences, the choice against the best of its candidates with the
-// workgroups dealt out one by one: 0.3 % on average, 12 % at the most (without the factor 0.8 and 41 %; one width for all 17 and 40 %).
-constexpr float SHARE_PACKING = 1.15f;
-struct ShareLds {
-    float steps[SHARE_MAX_N];                             // of the sequences from the longest down, and which they are
-    int seq[SHARE_MAX_N];
-    unsigned long long best[2];
-};
-__device__ __forceinline__ int share_code(int pass, float steps, float limit) {
-    return steps * SHARE_STEP[pass][0] <= limit ? 0 : steps * SHARE_STEP[pass][1] <= limit ? 1 : 2;
-}
-// (all threads; returns the bits that go beside order[t])
-__device__ __forceinline__ int share_device(ShareLds& sh, int N, int H, int V, int t) {
-    if (t < 2) sh.best[t] = ~0ull;
-    __syncthreads();
-    auto limit = [&](int pass, int i) { return sh.steps[i / 3] * SHARE_STEP[pass][i % 3]; };
-    for (int i = t; i < 6 * N; i += TABLE_THREADS) {
-        const int pass = i >= 3 * N, cand = pass ? i - 3 * N : i;
-        const float x = limit(pass, cand);
-        float chain = 0.f, work = 0.f;
-        int groups = 0;
-        for (int j = 0; j < N; ++j) {
-            const int code = share_code(pass, sh.steps[j], x), g = (V / 64) << code;
-            const float time = sh.steps[j] * SHARE_STEP[pass][code];
-            chain = max(chain, time);
-            work += time * (float)g;
-            groups += g;
-        }
-        if (groups <= share_most(H, 1 + pass, N, V)) {
-            const int slots = share_slots(H, 1 + pass);
-            const float cost = groups <= slots ? chain : max(chain, SHARE_PACKING * work / (float)slots);
-            atomicMin(&sh.best[pass], (unsigned long long)__float_as_uint(cost) << 32 | (unsigned)cand);
-        }
-    }
-    __syncthreads();
-    int codes = 0;
-    if (t < N) {
-        codes = share_code(0, sh.steps[t], limit(0, (int)(unsigned)sh.best[0])) << ORDER_OUT;
-        codes |= (int)((unsigned)share_code(1, sh.steps[t], limit(1, (int)(unsigned)sh.best[1])) << ORDER_GRAD);
-    }
-    return codes;
-}
-__global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const int64_t* cu, int N, int T, int nch, int H, int V,
-                                                                          int32_t* chunk_off, int32_t* chunk_seq, int rankers, PackedOut out) {
-    constexpr int LONG_SEQ = 64, LONG_LIST = 512;
-    __shared__ long long strip[2][TABLE_THREADS];
-    __shared__ __attribute__((aligned(16))) int32_t len[ORDER_MAX_N];
-    __shared__ int n_long, long_seq[LONG_LIST], long_c0[LONG_LIST], long_c1[LONG_LIST];
-    const int t = threadIdx.x;
-    auto chunks_of = [&](int n) {
-        int64_t bos, eos;
-        packed_bounds(cu, n, T, bos, eos);
-        return (long long)((eos - bos + CH - 1) / CH);
-    };
-    int32_t* order = chunk_off + N + 1;
-    if ((int)blockIdx.x > rankers) {
-        clear_uncovered(cu, N, T, out, (int)blockIdx.x - 1 - rankers, (int)gridDim.x - 1 - rankers, t);
-        return;
-    }
-    if (blockIdx.x > 0) {
-        // order[r] = the sequence with the r-th most chunks (ties by index): the scans start their workgroups in this
-        // order, so that when there are more workgroups than compute units the long sequences are not the ones that
-        // wait.  All counts go to LDS (entries past N hold -1 and rank behind everything); a thread reads them four at
-        // a time against its own.
-        for (int n = t; n < ORDER_MAX_N; n += TABLE_THREADS) len[n] = n < N ? (int)min(chunks_of(n), (long long)0x7fffffff) : -1;
-        __syncthreads();
-        const int n = ((int)blockIdx.x - 1) * TABLE_THREADS + t;
-        const bool shared = V > 0 && N > 1 && N <= SHARE_MAX_N;
-        if (n >= N && !shared) return;
-        const int mine = len[n];
-        int r = 0;
-        for (int m = 0; m < N; m += 4) {
-            const i32x4 lm = *reinterpret_cast<const i32x4*>(&len[m]);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) r += (lm[j] > mine || (lm[j] == mine && m + j < n)) ? 1 : 0;
-        }
-        if (!shared) {
-            order[r] = n;
-            return;
-        }
-        __shared__ ShareLds sh;
-        if (n < N) {
-            sh.steps[r] = (float)mine + SHARE_PROLOGUE;
-            sh.seq[r] = n;
-        }
-        const int codes = share_device(sh, N, H, V, t);
-        if (t < N) order[t] = sh.seq[t] | codes;
-        return;
-    }
-    // chunk_off = exclusive prefix sum of the sequences' chunk counts: every thread sums a strip of consecutive
-    // sequences, the strip sums are scanned in LDS, and the strips are walked a second time.
-    const int per = (N + TABLE_THREADS - 1) / TABLE_THREADS;
-    const int n0 = min(t * per, N), n1 = min(n0 + per, N);
-    long long own = 0;
-#pragma unroll 8
-    for (int n = n0; n < n1; ++n) own += chunks_of(n);
-    strip[0][t] = own;
-    if (t == 0) n_long = 0;
-    __syncthreads();
-    int cur = 0;
-    for (int d = 1; d < TABLE_THREADS; d <<= 1) {         // inclusive scan, one doubling step per round
-        strip[cur ^ 1][t] = strip[cur][t] + (t >= d ? strip[cur][t - d] : 0);
-        cur ^= 1;
-        __syncthreads();
-    }
-    // chunk_off, and chunk_seq: a thread writes the entries of its own strip's sequences; sequences of more than
-    // LONG_SEQ chunks are put on a list and written by the whole workgroup afterwards (a thread that finds the list
-    // full writes its own).  Offsets never go beyond the slots the workspace has (cannot happen for a non-decreasing
-    // table that ends at T).
-    long long acc = strip[cur][t] - own;
-    for (int n = n0; n < n1; ++n) {
-        const long long nx = acc + chunks_of(n);
-        const int c0 = (int)min(acc, (long long)nch), c1 = (int)min(nx, (long long)nch);
-        acc = nx;
-        chunk_off[n] = c0;
-        int slot = LONG_LIST;
-        if (c1 - c0 > LONG_SEQ) slot = atomicAdd(&n_long, 1);
-        if (slot < LONG_LIST) { long_seq[slot] = n; long_c0[slot] = c0; long_c1[slot] = c1; }
-        else for (int cid = c0; cid < c1; ++cid) chunk_seq[cid] = n;
-    }
-    if (t == 0) chunk_off[N] = (int)min(strip[cur][TABLE_THREADS - 1], (long long)nch);
-    __syncthreads();
-    const int nl = min(n_long, LONG_LIST);
-    for (int i = 0; i < nl; ++i)
-        for (int cid = long_c0[i] + t; cid < long_c1[i]; cid += TABLE_THREADS) chunk_seq[cid] = long_seq[i];
-    if (N > ORDER_MAX_N)                                  // too many to rank: as they come
-        for (int n = t; n < N; n += TABLE_THREADS) order[n] = n;
-}
-
 template <typename T, int K, int V, bool HD>
-static hipError_t launch_prep_kv(const ChunkArgs<T>& a, int mode, hipStream_t stream) {
-    dim3 grid(a.st.nch * a.H), block(K);
+static hipError_t launch_prep_kv(const ChunkArgs<T>& a, int mode, const FewTable& few, hipStream_t stream) {
+    const int makers = few.chunk_off ? 2 + std::min(FEW_CLEARERS, clearing_workgroups(a.st.N, a.st.T, few.out)) : 0;
+    dim3 grid(a.st.nch * a.H + makers), block(K);
     constexpr bool kAlwaysF32 = sizeof(T) == 4;
     const bool gkf32 = kAlwaysF32 || a.gk_f32;
-#define HDLA_PREP_LAUNCH(GK, MODE) hipLaunchKernelGGL((prep_kernel<T, GK, K, V, MODE, HD>), grid, block, 0, stream, a)
+#define HDLA_PREP_LAUNCH(GK, MODE) hipLaunchKernelGGL((prep_kernel<T, GK, K, V, MODE, HD>), grid, block, 0, stream, a, few)
     if (gkf32) {
         if (mode == PREP_FWD) HDLA_PREP_LAUNCH(true, PREP_FWD);
         else if (mode == PREP_BWD) HDLA_PREP_LAUNCH(true, PREP_BWD);
@@ -662,29 +720,23 @@ static hipError_t launch_prep_kv(const ChunkArgs<T>& a, int mode, hipStream_t st
 }
 
 template <typename T, bool HD>
-static hipError_t launch_prep_hd(const ChunkArgs<T>& a, int K, int V, int mode, hipStream_t stream) {
-    if (K == 64 && V == 64) return launch_prep_kv<T, 64, 64, HD>(a, mode, stream);
-    if (K == 128 && V == 128) return launch_prep_kv<T, 128, 128, HD>(a, mode, stream);
-    if (K == 64 && V == 128) return launch_prep_kv<T, 64, 128, HD>(a, mode, stream);
-    if (K == 128 && V == 64) return launch_prep_kv<T, 128, 64, HD>(a, mode, stream);
+static hipError_t launch_prep_hd(const ChunkArgs<T>& a, int K, int V, int mode, const FewTable& few, hipStream_t stream) {
+    if (K == 64 && V == 64) return launch_prep_kv<T, 64, 64, HD>(a, mode, few, stream);
+    if (K == 128 && V == 128) return launch_prep_kv<T, 128, 128, HD>(a, mode, few, stream);
+    if (K == 64 && V == 128) return launch_prep_kv<T, 64, 128, HD>(a, mode, few, stream);
+    if (K == 128 && V == 64) return launch_prep_kv<T, 128, 64, HD>(a, mode, few, stream);
     return hipErrorInvalidValue;
 }
 
 template <typename T>
-hipError_t launch_prep(const ChunkArgs<T>& a, int K, int V, int mode, hipStream_t stream) {
-    return a.beta ? launch_prep_hd<T, true>(a, K, V, mode, stream) : launch_prep_hd<T, false>(a, K, V, mode, stream);
+hipError_t launch_prep(const ChunkArgs<T>& a, int K, int V, int mode, const PackedOut* out, int share_V, hipStream_t stream) {
+    FewTable few{};
+    if (out) few = FewTable{const_cast<int32_t*>(a.st.chunk_off), const_cast<int32_t*>(a.st.chunk_seq), share_V, *out};
+    return a.beta ? launch_prep_hd<T, true>(a, K, V, mode, few, stream) : launch_prep_hd<T, false>(a, K, V, mode, few, stream);
 }
-template hipError_t launch_prep<bf16>(const ChunkArgs<bf16>&, int, int, int, hipStream_t);
-template hipError_t launch_prep<float>(const ChunkArgs<float>&, int, int, int, hipStream_t);
+template hipError_t launch_prep<bf16>(const ChunkArgs<bf16>&, int, int, int, const PackedOut*, int, hipStream_t);
+template hipError_t launch_prep<float>(const ChunkArgs<float>&, int, int, int, const PackedOut*, int, hipStream_t);
 
-// workgroups that look for rows to clear: one for every 16 KiB they might have to write, as many as fill the device, and fewer
-// where each has a long table to read first
-static int clearing_workgroups(int N, int T, const PackedOut& out) {
-    long long bytes = 0;
-    for (int b = 0; b < out.n; ++b) bytes += out.row[b] * T;
-    const long long most = max(32, min(512, (1 << 20) / N));
-    return (int)min((bytes + 16383) / 16384, most);
-}
 hipError_t launch_clear_uncovered(const int64_t* cu, int N, int T, const PackedOut& out, hipStream_t stream) {
     const int clearers = clearing_workgroups(N, T, out);
     if (clearers == 0) return hipSuccess;
