@@ -50,7 +50,7 @@ struct Api {
     HDLA_FN(recurrent_fwd); HDLA_FN(param_recurrent_fwd); HDLA_FN(normalize_fwd); HDLA_FN(normalize_bwd_as);
     HDLA_FN(normalize_workspace_bytes); HDLA_FN(layer_pre_fwd); HDLA_FN(layer_pre_bwd); HDLA_FN(layer_up_fwd); HDLA_FN(layer_down);
     HDLA_FN(layer_up_wgrad); HDLA_FN(layer_up_wgrad_workspace_bytes); HDLA_FN(rows_gemm); HDLA_FN(sum_partials); HDLA_FN(stack_rows);
-    HDLA_FN(weight_grad); HDLA_FN(weight_grad_workspace_bytes);
+    HDLA_FN(weight_grad); HDLA_FN(weight_grad_workspace_bytes); HDLA_FN(weight_grad_pair); HDLA_FN(weight_grad_pair_workspace_bytes);
     HDLA_FN(layer_step); HDLA_FN(rows_gemm_norm);
 #undef HDLA_FN
 } api;
@@ -783,10 +783,14 @@ void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, Plan& p
 // 44 -> 38), but a second round of workgroups for a few tiles costs what it gains: 288 tiles, 1000 / 2048 / 4096 / 8192 rows 27 -> 23, 33 -> 35, 59 -> 62,
 // 114 -> 115; 512 tiles 29 -> 30, 39 -> 43, 68 -> 75, 130 -> 135.  Others: an output of few tiles would leave most of the chip idle (1024 x 1024 over 8192 rows: 54 us), so the rows are split over a batch
 // of products whose fp32 results one kernel adds (28 + 4 us).
+bool own_weight_grad(const Tensor& dy, const Tensor& x) {
+    const int64_t rows = dy.size(0), n = dy.size(1), k = x.size(1);
+    return rows > 0 && rows <= 0x7fff0000 && n > 0 && k > 0 && n % 128 == 0 && k % 128 == 0 && n / 128 * (k / 128) <= 256 && dy.stride(1) == 1 &&
+           x.stride(1) == 1 && dy.stride(0) >= n && x.stride(0) >= k && dy.stride(0) % 8 == 0 && x.stride(0) % 8 == 0 && !off_grid(dy) && !off_grid(x);
+}
 Tensor weight_grad(const Tensor& dy, const Tensor& x) {
     const int64_t rows = dy.size(0), n = dy.size(1), k = x.size(1);
-    if (rows > 0 && rows <= 0x7fff0000 && n > 0 && k > 0 && n % 128 == 0 && k % 128 == 0 && n / 128 * (k / 128) <= 256 && dy.stride(1) == 1 &&
-        x.stride(1) == 1 && dy.stride(0) >= n && x.stride(0) >= k && dy.stride(0) % 8 == 0 && x.stride(0) % 8 == 0 && !off_grid(dy) && !off_grid(x)) {
+    if (own_weight_grad(dy, x)) {
         const Tensor dw = at::empty({n, k}, dy.options());
         const size_t nws = api.weight_grad_workspace_bytes(rows, (int32_t)n, (int32_t)k);
         const Tensor ws = nws ? bytes_like(x, nws) : Tensor();
@@ -802,6 +806,30 @@ Tensor weight_grad(const Tensor& dy, const Tensor& x) {
     const Tensor dw = at::empty({n, k}, dy.options());
     check(api.sum_partials(fptr(part), (int32_t)S, n * k, ptr(dw), stream_of(dy)), "hdla_sum_partials");
     return dw;
+}
+// Two of them over the same rows: in one launch where each is the library's own (figures in wgrad.hip).
+void weight_grads(const Tensor (&dy)[2], const Tensor (&x)[2], Tensor (&dw)[2]) {
+    if (!own_weight_grad(dy[0], x[0]) || !own_weight_grad(dy[1], x[1])) {
+        for (int i = 0; i < 2; ++i) dw[i] = weight_grad(dy[i], x[i]);
+        return;
+    }
+    int32_t n[2], k[2];
+    int64_t ldy[2], ldx[2];
+    const void *pdy[2], *px[2];
+    void* pdw[2];
+    for (int i = 0; i < 2; ++i) {
+        n[i] = (int32_t)dy[i].size(1);
+        k[i] = (int32_t)x[i].size(1);
+        dw[i] = at::empty({n[i], k[i]}, dy[i].options());
+        ldy[i] = dy[i].stride(0);
+        ldx[i] = x[i].stride(0);
+        pdy[i] = ptr(dy[i]);
+        px[i] = ptr(x[i]);
+        pdw[i] = ptr(dw[i]);
+    }
+    const size_t nws = api.weight_grad_pair_workspace_bytes(dy[0].size(0), n, k);
+    const Tensor ws = nws ? bytes_like(x[0], nws) : Tensor();
+    check(api.weight_grad_pair(dy[0].size(0), n, k, pdy, ldy, px, ldx, pdw, ptr(ws), nws, stream_of(dy[0])), "hdla_weight_grad_pair");
 }
 struct LayerFn : torch::autograd::Function<LayerFn> {
     static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& wq, const Tensor& wk, const Tensor& wv, const Tensor& wf0,
@@ -843,7 +871,8 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
 
         // output projection and gated norm
         const Tensor dout = grads[0].defined() ? grads[0].to(at::kBFloat16).contiguous().view({rows, d}) : at::zeros({rows, d}, opt);
-        if (need(10)) out[10] = weight_grad(dout, n);
+        const bool projections = need(1) || need(2) || need(3) || need(4) || need(5) || need(6);
+        if (need(10) && !projections) out[10] = weight_grad(dout, n);     // (else with theirs)
         const Tensor dn = at::mm(dout, wo);
         const Tensor o2 = o.view({rows, d}), d_o = at::empty({rows, d}, opt), dgate = at::empty({rows, d}, opt);
         const Tensor dwn = at::empty(wnorm.sizes(), wnorm.options());
@@ -886,8 +915,16 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
         }
 
         // the projections of x
-        if (need(1) || need(2) || need(3) || need(4) || need(5) || need(6)) {
-            const Tensor dw = weight_grad(dy, x);
+        if (projections) {
+            Tensor dw;
+            if (need(10)) {
+                Tensor both[2];
+                weight_grads({dy, dout}, {x, n}, both);
+                dw = both[0];
+                out[10] = both[1];
+            } else {
+                dw = weight_grad(dy, x);
+            }
             const int64_t at_row[7] = {0, d, 2 * d, L.f0, L.g0, L.beta, L.used};
             for (int i = 0; i < 6; ++i) out[1 + i] = dw.narrow(0, at_row[i], at_row[i + 1] - at_row[i]);
         }
@@ -1117,7 +1154,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HDLA_FN(recurrent_fwd) HDLA_FN(param_recurrent_fwd) HDLA_FN(normalize_fwd) HDLA_FN(normalize_bwd_as)
     HDLA_FN(normalize_workspace_bytes) HDLA_FN(layer_pre_fwd) HDLA_FN(layer_pre_bwd) HDLA_FN(layer_up_fwd) HDLA_FN(layer_down)
     HDLA_FN(layer_up_wgrad) HDLA_FN(layer_up_wgrad_workspace_bytes) HDLA_FN(rows_gemm) HDLA_FN(sum_partials) HDLA_FN(stack_rows) HDLA_FN(layer_step)
-    HDLA_FN(weight_grad) HDLA_FN(weight_grad_workspace_bytes)
+    HDLA_FN(weight_grad) HDLA_FN(weight_grad_workspace_bytes) HDLA_FN(weight_grad_pair) HDLA_FN(weight_grad_pair_workspace_bytes)
     HDLA_FN(rows_gemm_norm)
 #undef HDLA_FN
     Py_INCREF(a[1]);

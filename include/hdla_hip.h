@@ -336,6 +336,11 @@ int hdla_sum_partials(const float* part, int32_t count, int64_t n, void* out, vo
 size_t hdla_weight_grad_workspace_bytes(int64_t M, int32_t N, int32_t K);
 int hdla_weight_grad(int64_t M, int32_t N, int32_t K, const void* dY, int64_t ldy, const void* X, int64_t ldx, void* dW, void* workspace,
                      size_t workspace_bytes, void* stream);
+/* Two such products with the same rows in one launch, of up to 256 tiles of 128 x 128 each (else HDLA_ERR_SHAPE); every argument but M, the workspace
+ * and the stream is an array of two. */
+size_t hdla_weight_grad_pair_workspace_bytes(int64_t M, const int32_t* N, const int32_t* K);
+int hdla_weight_grad_pair(int64_t M, const int32_t* N, const int32_t* K, const void* const* dY, const int64_t* ldy, const void* const* X,
+                          const int64_t* ldx, void* const* dW, void* workspace, size_t workspace_bytes, void* stream);
 /* out [total_rows, width] (2-byte elements) = the rows of parts[0 .. count) one part behind the other, parts[m] being [rows[m], width],
  * then zeros; count <= 8, width a multiple of 8, everything contiguous and 16-byte aligned.  parts and rows are host arrays. */
 int hdla_stack_rows(const void* const* parts, const int64_t* rows, int32_t count, int64_t width, void* out, int64_t total_rows, void* stream);
