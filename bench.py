@@ -632,7 +632,7 @@ def main():
                 "config": {"workload": "gated RMS norm of the layer at configuration 2's shape: 8192 rows x 1024 channels, "
                                        "bf16 tensors, fp32 weight, gate before the norm; forward + backward"},
                 "shapes": out,
-                "roofline": {"bound": "hbm", "kernel": "normalize_bwd_kernel (+ normalize_dw_kernel), 262144 rows",
+                "roofline": {"bound": "hbm", "kernel": "normalize_bwd_kernel (+ the sum of its partial weight gradients), 262144 rows",
                              "achieved": big["bwd_GB/s"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                              "frac": big["bwd_GB/s"] / HBM_PEAK_GBS, "traffic": norm_traffic(262144),
                              "bytes_per_launch": big["bwd_bytes"], "ms_per_launch": big["bwd_ms"],

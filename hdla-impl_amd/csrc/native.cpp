@@ -51,6 +51,7 @@ struct Api {
     HDLA_FN(normalize_workspace_bytes); HDLA_FN(layer_pre_fwd); HDLA_FN(layer_pre_bwd); HDLA_FN(layer_up_fwd); HDLA_FN(layer_down);
     HDLA_FN(layer_up_wgrad); HDLA_FN(layer_up_wgrad_workspace_bytes); HDLA_FN(rows_gemm); HDLA_FN(sum_partials); HDLA_FN(stack_rows);
     HDLA_FN(weight_grad); HDLA_FN(weight_grad_workspace_bytes); HDLA_FN(weight_grad_pair); HDLA_FN(weight_grad_pair_workspace_bytes);
+    HDLA_FN(normalize_bwd_later); HDLA_FN(layer_up_wgrad_later); HDLA_FN(run_sums);
     HDLA_FN(layer_step); HDLA_FN(rows_gemm_norm);
 #undef HDLA_FN
 } api;
@@ -807,8 +808,13 @@ Tensor weight_grad(const Tensor& dy, const Tensor& x) {
     check(api.sum_partials(fptr(part), (int32_t)S, n * k, ptr(dw), stream_of(dy)), "hdla_sum_partials");
     return dw;
 }
+// Sums over partial results that a backward pass leaves for its end, and what they are read from
+struct Sums {
+    hdla_sum of[4] = {};
+    Tensor room[3];
+};
 // Two of them over the same rows: in one launch where each is the library's own (figures in wgrad.hip).
-void weight_grads(const Tensor (&dy)[2], const Tensor (&x)[2], Tensor (&dw)[2]) {
+void weight_grads(const Tensor (&dy)[2], const Tensor (&x)[2], Tensor (&dw)[2], hdla_sum& sum, Tensor& ws) {
     if (!own_weight_grad(dy[0], x[0]) || !own_weight_grad(dy[1], x[1])) {
         for (int i = 0; i < 2; ++i) dw[i] = weight_grad(dy[i], x[i]);
         return;
@@ -828,8 +834,8 @@ void weight_grads(const Tensor (&dy)[2], const Tensor (&x)[2], Tensor (&dw)[2]) 
         pdw[i] = ptr(dw[i]);
     }
     const size_t nws = api.weight_grad_pair_workspace_bytes(dy[0].size(0), n, k);
-    const Tensor ws = nws ? bytes_like(x[0], nws) : Tensor();
-    check(api.weight_grad_pair(dy[0].size(0), n, k, pdy, ldy, px, ldx, pdw, ptr(ws), nws, stream_of(dy[0])), "hdla_weight_grad_pair");
+    if (nws) ws = bytes_like(x[0], nws);
+    check(api.weight_grad_pair(dy[0].size(0), n, k, pdy, ldy, px, ldx, pdw, ptr(ws), nws, &sum, stream_of(dy[0])), "hdla_weight_grad_pair");
 }
 struct LayerFn : torch::autograd::Function<LayerFn> {
     static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& wq, const Tensor& wk, const Tensor& wv, const Tensor& wf0,
@@ -868,6 +874,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
         const auto opt = x.options();
         const auto need = [&](size_t i) { return ctx->needs_input_grad(i); };
         variable_list out(15);
+        Sums sums;
 
         // output projection and gated norm
         const Tensor dout = grads[0].defined() ? grads[0].to(at::kBFloat16).contiguous().view({rows, d}) : at::zeros({rows, d}, opt);
@@ -879,9 +886,9 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
         {
             const hdla_norm_dims nd = norm_dims(o2, wnorm, cfg.gate_pos, cfg.c, cfg.eps, cfg.groups);
             const size_t nws = api.normalize_workspace_bytes(&nd);
-            const Tensor ws = bytes_like(x, nws < 16 ? 16 : nws);
-            check(api.normalize_bwd_as(&nd, ptr(o2), ptr(wnorm), ptr(g), ptr(dn), ptr(d_o), ptr(dgate), ptr(dwn), ptr(ws), nws, stream),
-                  "hdla_normalize_bwd_as");
+            sums.room[0] = bytes_like(x, nws < 16 ? 16 : nws);
+            check(api.normalize_bwd_later(&nd, ptr(o2), ptr(wnorm), ptr(g), ptr(dn), ptr(d_o), ptr(dgate), ptr(dwn), ptr(sums.room[0]), nws, &sums.of[0], stream),
+                  "hdla_normalize_bwd_later");
         }
         if (need(9)) out[9] = dwn;
 
@@ -909,9 +916,9 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
             out[7] = at::empty_like(wf1);
             out[8] = at::empty_like(wg1);
             const size_t nws = api.layer_up_wgrad_workspace_bytes(&ud);
-            const Tensor ws = bytes_like(x, nws);
-            check(api.layer_up_wgrad(&ud, ptr(y), ptr(f), ptr(dgk), ptr(dgate), ptr(out[7]), ptr(out[8]), ptr(ws), nws, stream),
-                  "hdla_layer_up_wgrad");
+            sums.room[1] = bytes_like(x, nws);
+            check(api.layer_up_wgrad_later(&ud, ptr(y), ptr(f), ptr(dgk), ptr(dgate), ptr(out[7]), ptr(out[8]), ptr(sums.room[1]), nws, &sums.of[1], stream),
+                  "hdla_layer_up_wgrad_later");
         }
 
         // the projections of x
@@ -919,7 +926,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
             Tensor dw;
             if (need(10)) {
                 Tensor both[2];
-                weight_grads({dy, dout}, {x, n}, both);
+                weight_grads({dy, dout}, {x, n}, both, sums.of[3], sums.room[2]);
                 dw = both[0];
                 out[10] = both[1];
             } else {
@@ -928,6 +935,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
             const int64_t at_row[7] = {0, d, 2 * d, L.f0, L.g0, L.beta, L.used};
             for (int i = 0; i < 6; ++i) out[1 + i] = dw.narrow(0, at_row[i], at_row[i + 1] - at_row[i]);
         }
+        check(api.run_sums(sums.of, 4, stream), "hdla_run_sums");
         if (need(0)) out[0] = at::mm(dy, w).view({B, T, d});
         return out;
     }
@@ -1155,6 +1163,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HDLA_FN(normalize_workspace_bytes) HDLA_FN(layer_pre_fwd) HDLA_FN(layer_pre_bwd) HDLA_FN(layer_up_fwd) HDLA_FN(layer_down)
     HDLA_FN(layer_up_wgrad) HDLA_FN(layer_up_wgrad_workspace_bytes) HDLA_FN(rows_gemm) HDLA_FN(sum_partials) HDLA_FN(stack_rows) HDLA_FN(layer_step)
     HDLA_FN(weight_grad) HDLA_FN(weight_grad_workspace_bytes) HDLA_FN(weight_grad_pair) HDLA_FN(weight_grad_pair_workspace_bytes)
+    HDLA_FN(normalize_bwd_later) HDLA_FN(layer_up_wgrad_later) HDLA_FN(run_sums)
     HDLA_FN(rows_gemm_norm)
 #undef HDLA_FN
     Py_INCREF(a[1]);

@@ -15,7 +15,7 @@
 // groups such that a lane always meets the same weight columns: weights are loaded once, and the weight gradient
 // accumulates in registers and leaves as one partial row per (wavefront, group position), summed by a second small
 // kernel in a fixed order (results do not depend on timing).
-#include "hdla_common.cuh"
+#include "sums.cuh"
 #include "../../include/hdla_hip.h"
 
 namespace hdla {
@@ -382,34 +382,6 @@ __global__ __launch_bounds__(256) void normalize_bwd_kernel(NormArgs p) {
     }
 }
 
-// dw[g*E + e] = sum of the partial rows idx = g, g + G, g + 2G, ... ; one workgroup per 16 columns: 4 lanes of four
-// columns each, 64 row phases, summed through LDS in a fixed order.  dw in 32 bits or (O: bf16) in the weight's own 16, rounded once (as a launch of its
-// own that was 4.8 us of a training step of the layer).
-template <typename O>
-__global__ __launch_bounds__(256) void normalize_dw_kernel(const float* __restrict__ partial, O* __restrict__ dw,
-                                                           long long nrow, int G, int E) {
-    __shared__ f32x4 red[64][4];
-    const int cq = threadIdx.x & 3, rl = threadIdx.x >> 2;
-    const long long col = (long long)blockIdx.x * 16 + cq * 4;
-    const long long D = (long long)G * E;
-    f32x4 acc = zero4();
-    if (col < D) {
-        const int g = (int)(col / E), e = (int)(col % E);
-#pragma unroll 8
-        for (long long idx = g + (long long)rl * G; idx < nrow; idx += 64LL * G)
-            acc += *reinterpret_cast<const f32x4*>(partial + idx * E + e);
-    }
-    red[rl][cq] = acc;
-    __syncthreads();
-    if (rl == 0 && col < D) {
-        f32x4 s = red[0][cq];
-#pragma unroll
-        for (int r = 1; r < 64; ++r) s += red[r][cq];
-        if constexpr (sizeof(O) == 4) *reinterpret_cast<f32x4*>(dw + col) = s;
-        else st_frag(dw + col, to_frag<bf16>(s));
-    }
-}
-
 // Launch shape shared by both passes and by the workspace size.
 struct NormCfg {
     int n, nv, lpr_log2, rpw, wg_reduce, wg_row;
@@ -527,7 +499,7 @@ extern "C" int hdla_normalize_fwd(const hdla_norm_dims* dims, const void* x, con
 }
 
 static int normalize_bwd(const hdla_norm_dims* dims, const void* x, const void* weight, const void* gate, const void* d_o, void* dx, void* dgate, void* dw,
-                         bool dw_f32, void* workspace, size_t workspace_bytes, void* stream) {
+                         bool dw_f32, void* workspace, size_t workspace_bytes, hdla_sum* later, void* stream) {
     NormCfg c;
     const int rc = norm_config(dims, true, c);
     if (rc) return rc;
@@ -545,23 +517,26 @@ static int normalize_bwd(const hdla_norm_dims* dims, const void* x, const void* 
         const hipError_t e = dims->dtype == HDLA_BF16 ? launch_norm<bf16>(a, c, true, s) : launch_norm<float>(a, c, true, s);
         if (e != hipSuccess) return (int)e;
     }
-    if (weight) {
-        const long long D = (long long)dims->G * dims->E;
-        const dim3 grid((unsigned)((D + 15) / 16));
-        const long long rows = dims->rows > 0 ? c.partial_rows() : 0LL;
-        if (dw_f32) hipLaunchKernelGGL((normalize_dw_kernel<float>), grid, dim3(256), 0, s, a.partial, static_cast<float*>(dw), rows, dims->G, dims->E);
-        else hipLaunchKernelGGL((normalize_dw_kernel<bf16>), grid, dim3(256), 0, s, a.partial, static_cast<bf16*>(dw), rows, dims->G, dims->E);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return (int)e;
-    }
-    return HDLA_OK;
+    if (!weight) return later ? sum_now_or_later(SumJob{}, later, s) : HDLA_OK;
+    // (dw in 32 bits or in the weight's own 16, rounded once: as a launch of its own that was 4.8 us of a training step of the layer)
+    SumJob job{};
+    job.kind = SUM_ROWS;
+    job.blocks = (int)(((long long)dims->G * dims->E + 15) / 16);
+    job.part = a.partial; job.out[0] = dw; job.f32 = dw_f32; job.G = dims->G; job.E = dims->E;
+    job.n = dims->rows > 0 ? c.partial_rows() : 0LL;
+    return sum_now_or_later(job, later, s);
 }
 extern "C" int hdla_normalize_bwd(const hdla_norm_dims* dims, const void* x, const void* weight, const void* gate,
                                   const void* d_o, void* dx, void* dgate, float* dw, void* workspace,
                                   size_t workspace_bytes, void* stream) {
-    return normalize_bwd(dims, x, weight, gate, d_o, dx, dgate, dw, true, workspace, workspace_bytes, stream);
+    return normalize_bwd(dims, x, weight, gate, d_o, dx, dgate, dw, true, workspace, workspace_bytes, nullptr, stream);
 }
 extern "C" int hdla_normalize_bwd_as(const hdla_norm_dims* dims, const void* x, const void* weight, const void* gate, const void* d_o, void* dx,
                                      void* dgate, void* dw, void* workspace, size_t workspace_bytes, void* stream) {
-    return normalize_bwd(dims, x, weight, gate, d_o, dx, dgate, dw, !dims || dims->weight_dtype == HDLA_FP32, workspace, workspace_bytes, stream);
+    return normalize_bwd(dims, x, weight, gate, d_o, dx, dgate, dw, !dims || dims->weight_dtype == HDLA_FP32, workspace, workspace_bytes, nullptr, stream);
+}
+extern "C" int hdla_normalize_bwd_later(const hdla_norm_dims* dims, const void* x, const void* weight, const void* gate, const void* d_o, void* dx,
+                                        void* dgate, void* dw, void* workspace, size_t workspace_bytes, hdla_sum* sum, void* stream) {
+    if (!sum) return HDLA_ERR_NULL;
+    return normalize_bwd(dims, x, weight, gate, d_o, dx, dgate, dw, !dims || dims->weight_dtype == HDLA_FP32, workspace, workspace_bytes, sum, stream);
 }

@@ -10,6 +10,7 @@
 // The contraction index (the row) must be the inner index of both MFMA operands, and both are stored with the row outermost: tiles of
 // 32 rows go through LDS as they come (RowTile) and the transposing LDS read takes them from there.
 #include "row_tile.cuh"
+#include "sums.cuh"
 #include "../../include/hdla_hip.h"
 
 namespace hdla {
@@ -111,27 +112,6 @@ __global__ __launch_bounds__(64 * WW) void skinny_wgrad_kernel(WgradArgs p) {
     }
 }
 
-// dW = sum over the row ranges of their partial results, eight outputs a thread
-__global__ __launch_bounds__(256) void skinny_wgrad_sum_kernel(const float* __restrict__ part0, const float* __restrict__ part1,
-                                                               bf16* __restrict__ dW0, bf16* __restrict__ dW1, long long kn, int S) {
-    const float* const part = blockIdx.y ? part1 : part0;
-    bf16* const dW = blockIdx.y ? dW1 : dW0;
-    const long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 8;
-    if (i >= kn) return;
-    f32x4 a = zero4(), b = zero4();
-    for (int s = 0; s < S; ++s) {
-        a += *reinterpret_cast<const f32x4*>(part + s * kn + i);
-        b += *reinterpret_cast<const f32x4*>(part + s * kn + i + 4);
-    }
-    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-    u32x4 o;
-    o[0] = (uint32_t)f2bf(a[0]) | ((uint32_t)f2bf(a[1]) << 16);
-    o[1] = (uint32_t)f2bf(a[2]) | ((uint32_t)f2bf(a[3]) << 16);
-    o[2] = (uint32_t)f2bf(b[0]) | ((uint32_t)f2bf(b[1]) << 16);
-    o[3] = (uint32_t)f2bf(b[2]) | ((uint32_t)f2bf(b[3]) << 16);
-    *reinterpret_cast<u32x4*>(dW + i) = o;
-}
-
 // row ranges: enough workgroups for the chip (and, when there are many rows, several per CU, about 1024 rows each, so
 // that enough loads are in flight to cover the latency of HBM), whole 32-row tiles each
 static int wgrad_split(long long M, int K, int& rows_per) {
@@ -151,7 +131,7 @@ static int wgrad_split(long long M, int K, int& rows_per) {
 using namespace hdla;
 
 // `count` products (1 or 2), then the sums of their partial results
-static int wgrad_launch(const WgradArgs& a, int N, int S, int count, bf16* dW0, bf16* dW1, hipStream_t s) {
+static int wgrad_launch(const WgradArgs& a, int N, int S, int count, bf16* dW0, bf16* dW1, hdla_sum* later, hipStream_t s) {
     const dim3 block(256);
     // Columns of dY and wavefronts a workgroup.  Many rows, N = 64: whole cache lines of dY and half of the reads of X0; few rows leave
     // some of eight wavefronts without any.  Both products and their sums, us, 32 columns and 4 wavefronts / 64 and 8: 8192 x 1024
@@ -162,10 +142,16 @@ static int wgrad_launch(const WgradArgs& a, int N, int S, int count, bf16* dW0, 
     else hipLaunchKernelGGL((skinny_wgrad_kernel<128, 2, 4>), dim3(a.K / 32, S, count), block, 0, s, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
-    const long long kn = (long long)a.K * N;
-    hipLaunchKernelGGL(skinny_wgrad_sum_kernel, dim3((unsigned)((kn / 8 + 255) / 256), count), block, 0, s, a.part[0], a.part[1], dW0, dW1, kn, S);
-    e = hipGetLastError();
-    return e == hipSuccess ? HDLA_OK : (int)e;
+    SumJob job{};
+    job.kind = SUM_PARTS; job.count = S; job.n = (long long)a.K * N;
+    job.blocks = (int)((job.n / 8 + 255) / 256);
+    hdla_sum own[2];
+    for (int i = 0; i < count; ++i) {
+        job.part = a.part[i];
+        job.out[0] = i ? dW1 : dW0;
+        sum_now_or_later(job, (later ? later : own) + i, s);
+    }
+    return later ? HDLA_OK : hdla_run_sums(own, count, s);
 }
 
 static int wgrad_check(int dtype, int64_t M, int32_t N, int32_t K) {
@@ -198,7 +184,7 @@ extern "C" int hdla_skinny_wgrad(int dtype, int64_t M, int32_t N, int32_t K, con
     WgradArgs a{};
     a.dY[0] = static_cast<const bf16*>(dY); a.X0[0] = static_cast<const bf16*>(X0); a.part[0] = static_cast<float*>(workspace);
     a.ldy = ldy; a.ldx = ldx; a.M = (int)M; a.K = K; a.rows_per = rows_per;
-    return wgrad_launch(a, N, S, 1, static_cast<bf16*>(dW), nullptr, static_cast<hipStream_t>(stream));
+    return wgrad_launch(a, N, S, 1, static_cast<bf16*>(dW), nullptr, nullptr, static_cast<hipStream_t>(stream));
 }
 
 static int up_wgrad_check(const hdla_up_dims* q) {
@@ -215,8 +201,8 @@ extern "C" size_t hdla_layer_up_wgrad_workspace_bytes(const hdla_up_dims* dims) 
     return (size_t)wgrad_split(dims->rows, dims->d, rows_per) * dims->d * dims->D * sizeof(float) * 2;
 }
 
-extern "C" int hdla_layer_up_wgrad(const hdla_up_dims* dims, const void* y, const void* f, const void* dlog_f, const void* dgate, void* dwf,
-                                   void* dwg, void* workspace, size_t workspace_bytes, void* stream) {
+static int layer_up_wgrad(const hdla_up_dims* dims, const void* y, const void* f, const void* dlog_f, const void* dgate, void* dwf, void* dwg, void* workspace,
+                          size_t workspace_bytes, hdla_sum* later, void* stream) {
     const int rc = up_wgrad_check(dims);
     if (rc) return rc;
     if (!y || !f || !dlog_f || !dgate || !dwf || !dwg) return HDLA_ERR_NULL;
@@ -232,7 +218,16 @@ extern "C" int hdla_layer_up_wgrad(const hdla_up_dims* dims, const void* y, cons
     a.X0[0] = static_cast<const bf16*>(y) + dims->col_f; a.X0[1] = static_cast<const bf16*>(y) + dims->col_g;
     a.part[0] = static_cast<float*>(workspace); a.part[1] = a.part[0] + one;
     a.ldy = dims->d; a.ldx = dims->ld; a.M = (int)dims->rows; a.K = dims->d; a.rows_per = rows_per;
-    return wgrad_launch(a, dims->D, S, 2, static_cast<bf16*>(dwf), static_cast<bf16*>(dwg), static_cast<hipStream_t>(stream));
+    return wgrad_launch(a, dims->D, S, 2, static_cast<bf16*>(dwf), static_cast<bf16*>(dwg), later, static_cast<hipStream_t>(stream));
+}
+extern "C" int hdla_layer_up_wgrad(const hdla_up_dims* dims, const void* y, const void* f, const void* dlog_f, const void* dgate, void* dwf,
+                                   void* dwg, void* workspace, size_t workspace_bytes, void* stream) {
+    return layer_up_wgrad(dims, y, f, dlog_f, dgate, dwf, dwg, workspace, workspace_bytes, nullptr, stream);
+}
+extern "C" int hdla_layer_up_wgrad_later(const hdla_up_dims* dims, const void* y, const void* f, const void* dlog_f, const void* dgate, void* dwf,
+                                         void* dwg, void* workspace, size_t workspace_bytes, hdla_sum* sums, void* stream) {
+    if (!sums) return HDLA_ERR_NULL;
+    return layer_up_wgrad(dims, y, f, dlog_f, dgate, dwf, dwg, workspace, workspace_bytes, sums, stream);
 }
 
 extern "C" int hdla_sum_partials(const float* part, int32_t count, int64_t n, void* out, void* stream) {
@@ -241,8 +236,8 @@ extern "C" int hdla_sum_partials(const float* part, int32_t count, int64_t n, vo
     if (!part || !out) return HDLA_ERR_NULL;
     if (((reinterpret_cast<uintptr_t>(part) | reinterpret_cast<uintptr_t>(out)) & 15) != 0) return HDLA_ERR_ALIGN;
     if ((n / 8 + 255) / 256 > 0x7fffffffLL) return HDLA_ERR_SHAPE;
-    hipLaunchKernelGGL(skinny_wgrad_sum_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream), part,
-                       part, static_cast<bf16*>(out), static_cast<bf16*>(out), (long long)n, (int)count);
-    const hipError_t e = hipGetLastError();
-    return e == hipSuccess ? HDLA_OK : (int)e;
+    SumJob job{};
+    job.kind = SUM_PARTS; job.count = (int)count; job.n = (long long)n; job.part = part; job.out[0] = out;
+    job.blocks = (int)((n / 8 + 255) / 256);
+    return sum_now_or_later(job, nullptr, static_cast<hipStream_t>(stream));
 }

@@ -19,8 +19,7 @@
 // computing waves with 128 x 64 each, three quarters of the LDS reads but one wave a SIMD: 74 for the first.
 // A pair, in a training step of the layer: 208 and 64 tiles over 8192 rows, the second in four shares in a launch of its own 82 + 30 us -> 94 together (256 whole
 // tiles, 16 in 16 shares) and 5 for their sums; the step 714 -> 693, with 4096 rows 442 -> 417; 56 and 16 tiles, 8192 rows 408 -> 395.
-#include "hdla_common.cuh"
-#include "../../include/hdla_hip.h"
+#include "sums.cuh"
 
 #include <algorithm>
 
@@ -40,7 +39,7 @@ struct WeightGradArgs {
     int M;
 };
 
-constexpr int WG_TILE = 128, WG_ROWS = 64, WG_SLOTS = 5, WG_LOADERS = 4, WG_COMPUTE = 8;
+constexpr int WG_TILE = SUM_TILE, WG_ROWS = 64, WG_SLOTS = 5, WG_LOADERS = 4, WG_COMPUTE = 8;
 constexpr int WG_OPERAND = WG_ROWS * WG_TILE * 2, WG_STAGE = 2 * WG_OPERAND;
 // loads of a loading wave per stage, and of all stages but the one that is waited for
 constexpr int WG_LOADS = WG_STAGE / 1024 / WG_LOADERS;
@@ -232,26 +231,6 @@ __global__ __launch_bounds__(64 * (WG_LOADERS + WG_COMPUTE)) void weight_grad_ke
     }
 }
 
-// The tiles in shares: their sums, share by share, eight columns a thread
-__global__ __launch_bounds__(256) void weight_grad_sum_kernel(WeightGradArgs p) {
-    const int r = (int)blockIdx.x / 8, e = ((int)blockIdx.x % 8 * 256 + (int)threadIdx.x) * 8;
-    const float* from = p.part + (long long)r * (WG_TILE * WG_TILE) + e;
-    const long long apart = (long long)p.rest * (WG_TILE * WG_TILE);
-    f32x4 lo = zero4(), hi = zero4();
-#pragma unroll 4
-    for (int s = 0; s < p.shares; ++s, from += apart) {
-        lo += *reinterpret_cast<const f32x4*>(from);
-        hi += *reinterpret_cast<const f32x4*>(from + 4);
-    }
-    int tile = p.whole + r;
-    const bool second = tile >= p.first;
-    const WeightGradProduct& of = p.of[second ? 1 : 0];
-    if (second) tile -= p.first;
-    const int kts = of.K / WG_TILE;
-    *reinterpret_cast<s16x8*>(of.dw + (long long)(tile / kts * WG_TILE + e / WG_TILE) * of.K + tile % kts * WG_TILE + e % WG_TILE) =
-        __builtin_shufflevector(to_frag<bf16>(lo).v, to_frag<bf16>(hi).v, 0, 1, 2, 3, 4, 5, 6, 7);
-}
-
 // Tiles and shares of the rows.  Shares: as many as give each compute unit a workgroup, of at least eight stages.  One product has them of all its tiles
 // (none, where they fill the device).
 constexpr int WG_UNITS = 256;                                     // compute units, a workgroup each
@@ -286,7 +265,7 @@ static bool weight_grad_pair(int64_t M, const int32_t* N, const int32_t* K) {
     return true;
 }
 static int weight_grad_run(int64_t M, int count, const int32_t* N, const int32_t* K, const void* const* dY, const int64_t* ldy, const void* const* X,
-                           const int64_t* ldx, void* const* dW, void* workspace, size_t workspace_bytes, void* stream) {
+                           const int64_t* ldx, void* const* dW, void* workspace, size_t workspace_bytes, hdla_sum* later, void* stream) {
     WeightGradArgs a{};
     auto al16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     for (int i = 0; i < count; ++i) if (ldy[i] < N[i] || ldx[i] < K[i] || ldy[i] % 8 || ldx[i] % 8) return HDLA_ERR_SHAPE;
@@ -301,12 +280,16 @@ static int weight_grad_run(int64_t M, int count, const int32_t* N, const int32_t
     a.part = static_cast<float*>(workspace);
     const hipStream_t s = static_cast<hipStream_t>(stream);
     hipLaunchKernelGGL(weight_grad_kernel, dim3((unsigned)(a.whole ? a.whole : a.rest * a.shares)), dim3(64 * (WG_LOADERS + WG_COMPUTE)), 0, s, a);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess && a.shares > 1) {
-        hipLaunchKernelGGL(weight_grad_sum_kernel, dim3((unsigned)(8 * a.rest)), dim3(256), 0, s, a);
-        e = hipGetLastError();
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return (int)e;
+    SumJob job{};
+    if (a.shares > 1) {
+        job.kind = SUM_TILES; job.blocks = 8 * a.rest; job.count = a.shares;
+        job.first = a.first; job.whole = a.whole; job.rest = a.rest;
+        for (int i = 0; i < count; ++i) { job.K[i] = K[i]; job.out[i] = dW[i]; }
+        job.part = a.part;
     }
-    return e == hipSuccess ? HDLA_OK : (int)e;
+    return sum_now_or_later(job, later, s);
 }
 
 extern "C" size_t hdla_weight_grad_workspace_bytes(int64_t M, int32_t N, int32_t K) {
@@ -318,7 +301,7 @@ extern "C" size_t hdla_weight_grad_workspace_bytes(int64_t M, int32_t N, int32_t
 extern "C" int hdla_weight_grad(int64_t M, int32_t N, int32_t K, const void* dY, int64_t ldy, const void* X, int64_t ldx, void* dW, void* workspace,
                                 size_t workspace_bytes, void* stream) {
     if (!weight_grad_shape(M, N, K)) return HDLA_ERR_SHAPE;
-    return weight_grad_run(M, 1, &N, &K, &dY, &ldy, &X, &ldx, &dW, workspace, workspace_bytes, stream);
+    return weight_grad_run(M, 1, &N, &K, &dY, &ldy, &X, &ldx, &dW, workspace, workspace_bytes, nullptr, stream);
 }
 extern "C" size_t hdla_weight_grad_pair_workspace_bytes(int64_t M, const int32_t* N, const int32_t* K) {
     if (!weight_grad_pair(M, N, K)) return 0;
@@ -327,8 +310,8 @@ extern "C" size_t hdla_weight_grad_pair_workspace_bytes(int64_t M, const int32_t
     return weight_grad_room(a);
 }
 extern "C" int hdla_weight_grad_pair(int64_t M, const int32_t* N, const int32_t* K, const void* const* dY, const int64_t* ldy, const void* const* X,
-                                     const int64_t* ldx, void* const* dW, void* workspace, size_t workspace_bytes, void* stream) {
+                                     const int64_t* ldx, void* const* dW, void* workspace, size_t workspace_bytes, hdla_sum* sum, void* stream) {
     if (!dY || !ldy || !X || !ldx || !dW) return HDLA_ERR_NULL;
     if (!weight_grad_pair(M, N, K)) return HDLA_ERR_SHAPE;
-    return weight_grad_run(M, 2, N, K, dY, ldy, X, ldx, dW, workspace, workspace_bytes, stream);
+    return weight_grad_run(M, 2, N, K, dY, ldy, X, ldx, dW, workspace, workspace_bytes, sum, stream);
 }

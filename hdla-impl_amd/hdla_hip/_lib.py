@@ -168,7 +168,7 @@ def load():
     lib.hdla_weight_grad_pair_workspace_bytes.restype = ctypes.c_size_t
     lib.hdla_weight_grad_pair_workspace_bytes.argtypes = [ctypes.c_int64, P, P]
     lib.hdla_weight_grad_pair.restype = ctypes.c_int
-    lib.hdla_weight_grad_pair.argtypes = [ctypes.c_int64, P, P, P, P, P, P, P, P, ctypes.c_size_t, P]
+    lib.hdla_weight_grad_pair.argtypes = [ctypes.c_int64, P, P, P, P, P, P, P, P, ctypes.c_size_t, P, P]
     lib.hdla_stack_rows.restype = ctypes.c_int
     lib.hdla_stack_rows.argtypes = [P, P, ctypes.c_int32, ctypes.c_int64, P, ctypes.c_int64, P]
     _lib = lib

@@ -281,6 +281,11 @@ typedef struct hdla_norm_dims {
 /* weight and gate may be NULL (gate only with gate_pos 0). */
 int hdla_normalize_fwd(const hdla_norm_dims* dims, const void* x, const void* weight, const void* gate, void* o,
                        void* stream);
+/* A sum over partial results in a workspace, left to hdla_run_sums() by the functions that take one (or, hdla_layer_up_wgrad_later(), two): their gradients of
+ * weights are complete, and their workspaces free, behind it.  One launch for up to eight of them.  Opaque; all zeros: nothing to add up. */
+typedef struct hdla_sum { int64_t word[12]; } hdla_sum;
+int hdla_run_sums(const hdla_sum* sums, int32_t count, void* stream);
+
 /* Backward pass; sigma is recomputed.  dw: fp32 [G*E], required iff weight is given; it is summed over rows in a
  * fixed order through `workspace` (hdla_normalize_workspace_bytes() bytes, 16-byte aligned; not needed without a
  * weight).  dgate is required iff gate_pos != 0. */
@@ -290,6 +295,9 @@ int hdla_normalize_bwd(const hdla_norm_dims* dims, const void* x, const void* we
 /* The same with dw [G*E] in the weight's type, rounded once. */
 int hdla_normalize_bwd_as(const hdla_norm_dims* dims, const void* x, const void* weight, const void* gate, const void* d_o, void* dx, void* dgate,
                           void* dw, void* workspace, size_t workspace_bytes, void* stream);
+/* The same, dw's sum left to hdla_run_sums(). */
+int hdla_normalize_bwd_later(const hdla_norm_dims* dims, const void* x, const void* weight, const void* gate, const void* d_o, void* dx, void* dgate,
+                             void* dw, void* workspace, size_t workspace_bytes, hdla_sum* sum, void* stream);
 size_t hdla_normalize_workspace_bytes(const hdla_norm_dims* dims);
 
 /* What the HDLA layer does between its projections and the operator, one pass per direction
@@ -337,10 +345,10 @@ size_t hdla_weight_grad_workspace_bytes(int64_t M, int32_t N, int32_t K);
 int hdla_weight_grad(int64_t M, int32_t N, int32_t K, const void* dY, int64_t ldy, const void* X, int64_t ldx, void* dW, void* workspace,
                      size_t workspace_bytes, void* stream);
 /* Two such products with the same rows in one launch, of up to 256 tiles of 128 x 128 each (else HDLA_ERR_SHAPE); every argument but M, the workspace
- * and the stream is an array of two. */
+ * and those behind dW is an array of two.  sum may be NULL, see hdla_run_sums(). */
 size_t hdla_weight_grad_pair_workspace_bytes(int64_t M, const int32_t* N, const int32_t* K);
 int hdla_weight_grad_pair(int64_t M, const int32_t* N, const int32_t* K, const void* const* dY, const int64_t* ldy, const void* const* X,
-                          const int64_t* ldx, void* const* dW, void* workspace, size_t workspace_bytes, void* stream);
+                          const int64_t* ldx, void* const* dW, void* workspace, size_t workspace_bytes, hdla_sum* sum, void* stream);
 /* out [total_rows, width] (2-byte elements) = the rows of parts[0 .. count) one part behind the other, parts[m] being [rows[m], width],
  * then zeros; count <= 8, width a multiple of 8, everything contiguous and 16-byte aligned.  parts and rows are host arrays. */
 int hdla_stack_rows(const void* const* parts, const int64_t* rows, int32_t count, int64_t width, void* out, int64_t total_rows, void* stream);
@@ -365,6 +373,9 @@ int hdla_layer_down(const hdla_up_dims* dims, const void* wf, const void* wg, co
  * hdla_skinny_wgrad for the pair.  workspace: hdla_layer_up_wgrad_workspace_bytes() bytes, 16-byte aligned. */
 int hdla_layer_up_wgrad(const hdla_up_dims* dims, const void* y, const void* f, const void* dlog_f, const void* dgate,
                         void* dwf, void* dwg, void* workspace, size_t workspace_bytes, void* stream);
+/* The same, the two sums left to hdla_run_sums(). */
+int hdla_layer_up_wgrad_later(const hdla_up_dims* dims, const void* y, const void* f, const void* dlog_f, const void* dgate, void* dwf,
+                              void* dwg, void* workspace, size_t workspace_bytes, hdla_sum* sums, void* stream);
 size_t hdla_layer_up_wgrad_workspace_bytes(const hdla_up_dims* dims);
 
 /* hdla_layer_pre_fwd and hdla_param_recurrent_fwd (scale 1, forward) in one launch, for sequences of T tokens each (rows = N T);

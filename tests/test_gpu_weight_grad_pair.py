@@ -24,7 +24,7 @@ def _call(M, N, K, dy, x, room=None):
     dw = [torch.full((N[i], K[i]), float("nan"), dtype=torch.bfloat16, device=DEV) for i in range(2)]
     p = lambda t: _arr(ctypes.c_void_p, [_lib.ptr(a) for a in t])
     s = lambda t: _arr(ctypes.c_int64, [a.stride(0) for a in t])
-    rc = lib.hdla_weight_grad_pair(M, n, k, p(dy), s(dy), p(x), s(x), p(dw), _lib.ptr(ws), nws if room is None else room, _lib.current_stream(DEV))
+    rc = lib.hdla_weight_grad_pair(M, n, k, p(dy), s(dy), p(x), s(x), p(dw), _lib.ptr(ws), nws if room is None else room, None, _lib.current_stream(DEV))
     return rc, dw, nws
 
 
