@@ -747,6 +747,16 @@ static hipError_t launch_scan_nwc(const ChunkArgs<T>& a, ScanKind kind, hipStrea
 
 template <typename T, int K, int V>
 hipError_t launch_scan_shape(const ChunkArgs<T>& a, ScanKind kind, hipStream_t stream) {
+    // V = 128: all eight column blocks of a head in a workgroup are two waves a SIMD, which wait for each other's products, while compute units without
+    // a workgroup have nothing to do.  Four of them a workgroup take 0.6 of the step (and fetch a chunk's operands twice), so: where twice the workgroups
+    // come in rounds that are the sooner done.  us, fp32 forward passes, eight -> four, K = V = 128 / K = 64: 64 lanes of 19 chunks 165 -> 118 / 102 -> 75, 80 of
+    // 22 201 -> 146 / 114 -> 82, 128 of 19 201 -> 160 / 120 -> 92, but 160 of 19 219 -> 250 / 131 -> 141, 256 of 13 195 -> 219 / 123 -> 132, and again 320 of 13
+    // 301 -> 296 / 186 -> 175; 10 packed sequences of 8 heads, 3546 tokens 418 -> 278 / 231 -> 148.  The same bits.
+    if constexpr (V == 128) {
+        const long long lanes = (long long)a.H * a.st.N * a.seg.nseg * (kind == SCAN_PAIR ? 2 : 1);
+        auto rounds = [](long long workgroups) { return (workgroups + SCAN_TARGET_WORKGROUPS - 1) / SCAN_TARGET_WORKGROUPS; };
+        if (6 * rounds(2 * lanes) < 10 * rounds(lanes)) return launch_scan_nwc<T, K, V, 4>(a, kind, stream);
+    }
     return launch_scan_nwc<T, K, V, V / 16>(a, kind, stream);
 }
 
