@@ -8,7 +8,9 @@
 // A wave owns one 16-column block of the fp32 state of a (sequence, head) for the whole sequence, in
 // registers as the row fragment of S^T (rows = value column, inner = channel), which is at once the operand
 // layout of the next product: w S, qg S and the rank updates chain through registers with no cross-lane
-// movement.  A workgroup holds NWC such waves; a head's V/16 column blocks are split over (V/16)/NWC workgroups.
+// movement.  A workgroup holds NWC such waves; a head's V/16 column blocks are split over (V/16)/NWC workgroups.  (KS = 2: two waves
+// a block, half of the channels each, which hand each other their parts of v_new through LDS, one barrier more a step.  A step of 4-byte elements is
+// bound by its products, 27 of 128 cycles at K = 64 with the output, and so a little more than half as long.)
 //
 // This file: 4-byte elements, and the chaining of the segments' records for both element sizes (2-byte elements: scan_out.cuh,
 // scan_grad.cuh).  All column blocks of a head need the same w / kg / bg / qg tiles: a workgroup fetches the chunk's shared operand block
@@ -27,10 +29,16 @@ namespace hdla {
 
 constexpr int NSLOT = 3;
 
-template <typename T, int K, int V, int NWC> struct ScanCfg {
+template <typename T, int K, int V, int NWC, int KS = 1> struct ScanCfg {
     static constexpr int VT = V / 16, SPLIT = VT / NWC;   // workgroups per head
     static constexpr int KB = K * (int)sizeof(T);         // bytes of one operand row
-    static constexpr int THREADS = 64 * NWC;
+    static constexpr int THREADS = 64 * NWC * KS;
+    // KS = 2, K = 64: two waves a column block, half of the channels each.  v_new and its gradient are then two sums over the channels, of either half; one wave forms
+    // them so too, so that the bits do not depend on how many do.
+    static constexpr bool HALVES = K == 64;
+    static_assert(KS == 1 || (KS == 2 && HALVES), "");
+    // 16-byte pieces that waves of a column block hand each other: the parts of both v_new, and of o
+    static constexpr int HANDED = KS > 1 ? NWC * KS * 3 * 64 : 1;
     // Depth of the register ring of block shares (chunks in flight from global memory) and of the waves' own tiles; a multiple of the
     // number of slots so that slot numbers are static in the unrolled loops; 0: no ring, one chunk at a time.
     static constexpr int DR = KB <= 256 ? 3 : 0;
@@ -116,54 +124,55 @@ constexpr int SCAN_TARGET_WORKGROUPS = 256;               // compute units of th
 // At the end of a segment: column block j of the state, or (trans) of the transition matrix X, whose tile (kt, j) is kept
 // with rows k, inner k', which is how the chain takes it.  turned: where the backward pass will find its own, or null: what the state's gradient
 // meets on its way back through a segment is the transpose of what the state met on its way there.
-template <typename T, int K>
-__device__ __forceinline__ void store_record(const f32x4 (&S)[K / 16], float* loc, float* tr, float* turned, int64_t rec, int V, int j, bool trans) {
-    constexpr int KT = K / 16;
+template <typename T, int K, int KS>
+__device__ __forceinline__ void store_record(const f32x4 (&S)[K / 16 / KS], int kt0, float* loc, float* tr, float* turned, int64_t rec, int V, int j, bool trans) {
+    constexpr int KT = K / 16, KTW = KT / KS;
     if (trans) {
         const Frag<float> ident = ident_frag<float>();
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt) {
+        for (int kt = 0; kt < KTW; ++kt) {
             Frag<float> f;
             f.v = S[kt];
             f = transpose(f, ident);                      // exact: fp32 products with ones and zeros
-            *reinterpret_cast<f32x4*>(tr + rec * (K * K) + (kt * KT + j) * TILE + 4 * lane_id()) = f.v;
+            *reinterpret_cast<f32x4*>(tr + rec * (K * K) + ((kt0 + kt) * KT + j) * TILE + 4 * lane_id()) = f.v;
         }
         if (turned) {
 #pragma unroll
-            for (int kt = 0; kt < KT; ++kt) *reinterpret_cast<f32x4*>(turned + rec * (K * K) + (j * KT + kt) * TILE + 4 * lane_id()) = S[kt];
+            for (int kt = 0; kt < KTW; ++kt) *reinterpret_cast<f32x4*>(turned + rec * (K * K) + (j * KT + kt0 + kt) * TILE + 4 * lane_id()) = S[kt];
         }
     } else {
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt) *reinterpret_cast<f32x4*>(loc + rec * (K * V) + (j * KT + kt) * TILE + 4 * lane_id()) = S[kt];
+        for (int kt = 0; kt < KTW; ++kt) *reinterpret_cast<f32x4*>(loc + rec * (K * V) + (j * KT + kt0 + kt) * TILE + 4 * lane_id()) = S[kt];
     }
 }
 // the columns a segment starts from when it does not start from h0 / dht: the chained state, zeros, or the identity
-template <typename T, int K, bool SUM>
-__device__ __forceinline__ void load_entry(f32x4 (&S)[K / 16], const float* in, int64_t rec, int V, int j, bool trans) {
+template <typename T, int K, bool SUM, int KS>
+__device__ __forceinline__ void load_entry(f32x4 (&S)[K / 16 / KS], int kt0, const float* in, int64_t rec, int V, int j, bool trans) {
     const int l = lane_id(), g = l >> 4, c = l & 15;
 #pragma unroll
-    for (int kt = 0; kt < K / 16; ++kt) {
-        if (!SUM) S[kt] = *reinterpret_cast<const f32x4*>(in + rec * (K * V) + (j * (K / 16) + kt) * TILE + 4 * l);
+    for (int kt = 0; kt < K / 16 / KS; ++kt) {
+        if (!SUM) S[kt] = *reinterpret_cast<const f32x4*>(in + rec * (K * V) + (j * (K / 16) + kt0 + kt) * TILE + 4 * l);
         else if (trans) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) S[kt][i] = (16 * kt + 4 * g + i == 16 * j + c) ? 1.f : 0.f;
+            for (int i = 0; i < 4; ++i) S[kt][i] = (16 * (kt0 + kt) + 4 * g + i == 16 * j + c) ? 1.f : 0.f;
         } else S[kt] = zero4();
     }
 }
 
 // ---- forward -------------------------------------------------------------------------------------------------
 // split: which of the SPLIT groups of NWC column blocks; from SPLIT on (OUT_SUM only), of the transition matrix's
-template <typename T, int K, int V, int NWC, ScanOut OUT>
-__device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem, int n, int seg, int split) {
+template <typename T, int K, int V, int NWC, ScanOut OUT, int KS>
+__device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem, f32x4* handed, int n, int seg, int split) {
     constexpr bool WRITE_O = OUT == OUT_O, SUM = OUT == OUT_SUM;
-    typedef ScanCfg<T, K, V, NWC> C;
-    constexpr int KT = K / 16, KT2 = KT / 2, VT = V / 16;
+    typedef ScanCfg<T, K, V, NWC, KS> C;
+    constexpr int KT = K / 16, KT2 = KT / 2, VT = V / 16, KTW = KT / KS, KTW2 = KTW / 2;
     constexpr BlkF B = blk_fwd(K, sizeof(T), WRITE_O);
     constexpr bool PIPE = C::pipelined(WRITE_O), PIPE_UPD = PIPE && C::early_update_reads();
     constexpr int SLOT = B.SIZE, NI = SLOT / 1024;
 
     const int h = blockIdx.x;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int cb = wv % NWC, ks = KS == 1 ? 0 : wv / NWC, kt0 = ks * KTW, kp0 = kt0 / 2;   // own column block and channel tiles
     const bool trans = SUM && split >= C::SPLIT;
     const int vt0 = (trans ? split - C::SPLIT : split) * NWC;     // first column block of this workgroup
     const int own0 = trans ? 0 : vt0;                     // of its tiles of u^T, v^T (transition columns take none: never used)
@@ -187,36 +196,36 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
         return BlockOne{b};
     };
 
-    const int vt = vt0 + wv;
+    const int vt = vt0 + cb;
     // state block: lane (g,c) reg i of tile kt = S[16kt + 4g + i][16vt + c]
-    f32x4 S[KT];
+    f32x4 S[KTW];
     const int64_t soff = ((int64_t)n * H + h) * K * V + 16 * vt + c;
 #pragma unroll
-    for (int kt = 0; kt < KT; ++kt) S[kt] = zero4();
+    for (int kt = 0; kt < KTW; ++kt) S[kt] = zero4();
     if (seg > 0) {
-        load_entry<T, K, SUM>(S, p.seg.in, rec, V, vt, trans);
+        load_entry<T, K, SUM, KS>(S, kt0, p.seg.in, rec, V, vt, trans);
     } else if (p.h0) {
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt)
+        for (int kt = 0; kt < KTW; ++kt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) S[kt][i] = p.h0[soff + (int64_t)(16 * kt + 4 * g + i) * V];
+            for (int i = 0; i < 4; ++i) S[kt][i] = p.h0[soff + (int64_t)(16 * (kt0 + kt) + 4 * g + i) * V];
     }
     struct Own { Frag<T> ut[2], vtt; };                   // the tiles only this wave reads
     auto load_own = [&](Own& o, int t) __attribute__((always_inline)) {
         const int64_t chw = chw0 + min(c0 + t, last);
-        ld_pair(p.ws.UT + (chw * VT + own0 + wv % VT) * PAIR, o.ut[0], o.ut[1]);
-        o.vtt = ld_tile(p.ws.VTT + (chw * VT + own0 + wv % VT) * TILE);
+        ld_pair(p.ws.UT + (chw * VT + own0 + cb % VT) * PAIR, o.ut[0], o.ut[1]);
+        o.vtt = ld_tile(p.ws.VTT + (chw * VT + own0 + cb % VT) * TILE);
     };
 
-    Frag<T> w[2][KT];                                     // phase-1 operands; when pipelined, read a step ahead
+    Frag<T> w[2][KTW];                                     // phase-1 operands; when pipelined, read a step ahead
     auto read_w = [&](const char* slot, int kp) __attribute__((always_inline)) {
         const T* sW = reinterpret_cast<const T*>(slot + B.W);
-        ld_pair(sW + (0 * KT2 + kp) * PAIR, w[0][2 * kp], w[0][2 * kp + 1]);
-        ld_pair(sW + (1 * KT2 + kp) * PAIR, w[1][2 * kp], w[1][2 * kp + 1]);
+        ld_pair(sW + (0 * KT2 + kp0 + kp) * PAIR, w[0][2 * kp], w[0][2 * kp + 1]);
+        ld_pair(sW + (1 * KT2 + kp0 + kp) * PAIR, w[1][2 * kp], w[1][2 * kp + 1]);
     };
     auto read_w_all = [&](const char* slot) __attribute__((always_inline)) {
 #pragma unroll
-        for (int kp = 0; kp < KT2; ++kp) read_w(slot, kp);
+        for (int kp = 0; kp < KTW2; ++kp) read_w(slot, kp);
     };
 
     // one chunk: shared operands from `slot`, the phase-1 operands of the next chunk from `slot_next`
@@ -229,44 +238,69 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
         const T* sBGT = reinterpret_cast<const T*>(slot + B.BGT);
         const T* sKGT = reinterpret_cast<const T*>(slot + B.KGT);
         const float* sEGL = reinterpret_cast<const float*>(slot + B.EGL);
-        Frag<T> qg[WRITE_O ? KT : 1], aqk, aqb[2], kgt[KT], bgt[2][KT];
-        f32x4 egl[KT];
+        Frag<T> qg[WRITE_O ? KTW : 1], aqk, aqb[2], kgt[KTW], bgt[2][KTW];
+        f32x4 egl[KTW];
         auto read_qg = [&](int kp) __attribute__((always_inline)) {
-            ld_pair(reinterpret_cast<const T*>(slot + B.QG) + kp * PAIR, qg[2 * kp], qg[2 * kp + 1]);
+            ld_pair(reinterpret_cast<const T*>(slot + B.QG) + (kp0 + kp) * PAIR, qg[2 * kp], qg[2 * kp + 1]);
         };
         auto read_upd = [&](int kp) __attribute__((always_inline)) {
-            ld_pair(sKGT + kp * PAIR, kgt[2 * kp], kgt[2 * kp + 1]);
-            ld_pair(sBGT + (0 * KT2 + kp) * PAIR, bgt[0][2 * kp], bgt[0][2 * kp + 1]);
-            ld_pair(sBGT + (1 * KT2 + kp) * PAIR, bgt[1][2 * kp], bgt[1][2 * kp + 1]);
-            egl[2 * kp] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (2 * kp) + 4 * g);
-            egl[2 * kp + 1] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (2 * kp + 1) + 4 * g);
+            ld_pair(sKGT + (kp0 + kp) * PAIR, kgt[2 * kp], kgt[2 * kp + 1]);
+            ld_pair(sBGT + (0 * KT2 + kp0 + kp) * PAIR, bgt[0][2 * kp], bgt[0][2 * kp + 1]);
+            ld_pair(sBGT + (1 * KT2 + kp0 + kp) * PAIR, bgt[1][2 * kp], bgt[1][2 * kp + 1]);
+            egl[2 * kp] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (kt0 + 2 * kp) + 4 * g);
+            egl[2 * kp + 1] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (kt0 + 2 * kp + 1) + 4 * g);
         };
         if (WRITE_O) {
             ld_pair(reinterpret_cast<const T*>(slot + B.AQB), aqb[0], aqb[1]);
             aqk = ld_tile(reinterpret_cast<const T*>(slot + B.AQK));
         }
-        Frag<T> sb[KT];
+        Frag<T> sb[KTW];
         // v_new^T (rows value, inner token) = u^T + S^T w^T; what is read on the way is used a group of products later or after
-        f32x4 vn[2] = {to_f32(own.ut[0]), to_f32(own.ut[1])};
+        f32x4 vn[2] = {to_f32(own.ut[0]), to_f32(own.ut[1])}, rest = zero4();
+        if (ks) { vn[0] = zero4(); vn[1] = zero4(); }
+        if constexpr (KS == 1 && PIPE && C::HALVES) {
 #pragma unroll
-        for (int kp = 0; kp < KT2; ++kp) {
-            if (PIPE && WRITE_O) read_qg(kp);
-            if (PIPE_UPD && !WRITE_O) read_upd(kp);
-            if (!PIPE) read_w(slot, kp);
-            if (PIPE) __builtin_amdgcn_sched_barrier(0);
+            for (int kt = 0; kt < KT; ++kt) sb[kt] = to_frag<T>(S[kt]);
 #pragma unroll
-            for (int kt = 2 * kp; kt < 2 * kp + 2; ++kt) {
-                sb[kt] = to_frag<T>(S[kt]);
-                vn[0] = mm(sb[kt], w[0][kt], vn[0]);
-                vn[1] = mm(sb[kt], w[1][kt], vn[1]);
+            for (int r = 0; r < 2; ++r) {
+                if (WRITE_O) read_qg(r);
+                if (PIPE_UPD && !WRITE_O) read_upd(r);
+                __builtin_amdgcn_sched_barrier(0);
+                if (r) vn[0] += rest;                     // (in the shadow of the products)
+                rest = zero4();
+#pragma unroll
+                for (int kt = 0; kt < KT; ++kt) {
+                    f32x4& x = kt < KT2 ? vn[r] : rest;
+                    x = mm(sb[kt], w[r][kt], x);
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
-            if (PIPE) __builtin_amdgcn_sched_barrier(0);
-        }
-        f32x4 o = zero4();
-        if (WRITE_O) {
-            // o (rows token, inner value) = qg S + A_qk v + sum_s A_qb^s v_new_s; the first two terms here
+        } else {
+            f32x4 x2[2] = {zero4(), zero4()};
 #pragma unroll
-            for (int kp = 0; kp < KT2; ++kp) {
+            for (int kp = 0; kp < KTW2; ++kp) {
+                if (PIPE && WRITE_O) read_qg(kp);
+                if (PIPE_UPD && !WRITE_O) read_upd(kp);
+                if (!PIPE) read_w(slot, kp);
+                if (PIPE) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int kt = 2 * kp; kt < 2 * kp + 2; ++kt) {
+                    sb[kt] = to_frag<T>(S[kt]);
+                    f32x4 (&x)[2] = C::HALVES && kt >= KT2 ? x2 : vn;
+                    x[0] = mm(sb[kt], w[0][kt], x[0]);
+                    x[1] = mm(sb[kt], w[1][kt], x[1]);
+                }
+                if (PIPE) __builtin_amdgcn_sched_barrier(0);
+            }
+            if (KS == 1 && C::HALVES) { vn[0] += x2[0]; rest = x2[1]; }
+        }
+        f32x4* const mine = handed + (cb * KS + ks) * 192 + l;
+        const f32x4* const other = handed + (cb * KS + (ks ^ 1)) * 192 + l;
+        if (KS > 1) { mine[0] = vn[0]; mine[64] = vn[1]; }
+        f32x4 o = zero4();
+        auto out_of_state = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int kp = 0; kp < KTW2; ++kp) {
                 if (PIPE_UPD) read_upd(kp);
                 if (!PIPE) read_qg(kp);
                 if (PIPE) __builtin_amdgcn_sched_barrier(0);
@@ -274,38 +308,56 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
                 o = mm(qg[2 * kp + 1], sb[2 * kp + 1], o);
                 if (PIPE) __builtin_amdgcn_sched_barrier(0);
             }
-            o = mm(aqk, own.vtt, o);
+        };
+        // o (rows token, inner value) = qg S + A_qk v + sum_s A_qb^s v_new_s, one sum in this order: the wave of the channels' first half begins it
+        // and the one of the second half goes on, when the first two of these are there
+        if (WRITE_O && !ks) {
+            out_of_state();
+            if (KS > 1) mine[128] = o;
         }
+        if (KS > 1) lds_barrier();
+        if (WRITE_O && KS > 1 && ks) {
+            o = other[128];
+            out_of_state();
+        }
+        if (WRITE_O && ks == KS - 1) o = mm(aqk, own.vtt, o);
+        Frag<T> vnb[2];
+        auto sum_up = [&]() __attribute__((always_inline)) {
+            if (KS > 1) { vn[0] += other[0]; vn[1] += other[64]; }
+            else if (C::HALVES) vn[1] += rest;
+            vnb[0] = to_frag<T>(vn[0]);
+            vnb[1] = to_frag<T>(vn[1]);
+        };
+        if (WRITE_O || KS > 1) sum_up();
         if (PIPE) __builtin_amdgcn_sched_barrier(0);
-        const Frag<T> vnb[2] = {to_frag<T>(vn[0]), to_frag<T>(vn[1])};
         if (OUT == OUT_STATE) {
             // checkpoint of the entering state, as the fragments held here (tile pairs, 16 bytes per lane, whole
             // cache lines): the chunk_grad kernel turns them the way it needs them
             T* hc = p.ws.HC + chw * (K * V) + vt * PAIR;
             constexpr int HSTR = VT * PAIR;               // elements between the pairs of consecutive channel tiles
 #pragma unroll
-            for (int kp = 0; kp < KT2; ++kp) st_pair2(hc + kp * HSTR, sb[2 * kp], sb[2 * kp + 1]);
+            for (int kp = 0; kp < KTW2; ++kp) st_pair2(hc + (kp0 + kp) * HSTR, sb[2 * kp], sb[2 * kp + 1]);
         }
-        if (WRITE_O) {
+        if (WRITE_O && ks == KS - 1) {
             o = mm(aqb[0], vnb[0], o);
             o = mm(aqb[1], vnb[1], o);
             if (c < len) st_frag(p.o + ((tok0 + c) * H + h) * V + 16 * vt + 4 * g, to_frag<T>(o));
         }
         // S <- exp(g_last) S + kg^T v + sum_s bg_s^T v_new_s
 #pragma unroll
-        for (int kp = 0; kp < KT2; ++kp) {
+        for (int kp = 0; kp < KTW2; ++kp) {
             if (!PIPE_UPD) read_upd(kp);
             if (PIPE) {                             // (those of phase 1, whose products have taken them already)
                 read_w(slot_next, kp);
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
+            for (int kt = 2 * kp; kt < 2 * kp + 2; ++kt) S[kt] = mm(own.vtt, kgt[kt], S[kt] * egl[kt]);
+            if (kp == 0 && !WRITE_O && KS == 1) sum_up();   // (in the shadow of these)
+#pragma unroll
             for (int kt = 2 * kp; kt < 2 * kp + 2; ++kt) {
-                f32x4 x = S[kt] * egl[kt];
-                x = mm(own.vtt, kgt[kt], x);
-                x = mm(vnb[0], bgt[0][kt], x);
-                x = mm(vnb[1], bgt[1][kt], x);
-                S[kt] = x;
+                S[kt] = mm(vnb[0], bgt[0][kt], S[kt]);
+                S[kt] = mm(vnb[1], bgt[1][kt], S[kt]);
             }
             if (PIPE) __builtin_amdgcn_sched_barrier(0);
         }
@@ -315,7 +367,7 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
         constexpr int DR = C::DR;
         int done = 0;
         if constexpr (DR > 0) {
-            Share<T, NI, NWC> sh[DR];
+            Share<T, NI, NWC * KS> sh[DR];
             Own own[DR];
 #pragma unroll
             for (int d = 0; d < DR; ++d) {
@@ -345,7 +397,7 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
             }
             done = nfull * DR;
         } else {
-            Share<T, NI, NWC> tmp;
+            Share<T, NI, NWC * KS> tmp;
             tmp.load(blk(0), wv);
             tmp.to_lds(smem, wv);
             tmp.load(blk(1), wv);
@@ -360,7 +412,7 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
 #pragma unroll 1
             for (int t = done; t < nchunks; ++t) {
                 lds_barrier();
-                Share<T, NI, NWC> tmp;
+                Share<T, NI, NWC * KS> tmp;
                 tmp.load(blk(t + 2), wv);
                 Own nxt;
                 load_own(nxt, t + 1);
@@ -371,22 +423,22 @@ __device__ __forceinline__ void scan_fwd_body(const ChunkArgs<T>& p, char* smem,
         }
     }
     if (SUM) {
-        store_record<T, K>(S, p.seg.loc, p.seg.tr, p.seg.turned, rec, V, vt, trans);
+        store_record<T, K, KS>(S, kt0, p.seg.loc, p.seg.tr, p.seg.turned, rec, V, vt, trans);
     } else if (p.ht && seg == p.seg.nseg - 1) {
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt)
+        for (int kt = 0; kt < KTW; ++kt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) p.ht[soff + (int64_t)(16 * kt + 4 * g + i) * V] = S[kt][i];
+            for (int i = 0; i < 4; ++i) p.ht[soff + (int64_t)(16 * (kt0 + kt) + 4 * g + i) * V] = S[kt][i];
     }
 }
 
 // ---- backward ------------------------------------------------------------------------------------------------
 // Step t handles chunk c1-1-t.
-template <typename T, int K, int V, int NWC, ScanOut OUT>
-__device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem, int n, int seg, int split) {
+template <typename T, int K, int V, int NWC, ScanOut OUT, int KS>
+__device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem, f32x4* handed, int n, int seg, int split) {
     constexpr bool SUM = OUT == OUT_SUM;
-    typedef ScanCfg<T, K, V, NWC> C;
-    constexpr int KT = K / 16, KT2 = KT / 2, VT = V / 16;
+    typedef ScanCfg<T, K, V, NWC, KS> C;
+    constexpr int KT = K / 16, KT2 = KT / 2, VT = V / 16, KTW = KT / KS, KTW2 = KTW / 2;
     // LDS slot: [BG | WT] (BGT and W of the forward-scan block, transposed on their way in) | EGL | QGT | AQBT
     constexpr SlotB B = slot_bwd(K, sizeof(T));
     constexpr int SBWD = blk_bwd(K, sizeof(T)).SIZE, NT = B.NIF;
@@ -396,6 +448,7 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
 
     const int h = blockIdx.x;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int cb = wv % NWC, ks = KS == 1 ? 0 : wv / NWC, kt0 = ks * KTW, kp0 = kt0 / 2;   // own column block and channel tiles
     const bool trans = SUM && split >= C::SPLIT;
     const int vt0 = (trans ? split - C::SPLIT : split) * NWC;
     const int l = lane_id(), g = l >> 4, c = l & 15;
@@ -414,18 +467,18 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
         return BlockTwo<T, K>{reinterpret_cast<const char*>(p.ws.W) + slot * SFWD, reinterpret_cast<const char*>(p.ws.QGT) + slot * SBWD};
     };
 
-    const int vt = vt0 + wv;
-    f32x4 dS[KT];   // lane (g,c) reg i of tile kt = dS[16kt + 4g + i][16vt + c]
+    const int vt = vt0 + cb;
+    f32x4 dS[KTW];   // lane (g,c) reg i of tile kt = dS[16kt + 4g + i][16vt + c]
     const int64_t soff = ((int64_t)n * H + h) * K * V + 16 * vt + c;
 #pragma unroll
-    for (int kt = 0; kt < KT; ++kt) dS[kt] = zero4();
+    for (int kt = 0; kt < KTW; ++kt) dS[kt] = zero4();
     if (seg < p.seg.nseg - 1) {
-        load_entry<T, K, SUM>(dS, p.seg.rin, rec, V, vt, trans);
+        load_entry<T, K, SUM, KS>(dS, kt0, p.seg.rin, rec, V, vt, trans);
     } else if (p.dht) {
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt)
+        for (int kt = 0; kt < KTW; ++kt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) dS[kt][i] = p.dht[soff + (int64_t)(16 * kt + 4 * g + i) * V];
+            for (int i = 0; i < 4; ++i) dS[kt][i] = p.dht[soff + (int64_t)(16 * (kt0 + kt) + 4 * g + i) * V];
     }
     const Frag<T> ident = ident_frag<T>();
     // rows of do; rows past the end of a ragged chunk alias its last row and are zeroed where used
@@ -436,16 +489,16 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
         don = ld_frag(p.dout + ((tok0 + min(c, len - 1)) * H + h) * V + 16 * (trans ? 0 : vt) + 4 * g);
     };
 
-    Frag<T> aq[2], bg[2][KT];                             // phase-1 operands; when pipelined, read a step ahead
+    Frag<T> aq[2], bg[2][KTW];                             // phase-1 operands; when pipelined, read a step ahead
     auto read_bg = [&](const char* slot, int kp) __attribute__((always_inline)) {
         const T* sBG = reinterpret_cast<const T*>(slot + B.BGT);
-        ld_pair(sBG + (0 * KT2 + kp) * PAIR, bg[0][2 * kp], bg[0][2 * kp + 1]);
-        ld_pair(sBG + (1 * KT2 + kp) * PAIR, bg[1][2 * kp], bg[1][2 * kp + 1]);
+        ld_pair(sBG + (0 * KT2 + kp0 + kp) * PAIR, bg[0][2 * kp], bg[0][2 * kp + 1]);
+        ld_pair(sBG + (1 * KT2 + kp0 + kp) * PAIR, bg[1][2 * kp], bg[1][2 * kp + 1]);
     };
     auto read_p1_all = [&](const char* slot) __attribute__((always_inline)) {
         ld_pair(reinterpret_cast<const T*>(slot + B.AQBT), aq[0], aq[1]);
 #pragma unroll
-        for (int kp = 0; kp < KT2; ++kp) read_bg(slot, kp);
+        for (int kp = 0; kp < KTW2; ++kp) read_bg(slot, kp);
     };
 
     auto step = [&](const char* slot, const char* slot_next, Frag<T> don, int t) __attribute__((always_inline)) {
@@ -454,50 +507,84 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
         const T* sWT = reinterpret_cast<const T*>(slot + B.W);
         const T* sQGT = reinterpret_cast<const T*>(slot + B.QGT);
         const float* sEGL = reinterpret_cast<const float*>(slot + B.EGL);
-        Frag<T> qgt[KT], wt[2][KT];
-        f32x4 egl[KT];
+        Frag<T> qgt[KTW], wt[2][KTW];
+        f32x4 egl[KTW];
         auto read_upd = [&](int kp) __attribute__((always_inline)) {
-            ld_pair(sQGT + kp * PAIR, qgt[2 * kp], qgt[2 * kp + 1]);
-            ld_pair(sWT + (0 * KT2 + kp) * PAIR, wt[0][2 * kp], wt[0][2 * kp + 1]);
-            ld_pair(sWT + (1 * KT2 + kp) * PAIR, wt[1][2 * kp], wt[1][2 * kp + 1]);
-            egl[2 * kp] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (2 * kp) + 4 * g);
-            egl[2 * kp + 1] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (2 * kp + 1) + 4 * g);
+            ld_pair(sQGT + (kp0 + kp) * PAIR, qgt[2 * kp], qgt[2 * kp + 1]);
+            ld_pair(sWT + (0 * KT2 + kp0 + kp) * PAIR, wt[0][2 * kp], wt[0][2 * kp + 1]);
+            ld_pair(sWT + (1 * KT2 + kp0 + kp) * PAIR, wt[1][2 * kp], wt[1][2 * kp + 1]);
+            egl[2 * kp] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (kt0 + 2 * kp) + 4 * g);
+            egl[2 * kp + 1] = *reinterpret_cast<const f32x4*>(sEGL + 16 * (kt0 + 2 * kp + 1) + 4 * g);
         };
         if (!PIPE) ld_pair(reinterpret_cast<const T*>(slot + B.AQBT), aq[0], aq[1]);
-        Frag<T> dsb[KT];
+        Frag<T> dsb[KTW];
         const int len = (int)min((int64_t)CH, eos - (bos + (int64_t)(cid - c0) * CH));
         if (c >= len || trans) don = zero_frag<T>();
         const Frag<T> doT = transpose(don, ident);          // rows value, inner token
         // dv_new_s^T (rows value, inner token) = do^T A_qb^s + dS^T bg_s^T; what is read here is used a phase later
-        f32x4 dvn[2];
-        dvn[0] = mm(doT, aq[0], zero4());
-        dvn[1] = mm(doT, aq[1], zero4());
-#pragma unroll
-        for (int kp = 0; kp < KT2; ++kp) {
-            if (PIPE_UPD) read_upd(kp);
-            if (!PIPE) read_bg(slot, kp);
-            if (PIPE) __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int kt = 2 * kp; kt < 2 * kp + 2; ++kt) {
-                dsb[kt] = to_frag<T>(dS[kt]);
-                dvn[0] = mm(dsb[kt], bg[0][kt], dvn[0]);
-                dvn[1] = mm(dsb[kt], bg[1][kt], dvn[1]);
-            }
-            if (PIPE) __builtin_amdgcn_sched_barrier(0);
+        f32x4 dvn[2] = {zero4(), zero4()}, rest = zero4();
+        if (!ks) {
+            dvn[0] = mm(doT, aq[0], zero4());
+            dvn[1] = mm(doT, aq[1], zero4());
         }
-        const Frag<T> dvb[2] = {to_frag<T>(dvn[0]), to_frag<T>(dvn[1])};
+        if constexpr (KS == 1 && PIPE_UPD && C::HALVES) {
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt) dsb[kt] = to_frag<T>(dS[kt]);
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                read_upd(r);
+                __builtin_amdgcn_sched_barrier(0);
+                if (r) dvn[0] += rest;                    // (in the shadow of the products)
+                rest = zero4();
+#pragma unroll
+                for (int kt = 0; kt < KT; ++kt) {
+                    f32x4& x = kt < KT2 ? dvn[r] : rest;
+                    x = mm(dsb[kt], bg[r][kt], x);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+            f32x4 x2[2] = {zero4(), zero4()};
+#pragma unroll
+            for (int kp = 0; kp < KTW2; ++kp) {
+                if (PIPE_UPD) read_upd(kp);
+                if (!PIPE) read_bg(slot, kp);
+                if (PIPE) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int kt = 2 * kp; kt < 2 * kp + 2; ++kt) {
+                    dsb[kt] = to_frag<T>(dS[kt]);
+                    f32x4 (&x)[2] = C::HALVES && kt >= KT2 ? x2 : dvn;
+                    x[0] = mm(dsb[kt], bg[0][kt], x[0]);
+                    x[1] = mm(dsb[kt], bg[1][kt], x[1]);
+                }
+                if (PIPE) __builtin_amdgcn_sched_barrier(0);
+            }
+            if (KS == 1 && C::HALVES) { dvn[0] += x2[0]; rest = x2[1]; }
+        }
+        f32x4* const mine = handed + (cb * KS + ks) * 192 + l;
+        const f32x4* const other = handed + (cb * KS + (ks ^ 1)) * 192 + l;
+        if (KS > 1) {
+            mine[0] = dvn[0];
+            mine[64] = dvn[1];
+            lds_barrier();
+        }
+        Frag<T> dvb[2];
+        auto sum_up = [&]() __attribute__((always_inline)) {
+            if (KS > 1) { dvn[0] += other[0]; dvn[1] += other[64]; }
+            else if (C::HALVES) dvn[1] += rest;
+            dvb[0] = to_frag<T>(dvn[0]);
+            dvb[1] = to_frag<T>(dvn[1]);
+        };
         // gradient of the state leaving the chunk and of v_new, as the fragments held here (tile pairs)
         if constexpr (!SUM) {
-        T* dhc = p.ws.DHC + chw * (K * V) + vt * PAIR;
-        T* dvp = p.ws.DVN + chw * (2 * CH * V) + vt * PAIR;
-        constexpr int HSTR = VT * PAIR;
+            T* dhc = p.ws.DHC + chw * (K * V) + vt * PAIR;
+            constexpr int HSTR = VT * PAIR;
 #pragma unroll
-        for (int kp = 0; kp < KT2; ++kp) st_pair2(dhc + kp * HSTR, dsb[2 * kp], dsb[2 * kp + 1]);
-        st_pair2(dvp, dvb[0], dvb[1]);
+            for (int kp = 0; kp < KTW2; ++kp) st_pair2(dhc + (kp0 + kp) * HSTR, dsb[2 * kp], dsb[2 * kp + 1]);
         }
         // dS <- exp(g_last) dS + qg^T do + sum_s w_s^T dv_new_s
 #pragma unroll
-        for (int kp = 0; kp < KT2; ++kp) {
+        for (int kp = 0; kp < KTW2; ++kp) {
             if (!PIPE_UPD) read_upd(kp);
             if (PIPE) {                             // (those of phase 1, whose products have taken them already)
                 if (kp == 0) ld_pair(reinterpret_cast<const T*>(slot_next + B.AQBT), aq[0], aq[1]);
@@ -505,22 +592,23 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
+            for (int kt = 2 * kp; kt < 2 * kp + 2; ++kt) dS[kt] = mm(doT, qgt[kt], dS[kt] * egl[kt]);
+            if (kp == 0) sum_up();                          // (in the shadow of these)
+#pragma unroll
             for (int kt = 2 * kp; kt < 2 * kp + 2; ++kt) {
-                f32x4 x = dS[kt] * egl[kt];
-                x = mm(doT, qgt[kt], x);
-                x = mm(dvb[0], wt[0][kt], x);
-                x = mm(dvb[1], wt[1][kt], x);
-                dS[kt] = x;
+                dS[kt] = mm(dvb[0], wt[0][kt], dS[kt]);
+                dS[kt] = mm(dvb[1], wt[1][kt], dS[kt]);
             }
             if (PIPE) __builtin_amdgcn_sched_barrier(0);
         }
+        if (!SUM && !ks) st_pair2(p.ws.DVN + chw * (2 * CH * V) + vt * PAIR, dvb[0], dvb[1]);
     };
 
     if (nchunks > 0) {
         constexpr int DR = C::DR;
         int done = 0;
         if constexpr (DR > 0) {
-            Share<T, NI, NWC, NT> sh[DR];
+            Share<T, NI, NWC * KS, NT> sh[DR];
             Frag<T> own[DR];
 #pragma unroll
             for (int d = 0; d < DR; ++d) {
@@ -548,7 +636,7 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
             }
             done = nfull * DR;
         } else {
-            Share<T, NI, NWC, NT> tmp;
+            Share<T, NI, NWC * KS, NT> tmp;
             tmp.load(blk(0), wv);
             tmp.to_lds(smem, wv);
             tmp.load(blk(1), wv);
@@ -562,7 +650,7 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
 #pragma unroll 1
             for (int t = done; t < nchunks; ++t) {
                 lds_barrier();
-                Share<T, NI, NWC, NT> tmp;
+                Share<T, NI, NWC * KS, NT> tmp;
                 tmp.load(blk(t + 2), wv);
                 Frag<T> nxt;
                 load_own(nxt, t + 1);
@@ -573,12 +661,12 @@ __device__ __forceinline__ void scan_bwd_body(const ChunkArgs<T>& p, char* smem,
         }
     }
     if (SUM) {
-        store_record<T, K>(dS, p.seg.rloc, p.seg.rtr, nullptr, rec, V, vt, trans);
+        store_record<T, K, KS>(dS, kt0, p.seg.rloc, p.seg.rtr, nullptr, rec, V, vt, trans);
     } else if (p.dh0 && seg == 0) {
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt)
+        for (int kt = 0; kt < KTW; ++kt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) p.dh0[soff + (int64_t)(16 * kt + 4 * g + i) * V] = dS[kt][i];
+            for (int i = 0; i < 4; ++i) p.dh0[soff + (int64_t)(16 * (kt0 + kt) + 4 * g + i) * V] = dS[kt][i];
     }
 }
 
@@ -609,48 +697,52 @@ template <int V> __device__ __forceinline__ bool scan_share(const SeqTab& st, in
     split = unit - __builtin_amdgcn_readlane(end - own, r);
     return true;
 }
-template <typename T, int K, int V, int NWC, bool WRITE_O>
-__global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_fwd_kernel(ChunkArgs<T> p) {
+template <typename T, int K, int V, int NWC, int KS, bool WRITE_O>
+__global__ __launch_bounds__((ScanCfg<T, K, V, NWC, KS>::THREADS)) void scan_fwd_kernel(ChunkArgs<T> p) {
     constexpr ScanOut OUT = WRITE_O ? OUT_O : OUT_STATE;
     __shared__ __attribute__((aligned(16))) char smem[NSLOT * blk_fwd(K, sizeof(T), WRITE_O).SIZE];
+    __shared__ f32x4 handed[ScanCfg<T, K, V, NWC, KS>::HANDED];
     const int z = blockIdx.z / p.seg.nseg, seg = blockIdx.z % p.seg.nseg;
-    scan_fwd_body<T, K, V, NWC, OUT>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
+    scan_fwd_body<T, K, V, NWC, OUT, KS>(p, smem, handed, scan_sequence(p.st, z), seg, blockIdx.y);
 }
-template <typename T, int K, int V, int NWC>
-__global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_bwd_kernel(ChunkArgs<T> p) {
+template <typename T, int K, int V, int NWC, int KS>
+__global__ __launch_bounds__((ScanCfg<T, K, V, NWC, KS>::THREADS)) void scan_bwd_kernel(ChunkArgs<T> p) {
     __shared__ __attribute__((aligned(16))) char smem[NSLOT * slot_bwd(K, sizeof(T)).SIZE];
+    __shared__ f32x4 handed[ScanCfg<T, K, V, NWC, KS>::HANDED];
     const int z = blockIdx.z / p.seg.nseg, seg = blockIdx.z % p.seg.nseg;
-    scan_bwd_body<T, K, V, NWC, OUT_GRAD>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
+    scan_bwd_body<T, K, V, NWC, OUT_GRAD, KS>(p, smem, handed, scan_sequence(p.st, z), seg, blockIdx.y);
 }
 // Both scans of the backward pass in one launch: they depend on the prep kernel only, not on each other.
-template <typename T, int K, int V, int NWC>
-__global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_pair_kernel(ChunkArgs<T> p) {
+template <typename T, int K, int V, int NWC, int KS>
+__global__ __launch_bounds__((ScanCfg<T, K, V, NWC, KS>::THREADS)) void scan_pair_kernel(ChunkArgs<T> p) {
     constexpr int NF = NSLOT * blk_fwd(K, sizeof(T), false).SIZE;
     constexpr int NB = NSLOT * slot_bwd(K, sizeof(T)).SIZE;
-    constexpr int SPLIT = ScanCfg<T, K, V, NWC>::SPLIT;
+    constexpr int SPLIT = ScanCfg<T, K, V, NWC, KS>::SPLIT;
     __shared__ __attribute__((aligned(16))) char smem[NF > NB ? NF : NB];
+    __shared__ f32x4 handed[ScanCfg<T, K, V, NWC, KS>::HANDED];
     const int z = blockIdx.z / p.seg.nseg, seg = blockIdx.z % p.seg.nseg;
     const int n = scan_sequence(p.st, z);
-    if (blockIdx.y < SPLIT) scan_fwd_body<T, K, V, NWC, OUT_STATE>(p, smem, n, seg, blockIdx.y);
-    else scan_bwd_body<T, K, V, NWC, OUT_GRAD>(p, smem, n, seg, blockIdx.y - SPLIT);
+    if (blockIdx.y < SPLIT) scan_fwd_body<T, K, V, NWC, OUT_STATE, KS>(p, smem, handed, n, seg, blockIdx.y);
+    else scan_bwd_body<T, K, V, NWC, OUT_GRAD, KS>(p, smem, handed, n, seg, blockIdx.y - SPLIT);
 }
 // The segments' records: grid = (H, directions * (V + K) / 16 / NWC, N * (segments - 1)); forward the segments before the
 // last, in reverse those behind the first.  first_y: blockIdx.y counts from there on (SEG_BWD_KEPT: the reverse direction's V / 16 / NWC, which
 // leave out the transitions' columns; see sum_splits).
-template <typename T, int K, int V, int NWC, bool BOTH>
-__global__ __launch_bounds__((ScanCfg<T, K, V, NWC>::THREADS)) void scan_sum_kernel(ChunkArgs<T> p, int first_y) {
+template <typename T, int K, int V, int NWC, int KS, bool BOTH>
+__global__ __launch_bounds__((ScanCfg<T, K, V, NWC, KS>::THREADS)) void scan_sum_kernel(ChunkArgs<T> p, int first_y) {
     constexpr int NF = NSLOT * blk_fwd(K, sizeof(T), false).SIZE;
     constexpr int NB = NSLOT * slot_bwd(K, sizeof(T)).SIZE;
-    constexpr int SPLIT = ScanCfg<T, K, V, NWC>::SPLIT, COLS = (V + K) / 16 / NWC;
+    constexpr int SPLIT = ScanCfg<T, K, V, NWC, KS>::SPLIT, COLS = (V + K) / 16 / NWC;
     __shared__ __attribute__((aligned(16))) char smem[BOTH && NB > NF ? NB : NF];
+    __shared__ f32x4 handed[ScanCfg<T, K, V, NWC, KS>::HANDED];
     const int z = blockIdx.z / (p.seg.nseg - 1), seg = blockIdx.z % (p.seg.nseg - 1);
     const int n = scan_sequence(p.st, z), y = blockIdx.y + first_y, split = y % COLS;
     if (!BOTH || y < COLS) {
         if (seg == 0 && split >= SPLIT) return;           // starts from h0: nobody asks for its transition
-        scan_fwd_body<T, K, V, NWC, OUT_SUM>(p, smem, n, seg, split);
+        scan_fwd_body<T, K, V, NWC, OUT_SUM, KS>(p, smem, handed, n, seg, split);
     } else {
         if (seg + 1 == p.seg.nseg - 1 && split >= SPLIT) return;
-        scan_bwd_body<T, K, V, NWC, OUT_SUM>(p, smem, n, seg + 1, split);
+        scan_bwd_body<T, K, V, NWC, OUT_SUM, KS>(p, smem, handed, n, seg + 1, split);
     }
 }
 // The records chained into what enters the segments, X <- M_s X + X_loc(s) from the segment that starts the sequence (or, in
@@ -732,15 +824,15 @@ __global__ __launch_bounds__(64 * (K / 16)) void scan_chain_kernel(ChunkArgs<T> 
 }
 
 // ---- launchers -------------------------------------------------------------------------------------------------
-template <typename T, int K, int V, int NWC>
+template <typename T, int K, int V, int NWC, int KS>
 static hipError_t launch_scan_nwc(const ChunkArgs<T>& a, ScanKind kind, hipStream_t stream) {
-    typedef ScanCfg<T, K, V, NWC> C;
+    typedef ScanCfg<T, K, V, NWC, KS> C;
     dim3 grid(a.H, C::SPLIT * (kind == SCAN_PAIR ? 2 : 1), a.st.N * a.seg.nseg), block(C::THREADS);
     switch (kind) {
-        case SCAN_FWD_O: hipLaunchKernelGGL((scan_fwd_kernel<T, K, V, NWC, true>), grid, block, 0, stream, a); break;
-        case SCAN_FWD: hipLaunchKernelGGL((scan_fwd_kernel<T, K, V, NWC, false>), grid, block, 0, stream, a); break;
-        case SCAN_BWD: hipLaunchKernelGGL((scan_bwd_kernel<T, K, V, NWC>), grid, block, 0, stream, a); break;
-        case SCAN_PAIR: hipLaunchKernelGGL((scan_pair_kernel<T, K, V, NWC>), grid, block, 0, stream, a); break;
+        case SCAN_FWD_O: hipLaunchKernelGGL((scan_fwd_kernel<T, K, V, NWC, KS, true>), grid, block, 0, stream, a); break;
+        case SCAN_FWD: hipLaunchKernelGGL((scan_fwd_kernel<T, K, V, NWC, KS, false>), grid, block, 0, stream, a); break;
+        case SCAN_BWD: hipLaunchKernelGGL((scan_bwd_kernel<T, K, V, NWC, KS>), grid, block, 0, stream, a); break;
+        case SCAN_PAIR: hipLaunchKernelGGL((scan_pair_kernel<T, K, V, NWC, KS>), grid, block, 0, stream, a); break;
     }
     return hipGetLastError();
 }
@@ -752,12 +844,19 @@ hipError_t launch_scan_shape(const ChunkArgs<T>& a, ScanKind kind, hipStream_t s
     // come in rounds that are the sooner done.  us, fp32 forward passes, eight -> four, K = V = 128 / K = 64: 64 lanes of 19 chunks 165 -> 118 / 102 -> 75, 80 of
     // 22 201 -> 146 / 114 -> 82, 128 of 19 201 -> 160 / 120 -> 92, but 160 of 19 219 -> 250 / 131 -> 141, 256 of 13 195 -> 219 / 123 -> 132, and again 320 of 13
     // 301 -> 296 / 186 -> 175; 10 packed sequences of 8 heads, 3546 tokens 418 -> 278 / 231 -> 148.  The same bits.
-    if constexpr (V == 128) {
-        const long long lanes = (long long)a.H * a.st.N * a.seg.nseg * (kind == SCAN_PAIR ? 2 : 1);
-        auto rounds = [](long long workgroups) { return (workgroups + SCAN_TARGET_WORKGROUPS - 1) / SCAN_TARGET_WORKGROUPS; };
-        if (6 * rounds(2 * lanes) < 10 * rounds(lanes)) return launch_scan_nwc<T, K, V, 4>(a, kind, stream);
+    const long long lanes = (long long)a.H * a.st.N * a.seg.nseg * (kind == SCAN_PAIR ? 2 : 1);
+    // K = 64, few sequences: two waves a column block, two blocks a workgroup, where these fit the device.  us, one wave a block -> two, fp32, V = 64 / V = 128:
+    // forward passes of 64 lanes of 19 chunks 68.7 -> 61.3 / 73.5 -> 66.3, 128 of 19 83 -> 76 / (not chosen), 2 of 19 44 -> 40 / 46 -> 42, 10 packed sequences of 8
+    // heads, 3546 tokens 142 -> 120; training steps of 64 lanes of 13 134 -> 122 / 173 -> 169, 2 x 1003 tokens of 8 heads 173 -> 169; where it is not chosen 0.99 to
+    // 1.01.  Errors against float64, two sums over the channels instead of one, now to before: 0.92 (da) to 0.98 (dk), o 0.96 (3 shapes, 4 inputs each).
+    if constexpr (K == 64) {
+        if (lanes * (V / 32) <= SCAN_TARGET_WORKGROUPS) return launch_scan_nwc<T, K, V, 2, 2>(a, kind, stream);
     }
-    return launch_scan_nwc<T, K, V, V / 16>(a, kind, stream);
+    if constexpr (V == 128) {
+        auto rounds = [](long long workgroups) { return (workgroups + SCAN_TARGET_WORKGROUPS - 1) / SCAN_TARGET_WORKGROUPS; };
+        if (6 * rounds(2 * lanes) < 10 * rounds(lanes)) return launch_scan_nwc<T, K, V, 4, 1>(a, kind, stream);
+    }
+    return launch_scan_nwc<T, K, V, V / 16, 1>(a, kind, stream);
 }
 
 template <typename T, int K, int V>
@@ -773,15 +872,26 @@ template <int K, int V, int NWC> static int sum_splits(SegStart what, bool turne
     return what == SEG_BWD_KEPT ? state : what != SEG_BWD ? all : turned ? all + state : 2 * all;
 }
 template <int K, int V, int NWC> static int sum_first(SegStart what) { return what == SEG_BWD_KEPT ? (V + K) / 16 / NWC : 0; }
+template <typename T, int K, int V, int NWC, int KS>
+static hipError_t launch_scan_sum(const ChunkArgs<T>& a, SegStart what, dim3 grid, hipStream_t stream) {
+    const dim3 block(ScanCfg<T, K, V, NWC, KS>::THREADS);
+    const int first = sum_first<K, V, NWC>(what);
+    if (what == SEG_BWD || what == SEG_BWD_KEPT) hipLaunchKernelGGL((scan_sum_kernel<T, K, V, NWC, KS, true>), grid, block, 0, stream, a, first);
+    else hipLaunchKernelGGL((scan_sum_kernel<T, K, V, NWC, KS, false>), grid, block, 0, stream, a, first);
+    return hipGetLastError();
+}
 template <typename T, int K, int V>
 hipError_t launch_scan_segments_shape(const ChunkArgs<T>& a, SegStart what, hipStream_t stream) {
-    constexpr int NWC = 4;                                // column blocks per workgroup: each fetches the chunks' operands once for them
-    typedef ScanCfg<T, K, V, NWC> C;
-    const dim3 grid(a.H, sum_splits<K, V, NWC>(what, a.seg.turned), a.st.N * (a.seg.nseg - 1)), block(C::THREADS);
-    const int first = sum_first<K, V, NWC>(what);
-    if (what == SEG_BWD || what == SEG_BWD_KEPT) hipLaunchKernelGGL((scan_sum_kernel<T, K, V, NWC, true>), grid, block, 0, stream, a, first);
-    else hipLaunchKernelGGL((scan_sum_kernel<T, K, V, NWC, false>), grid, block, 0, stream, a, first);
-    const hipError_t e = hipGetLastError();
+    // four column blocks per workgroup, each fetches the chunks' operands once for them; or two, where these fit the device (launch_scan_shape)
+    auto grid = [&](int splits) { return dim3(a.H, splits, a.st.N * (a.seg.nseg - 1)); };
+    hipError_t e = hipErrorInvalidValue;
+    bool done = false;
+    if constexpr (K == 64) {
+        const dim3 g = grid(sum_splits<K, V, 2>(what, a.seg.turned));
+        done = (long long)g.x * g.y * g.z <= SCAN_TARGET_WORKGROUPS;
+        if (done) e = launch_scan_sum<T, K, V, 2, 2>(a, what, g, stream);
+    }
+    if (!done) e = launch_scan_sum<T, K, V, 4, 1>(a, what, grid(sum_splits<K, V, 4>(what, a.seg.turned)), stream);
     return e == hipSuccess ? launch_scan_chain<T, K, V>(a, what, stream) : e;
 }
 

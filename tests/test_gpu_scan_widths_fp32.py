@@ -1,5 +1,6 @@
-"""fp32, V = 128: the scans of many sequences have all column blocks of a head in a workgroup, those of few have half of them.  Column blocks do not meet in
-a scan, so outputs and gradients have the bits of a call for each sequence by itself."""
+"""fp32: the scans of many sequences have all column blocks of a head in a workgroup, those of few have half of them, or two of them with two waves each that
+share the channels.  Column blocks do not meet in a scan, and the sums over channels are those of two halves whoever forms them, so outputs and gradients have
+the bits of a call for each sequence by itself."""
 import pytest
 import torch
 
@@ -10,12 +11,14 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-@pytest.mark.parametrize("K", [64, 128])
-@pytest.mark.parametrize("B", [8, 9, 16, 20])              # of 16 heads: half, all, all, half (forward pass); half, half, all, half (backward pass)
-def test_the_bits_of_each_sequence_by_itself(K, B, monkeypatch):
+# of 16 heads: at K = V = 64 the first three are two waves' a block in the forward pass, the first two in the backward pass; at K = V = 128 all column blocks are
+# a workgroup's at 9 and 16 in the forward pass, at 16 in the backward pass
+@pytest.mark.parametrize("K,V", [(64, 64), (64, 128), (128, 64), (128, 128)])
+@pytest.mark.parametrize("B", [2, 4, 8, 9, 16, 20])
+def test_the_bits_of_each_sequence_by_itself(K, V, B, monkeypatch):
     monkeypatch.setenv("HDLA_HIP_ROUTE", "classic")
     monkeypatch.setenv("HDLA_HIP_SEGMENTS", "1")
-    inp = make_inputs(2300 + B, B, 37, 16, K, 128, gk_div=4.0)
+    inp = make_inputs(2300 + B, B, 61, 16, K, V, gk_div=4.0)
     x = [t.to(DEV) for t in (inp.q, inp.k, inp.v, inp.a, inp.b, inp.gk, inp.h0)]
     do, dht = inp.do.to(DEV), inp.dht.to(DEV)
 
