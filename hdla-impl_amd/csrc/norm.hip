@@ -395,6 +395,8 @@ static long long gcd_ll(long long a, long long b) { while (b) { const long long 
 // would come in a round of its own.  us, 1024 workgroups -> as many as are resident, evenly filled: 20000 x 1024 43.0 -> 38.8, 65536 x 4096 548 -> 516.
 // (The forward kernel, and 4-byte elements, were the same or slower so.)
 constexpr long long NORM_RESIDENT = 3 * 256;
+// Workgroups after which a launch meets the same groups again, at the most
+constexpr long long NORM_PERIOD = 65536;
 static int norm_config(const hdla_norm_dims* d, bool bwd, NormCfg& c) {
     if (!d) return HDLA_ERR_NULL;
     if (d->dtype != HDLA_BF16 && d->dtype != HDLA_FP32) return HDLA_ERR_DTYPE;
@@ -410,7 +412,8 @@ static int norm_config(const hdla_norm_dims* d, bool bwd, NormCfg& c) {
     // groups of more than two pieces a lane, whose wavefronts would have the registers of few, and of two when there are too few of them
     // to fill the chip one wavefront each (a decode step: a few hundred rows).  us, both passes, one wavefront a group -> four: bf16 65536 x 4096 1000 -> 838,
     // 10000 x 4096 202 -> 135, 20000 x 2048 130 -> 122; fp32 5000 x 2048 81 -> 68, 20000 x 1024 124 -> 115, 30000 x 2048 362 both.
-    c.wg_row = pieces > 64 * 2 || (pieces >= 128 && c.nslot <= 2048);
+    // (Up to NORM_PERIOD groups: the grid is a multiple of their number then, and of a quarter of it where each wavefront has one.)
+    c.wg_row = pieces > 64 * 8 || (pieces > 64 * 2 && d->G <= NORM_PERIOD) || (pieces >= 128 && c.nslot <= 2048);
     if (c.wg_row) {
         // one group per workgroup pass, 256 lanes across it
         c.nv = 1;
@@ -439,7 +442,7 @@ static int norm_config(const hdla_norm_dims* d, bool bwd, NormCfg& c) {
         nwg = (c.nsg + owners * passes - 1) / (owners * passes);
     }
     const long long m = d->G / gcd_ll(d->G, owners * c.rpw);
-    if (m > 65536) return HDLA_ERR_SHAPE;
+    if (m > NORM_PERIOD) return HDLA_ERR_SHAPE;
     c.nwg = (nwg + m - 1) / m * m;
     return HDLA_OK;
 }
