@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-#define HDLA_VERSION 207
+#define HDLA_VERSION 208
 
 enum { HDLA_BF16 = 0, HDLA_FP32 = 1 };
 
