@@ -803,7 +803,7 @@ def run_chunk_workload(wl, cfg, steps, warmup, dev, keep_variant=True):
             variants["inputs_only"] = time_steps(step, steps, warmup)
             del os.environ["HDLA_HIP_INPUTS_ONLY"]
         if _l.workspace_layout(probe, 0)["ERR"] >= 0:
-            os.environ["HDLA_HIP_ROUTE"] = "classic"
+            os.environ["HDLA_HIP_ROUTE"] = "plain"
             variants["classic_route"] = time_steps(step, steps, warmup)
             del os.environ["HDLA_HIP_ROUTE"]
     # the same step with keep_forward=True (an option, off by default: the forward pass's per-chunk intermediates stay
@@ -852,7 +852,7 @@ def run_chunk_workload(wl, cfg, steps, warmup, dev, keep_variant=True):
                     "pass re-derives the states at the time-segment boundaries with one more pass (kernel time under summary_ms)",
             "ms_per_step": variants["inputs_only"] * 1e3, "value": tokens / variants["inputs_only"], "summary_ms": summary_ms}
     if "classic_route" in variants:
-        other["classic_route"] = {"what": "the same step with HDLA_HIP_ROUTE=classic: prep, scan and chunk_grad kernels with the "
+        other["classic_route"] = {"what": "the same step with HDLA_HIP_ROUTE=plain: prep, scan and chunk_grad kernels with the "
                                           "scans' operands passed through the workspace",
                                   "ms_per_step": variants["classic_route"] * 1e3, "value": tokens / variants["classic_route"]}
     return dict(

@@ -32,7 +32,8 @@ int check_dims(const hdla_dims* d, int max_dim = 128) {
     if (d->in_dtype == HDLA_FP32 && d->gk_dtype != HDLA_FP32) return HDLA_ERR_DTYPE;
     if (d->cu_seqlens) { if (d->B != 1) return HDLA_ERR_SEQ; }
     else if (d->N != d->B) return HDLA_ERR_SEQ;
-    if (d->route < HDLA_ROUTE_AUTO || d->route > HDLA_ROUTE_FUSED || d->segments < 0) return HDLA_ERR_ROUTE;
+    if (d->route != HDLA_ROUTE_AUTO && d->route != HDLA_ROUTE_CLASSIC && d->route != HDLA_ROUTE_FUSED && d->route != HDLA_ROUTE_PLAIN) return HDLA_ERR_ROUTE;
+    if (d->segments < 0) return HDLA_ERR_ROUTE;
     return HDLA_OK;
 }
 
@@ -65,7 +66,7 @@ int short_least(int pass) { return pass == HDLA_PASS_FWD ? SHORT_MIN_CHUNKS_FWD 
 // whether the plain entry points take the fused route for these dimensions; HDLA_ROUTE_FUSED on another shape is an error.
 // with_boundary: a boundary (or record) buffer is given: then it is the fused route's.
 int pick_route(const hdla_dims* d, int pass, bool with_boundary, bool& fused) {
-    fused = d->route != HDLA_ROUTE_CLASSIC && fused_shape(d) && (with_boundary || !few_short_sequences(d, short_least(pass)));
+    fused = d->route != HDLA_ROUTE_CLASSIC && d->route != HDLA_ROUTE_PLAIN && fused_shape(d) && (with_boundary || !few_short_sequences(d, short_least(pass)));
     if (d->route == HDLA_ROUTE_FUSED && !fused) return HDLA_ERR_ROUTE;
     return HDLA_OK;
 }
@@ -276,7 +277,9 @@ int make_layout(const hdla_dims* d, int pass, WsLayout& L, int& nch) {
             L.TM = take(chw * 1536 * es);                         // the scan forms u itself (scan_out.cuh)
         } else {
             // (2-byte elements: the scans form u and v^T themselves.  chunk_grad reads u beside fp32 decays; v^T is there, and u, for whoever names the classic
-            // route and looks at a backward pass's buffers.  A kept forward pass's layout does not depend on the route.)
+            // route and looks at a backward pass's buffers.  The library's own plans name the plain one: us a training step that finds no room to keep its
+            // forward pass, classic -> plain, 4 x 1000 tokens of 16 heads, K = V = 128 413 -> 392, 4 x 2048, K = 64, V = 128 490 -> 465.  A kept forward
+            // pass's layout does not depend on the route.)
             const bool shown = pass == HDLA_PASS_BWD && d->route == HDLA_ROUTE_CLASSIC;
             if (d->gk_dtype == HDLA_FP32 || shown || pass == HDLA_PASS_FWD_KEEP) L.UT = take(chw * 2 * V * 16 * es);
             if (es == 4 || shown) L.VTT = take(chw * V * 16 * es);
@@ -599,7 +602,7 @@ const char* hdla_strerror(int code) {
         case HDLA_ERR_WORKSPACE: return "workspace is NULL, not 256-byte aligned, smaller than hdla_workspace_bytes(), or kept with another number of segments";
         case HDLA_ERR_ALIGN: return "tensor pointers must be 16-byte aligned";
         case HDLA_ERR_SEQ: return "cu_seqlens needs B == 1; without it N must equal B";
-        case HDLA_ERR_ROUTE: return "route must be HDLA_ROUTE_AUTO, _CLASSIC or _FUSED (the fused route: bf16 inputs, K = V = 64) and segments >= 0";
+        case HDLA_ERR_ROUTE: return "route must be HDLA_ROUTE_AUTO, _CLASSIC, _PLAIN or _FUSED (the fused route: bf16 inputs, K = V = 64) and segments >= 0";
         case HDLA_ERR_STATIC_LIMIT: return "the call needs more scratch memory than the built-in HDLA_STATIC_WORKSPACE_BYTES; use hdla_chunk_fwd with a caller-owned workspace";
         default: return code > 0 ? hipGetErrorString((hipError_t)code) : "unknown error code";
     }

@@ -111,6 +111,7 @@ bool read_plan(Plan& p) {
     const char* r = env("HDLA_HIP_ROUTE");
     if (!r || !*r || !strcmp(r, "auto")) p.route = HDLA_ROUTE_AUTO;
     else if (!strcmp(r, "classic")) p.route = HDLA_ROUTE_CLASSIC;
+    else if (!strcmp(r, "plain")) p.route = HDLA_ROUTE_PLAIN;
     else if (!strcmp(r, "fused")) p.route = HDLA_ROUTE_FUSED;
     else return false;
     p.record = env_is("HDLA_HIP_INPUTS_ONLY", {"", "0", "false", "False"}, true);
@@ -214,7 +215,7 @@ void chunk_forward(const ChunkIn& x, const hdla_dims& d, bool want_ht, Plan* pla
         const size_t n = plan->record && !nb ? api.keep_plan(&d, &k.segments, &for_bwd) : 0;
         if (n) {                                          // one plan for the backward pass, kept or not
             plan->segments = for_bwd;
-            if (for_bwd == 1) plan->route = HDLA_ROUTE_CLASSIC;   // (one segment, also where a number asked for would be the fused route's)
+            if (for_bwd == 1) plan->route = HDLA_ROUTE_PLAIN;   // (one segment, also where a number asked for would be the fused route's)
             left = kept_room(x.q, (int64_t)n);
         }
         plan->keep = left.defined();

@@ -12,9 +12,9 @@ from typing import Optional, Tuple
 import torch
 
 HDLA_BF16, HDLA_FP32 = 0, 1
-HDLA_VERSION = 208          # the header this binding was written against (struct layouts, entry points)
-ROUTE_AUTO, ROUTE_CLASSIC, ROUTE_FUSED = 0, 1, 2
-_ROUTES = {"": ROUTE_AUTO, "auto": ROUTE_AUTO, "classic": ROUTE_CLASSIC, "fused": ROUTE_FUSED}
+HDLA_VERSION = 209          # the header this binding was written against (struct layouts, entry points)
+ROUTE_AUTO, ROUTE_CLASSIC, ROUTE_FUSED, ROUTE_PLAIN = 0, 1, 2, 4
+_ROUTES = {"": ROUTE_AUTO, "auto": ROUTE_AUTO, "classic": ROUTE_CLASSIC, "plain": ROUTE_PLAIN, "fused": ROUTE_FUSED}
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB_NAME = "libhdla_hip.so"
 _lib = None
@@ -256,10 +256,11 @@ def dtype_code(dt: torch.dtype) -> int:
 
 def default_route() -> int:
     """Launch plan of the chunked operators when the caller does not say: environment variable HDLA_HIP_ROUTE =
-    auto (the library chooses: the fused kernels where they are built), classic or fused."""
+    auto (the library chooses: the fused kernels where they are built), classic, plain (the same without the buffers that are
+    there to be looked at) or fused."""
     name = os.environ.get("HDLA_HIP_ROUTE", "auto").lower()
     if name not in _ROUTES:
-        raise HdlaError(f"HDLA_HIP_ROUTE must be one of auto, classic, fused (got {name!r})")
+        raise HdlaError(f"HDLA_HIP_ROUTE must be one of auto, classic, plain, fused (got {name!r})")
     return _ROUTES[name]
 
 

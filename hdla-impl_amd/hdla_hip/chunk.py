@@ -110,7 +110,7 @@ def keep_plan(q, v, gk, scale, cu_seqlens):
     if not n or _lib.load().hdla_record_bytes(ctypes.byref(dims)):
         return None
     room = _lib.native().kept_room(q, n)
-    return (dims.route, fwd), (_lib.ROUTE_CLASSIC if bwd == 1 else dims.route, bwd), False if room is None else room
+    return (dims.route, fwd), (_lib.ROUTE_PLAIN if bwd == 1 else dims.route, bwd), False if room is None else room
 
 
 def one_segment(plan):

@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-#define HDLA_VERSION 208
+#define HDLA_VERSION 209
 
 enum { HDLA_BF16 = 0, HDLA_FP32 = 1 };
 
@@ -71,8 +71,10 @@ enum {
  * where it is built, except for few short sequences (at most 64 pairs of a sequence and a head, at most 31 chunks a
  * sequence on average, at least 16 in a forward and 6 in a backward pass, no segments asked for), where the classic
  * kernels are through sooner, unless a call is given a boundary or record buffer (hdla_record_bytes is 0 where the backward pass takes the
- * classic kernels).  Both routes compute the same function; they differ in rounding only where segments > 1. */
-enum { HDLA_ROUTE_AUTO = 0, HDLA_ROUTE_CLASSIC = 1, HDLA_ROUTE_FUSED = 2 };
+ * classic kernels).  Both routes compute the same function; they differ in rounding only where segments > 1.
+ * HDLA_ROUTE_CLASSIC also leaves buffers in a backward pass's workspace that no kernel reads, for callers who look at them (hdla_ws_layout);
+ * HDLA_ROUTE_PLAIN is the same plan, to the bit, without them. */
+enum { HDLA_ROUTE_AUTO = 0, HDLA_ROUTE_CLASSIC = 1, HDLA_ROUTE_FUSED = 2, HDLA_ROUTE_PLAIN = 4 };
 #define HDLA_FUSED_ABORTED 0x48444c00
 
 typedef struct hdla_dims {
@@ -176,7 +178,7 @@ size_t hdla_record_workspace_bytes(const hdla_dims* dims);
  * buffer for hdla_chunk_fwd_keep and hdla_chunk_bwd_kept that the library suggests to keep, and the `segments` to give the one and the other in
  * dims; 0 where it suggests none (the fused route has its record; a buffer of more than 256 MiB; no tokens).  The suggestion is for one call: a
  * program with many calls between a forward and its backward pass holds as many buffers, and bounds what they come to (the Python package: 1 GiB and
- * 256 calls a device).  A backward pass without the buffer, hdla_chunk_bwd_b with bwd_segments in dims (and, where that is 1, HDLA_ROUTE_CLASSIC), has the same
+ * 256 calls a device).  A backward pass without the buffer, hdla_chunk_bwd_b with bwd_segments in dims (and, where that is 1, HDLA_ROUTE_PLAIN), has the same
  * bits. */
 size_t hdla_keep_plan(const hdla_dims* dims, int32_t* fwd_segments, int32_t* bwd_segments);
 int hdla_chunk_fwd_b(const hdla_dims* dims, const void* q, const void* k, const void* v, const void* a, const void* b,
