@@ -150,9 +150,9 @@ int scan_segments(const hdla_dims* d, bool bwd) {
 int kept_segments(const hdla_dims* d) { return d->segments > 0 ? scan_segments(d, false) : 1; }
 
 // What a training call keeps of its forward pass where nothing else is said: all that the prep kernel forms, which the backward pass would form
-// again (1.6 times the inputs' bytes at K = V = 64), and the records of the segments; of one call this much, 0.1 % of the device's memory (what all of them hold,
+// again (in 16 bits 1.06 to 1.25 times the inputs' bytes, in 32 1.3 to 1.7), and the records of the segments; of one call this much, 0.1 % of the device's memory (what all of them hold,
 // the caller bounds: native.cpp, kept_room).  With its scratch a call's backward pass
-// then has 5 % more than one that recomputes has, median of 839 shapes, 41 % at the most, where the forward pass alone is in segments.  us on the device, a training step
+// then has 5 % more than one that recomputes has, median of 949 shapes, 45 % at the most, where the forward pass alone is in segments.  us on the device, a training step
 // that keeps the inputs -> this: 1 x 256 tokens, 2 heads, K = V = 64 43 -> 37; 2 x 1537 tokens, 8 heads, K = V = 128 214 -> 185;
 // 4 x 1000 tokens, 16 heads 430 -> 393; 4 x 500, 8 heads 127 -> 107; fp32, 2 x 1003 tokens, 8 heads, K = V = 64 227 -> 190.
 constexpr size_t KEEP_MOST = (size_t)256 << 20;
@@ -278,10 +278,9 @@ int make_layout(const hdla_dims* d, int pass, WsLayout& L, int& nch) {
         } else {
             // (2-byte elements: the scans form u and v^T themselves.  chunk_grad reads u beside fp32 decays; v^T is there, and u, for whoever names the classic
             // route and looks at a backward pass's buffers.  The library's own plans name the plain one: us a training step that finds no room to keep its
-            // forward pass, classic -> plain, 4 x 1000 tokens of 16 heads, K = V = 128 413 -> 392, 4 x 2048, K = 64, V = 128 490 -> 465.  A kept forward
-            // pass's layout does not depend on the route.)
+            // forward pass, classic -> plain, 4 x 1000 tokens of 16 heads, K = V = 128 413 -> 392, 4 x 2048, K = 64, V = 128 490 -> 465.)
             const bool shown = pass == HDLA_PASS_BWD && d->route == HDLA_ROUTE_CLASSIC;
-            if (d->gk_dtype == HDLA_FP32 || shown || pass == HDLA_PASS_FWD_KEEP) L.UT = take(chw * 2 * V * 16 * es);
+            if (d->gk_dtype == HDLA_FP32 || shown) L.UT = take(chw * 2 * V * 16 * es);
             if (es == 4 || shown) L.VTT = take(chw * V * 16 * es);
             if (es == 2) { L.AAK = take(chw * 512 * es); L.SUM = take(chw * 64); }
         }
@@ -311,6 +310,8 @@ int make_layout(const hdla_dims* d, int pass, WsLayout& L, int& nch) {
         if (pass == HDLA_PASS_BWD) { L.SEG_RLOC = take(state); L.SEG_RTR = take(matrix); L.SEG_RIN = take(state); }
         if (pass == HDLA_PASS_BWD_KEPT) { L.SEG_RLOC = take(state); L.SEG_RIN = take(state); }
     }
+    // (behind the rest: where a backward pass finds what it reads does not depend on the routes that the two passes are called with)
+    if (pass == HDLA_PASS_FWD_KEEP && d->route == HDLA_ROUTE_CLASSIC && !L.UT) L.UT = take(chw * 2 * V * 16 * es);
     L.total = off > 0 ? off : 256;
     return HDLA_OK;
 }
@@ -322,7 +323,7 @@ template <typename T>
 void bind_ws(ChunkArgs<T>& a, const hdla_dims* d, const WsLayout& LP, void* prep_ws, const WsLayout& LS, void* scan_ws, int nch) {
     char* base = static_cast<char*>(prep_ws);
     auto at = [&](size_t o) { return reinterpret_cast<T*>(base + o); };
-    a.ws.W = at(LP.W); a.ws.UT = at(LP.UT); a.ws.KGT = at(LP.KGT); a.ws.BGT = at(LP.BGT);
+    a.ws.W = at(LP.W); a.ws.UT = LP.UT ? at(LP.UT) : nullptr; a.ws.KGT = at(LP.KGT); a.ws.BGT = at(LP.BGT);
     a.ws.VTT = LP.VTT ? at(LP.VTT) : nullptr; a.ws.AAK = at(LP.AAK); a.ws.aak_stride = 512;
     a.ws.SUM = reinterpret_cast<float*>(base + LP.SUM);
     a.ws.QG = at(LP.QG); a.ws.AQK = at(LP.AQK); a.ws.AQB = at(LP.AQB);
@@ -369,7 +370,9 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
     int nch = 0;
     const bool fwd = pass == HDLA_PASS_FWD || pass == HDLA_PASS_FWD_KEEP;
     const bool on_kept = pass == HDLA_PASS_FWD_KEEP || pass == HDLA_PASS_BWD_KEPT;
-    int rc = make_layout(d, on_kept ? HDLA_PASS_FWD_KEEP : pass, LP, nch);
+    hdla_dims kept_dims = *d;
+    if (pass == HDLA_PASS_BWD_KEPT && d->route == HDLA_ROUTE_CLASSIC) kept_dims.route = HDLA_ROUTE_PLAIN;   // (what this pass reads)
+    int rc = make_layout(&kept_dims, on_kept ? HDLA_PASS_FWD_KEEP : pass, LP, nch);
     if (rc) return rc;
     void* prep_ws = on_kept ? kept : workspace;
     if (bad_ws(prep_ws, on_kept ? kept_bytes : workspace_bytes, LP.total)) return HDLA_ERR_WORKSPACE;

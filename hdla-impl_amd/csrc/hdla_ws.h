@@ -124,7 +124,7 @@ template <typename T>
 struct Ws {
     T *W, *UT, *KGT, *BGT, *VTT, *QG, *AQK, *AQB, *AQBT, *QGT, *HC, *DHC, *DVN;
     float* SUM;
-    T* AAK;                   // VTT: null where nobody asks for u and v^T that the scans of 2-byte elements form themselves
+    T* AAK;                   // UT, VTT: null where nobody asks for u and v^T that the scans of 2-byte elements form themselves
     float *EGL;
     T* TM;
     int32_t* STRONG;

@@ -259,7 +259,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
     // the forward pass's scan of 2-byte elements forms u itself and takes the ranks of b^T side by side (scan_out.cuh): v is not read
     constexpr bool SCAN_U = MODE == PREP_FWD && sizeof(T) == 2;
     // The other scans of 2-byte elements form u too, from (I - A_ab)^-1, A_ak and v; u is written where chunk_grad reads it (its REBUILD_U), or where the
-    // caller has named the classic route, whose buffers can be looked at (VTT is given).  This mode at K = V = 128, 16384 tokens of 16 heads, us: 221 -> 178,
+    // caller has named the classic route, whose buffers can be looked at (UT is given).  This mode at K = V = 128, 16384 tokens of 16 heads, us: 221 -> 178,
     // for 12 KB not written and v not read of 85 a chunk and head.
     constexpr bool WRITE_U = sizeof(T) == 4 || GKF32;
     constexpr int NWP = K / 64;                       // waves per (chunk, head)
@@ -670,7 +670,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
     if (sizeof(T) == 2 && w == NWP - 1) st_pair2(p.ws.AAK + chw * PAIR, aakf[0], aakf[1]);
     const bool vtt = sizeof(T) == 4 || p.ws.VTT;
     if (!WRITE_U) {
-        if (!vtt) return;
+        if (!p.ws.UT) return;
 #pragma unroll
         for (int vp = 0; vp < VTW / 2; ++vp) lv[vp].load(vrow + 32 * vp, H * V, cp.len, l);
     }

@@ -270,7 +270,7 @@ def chunk_hrdplr_delta_rule(
     [N,H,K,V] fp32 or None)``.
 
     ``keep_forward`` (keyword-only, not in the reference): True keeps the forward pass's per-chunk intermediates alive
-    until the backward pass (about 1.6 times the bytes of q, k, v, a, b, gk together), which then skips recomputing
+    until the backward pass (1.1 to 1.7 times the bytes of q, k, v, a, b, gk together), which then skips recomputing
     them; False is closest to the reference's behaviour, where only the inputs are kept (hrdplr.py:137) and the backward pass
     recomputes (:161-198): here the fused route's record is kept beside them.  None (and HDLA_HIP_KEEP_FORWARD unset): kept
     where that is at most 256 MiB and the route has no record, and only as long as all calls whose backward pass is still to come hold

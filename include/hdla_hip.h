@@ -100,7 +100,7 @@ typedef struct hdla_dims {
  * (and W, UT where chunk_grad reads them instead of rebuilding them: fp32 decays beside bf16 inputs) are written, in the backward pass.  In a forward pass on bf16 inputs (HDLA_PASS_FWD, classic route) the scan forms u
  * itself: there is no UT and no VTT, TM holds three tile pairs a slot, the blocks of (I - A_ab)^-1 (not transposed: rows i, inner j) and
  * the two ranks of A_ak, and the tile pairs of BGT are the two ranks of a channel tile.  The other passes' scans of bf16 inputs form u themselves
- * as well: there is VTT, and UT is filled, in a backward pass under HDLA_ROUTE_CLASSIC only (UT also beside fp32 decays). */
+ * as well: there is VTT in a backward pass, and UT there and in HDLA_PASS_FWD_KEEP, under HDLA_ROUTE_CLASSIC only (UT also beside fp32 decays). */
 typedef struct hdla_ws_layout {
     int64_t nch;               /* chunk slots per head */
     int64_t W, UT, KGT, BGT, VTT, EGL, QG, AQK, AQB, AQBT, QGT, TM, HC, DHC, DVN;
@@ -211,7 +211,7 @@ int hdla_param_chunk_bwd(const hdla_dims* dims, const void* q, const void* k, co
  * hdla_chunk_bwd_kept is hdla_chunk_bwd (hdla_param_chunk_bwd with beta: dbeta is written, da and db are not) that reads
  * them there instead of recomputing them from the inputs, which saves the backward pass its first kernel.  The reference
  * keeps only the inputs between the passes and recomputes (ctx.save_for_backward at HRDPLR/hrdplr.py:137, recompute at
- * :161-198); these two trade that for about 1.6x the inputs' bytes of extra memory held between the passes.  `kept` is
+ * :161-198); these two trade that for 1.1 to 1.7x the inputs' bytes of extra memory held between the passes.  `kept` is
  * only read by the backward call (it can be used again); `workspace` is scratch of
  * hdla_workspace_bytes(dims, HDLA_PASS_BWD_KEPT) bytes.  Same dims, inputs and stream ordering as the forward call.
  * Time segments: one where dims->segments is 0, otherwise (HDLA_ROUTE_AUTO) as many as it says; the states that enter them and their transitions
