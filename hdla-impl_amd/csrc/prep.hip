@@ -13,8 +13,6 @@
 #include "hdla_common.cuh"
 #include "hdla_launch.h"
 
-#include <algorithm>
-
 namespace hdla {
 
 // ---- chunk table for packed variable-length batches ----------------------------------------------------------
@@ -27,7 +25,7 @@ constexpr int TABLE_THREADS = 256;
 // outputs for every call took 88 of 2050 us of a training step on 16384 tokens, H = 16, K = V = 128).  A table that does not
 // decrease leaves out only what lies before its first and behind its last entry (a batch padded at its end); one that does may
 // leave out anything, and the outputs are cleared whole.
-// Measured, 16384 tokens of 16 heads, K = V = 128, the last 200 in no sequence, forward and backward pass: 1.79 ms (a full batch 1.94);
+// Measured, 16384 tokens of 16 heads, K = V = 128, the last 200 in no sequence, forward and backward pass: 1.62 ms (a full batch 1.64);
 // with all outputs cleared by workgroup 0, two bytes a lane, 21.6.
 struct ClearRange { long long lo, hi; };                  // tokens [0, lo) and [hi, T)
 __device__ __forceinline__ ClearRange uncovered(const int64_t* cu, int N, int T, int t, int threads) {
@@ -230,14 +228,16 @@ __global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const 
 // for, and prep_kernel's other workgroups find their chunks by themselves (locate_few).  us, forward passes, table first -> this: 90 tokens in 4 sequences,
 // 4 heads 15.8 -> 13.0; 520 in 8, 8 heads, K = V = 128 27.5 -> 23.2; 3000 in 12, 16 heads, K = 64, V = 128 54.3 -> 47.4, in 30, K = V = 128 98.6 -> 91.8;
 // 5003 in 4 130.7 -> 127.0; fp32, 700 in 4 61.6 -> 57.1; training step of 16384 in 4 1649 -> 1634.  The fused route, whose first kernel walks
-// sequences, has the table first, in registers too: 2500 tokens in 5, 16 heads 52.0 -> 50.1.  FEW_CLEARERS: a workgroup a compute unit, beside prep's own.
+// sequences, has the table first, in registers too: 2500 tokens in 5, 16 heads 52.0 -> 50.1.  FEW_CLEARERS: as many threads at K = 128 as the other launch's workgroups,
+// four times as large, have.  A training step with 14384 of 16384 rows to clear, 16 heads, K = V = 128, by 256 / 512 / 1024 of them 394 / 386 / 384 us (by a launch of its own in
+// front 387), K = 64, V = 128 233 / 240 / 234 (247); batches without such rows the same.
 struct FewTable {
     int32_t *chunk_off, *chunk_seq;       // null: the table is there
     int V;
     PackedOut out;
 };
 static_assert(FEW_SEQS == 64 && SHARE_MAX_N <= FEW_SEQS, "a lane each (prep_makes_table)");
-constexpr int FEW_CLEARERS = 256;
+constexpr int FEW_CLEARERS = 1024;
 
 constexpr int LDP = 36;   // padded row length of the 32x32 LDS matrices (keeps 16-byte row alignment)
 
@@ -691,17 +691,17 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
     }
 }
 
-// workgroups that look for rows to clear: one for every 16 KiB they might have to write, as many as fill the device, and fewer
+// workgroups that look for rows to clear: one for every 16 KiB they might have to write, as many as fill the device (of 256 threads 512), and fewer
 // where each has a long table to read first
-static int clearing_workgroups(int N, int T, const PackedOut& out) {
+static int clearing_workgroups(int N, int T, const PackedOut& out, int fill = 512) {
     long long bytes = 0;
     for (int b = 0; b < out.n; ++b) bytes += out.row[b] * T;
-    const long long most = max(32, min(512, (1 << 20) / N));
+    const long long most = max(32, min(fill, (1 << 20) / N));
     return (int)min((bytes + 16383) / 16384, most);
 }
 template <typename T, int K, int V, bool HD>
 static hipError_t launch_prep_kv(const ChunkArgs<T>& a, int mode, const FewTable& few, hipStream_t stream) {
-    const int makers = few.chunk_off ? 2 + std::min(FEW_CLEARERS, clearing_workgroups(a.st.N, a.st.T, few.out)) : 0;
+    const int makers = few.chunk_off ? 2 + clearing_workgroups(a.st.N, a.st.T, few.out, FEW_CLEARERS) : 0;
     dim3 grid(a.st.nch * a.H + makers), block(K);
     constexpr bool kAlwaysF32 = sizeof(T) == 4;
     const bool gkf32 = kAlwaysF32 || a.gk_f32;
