@@ -65,7 +65,7 @@ __device__ __forceinline__ void scan_rev_body(const ChunkArgs<bf16>& p, char* sm
     if (wv >= C::NC) {
         // ---- waves that move data; barriers as in scan_out.cuh, without one for a last output
         if (nchunks <= 0) return;
-        const int hw = wv - C::NC;
+        const int hw = forming_first<C>(wv - C::NC);
         if (hw < C::NL) {
             const int sf = p.ws.sa_stride;
             constexpr int SB = blk_bwd(K, 2).SIZE;
@@ -101,20 +101,21 @@ __device__ __forceinline__ void scan_rev_body(const ChunkArgs<bf16>& p, char* sm
             constexpr int UD = 3;
             struct Own { i32x4 aq; Frag<T> d[NWC]; };
             const Frag<T> ident = ident_frag<T>();
+            // rows of do, as those of v in scan_out.cuh
+            const int len_last = (int)min((int64_t)CH, eos - (bos + (int64_t)last * CH));
+            const uint32_t row = (uint32_t)(H * V) * sizeof(T), whole = c * row + 8 * g, ragged = min(c, len_last - 1) * row + 8 * g;
+            const T* const do0 = p.dout + (bos * H + h) * V + 16 * (trans ? 0 : vt0);
             auto request = [&](int t) __attribute__((always_inline)) {
-                const int at = max(last - t, 0);
-                const int64_t tok0 = bos + (int64_t)at * CH;
-                const int len = (int)min((int64_t)CH, eos - tok0);
+                const int i = max(last - t, 0);
                 Own o;
-                o.aq = *reinterpret_cast<const i32x4*>(reinterpret_cast<const char*>(p.ws.QGT) + (chw0 + at) * blk_bwd(K, 2).SIZE +
+                o.aq = *reinterpret_cast<const i32x4*>(reinterpret_cast<const char*>(p.ws.QGT) + (chw0 + i) * blk_bwd(K, 2).SIZE +
                                                        blk_bwd(K, 2).AQBT + 16 * l);
 #pragma unroll
-                for (int j = 0; j < NWC; ++j)
-                    o.d[j] = ld_frag(p.dout + ((tok0 + min(c, len - 1)) * H + h) * V + 16 * (trans ? 0 : vt0 + j) + 4 * g);
+                for (int j = 0; j < NWC; ++j) o.d[j] = ld_frag(at(do0 + (int64_t)i * (CH * H * V) + (trans ? 0 : 16 * j), i == last ? ragged : whole));
                 return o;
             };
             auto form = [&](int t, const Own& o) __attribute__((always_inline)) {
-                const int len = (int)min((int64_t)CH, eos - (bos + (int64_t)max(last - t, 0) * CH));
+                const int len = t > 0 ? CH : len_last;
                 char* const db = smem + C::DBUF + (t & 1) * C::DB;
                 const s16x8 y = __builtin_bit_cast(s16x8, o.aq);
                 Frag<T> aq[2], doT[NWC];

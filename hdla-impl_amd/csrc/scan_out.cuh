@@ -50,6 +50,16 @@ template <int K, int V, int NWC, ScanOut OUT> struct OutCfg {
     static constexpr int OUTBOX = SLOTS * SLOT, UBUF = OUTBOX + 2 * OB, XBUF = UBUF + 2 * UB, BYTES = XBUF + 2 * XB;
 };
 
+// Roles of the NM waves behind the computing ones: NL that load, the one that forms, the one that copies the output out.  The forming wave comes first, then
+// (with the output) the copying one, so that none of them is on a SIMD with a computing wave where there are one or two of those: waves go round
+// the four SIMDs, and the forming one has half as many instructions a step as a computing one, a loading one a tenth.  It also finds its
+// rows of v and do by 32-bit offsets from one base, 76 -> 55 instructions a chunk.  us a training step, before -> order -> both: K = 64, V = 128, 2 x 900 tokens
+// of 16 heads 112.3 -> 109.5 -> 107.5 (while the passes read u 109.1), 2 x 1400 152.5 -> 148.4 -> 144.7, K = V = 64, 1 x 256 of 2 35.7 -> 35.8 -> 35.5 (35.2),
+// K = V = 128, 2 x 1537 of 8 175.7 -> 169.4 -> 168.4, K = 128, V = 64, 2 x 900 of 16 133.9 -> 129.6 -> 129.8.  A forward pass that keeps nothing goes without: its forming
+// wave does not turn (I - A_ab)^-1 and was done in time, and one that is done sooner meets the computing waves in LDS: K = V = 128, 2 x 1537 of 8
+// heads 68.5 -> 68.6 -> 69.5, 2 x 1000 49.3 -> 49.6 -> 50.1 (segments' records by themselves: 22.1 -> 20.4).
+template <typename C> __device__ __forceinline__ int forming_first(int wave) { return (wave + C::NL) % C::NM; }
+
 // OUT_O: with the output; OUT_STATE: the forward scan of the backward pass, which leaves the state that enters each chunk; OUT_SUM:
 // records of segments.
 // KEPT: on a workspace of the backward pass (or that it will read, PREP_KEEP): (I - A_ab)^-1 is there turned, as chunk_grad takes it, A_ak in a place of its
@@ -59,6 +69,7 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
     typedef OutCfg<K, V, NWC, OUT> C;
     typedef bf16 T;
     constexpr bool WITH_O = OUT == OUT_O, SUM = OUT == OUT_SUM;
+    constexpr bool FWD = WITH_O && !KEPT;                 // a forward pass that keeps nothing (see forming_first)
     constexpr int KT = C::KT, KT2 = KT / 2, SLOTS = C::SLOTS, SLOT = C::SLOT, PARTS = C::PARTS, KH = C::KH, KH2 = KH / 2;
     constexpr BlkF B = C::B;
     const int h = blockIdx.x;
@@ -81,7 +92,7 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
         // ---- waves that move data.  Barriers: one closing the prologue, one per step, one handing over the last output; the computing
         // waves execute the same sequence.  From the barrier of step t on chunk t + 1 is in LDS and the slot of chunk t is free.
         if (nchunks <= 0) return;
-        const int hw = wv - C::NC;
+        const int hw = FWD ? wv - C::NC : forming_first<C>(wv - C::NC);
         if (hw < C::NL) {
             const int stride = KEPT ? p.ws.sa_stride : B.SIZE;
             const char* const blk = reinterpret_cast<const char*>(p.ws.W) + chw0 * stride + l * 16;
@@ -114,10 +125,17 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
             constexpr int UD = 3;
             struct Own { i32x4 tm[3]; Frag<T> v[NWC]; };
             const Frag<T> ident = ident_frag<T>();
+            // rows of v; behind the end of the last chunk its last row again
+            auto len_of = [&](int t) __attribute__((always_inline)) { return (int)min((int64_t)CH, eos - (bos + (int64_t)min(t, last) * CH)); };
+            const int len_last = len_of(last);
+            const uint32_t row = (uint32_t)(H * V) * sizeof(T), whole = c * row + 8 * g, ragged = min(c, len_last - 1) * row + 8 * g;
+            const T* const v0 = p.v + (bos * H + h) * V + 16 * (trans ? 0 : vt0);
+            auto rows = [&](int t) __attribute__((always_inline)) {
+                if constexpr (FWD) return p.v + ((bos + (int64_t)t * CH + min(c, len_of(t) - 1)) * H + h) * V + 16 * vt0 + 4 * g;
+                else return at(v0 + (int64_t)t * (CH * H * V), t == last ? ragged : whole);
+            };
             auto request = [&](int t) __attribute__((always_inline)) {
                 t = min(t, last);
-                const int64_t tok0 = bos + (int64_t)t * CH;
-                const int len = (int)min((int64_t)CH, eos - tok0);
                 Own o;
 #pragma unroll
                 for (int i = 0; i < 3; ++i) {
@@ -126,8 +144,7 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
                     o.tm[i] = *reinterpret_cast<const i32x4*>(from + 8 * l);
                 }
 #pragma unroll
-                for (int j = 0; j < NWC; ++j)
-                    o.v[j] = ld_frag(p.v + ((tok0 + min(c, len - 1)) * H + h) * V + 16 * (trans ? 0 : vt0 + j) + 4 * g);
+                for (int j = 0; j < NWC; ++j) o.v[j] = ld_frag(rows(t) + (trans ? 0 : 16 * j));
                 return o;
             };
             auto pair = [](i32x4 x, Frag<T>& f0, Frag<T>& f1) __attribute__((always_inline)) {
@@ -136,7 +153,7 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
                 f1.v = __builtin_shufflevector(y, y, 4, 5, 6, 7);
             };
             auto form = [&](int t, const Own& o) __attribute__((always_inline)) {
-                const int len = (int)min((int64_t)CH, eos - (bos + (int64_t)min(t, last) * CH));
+                const int len = FWD ? len_of(t) : t < last ? CH : len_last;
                 T* const ub = reinterpret_cast<T*>(smem + C::UBUF + (t & 1) * C::UB);
                 Frag<T> tm[2][2], aak[2], vT[NWC], mT[NWC][2];
                 pair(o.tm[0], tm[0][0], tm[0][1]);
