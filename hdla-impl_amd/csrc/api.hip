@@ -15,6 +15,7 @@ using namespace hdla;
 namespace {
 
 constexpr int CHUNK = 16;
+constexpr int AAK_STRIDE = 512, AAK_STRIDE_RECORD = 1024;    // elements between the tile pairs of A_ak: by themselves, in the record beside those of A_qb
 
 inline size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -324,7 +325,7 @@ void bind_ws(ChunkArgs<T>& a, const hdla_dims* d, const WsLayout& LP, void* prep
     char* base = static_cast<char*>(prep_ws);
     auto at = [&](size_t o) { return reinterpret_cast<T*>(base + o); };
     a.ws.W = at(LP.W); a.ws.UT = LP.UT ? at(LP.UT) : nullptr; a.ws.KGT = at(LP.KGT); a.ws.BGT = at(LP.BGT);
-    a.ws.VTT = LP.VTT ? at(LP.VTT) : nullptr; a.ws.AAK = at(LP.AAK); a.ws.aak_stride = 512;
+    a.ws.VTT = LP.VTT ? at(LP.VTT) : nullptr; a.ws.AAK = at(LP.AAK); a.ws.aak_stride = AAK_STRIDE;
     a.ws.SUM = reinterpret_cast<float*>(base + LP.SUM);
     a.ws.QG = at(LP.QG); a.ws.AQK = at(LP.AQK); a.ws.AQB = at(LP.AQB);
     a.ws.AQBT = at(LP.AQBT); a.ws.QGT = at(LP.QGT);
@@ -503,7 +504,7 @@ int run_fused(const hdla_dims* d, bool fwd, const void* q, const void* k, const 
         f.aq = reinterpret_cast<T*>(base + L.AQ);
         f.mt = reinterpret_cast<float*>(base + L.MT);
     }
-    a.ws.AAK = f.aq; a.ws.aak_stride = 1024;                       // (of the record's pairs, the first)
+    a.ws.AAK = f.aq; a.ws.aak_stride = AAK_STRIDE_RECORD;          // (of the record's pairs, the first)
     a.ws.SUM = reinterpret_cast<float*>(base + L.SUM);
     a.ws.sa_stride = 2 * d->K * 16 * 2;                            // chunk_grad's view of w: [2][K/16] tiles per slot
     a.st.cu = d->cu_seqlens;
@@ -682,6 +683,7 @@ int hdla_workspace_layout(const hdla_dims* dims, int pass, hdla_ws_layout* out) 
         out->CHUNK_OFF = F.CHUNK_OFF; out->CHUNK_SEQ = F.CHUNK_SEQ;
         out->total = F.total;
         out->ERR = F.ERR;
+        if (pass == HDLA_PASS_BWD) { out->AAK = F.AQ; out->AAK_STRIDE = AAK_STRIDE_RECORD * 2; out->SUM = F.SUM; }
         return HDLA_OK;
     }
     rc = make_layout(dims, pass, L, nch);
@@ -695,6 +697,7 @@ int hdla_workspace_layout(const hdla_dims* dims, int pass, hdla_ws_layout* out) 
     out->CHUNK_OFF = L.CHUNK_OFF; out->CHUNK_SEQ = L.CHUNK_SEQ;
     out->total = L.total;
     out->ERR = -1;
+    out->AAK = L.AAK; out->AAK_STRIDE = L.AAK ? AAK_STRIDE * 2 : 0; out->SUM = L.SUM;
     return HDLA_OK;
 }
 

@@ -12,7 +12,7 @@ from typing import Optional, Tuple
 import torch
 
 HDLA_BF16, HDLA_FP32 = 0, 1
-HDLA_VERSION = 209          # the header this binding was written against (struct layouts, entry points)
+HDLA_VERSION = 210          # the header this binding was written against (struct layouts, entry points)
 ROUTE_AUTO, ROUTE_CLASSIC, ROUTE_FUSED, ROUTE_PLAIN = 0, 1, 2, 4
 _ROUTES = {"": ROUTE_AUTO, "auto": ROUTE_AUTO, "classic": ROUTE_CLASSIC, "plain": ROUTE_PLAIN, "fused": ROUTE_FUSED}
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -32,7 +32,7 @@ class HdlaDims(ctypes.Structure):
 
 class HdlaWsLayout(ctypes.Structure):
     _names = ["nch", "W", "UT", "KGT", "BGT", "VTT", "EGL", "QG", "AQK", "AQB", "AQBT", "QGT", "TM",
-              "HC", "DHC", "DVN", "STRONG", "SA_STRIDE", "SB_STRIDE", "CHUNK_OFF", "CHUNK_SEQ", "total", "ERR"]
+              "HC", "DHC", "DVN", "STRONG", "SA_STRIDE", "SB_STRIDE", "CHUNK_OFF", "CHUNK_SEQ", "total", "ERR", "AAK", "AAK_STRIDE", "SUM"]
     _fields_ = [(n, ctypes.c_int64) for n in _names]
 
 

@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-#define HDLA_VERSION 209
+#define HDLA_VERSION 210
 
 enum { HDLA_BF16 = 0, HDLA_FP32 = 1 };
 
@@ -113,6 +113,9 @@ typedef struct hdla_ws_layout {
     int64_t ERR;               /* fused route: int32 that reads (HDLA_FUSED_ABORTED | 1..3) only if a wave's bounded wait for
                                 * another wave ran out (the kernels then stop early and the results are invalid); the
                                 * library never clears it; -1 on the classic route */
+    int64_t AAK, AAK_STRIDE;   /* bf16 inputs, in the passes whose scans form u themselves (HDLA_PASS_FWD: in TM): the two ranks of A_ak, a tile pair
+                                * (rows i, inner j) per slot, slots AAK_STRIDE bytes apart */
+    int64_t SUM;               /* likewise, the hdla_param_ forms: fp32 [16] per slot, sum over the channels of k^2 exp(gk) */
 } hdla_ws_layout;
 
 int hdla_version(void);
