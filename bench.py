@@ -208,7 +208,7 @@ def norm_traffic(rows):
     from the committed counter summary, or None."""
     try:
         table = json.load(open(os.path.join(ROOT, "profiles", "hbm_traffic.json"))).get("norm", {})
-        return sum(table[f"{k}@{rows}rows"]["hbm_bytes_per_launch"] for k in ("normalize_bwd_kernel<bf16, 2>", "normalize_dw_kernel"))
+        return sum(table[f"{k}@{rows}rows"]["hbm_bytes_per_launch"] for k in ("normalize_bwd_kernel<bf16, 2>", "sums_kernel"))
     except (OSError, ValueError, KeyError):
         return None
 

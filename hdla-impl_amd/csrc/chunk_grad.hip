@@ -61,7 +61,7 @@ template <typename T, int K, int V> struct CgLds {
     // per wave and token: three partial sums over channels of the backward of the HDLA parameterisation
     static constexpr int RED = KG + KG_B, RED_B = NW * 3 * CH * 4;
     static constexpr int R1 = RED + RED_B, WALL = R1 + PART_B, R1_B = PART_B + WALL_B > OUT_B ? PART_B + WALL_B : OUT_B;
-    // tiles of 4-byte elements that are turned, per wave (K = V = 128 has no registers for it)
+    // tiles of 4-byte elements that are turned from registers, per wave (K = V = 128 has no registers for it; what lies in LDS as rows is read by columns there too)
     static constexpr bool BY_LDS = ES == 4 && K * V < 128 * 128;
     static constexpr int TURNING = R1 + R1_B;
     static constexpr int BYTES = TURNING + (BY_LDS ? NW * TURN_SCRATCH : 0);
