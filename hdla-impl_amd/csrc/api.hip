@@ -8,6 +8,7 @@
 
 #include "fused_shapes.h"
 #include "hdla_launch.h"
+#include "host_path.h"
 #include "hdla_ws.h"
 
 using namespace hdla;
@@ -173,6 +174,20 @@ int kept_plan_segments(const hdla_dims* d, int32_t& bwd) {
     return fwd;
 }
 
+// Whether a training call leaves the states that enter the chunks as well (hdla_states_plan), 2.0 times the inputs' bytes in all at K = V = 128 where the chunks'
+// operands alone are 1.1: the forward pass's scan has them, and the backward pass's reverse scan has the device to itself.  Not where both scans of that
+// pass fit the device in their narrowest workgroups: side by side they take no longer than one.  us a training step, without the states -> with them, 2-byte elements, K = V = 128:
+// 16384 tokens of 16 heads in 4 sequences, where nothing was kept before, 1635 -> 1425 (the pair of scans 510 -> 328, the forward pass's 253 -> 378, prep 348 -> 190), 4 x 2048, beta
+// form 718 -> 640, 4 x 1000 of 16 338 -> 335, 36 lanes of 63 chunks 223 -> 194, 32 167 -> 156, 24 148 -> 131; on the other side of the line, as a graph's replay, 16 of 63 116 -> 115, 16 of
+// 97 162 -> 159, 8 of 63 98.4 -> 98.0, 2 of 7 37.7 -> 38.0, 16 heads of 256 tokens 47.1 -> 46.7.  K = 64, V = 128, 48 lanes 143 -> 129, 16 67.0 -> 65.9; K = 128, V = 64, 48 lanes 198 -> 178, 32
+// 134.4 -> 131.5.  STATES_MOST: what calls may hold on a device in all (native.cpp, kept_room).
+constexpr size_t STATES_MOST = (size_t)1 << 30;
+constexpr long long SCAN_PAIR_WORKGROUPS = 256;               // one a compute unit (launch_scan_grad_shape)
+bool leaves_states(const hdla_dims* d) {
+    if (d->in_dtype != HDLA_BF16 || d->route != HDLA_ROUTE_AUTO || d->segments > 1 || scan_segments(d, false) > 1 || scan_segments(d, true) > 1) return false;
+    return 2LL * d->N * d->H * (d->V / 16) > SCAN_PAIR_WORKGROUPS;
+}
+
 struct FusedLayout {
     size_t OL, GW, SLOC, MSEG, RSEG, SIN, ERR;                 // fused kernels' own
     size_t HC, DHC, DVN, TM, UT, W, SUM, STRONG;               // what chunk_grad reads (backward pass; UT and W beside fp32 decays)
@@ -249,7 +264,9 @@ FusedRecord fused_record(const hdla_dims* d, const FusedLayout& L) {
 }
 
 // pass: HDLA_PASS_FWD, _BWD, _FWD_KEEP (a forward pass that leaves what the backward pass needs of it), _BWD_KEPT (the
-// scratch of a backward pass that runs on such a workspace: only what its own scans write)
+// scratch of a backward pass that runs on such a workspace: only what its own scans write), PASS_FWD_STATES and PASS_BWD_STATES (the same two where the
+// states that enter the chunks are left as well)
+constexpr int PASS_FWD_STATES = 4, PASS_BWD_STATES = 5;
 int make_layout(const hdla_dims* d, int pass, WsLayout& L, int& nch) {
     const int rc = check_dims(d);
     if (rc) return rc;
@@ -264,15 +281,17 @@ int make_layout(const hdla_dims* d, int pass, WsLayout& L, int& nch) {
     size_t off = 0;
     auto take = [&](size_t bytes) { const size_t o = off; off += up256(bytes); return o; };
     L = WsLayout{};
-    const bool prep_out = pass != HDLA_PASS_BWD_KEPT;             // what the prep kernel writes
+    const bool states = pass == PASS_FWD_STATES;
+    const bool prep_out = pass != HDLA_PASS_BWD_KEPT && pass != PASS_BWD_STATES;   // what the prep kernel writes
     const bool with_o = pass == HDLA_PASS_FWD || pass == HDLA_PASS_FWD_KEEP;
-    const bool bwd_parts = pass == HDLA_PASS_BWD || pass == HDLA_PASS_FWD_KEEP;
-    const bool scan_out = pass == HDLA_PASS_BWD || pass == HDLA_PASS_BWD_KEPT;
+    const bool bwd_parts = pass == HDLA_PASS_BWD || pass == HDLA_PASS_FWD_KEEP || states;
+    const bool scan_out = pass == HDLA_PASS_BWD || pass == HDLA_PASS_BWD_KEPT || pass == PASS_BWD_STATES;
     if (prep_out) {
         const BlkF bf = blk_fwd(d->K, (int)es, with_o);
         const size_t sa = take(chw * (size_t)bf.SIZE);
         L.SA_STRIDE = bf.SIZE;
         L.W = sa + bf.W; L.BGT = sa + bf.BGT; L.KGT = sa + bf.KGT; L.EGL = sa + bf.EGL;
+        if (states) L.AQK = sa + blk_fwd(d->K, (int)es, true).AQK;   // (q's tiles and A_qb are in the forward pass's own workspace)
         if (with_o) { L.QG = sa + bf.QG; L.AQB = sa + bf.AQB; L.AQK = sa + bf.AQK; }
         if (pass == HDLA_PASS_FWD && es == 2) {
             L.TM = take(chw * 1536 * es);                         // the scan forms u itself (scan_out.cuh)
@@ -295,15 +314,16 @@ int make_layout(const hdla_dims* d, int pass, WsLayout& L, int& nch) {
         L.STRONG = take(chw * 4);
     }
     if (scan_out) {
-        L.HC = take(chw * K * V * es);
+        if (pass != PASS_BWD_STATES) L.HC = take(chw * K * V * es);
         L.DHC = take(chw * K * V * es);
         L.DVN = take(chw * 2 * 16 * V * es);
     }
+    if (states) L.HC = take(chw * K * V * es);
     if (d->cu_seqlens && prep_out) {
         L.CHUNK_OFF = take((size_t)(2 * d->N + 1) * 4);          // chunk_off [N+1], then order [N]
         L.CHUNK_SEQ = take((size_t)(nch > 0 ? nch : 1) * 4);
     }
-    const int nseg = pass == HDLA_PASS_FWD || pass == HDLA_PASS_BWD ? scan_segments(d, pass == HDLA_PASS_BWD) : kept_segments(d);
+    const int nseg = states || pass == PASS_BWD_STATES ? 1 : pass == HDLA_PASS_FWD || pass == HDLA_PASS_BWD ? scan_segments(d, pass == HDLA_PASS_BWD) : kept_segments(d);
     if (nseg > 1) {
         const size_t recs = (size_t)d->N * d->H * nseg, state = recs * K * V * 4, matrix = recs * K * K * 4;
         if (prep_out) { L.SEG_LOC = take(state); L.SEG_TR = take(matrix); L.SEG_IN = take(state); }
@@ -359,8 +379,11 @@ inline bool bad_ws(const void* p, size_t have, size_t need) {
     return !p || (reinterpret_cast<uintptr_t>(p) & 255) || have < need;
 }
 
+// what a forward pass that leaves the states has for itself
+size_t states_fwd_workspace(const hdla_dims* d, int nch) { return std::max<size_t>(256, up256((size_t)d->H * nch * blk_q(d->K, 2))); }
+
 // pass: HDLA_PASS_FWD / _BWD on `workspace`; HDLA_PASS_FWD_KEEP on `kept`; HDLA_PASS_BWD_KEPT on `kept` (read) and
-// `workspace` (what the scans write)
+// `workspace` (what the scans write); PASS_FWD_STATES and PASS_BWD_STATES on both
 template <typename T>
 int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const void* v, const void* a_,
               const void* b, const void* gk, const float* h0, void* o, float* ht, const void* d_o,
@@ -369,21 +392,23 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
               const void* beta = nullptr, void* dbeta = nullptr, void* kept = nullptr, size_t kept_bytes = 0) {
     WsLayout LP, LS;
     int nch = 0;
-    const bool fwd = pass == HDLA_PASS_FWD || pass == HDLA_PASS_FWD_KEEP;
-    const bool on_kept = pass == HDLA_PASS_FWD_KEEP || pass == HDLA_PASS_BWD_KEPT;
+    const bool states = pass == PASS_FWD_STATES || pass == PASS_BWD_STATES;
+    const bool fwd = pass == HDLA_PASS_FWD || pass == HDLA_PASS_FWD_KEEP || pass == PASS_FWD_STATES;
+    const bool on_kept = pass == HDLA_PASS_FWD_KEEP || pass == HDLA_PASS_BWD_KEPT || states;
     hdla_dims kept_dims = *d;
     if (pass == HDLA_PASS_BWD_KEPT && d->route == HDLA_ROUTE_CLASSIC) kept_dims.route = HDLA_ROUTE_PLAIN;   // (what this pass reads)
-    int rc = make_layout(&kept_dims, on_kept ? HDLA_PASS_FWD_KEEP : pass, LP, nch);
+    int rc = make_layout(&kept_dims, states ? PASS_FWD_STATES : on_kept ? HDLA_PASS_FWD_KEEP : pass, LP, nch);
     if (rc) return rc;
     void* prep_ws = on_kept ? kept : workspace;
     if (bad_ws(prep_ws, on_kept ? kept_bytes : workspace_bytes, LP.total)) return HDLA_ERR_WORKSPACE;
     LS = LP;
-    if (pass == HDLA_PASS_BWD_KEPT) {
+    if (pass == PASS_FWD_STATES && bad_ws(workspace, workspace_bytes, states_fwd_workspace(d, nch))) return HDLA_ERR_WORKSPACE;
+    if (pass == HDLA_PASS_BWD_KEPT || pass == PASS_BWD_STATES) {
         rc = make_layout(d, pass, LS, nch);
         if (rc) return rc;
         if (bad_ws(workspace, workspace_bytes, LS.total)) return HDLA_ERR_WORKSPACE;
         // (the records lie where their number puts them: another number's buffer, which another size shows, would be read wrongly)
-        if (kept_segments(d) > 1 && kept_bytes != LP.total) return HDLA_ERR_WORKSPACE;
+        if (!states && kept_segments(d) > 1 && kept_bytes != LP.total) return HDLA_ERR_WORKSPACE;
     }
     ChunkArgs<T> a{};
     a.q = static_cast<const T*>(q); a.k = static_cast<const T*>(k); a.v = static_cast<const T*>(v);
@@ -395,9 +420,16 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
     a.dq = static_cast<T*>(dq); a.dk = static_cast<T*>(dk); a.dv = static_cast<T*>(dv);
     a.da = static_cast<T*>(da); a.db = static_cast<T*>(db); a.dgk = dgk;
     a.beta = static_cast<const T*>(beta); a.dbeta = static_cast<T*>(dbeta);
-    bind_ws(a, d, LP, prep_ws, LS, pass == HDLA_PASS_BWD_KEPT ? workspace : prep_ws, nch);
+    bind_ws(a, d, LP, prep_ws, LS, pass == HDLA_PASS_BWD_KEPT || pass == PASS_BWD_STATES ? workspace : prep_ws, nch);
+    if (states) a.ws.HC = reinterpret_cast<T*>(static_cast<char*>(kept) + LP.HC);
+    if (pass == PASS_FWD_STATES) {
+        constexpr int es = 2;
+        const BlkF b = blk_fwd(d->K, es, true);
+        a.ws.QG = static_cast<T*>(workspace);
+        a.ws.AQB = reinterpret_cast<T*>(static_cast<char*>(workspace) + (b.AQB - b.QG));
+    }
     a.seg = SegRec{1, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-    const int nseg = on_kept ? kept_segments(d) : scan_segments(d, !fwd);
+    const int nseg = states ? 1 : on_kept ? kept_segments(d) : scan_segments(d, !fwd);
     if (nseg > 1) {
         const auto at = [](void* base, size_t o) { return reinterpret_cast<float*>(static_cast<char*>(base) + o); };
         a.seg = SegRec{nseg, at(prep_ws, LP.SEG_LOC), at(prep_ws, LP.SEG_TR), at(prep_ws, LP.SEG_IN), nullptr, nullptr, nullptr, nullptr};
@@ -407,7 +439,8 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
         if (pass == HDLA_PASS_FWD_KEEP || (pass == HDLA_PASS_BWD && d->segments > 0)) a.seg.turned = at(prep_ws, LP.SEG_RTR);
     }
     hipError_t e;
-    if (pass == HDLA_PASS_BWD_KEPT) {
+    if (pass == PASS_BWD_STATES) stages &= ~HDLA_STAGE_SCAN_FWD;   // the forward pass has left what it leaves
+    if (pass == HDLA_PASS_BWD_KEPT || pass == PASS_BWD_STATES) {
         stages &= ~HDLA_STAGE_PREP;                                // the forward pass has run it
         if (d->cu_seqlens) {
             e = launch_clear_uncovered(d->cu_seqlens, d->N, d->T, packed_outputs(d, a), stream);
@@ -427,7 +460,7 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
             if (e != hipSuccess) return (int)e;
         }
         if (nch > 0) {
-            e = launch_prep<T>(a, d->K, d->V, pass == HDLA_PASS_FWD ? 0 : pass == HDLA_PASS_BWD ? 1 : 2, made ? &out : nullptr, share_V, stream);
+            e = launch_prep<T>(a, d->K, d->V, pass == HDLA_PASS_FWD ? 0 : pass == HDLA_PASS_BWD ? 1 : pass == PASS_FWD_STATES ? 3 : 2, made ? &out : nullptr, share_V, stream);
             if (e != hipSuccess) return (int)e;
         }
     }
@@ -442,7 +475,7 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
         e = launch_scan_pair<T>(a, d->K, d->V, stream);
         if (e != hipSuccess) return (int)e;
     } else if (stages & HDLA_STAGE_SCAN_FWD) {
-        e = fwd ? launch_scan_out<T>(a, d->K, d->V, pass == HDLA_PASS_FWD_KEEP, stream) : launch_scan_fwd<T>(a, d->K, d->V, stream);
+        e = fwd ? launch_scan_out<T>(a, d->K, d->V, pass == PASS_FWD_STATES ? 2 : pass == HDLA_PASS_FWD_KEEP, stream) : launch_scan_fwd<T>(a, d->K, d->V, stream);
         if (e != hipSuccess) return (int)e;
     }
     if (!fwd) {
@@ -662,6 +695,18 @@ size_t hdla_keep_plan(const hdla_dims* dims, int32_t* fwd_segments, int32_t* bwd
     return L.total;
 }
 
+size_t hdla_states_plan(const hdla_dims* dims, size_t* fwd_workspace, size_t* bwd_workspace) {
+    bool fused_fwd, fused_bwd;
+    if (!fwd_workspace || !bwd_workspace || check_dims(dims) || dims->T < 1) return 0;
+    if (pick_route(dims, HDLA_PASS_FWD, false, fused_fwd) || pick_route(dims, HDLA_PASS_BWD, false, fused_bwd) || fused_fwd || fused_bwd) return 0;
+    WsLayout L, S;
+    int nch;
+    if (!leaves_states(dims) || make_layout(dims, PASS_FWD_STATES, L, nch) || L.total > STATES_MOST || make_layout(dims, PASS_BWD_STATES, S, nch)) return 0;
+    *fwd_workspace = states_fwd_workspace(dims, nch);
+    *bwd_workspace = S.total;
+    return L.total;
+}
+
 int hdla_workspace_layout(const hdla_dims* dims, int pass, hdla_ws_layout* out) {
     if (!out) return HDLA_ERR_NULL;
     if (pass < HDLA_PASS_FWD || pass > HDLA_PASS_BWD_KEPT) return HDLA_ERR_SHAPE;
@@ -816,32 +861,43 @@ int hdla_chunk_bwd_b(const hdla_dims* dims, const void* q, const void* k, const 
                          boundary_bytes, workspace, workspace_bytes, stream);
 }
 
-int hdla_chunk_fwd_keep(const hdla_dims* dims, const void* q, const void* k, const void* v, const void* a,
-                        const void* b, const void* beta, const void* gk, const float* h0, void* o, float* ht,
-                        void* kept, size_t kept_bytes, void* stream) {
-    const int rc = check_dims(dims);
-    if (rc) return rc;
+// pass: HDLA_PASS_FWD_KEEP or PASS_FWD_STATES
+static int chunk_fwd_kept(const hdla_dims* dims, int pass, const void* q, const void* k, const void* v, const void* a,
+                          const void* b, const void* beta, const void* gk, const float* h0, void* o, float* ht,
+                          void* kept, size_t kept_bytes, void* workspace, size_t workspace_bytes, void* stream) {
     if (dims->T > 0 && (!q || !k || !v || !gk || !o || (!beta && (!a || !b)))) return HDLA_ERR_NULL;
     if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(a) || !aligned16(b) || !aligned16(gk) ||
         !aligned16(o) || !aligned16(h0) || !aligned16(ht)) return HDLA_ERR_ALIGN;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (beta) { a = nullptr; b = nullptr; }
     if (dims->in_dtype == HDLA_BF16)
-        return run_chunk<bf16>(dims, HDLA_PASS_FWD_KEEP, q, k, v, a, b, gk, h0, o, ht, nullptr, nullptr, nullptr, nullptr,
-                               nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, s, HDLA_STAGE_ALL, beta, nullptr,
+        return run_chunk<bf16>(dims, pass, q, k, v, a, b, gk, h0, o, ht, nullptr, nullptr, nullptr, nullptr,
+                               nullptr, nullptr, nullptr, nullptr, nullptr, workspace, workspace_bytes, s, HDLA_STAGE_ALL, beta, nullptr,
                                kept, kept_bytes);
-    return run_chunk<float>(dims, HDLA_PASS_FWD_KEEP, q, k, v, a, b, gk, h0, o, ht, nullptr, nullptr, nullptr, nullptr,
-                            nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, s, HDLA_STAGE_ALL, beta, nullptr,
+    return run_chunk<float>(dims, pass, q, k, v, a, b, gk, h0, o, ht, nullptr, nullptr, nullptr, nullptr,
+                            nullptr, nullptr, nullptr, nullptr, nullptr, workspace, workspace_bytes, s, HDLA_STAGE_ALL, beta, nullptr,
                             kept, kept_bytes);
 }
-
-int hdla_chunk_bwd_kept(const hdla_dims* dims, const void* q, const void* k, const void* v, const void* a,
-                        const void* b, const void* beta, const void* gk, const float* h0, const void* d_o,
-                        const float* dht, void* dq, void* dk, void* dv, void* da, void* db, void* dbeta, void* dgk,
-                        float* dh0, void* kept, size_t kept_bytes, void* workspace, size_t workspace_bytes,
-                        void* stream) {
+int hdla_chunk_fwd_keep(const hdla_dims* dims, const void* q, const void* k, const void* v, const void* a,
+                        const void* b, const void* beta, const void* gk, const float* h0, void* o, float* ht,
+                        void* kept, size_t kept_bytes, void* stream) {
     const int rc = check_dims(dims);
     if (rc) return rc;
+    return chunk_fwd_kept(dims, HDLA_PASS_FWD_KEEP, q, k, v, a, b, beta, gk, h0, o, ht, kept, kept_bytes, nullptr, 0, stream);
+}
+int hdla_chunk_fwd_states(const hdla_dims* dims, const void* q, const void* k, const void* v, const void* a, const void* b, const void* beta, const void* gk,
+                          const float* h0, void* o, float* ht, void* kept, size_t kept_bytes, void* workspace, size_t workspace_bytes, void* stream) {
+    const int rc = check_dims(dims);
+    if (rc) return rc;
+    if (!leaves_states(dims)) return HDLA_ERR_SHAPE;
+    return chunk_fwd_kept(dims, PASS_FWD_STATES, q, k, v, a, b, beta, gk, h0, o, ht, kept, kept_bytes, workspace, workspace_bytes, stream);
+}
+
+static int chunk_bwd_kept(const hdla_dims* dims, int pass, const void* q, const void* k, const void* v, const void* a,
+                          const void* b, const void* beta, const void* gk, const float* h0, const void* d_o,
+                          const float* dht, void* dq, void* dk, void* dv, void* da, void* db, void* dbeta, void* dgk,
+                          float* dh0, void* kept, size_t kept_bytes, void* workspace, size_t workspace_bytes,
+                          void* stream) {
     if (dims->T > 0 && (!q || !k || !v || !gk || !d_o || !dq || !dk || !dv || !dgk)) return HDLA_ERR_NULL;
     if (dims->T > 0 && (beta ? !dbeta : (!a || !b || !da || !db))) return HDLA_ERR_NULL;
     if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(a) || !aligned16(b) || !aligned16(gk) ||
@@ -850,10 +906,29 @@ int hdla_chunk_bwd_kept(const hdla_dims* dims, const void* q, const void* k, con
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (beta) { a = nullptr; b = nullptr; da = nullptr; db = nullptr; }
     if (dims->in_dtype == HDLA_BF16)
-        return run_chunk<bf16>(dims, HDLA_PASS_BWD_KEPT, q, k, v, a, b, gk, h0, nullptr, nullptr, d_o, dht, dq, dk, dv, da,
+        return run_chunk<bf16>(dims, pass, q, k, v, a, b, gk, h0, nullptr, nullptr, d_o, dht, dq, dk, dv, da,
                                db, dgk, dh0, workspace, workspace_bytes, s, HDLA_STAGE_ALL, beta, dbeta, kept, kept_bytes);
-    return run_chunk<float>(dims, HDLA_PASS_BWD_KEPT, q, k, v, a, b, gk, h0, nullptr, nullptr, d_o, dht, dq, dk, dv, da,
+    return run_chunk<float>(dims, pass, q, k, v, a, b, gk, h0, nullptr, nullptr, d_o, dht, dq, dk, dv, da,
                             db, dgk, dh0, workspace, workspace_bytes, s, HDLA_STAGE_ALL, beta, dbeta, kept, kept_bytes);
+}
+int hdla_chunk_bwd_kept(const hdla_dims* dims, const void* q, const void* k, const void* v, const void* a,
+                        const void* b, const void* beta, const void* gk, const float* h0, const void* d_o,
+                        const float* dht, void* dq, void* dk, void* dv, void* da, void* db, void* dbeta, void* dgk,
+                        float* dh0, void* kept, size_t kept_bytes, void* workspace, size_t workspace_bytes,
+                        void* stream) {
+    const int rc = check_dims(dims);
+    if (rc) return rc;
+    return chunk_bwd_kept(dims, HDLA_PASS_BWD_KEPT, q, k, v, a, b, beta, gk, h0, d_o, dht, dq, dk, dv, da, db, dbeta, dgk, dh0, kept, kept_bytes, workspace,
+                          workspace_bytes, stream);
+}
+int hdla_chunk_bwd_states(const hdla_dims* dims, const void* q, const void* k, const void* v, const void* a, const void* b, const void* beta, const void* gk,
+                          const float* h0, const void* d_o, const float* dht, void* dq, void* dk, void* dv, void* da, void* db, void* dbeta, void* dgk, float* dh0,
+                          void* kept, size_t kept_bytes, void* workspace, size_t workspace_bytes, void* stream) {
+    const int rc = check_dims(dims);
+    if (rc) return rc;
+    if (!leaves_states(dims)) return HDLA_ERR_SHAPE;
+    return chunk_bwd_kept(dims, PASS_BWD_STATES, q, k, v, a, b, beta, gk, h0, d_o, dht, dq, dk, dv, da, db, dbeta, dgk, dh0, kept, kept_bytes, workspace,
+                          workspace_bytes, stream);
 }
 
 int hdla_chunk_stages(const hdla_dims* dims, int pass, int stages, const void* q, const void* k, const void* v,

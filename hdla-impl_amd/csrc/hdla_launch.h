@@ -21,14 +21,15 @@ hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int H, i
 hipError_t launch_clear_uncovered(const int64_t* cu, int N, int T, const PackedOut& out, hipStream_t stream);
 
 // K, V in {64, 128}; returns hipErrorInvalidValue for any other pair.
-// mode: 0 = for the forward pass, 1 = for the backward pass, 2 = forward pass whose workspace the backward pass will use
+// mode: 0 = for the forward pass, 1 = for the backward pass, 2 = forward pass whose workspace the backward pass will use, 3 = the same with the
+// states that enter the chunks in it (2-byte elements)
 // out: with it the launch leaves the chunk table too and does launch_chunk_table's other work (prep_makes_table says whether it can); share_V as V there
 inline bool prep_makes_table(const int64_t* cu, int N, int H, int nch) { return cu && N <= 64 /* FEW_SEQS */ && nch > 0 && (long long)H * nch < 0x7ffff000LL; }
 template <typename T> hipError_t launch_prep(const ChunkArgs<T>& a, int K, int V, int mode, const PackedOut* out, int share_V, hipStream_t stream);
 // the two scans of the backward pass
 template <typename T> hipError_t launch_scan_fwd(const ChunkArgs<T>& a, int K, int V, hipStream_t stream);
-// the scan of the forward pass, with the output (kept: after launch_prep of mode 2, otherwise of mode 0)
-template <typename T> hipError_t launch_scan_out(const ChunkArgs<T>& a, int K, int V, bool kept, hipStream_t stream);
+// the scan of the forward pass, with the output (kept: 0 after launch_prep of mode 0, 1 of mode 2, 2 of mode 3)
+template <typename T> hipError_t launch_scan_out(const ChunkArgs<T>& a, int K, int V, int kept, hipStream_t stream);
 template <typename T> hipError_t launch_scan_bwd(const ChunkArgs<T>& a, int K, int V, hipStream_t stream);
 // both in one launch
 template <typename T> hipError_t launch_scan_pair(const ChunkArgs<T>& a, int K, int V, hipStream_t stream);

@@ -73,6 +73,10 @@ constexpr BlkB blk_bwd(int K, int es) {
     return b;
 }
 
+// what the block with the output's part has behind the one without: q's tiles and A_qb, which lie by themselves where the forward pass leaves the
+// states as well (PREP_STATES; A_qk is in the second half of the EGL piece)
+constexpr int blk_q(int K, int es) { return blk_fwd(K, es, true).SIZE - blk_fwd(K, es, false).SIZE; }
+
 // LDS slot of the reverse scan, assembled from 1-KiB pieces of both blocks of a (chunk, head): W and BGT (the first
 // NIF pieces of the forward-scan block), the piece holding EGL, then the reverse-scan block.
 struct SlotB { int W, BGT, EGL, QGT, AQBT, SIZE, NIF, EGL_SRC; };

@@ -1,0 +1,16 @@
+// Entry points of libhdla_hip.so that native.cpp calls beside those of include/hdla_hip.h.  Both are built together: they are no part of the C ABI and of
+// its version number.
+#pragma once
+#include "../../include/hdla_hip.h"
+
+extern "C" {
+// A training call that leaves its backward pass, beside what hdla_chunk_fwd_keep leaves, the states that enter the chunks: that pass runs the reverse
+// scan alone.  hdla_states_plan: bytes of the buffer to hold between the passes, 0 where it does not pay or is too large; fwd_workspace, bwd_workspace: bytes of scratch of the
+// two calls.  One segment in both passes; the results, and those of a backward pass without the buffer (HDLA_ROUTE_PLAIN), are the same bits.
+size_t hdla_states_plan(const hdla_dims* dims, size_t* fwd_workspace, size_t* bwd_workspace);
+int hdla_chunk_fwd_states(const hdla_dims* dims, const void* q, const void* k, const void* v, const void* a, const void* b, const void* beta, const void* gk,
+                          const float* h0, void* o, float* ht, void* kept, size_t kept_bytes, void* workspace, size_t workspace_bytes, void* stream);
+int hdla_chunk_bwd_states(const hdla_dims* dims, const void* q, const void* k, const void* v, const void* a, const void* b, const void* beta, const void* gk,
+                          const float* h0, const void* d_o, const float* dht, void* dq, void* dk, void* dv, void* da, void* db, void* dbeta, void* dgk, float* dh0,
+                          void* kept, size_t kept_bytes, void* workspace, size_t workspace_bytes, void* stream);
+}

@@ -35,6 +35,7 @@
 #include <vector>
 
 #include "../../include/hdla_hip.h"
+#include "host_path.h"
 
 namespace {
 
@@ -46,7 +47,7 @@ using torch::autograd::variable_list;
 struct Api {
 #define HDLA_FN(name) decltype(&hdla_##name) name
     HDLA_FN(strerror); HDLA_FN(workspace_bytes); HDLA_FN(record_bytes); HDLA_FN(record_workspace_bytes); HDLA_FN(chunk_fwd_b); HDLA_FN(chunk_bwd_b);
-    HDLA_FN(keep_plan); HDLA_FN(chunk_fwd_keep); HDLA_FN(chunk_bwd_kept);
+    HDLA_FN(keep_plan); HDLA_FN(chunk_fwd_keep); HDLA_FN(chunk_bwd_kept); HDLA_FN(states_plan); HDLA_FN(chunk_fwd_states); HDLA_FN(chunk_bwd_states);
     HDLA_FN(recurrent_fwd); HDLA_FN(param_recurrent_fwd); HDLA_FN(normalize_fwd); HDLA_FN(normalize_bwd_as);
     HDLA_FN(normalize_workspace_bytes); HDLA_FN(layer_pre_fwd); HDLA_FN(layer_pre_bwd); HDLA_FN(layer_up_fwd); HDLA_FN(layer_down);
     HDLA_FN(layer_up_wgrad); HDLA_FN(layer_up_wgrad_workspace_bytes); HDLA_FN(rows_gemm); HDLA_FN(sum_partials); HDLA_FN(stack_rows);
@@ -105,7 +106,9 @@ bool env_is(const char* name, std::initializer_list<const char*> values, bool un
 bool keep_forward_default() { return !env_is("HDLA_HIP_KEEP_FORWARD", {"", "0", "false", "False"}, true); }
 bool keep_forward_unsaid() { return env("HDLA_HIP_KEEP_FORWARD") == nullptr; }
 // launch plan of a chunked call, and what its backward pass may be given: the record, and where the route has none the forward pass's workspace
-struct Plan { int32_t route, segments; bool record, keep; };
+// (keep: KEEP_STATES with the states that enter the chunks)
+enum Keep : int32_t { KEEP_NOTHING, KEEP_FORWARD, KEEP_STATES };
+struct Plan { int32_t route, segments; bool record; Keep keep; };
 // false: the Python code has to look at it (another spelling, a number that is none)
 bool read_plan(Plan& p) {
     const char* r = env("HDLA_HIP_ROUTE");
@@ -115,7 +118,7 @@ bool read_plan(Plan& p) {
     else if (!strcmp(r, "fused")) p.route = HDLA_ROUTE_FUSED;
     else return false;
     p.record = env_is("HDLA_HIP_INPUTS_ONLY", {"", "0", "false", "False"}, true);
-    p.keep = false;
+    p.keep = KEEP_NOTHING;
     p.segments = 0;
     const char* s = env("HDLA_HIP_SEGMENTS");
     if (!s) return true;
@@ -146,7 +149,7 @@ void chunk_dims(const ChunkIn& x, double scale, const Plan& p, hdla_dims& d) {
 void save_plan(AutogradContext* ctx, const Plan& p) { ctx->saved_data["plan"] = std::vector<int64_t>{p.route, p.segments, p.keep}; }
 Plan saved_plan(AutogradContext* ctx) {
     const auto p = ctx->saved_data["plan"].toIntVector();
-    return {(int32_t)p[0], (int32_t)p[1], false, p[2] != 0};
+    return {(int32_t)p[0], (int32_t)p[1], false, (Keep)p[2]};
 }
 
 // with_record: of a backward pass that is given the forward pass's record
@@ -212,13 +215,23 @@ void chunk_forward(const ChunkIn& x, const hdla_dims& d, bool want_ht, Plan* pla
     if (plan && plan->keep) {
         hdla_dims k = d;
         int32_t for_bwd = 0;
+        size_t ws_fwd = 0, ws_bwd = 0;                    // first the larger of the two buffers that it may be given
+        const size_t all = plan->record && !nb ? api.states_plan(&d, &ws_fwd, &ws_bwd) : 0;
+        if (all) left = kept_room(x.q, (int64_t)all);
+        if (left.defined()) {
+            plan->keep = KEEP_STATES;
+            const Tensor ws = bytes_like(x.q, ws_fwd);
+            check(api.chunk_fwd_states(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.beta), ptr(x.gk), fptr(x.h0), ptr(o), fptr(ht),
+                                       ptr(left), all, ptr(ws), ws_fwd, stream_of(x.q)), "hdla_chunk_fwd_states");
+            return;
+        }
         const size_t n = plan->record && !nb ? api.keep_plan(&d, &k.segments, &for_bwd) : 0;
         if (n) {                                          // one plan for the backward pass, kept or not
             plan->segments = for_bwd;
             if (for_bwd == 1) plan->route = HDLA_ROUTE_PLAIN;   // (one segment, also where a number asked for would be the fused route's)
             left = kept_room(x.q, (int64_t)n);
         }
-        plan->keep = left.defined();
+        plan->keep = left.defined() ? KEEP_FORWARD : KEEP_NOTHING;
         if (plan->keep) {
             check(api.chunk_fwd_keep(&k, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.beta), ptr(x.gk), fptr(x.h0), ptr(o), fptr(ht),
                                      ptr(left), n, stream_of(x.q)), "hdla_chunk_fwd_keep");
@@ -233,14 +246,21 @@ void chunk_forward(const ChunkIn& x, const hdla_dims& d, bool want_ht, Plan* pla
 
 struct ChunkGrads { Tensor q, k, v, a, b, beta, gk, h0; };      // of what is defined
 Tensor backward_workspace(const hdla_dims& d, const Plan& plan, const Tensor& like, const Tensor& left) {
+    if (plan.keep == KEEP_STATES) {
+        size_t fwd = 0, bwd = 0;
+        if (!api.states_plan(&d, &fwd, &bwd)) throw AbiError("hdla_states_plan: not the forward pass's dimensions");
+        return bytes_like(like, bwd);
+    }
     return plan.keep ? workspace(d, HDLA_PASS_BWD_KEPT, like) : workspace(d, HDLA_PASS_BWD, like, left.defined());
 }
 void chunk_backward(const ChunkIn& x, const hdla_dims& d, const Plan& plan, const Tensor& d_o, const Tensor& dht, const Tensor& left, const Tensor& ws,
                     const ChunkGrads& g) {
     if (plan.keep) {
-        check(api.chunk_bwd_kept(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.beta), ptr(x.gk), fptr(x.h0), ptr(d_o), fptr(dht),
-                                 ptr(g.q), ptr(g.k), ptr(g.v), ptr(g.a), ptr(g.b), ptr(g.beta), ptr(g.gk), fptr(g.h0), ptr(left),
-                                 (size_t)left.numel(), ptr(ws), (size_t)ws.numel(), stream_of(x.q)), "hdla_chunk_bwd_kept");
+        const bool states = plan.keep == KEEP_STATES;
+        check((states ? api.chunk_bwd_states : api.chunk_bwd_kept)(
+                  &d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.beta), ptr(x.gk), fptr(x.h0), ptr(d_o), fptr(dht),
+                  ptr(g.q), ptr(g.k), ptr(g.v), ptr(g.a), ptr(g.b), ptr(g.beta), ptr(g.gk), fptr(g.h0), ptr(left),
+                  (size_t)left.numel(), ptr(ws), (size_t)ws.numel(), stream_of(x.q)), states ? "hdla_chunk_bwd_states" : "hdla_chunk_bwd_kept");
         return;
     }
     check(api.chunk_bwd_b(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.beta), ptr(x.gk), fptr(x.h0), ptr(d_o), fptr(dht),
@@ -429,7 +449,7 @@ PyObject* run_chunk(ChunkIn& x, PyObject* pscale, PyObject* pwant, PyObject* pke
     else if (!number(pscale, scale)) return none();
     Plan plan;
     if (!read_plan(plan)) return none();
-    plan.keep = pkeep == Py_None && keep_forward_unsaid();
+    plan.keep = pkeep == Py_None && keep_forward_unsaid() ? KEEP_FORWARD : KEEP_NOTHING;
     return guarded([&]() -> PyObject* {
         hdla_dims d;
         chunk_dims(x, scale, plan, d);
@@ -1071,7 +1091,7 @@ PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (keep_forward_default() && grad) return none();
     Plan plan;
     if (!read_plan(plan)) return none();
-    plan.keep = keep_forward_unsaid();
+    plan.keep = keep_forward_unsaid() ? KEEP_FORWARD : KEEP_NOTHING;
     return guarded([&]() -> PyObject* {
         Tensor out, ht;
         if (grad) {
@@ -1159,7 +1179,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
         return nullptr;                                                                                            \
     }
     HDLA_FN(strerror) HDLA_FN(workspace_bytes) HDLA_FN(record_bytes) HDLA_FN(record_workspace_bytes) HDLA_FN(chunk_fwd_b) HDLA_FN(chunk_bwd_b)
-    HDLA_FN(keep_plan) HDLA_FN(chunk_fwd_keep) HDLA_FN(chunk_bwd_kept)
+    HDLA_FN(keep_plan) HDLA_FN(chunk_fwd_keep) HDLA_FN(chunk_bwd_kept) HDLA_FN(states_plan) HDLA_FN(chunk_fwd_states) HDLA_FN(chunk_bwd_states)
     HDLA_FN(recurrent_fwd) HDLA_FN(param_recurrent_fwd) HDLA_FN(normalize_fwd) HDLA_FN(normalize_bwd_as)
     HDLA_FN(normalize_workspace_bytes) HDLA_FN(layer_pre_fwd) HDLA_FN(layer_pre_bwd) HDLA_FN(layer_up_fwd) HDLA_FN(layer_down)
     HDLA_FN(layer_up_wgrad) HDLA_FN(layer_up_wgrad_workspace_bytes) HDLA_FN(rows_gemm) HDLA_FN(sum_partials) HDLA_FN(stack_rows) HDLA_FN(layer_step)

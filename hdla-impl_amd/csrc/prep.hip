@@ -243,8 +243,9 @@ constexpr int LDP = 36;   // padded row length of the 32x32 LDS matrices (keeps 
 
 // MODE: what the kernel leaves in the workspace -- PREP_FWD: what the forward pass's scan reads (which also forms the
 // output); PREP_BWD: what the two scans of the backward pass and the chunk_grad kernels read; PREP_KEEP: both, for a
-// forward pass whose workspace the backward pass will use instead of running this kernel again.
-enum PrepMode { PREP_FWD = 0, PREP_BWD = 1, PREP_KEEP = 2 };
+// forward pass whose workspace the backward pass will use instead of running this kernel again; PREP_STATES: the same beside the states that
+// enter the chunks, where what only the forward pass reads is in a place of its own.
+enum PrepMode { PREP_FWD = 0, PREP_BWD = 1, PREP_KEEP = 2, PREP_STATES = 3 };
 // Waves a SIMD: what the registers of a wave allow.  Three of 2-byte elements (with fp32 decays beside plain a, b: two): a tile's factors, operands
 // and gated copies are done with before the next one's begin, the copies that need nothing else leave at once, and (I - A_ab)^-1 lies where the
 // parts of the score tiles were (20 KB of LDS a workgroup of two waves instead of 37).  Three exponentials a tile instead of seven (TileDecay).
@@ -264,7 +265,9 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
     constexpr bool WRITE_U = sizeof(T) == 4 || GKF32;
     constexpr int NWP = K / 64;                       // waves per (chunk, head)
     constexpr int KTW = 4, VT = V / 16, VTW = VT / NWP, KT2 = K / 32;
-    constexpr int SAS = blk_fwd(K, sizeof(T), !BWD).SIZE / (int)sizeof(T);   // elements between (chunk, head) slots
+    constexpr bool APART = MODE == PREP_STATES;
+    constexpr int SAS = blk_fwd(K, sizeof(T), !BWD && !APART).SIZE / (int)sizeof(T);   // elements between (chunk, head) slots
+    constexpr int SQS = APART ? blk_q(K, sizeof(T)) / (int)sizeof(T) : SAS;            // and between those of q's tiles and A_qb
     constexpr int SBS = blk_bwd(K, sizeof(T)).SIZE / (int)sizeof(T);
     constexpr int NPART = BWD ? 8 : 9;                                    // score tiles that are summed over the waves
     // Per wave: A_ab, rank-major, and (I - A_ab)^-1.  A wave's matrices lie where the other wave's parts of the score tiles were, which it
@@ -472,7 +475,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
             if (SCAN_U) st_pair2(p.ws.BGT + chw * SAS + (2 * pair + s) * PAIR, bgT[0][s], bgT[1][s]);   // (s: the tile of the pair)
             else st_pair2(p.ws.BGT + chw * SAS + (s * KT2 + pair) * PAIR, bgT[s][0], bgT[s][1]);
         }
-        if (!BWD) st_pair2(p.ws.QG + chw * SAS + pair * PAIR, qg[0], qg[1]);
+        if (!BWD) st_pair2(p.ws.QG + chw * SQS + pair * PAIR, qg[0], qg[1]);
         if (WB) st_pair2(p.ws.QGT + chw * SBS + pair * PAIR, turn(qg[0], ident, scratch), turn(qg[1], ident, scratch));
     }
     // Each wave decides for its own channels (the parts of the score tiles add up whichever way they were formed); the
@@ -562,7 +565,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
     if (w == 0) {
         if (!BWD) {
             st_tile(p.ws.AQK + chw * SAS, to_frag<T>(aqk));
-            st_pair2(p.ws.AQB + chw * SAS, to_frag<T>(aqb[0]), to_frag<T>(aqb[1]));
+            st_pair2(p.ws.AQB + chw * SQS, to_frag<T>(aqb[0]), to_frag<T>(aqb[1]));
         }
         if (BWD || WB) {
             // the other orientation is the rounded tile turned (a product with the identity: exact), in every mode, so
@@ -705,15 +708,19 @@ static hipError_t launch_prep_kv(const ChunkArgs<T>& a, int mode, const FewTable
     dim3 grid(a.st.nch * a.H + makers), block(K);
     constexpr bool kAlwaysF32 = sizeof(T) == 4;
     const bool gkf32 = kAlwaysF32 || a.gk_f32;
+    constexpr int STATES = sizeof(T) == 2 ? PREP_STATES : PREP_KEEP;
+    if (sizeof(T) == 4 && mode == PREP_STATES) return hipErrorInvalidValue;
 #define HDLA_PREP_LAUNCH(GK, MODE) hipLaunchKernelGGL((prep_kernel<T, GK, K, V, MODE, HD>), grid, block, 0, stream, a, few)
     if (gkf32) {
         if (mode == PREP_FWD) HDLA_PREP_LAUNCH(true, PREP_FWD);
         else if (mode == PREP_BWD) HDLA_PREP_LAUNCH(true, PREP_BWD);
-        else HDLA_PREP_LAUNCH(true, PREP_KEEP);
+        else if (mode == PREP_KEEP) HDLA_PREP_LAUNCH(true, PREP_KEEP);
+        else HDLA_PREP_LAUNCH(true, STATES);
     } else {
         if (mode == PREP_FWD) HDLA_PREP_LAUNCH(kAlwaysF32, PREP_FWD);
         else if (mode == PREP_BWD) HDLA_PREP_LAUNCH(kAlwaysF32, PREP_BWD);
-        else HDLA_PREP_LAUNCH(kAlwaysF32, PREP_KEEP);
+        else if (mode == PREP_KEEP) HDLA_PREP_LAUNCH(kAlwaysF32, PREP_KEEP);
+        else HDLA_PREP_LAUNCH(kAlwaysF32, STATES);
     }
 #undef HDLA_PREP_LAUNCH
     return hipGetLastError();

@@ -25,7 +25,7 @@ hipError_t launch_scan_fwd(const ChunkArgs<T>& a, int K, int V, hipStream_t stre
     return launch_scan<T>(a, K, V, SCAN_FWD, stream);
 }
 template <typename T>
-hipError_t launch_scan_out(const ChunkArgs<T>& a, int K, int V, bool kept, hipStream_t stream) {
+hipError_t launch_scan_out(const ChunkArgs<T>& a, int K, int V, int kept, hipStream_t stream) {
     if constexpr (sizeof(T) == 2) {
         if (K == 64 && V == 64) return launch_scan_out_shape<64, 64>(a, kept, stream);
         if (K == 128 && V == 128) return launch_scan_out_shape<128, 128>(a, kept, stream);
@@ -63,8 +63,8 @@ template hipError_t launch_scan_segments<bf16>(const ChunkArgs<bf16>&, int, int,
 template hipError_t launch_scan_segments<float>(const ChunkArgs<float>&, int, int, SegStart, hipStream_t);
 template hipError_t launch_scan_fwd<bf16>(const ChunkArgs<bf16>&, int, int, hipStream_t);
 template hipError_t launch_scan_fwd<float>(const ChunkArgs<float>&, int, int, hipStream_t);
-template hipError_t launch_scan_out<bf16>(const ChunkArgs<bf16>&, int, int, bool, hipStream_t);
-template hipError_t launch_scan_out<float>(const ChunkArgs<float>&, int, int, bool, hipStream_t);
+template hipError_t launch_scan_out<bf16>(const ChunkArgs<bf16>&, int, int, int, hipStream_t);
+template hipError_t launch_scan_out<float>(const ChunkArgs<float>&, int, int, int, hipStream_t);
 template hipError_t launch_scan_bwd<bf16>(const ChunkArgs<bf16>&, int, int, hipStream_t);
 template hipError_t launch_scan_bwd<float>(const ChunkArgs<float>&, int, int, hipStream_t);
 template hipError_t launch_scan_pair<bf16>(const ChunkArgs<bf16>&, int, int, hipStream_t);

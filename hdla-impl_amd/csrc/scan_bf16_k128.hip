@@ -2,11 +2,11 @@
 #include "scan_grad.cuh"
 
 namespace hdla {
-template hipError_t launch_scan_out_shape<128, 64>(const ChunkArgs<bf16>&, bool, hipStream_t);
+template hipError_t launch_scan_out_shape<128, 64>(const ChunkArgs<bf16>&, int, hipStream_t);
 template hipError_t launch_scan_out_segments_shape<128, 64>(const ChunkArgs<bf16>&, hipStream_t);
 template hipError_t launch_scan_grad_shape<128, 64>(const ChunkArgs<bf16>&, ScanKind, hipStream_t);
 template hipError_t launch_scan_grad_segments_shape<128, 64>(const ChunkArgs<bf16>&, SegStart, hipStream_t);
-template hipError_t launch_scan_out_shape<128, 128>(const ChunkArgs<bf16>&, bool, hipStream_t);
+template hipError_t launch_scan_out_shape<128, 128>(const ChunkArgs<bf16>&, int, hipStream_t);
 template hipError_t launch_scan_out_segments_shape<128, 128>(const ChunkArgs<bf16>&, hipStream_t);
 template hipError_t launch_scan_grad_shape<128, 128>(const ChunkArgs<bf16>&, ScanKind, hipStream_t);
 template hipError_t launch_scan_grad_segments_shape<128, 128>(const ChunkArgs<bf16>&, SegStart, hipStream_t);

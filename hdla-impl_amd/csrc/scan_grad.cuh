@@ -318,7 +318,7 @@ __global__ __launch_bounds__((RevCfg<K, V, NWC, false>::THREADS)) void scan_grad
     __shared__ __attribute__((aligned(16))) char smem[grad_lds<K, V, NWC>()];
     const int z = blockIdx.z / p.seg.nseg, seg = blockIdx.z % p.seg.nseg;
     const int n = scan_sequence(p.st, z), y = blockIdx.y + first_dir * R::SPLIT;
-    if (y < R::SPLIT) scan_out_body<K, V, NWC, OUT_STATE, true>(p, smem, n, seg, y);
+    if (y < R::SPLIT) scan_out_body<K, V, NWC, OUT_STATE, 1>(p, smem, n, seg, y);
     else scan_rev_body<K, V, NWC, false>(p, smem, n, seg, y - R::SPLIT);
 }
 // packed sequences that share the device by their lengths, as scan_out_share_kernel; the two directions in turn
@@ -333,11 +333,23 @@ __global__ __launch_bounds__((RevCfg<K, V, 4, false>::THREADS)) void scan_grad_s
         constexpr int NWC = decltype(nwc)::value;
         if ((int)threadIdx.x >= RevCfg<K, V, NWC, false>::THREADS) return;
         if (rev) scan_rev_body<K, V, NWC, false>(p, smem, n, 0, split);
-        else scan_out_body<K, V, NWC, OUT_STATE, true>(p, smem, n, 0, split);
+        else scan_out_body<K, V, NWC, OUT_STATE, 1>(p, smem, n, 0, split);
     };
     if (code == 0) walk(std::integral_constant<int, 4>());
     else if (code == 1) walk(std::integral_constant<int, 2>());
     else walk(std::integral_constant<int, 1>());
+}
+// the reverse scan alone, behind a forward pass that has left the entering states: in the widths of that one's scan (a direction has as many slots).
+// us a training step, two blocks a workgroup for all -> this, 16 heads, K = V = 128: 16384 tokens in 4 sequences 1443 -> 1425, 9000 in 6, the longest 3700, 905 -> 855
+template <int K, int V>
+__global__ __launch_bounds__((RevCfg<K, V, 4, false>::THREADS)) void scan_rev_share_kernel(ChunkArgs<bf16> p) {
+    constexpr int B1 = RevCfg<K, V, 1, false>::BYTES, B2 = RevCfg<K, V, 2, false>::BYTES, B4 = RevCfg<K, V, 4, false>::BYTES;
+    __shared__ __attribute__((aligned(16))) char smem[B4 > B2 ? (B4 > B1 ? B4 : B1) : B2 > B1 ? B2 : B1];
+    int n, code, split;
+    if (!scan_share<V>(p.st, blockIdx.y, ORDER_OUT, n, code, split)) return;
+    if (code == 0) scan_rev_body<K, V, 4, false>(p, smem, n, 0, split);
+    else if (code == 1) { if ((int)threadIdx.x < RevCfg<K, V, 2, false>::THREADS) scan_rev_body<K, V, 2, false>(p, smem, n, 0, split); }
+    else if ((int)threadIdx.x < RevCfg<K, V, 1, false>::THREADS) scan_rev_body<K, V, 1, false>(p, smem, n, 0, split);
 }
 // the segments' records on a workspace of the backward pass (or that it will read): grid and first_y as scan_sum_kernel's
 template <int K, int V, int NWC>
@@ -351,7 +363,7 @@ __global__ __launch_bounds__((RevCfg<K, V, NWC, true>::THREADS)) void scan_grad_
     const int n = scan_sequence(p.st, z), y = blockIdx.y + first_y, split = y % COLS;
     if (y < COLS) {
         if (seg == 0 && split >= R::SPLIT) return;        // starts from h0: nobody asks for its transition
-        scan_out_body<K, V, NWC, OUT_SUM, true>(p, smem, n, seg, split);
+        scan_out_body<K, V, NWC, OUT_SUM, 1>(p, smem, n, seg, split);
     } else {
         if (seg + 1 == p.seg.nseg - 1 && split >= R::SPLIT) return;
         scan_rev_body<K, V, NWC, true>(p, smem, n, seg + 1, split);
@@ -373,6 +385,10 @@ template <int K, int V> hipError_t launch_scan_grad_shape(const ChunkArgs<bf16>&
     if (kind == SCAN_PAIR && scan_shares(a.st.cu, a.st.N, a.H, V, a.seg.nseg, 2)) {
         hipLaunchKernelGGL((scan_grad_share_kernel<K, V>), dim3(a.H, 2 * share_most(a.H, 2, a.st.N, V)), dim3(RevCfg<K, V, 4, false>::THREADS), 0,
                            stream, a);
+        return hipGetLastError();
+    }
+    if (kind == SCAN_BWD && scan_shares(a.st.cu, a.st.N, a.H, V, a.seg.nseg, 1)) {
+        hipLaunchKernelGGL((scan_rev_share_kernel<K, V>), dim3(a.H, share_most(a.H, 1, a.st.N, V)), dim3(RevCfg<K, V, 4, false>::THREADS), 0, stream, a);
         return hipGetLastError();
     }
     if (lanes * (VT / 2) <= SCAN_TARGET_WORKGROUPS) return launch_scan_grad_nwc<K, V, 2>(a, kind, stream);

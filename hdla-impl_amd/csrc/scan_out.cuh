@@ -64,12 +64,13 @@ template <typename C> __device__ __forceinline__ int forming_first(int wave) { r
 // records of segments.
 // KEPT: on a workspace of the backward pass (or that it will read, PREP_KEEP): (I - A_ab)^-1 is there turned, as chunk_grad takes it, A_ak in a place of its
 // own, and b^T's pairs are of two channel tiles, as the reverse scan takes them.  The same products in the same order: the same bits.
-template <int K, int V, int NWC, ScanOut OUT, bool KEPT>
+// KEPT 2 (PREP_STATES): the states that enter the chunks are left for the backward pass, and q's part of the block is not the kept buffer's.
+template <int K, int V, int NWC, ScanOut OUT, int KEPT>
 __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* smem, int n, int seg, int split) {
     typedef OutCfg<K, V, NWC, OUT> C;
     typedef bf16 T;
     constexpr bool WITH_O = OUT == OUT_O, SUM = OUT == OUT_SUM;
-    constexpr bool FWD = WITH_O && !KEPT;                 // a forward pass that keeps nothing (see forming_first)
+    constexpr bool FWD = WITH_O && !KEPT, STATES = KEPT == 2;   // a forward pass that keeps nothing (see forming_first)
     constexpr int KT = C::KT, KT2 = KT / 2, SLOTS = C::SLOTS, SLOT = C::SLOT, PARTS = C::PARTS, KH = C::KH, KH2 = KH / 2;
     constexpr BlkF B = C::B;
     const int h = blockIdx.x;
@@ -96,14 +97,18 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
         if (hw < C::NL) {
             const int stride = KEPT ? p.ws.sa_stride : B.SIZE;
             const char* const blk = reinterpret_cast<const char*>(p.ws.W) + chw0 * stride + l * 16;
+            constexpr int PRE = STATES ? blk_fwd(K, 2, false).SIZE / 1024 : C::NI, STRIDE_Q = blk_q(K, 2);
+            const char* const blk_of_q = reinterpret_cast<const char*>(p.ws.QG) + chw0 * STRIDE_Q + l * 16;
             int slot = 0;
             auto load = [&](int t) __attribute__((always_inline)) {
                 // past the end: the last chunk again, never looked at
                 const char* const bt = blk + (int64_t)min(t, last) * stride;
+                const char* const qt = blk_of_q + (int64_t)min(t, last) * STRIDE_Q;
 #pragma unroll
                 for (int j = 0; j < C::CNT; ++j) {
                     const int i = min(hw + j * C::NL, C::NI - 1);
-                    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(bt + i * 1024),
+                    const char* const src = !STATES || i < PRE ? bt + i * 1024 : qt + (i - PRE) * 1024;
+                    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
                                                      (__attribute__((address_space(3))) void*)(smem + slot * SLOT + i * 1024), 16, 0, 0);
                 }
                 slot = slot + 1 == SLOTS ? 0 : slot + 1;
@@ -327,7 +332,7 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
 #pragma unroll
                 for (int kp = 0; kp < KH2; ++kp) o = mm2(qg[2 * kp], qg[2 * kp + 1], sb[2 * kp], sb[2 * kp + 1], o);
             }
-            if constexpr (OUT == OUT_STATE) {
+            if constexpr (OUT == OUT_STATE || STATES) {
                 // checkpoint of the entering state, as the fragments held here (tile pairs, 16 bytes per lane, whole cache lines): the
                 // chunk_grad kernel turns them the way it needs them
                 T* const hc = p.ws.HC + (chw0 + t) * (K * V) + (part * KH2 * (V / 16) + vt) * PAIR;
@@ -410,7 +415,7 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
 }
 
 // grid = (H, SPLIT, N * segments), as the other scans' (scan_impl.cuh)
-template <int K, int V, int NWC, bool KEPT>
+template <int K, int V, int NWC, int KEPT>
 __global__ __launch_bounds__((OutCfg<K, V, NWC, OUT_O>::THREADS)) void scan_out_kernel(ChunkArgs<bf16> p) {
     __shared__ __attribute__((aligned(16))) char smem[OutCfg<K, V, NWC, OUT_O>::BYTES];
     const int z = blockIdx.z / p.seg.nseg, seg = blockIdx.z % p.seg.nseg;
@@ -422,7 +427,7 @@ __global__ __launch_bounds__((OutCfg<K, V, NWC, OUT_O>::THREADS)) void scan_out_
 // similar lengths 137.7 -> 138.0; 12000 in 12, 8 heads 209 -> 186; training steps of 6000 in 6 748 -> 683, of 1500 in 7, 12 heads 174 -> 153, of
 // 16384 in 4 1726 -> 1705 (its two scans are at their traffic, 2.2 GB in 520 us, in every width).  Where one block a workgroup for all fits the device,
 // that is faster still and stays.  Beyond 32 sequences the device is full with the widest workgroups for all but the last few steps.
-template <int K, int V, bool KEPT>
+template <int K, int V, int KEPT>
 __global__ __launch_bounds__((OutCfg<K, V, 4, OUT_O>::THREADS)) void scan_out_share_kernel(ChunkArgs<bf16> p) {
     typedef OutCfg<K, V, 4, OUT_O> C4;
     typedef OutCfg<K, V, 2, OUT_O> C2;
@@ -440,28 +445,30 @@ __global__ __launch_bounds__((OutCfg<K, V, NWC, OUT_SUM>::THREADS)) void scan_ou
     __shared__ __attribute__((aligned(16))) char smem[OutCfg<K, V, NWC, OUT_SUM>::BYTES];
     const int z = blockIdx.z / (p.seg.nseg - 1), seg = blockIdx.z % (p.seg.nseg - 1);
     if (seg == 0 && (int)blockIdx.y >= OutCfg<K, V, NWC, OUT_SUM>::SPLIT) return;   // starts from h0: nobody asks for its transition
-    scan_out_body<K, V, NWC, OUT_SUM, false>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
+    scan_out_body<K, V, NWC, OUT_SUM, 0>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
 }
 
-template <int K, int V, int NWC> static hipError_t launch_scan_out_nwc(const ChunkArgs<bf16>& a, bool kept, hipStream_t stream) {
+template <int K, int V, int NWC> static hipError_t launch_scan_out_nwc(const ChunkArgs<bf16>& a, int kept, hipStream_t stream) {
     typedef OutCfg<K, V, NWC, OUT_O> C;
     const dim3 grid(a.H, C::SPLIT, a.st.N * a.seg.nseg), block(C::THREADS);
-    if (kept) hipLaunchKernelGGL((scan_out_kernel<K, V, NWC, true>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((scan_out_kernel<K, V, NWC, false>), grid, block, 0, stream, a);
+    if (kept == 2) hipLaunchKernelGGL((scan_out_kernel<K, V, NWC, 2>), grid, block, 0, stream, a);
+    else if (kept) hipLaunchKernelGGL((scan_out_kernel<K, V, NWC, 1>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((scan_out_kernel<K, V, NWC, 0>), grid, block, 0, stream, a);
     return hipGetLastError();
 }
 // Column blocks a workgroup: as few as give each workgroup a compute unit of its own (every workgroup fetches the chunks' blocks for
 // itself).  A forward pass, us, two blocks and one, 128 chunks in one segment: K = V = 128, 1 lane 82 and 73, 16 lanes 102 and 96, 32 lanes 135 and
 // 127; K = 64, V = 128, 8 lanes 71 and 59, 32 lanes 88 and 79; of 16 chunks K = V = 128 22.3 and 20.8.  The scan alone, two and four: K = V = 128,
 // 128 heads 193 and 146, 64 heads 101 and 114.
-template <int K, int V> hipError_t launch_scan_out_shape(const ChunkArgs<bf16>& a, bool kept, hipStream_t stream) {
+template <int K, int V> hipError_t launch_scan_out_shape(const ChunkArgs<bf16>& a, int kept, hipStream_t stream) {
     constexpr int VT = V / 16;
     const int lanes = a.H * a.st.N * a.seg.nseg;
     if (lanes * VT <= SCAN_TARGET_WORKGROUPS) return launch_scan_out_nwc<K, V, 1>(a, kept, stream);
     if (scan_shares(a.st.cu, a.st.N, a.H, V, a.seg.nseg, 1)) {
         const dim3 grid(a.H, share_most(a.H, 1, a.st.N, V)), block(OutCfg<K, V, 4, OUT_O>::THREADS);
-        if (kept) hipLaunchKernelGGL((scan_out_share_kernel<K, V, true>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((scan_out_share_kernel<K, V, false>), grid, block, 0, stream, a);
+        if (kept == 2) hipLaunchKernelGGL((scan_out_share_kernel<K, V, 2>), grid, block, 0, stream, a);
+        else if (kept) hipLaunchKernelGGL((scan_out_share_kernel<K, V, 1>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((scan_out_share_kernel<K, V, 0>), grid, block, 0, stream, a);
         return hipGetLastError();
     }
     if (lanes * (VT / 2) <= SCAN_TARGET_WORKGROUPS) return launch_scan_out_nwc<K, V, 2>(a, kept, stream);

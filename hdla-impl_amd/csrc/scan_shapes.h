@@ -9,7 +9,7 @@ enum ScanKind { SCAN_FWD_O, SCAN_FWD, SCAN_BWD, SCAN_PAIR };   // forward scan w
 
 template <typename T, int K, int V> hipError_t launch_scan_shape(const ChunkArgs<T>& a, ScanKind kind, hipStream_t stream);
 // the forward pass's scan for 2-byte elements, and its segments' records and entering states (scan_out.cuh)
-template <int K, int V> hipError_t launch_scan_out_shape(const ChunkArgs<bf16>& a, bool kept, hipStream_t stream);
+template <int K, int V> hipError_t launch_scan_out_shape(const ChunkArgs<bf16>& a, int kept, hipStream_t stream);
 template <int K, int V> hipError_t launch_scan_out_segments_shape(const ChunkArgs<bf16>& a, hipStream_t stream);   // SEG_FWD
 // the scans of the backward pass for 2-byte elements, and their segments' (scan_grad.cuh)
 template <int K, int V> hipError_t launch_scan_grad_shape(const ChunkArgs<bf16>& a, ScanKind kind, hipStream_t stream);
