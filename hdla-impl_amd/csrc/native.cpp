@@ -48,6 +48,7 @@ struct Api {
 #define HDLA_FN(name) decltype(&hdla_##name) name
     HDLA_FN(strerror); HDLA_FN(workspace_bytes); HDLA_FN(record_bytes); HDLA_FN(record_workspace_bytes); HDLA_FN(chunk_fwd_b); HDLA_FN(chunk_bwd_b);
     HDLA_FN(keep_plan); HDLA_FN(chunk_fwd_keep); HDLA_FN(chunk_bwd_kept); HDLA_FN(states_plan); HDLA_FN(chunk_fwd_states); HDLA_FN(chunk_bwd_states);
+    HDLA_FN(tile_gemm);
     HDLA_FN(recurrent_fwd); HDLA_FN(param_recurrent_fwd); HDLA_FN(normalize_fwd); HDLA_FN(normalize_bwd_as);
     HDLA_FN(normalize_workspace_bytes); HDLA_FN(layer_pre_fwd); HDLA_FN(layer_pre_bwd); HDLA_FN(layer_up_fwd); HDLA_FN(layer_down);
     HDLA_FN(layer_up_wgrad); HDLA_FN(layer_up_wgrad_workspace_bytes); HDLA_FN(rows_gemm); HDLA_FN(sum_partials); HDLA_FN(stack_rows);
@@ -682,6 +683,17 @@ hdla_up_dims up_dims(const LayerCols& L, int64_t rows) {
     u.rows = rows; u.d = (int32_t)L.d; u.D = (int32_t)L.D; u.ld = L.ld; u.col_f = (int32_t)L.f0; u.col_g = (int32_t)L.g0;
     return u;
 }
+// Products of some hundred rows by hdla_tile_gemm: what is one round of its workgroups on the device (figures there).  us a call, BLAS -> this: a decode step
+// of 100 sequences, 1024 channels 58 -> 37, of 256, 512 57 -> 30; training steps, bound by the host, 4 x 121 tokens, 256 channels 334 -> 261, 1 x 512, 1024 333 -> 285,
+// 4 x 1000, 512 320 -> 317; 2 x 1024, 2048 channels, one product of four, 579 -> 565.
+Tensor tile_gemm(const Tensor& x, const Tensor& w, bool turned) {
+    const int64_t M = x.size(0), K = x.size(1), N = w.size(turned ? 1 : 0);
+    if ((M + 63) / 64 * ((N + 63) / 64) > 256 || K < 8 || K % 8 || N < 8 || N % (turned ? 64 : 8) || x.stride(1) != 1 || w.stride(1) != 1 || x.stride(0) % 8 ||
+        w.stride(0) % 8 || x.stride(0) < K || w.stride(0) < w.size(1) || off_grid(x) || off_grid(w)) return at::mm(x, turned ? w : w.t());
+    const Tensor y = at::empty({M, N}, x.options());
+    check(api.tile_gemm((int32_t)M, (int32_t)N, (int32_t)K, ptr(x), x.stride(0), ptr(w), w.stride(0), turned, ptr(y), N, stream_of(x)), "hdla_tile_gemm");
+    return y;
+}
 // x w^T.  For the few rows of a decode step by hdla_rows_gemm, which is a launch where the BLAS call is 19 us of host time.
 // GPU time alone (us, here / there, weights from HBM): 16 x 6416 x 2048 9.0/13.0,
 // 64 x 6416 x 2048 12.1/13.5, 64 x 4096 x 4096 14.6/15.0, 16 x 12576 x 4096 24.4/27.0; with more than 16 rows of x, which every
@@ -689,7 +701,8 @@ hdla_up_dims up_dims(const LayerCols& L, int64_t rows) {
 constexpr int64_t FEW_ROWS = 64;
 Tensor project(const Tensor& x, const Tensor& w) {
     const int64_t M = x.size(0), most = (M <= 16 ? int64_t(64) : int64_t(16)) << 20;
-    if (M > FEW_ROWS || w.numel() > most) return at::mm(x, w.t());
+    if (M > FEW_ROWS) return tile_gemm(x, w, false);
+    if (w.numel() > most) return at::mm(x, w.t());
     const Tensor y = at::empty({x.size(0), w.size(0)}, x.options());
     check(api.rows_gemm((int32_t)x.size(0), (int32_t)w.size(0), (int32_t)w.size(1), ptr(x), x.stride(0), ptr(w), w.stride(0), ptr(y), y.stride(0),
                         stream_of(x)), "hdla_rows_gemm");
@@ -901,7 +914,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
         const Tensor dout = grads[0].defined() ? grads[0].to(at::kBFloat16).contiguous().view({rows, d}) : at::zeros({rows, d}, opt);
         const bool projections = need(1) || need(2) || need(3) || need(4) || need(5) || need(6);
         if (need(10) && !projections) out[10] = weight_grad(dout, n);     // (else with theirs)
-        const Tensor dn = at::mm(dout, wo);
+        const Tensor dn = tile_gemm(dout, wo, true);
         const Tensor o2 = o.view({rows, d}), d_o = at::empty({rows, d}, opt), dgate = at::empty({rows, d}, opt);
         const Tensor dwn = at::empty(wnorm.sizes(), wnorm.options());
         {
@@ -957,7 +970,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
             for (int i = 0; i < 6; ++i) out[1 + i] = dw.narrow(0, at_row[i], at_row[i + 1] - at_row[i]);
         }
         check(api.run_sums(sums.of, 4, stream), "hdla_run_sums");
-        if (need(0)) out[0] = at::mm(dy, w).view({B, T, d});
+        if (need(0)) out[0] = tile_gemm(dy, w, true).view({B, T, d});
         return out;
     }
 };
@@ -1179,7 +1192,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
         return nullptr;                                                                                            \
     }
     HDLA_FN(strerror) HDLA_FN(workspace_bytes) HDLA_FN(record_bytes) HDLA_FN(record_workspace_bytes) HDLA_FN(chunk_fwd_b) HDLA_FN(chunk_bwd_b)
-    HDLA_FN(keep_plan) HDLA_FN(chunk_fwd_keep) HDLA_FN(chunk_bwd_kept) HDLA_FN(states_plan) HDLA_FN(chunk_fwd_states) HDLA_FN(chunk_bwd_states)
+    HDLA_FN(keep_plan) HDLA_FN(chunk_fwd_keep) HDLA_FN(chunk_bwd_kept) HDLA_FN(states_plan) HDLA_FN(chunk_fwd_states) HDLA_FN(chunk_bwd_states) HDLA_FN(tile_gemm)
     HDLA_FN(recurrent_fwd) HDLA_FN(param_recurrent_fwd) HDLA_FN(normalize_fwd) HDLA_FN(normalize_bwd_as)
     HDLA_FN(normalize_workspace_bytes) HDLA_FN(layer_pre_fwd) HDLA_FN(layer_pre_bwd) HDLA_FN(layer_up_fwd) HDLA_FN(layer_down)
     HDLA_FN(layer_up_wgrad) HDLA_FN(layer_up_wgrad_workspace_bytes) HDLA_FN(rows_gemm) HDLA_FN(sum_partials) HDLA_FN(stack_rows) HDLA_FN(layer_step)
