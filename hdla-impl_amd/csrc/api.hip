@@ -184,8 +184,8 @@ int kept_plan_segments(const hdla_dims* d, int32_t& bwd) {
 constexpr size_t STATES_MOST = (size_t)1 << 30;
 constexpr long long SCAN_PAIR_WORKGROUPS = 256;               // one a compute unit (launch_scan_grad_shape)
 bool leaves_states(const hdla_dims* d) {
-    if (d->in_dtype != HDLA_BF16 || d->route != HDLA_ROUTE_AUTO || d->segments > 1 || scan_segments(d, false) > 1 || scan_segments(d, true) > 1) return false;
-    return 2LL * d->N * d->H * (d->V / 16) > SCAN_PAIR_WORKGROUPS;
+    if (2LL * d->N * d->H * (d->V / 16) <= SCAN_PAIR_WORKGROUPS || d->in_dtype != HDLA_BF16 || d->route != HDLA_ROUTE_AUTO || d->segments > 1) return false;
+    return scan_segments(d, false) == 1 && scan_segments(d, true) == 1;
 }
 
 struct FusedLayout {
@@ -697,11 +697,11 @@ size_t hdla_keep_plan(const hdla_dims* dims, int32_t* fwd_segments, int32_t* bwd
 
 size_t hdla_states_plan(const hdla_dims* dims, size_t* fwd_workspace, size_t* bwd_workspace) {
     bool fused_fwd, fused_bwd;
-    if (!fwd_workspace || !bwd_workspace || check_dims(dims) || dims->T < 1) return 0;
+    if (!fwd_workspace || !bwd_workspace || check_dims(dims) || dims->T < 1 || !leaves_states(dims)) return 0;
     if (pick_route(dims, HDLA_PASS_FWD, false, fused_fwd) || pick_route(dims, HDLA_PASS_BWD, false, fused_bwd) || fused_fwd || fused_bwd) return 0;
     WsLayout L, S;
     int nch;
-    if (!leaves_states(dims) || make_layout(dims, PASS_FWD_STATES, L, nch) || L.total > STATES_MOST || make_layout(dims, PASS_BWD_STATES, S, nch)) return 0;
+    if (make_layout(dims, PASS_FWD_STATES, L, nch) || L.total > STATES_MOST || make_layout(dims, PASS_BWD_STATES, S, nch)) return 0;
     *fwd_workspace = states_fwd_workspace(dims, nch);
     *bwd_workspace = S.total;
     return L.total;

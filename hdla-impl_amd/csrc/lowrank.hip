@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256) void layer_down_kernel(DownArgs p) {
     }
 }
 
-// y [M, N] = x [M, K] W [N, K]^T, M <= 16 MT.  A workgroup per 16 RT rows of W; its eight waves take an eighth of K each and
+// y [M, N] = x [M, K] W [N, K]^T, M <= 16 MT.  A workgroup per 16 RT rows of W; its RW waves (eight) take as many parts of K and
 // add up through LDS.
 //
 // What bounds it is the path from memory into the compute unit, and on that the order of the lanes: a fragment's lane order
@@ -241,7 +241,7 @@ __global__ __launch_bounds__(256) void layer_down_kernel(DownArgs p) {
 // 11.0 -> 5.6, 13.8 -> 8.3; 16 x 512 x 512, one launch's time, 2.65 -> 2.3.  (The 26 MB of the first at copy rate: 5.4.)
 // UNR: a wave's whole share of K up to 2048 (16 rows) in one or two goes; twice as many is no faster (16 x 6416 x 2048 5.0,
 // 64 x 6416 x 2048 7.6 -> 8.7) and asks twice for K = 512 what is there once (1 -> 2 blocks a wave too many, 2.5 -> 3.0 for 32 rows).
-constexpr int RW = 8;                                     // waves
+constexpr int ROW_WAVES = 8;
 // NORM (one row tile): x is formed on the way in, x = gated c / sqrt(K) / sqrt(sum of the row's parts / K + eps) weight, rounded to bf16
 // as the norm's output is: one launch less, and no pass over a few rows that is all latency (16 x 2048 x 2048: norm 4.1 and product 4.4
 // -> 7.6 us).
@@ -251,7 +251,7 @@ struct NormIn {
     int parts, w_f32;
     float cn, inv_e, eps;
 };
-template <int MT, int RT, int UNR, bool NORM>
+template <int MT, int RT, int UNR, bool NORM, int RW = 8>
 __global__ __launch_bounds__(64 * RW) void rows_gemm_kernel(const bf16* __restrict__ x, long long ldx, const bf16* __restrict__ w, long long ldw,
                                                             bf16* __restrict__ y, long long ldy, int M, int N, int K, NormIn nrm) {
     static_assert(!NORM || MT == 1, "one row tile");
@@ -501,12 +501,12 @@ extern "C" int hdla_rows_gemm(int32_t M, int32_t N, int32_t K, const void* x, in
     // one tile each is more than a workgroup a compute unit.  One tile / two, weights in the last-level cache, us: K = 2048, 64 rows,
     // 4096 columns 6.5 / 7.3, 5120 9.2 / 7.4, 6416 9.4 / 7.5; 32 rows 4.4 / 5.9, 6.6 / 6.1, 6.5 / 6.25.
     const bool two = M > 16 && N > 16 * 256;
-    const dim3 grid((N + (two ? 31 : 15)) / (two ? 32 : 16)), block(64 * RW);
+    const dim3 grid((N + (two ? 31 : 15)) / (two ? 32 : 16)), block(64 * ROW_WAVES);
 #define HDLA_ROWS(MT, RT, UNR) \
     hipLaunchKernelGGL((rows_gemm_kernel<MT, RT, UNR, false>), grid, block, 0, s, xp, (long long)ldx, wp, (long long)ldw, yp, (long long)ldy, M, N, K, NormIn{})
-    if (M <= 16 && K <= 64 * RW) HDLA_ROWS(1, 1, 2);
+    if (M <= 16 && K <= 64 * ROW_WAVES) HDLA_ROWS(1, 1, 2);
     else if (M <= 16) HDLA_ROWS(1, 1, 4);
-    else if (M <= 32 && !two && K <= 64 * RW) HDLA_ROWS(2, 1, 2);
+    else if (M <= 32 && !two && K <= 64 * ROW_WAVES) HDLA_ROWS(2, 1, 2);
     else if (M <= 32 && !two) HDLA_ROWS(2, 1, 4);
     else if (M <= 32) HDLA_ROWS(2, 2, 4);
     else if (!two) HDLA_ROWS(4, 1, 2);
@@ -525,13 +525,18 @@ extern "C" int hdla_rows_gemm_norm(int32_t M, int32_t N, int32_t K, const float*
     if (!gated || !w || !y) return HDLA_ERR_NULL;
     if (!lr_al(gated, 16) || !lr_al(weight, 16) || !lr_al(w, 16) || !lr_al(y, 8) || ldw % 8 || ldy % 4) return HDLA_ERR_ALIGN;
     const NormIn nrm{gated, gated + (int64_t)M * K, weight, parts, norm->weight_dtype == HDLA_FP32, norm->c / sqrtf((float)K), 1.f / (float)K, norm->eps};
-    const dim3 grid((N + 15) / 16), block(64 * RW);
+    const dim3 grid((N + 15) / 16);
     const hipStream_t s = static_cast<hipStream_t>(stream);
     const bf16* wp = static_cast<const bf16*>(w);
     bf16* yp = static_cast<bf16*>(y);
-    if (K <= 64 * RW)
-        hipLaunchKernelGGL((rows_gemm_kernel<1, 1, 2, true>), grid, block, 0, s, nullptr, 0LL, wp, (long long)ldw, yp, (long long)ldy, M, N, K, nrm);
-    else
-        hipLaunchKernelGGL((rows_gemm_kernel<1, 1, 4, true>), grid, block, 0, s, nullptr, 0LL, wp, (long long)ldw, yp, (long long)ldy, M, N, K, nrm);
+    // Waves and blocks a go as ask for all of K at once, as far as the registers reach: sixteen waves for K = 2048, where eight asked twice.  us a decode step of
+    // the layer, as a graph's replay, eight / sixteen: 16 sequences, 2048 channels 24.4 / 23.4, 4 21.4 / 20.5, 1 20.9 / 19.8; 16, 1024 channels, whose K eight have in one
+    // go, 13.9 / 14.6.
+#define HDLA_ROWS(UNR, WAVES)                                                                                                                       \
+    hipLaunchKernelGGL((rows_gemm_kernel<1, 1, UNR, true, WAVES>), grid, dim3(64 * WAVES), 0, s, nullptr, 0LL, wp, (long long)ldw, yp, (long long)ldy, M, N, K, nrm)
+    if (K <= 64 * ROW_WAVES) HDLA_ROWS(2, ROW_WAVES);
+    else if (K <= 128 * ROW_WAVES) HDLA_ROWS(4, ROW_WAVES);
+    else HDLA_ROWS(4, 16);
+#undef HDLA_ROWS
     return (int)hipGetLastError();
 }
