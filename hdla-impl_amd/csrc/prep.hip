@@ -263,6 +263,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
     // caller has named the classic route, whose buffers can be looked at (UT is given).  This mode at K = V = 128, 16384 tokens of 16 heads, us: 221 -> 178,
     // for 12 KB not written and v not read of 85 a chunk and head.
     constexpr bool WRITE_U = sizeof(T) == 4 || GKF32;
+    constexpr bool KG_IS_B = HD && sizeof(T) == 2;    // kg^T is bg_2^T, which the scans of 2-byte elements know (OutCfg)
     constexpr int NWP = K / 64;                       // waves per (chunk, head)
     constexpr int KTW = 4, VT = V / 16, VTW = VT / NWP, KT2 = K / 32;
     constexpr bool APART = MODE == PREP_STATES;
@@ -430,7 +431,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
             const TileDecay<T> d(in[e].g, c);
             strong |= d.strong;
             qg[e] = to_frag<T>(to_f32(in[e].q) * d.egi * scale);
-            kgT[e] = turn(to_frag<T>(to_f32(in[e].k) * d.edn), ident, scratch);
+            if (!KG_IS_B) kgT[e] = turn(to_frag<T>(to_f32(in[e].k) * d.edn), ident, scratch);
 #pragma unroll
             for (int r = 0; r < 2; ++r) {
                 ag[r][kt] = to_frag<T>(to_f32(in[e].a[r]) * d.ege);
@@ -469,7 +470,7 @@ __global__ __launch_bounds__(K) __attribute__((amdgpu_waves_per_eu(prep_waves<T,
             if (TIGHT) __builtin_amdgcn_sched_barrier(0);
         }
         const int pair = kt0 / 2 + kp;
-        st_pair2(p.ws.KGT + chw * SAS + pair * PAIR, kgT[0], kgT[1]);
+        if (!KG_IS_B) st_pair2(p.ws.KGT + chw * SAS + pair * PAIR, kgT[0], kgT[1]);
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             if (SCAN_U) st_pair2(p.ws.BGT + chw * SAS + (2 * pair + s) * PAIR, bgT[0][s], bgT[1][s]);   // (s: the tile of the pair)

@@ -305,26 +305,26 @@ __device__ __forceinline__ void scan_rev_body(const ChunkArgs<bf16>& p, char* sm
     }
 }
 
-template <int K, int V, int NWC> constexpr int grad_lds() {
-    return OutCfg<K, V, NWC, OUT_STATE>::BYTES > RevCfg<K, V, NWC, false>::BYTES ? OutCfg<K, V, NWC, OUT_STATE>::BYTES : RevCfg<K, V, NWC, false>::BYTES;
+template <int K, int V, int NWC, bool HD> constexpr int grad_lds() {
+    return OutCfg<K, V, NWC, OUT_STATE, HD>::BYTES > RevCfg<K, V, NWC, false>::BYTES ? OutCfg<K, V, NWC, OUT_STATE, HD>::BYTES : RevCfg<K, V, NWC, false>::BYTES;
 }
 // grid = (H, directions * SPLIT, N * segments), as scan_impl.cuh's; blockIdx.y counts from the forward scan's splits on, or (first_dir 1) from
 // the reverse one's
-template <int K, int V, int NWC>
+template <int K, int V, int NWC, bool HD>
 __global__ __launch_bounds__((RevCfg<K, V, NWC, false>::THREADS)) void scan_grad_kernel(ChunkArgs<bf16> p, int first_dir) {
-    typedef OutCfg<K, V, NWC, OUT_STATE> F;
+    typedef OutCfg<K, V, NWC, OUT_STATE, HD> F;
     typedef RevCfg<K, V, NWC, false> R;
     static_assert(F::THREADS == R::THREADS, "one launch");
-    __shared__ __attribute__((aligned(16))) char smem[grad_lds<K, V, NWC>()];
+    __shared__ __attribute__((aligned(16))) char smem[grad_lds<K, V, NWC, HD>()];
     const int z = blockIdx.z / p.seg.nseg, seg = blockIdx.z % p.seg.nseg;
     const int n = scan_sequence(p.st, z), y = blockIdx.y + first_dir * R::SPLIT;
-    if (y < R::SPLIT) scan_out_body<K, V, NWC, OUT_STATE, 1>(p, smem, n, seg, y);
+    if (y < R::SPLIT) scan_out_body<K, V, NWC, OUT_STATE, 1, HD>(p, smem, n, seg, y);
     else scan_rev_body<K, V, NWC, false>(p, smem, n, seg, y - R::SPLIT);
 }
 // packed sequences that share the device by their lengths, as scan_out_share_kernel; the two directions in turn
-template <int K, int V>
+template <int K, int V, bool HD>
 __global__ __launch_bounds__((RevCfg<K, V, 4, false>::THREADS)) void scan_grad_share_kernel(ChunkArgs<bf16> p) {
-    constexpr int B1 = grad_lds<K, V, 1>(), B2 = grad_lds<K, V, 2>(), B4 = grad_lds<K, V, 4>();
+    constexpr int B1 = grad_lds<K, V, 1, HD>(), B2 = grad_lds<K, V, 2, HD>(), B4 = grad_lds<K, V, 4, HD>();
     __shared__ __attribute__((aligned(16))) char smem[B4 > B2 ? (B4 > B1 ? B4 : B1) : B2 > B1 ? B2 : B1];
     int n, code, split;
     if (!scan_share<V>(p.st, blockIdx.y >> 1, ORDER_GRAD, n, code, split)) return;
@@ -333,7 +333,7 @@ __global__ __launch_bounds__((RevCfg<K, V, 4, false>::THREADS)) void scan_grad_s
         constexpr int NWC = decltype(nwc)::value;
         if ((int)threadIdx.x >= RevCfg<K, V, NWC, false>::THREADS) return;
         if (rev) scan_rev_body<K, V, NWC, false>(p, smem, n, 0, split);
-        else scan_out_body<K, V, NWC, OUT_STATE, 1>(p, smem, n, 0, split);
+        else scan_out_body<K, V, NWC, OUT_STATE, 1, HD>(p, smem, n, 0, split);
     };
     if (code == 0) walk(std::integral_constant<int, 4>());
     else if (code == 1) walk(std::integral_constant<int, 2>());
@@ -352,9 +352,9 @@ __global__ __launch_bounds__((RevCfg<K, V, 4, false>::THREADS)) void scan_rev_sh
     else if ((int)threadIdx.x < RevCfg<K, V, 1, false>::THREADS) scan_rev_body<K, V, 1, false>(p, smem, n, 0, split);
 }
 // the segments' records on a workspace of the backward pass (or that it will read): grid and first_y as scan_sum_kernel's
-template <int K, int V, int NWC>
+template <int K, int V, int NWC, bool HD>
 __global__ __launch_bounds__((RevCfg<K, V, NWC, true>::THREADS)) void scan_grad_sum_kernel(ChunkArgs<bf16> p, int first_y) {
-    typedef OutCfg<K, V, NWC, OUT_SUM> F;
+    typedef OutCfg<K, V, NWC, OUT_SUM, HD> F;
     typedef RevCfg<K, V, NWC, true> R;
     static_assert(F::THREADS == R::THREADS, "one launch");
     constexpr int COLS = (V + K) / 16 / NWC;
@@ -363,7 +363,7 @@ __global__ __launch_bounds__((RevCfg<K, V, NWC, true>::THREADS)) void scan_grad_
     const int n = scan_sequence(p.st, z), y = blockIdx.y + first_y, split = y % COLS;
     if (y < COLS) {
         if (seg == 0 && split >= R::SPLIT) return;        // starts from h0: nobody asks for its transition
-        scan_out_body<K, V, NWC, OUT_SUM, 1>(p, smem, n, seg, split);
+        scan_out_body<K, V, NWC, OUT_SUM, 1, HD>(p, smem, n, seg, split);
     } else {
         if (seg + 1 == p.seg.nseg - 1 && split >= R::SPLIT) return;
         scan_rev_body<K, V, NWC, true>(p, smem, n, seg + 1, split);
@@ -373,7 +373,8 @@ __global__ __launch_bounds__((RevCfg<K, V, NWC, true>::THREADS)) void scan_grad_
 template <int K, int V, int NWC> static hipError_t launch_scan_grad_nwc(const ChunkArgs<bf16>& a, ScanKind kind, hipStream_t stream) {
     typedef RevCfg<K, V, NWC, false> C;
     const dim3 grid(a.H, C::SPLIT * (kind == SCAN_PAIR ? 2 : 1), a.st.N * a.seg.nseg);
-    hipLaunchKernelGGL((scan_grad_kernel<K, V, NWC>), grid, dim3(C::THREADS), 0, stream, a, (int)(kind == SCAN_BWD));
+    if (a.beta) hipLaunchKernelGGL((scan_grad_kernel<K, V, NWC, true>), grid, dim3(C::THREADS), 0, stream, a, (int)(kind == SCAN_BWD));
+    else hipLaunchKernelGGL((scan_grad_kernel<K, V, NWC, false>), grid, dim3(C::THREADS), 0, stream, a, (int)(kind == SCAN_BWD));
     return hipGetLastError();
 }
 // Column blocks a workgroup: as few as give each workgroup a compute unit of its own.  K = V = 128, 2 x 1537 tokens of 8 heads, one and two
@@ -383,8 +384,9 @@ template <int K, int V> hipError_t launch_scan_grad_shape(const ChunkArgs<bf16>&
     const int lanes = a.H * a.st.N * a.seg.nseg * (kind == SCAN_PAIR ? 2 : 1);
     if (lanes * VT <= SCAN_TARGET_WORKGROUPS) return launch_scan_grad_nwc<K, V, 1>(a, kind, stream);
     if (kind == SCAN_PAIR && scan_shares(a.st.cu, a.st.N, a.H, V, a.seg.nseg, 2)) {
-        hipLaunchKernelGGL((scan_grad_share_kernel<K, V>), dim3(a.H, 2 * share_most(a.H, 2, a.st.N, V)), dim3(RevCfg<K, V, 4, false>::THREADS), 0,
-                           stream, a);
+        const dim3 grid(a.H, 2 * share_most(a.H, 2, a.st.N, V)), block(RevCfg<K, V, 4, false>::THREADS);
+        if (a.beta) hipLaunchKernelGGL((scan_grad_share_kernel<K, V, true>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((scan_grad_share_kernel<K, V, false>), grid, block, 0, stream, a);
         return hipGetLastError();
     }
     if (kind == SCAN_BWD && scan_shares(a.st.cu, a.st.N, a.H, V, a.seg.nseg, 1)) {
@@ -397,8 +399,9 @@ template <int K, int V> hipError_t launch_scan_grad_shape(const ChunkArgs<bf16>&
 template <int K, int V> hipError_t launch_scan_grad_segments_shape(const ChunkArgs<bf16>& a, SegStart what, hipStream_t stream) {
     constexpr int NWC = 4;
     typedef RevCfg<K, V, NWC, true> C;
-    hipLaunchKernelGGL((scan_grad_sum_kernel<K, V, NWC>), dim3(a.H, sum_splits<K, V, NWC>(what, a.seg.turned), a.st.N * (a.seg.nseg - 1)), dim3(C::THREADS), 0,
-                       stream, a, sum_first<K, V, NWC>(what));
+    const dim3 grid(a.H, sum_splits<K, V, NWC>(what, a.seg.turned), a.st.N * (a.seg.nseg - 1)), block(C::THREADS);
+    if (a.beta) hipLaunchKernelGGL((scan_grad_sum_kernel<K, V, NWC, true>), grid, block, 0, stream, a, (sum_first<K, V, NWC>(what)));
+    else hipLaunchKernelGGL((scan_grad_sum_kernel<K, V, NWC, false>), grid, block, 0, stream, a, (sum_first<K, V, NWC>(what)));
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? launch_scan_chain<bf16, K, V>(a, what, stream) : e;
 }

@@ -27,12 +27,19 @@
 
 namespace hdla {
 
-template <int K, int V, int NWC, ScanOut OUT> struct OutCfg {
+// HD: with the HDLA parameterisation b_2 is k, so the gated copies of the two are the same tiles: kg^T is neither stored nor moved nor read (4 of a chunk and head's 42
+// KB that prep moves at K = V = 128, of 37 that a forward pass's scan does).  us as a graph's replay, before -> after, the same bits, K = V = 128: forward pass of 4 x 2048 tokens of 16 heads 183 -> 164, 5003 packed
+// 111 -> 108, 1 x 2048 79.8 -> 77.9; training step of 2 x 1537 of 8 162.3 -> 159.0; K = 128, V = 64, 1 x 3000 of 16 254 -> 248; K = 64, V = 128, 2 x 2000 of 4, forward 49.4 -> 48.7.
+template <int K, int V, int NWC, ScanOut OUT, bool HD> struct OutCfg {
     static constexpr bool WITH_O = OUT == OUT_O;
     static constexpr int VT = V / 16, SPLIT = VT / NWC, KT = K / 16;
-    static constexpr BlkF B = blk_fwd(K, 2, true);
-    // 1-KiB pieces of a chunk's block that the scan needs (without o: without q's and the scores')
-    static constexpr int NI = (WITH_O ? B.SIZE : B.EGL + 1024) / 1024, SLOT = NI * 1024;
+    static constexpr BlkF STORED = blk_fwd(K, 2, true);
+    // 1-KiB pieces of a chunk's block that the scan needs (without o: without q's and the scores'), and where they are in LDS: HD without the CUT pieces from AT on
+    static constexpr int CUT = HD ? KT / 2 : 0, AT = STORED.KGT / 1024;
+    static constexpr int NI = (WITH_O ? STORED.SIZE : STORED.EGL + 1024) / 1024 - CUT, SLOT = NI * 1024;
+    static constexpr BlkF slot_of(BlkF b) { b.EGL -= CUT * 1024; b.QG -= CUT * 1024; b.AQB -= CUT * 1024; b.AQK -= CUT * 1024; return b; }
+    static constexpr BlkF B = slot_of(STORED);
+    static __device__ __forceinline__ int stored(int i) { return HD && i >= AT ? i + CUT : i; }
     // computing waves of a column block, each holding KH channel tiles of the state
     static constexpr int PARTS = K / 64, KH = KT / PARTS, NC = NWC * PARTS;
     static constexpr int NL = 2, NM = NL + 1 + WITH_O;    // waves that load, with the one that forms u and the one that copies the output out
@@ -65,9 +72,9 @@ template <typename C> __device__ __forceinline__ int forming_first(int wave) { r
 // KEPT: on a workspace of the backward pass (or that it will read, PREP_KEEP): (I - A_ab)^-1 is there turned, as chunk_grad takes it, A_ak in a place of its
 // own, and b^T's pairs are of two channel tiles, as the reverse scan takes them.  The same products in the same order: the same bits.
 // KEPT 2 (PREP_STATES): the states that enter the chunks are left for the backward pass, and q's part of the block is not the kept buffer's.
-template <int K, int V, int NWC, ScanOut OUT, int KEPT>
+template <int K, int V, int NWC, ScanOut OUT, int KEPT, bool HD>
 __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* smem, int n, int seg, int split) {
-    typedef OutCfg<K, V, NWC, OUT> C;
+    typedef OutCfg<K, V, NWC, OUT, HD> C;
     typedef bf16 T;
     constexpr bool WITH_O = OUT == OUT_O, SUM = OUT == OUT_SUM;
     constexpr bool FWD = WITH_O && !KEPT, STATES = KEPT == 2;   // a forward pass that keeps nothing (see forming_first)
@@ -95,9 +102,9 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
         if (nchunks <= 0) return;
         const int hw = FWD ? wv - C::NC : forming_first<C>(wv - C::NC);
         if (hw < C::NL) {
-            const int stride = KEPT ? p.ws.sa_stride : B.SIZE;
+            const int stride = KEPT ? p.ws.sa_stride : C::STORED.SIZE;
             const char* const blk = reinterpret_cast<const char*>(p.ws.W) + chw0 * stride + l * 16;
-            constexpr int PRE = STATES ? blk_fwd(K, 2, false).SIZE / 1024 : C::NI, STRIDE_Q = blk_q(K, 2);
+            constexpr int PRE = STATES ? blk_fwd(K, 2, false).SIZE / 1024 - C::CUT : C::NI, STRIDE_Q = blk_q(K, 2);
             const char* const blk_of_q = reinterpret_cast<const char*>(p.ws.QG) + chw0 * STRIDE_Q + l * 16;
             int slot = 0;
             auto load = [&](int t) __attribute__((always_inline)) {
@@ -107,7 +114,7 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
 #pragma unroll
                 for (int j = 0; j < C::CNT; ++j) {
                     const int i = min(hw + j * C::NL, C::NI - 1);
-                    const char* const src = !STATES || i < PRE ? bt + i * 1024 : qt + (i - PRE) * 1024;
+                    const char* const src = !STATES || i < PRE ? bt + C::stored(i) * 1024 : qt + (i - PRE) * 1024;
                     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
                                                      (__attribute__((address_space(3))) void*)(smem + slot * SLOT + i * 1024), 16, 0, 0);
                 }
@@ -265,7 +272,7 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
         constexpr bool ALONE = NWC == 1 && PARTS > 1;
         constexpr bool first = part == 0, from_u = part == PARTS - 1;   // the wave with the output, and the one that starts v_new from u
         // A chunk's operands, read as soon as the chunk before has been through with their registers: half a step and more before they are used
-        Frag<T> w[2][KH], qg[WITH_O ? KH : 1], kgt[KH], bgt[2][KH], aqk, aqb[2], ut[2], vtt;
+        Frag<T> w[2][KH], qg[WITH_O ? KH : 1], kgt[HD ? 1 : KH], bgt[2][KH], aqk, aqb[2], ut[2], vtt;
         f32x4 egl[KH];
         // (the lane's offset is all of an address that the wave holds in vector registers: the rest is the slot's and immediate)
         const uint32_t lo = 16 * l, ge = 16 * g;
@@ -288,7 +295,7 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
 #pragma unroll
             for (int kp = 0; kp < KH2; ++kp) {
                 if constexpr (WITH_O) pair_at(so, B.QG + (part * KH2 + kp) * 1024, qg[2 * kp], qg[2 * kp + 1]);
-                pair_at(so, B.KGT + (part * KH2 + kp) * 1024, kgt[2 * kp], kgt[2 * kp + 1]);
+                if constexpr (!HD) pair_at(so, B.KGT + (part * KH2 + kp) * 1024, kgt[2 * kp], kgt[2 * kp + 1]);
             }
 #pragma unroll
             for (int k = 0; k < KH; ++k) egl[k] = *reinterpret_cast<const f32x4*>(smem + so + ge + B.EGL + 64 * (kt0 + k));
@@ -342,7 +349,7 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
             // ---- what is one product a sum: the chunk's own part of the state, A_qk v
             f32x4 x[KH + 1];
 #pragma unroll
-            for (int k = 0; k < KH; ++k) x[k] = mm(vtt, kgt[k], S[k] * egl[k]);
+            for (int k = 0; k < KH; ++k) x[k] = mm(vtt, HD ? bgt[1][k] : kgt[HD ? 0 : k], S[k] * egl[k]);
             x[KH] = zero4();
             if constexpr (WITH_O && first) x[KH] = mm(aqk, vtt, x[KH]);
             if constexpr (PARTS > 1) {
@@ -415,11 +422,11 @@ __device__ __forceinline__ void scan_out_body(const ChunkArgs<bf16>& p, char* sm
 }
 
 // grid = (H, SPLIT, N * segments), as the other scans' (scan_impl.cuh)
-template <int K, int V, int NWC, int KEPT>
-__global__ __launch_bounds__((OutCfg<K, V, NWC, OUT_O>::THREADS)) void scan_out_kernel(ChunkArgs<bf16> p) {
-    __shared__ __attribute__((aligned(16))) char smem[OutCfg<K, V, NWC, OUT_O>::BYTES];
+template <int K, int V, int NWC, int KEPT, bool HD>
+__global__ __launch_bounds__((OutCfg<K, V, NWC, OUT_O, HD>::THREADS)) void scan_out_kernel(ChunkArgs<bf16> p) {
+    __shared__ __attribute__((aligned(16))) char smem[OutCfg<K, V, NWC, OUT_O, HD>::BYTES];
     const int z = blockIdx.z / p.seg.nseg, seg = blockIdx.z % p.seg.nseg;
-    scan_out_body<K, V, NWC, OUT_O, KEPT>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
+    scan_out_body<K, V, NWC, OUT_O, KEPT, HD>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
 }
 // Packed sequences that share the device by their lengths (see share_device, prep.hip): grid = (H, workgroups of a head).  Waves that a narrow
 // workgroup has no use for end at once; barriers are among those that are left.  Measured, us, one width for all -> this, K = V = 128, 16 heads: forward
@@ -427,58 +434,62 @@ __global__ __launch_bounds__((OutCfg<K, V, NWC, OUT_O>::THREADS)) void scan_out_
 // similar lengths 137.7 -> 138.0; 12000 in 12, 8 heads 209 -> 186; training steps of 6000 in 6 748 -> 683, of 1500 in 7, 12 heads 174 -> 153, of
 // 16384 in 4 1726 -> 1705 (its two scans are at their traffic, 2.2 GB in 520 us, in every width).  Where one block a workgroup for all fits the device,
 // that is faster still and stays.  Beyond 32 sequences the device is full with the widest workgroups for all but the last few steps.
-template <int K, int V, int KEPT>
-__global__ __launch_bounds__((OutCfg<K, V, 4, OUT_O>::THREADS)) void scan_out_share_kernel(ChunkArgs<bf16> p) {
-    typedef OutCfg<K, V, 4, OUT_O> C4;
-    typedef OutCfg<K, V, 2, OUT_O> C2;
-    typedef OutCfg<K, V, 1, OUT_O> C1;
+template <int K, int V, int KEPT, bool HD>
+__global__ __launch_bounds__((OutCfg<K, V, 4, OUT_O, HD>::THREADS)) void scan_out_share_kernel(ChunkArgs<bf16> p) {
+    typedef OutCfg<K, V, 4, OUT_O, HD> C4;
+    typedef OutCfg<K, V, 2, OUT_O, HD> C2;
+    typedef OutCfg<K, V, 1, OUT_O, HD> C1;
     __shared__ __attribute__((aligned(16))) char smem[C4::BYTES > C2::BYTES ? (C4::BYTES > C1::BYTES ? C4::BYTES : C1::BYTES) : C2::BYTES > C1::BYTES ? C2::BYTES : C1::BYTES];
     int n, code, split;
     if (!scan_share<V>(p.st, blockIdx.y, ORDER_OUT, n, code, split)) return;
-    if (code == 0) scan_out_body<K, V, 4, OUT_O, KEPT>(p, smem, n, 0, split);
-    else if (code == 1) { if ((int)threadIdx.x < C2::THREADS) scan_out_body<K, V, 2, OUT_O, KEPT>(p, smem, n, 0, split); }
-    else if ((int)threadIdx.x < C1::THREADS) scan_out_body<K, V, 1, OUT_O, KEPT>(p, smem, n, 0, split);
+    if (code == 0) scan_out_body<K, V, 4, OUT_O, KEPT, HD>(p, smem, n, 0, split);
+    else if (code == 1) { if ((int)threadIdx.x < C2::THREADS) scan_out_body<K, V, 2, OUT_O, KEPT, HD>(p, smem, n, 0, split); }
+    else if ((int)threadIdx.x < C1::THREADS) scan_out_body<K, V, 1, OUT_O, KEPT, HD>(p, smem, n, 0, split);
 }
 // the segments' records in the forward direction: grid = (H, (V + K) / 16 / NWC, N * (segments - 1))
-template <int K, int V, int NWC>
-__global__ __launch_bounds__((OutCfg<K, V, NWC, OUT_SUM>::THREADS)) void scan_out_sum_kernel(ChunkArgs<bf16> p) {
-    __shared__ __attribute__((aligned(16))) char smem[OutCfg<K, V, NWC, OUT_SUM>::BYTES];
+template <int K, int V, int NWC, bool HD>
+__global__ __launch_bounds__((OutCfg<K, V, NWC, OUT_SUM, HD>::THREADS)) void scan_out_sum_kernel(ChunkArgs<bf16> p) {
+    __shared__ __attribute__((aligned(16))) char smem[OutCfg<K, V, NWC, OUT_SUM, HD>::BYTES];
     const int z = blockIdx.z / (p.seg.nseg - 1), seg = blockIdx.z % (p.seg.nseg - 1);
-    if (seg == 0 && (int)blockIdx.y >= OutCfg<K, V, NWC, OUT_SUM>::SPLIT) return;   // starts from h0: nobody asks for its transition
-    scan_out_body<K, V, NWC, OUT_SUM, 0>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
+    if (seg == 0 && (int)blockIdx.y >= OutCfg<K, V, NWC, OUT_SUM, HD>::SPLIT) return;   // starts from h0: nobody asks for its transition
+    scan_out_body<K, V, NWC, OUT_SUM, 0, HD>(p, smem, scan_sequence(p.st, z), seg, blockIdx.y);
 }
 
-template <int K, int V, int NWC> static hipError_t launch_scan_out_nwc(const ChunkArgs<bf16>& a, int kept, hipStream_t stream) {
-    typedef OutCfg<K, V, NWC, OUT_O> C;
+template <int K, int V, int NWC, bool HD> static hipError_t launch_scan_out_nwc(const ChunkArgs<bf16>& a, int kept, hipStream_t stream) {
+    typedef OutCfg<K, V, NWC, OUT_O, HD> C;
     const dim3 grid(a.H, C::SPLIT, a.st.N * a.seg.nseg), block(C::THREADS);
-    if (kept == 2) hipLaunchKernelGGL((scan_out_kernel<K, V, NWC, 2>), grid, block, 0, stream, a);
-    else if (kept) hipLaunchKernelGGL((scan_out_kernel<K, V, NWC, 1>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((scan_out_kernel<K, V, NWC, 0>), grid, block, 0, stream, a);
+    if (kept == 2) hipLaunchKernelGGL((scan_out_kernel<K, V, NWC, 2, HD>), grid, block, 0, stream, a);
+    else if (kept) hipLaunchKernelGGL((scan_out_kernel<K, V, NWC, 1, HD>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((scan_out_kernel<K, V, NWC, 0, HD>), grid, block, 0, stream, a);
     return hipGetLastError();
 }
 // Column blocks a workgroup: as few as give each workgroup a compute unit of its own (every workgroup fetches the chunks' blocks for
 // itself).  A forward pass, us, two blocks and one, 128 chunks in one segment: K = V = 128, 1 lane 82 and 73, 16 lanes 102 and 96, 32 lanes 135 and
 // 127; K = 64, V = 128, 8 lanes 71 and 59, 32 lanes 88 and 79; of 16 chunks K = V = 128 22.3 and 20.8.  The scan alone, two and four: K = V = 128,
 // 128 heads 193 and 146, 64 heads 101 and 114.
-template <int K, int V> hipError_t launch_scan_out_shape(const ChunkArgs<bf16>& a, int kept, hipStream_t stream) {
+template <int K, int V, bool HD> static hipError_t launch_scan_out_hd(const ChunkArgs<bf16>& a, int kept, hipStream_t stream) {
     constexpr int VT = V / 16;
     const int lanes = a.H * a.st.N * a.seg.nseg;
-    if (lanes * VT <= SCAN_TARGET_WORKGROUPS) return launch_scan_out_nwc<K, V, 1>(a, kept, stream);
+    if (lanes * VT <= SCAN_TARGET_WORKGROUPS) return launch_scan_out_nwc<K, V, 1, HD>(a, kept, stream);
     if (scan_shares(a.st.cu, a.st.N, a.H, V, a.seg.nseg, 1)) {
-        const dim3 grid(a.H, share_most(a.H, 1, a.st.N, V)), block(OutCfg<K, V, 4, OUT_O>::THREADS);
-        if (kept == 2) hipLaunchKernelGGL((scan_out_share_kernel<K, V, 2>), grid, block, 0, stream, a);
-        else if (kept) hipLaunchKernelGGL((scan_out_share_kernel<K, V, 1>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((scan_out_share_kernel<K, V, 0>), grid, block, 0, stream, a);
+        const dim3 grid(a.H, share_most(a.H, 1, a.st.N, V)), block(OutCfg<K, V, 4, OUT_O, HD>::THREADS);
+        if (kept == 2) hipLaunchKernelGGL((scan_out_share_kernel<K, V, 2, HD>), grid, block, 0, stream, a);
+        else if (kept) hipLaunchKernelGGL((scan_out_share_kernel<K, V, 1, HD>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((scan_out_share_kernel<K, V, 0, HD>), grid, block, 0, stream, a);
         return hipGetLastError();
     }
-    if (lanes * (VT / 2) <= SCAN_TARGET_WORKGROUPS) return launch_scan_out_nwc<K, V, 2>(a, kept, stream);
-    return launch_scan_out_nwc<K, V, 4>(a, kept, stream);
+    if (lanes * (VT / 2) <= SCAN_TARGET_WORKGROUPS) return launch_scan_out_nwc<K, V, 2, HD>(a, kept, stream);
+    return launch_scan_out_nwc<K, V, 4, HD>(a, kept, stream);
+}
+template <int K, int V> hipError_t launch_scan_out_shape(const ChunkArgs<bf16>& a, int kept, hipStream_t stream) {
+    return a.beta ? launch_scan_out_hd<K, V, true>(a, kept, stream) : launch_scan_out_hd<K, V, false>(a, kept, stream);
 }
 // the segments' records, chained into what enters the segments
 template <int K, int V> hipError_t launch_scan_out_segments_shape(const ChunkArgs<bf16>& a, hipStream_t stream) {
     constexpr int NWC = 4;
-    typedef OutCfg<K, V, NWC, OUT_SUM> C;
-    hipLaunchKernelGGL((scan_out_sum_kernel<K, V, NWC>), dim3(a.H, (V + K) / 16 / NWC, a.st.N * (a.seg.nseg - 1)), dim3(C::THREADS), 0, stream, a);
+    const dim3 grid(a.H, (V + K) / 16 / NWC, a.st.N * (a.seg.nseg - 1)), block(OutCfg<K, V, NWC, OUT_SUM, false>::THREADS);
+    if (a.beta) hipLaunchKernelGGL((scan_out_sum_kernel<K, V, NWC, true>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((scan_out_sum_kernel<K, V, NWC, false>), grid, block, 0, stream, a);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? launch_scan_chain<bf16, K, V>(a, SEG_FWD, stream) : e;
 }
