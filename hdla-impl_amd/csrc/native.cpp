@@ -645,8 +645,11 @@ constexpr double PRE_EPS = 1e-5;                 // l2_norm's
 // Columns of y: q, k, v (d each), the inner activations of decay and gate (D each), beta (H), padding.
 struct LayerCols {
     int64_t d, D, H, f0, g0, beta, used, ld;
-    LayerCols(int64_t d_, int64_t H_, bool padded) : d(d_), D(d_ / H_), H(H_) {
-        f0 = 3 * d; g0 = f0 + D; beta = g0 + D; used = beta + H;
+    // of a concatenated weight that has ld_ rows
+    LayerCols(int64_t d_, int64_t H_, int64_t ld_) : d(d_), D(d_ / H_), H(H_) {
+        f0 = 3 * d; g0 = f0 + D; beta = g0 + D; used = beta + H; ld = ld_;
+    }
+    LayerCols(int64_t d_, int64_t H_, bool padded) : LayerCols(d_, H_, int64_t(0)) {
         // The GEMM on x runs at its best on output widths that are whole tiles of 256 (8192 x 3216 x 1024: 82 us, with
         // 3328 columns 50; its input gradient 60 -> 55, its weight gradient 86 -> 80).  Short calls read the weight once and are
         // bound by that: there only up to the 16 bytes that rows are aligned to.
@@ -654,6 +657,15 @@ struct LayerCols {
     }
 };
 constexpr int64_t PAD_FROM_ROWS = 1024;
+// In training, where that makes the weight's gradient one of the library's own (own_weight_grad), up to whole tiles of its kernel: a
+// BLAS call less, and both weight gradients in one launch.  us a training step (all of these are bound by the host): 4 x 121 tokens, 256 channels 239 -> 218, 1 x 64, 512 246 -> 222,
+// 2 x 500, 512 275 -> 248, 1 x 512, 1024 271 -> 245, 1 x 1000, 1024 273 -> 246.  Wider layers, whose gradient has more tiles, stay as they are (1 x 900, 2048 384 and 379).
+LayerCols training_cols(int64_t d, int64_t H, int64_t rows) {
+    LayerCols L(d, H, rows >= PAD_FROM_ROWS);
+    const int64_t tiles = (L.used + 127) / 128;
+    if (rows < PAD_FROM_ROWS && d % 128 == 0 && tiles * (d / 128) <= 256) L.ld = 128 * tiles;
+    return L;
+}
 
 // the concatenated projection weight [ld, d], in `out` if there is one; rows behind the last projection are zero
 Tensor gather_weights(const Tensor* w, const LayerCols& L, Tensor out = Tensor()) {       // wq, wk, wv, wf0, wg0, wbeta
@@ -776,7 +788,7 @@ bool in_few_launches(int64_t rows, int64_t T, int64_t d, bool norm_in_step) {
 void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, Plan& plan, const Tensor& h0, bool want_ht, bool chunked, bool keep,
                    LayerFwd& r) {
     const int64_t B = x3.size(0), T = x3.size(1), d = x3.size(2), rows = B * T;
-    const LayerCols L(d, f.H, r.w.size(0) != LayerCols(d, f.H, false).ld);
+    const LayerCols L(d, f.H, r.w.size(0));
     const auto opt = x3.options();
     r.x = x3.contiguous().view({rows, d});
     r.y = project(r.x, r.w);
@@ -877,7 +889,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
                                  const Tensor& wo, const Maybe& h0, const LayerCfg& f, bool want_ht, Plan plan) {
         const Tensor P[10] = {wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo};
         LayerFwd r;
-        r.w = gather_weights(P, LayerCols(x.size(2), f.H, x.size(0) * x.size(1) >= PAD_FROM_ROWS));
+        r.w = gather_weights(P, training_cols(x.size(2), f.H, x.size(0) * x.size(1)));
         layer_forward(x, P, f, plan, value(h0), want_ht, true, true, r);
         save_plan(ctx, plan);
         ctx->save_for_backward({r.x, r.w, r.y, r.f, r.g, r.o, r.n, r.left, r.op.q, r.op.k, r.op.v, r.op.beta, r.op.gk, value(h0), wf1, wg1,
@@ -903,7 +915,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
         const auto ci = ctx->saved_data["i"].toIntVector();
         const LayerCfg cfg{ci[0], ci[1], ci[2] != 0, ci[3] != 0, cc[0], cc[1], cc[2], (int)ci[4]};
         const int64_t B = ci[5], T = ci[6], rows = x.size(0), d = x.size(1);
-        const LayerCols L(d, cfg.H, w.size(0) != LayerCols(d, cfg.H, false).ld);
+        const LayerCols L(d, cfg.H, w.size(0));
         void* const stream = stream_of(x);
         const auto opt = x.options();
         const auto need = [&](size_t i) { return ctx->needs_input_grad(i); };
