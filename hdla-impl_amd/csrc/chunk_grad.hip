@@ -81,6 +81,15 @@ __device__ __forceinline__ void chunk_grad_strong_pair(const ChunkArgs<T>& p, in
 #include "chunk_grad_body.inc"
 #undef CG_STRONG
 }
+// a common pair; a flagged one is left alone, and said to be
+template <typename T, bool GKF32, int K, int V, bool HD>
+__device__ __forceinline__ void chunk_grad_common_pair(const ChunkArgs<T>& p, int cid, int h, char* smem, bool& was_flagged) {
+#define CG_STRONG 0
+#define CG_LEAVE do { was_flagged = true; return; } while (0)
+#include "chunk_grad_body.inc"
+#undef CG_LEAVE
+#undef CG_STRONG
+}
 
 // The common pairs, one workgroup per (chunk, head), which leave the flagged ones alone; and behind them, or in a launch of their own, what looks for
 // the flagged pairs and works them off.  They are rare (a channel must lose more than e^-70 within eight tokens), so this is a small number of
@@ -90,15 +99,21 @@ __device__ __forceinline__ void chunk_grad_strong_pair(const ChunkArgs<T>& p, in
 // limit of their occupancy, pay nothing for them, and when nothing is flagged, which is the rule, their launch costs its start-up and one round of flag
 // reads, 4 to 5 us.  fp32, training step of 2 x 1003 tokens, 8 heads, K = V = 64, two launches -> one: 185.6 -> 181.5 us;
 // 838 tokens, 12 heads, K = V = 128 382 -> 377; beta form, 900 tokens, 8 heads 141.6 -> 138.6; 2 x 2000 tokens, 16 heads 547 both.
-enum CgPairs { CG_COMMON, CG_FLAGGED, CG_ALL };
+// CG_EACH (2-byte elements): one launch for no more pairs than the device holds at once, where occupancy is nothing and a workgroup may have more registers: each does its own pair,
+// flagged or not.  us a training step as
+// a graph's replay, two launches -> one: 32 pairs of K = V = 64 36.0 -> 34.2, 252 82.7 -> 80.4 (beta form), 480 54.4 -> 50.1 (beta form), 512 64.6 -> 61.9; K = V = 128, 14 37.7 -> 36.2,
+// 256 (beta form, with less to store and read in the scans) 65.4 -> 62.7.  Beyond, with one workgroup a compute unit: 960 of K = V = 64 62.5 -> 68.4, K = V = 128 528 90 -> 96, 1552 159 -> 188.
+enum CgPairs { CG_COMMON, CG_FLAGGED, CG_ALL, CG_EACH };
 constexpr int CG_STRONG_GRID = 256;
+// CG_EACH's waves per SIMD, and so workgroups a compute unit: what its registers allow
+template <bool GKF32, int K, int V> constexpr int cg_each_waves() { return !GKF32 && K == 64 && V == 64 ? 2 : 1; }
 template <typename T, bool GKF32, int K, int V, bool HD, CgPairs WHAT>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WHAT == CG_FLAGGED ? 1 : cg_waves<T, GKF32, K, V, HD>(false),
-                                                                         WHAT == CG_FLAGGED ? 1 : cg_waves<T, GKF32, K, V, HD>(true))))
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WHAT == CG_EACH ? cg_each_waves<GKF32, K, V>() : WHAT == CG_FLAGGED ? 1 : cg_waves<T, GKF32, K, V, HD>(false),
+                                                                         WHAT == CG_EACH ? cg_each_waves<GKF32, K, V>() : WHAT == CG_FLAGGED ? 1 : cg_waves<T, GKF32, K, V, HD>(true))))
 void chunk_grad_kernel(ChunkArgs<T> p) {
     __shared__ __attribute__((aligned(16))) char smem[CgLds<T, K, V>::BYTES];
     const int total = p.H * p.st.nch;
-    if (WHAT != CG_COMMON && (WHAT == CG_FLAGGED || (int)blockIdx.x >= total)) {
+    if (WHAT != CG_COMMON && WHAT != CG_EACH && (WHAT == CG_FLAGGED || (int)blockIdx.x >= total)) {
         __shared__ unsigned long long sMask[NW];
         constexpr int nth = 64 * NW;
         const int group = (int)blockIdx.x - (WHAT == CG_ALL ? total : 0), groups = (int)gridDim.x - (WHAT == CG_ALL ? total : 0);
@@ -130,9 +145,17 @@ void chunk_grad_kernel(ChunkArgs<T> p) {
     const bool head_fastest = (uint32_t)(p.H * K) * sizeof(T) >= 4096;
     const int cid = head_fastest ? blockIdx.x / p.H : blockIdx.x % p.st.nch;
     const int h = head_fastest ? blockIdx.x % p.H : blockIdx.x / p.st.nch;
+    if constexpr (WHAT == CG_EACH) {
+        bool flagged = false;                                 // (uniform over the workgroup)
+        chunk_grad_common_pair<T, GKF32, K, V, HD>(p, cid, h, smem, flagged);
+        if (flagged) chunk_grad_strong_pair<T, GKF32, K, V, HD>(p, cid, h, smem);
+    } else {
 #define CG_STRONG 0
+#define CG_LEAVE return
 #include "chunk_grad_body.inc"
+#undef CG_LEAVE
 #undef CG_STRONG
+    }
 }
 
 template <typename T, bool GKF32, int K, int V, bool HD>
@@ -140,6 +163,8 @@ static hipError_t launch_chunk_grad_gk(const ChunkArgs<T>& a, hipStream_t stream
     const int total = a.st.nch * a.H, strong = total < CG_STRONG_GRID ? total : CG_STRONG_GRID;
     if constexpr (sizeof(T) == 4) {
         hipLaunchKernelGGL((chunk_grad_kernel<T, GKF32, K, V, HD, CG_ALL>), dim3(total + strong), dim3(64 * NW), 0, stream, a);
+    } else if (total <= 256 * cg_each_waves<GKF32, K, V>()) {
+        hipLaunchKernelGGL((chunk_grad_kernel<T, GKF32, K, V, HD, CG_EACH>), dim3(total), dim3(64 * NW), 0, stream, a);
     } else {
         hipLaunchKernelGGL((chunk_grad_kernel<T, GKF32, K, V, HD, CG_COMMON>), dim3(total), dim3(64 * NW), 0, stream, a);
         hipLaunchKernelGGL((chunk_grad_kernel<T, GKF32, K, V, HD, CG_FLAGGED>), dim3(strong), dim3(64 * NW), 0, stream, a);
