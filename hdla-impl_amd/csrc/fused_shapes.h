@@ -15,6 +15,10 @@ template <typename T>
 struct FusedArgs {
     ChunkArgs<T> c;
     int nseg;              // time segments per sequence
+    // packed sequences whose segments go by their lengths (share_segments, prep.hip), `slots` = N nseg at most; null: nseg each.  Of the records below a sequence then has
+    // its own number, those of a sequence and head side by side.
+    const SegSlot* seg_tab;
+    int slots;
     // records per (sequence, head, segment), fp32 tiles in fragment order (see fused_impl.cuh)
     float* sloc;           // [N][H][nseg][K*V]
     float* mseg;           // [N][H][nseg][K*K]

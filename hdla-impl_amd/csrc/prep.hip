@@ -110,10 +110,50 @@ __device__ __forceinline__ int share_device(ShareLds& sh, int N, int H, int V, i
     }
     return codes;
 }
+// Time segments by length (fused route): `slots` of them for N sequences, each sequence as many as make the longest segment as short as can be, of SHARE_SEGMENT_CHUNKS chunks at the
+// least (a sequence's last one may be shorter).  A wave, a lane a sequence.  Equal numbers wait for the longest sequence's: 16 heads, K = V = 64, sequences of 4100, 1500, 2000 and 592
+// tokens, us, forward pass 123 -> 86, training step 364 -> 287; of 300, 700, 2500, 200, 1300, 1000 tokens (HDLA parameterisation) 145 -> 89, 351 -> 243; 8 heads, of 2600, 1000 and 400
+// tokens 59.6 -> 54.1, 145 -> 138; 32 heads, of 5000, 2000, 2500 and 500 tokens, training step 937 -> 777; equal lengths get equal numbers, in the same time (a slot says its
+// chunks itself: one round of loads at a kernel's start; with a table of the sequences instead training on 4 x 2048 tokens took 276 against 272).
+constexpr int SHARE_SEGMENT_CHUNKS = 8, SHARE_SEGMENTS = 64;
+__device__ __forceinline__ void share_segments(const FewSeqs& f, int N, int slots, SegSlot* seg_tab) {
+    const int n = lane_id();
+    const unsigned own = n < N ? f.chunks : 0, cap = max(1u, min((unsigned)SHARE_SEGMENTS, own / SHARE_SEGMENT_CHUNKS));
+    auto of_length = [&](unsigned len) __attribute__((always_inline)) { return n < N ? (int)min(cap, max(1u, (own + len - 1) / len)) : 0; };
+    auto ends = [](int x) __attribute__((always_inline)) { return sum_lanes(x, 0x3fffffff); };
+    // Segments of hi chunks are few enough in the end (a sequence of at most hi chunks has one, and slots >= N), of lo not or needlessly short.
+    const unsigned all = of_lane(ends((int)own), 63);
+    unsigned hi = max((unsigned)SHARE_SEGMENT_CHUNKS, (all + slots - 1) / (unsigned)slots), lo = hi - 1;
+    int mine = of_length(hi), end = ends(mine);
+    while (of_lane(end, 63) > slots) {
+        lo = hi;
+        hi *= 2;
+        mine = of_length(hi);
+        end = ends(mine);
+    }
+    while (hi - lo > 1) {
+        const unsigned mid = lo + (hi - lo) / 2;
+        const int m = of_length(mid), e = ends(m);
+        if (of_lane(e, 63) > slots) {
+            lo = mid;
+        } else {
+            hi = mid;
+            mine = m;
+            end = e;
+        }
+    }
+    const int before = __shfl_up(f.end, 1), c0 = n == 0 ? 0 : before, first = end - mine;
+    for (int s = 0; n < N && s < mine; ++s) {
+        SegSlot x{n | s << 8 | mine << 16, first, 0, 0};
+        seg_range(c0, f.end, mine, s, x.s0, x.s1);
+        seg_tab[first + s] = x;
+    }
+    for (int i = of_lane(end, 63) + n; i < slots; i += 64) seg_tab[i] = SegSlot{-1, 0, 0, 0};
+}
 // A table of at most FEW_SEQS sequences, in registers: work 0 writes chunk_off and chunk_seq, work 1 ranks the sequences (V: as in
 // launch_chunk_table).  All threads of a workgroup, at least a wave, each wave for itself but for the widths.
 __device__ __forceinline__ void few_table(int work, const int64_t* cu, int N, int T, int nch, int H, int V, int32_t* chunk_off, int32_t* chunk_seq,
-                                          ShareLds& sh, int t, int threads) {
+                                          ShareLds& sh, int t, int threads, SegSlot* seg_tab = nullptr, int slots = 0) {
     const FewSeqs f = few_seqs(cu, N, T, nch);
     if (work == 0) {
         if (t < N) chunk_off[t + 1] = f.end;
@@ -127,6 +167,7 @@ __device__ __forceinline__ void few_table(int work, const int64_t* cu, int N, in
     }
     int32_t* const order = chunk_off + N + 1;
     const int n = lane_id();
+    if (seg_tab && t >> 6 == 1) share_segments(f, N, slots, seg_tab);   // (beside the ranking)
     int r = 0;
     for (int m = 0; m < N; ++m) {
         const int other = of_lane(f.chunks, m);
@@ -144,7 +185,7 @@ __device__ __forceinline__ void few_table(int work, const int64_t* cu, int N, in
     if (t < N) order[t] = sh.seq[t] | codes;
 }
 __global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const int64_t* cu, int N, int T, int nch, int H, int V,
-                                                                          int32_t* chunk_off, int32_t* chunk_seq, int rankers, PackedOut out) {
+                                                                          int32_t* chunk_off, int32_t* chunk_seq, int rankers, PackedOut out, SegSlot* seg_tab, int slots) {
     constexpr int LONG_SEQ = 64, LONG_LIST = 512;
     __shared__ long long strip[2][TABLE_THREADS];
     __shared__ __attribute__((aligned(16))) int32_t len[ORDER_MAX_N];
@@ -162,7 +203,7 @@ __global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const 
     }
     __shared__ ShareLds sh;
     if (N <= FEW_SEQS) {
-        few_table(blockIdx.x, cu, N, T, nch, H, V, chunk_off, chunk_seq, sh, t, TABLE_THREADS);
+        few_table(blockIdx.x, cu, N, T, nch, H, V, chunk_off, chunk_seq, sh, t, TABLE_THREADS, seg_tab, slots);
         return;
     }
     if (blockIdx.x > 0) {
@@ -751,11 +792,12 @@ hipError_t launch_clear_uncovered(const int64_t* cu, int N, int T, const PackedO
     hipLaunchKernelGGL(clear_uncovered_kernel, dim3(clearers), dim3(TABLE_THREADS), 0, stream, cu, N, T, out);
     return hipGetLastError();
 }
-hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int H, int V, int32_t* chunk_off, int32_t* chunk_seq,
-                              const PackedOut& out, hipStream_t stream) {
+hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int H, int V, int32_t* chunk_off, int32_t* chunk_seq, const PackedOut& out,
+                              SegSlot* seg_tab, int slots, hipStream_t stream) {
+    if (seg_tab && N > FEW_SEQS) return hipErrorInvalidValue;
     const int rankers = N <= ORDER_MAX_N ? (N + TABLE_THREADS - 1) / TABLE_THREADS : 0, clearers = clearing_workgroups(N, T, out);
     hipLaunchKernelGGL(build_chunk_table_kernel, dim3(1 + rankers + clearers), dim3(TABLE_THREADS), 0, stream, cu, N, T, nch, H, V, chunk_off,
-                       chunk_seq, rankers, out);
+                       chunk_seq, rankers, out, seg_tab, slots);
     return hipGetLastError();
 }
 
