@@ -70,16 +70,16 @@ __device__ __forceinline__ void seg_range(const SeqTab& st, int n, int nseg, int
     seg_range(c0, c1, nseg, seg, s0, s1);
 }
 
-// The sequence and segment of a workgroup (y, z: its place in the grid), how many segments the sequence has, the chunks of this one, and the record of the first one for head h.
-// False: there are fewer segments than slots.  (All scalars: see the note on `scale` in fused_replay.)
+// The sequence and segment of a workgroup (y, z: its place in the grid), how many segments the sequence has, and the record of the first one for head h; with TAB the chunks too.
+// False: there are fewer segments than slots.  (All scalars: see the note on `scale` in fused_replay.)  TAB: by the slots of seg_tab.  Kernels of their own, since one that looks which
+// way it is spills 31 scalars instead of 12: forward pass of 4 x 2048 tokens 66.3 -> 67.4 us.
 struct FusedSeg { int n, seg, count, s0, s1; int64_t rec0; };
-template <typename T> __device__ __forceinline__ bool fused_seg(const FusedArgs<T>& a, int y, int z, int h, FusedSeg& f) {
-    if (a.seg_tab == nullptr) {
+template <bool TAB, typename T> __device__ __forceinline__ bool fused_seg(const FusedArgs<T>& a, int y, int z, int h, FusedSeg& f) {
+    if constexpr (!TAB) {
         f.n = scan_sequence(a.c.st, z);
         f.seg = y;
         f.count = a.nseg;
         f.rec0 = ((int64_t)f.n * a.c.H + h) * a.nseg;
-        seg_range(a.c.st, f.n, a.nseg, y, f.s0, f.s1);
         return true;
     }
     const int4 x = *reinterpret_cast<const int4*>(a.seg_tab + y);
@@ -1456,16 +1456,17 @@ __device__ __forceinline__ void fused_consumer_rev(const FusedArgs<T>& a, char* 
 
 // ---- the kernel ------------------------------------------------------------------------------------------------------
 // grid = (H, nseg, N), or (H, slots, 1); block = 64 (V/16 + 2 FNP): waves 0 .. V/16-1 consume, the rest produce in pairs
-template <typename T, bool GKF32, int K, int V, int MODE, bool HD>
+template <typename T, bool GKF32, int K, int V, int MODE, bool HD, bool TAB>
 __global__ __launch_bounds__(64 * (V / 16 + 2 * FNP)) void fused_kernel(FusedArgs<T> a) {
     typedef FusedLds<T, K, V, MODE> L;
     __shared__ __attribute__((aligned(16))) char smem[L::BYTES];
     const int h = blockIdx.x;
-    FusedSeg fs;
-    if (!fused_seg(a, blockIdx.y, blockIdx.z, h, fs)) return;
+    FusedSeg fs{};
+    if (!fused_seg<TAB>(a, blockIdx.y, blockIdx.z, h, fs)) return;
     const int n = fs.n, seg = fs.seg;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int s0 = fs.s0, s1 = fs.s1;
+    int s0 = fs.s0, s1 = fs.s1;
+    if constexpr (!TAB) seg_range(a.c.st, n, fs.count, seg, s0, s1);
     // an empty segment leaves nothing behind (whoever chains the segments skips it), except that the first one of an
     // empty sequence still passes the state through
     if (s1 <= s0 && seg > 0) return;
@@ -1495,7 +1496,7 @@ __global__ __launch_bounds__(64 * (V / 16 + 2 * FNP)) void fused_kernel(FusedArg
 // where requests for 16 rows had met 16 cache lines each; those two read and o written are 9 at copy rate.
 constexpr int FIXUP_PARTS = 2;                            // workgroups that share one segment's chunks (measured: 1, 2, 4 -> 12.8, 12.8, 16.0 us)
 constexpr int FIXUP_STAGE = 3;                            // chain steps whose records are in LDS at a time
-template <typename T, int K, int V>
+template <typename T, int K, int V, bool TAB>
 __global__ __launch_bounds__(256) void fixup_kernel(FusedArgs<T> a) {
     constexpr int KT = K / 16, VT = V / 16, NB = 2, NQ = KT * KT / 4;
     static_assert(VT == 4 && KT == 4 && sizeof(T) == 2, "one column block per wave, a quarter of a transition record per wave");
@@ -1506,16 +1507,16 @@ __global__ __launch_bounds__(256) void fixup_kernel(FusedArgs<T> a) {
     const ChunkArgs<T>& p = a.c;
     const int h = blockIdx.x;
     const int part = (int)blockIdx.y % FIXUP_PARTS;
-    FusedSeg fs;
-    if (!fused_seg(a, (int)blockIdx.y / FIXUP_PARTS, blockIdx.z, h, fs)) return;
+    FusedSeg fs{};
+    if (!fused_seg<TAB>(a, (int)blockIdx.y / FIXUP_PARTS, blockIdx.z, h, fs)) return;
     const int n = fs.n, nseg = fs.count, target = fs.seg == 0 ? nseg : fs.seg;   // chain segments 0 .. target-1
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l = lane_id(), g = l >> 4, c = l & 15;
     const int H = p.H, vt = wv;
     int s0 = 0, s1 = 0;
     if (target < nseg) {
-        s0 = fs.s0;
-        s1 = fs.s1;
+        if constexpr (TAB) { s0 = fs.s0; s1 = fs.s1; }
+        else seg_range(p.st, n, nseg, target, s0, s1);
         // this workgroup's share of the segment's chunks
         const int per = (s1 - s0 + FIXUP_PARTS - 1) / FIXUP_PARTS;
         s0 = min(s0 + part * per, s1);
