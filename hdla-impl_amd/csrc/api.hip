@@ -566,7 +566,7 @@ int run_fused(const hdla_dims* d, bool fwd, const void* q, const void* k, const 
     if (d->cu_seqlens && (stages & HDLA_STAGE_PREP)) {
         e = launch_chunk_table(d->cu_seqlens, d->N, d->T, L.nch, d->H, 0, reinterpret_cast<int32_t*>(base + L.CHUNK_OFF),
                                reinterpret_cast<int32_t*>(base + L.CHUNK_SEQ), packed_outputs(d, a),
-                               L.slots ? reinterpret_cast<SegSlot*>(base + L.SEG_TAB) : nullptr, L.slots, stream);
+                               L.slots ? reinterpret_cast<SegSlot*>(base + L.SEG_TAB) : nullptr, L.nseg, stream);
         if (e != hipSuccess) return (int)e;
     }
     if (fwd) {

@@ -110,50 +110,51 @@ __device__ __forceinline__ int share_device(ShareLds& sh, int N, int H, int V, i
     }
     return codes;
 }
-// Time segments by length (fused route): `slots` of them for N sequences, each sequence as many as make the longest segment as short as can be, of SHARE_SEGMENT_CHUNKS chunks at the
-// least (a sequence's last one may be shorter).  A wave, a lane a sequence.  Equal numbers wait for the longest sequence's: 16 heads, K = V = 64, sequences of 4100, 1500, 2000 and 592
-// tokens, us, forward pass 123 -> 86, training step 364 -> 287; of 300, 700, 2500, 200, 1300, 1000 tokens (HDLA parameterisation) 145 -> 89, 351 -> 243; 8 heads, of 2600, 1000 and 400
-// tokens 59.6 -> 54.1, 145 -> 138; 32 heads, of 5000, 2000, 2500 and 500 tokens, training step 937 -> 777; equal lengths get equal numbers, in the same time (a slot says its
-// chunks itself: one round of loads at a kernel's start; with a table of the sequences instead training on 4 x 2048 tokens took 276 against 272).
+// Time segments by length (fused route): of N nseg in all each sequence gets as many as make the longest segment as short as can be, of SHARE_SEGMENT_CHUNKS chunks at the least (a
+// sequence's last one may be shorter), or nseg where that makes it no shorter.  Each wave by itself, a lane a sequence, then a thread a slot.  Equal numbers wait for the longest sequence's: 16 heads, K = V = 64, sequences
+// of 4100, 1500, 2000 and 592 tokens, us, forward pass 123 -> 87, training step 358 -> 285; of 300, 700, 2500, 200, 1300, 1000 tokens (HDLA parameterisation) 145 -> 89, 351 -> 242; 8 heads, of
+// 2600, 1000 and 400 tokens 59.8 -> 54.6, 146 -> 137; 32 heads, of 5000, 2000, 2500 and 500 tokens, training step 934 -> 770.  A slot says its chunks itself: one round of loads at a kernel's
+// start (with a table of the sequences instead training on 4 x 2048 tokens took 276 against 272).  Equal and nearly equal lengths pay for the look: forward pass of 8 sequences of 256 tokens
+// 26.0 -> 26.1, two of 2048 of 2 heads 42.2 -> 42.7, of 1824 and 1597 of 12 heads 48.3 -> 48.7 (searched with divisions, each lane writing its sequence's slots: 43.0, 49.2).
 constexpr int SHARE_SEGMENT_CHUNKS = 8, SHARE_SEGMENTS = 64;
-__device__ __forceinline__ void share_segments(const FewSeqs& f, int N, int slots, SegSlot* seg_tab) {
-    const int n = lane_id();
-    const unsigned own = n < N ? f.chunks : 0, cap = max(1u, min((unsigned)SHARE_SEGMENTS, own / SHARE_SEGMENT_CHUNKS));
-    auto of_length = [&](unsigned len) __attribute__((always_inline)) { return n < N ? (int)min(cap, max(1u, (own + len - 1) / len)) : 0; };
+__device__ __forceinline__ void share_segments(const FewSeqs& f, int N, int nseg, SegSlot* seg_tab, int t, int threads) {
+    const int n = lane_id(), slots = N * nseg;
+    const float own = n < N ? (float)f.chunks : 0.f, all = (float)of_lane(f.end, 63);
+    const int cap = max(1, min(SHARE_SEGMENTS, (int)(own * (1.f / SHARE_SEGMENT_CHUNKS))));
+    // (a / b rounded up; a hair less is as good: what counts is that the segments are no more than there are slots)
+    auto ratio = [](float a, float b) __attribute__((always_inline)) { return (int)ceilf(a * __builtin_amdgcn_rcpf(b) * (1.f - 1e-6f)); };
+    auto of_length = [&](int len) __attribute__((always_inline)) { return n < N ? min(cap, max(1, ratio(own, (float)len))) : 0; };
     auto ends = [](int x) __attribute__((always_inline)) { return sum_lanes(x, 0x3fffffff); };
-    // Segments of hi chunks are few enough in the end (a sequence of at most hi chunks has one, and slots >= N), of lo not or needlessly short.
-    const unsigned all = of_lane(ends((int)own), 63);
-    unsigned hi = max((unsigned)SHARE_SEGMENT_CHUNKS, (all + slots - 1) / (unsigned)slots), lo = hi - 1;
-    int mine = of_length(hi), end = ends(mine);
-    while (of_lane(end, 63) > slots) {
-        lo = hi;
-        hi *= 2;
-        mine = of_length(hi);
-        end = ends(mine);
-    }
-    while (hi - lo > 1) {
-        const unsigned mid = lo + (hi - lo) / 2;
-        const int m = of_length(mid), e = ends(m);
-        if (of_lane(e, 63) > slots) {
-            lo = mid;
-        } else {
-            hi = mid;
+    int mine = nseg, end = min(n + 1, N) * nseg;
+    // Segments of hi chunks are few enough: they are at most all / hi + N, and slots > N.  Of lo there would be too many, or it is too short.
+    int lo = max(SHARE_SEGMENT_CHUNKS, ratio(all, (float)slots)) - 1, hi = max(lo + 1, ratio(all, (float)(slots - N)));
+    if (__ballot(own > (float)(lo + 1) * nseg)) {
+        while (hi - lo > 1) {
+            const int mid = lo + (hi - lo) / 2;
+            if (of_lane(ends(of_length(mid)), 63) > slots) lo = mid;
+            else hi = mid;
+        }
+        const int m = of_length(hi), e = ends(m);
+        if (__ballot(own > (float)hi * nseg) && of_lane(e, 63) <= slots) {
             mine = m;
             end = e;
         }
     }
-    const int before = __shfl_up(f.end, 1), c0 = n == 0 ? 0 : before, first = end - mine;
-    for (int s = 0; n < N && s < mine; ++s) {
-        SegSlot x{n | s << 8 | mine << 16, first, 0, 0};
-        seg_range(c0, f.end, mine, s, x.s0, x.s1);
-        seg_tab[first + s] = x;
+    const int c0 = __builtin_amdgcn_update_dpp(0, f.end, 0x138, 0xf, 0xf, false);                 // (wave_shr:1)
+    for (int y0 = 0; y0 < slots; y0 += threads) {
+        const int y = y0 + t;
+        int k = 0;
+        for (int m = 0; m < N; ++m) k += of_lane(end, m) <= y;
+        const int from = min(k, N - 1), count = __shfl(mine, from), first = __shfl(end, from) - count, b0 = __shfl(c0, from), b1 = __shfl(f.end, from);
+        SegSlot x{k | (y - first) << 8 | count << 16, first, 0, 0};
+        seg_range(b0, b1, count, y - first, x.s0, x.s1);
+        if (y < slots) seg_tab[y] = k < N ? x : SegSlot{-1, 0, 0, 0};
     }
-    for (int i = of_lane(end, 63) + n; i < slots; i += 64) seg_tab[i] = SegSlot{-1, 0, 0, 0};
 }
 // A table of at most FEW_SEQS sequences, in registers: work 0 writes chunk_off and chunk_seq, work 1 ranks the sequences (V: as in
 // launch_chunk_table).  All threads of a workgroup, at least a wave, each wave for itself but for the widths.
 __device__ __forceinline__ void few_table(int work, const int64_t* cu, int N, int T, int nch, int H, int V, int32_t* chunk_off, int32_t* chunk_seq,
-                                          ShareLds& sh, int t, int threads, SegSlot* seg_tab = nullptr, int slots = 0) {
+                                          ShareLds& sh, int t, int threads, SegSlot* seg_tab = nullptr, int nseg = 0) {
     const FewSeqs f = few_seqs(cu, N, T, nch);
     if (work == 0) {
         if (t < N) chunk_off[t + 1] = f.end;
@@ -167,7 +168,7 @@ __device__ __forceinline__ void few_table(int work, const int64_t* cu, int N, in
     }
     int32_t* const order = chunk_off + N + 1;
     const int n = lane_id();
-    if (seg_tab && t >> 6 == 1) share_segments(f, N, slots, seg_tab);   // (beside the ranking)
+    if (seg_tab) share_segments(f, N, nseg, seg_tab, t, threads);
     int r = 0;
     for (int m = 0; m < N; ++m) {
         const int other = of_lane(f.chunks, m);
@@ -185,7 +186,7 @@ __device__ __forceinline__ void few_table(int work, const int64_t* cu, int N, in
     if (t < N) order[t] = sh.seq[t] | codes;
 }
 __global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const int64_t* cu, int N, int T, int nch, int H, int V,
-                                                                          int32_t* chunk_off, int32_t* chunk_seq, int rankers, PackedOut out, SegSlot* seg_tab, int slots) {
+                                                                          int32_t* chunk_off, int32_t* chunk_seq, int rankers, PackedOut out, SegSlot* seg_tab, int nseg) {
     constexpr int LONG_SEQ = 64, LONG_LIST = 512;
     __shared__ long long strip[2][TABLE_THREADS];
     __shared__ __attribute__((aligned(16))) int32_t len[ORDER_MAX_N];
@@ -203,7 +204,7 @@ __global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const 
     }
     __shared__ ShareLds sh;
     if (N <= FEW_SEQS) {
-        few_table(blockIdx.x, cu, N, T, nch, H, V, chunk_off, chunk_seq, sh, t, TABLE_THREADS, seg_tab, slots);
+        few_table(blockIdx.x, cu, N, T, nch, H, V, chunk_off, chunk_seq, sh, t, TABLE_THREADS, seg_tab, nseg);
         return;
     }
     if (blockIdx.x > 0) {
@@ -793,11 +794,11 @@ hipError_t launch_clear_uncovered(const int64_t* cu, int N, int T, const PackedO
     return hipGetLastError();
 }
 hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int H, int V, int32_t* chunk_off, int32_t* chunk_seq, const PackedOut& out,
-                              SegSlot* seg_tab, int slots, hipStream_t stream) {
+                              SegSlot* seg_tab, int nseg, hipStream_t stream) {
     if (seg_tab && N > FEW_SEQS) return hipErrorInvalidValue;
     const int rankers = N <= ORDER_MAX_N ? (N + TABLE_THREADS - 1) / TABLE_THREADS : 0, clearers = clearing_workgroups(N, T, out);
     hipLaunchKernelGGL(build_chunk_table_kernel, dim3(1 + rankers + clearers), dim3(TABLE_THREADS), 0, stream, cu, N, T, nch, H, V, chunk_off,
-                       chunk_seq, rankers, out, seg_tab, slots);
+                       chunk_seq, rankers, out, seg_tab, nseg);
     return hipGetLastError();
 }
 

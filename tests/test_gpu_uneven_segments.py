@@ -18,7 +18,7 @@ DEV = "cuda"
 # 64 sequences, most of them empty, and 65, which are cut in equal numbers; lengths of whole chunks and of a token more or less.
 CUTS = [
     (2, (0, 4100, 5600, 7600, 8192)), (3, (0, 300, 1000, 3500, 3700)), (4, (0, 0, 17, 1500, 1500, 1501, 2100, 2100)), (2, (5, 2300, 2310, 2900)), (1, (0, 10000, 10016)),
-    (1, (0, 257, 514, 770)), (16, (0, 2000, 2047, 3000)), (1, (0, 16, 33, 1040, 1600)), (1, tuple([0] * 40 + [9000, 9600] + [17000] * 23)), (1, tuple([0] * 41 + [9000, 9600] + [17000] * 23)),
+    (1, (0, 257, 514, 770)), (16, (0, 2000, 2047, 3000)), (12, (0, 1597, 3421)), (1, (0, 16, 33, 1040, 1600)), (1, tuple([0] * 40 + [9000, 9600] + [17000] * 23)), (1, tuple([0] * 41 + [9000, 9600] + [17000] * 23)),
 ]
 
 
@@ -29,7 +29,8 @@ def _chunk_segments(cu, slots):
     length = max(8, -(-sum(chunks) // slots))
     while sum(of(length)) > slots:
         length += 1
-    return of(length)
+    even = slots // len(chunks)
+    return of(length) if max(chunks) > length * even else [even] * len(chunks)
 
 
 @pytest.mark.parametrize("gk", [torch.bfloat16, torch.float32])
