@@ -75,6 +75,14 @@ template <typename T, bool GKF32, int K, int V, bool HD> constexpr int cg_waves(
     return small ? 3 : 2;
 }
 
+// x y + u v and x y - u v of the body's text.  Of the two products one is rounded by itself and the other added to it in one step: which, the compiler would decide by what stands
+// around them, in each kernel that has the text by itself.  FIRST: x y is the rounded one.  (4-byte elements: one kernel a shape, as it is compiled.)
+template <bool FIRST> __device__ __forceinline__ f32x4 sum_of_two(f32x4 x, f32x4 y, f32x4 u, f32x4 v) {
+    return FIRST ? __builtin_elementwise_fma(u, v, x * y) : __builtin_elementwise_fma(x, y, u * v);
+}
+#define CG_SUM(FIRST, x, y, u, v) (sizeof(T) == 4 ? x * y + u * v : sum_of_two<FIRST>(x, y, u, v))
+#define CG_DIFF(FIRST, x, y, u, v) (sizeof(T) == 4 ? x * y - u * v : sum_of_two<FIRST>(x, y, -(u), v))
+
 template <typename T, bool GKF32, int K, int V, bool HD>
 __device__ __forceinline__ void chunk_grad_strong_pair(const ChunkArgs<T>& p, int cid, int h, char* smem) {
 #define CG_STRONG 1
