@@ -176,10 +176,10 @@ def measured_traffic(workload, kernel_key, K, V):
     for k, rec in table.items():
         targs = [a.strip() for a in k[k.index("<") + 1:k.rindex(">")].split(",")] if "<" in k else []
         if fused_mode is not None or name == "fixup":
-            # fused_kernel<T, GKF32, K, V, MODE (0 forward, 1 summary, 2 checkpoint, 3 reverse), HD, TAB>, fixup_kernel<T, K, V, TAB>
+            # fused_kernel<T, GKF32, K, V, MODE (0 forward, 1 summary, 2 checkpoint, 3 reverse), HD>, fixup_kernel<T, K, V>
             if name == "fixup" and k.startswith("fixup_kernel<") and targs[1:3] == [str(K), str(V)]:
                 return rec["hbm_bytes_per_launch"]
-            if fused_mode is not None and k.startswith("fused_kernel<") and targs[2:6] == [str(K), str(V), fused_mode, "false"] and targs[6:] in ([], ["false"]):
+            if fused_mode is not None and k.startswith("fused_kernel<") and targs[2:] == [str(K), str(V), fused_mode, "false"]:
                 return rec["hbm_bytes_per_launch"]
             continue
         # scan_out<K, V, NWC, KEPT> (the forward pass's scan), scan_grad<K, V, NWC> (both of the backward pass); of packed sequences that share

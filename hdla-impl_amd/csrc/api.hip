@@ -188,22 +188,13 @@ bool leaves_states(const hdla_dims* d) {
     return scan_segments(d, false) == 1 && scan_segments(d, true) == 1;
 }
 
-// Packed sequences: the same segments in all, shared out by the sequences' lengths on the device (share_segments, prep.hip), so that no long sequence is waited for by itself.  No more of
-// them in all than in equal numbers: what a boundary costs in precision is said at fused_segments.  (Errors against 32-bit inputs over those of equal numbers, nine batches of 2 to 6
-// sequences, 12 inputs each: outputs and gradients 0.00 +- 0.01 % to + 0.1 +- 0.03 %, where all 256 workgroups were shared out up to + 0.3 %; final states by where a sequence's last
-// boundary falls, - 0.02 to + 3 %: a sequence too short for a cut has those of the same sequence by itself.)  0: each sequence has the same number (one, or a number asked for; many sequences).
-int fused_slots(const hdla_dims* d) {
-    const int nseg = fused_segments(d);
-    return d->cu_seqlens && d->segments == 0 && nseg > 1 && d->N > 1 && d->N <= 64 ? d->N * nseg : 0;
-}
-
 struct FusedLayout {
     size_t OL, GW, SLOC, MSEG, RSEG, SIN, ERR;                 // fused kernels' own
     size_t HC, DHC, DVN, TM, UT, W, SUM, STRONG;               // what chunk_grad reads (backward pass; UT and W beside fp32 decays)
     size_t MT, AQ;                                             // and the rest of the record
-    size_t CHUNK_OFF, CHUNK_SEQ, SEG_TAB;
+    size_t CHUNK_OFF, CHUNK_SEQ;
     size_t total;
-    int nch, nseg, slots;
+    int nch, nseg;
 };
 constexpr int PASS_BWD_RECORD = -2;          // a backward pass that is given the record (hdla_record_workspace_bytes)
 int make_fused_layout(const hdla_dims* d, int pass, FusedLayout& L) {
@@ -216,7 +207,6 @@ int make_fused_layout(const hdla_dims* d, int pass, FusedLayout& L) {
     L = FusedLayout{};
     L.nch = (int)nch64;
     L.nseg = fused_segments(d);
-    L.slots = fused_slots(d);
     const size_t es = 2, K = d->K, V = d->V;
     const size_t chw = (size_t)d->H * (size_t)L.nch, recs = (size_t)d->N * d->H * L.nseg;
     size_t off = 0;
@@ -248,7 +238,6 @@ int make_fused_layout(const hdla_dims* d, int pass, FusedLayout& L) {
     if (d->cu_seqlens) {
         L.CHUNK_OFF = take((size_t)(2 * d->N + 1) * 4);
         L.CHUNK_SEQ = take((size_t)(L.nch > 0 ? L.nch : 1) * 4);
-        if (L.slots) L.SEG_TAB = take((size_t)L.slots * sizeof(SegSlot));
     }
     L.total = off;
     return HDLA_OK;
@@ -467,7 +456,7 @@ int run_chunk(const hdla_dims* d, int pass, const void* q, const void* k, const 
         const bool made = prep_makes_table(d->cu_seqlens, d->N, d->H, nch);
         if (d->cu_seqlens && !made) {
             e = launch_chunk_table(d->cu_seqlens, d->N, d->T, nch, d->H, share_V, const_cast<int32_t*>(a.st.chunk_off), const_cast<int32_t*>(a.st.chunk_seq),
-                                   out, nullptr, 0, stream);
+                                   out, stream);
             if (e != hipSuccess) return (int)e;
         }
         if (nch > 0) {
@@ -557,16 +546,13 @@ int run_fused(const hdla_dims* d, bool fwd, const void* q, const void* k, const 
     a.st.order = d->cu_seqlens ? a.st.chunk_off + d->N + 1 : nullptr;
     a.st.T = d->T; a.st.NT = (d->T + CHUNK - 1) / CHUNK; a.st.N = d->N; a.st.nch = L.nch;
     f.nseg = L.nseg;
-    f.slots = L.slots;
-    f.seg_tab = L.slots ? reinterpret_cast<const SegSlot*>(base + L.SEG_TAB) : nullptr;
     f.sloc = reinterpret_cast<float*>(base + L.SLOC); f.mseg = reinterpret_cast<float*>(base + L.MSEG);
     f.rseg = reinterpret_cast<float*>(base + L.RSEG);
     f.err = reinterpret_cast<int*>(base + L.ERR);
     hipError_t e;
     if (d->cu_seqlens && (stages & HDLA_STAGE_PREP)) {
         e = launch_chunk_table(d->cu_seqlens, d->N, d->T, L.nch, d->H, 0, reinterpret_cast<int32_t*>(base + L.CHUNK_OFF),
-                               reinterpret_cast<int32_t*>(base + L.CHUNK_SEQ), packed_outputs(d, a),
-                               L.slots ? reinterpret_cast<SegSlot*>(base + L.SEG_TAB) : nullptr, L.nseg, stream);
+                               reinterpret_cast<int32_t*>(base + L.CHUNK_SEQ), packed_outputs(d, a), stream);
         if (e != hipSuccess) return (int)e;
     }
     if (fwd) {

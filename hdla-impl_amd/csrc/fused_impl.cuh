@@ -70,30 +70,6 @@ __device__ __forceinline__ void seg_range(const SeqTab& st, int n, int nseg, int
     seg_range(c0, c1, nseg, seg, s0, s1);
 }
 
-// The sequence and segment of a workgroup (y, z: its place in the grid), how many segments the sequence has, and the record of the first one for head h; with TAB the chunks too.
-// False: there are fewer segments than slots.  (All scalars: see the note on `scale` in fused_replay.)  TAB: by the slots of seg_tab.  Kernels of their own, since one that looks which
-// way it is spills 31 scalars instead of 12: forward pass of 4 x 2048 tokens 66.3 -> 67.4 us.
-struct FusedSeg { int n, seg, count, s0, s1; int64_t rec0; };
-template <bool TAB, typename T> __device__ __forceinline__ bool fused_seg(const FusedArgs<T>& a, int y, int z, int h, FusedSeg& f) {
-    if constexpr (!TAB) {
-        f.n = scan_sequence(a.c.st, z);
-        f.seg = y;
-        f.count = a.nseg;
-        f.rec0 = ((int64_t)f.n * a.c.H + h) * a.nseg;
-        return true;
-    }
-    const int4 x = *reinterpret_cast<const int4*>(a.seg_tab + y);
-    const int code = uniform(x.x);
-    if (code < 0) return false;
-    f.n = code & 255;
-    f.seg = code >> 8 & 255;
-    f.count = code >> 16;
-    f.s0 = uniform(x.z);
-    f.s1 = uniform(x.w);
-    f.rec0 = (int64_t)uniform(x.y) * a.c.H + (int64_t)h * f.count;
-    return true;
-}
-
 // Columns 16 j + 4 g .. + 3 of row c of a chunk's G, in elements from its start: pieces of eight columns, the 16 rows of a piece side by side
 __device__ __forceinline__ int gw_at(int j, int g, int c) { return (j >> 1) * PAIR + ((2 * (j & 1) + (g >> 1)) * 16 + c) * 8 + 4 * (g & 1); }
 
@@ -1004,8 +980,7 @@ __device__ __forceinline__ void fused_replay(const FusedArgs<T>& a, char* smem, 
 //   rseg  [V/16][K/16] tiles  F(R^T), R = sum_t G_t^T do_t (checkpoint kernel, segments > 0)
 //   sin   [V/16][K/16] tiles  F(S_in^T): the state entering the segment (segments > 0)
 template <typename T, int K, int V, int MODE>
-__device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* smem, const FusedSeg& fs, int h, int s0, int s1, int wv) {
-    const int n = fs.n, seg = fs.seg;
+__device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* smem, int n, int h, int seg, int s0, int s1, int wv) {
     typedef FusedLds<T, K, V, MODE> L;
     constexpr bool FWD = MODE == FUSED_FWD;
     constexpr int KT = K / 16, VT = V / 16, KT2 = KT / 2;
@@ -1017,7 +992,7 @@ __device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* 
     const int H = p.H, vt = wv;
     const int nst = s1 - s0;
     const bool pblk = seg > 0;                            // uniform over the workgroup
-    const int64_t rec = fs.rec0 + seg;
+    const int64_t rec = ((int64_t)n * H + h) * a.nseg + seg;
     const int64_t soff = ((int64_t)n * H + h) * K * V + 16 * vt + c;
 
     // state block: lane (g,c) reg i of tile kt = S[16kt + 4g + i][16vt + c]; likewise M with column 16vt + c
@@ -1165,8 +1140,7 @@ __device__ __forceinline__ void fused_consumer_fwd(const FusedArgs<T>& a, char* 
 // W_GLOBAL: chunk_grad reads u and w from the workspace where it cannot rebuild them (chunk_grad_body.inc: REBUILD_W).  (With the HDLA
 // parameterisation it rebuilds them too, from the sums over channels that the producers leave.)
 template <typename T, int K, int V, bool W_GLOBAL>
-__device__ __forceinline__ void fused_consumer_ckpt(const FusedArgs<T>& a, char* smem, const FusedSeg& fs, int h, int s0, int s1, int wv) {
-    const int n = fs.n, seg = fs.seg;
+__device__ __forceinline__ void fused_consumer_ckpt(const FusedArgs<T>& a, char* smem, int n, int h, int seg, int s0, int s1, int wv) {
     typedef FusedLds<T, K, V, FUSED_CKPT> L;
     constexpr int KT = K / 16, VT = V / 16, KT2 = KT / 2;
     static_assert(KT == VT, "consumer j owns column block j of the state and of G");
@@ -1177,7 +1151,7 @@ __device__ __forceinline__ void fused_consumer_ckpt(const FusedArgs<T>& a, char*
     const int H = p.H, vt = wv;
     const int nst = s1 - s0;
     const bool later = seg > 0;                           // uniform over the workgroup
-    const int64_t rec = fs.rec0 + seg;
+    const int64_t rec = ((int64_t)n * H + h) * a.nseg + seg;
     const int64_t soff = ((int64_t)n * H + h) * K * V + 16 * vt + c;
 
     f32x4 S[KT], R[VT];
@@ -1287,8 +1261,7 @@ __device__ __forceinline__ void fused_consumer_ckpt(const FusedArgs<T>& a, char*
 
 // ---- consumers, reverse direction ------------------------------------------------------------------------------------
 template <typename T, int K, int V>
-__device__ __forceinline__ void fused_consumer_rev(const FusedArgs<T>& a, char* smem, const FusedSeg& fs, int h, int s0, int s1, int wv) {
-    const int n = fs.n, seg = fs.seg;
+__device__ __forceinline__ void fused_consumer_rev(const FusedArgs<T>& a, char* smem, int n, int h, int seg, int s0, int s1, int wv) {
     typedef FusedLds<T, K, V, FUSED_REV> L;
     constexpr int KT = K / 16, VT = V / 16, KT2 = KT / 2;
     constexpr SlotB B = L::SB;
@@ -1322,15 +1295,15 @@ __device__ __forceinline__ void fused_consumer_rev(const FusedArgs<T>& a, char* 
         int sMo = L::CHAIN + 4 * l * (int)sizeof(T);
         asm volatile("" : "+v"(sMo));
         T* const sM = reinterpret_cast<T*>(smem + sMo);
-        const int64_t rec0 = fs.rec0;
-        int batch = 0, s = fs.count - 1;
+        const int64_t rec0 = ((int64_t)n * H + h) * a.nseg;
+        int batch = 0, s = a.nseg - 1;
         while (s > seg) {
             int step[STG], ns = 0, q0, q1;
 #pragma unroll
             for (int b = 0; b < STG; ++b) {
                 step[b] = 0;
                 while (s > seg) {
-                    seg_range(p.st, n, fs.count, s, q0, q1);
+                    seg_range(p.st, n, a.nseg, s, q0, q1);
                     if (q1 > q0) break;
                     --s;
                 }
@@ -1455,27 +1428,25 @@ __device__ __forceinline__ void fused_consumer_rev(const FusedArgs<T>& a, char* 
 }
 
 // ---- the kernel ------------------------------------------------------------------------------------------------------
-// grid = (H, nseg, N), or (H, slots, 1); block = 64 (V/16 + 2 FNP): waves 0 .. V/16-1 consume, the rest produce in pairs
-template <typename T, bool GKF32, int K, int V, int MODE, bool HD, bool TAB>
+// grid = (H, nseg, N); block = 64 (V/16 + 2 FNP): waves 0 .. V/16-1 consume, the rest produce in pairs
+template <typename T, bool GKF32, int K, int V, int MODE, bool HD>
 __global__ __launch_bounds__(64 * (V / 16 + 2 * FNP)) void fused_kernel(FusedArgs<T> a) {
     typedef FusedLds<T, K, V, MODE> L;
     __shared__ __attribute__((aligned(16))) char smem[L::BYTES];
-    const int h = blockIdx.x;
-    FusedSeg fs{};
-    if (!fused_seg<TAB>(a, blockIdx.y, blockIdx.z, h, fs)) return;
-    const int n = fs.n, seg = fs.seg;
+    const int h = blockIdx.x, seg = blockIdx.y;
+    const int n = scan_sequence(a.c.st, blockIdx.z);
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    int s0 = fs.s0, s1 = fs.s1;
-    if constexpr (!TAB) seg_range(a.c.st, n, fs.count, seg, s0, s1);
+    int s0, s1;
+    seg_range(a.c.st, n, a.nseg, seg, s0, s1);
     // an empty segment leaves nothing behind (whoever chains the segments skips it), except that the first one of an
     // empty sequence still passes the state through
     if (s1 <= s0 && seg > 0) return;
     if (threadIdx.x < 32) reinterpret_cast<int*>(smem + L::FLAGS)[threadIdx.x] = 0;
     __syncthreads();
     if (wv < V / 16) {
-        if constexpr (MODE == FUSED_REV) fused_consumer_rev<T, K, V>(a, smem, fs, h, s0, s1, wv);
-        else if constexpr (MODE == FUSED_CKPT) fused_consumer_ckpt<T, K, V, GKF32>(a, smem, fs, h, s0, s1, wv);
-        else fused_consumer_fwd<T, K, V, MODE>(a, smem, fs, h, s0, s1, wv);
+        if constexpr (MODE == FUSED_REV) fused_consumer_rev<T, K, V>(a, smem, n, h, seg, s0, s1, wv);
+        else if constexpr (MODE == FUSED_CKPT) fused_consumer_ckpt<T, K, V, GKF32>(a, smem, n, h, seg, s0, s1, wv);
+        else fused_consumer_fwd<T, K, V, MODE>(a, smem, n, h, seg, s0, s1, wv);
     } else {
         const int pp = (wv - V / 16) >> 1, half = (wv - V / 16) & 1;
         if constexpr (L::SOLVES) fused_producer<T, GKF32, K, V, MODE, HD>(a, smem, n, h, seg, s0, s1, pp, half);
@@ -1484,7 +1455,7 @@ __global__ __launch_bounds__(64 * (V / 16 + 2 * FNP)) void fused_kernel(FusedArg
 }
 
 // ---- forward pass, second kernel: the true entering states, and their part of the output ----------------------------
-// grid = (H, nseg * FIXUP_PARTS, N), or (H, slots * FIXUP_PARTS, 1), 256 threads.  blockIdx.y / FIXUP_PARTS = s in 1 .. nseg-1: segment s (chain the
+// grid = (H, nseg * FIXUP_PARTS, N), 256 threads.  blockIdx.y / FIXUP_PARTS = s in 1 .. nseg-1: segment s (chain the
 // records of segments 0 .. s-1 into S_in(s), keep it as the boundary record, add G S_in(s) to the segment's local
 // outputs); 0: the final state (all segments chained).  The kernel is a chain of dependent steps between two launches,
 // so everything is arranged for its latency: all loads that do not depend on the chain are issued at the start (the
@@ -1496,7 +1467,7 @@ __global__ __launch_bounds__(64 * (V / 16 + 2 * FNP)) void fused_kernel(FusedArg
 // where requests for 16 rows had met 16 cache lines each; those two read and o written are 9 at copy rate.
 constexpr int FIXUP_PARTS = 2;                            // workgroups that share one segment's chunks (measured: 1, 2, 4 -> 12.8, 12.8, 16.0 us)
 constexpr int FIXUP_STAGE = 3;                            // chain steps whose records are in LDS at a time
-template <typename T, int K, int V, bool TAB>
+template <typename T, int K, int V>
 __global__ __launch_bounds__(256) void fixup_kernel(FusedArgs<T> a) {
     constexpr int KT = K / 16, VT = V / 16, NB = 2, NQ = KT * KT / 4;
     static_assert(VT == 4 && KT == 4 && sizeof(T) == 2, "one column block per wave, a quarter of a transition record per wave");
@@ -1506,24 +1477,22 @@ __global__ __launch_bounds__(256) void fixup_kernel(FusedArgs<T> a) {
     __shared__ __attribute__((aligned(16))) T sM[FIXUP_STAGE][2][KT * KT * TILE];   // transition records, hi and lo halves
     const ChunkArgs<T>& p = a.c;
     const int h = blockIdx.x;
-    const int part = (int)blockIdx.y % FIXUP_PARTS;
-    FusedSeg fs{};
-    if (!fused_seg<TAB>(a, (int)blockIdx.y / FIXUP_PARTS, blockIdx.z, h, fs)) return;
-    const int n = fs.n, nseg = fs.count, target = fs.seg == 0 ? nseg : fs.seg;   // chain segments 0 .. target-1
+    const int n = scan_sequence(p.st, blockIdx.z);
+    const int ty = (int)blockIdx.y / FIXUP_PARTS, part = (int)blockIdx.y % FIXUP_PARTS;
+    const int target = ty == 0 ? a.nseg : ty;                            // chain segments 0 .. target-1
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l = lane_id(), g = l >> 4, c = l & 15;
     const int H = p.H, vt = wv;
     int s0 = 0, s1 = 0;
-    if (target < nseg) {
-        if constexpr (TAB) { s0 = fs.s0; s1 = fs.s1; }
-        else seg_range(p.st, n, nseg, target, s0, s1);
+    if (target < a.nseg) {
+        seg_range(p.st, n, a.nseg, target, s0, s1);
         // this workgroup's share of the segment's chunks
         const int per = (s1 - s0 + FIXUP_PARTS - 1) / FIXUP_PARTS;
         s0 = min(s0 + part * per, s1);
         s1 = min(s0 + per, s1);
         if (s1 <= s0 || (part > 0 && !a.ol)) return;
     } else if (!p.ht || part > 0) return;
-    const int64_t rec0 = fs.rec0;
+    const int64_t rec0 = ((int64_t)n * H + h) * a.nseg;
     const int64_t soff = ((int64_t)n * H + h) * K * V + 16 * vt + c;
 
     int c0, c1;
@@ -1545,14 +1514,14 @@ __global__ __launch_bounds__(256) void fixup_kernel(FusedArgs<T> a) {
             for (int j = 0; j < VT; ++j) OLr[b][j] = *reinterpret_cast<const f32x4*>(ol + j * TILE);
         }
     };
-    const bool outputs = target < nseg && a.ol != nullptr;
+    const bool outputs = target < a.nseg && a.ol != nullptr;
     if (outputs) request(s0 + wv);
 
     // S[kt]: lane (g,c) reg i = S[16kt + 4g + i][16vt + c].  Segment 0 ran from the initial state itself; only where it
     // is empty does the chain start from the initial state here.
     f32x4 S[KT];
     int q0, q1;
-    seg_range(p.st, n, nseg, 0, q0, q1);
+    seg_range(p.st, n, a.nseg, 0, q0, q1);
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) {
         if (q1 > q0) {
@@ -1573,7 +1542,7 @@ __global__ __launch_bounds__(256) void fixup_kernel(FusedArgs<T> a) {
         for (int b = 0; b < FIXUP_STAGE; ++b) {
             step[b] = 0;
             while (s < target) {
-                seg_range(p.st, n, nseg, s, q0, q1);
+                seg_range(p.st, n, a.nseg, s, q0, q1);
                 if (q1 > q0) break;
                 ++s;
             }
@@ -1628,7 +1597,7 @@ __global__ __launch_bounds__(256) void fixup_kernel(FusedArgs<T> a) {
             }
         }
     }
-    if (target == nseg) {
+    if (target == a.nseg) {
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll

@@ -27,10 +27,6 @@ struct FusedArgs {
     T* gw;                 // [H][nch][K/8][16][8]  G of segments > 0 (the forward pass's fixup_kernel needs it as well)
     T* aq;                 // [H][nch][2][2 tiles]  A_ak, A_qb
     int* err;              // set nonzero by a wave whose bounded wait ran out
-    // packed sequences whose segments go by their lengths (share_segments, prep.hip), `slots` = N nseg at most; null: nseg each.  Of the records a sequence then has
-    // its own number, those of a sequence and head side by side.
-    const SegSlot* seg_tab;
-    int slots;
 };
 
 // K = V = 64, 2-byte elements only; hipErrorInvalidValue otherwise

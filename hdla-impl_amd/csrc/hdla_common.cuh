@@ -452,21 +452,18 @@ struct FewSeqs {
 template <int CTRL, int ROWS> __device__ __forceinline__ int add_lanes(int x, int most) {
     return min(x + __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false), most);
 }
-// Lane n: the sum of lanes 0 .. n, no more than `most` (at most half of what an int holds)
-__device__ __forceinline__ int sum_lanes(int x, int most) {
-    x = add_lanes<0x111, 0xf>(min(x, most), most);    // row_shr:1
-    x = add_lanes<0x112, 0xf>(x, most);
-    x = add_lanes<0x114, 0xf>(x, most);
-    x = add_lanes<0x118, 0xf>(x, most);
-    x = add_lanes<0x142, 0xa>(x, most);               // row_bcast:15, into the second and the fourth row of lanes
-    return add_lanes<0x143, 0xc>(x, most);            // row_bcast:31, into the third and the fourth
-}
 __device__ __forceinline__ FewSeqs few_seqs(const int64_t* cu, int N, int T, int nch) {
     FewSeqs f;
     const int n = lane_id();
     packed_bounds(cu, min(n, N - 1), T, f.bos, f.eos);
     f.chunks = n < N ? (int)((f.eos - f.bos + CH - 1) / CH) : 0;
-    f.end = sum_lanes(f.chunks, nch);
+    f.end = min(f.chunks, nch);
+    f.end = add_lanes<0x111, 0xf>(f.end, nch);    // row_shr:1
+    f.end = add_lanes<0x112, 0xf>(f.end, nch);
+    f.end = add_lanes<0x114, 0xf>(f.end, nch);
+    f.end = add_lanes<0x118, 0xf>(f.end, nch);
+    f.end = add_lanes<0x142, 0xa>(f.end, nch);    // row_bcast:15, into the second and the fourth row of lanes
+    f.end = add_lanes<0x143, 0xc>(f.end, nch);    // row_bcast:31, into the third and the fourth
     return f;
 }
 __device__ __forceinline__ int of_lane(int x, int n) { return __builtin_amdgcn_readlane(x, n); }

@@ -15,9 +15,8 @@ struct PackedOut {
     void add(void* q, long long b) { if (q) { p[n] = q; row[n++] = b; } }
 };
 // (V: where a scan on the table is shared out by the sequences' lengths (scan_shares); else 0, and `order` holds no widths)
-// seg_tab, nseg: FusedArgs' (at most 64 sequences), or null
-hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int H, int V, int32_t* chunk_off, int32_t* chunk_seq, const PackedOut& out,
-                              SegSlot* seg_tab, int nseg, hipStream_t stream);
+hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int H, int V, int32_t* chunk_off, int32_t* chunk_seq,
+                              const PackedOut& out, hipStream_t stream);
 // only what clears the rows that belong to no sequence
 hipError_t launch_clear_uncovered(const int64_t* cu, int N, int T, const PackedOut& out, hipStream_t stream);
 

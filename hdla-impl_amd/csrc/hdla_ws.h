@@ -12,13 +12,6 @@ namespace hdla {
 
 struct bf16 { uint16_t x; };  // storage type tag for bf16 tensors (raw bits)
 
-// A time segment of packed sequences that are cut by their lengths (share_segments, prep.hip)
-struct alignas(16) SegSlot {
-    int32_t code;             // its sequence | which of its segments << 8 | how many it has << 16; negative: none
-    int32_t first;            // number of the sequence's first one
-    int32_t s0, s1;           // its chunks
-};
-
 // Tokens live on one flattened axis of B*T rows.  Without cu_seqlens sequence n covers rows [n*T, (n+1)*T) and
 // has NT = ceil(T/16) chunks; with cu_seqlens (device int64[N+1], batch 1) sequence n covers [cu[n], cu[n+1])
 // and its chunks are numbered from chunk_off[n] (device int32[N+1], built by build_chunk_table_kernel or prep_kernel, which leave

@@ -110,51 +110,10 @@ __device__ __forceinline__ int share_device(ShareLds& sh, int N, int H, int V, i
     }
     return codes;
 }
-// Time segments by length (fused route): of N nseg in all each sequence gets as many as make the longest segment as short as can be, of SHARE_SEGMENT_CHUNKS chunks at the least (a
-// sequence's last one may be shorter), or nseg where that makes it no shorter.  Each wave by itself, a lane a sequence, then a thread a slot.  Equal numbers wait for the longest sequence's: 16 heads, K = V = 64, sequences
-// of 4100, 1500, 2000 and 592 tokens, us, forward pass 123 -> 87, training step 358 -> 285; of 300, 700, 2500, 200, 1300, 1000 tokens (HDLA parameterisation) 145 -> 89, 351 -> 242; 8 heads, of
-// 2600, 1000 and 400 tokens 59.8 -> 54.6, 146 -> 137; 32 heads, of 5000, 2000, 2500 and 500 tokens, training step 934 -> 770.  A slot says its chunks itself: one round of loads at a kernel's
-// start (with a table of the sequences instead training on 4 x 2048 tokens took 276 against 272).  Equal and nearly equal lengths pay for the look: forward pass of 8 sequences of 256 tokens
-// 26.0 -> 26.1, two of 2048 of 2 heads 42.2 -> 42.7, of 1824 and 1597 of 12 heads 48.3 -> 48.7 (searched with divisions, each lane writing its sequence's slots: 43.0, 49.2).
-constexpr int SHARE_SEGMENT_CHUNKS = 8, SHARE_SEGMENTS = 64;
-__device__ __forceinline__ void share_segments(const FewSeqs& f, int N, int nseg, SegSlot* seg_tab, int t, int threads) {
-    const int n = lane_id(), slots = N * nseg;
-    const float own = n < N ? (float)f.chunks : 0.f, all = (float)of_lane(f.end, 63);
-    const int cap = max(1, min(SHARE_SEGMENTS, (int)(own * (1.f / SHARE_SEGMENT_CHUNKS))));
-    // (a / b rounded up; a hair less is as good: what counts is that the segments are no more than there are slots)
-    auto ratio = [](float a, float b) __attribute__((always_inline)) { return (int)ceilf(a * __builtin_amdgcn_rcpf(b) * (1.f - 1e-6f)); };
-    auto of_length = [&](int len) __attribute__((always_inline)) { return n < N ? min(cap, max(1, ratio(own, (float)len))) : 0; };
-    auto ends = [](int x) __attribute__((always_inline)) { return sum_lanes(x, 0x3fffffff); };
-    int mine = nseg, end = min(n + 1, N) * nseg;
-    // Segments of hi chunks are few enough: they are at most all / hi + N, and slots > N.  Of lo there would be too many, or it is too short.
-    int lo = max(SHARE_SEGMENT_CHUNKS, ratio(all, (float)slots)) - 1, hi = max(lo + 1, ratio(all, (float)(slots - N)));
-    if (__ballot(own > (float)(lo + 1) * nseg)) {
-        while (hi - lo > 1) {
-            const int mid = lo + (hi - lo) / 2;
-            if (of_lane(ends(of_length(mid)), 63) > slots) lo = mid;
-            else hi = mid;
-        }
-        const int m = of_length(hi), e = ends(m);
-        if (__ballot(own > (float)hi * nseg) && of_lane(e, 63) <= slots) {
-            mine = m;
-            end = e;
-        }
-    }
-    const int c0 = __builtin_amdgcn_update_dpp(0, f.end, 0x138, 0xf, 0xf, false);                 // (wave_shr:1)
-    for (int y0 = 0; y0 < slots; y0 += threads) {
-        const int y = y0 + t;
-        int k = 0;
-        for (int m = 0; m < N; ++m) k += of_lane(end, m) <= y;
-        const int from = min(k, N - 1), count = __shfl(mine, from), first = __shfl(end, from) - count, b0 = __shfl(c0, from), b1 = __shfl(f.end, from);
-        SegSlot x{k | (y - first) << 8 | count << 16, first, 0, 0};
-        seg_range(b0, b1, count, y - first, x.s0, x.s1);
-        if (y < slots) seg_tab[y] = k < N ? x : SegSlot{-1, 0, 0, 0};
-    }
-}
 // A table of at most FEW_SEQS sequences, in registers: work 0 writes chunk_off and chunk_seq, work 1 ranks the sequences (V: as in
 // launch_chunk_table).  All threads of a workgroup, at least a wave, each wave for itself but for the widths.
 __device__ __forceinline__ void few_table(int work, const int64_t* cu, int N, int T, int nch, int H, int V, int32_t* chunk_off, int32_t* chunk_seq,
-                                          ShareLds& sh, int t, int threads, SegSlot* seg_tab = nullptr, int nseg = 0) {
+                                          ShareLds& sh, int t, int threads) {
     const FewSeqs f = few_seqs(cu, N, T, nch);
     if (work == 0) {
         if (t < N) chunk_off[t + 1] = f.end;
@@ -168,7 +127,6 @@ __device__ __forceinline__ void few_table(int work, const int64_t* cu, int N, in
     }
     int32_t* const order = chunk_off + N + 1;
     const int n = lane_id();
-    if (seg_tab) share_segments(f, N, nseg, seg_tab, t, threads);
     int r = 0;
     for (int m = 0; m < N; ++m) {
         const int other = of_lane(f.chunks, m);
@@ -186,7 +144,7 @@ __device__ __forceinline__ void few_table(int work, const int64_t* cu, int N, in
     if (t < N) order[t] = sh.seq[t] | codes;
 }
 __global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const int64_t* cu, int N, int T, int nch, int H, int V,
-                                                                          int32_t* chunk_off, int32_t* chunk_seq, int rankers, PackedOut out, SegSlot* seg_tab, int nseg) {
+                                                                          int32_t* chunk_off, int32_t* chunk_seq, int rankers, PackedOut out) {
     constexpr int LONG_SEQ = 64, LONG_LIST = 512;
     __shared__ long long strip[2][TABLE_THREADS];
     __shared__ __attribute__((aligned(16))) int32_t len[ORDER_MAX_N];
@@ -204,7 +162,7 @@ __global__ __launch_bounds__(TABLE_THREADS) void build_chunk_table_kernel(const 
     }
     __shared__ ShareLds sh;
     if (N <= FEW_SEQS) {
-        few_table(blockIdx.x, cu, N, T, nch, H, V, chunk_off, chunk_seq, sh, t, TABLE_THREADS, seg_tab, nseg);
+        few_table(blockIdx.x, cu, N, T, nch, H, V, chunk_off, chunk_seq, sh, t, TABLE_THREADS);
         return;
     }
     if (blockIdx.x > 0) {
@@ -793,12 +751,11 @@ hipError_t launch_clear_uncovered(const int64_t* cu, int N, int T, const PackedO
     hipLaunchKernelGGL(clear_uncovered_kernel, dim3(clearers), dim3(TABLE_THREADS), 0, stream, cu, N, T, out);
     return hipGetLastError();
 }
-hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int H, int V, int32_t* chunk_off, int32_t* chunk_seq, const PackedOut& out,
-                              SegSlot* seg_tab, int nseg, hipStream_t stream) {
-    if (seg_tab && N > FEW_SEQS) return hipErrorInvalidValue;
+hipError_t launch_chunk_table(const int64_t* cu, int N, int T, int nch, int H, int V, int32_t* chunk_off, int32_t* chunk_seq,
+                              const PackedOut& out, hipStream_t stream) {
     const int rankers = N <= ORDER_MAX_N ? (N + TABLE_THREADS - 1) / TABLE_THREADS : 0, clearers = clearing_workgroups(N, T, out);
     hipLaunchKernelGGL(build_chunk_table_kernel, dim3(1 + rankers + clearers), dim3(TABLE_THREADS), 0, stream, cu, N, T, nch, H, V, chunk_off,
-                       chunk_seq, rankers, out, seg_tab, nseg);
+                       chunk_seq, rankers, out);
     return hipGetLastError();
 }
 

@@ -1,5 +1,6 @@
-"""Outputs and gradients of some calls of every kind of chunk_grad kernel (few pairs and many, common ones and flagged, decays of the inputs' type and fp32), bit for bit what they have been:
-which multiply is fused with which add is part of the kernels, and no matter of what else a file has or how it is compiled."""
+"""Outputs and gradients of some calls of every kind of chunk_grad kernel (few pairs and many, common ones and flagged, decays of the inputs' type and fp32) and of packed sequences on the
+fused route, bit for bit what they have been: which multiply is fused with which add and where a sequence is cut are part of the kernels, and no matter of what else a file has, how it is
+compiled or what a sequence is packed with."""
 import hashlib
 
 import pytest
@@ -24,6 +25,8 @@ CASES = [
     (("beta", "auto", BF, BF, 64, 64, 2, (256,), False), "410e8294307728a6"),
     (("beta", "fused", BF, BF, 64, 64, 16, (2048,), False), "8a4c0b87794f070b"),
     (("ab", "fused", BF, F32, 64, 64, 3, (700,), True), "ce98f932aee3720b"),
+    (("beta", "fused", BF, BF, 64, 64, 16, (2000, 17, 983), False), "e469513fe0726ae3"),
+    (("ab", "fused", BF, BF, 64, 64, 2, (48, 1200, 300, 5), True), "16e908c0b85e6754"),
     (("beta", "plain", F32, F32, 64, 64, 8, (501,), False), "254d916e912087e3"),
     (("ab", "plain", F32, F32, 128, 64, 2, (64, 30), True), "f51379d2e86e56e8"),
 ]

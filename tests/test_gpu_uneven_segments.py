@@ -1,5 +1,5 @@
-"""Packed sequences on the fused route in time segments by their lengths (share_segments, prep.hip), as many in all as in equal numbers: against the classic route, which cuts
-none of these, and the passes among each other."""
+"""Packed sequences of unequal lengths on the fused route, whose time segments are equal in number: against the classic route, which cuts none of these, the passes among each other,
+and the same sequence beside others."""
 import ctypes
 
 import pytest
@@ -14,23 +14,12 @@ from test_gpu_graph import _capture
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
-# Equal and unequal lengths; sequences of one token, of none, at the front, the end and between; tokens of no sequence; more segments than the long one may have (64, eight chunks each);
-# 64 sequences, most of them empty, and 65, which are cut in equal numbers; lengths of whole chunks and of a token more or less.
+# Equal and unequal lengths; sequences of one token, of none, at the front, the end and between; tokens of no sequence; one long sequence beside a short one;
+# 64 sequences, most of them empty, and 65; lengths of whole chunks and of a token more or less.
 CUTS = [
     (2, (0, 4100, 5600, 7600, 8192)), (3, (0, 300, 1000, 3500, 3700)), (4, (0, 0, 17, 1500, 1500, 1501, 2100, 2100)), (2, (5, 2300, 2310, 2900)), (1, (0, 10000, 10016)),
     (1, (0, 257, 514, 770)), (16, (0, 2000, 2047, 3000)), (12, (0, 1597, 3421)), (1, (0, 16, 33, 1040, 1600)), (1, tuple([0] * 40 + [9000, 9600] + [17000] * 23)), (1, tuple([0] * 41 + [9000, 9600] + [17000] * 23)),
 ]
-
-
-def _chunk_segments(cu, slots):
-    """share_segments on the host: segments of each sequence"""
-    chunks = [-(-(e - b) // 16) for b, e in zip(cu, cu[1:])]
-    of = lambda length: [max(1, min(64, c // 8, -(-c // length))) for c in chunks]
-    length = max(8, -(-sum(chunks) // slots))
-    while sum(of(length)) > slots:
-        length += 1
-    even = slots // len(chunks)
-    return of(length) if max(chunks) > length * even else [even] * len(chunks)
 
 
 @pytest.mark.parametrize("gk", [torch.bfloat16, torch.float32])
@@ -52,8 +41,7 @@ def test_against_classic_route(H, cu, gk):
     errs = {n: max(O.rel_l2(g[n], g_c[n]) for g in (kept, own)) for n in g_c}
     assert all(e <= 6e-3 for e in errs.values()), errs
     if N <= 64:                                                   # the states entering the segments are where the host's count of them says
-        counts = _chunk_segments(cu, slots)
-        assert sum(counts) <= slots
+        counts = [slots // N] * N
         # a record is 16 x 16 tiles [value block][key block], lane 16 g + c's four elements of one: keys 4 g + i of value column c
         rec = bnd.view(torch.float32).view(slots * H, 4, 4, 4, 16, 4).permute(0, 2, 3, 5, 1, 4).reshape(slots * H, 64, 64)
         first = 0
@@ -100,3 +88,28 @@ def test_operator_records_and_inputs_only():
         assert all(torch.equal(a, b) for a, b in zip(out, eager))
         train()
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("H,lens,others", [(16, (700, 1150, 1150), (700, 2290, 10)), (16, (1150, 700, 1150), (10, 1840, 1150)), (16, (40, 1960), (1960, 40)), (2, (700, 33, 767, 500), (500, 700, 40, 760))])
+def test_a_sequence_beside_others(H, lens, others):
+    """What a sequence gives and gets is its own: the same bits whatever the lengths of those packed with it, as many and as long in all."""
+    inp = make_inputs(63, 1, sum(lens), H, 64, 64, gk_div=4.0, n_states=len(lens))
+
+    def run(order, at):                                           # the first sequence of `lens` at place `at`, others of the same numbers
+        cu = [sum(order[:i]) for i in range(len(order) + 1)]
+        def place(t, r=1):
+            t = t.clone()
+            mine, T = t[:, :r * lens[0]].clone(), t.shape[1]
+            return torch.cat([t[:, T - r * cu[at]:], mine, t[:, r * lens[0]:T - r * cu[at]]], 1)
+        x = [place(getattr(inp, n), 2 if n in "ab" else 1).bfloat16().to(DEV).requires_grad_() for n in ("q", "k", "v", "a", "b", "gk")]
+        h0, dht = (torch.cat([t[len(lens) - at:], t[:1], t[1:len(lens) - at]]).to(DEV) for t in (inp.h0, inp.dht))
+        h0.requires_grad_()
+        with pytest.MonkeyPatch.context() as mp:
+            mp.setenv("HDLA_HIP_ROUTE", "fused")
+            o, ht = chunk_hrdplr_delta_rule(*x, 2, scale=0.7, initial_state=h0, output_final_state=True, cu_seqlens=torch.tensor(cu, device=DEV))
+            g = torch.autograd.grad([o, ht], x + [h0], [place(inp.do).bfloat16().to(DEV), dht])
+        tok = lambda t, r=1: t[0, r * cu[at]:r * cu[at + 1]]
+        return [tok(o), ht[at], *[tok(t, 2 if i in (3, 4) else 1) for i, t in enumerate(g[:6])], g[6][at]]
+
+    for a, b in zip(run(lens, 0), run(others, others.index(lens[0]))):
+        assert torch.equal(a, b)
