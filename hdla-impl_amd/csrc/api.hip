@@ -174,13 +174,12 @@ int kept_plan_segments(const hdla_dims* d, int32_t& bwd) {
     return fwd;
 }
 
-// Whether a training call leaves the states that enter the chunks as well (hdla_states_plan), 2.0 times the inputs' bytes in all at K = V = 128 where the chunks'
+// Whether a training call can leave the states that enter the chunks as well (hdla_states_plan), 2.0 times the inputs' bytes in all at K = V = 128 where the chunks'
 // operands alone are 1.1: the forward pass's scan has them, and the backward pass's reverse scan has the device to itself.  Not where both scans of that
 // pass fit the device in their narrowest workgroups: side by side they take no longer than one.  us a training step, without the states -> with them, 2-byte elements, K = V = 128:
-// 16384 tokens of 16 heads in 4 sequences, where nothing was kept before, 1635 -> 1425 (the pair of scans 510 -> 328, the forward pass's 253 -> 378, prep 348 -> 190), 4 x 2048, beta
-// form 718 -> 640, 4 x 1000 of 16 338 -> 335, 36 lanes of 63 chunks 223 -> 194, 32 167 -> 156, 24 148 -> 131; on the other side of the line, as a graph's replay, 16 of 63 116 -> 115, 16 of
-// 97 162 -> 159, 8 of 63 98.4 -> 98.0, 2 of 7 37.7 -> 38.0, 16 heads of 256 tokens 47.1 -> 46.7.  K = 64, V = 128, 48 lanes 143 -> 129, 16 67.0 -> 65.9; K = 128, V = 64, 48 lanes 198 -> 178, 32
-// 134.4 -> 131.5.  STATES_MOST: what calls may hold on a device in all (native.cpp, kept_room).
+// 16384 tokens of 16 heads in 4 sequences, where nothing is kept otherwise, 1630 -> 1424 (the pair of scans 510 -> 328, the forward pass's 253 -> 378, prep 348 -> 190), 4 x 2048, beta
+// form 717 -> 627; K = 64, V = 128, 32 x 300 of 32 1071 -> 880; K = 128, V = 64, 16 x 1000 of 16, beta form 983 -> 757.  On the other side of the line, as a graph's replay, 16 lanes of 63 chunks
+// 116 -> 115, 16 of 97 162 -> 159, 8 of 63 98.4 -> 98.0.  Which calls take them: native.cpp, chunk_forward.  STATES_MOST: what calls may hold on a device in all (kept_room there).
 constexpr size_t STATES_MOST = (size_t)1 << 30;
 constexpr long long SCAN_PAIR_WORKGROUPS = 256;               // one a compute unit (launch_scan_grad_shape)
 bool leaves_states(const hdla_dims* d) {

@@ -5,7 +5,7 @@
 
 extern "C" {
 // A training call that leaves its backward pass, beside what hdla_chunk_fwd_keep leaves, the states that enter the chunks: that pass runs the reverse
-// scan alone.  hdla_states_plan: bytes of the buffer to hold between the passes, 0 where it does not pay or is too large; fwd_workspace, bwd_workspace: bytes of scratch of the
+// scan alone.  hdla_states_plan: bytes of the buffer to hold between the passes, 0 where it does not pay or is too large (a gibibyte; whether a call takes it, native.cpp says); fwd_workspace, bwd_workspace: bytes of scratch of the
 // two calls.  One segment in both passes; the results, and those of a backward pass without the buffer (HDLA_ROUTE_PLAIN), are the same bits.
 size_t hdla_states_plan(const hdla_dims* dims, size_t* fwd_workspace, size_t* bwd_workspace);
 int hdla_chunk_fwd_states(const hdla_dims* dims, const void* q, const void* k, const void* v, const void* a, const void* b, const void* beta, const void* gk,

@@ -162,7 +162,7 @@ Tensor workspace(const hdla_dims& d, int pass, const Tensor& like, bool with_rec
     return bytes_like(like, n);
 }
 
-// Forward workspaces that calls hold for their backward passes because the library suggests it (hdla_keep_plan), and nobody asked: as much as KEPT_MOST
+// Forward workspaces that calls hold for their backward passes because the library suggests it (hdla_keep_plan, hdla_states_plan), and nobody asked: as much as KEPT_MOST
 // a device over all calls whose backward pass is still to come, 0.4 % of its memory, so that a stack of layers that trains within the device's memory
 // without them does so with them, and that of KEPT_CALLS calls, a microsecond to look through.  A call that finds no room, there or with the allocator,
 // keeps its inputs and recomputes, the same bits.  So does one under saved-tensor hooks: what these see of a call must not depend on the room that
@@ -216,21 +216,27 @@ void chunk_forward(const ChunkIn& x, const hdla_dims& d, bool want_ht, Plan* pla
     if (plan && plan->keep) {
         hdla_dims k = d;
         int32_t for_bwd = 0;
-        size_t ws_fwd = 0, ws_bwd = 0;                    // first the larger of the two buffers that it may be given
-        const size_t all = plan->record && !nb ? api.states_plan(&d, &ws_fwd, &ws_bwd) : 0;
-        if (all) left = kept_room(x.q, (int64_t)all);
-        if (left.defined()) {
-            plan->keep = KEEP_STATES;
-            const Tensor ws = bytes_like(x.q, ws_fwd);
-            check(api.chunk_fwd_states(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.beta), ptr(x.gk), fptr(x.h0), ptr(o), fptr(ht),
-                                       ptr(left), all, ptr(ws), ws_fwd, stream_of(x.q)), "hdla_chunk_fwd_states");
-            return;
-        }
-        const size_t n = plan->record && !nb ? api.keep_plan(&d, &k.segments, &for_bwd) : 0;
+        const bool may = plan->record && !nb;
+        const size_t n = may ? api.keep_plan(&d, &k.segments, &for_bwd) : 0;
         if (n) {                                          // one plan for the backward pass, kept or not
             plan->segments = for_bwd;
             if (for_bwd == 1) plan->route = HDLA_ROUTE_PLAIN;   // (one segment, also where a number asked for would be the fused route's)
             left = kept_room(x.q, (int64_t)n);
+        } else if (may) {
+            // Too large for that (KEEP_MOST, api.hip): with the states, 490 to 980 MiB that save 80 to 210 us.  Not where the smaller buffer is to be had: with them the gibibyte holds half
+            // as many calls, and one that finds no room loses more than the others gain.  us a step of several calls of 4 x 1000 tokens, 16 heads, K = V = 128, with states first / without: 1
+            // 350 / 363, 4 1399 / 1389, 8 2923 / 2841; 8 of 2 x 2048 3339 / 3276; 16 of 4 x 500 2937 / 2875.  Large ones, states / nothing: 1 and 3 of 16384 packed tokens 1424 / 1630,
+            // 4675 / 4877 (the first has the room), 4 of 4 x 2048, beta form 2621 / 2846; seven of the first behind a packed one 4063 / 4073.
+            size_t ws_fwd = 0, ws_bwd = 0;
+            const size_t all = api.states_plan(&d, &ws_fwd, &ws_bwd);
+            if (all) left = kept_room(x.q, (int64_t)all);
+            if (left.defined()) {
+                plan->keep = KEEP_STATES;
+                const Tensor ws = bytes_like(x.q, ws_fwd);
+                check(api.chunk_fwd_states(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.beta), ptr(x.gk), fptr(x.h0), ptr(o), fptr(ht),
+                                           ptr(left), all, ptr(ws), ws_fwd, stream_of(x.q)), "hdla_chunk_fwd_states");
+                return;
+            }
         }
         plan->keep = left.defined() ? KEEP_FORWARD : KEEP_NOTHING;
         if (plan->keep) {
