@@ -13,6 +13,8 @@ int hdla_chunk_fwd_states(const hdla_dims* dims, const void* q, const void* k, c
 int hdla_chunk_bwd_states(const hdla_dims* dims, const void* q, const void* k, const void* v, const void* a, const void* b, const void* beta, const void* gk,
                           const float* h0, const void* d_o, const float* dht, void* dq, void* dk, void* dv, void* da, void* db, void* dbeta, void* dgk, float* dh0,
                           void* kept, size_t kept_bytes, void* workspace, size_t workspace_bytes, void* stream);
+// hdla_layer_pre_bwd into a dy whose rows are lddy elements (ldy at the least, whole 16 bytes): its padding reaches there.
+int hdla_layer_pre_bwd_to(const hdla_pre_dims* dims, const void* y, const void* dq, const void* dk, const void* dv, const void* dbeta, void* dy, int32_t lddy, void* stream);
 // y [M, N] = x [M, K] W, W [N, K] taken turned or (turned) [K, N] as it is; bf16, sums in 32 bits.  N and K in eights (turned: N in 64s), rows 16 bytes aligned.
 int hdla_tile_gemm(int32_t M, int32_t N, int32_t K, const void* x, int64_t ldx, const void* w, int64_t ldw, int32_t turned, void* y, int64_t ldy, void* stream);
 }

@@ -10,7 +10,7 @@
 // HBM-bound byte work: a (row, head) pair is D elements = LPR lanes of 16 bytes, 64/LPR pairs per wavefront pass, the
 // sums over a head are butterflies inside the wavefront.
 #include "hdla_common.cuh"
-#include "../../include/hdla_hip.h"
+#include "host_path.h"
 
 namespace hdla {
 
@@ -18,12 +18,12 @@ struct PreArgs {
     const void* y;                            // [rows, ldy]
     void *q, *k, *v, *beta;                   // forward outputs: [rows, H, D] x 3, [rows, H]
     const void *dq, *dk, *dv, *dbeta;         // backward inputs
-    void* dy;                                 // backward output [rows, ldy]: the four column ranges are written
+    void* dy;                                 // backward output [rows, lddy]: the four column ranges are written
     long long nslot, nsg;                     // rows * H, wavefront passes
-    int H, D, ldy, cq, ck, cv, cb;            // column offsets in y; cb < 0: no beta
+    int H, D, ldy, lddy, cq, ck, cv, cb;      // column offsets in y and dy; cb < 0: no beta
     int lpr_log2, norm_q, norm_k, norm_v;
     float beta_scale, eps_d;                  // eps_d = D * eps: o = u / sqrt(sum u^2 + D eps)
-    int zero_from;                            // > 0: backward, columns zero_from .. ldy of dy are padding and become zero
+    int zero_from;                            // > 0: backward, columns zero_from .. lddy of dy are padding and become zero
 };
 
 typedef unsigned pre_u32x4 __attribute__((ext_vector_type(4)));
@@ -156,7 +156,7 @@ __global__ __launch_bounds__(256) void layer_pre_bwd_kernel(PreArgs p) {
         const bool live = slot < p.nslot;
         const long long row = live ? slot / p.H : 0;
         const int h = live ? (int)(slot - row * p.H) : 0;
-        const long long in = row * p.ldy + (long long)h * p.D + sl * N, out = slot * p.D + sl * N;
+        const long long in = row * p.ldy + (long long)h * p.D + sl * N, to = row * p.lddy + (long long)h * p.D + sl * N, out = slot * p.D + sl * N;
         float q[N], k[N], v[N], gq[N], gk[N], gv[N];
         if (live) {
             PrePiece<T>::ld(p.y, in + p.cq, q);
@@ -173,17 +173,17 @@ __global__ __launch_bounds__(256) void layer_pre_bwd_kernel(PreArgs p) {
         pre_bwd_one<T, N>(k, gk, p.norm_k != 0, p.eps_d, lpr);
         pre_bwd_one<T, N>(v, gv, p.norm_v != 0, p.eps_d, lpr);
         if (live) {
-            PrePiece<T>::st(p.dy, in + p.cq, gq);
-            PrePiece<T>::st(p.dy, in + p.ck, gk);
-            PrePiece<T>::st(p.dy, in + p.cv, gv);
+            PrePiece<T>::st(p.dy, to + p.cq, gq);
+            PrePiece<T>::st(p.dy, to + p.ck, gk);
+            PrePiece<T>::st(p.dy, to + p.cv, gv);
             if (p.cb >= 0 && sl == 0) {
                 const float b = pre_sigmoid<T>(ld_elem(static_cast<const T*>(p.y) + row * p.ldy + p.cb + h));
                 const float g = ld_elem(static_cast<const T*>(p.dbeta) + slot);
-                st_elem(static_cast<T*>(p.dy) + row * p.ldy + p.cb + h, g * p.beta_scale * b * (1.f - b));
+                st_elem(static_cast<T*>(p.dy) + row * p.lddy + p.cb + h, g * p.beta_scale * b * (1.f - b));
             }
             // the padding of the row, shared out over the lanes of its heads
             if (p.zero_from > 0)
-                for (int c = p.zero_from + h * lpr + sl; c < p.ldy; c += p.H * lpr) st_elem(static_cast<T*>(p.dy) + row * p.ldy + c, 0.f);
+                for (int c = p.zero_from + h * lpr + sl; c < p.lddy; c += p.H * lpr) st_elem(static_cast<T*>(p.dy) + row * p.lddy + c, 0.f);
         }
     }
 }
@@ -235,7 +235,7 @@ static int pre_config(const hdla_pre_dims* d, PreArgs& a, unsigned& nwg) {
     if (d->col_beta >= 0 && (long long)d->col_beta + d->H > d->ldy) return HDLA_ERR_SHAPE;
     if (d->rows > (1LL << 40) / d->H) return HDLA_ERR_SHAPE;
     a = PreArgs{};
-    a.nslot = d->rows * d->H; a.H = d->H; a.D = d->D; a.ldy = d->ldy;
+    a.nslot = d->rows * d->H; a.H = d->H; a.D = d->D; a.ldy = a.lddy = d->ldy;
     a.cq = d->col_q; a.ck = d->col_k; a.cv = d->col_v; a.cb = d->col_beta < 0 ? -1 : d->col_beta;
     a.lpr_log2 = 0;
     while ((1 << a.lpr_log2) < lpr) ++a.lpr_log2;
@@ -271,11 +271,14 @@ extern "C" int hdla_layer_pre_fwd(const hdla_pre_dims* dims, const void* y, void
     return e == hipSuccess ? HDLA_OK : (int)e;
 }
 
-extern "C" int hdla_layer_pre_bwd(const hdla_pre_dims* dims, const void* y, const void* dq, const void* dk,
-                                  const void* dv, const void* dbeta, void* dy, void* stream) {
+extern "C" int hdla_layer_pre_bwd_to(const hdla_pre_dims* dims, const void* y, const void* dq, const void* dk,
+                                     const void* dv, const void* dbeta, void* dy, int32_t lddy, void* stream) {
     PreArgs a; unsigned nwg;
     const int rc = pre_config(dims, a, nwg);
     if (rc) return rc;
+    if (lddy < dims->ldy) return HDLA_ERR_SHAPE;
+    if (lddy % (dims->dtype == HDLA_BF16 ? 8 : 4)) return HDLA_ERR_ALIGN;
+    a.lddy = lddy;
     if (dims->rows == 0) return HDLA_OK;
     if (!y || !dq || !dk || !dv || !dy || (a.cb >= 0 && !dbeta)) return HDLA_ERR_NULL;
     if (!pre_al16(y) || !pre_al16(dq) || !pre_al16(dk) || !pre_al16(dv) || !pre_al16(dy)) return HDLA_ERR_ALIGN;
@@ -285,6 +288,11 @@ extern "C" int hdla_layer_pre_bwd(const hdla_pre_dims* dims, const void* y, cons
     else hipLaunchKernelGGL(layer_pre_bwd_kernel<float>, dim3(nwg), dim3(256), 0, s, a);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? HDLA_OK : (int)e;
+}
+
+extern "C" int hdla_layer_pre_bwd(const hdla_pre_dims* dims, const void* y, const void* dq, const void* dk,
+                                  const void* dv, const void* dbeta, void* dy, void* stream) {
+    return hdla_layer_pre_bwd_to(dims, y, dq, dk, dv, dbeta, dy, dims ? dims->ldy : 0, stream);
 }
 
 static int logsigmoid_launch(int dtype, long long n, const void* x, const void* dy, void* out, bool bwd, void* stream) {

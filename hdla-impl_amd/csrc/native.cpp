@@ -48,7 +48,7 @@ struct Api {
 #define HDLA_FN(name) decltype(&hdla_##name) name
     HDLA_FN(strerror); HDLA_FN(workspace_bytes); HDLA_FN(record_bytes); HDLA_FN(record_workspace_bytes); HDLA_FN(chunk_fwd_b); HDLA_FN(chunk_bwd_b);
     HDLA_FN(keep_plan); HDLA_FN(chunk_fwd_keep); HDLA_FN(chunk_bwd_kept); HDLA_FN(states_plan); HDLA_FN(chunk_fwd_states); HDLA_FN(chunk_bwd_states);
-    HDLA_FN(tile_gemm);
+    HDLA_FN(tile_gemm); HDLA_FN(layer_pre_bwd_to);
     HDLA_FN(recurrent_fwd); HDLA_FN(param_recurrent_fwd); HDLA_FN(normalize_fwd); HDLA_FN(normalize_bwd_as);
     HDLA_FN(normalize_workspace_bytes); HDLA_FN(layer_pre_fwd); HDLA_FN(layer_pre_bwd); HDLA_FN(layer_up_fwd); HDLA_FN(layer_down);
     HDLA_FN(layer_up_wgrad); HDLA_FN(layer_up_wgrad_workspace_bytes); HDLA_FN(rows_gemm); HDLA_FN(sum_partials); HDLA_FN(stack_rows);
@@ -651,11 +651,8 @@ constexpr double PRE_EPS = 1e-5;                 // l2_norm's
 // Columns of y: q, k, v (d each), the inner activations of decay and gate (D each), beta (H), padding.
 struct LayerCols {
     int64_t d, D, H, f0, g0, beta, used, ld;
-    // of a concatenated weight that has ld_ rows
-    LayerCols(int64_t d_, int64_t H_, int64_t ld_) : d(d_), D(d_ / H_), H(H_) {
-        f0 = 3 * d; g0 = f0 + D; beta = g0 + D; used = beta + H; ld = ld_;
-    }
-    LayerCols(int64_t d_, int64_t H_, bool padded) : LayerCols(d_, H_, int64_t(0)) {
+    LayerCols(int64_t d_, int64_t H_, bool padded) : d(d_), D(d_ / H_), H(H_) {
+        f0 = 3 * d; g0 = f0 + D; beta = g0 + D; used = beta + H;
         // The GEMM on x runs at its best on output widths that are whole tiles of 256 (8192 x 3216 x 1024: 82 us, with
         // 3328 columns 50; its input gradient 60 -> 55, its weight gradient 86 -> 80).  Short calls read the weight once and are
         // bound by that: there only up to the 16 bytes that rows are aligned to.
@@ -663,19 +660,18 @@ struct LayerCols {
     }
 };
 constexpr int64_t PAD_FROM_ROWS = 1024;
-// In training, where that makes the weight's gradient one of the library's own (own_weight_grad), up to whole tiles of its kernel: a
-// BLAS call less, and both weight gradients in one launch.  us a training step (all of these are bound by the host): 4 x 121 tokens, 256 channels 239 -> 218, 1 x 64, 512 246 -> 222,
+// Rows of the weight in training, and columns of y's gradient: where that makes the weight's gradient one of the library's own (own_weight_grad), up to whole tiles of its kernel: a
+// BLAS call less, and both weight gradients in one launch.  (y itself is as wide as without gradients, and so the same call's, bit for bit: a part of a model that is checkpointed runs
+// once without them.)  us a training step (all of these are bound by the host): 4 x 121 tokens, 256 channels 239 -> 218, 1 x 64, 512 246 -> 222,
 // 2 x 500, 512 275 -> 248, 1 x 512, 1024 271 -> 245, 1 x 1000, 1024 273 -> 246.  Wider layers, whose gradient has more tiles, stay as they are (1 x 900, 2048 384 and 379).
-LayerCols training_cols(int64_t d, int64_t H, int64_t rows) {
-    LayerCols L(d, H, rows >= PAD_FROM_ROWS);
+int64_t training_rows(const LayerCols& L, int64_t rows) {
     const int64_t tiles = (L.used + 127) / 128;
-    if (rows < PAD_FROM_ROWS && d % 128 == 0 && tiles * (d / 128) <= 256) L.ld = 128 * tiles;
-    return L;
+    return rows < PAD_FROM_ROWS && L.d % 128 == 0 && tiles * (L.d / 128) <= 256 ? 128 * tiles : L.ld;
 }
 
-// the concatenated projection weight [ld, d], in `out` if there is one; rows behind the last projection are zero
-Tensor gather_weights(const Tensor* w, const LayerCols& L, Tensor out = Tensor()) {       // wq, wk, wv, wf0, wg0, wbeta
-    if (!out.defined()) out = at::empty({L.ld, L.d}, w[0].options());
+// the concatenated projection weight [n, d], in `out` if there is one; rows behind the last projection are zero
+Tensor gather_weights(const Tensor* w, const LayerCols& L, int64_t n, Tensor out = Tensor()) {       // wq, wk, wv, wf0, wg0, wbeta
+    if (!out.defined()) out = at::empty({n, L.d}, w[0].options());
     const void* parts[6];
     int64_t rows[6];
     std::vector<Tensor> whole(6);                                  // (a parameter may be a view at any address)
@@ -684,7 +680,7 @@ Tensor gather_weights(const Tensor* w, const LayerCols& L, Tensor out = Tensor()
         parts[i] = whole[i].data_ptr();
         rows[i] = whole[i].size(0);
     }
-    check(api.stack_rows(parts, rows, 6, L.d, ptr(out), L.ld, stream_of(out)), "hdla_stack_rows");
+    check(api.stack_rows(parts, rows, 6, L.d, ptr(out), n, stream_of(out)), "hdla_stack_rows");
     return out;
 }
 hdla_pre_dims pre_dims(const LayerCols& L, const LayerCfg& f, int64_t rows) {
@@ -696,9 +692,9 @@ hdla_pre_dims pre_dims(const LayerCols& L, const LayerCfg& f, int64_t rows) {
     p.zero_from = (int32_t)L.used;
     return p;
 }
-hdla_up_dims up_dims(const LayerCols& L, int64_t rows) {
+hdla_up_dims up_dims(const LayerCols& L, int64_t rows, int64_t ld) {
     hdla_up_dims u{};
-    u.rows = rows; u.d = (int32_t)L.d; u.D = (int32_t)L.D; u.ld = L.ld; u.col_f = (int32_t)L.f0; u.col_g = (int32_t)L.g0;
+    u.rows = rows; u.d = (int32_t)L.d; u.D = (int32_t)L.D; u.ld = ld; u.col_f = (int32_t)L.f0; u.col_g = (int32_t)L.g0;
     return u;
 }
 // Products of some hundred rows by hdla_tile_gemm: what is one round of its workgroups on the device (figures there).  us a call, BLAS -> this: a decode step
@@ -746,7 +742,7 @@ void layer_step(const Tensor* P, const LayerCfg& f, const LayerCols& L, const hd
     // device: 3 x 2560, 40 23.4 / 24.6 (the host 25.3 / 24.7), 3 x 3072, 48 26.6 / 28.6, 3 x 3584, 28 33.1 / 35.3, 1 x 4096, 32 39.2 / 41.8.
     const bool later = !norm_in_step && f.groups == 1 && rows <= 16 && L.d <= 2048, own_norm = !norm_in_step && !later;
     if (!later) r.n = at::empty({rows, L.d}, opt);
-    const hdla_up_dims ud = up_dims(L, rows);
+    const hdla_up_dims ud = up_dims(L, rows, L.ld);
     const hdla_norm_dims nd = norm_dims(r.x, P[8], f.gate_pos, f.c, f.eps, f.groups);
     // gate, o, log_f and the gated o (fp32) with its sums, as far as they are handed on
     const int64_t one = rows * L.d, parts = (own_norm ? 2 : 0) + (in_step ? 0 : own_norm ? 1 : 2);
@@ -794,10 +790,10 @@ bool in_few_launches(int64_t rows, int64_t T, int64_t d, bool norm_in_step) {
 void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, Plan& plan, const Tensor& h0, bool want_ht, bool chunked, bool keep,
                    LayerFwd& r) {
     const int64_t B = x3.size(0), T = x3.size(1), d = x3.size(2), rows = B * T;
-    const LayerCols L(d, f.H, r.w.size(0));
+    const LayerCols L(d, f.H, rows >= PAD_FROM_ROWS);
     const auto opt = x3.options();
     r.x = x3.contiguous().view({rows, d});
-    r.y = project(r.x, r.w);
+    r.y = project(r.x, r.w.size(0) == L.ld ? r.w : r.w.narrow(0, 0, L.ld));
     const hdla_pre_dims pd = pre_dims(L, f, rows);
     if (!chunked && T < RECURRENT_BELOW && in_few_launches(rows, T, d, f.groups == f.H)) {
         layer_step(P, f, L, pd, T, h0, want_ht, r);
@@ -809,7 +805,7 @@ void layer_forward(const Tensor& x3, const Tensor* P, const LayerCfg& f, Plan& p
     in.beta = at::empty({B, T, L.H, 1}, opt);
     void* const s = stream_of(x3);
     check(api.layer_pre_fwd(&pd, ptr(r.y), ptr(in.q), ptr(in.k), ptr(in.v), ptr(in.beta), s), "hdla_layer_pre_fwd");
-    const hdla_up_dims ud = up_dims(L, rows);
+    const hdla_up_dims ud = up_dims(L, rows, L.ld);
     if (keep) r.f = at::empty({rows, d}, opt);
     in.gk = at::empty({B, T, L.H, L.D}, opt);
     r.g = at::empty({rows, d}, opt);
@@ -895,7 +891,9 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
                                  const Tensor& wo, const Maybe& h0, const LayerCfg& f, bool want_ht, Plan plan) {
         const Tensor P[10] = {wq, wk, wv, wf0, wg0, wbeta, wf1, wg1, wnorm, wo};
         LayerFwd r;
-        r.w = gather_weights(P, training_cols(x.size(2), f.H, x.size(0) * x.size(1)));
+        const int64_t rows = x.size(0) * x.size(1);
+        const LayerCols L(x.size(2), f.H, rows >= PAD_FROM_ROWS);
+        r.w = gather_weights(P, L, training_rows(L, rows));
         layer_forward(x, P, f, plan, value(h0), want_ht, true, true, r);
         save_plan(ctx, plan);
         ctx->save_for_backward({r.x, r.w, r.y, r.f, r.g, r.o, r.n, r.left, r.op.q, r.op.k, r.op.v, r.op.beta, r.op.gk, value(h0), wf1, wg1,
@@ -921,7 +919,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
         const auto ci = ctx->saved_data["i"].toIntVector();
         const LayerCfg cfg{ci[0], ci[1], ci[2] != 0, ci[3] != 0, cc[0], cc[1], cc[2], (int)ci[4]};
         const int64_t B = ci[5], T = ci[6], rows = x.size(0), d = x.size(1);
-        const LayerCols L(d, cfg.H, w.size(0));
+        const LayerCols L(d, cfg.H, rows >= PAD_FROM_ROWS);
         void* const stream = stream_of(x);
         const auto opt = x.options();
         const auto need = [&](size_t i) { return ctx->needs_input_grad(i); };
@@ -959,11 +957,11 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
         }
 
         // gradient of y, each part written where it belongs
-        const Tensor dy = at::empty_like(y);
+        const Tensor dy = at::empty({rows, w.size(0)}, opt);
         const hdla_pre_dims pd = pre_dims(L, cfg, rows);
-        check(api.layer_pre_bwd(&pd, ptr(y), ptr(dq), ptr(dk), ptr(dv), ptr(dbeta), ptr(dy), stream), "hdla_layer_pre_bwd");
-        const hdla_up_dims ud = up_dims(L, rows);
-        check(api.layer_down(&ud, ptr(wf1), ptr(wg1), ptr(f), ptr(dgk), ptr(dgate), ptr(dy), stream), "hdla_layer_down");
+        check(api.layer_pre_bwd_to(&pd, ptr(y), ptr(dq), ptr(dk), ptr(dv), ptr(dbeta), ptr(dy), (int32_t)w.size(0), stream), "hdla_layer_pre_bwd_to");
+        const hdla_up_dims ud = up_dims(L, rows, L.ld), down = up_dims(L, rows, w.size(0));
+        check(api.layer_down(&down, ptr(wf1), ptr(wg1), ptr(f), ptr(dgk), ptr(dgate), ptr(dy), stream), "hdla_layer_down");
         if (need(7) || need(8)) {
             out[7] = at::empty_like(wf1);
             out[8] = at::empty_like(wg1);
@@ -1169,7 +1167,7 @@ PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
         std::optional<c10::Event> ready;
         unlocked([&] {
             if (built) {
-                r.w = gather_weights(P, L, r.w);
+                r.w = gather_weights(P, L, L.ld, r.w);
                 // (one gathered under capture is not there before the graph is replayed, and belongs to it)
                 if (cached && !capturing()) {
                     ready.emplace(c10::DeviceType::CUDA);
@@ -1211,6 +1209,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     HDLA_FN(strerror) HDLA_FN(workspace_bytes) HDLA_FN(record_bytes) HDLA_FN(record_workspace_bytes) HDLA_FN(chunk_fwd_b) HDLA_FN(chunk_bwd_b)
     HDLA_FN(keep_plan) HDLA_FN(chunk_fwd_keep) HDLA_FN(chunk_bwd_kept) HDLA_FN(states_plan) HDLA_FN(chunk_fwd_states) HDLA_FN(chunk_bwd_states) HDLA_FN(tile_gemm)
+    HDLA_FN(layer_pre_bwd_to)
     HDLA_FN(recurrent_fwd) HDLA_FN(param_recurrent_fwd) HDLA_FN(normalize_fwd) HDLA_FN(normalize_bwd_as)
     HDLA_FN(normalize_workspace_bytes) HDLA_FN(layer_pre_fwd) HDLA_FN(layer_pre_bwd) HDLA_FN(layer_up_fwd) HDLA_FN(layer_down)
     HDLA_FN(layer_up_wgrad) HDLA_FN(layer_up_wgrad_workspace_bytes) HDLA_FN(rows_gemm) HDLA_FN(sum_partials) HDLA_FN(stack_rows) HDLA_FN(layer_step)

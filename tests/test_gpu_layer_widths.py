@@ -30,3 +30,29 @@ def test_against_the_python_code(B, T, d, H):
         assert a.shape == b.shape and torch.isfinite(a.float()).all(), n
         rel = (a.double() - b.double()).norm() / b.double().norm().clamp_min(1e-30)
         assert rel <= 12 * 2.0 ** -8, (n, float(rel))
+
+
+# rows that the layer's own products take, on both sides of the number of their tiles with and without the padding (257 .. 320 of 1024 channels), and that are the BLAS library's
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,T,d,H", [(1, 33, 1024, 16), (1, 65, 512, 8), (1, 257, 1024, 16), (4, 80, 1024, 16), (1, 321, 1024, 16), (2, 500, 1024, 16), (1, 700, 512, 4), (1, 1023, 768, 6), (1, 1024, 768, 6)])
+def test_outputs_with_and_without_gradients(B, T, d, H):
+    """The same bits, as a recomputation in place of a pass without gradients expects them; so are the gradients behind one."""
+    from torch.utils.checkpoint import checkpoint
+    torch.manual_seed(4)
+    with torch.device(DEV):
+        m = HDLA_Custom(d, H, token_mixer_init_type=2, rescale_type=0).bfloat16().train()
+        x, do = torch.randn(B, T, d).bfloat16().requires_grad_(), torch.randn(B, T, d).bfloat16()
+    y = m(x)[0]
+    want = torch.autograd.grad(y, [x, *m.parameters()], do)
+    with torch.no_grad():
+        assert torch.equal(m(x)[0], y)
+        m.eval()
+        assert torch.equal(m(x)[0], y)
+        m.train()
+    y2 = checkpoint(lambda t: m(t)[0], x, use_reentrant=True)
+    assert torch.equal(y2, y)
+    for p in [x, *m.parameters()]:
+        p.grad = None
+    y2.backward(do)
+    for p, w in zip([x, *m.parameters()], want):
+        assert torch.equal(p.grad, w)
