@@ -10,8 +10,12 @@
 // are more than there are compute units the BLAS kernels' larger tiles win.  us on the device, operands from HBM, BLAS / 32 x 32 / 64 x 32 / 64 x 64 (* the choice):
 // 100 x 3216 x 1024 9.0 / 9.3 / 6.2* / 7.0, 100 x 1024 x 1024 7.8 / 4.6* / 5.4 / 6.4, 256 x 3216 x 1024 9.5 / 17.0 / 11.2 / 8.8*, 484 x 904 x 256 5.3 / 6.3 / 4.6* / 5.0,
 // 512 x 1024 x 3216 17.1 / 19.8 / 14.8* / 17.2, 256 x 4096 x 4096 21.7 / 37 / 27 / 18.9*, 1024 x 1024 x 1024 9.2 / 14.3 / 9.9 / 7.6*; turned 484 x 256 x 904 9.6 / 6.3* / 7.4 / 8.1,
-// 512 x 1024 x 3216 19.0 / 23.9 / 16.2* / 18.8, 1024 x 1024 x 3328 19.2 / 44 / 28 / 18.9*; but 2000 x 512 x 1792 10.7 / - / - / 12.9*, turned 12.3 / - / - / 15.2*.  Beyond the line
-// 256 x 6416 x 2048 23.8 / 41 / 29 / 24.5, 512 x 3216 x 1024 11.6 / 28 / 20 / 15.6.
+// 512 x 1024 x 3216 19.0 / 23.9 / 16.2* / 18.8, 1024 x 1024 x 3328 19.2 / 44 / 28 / 18.9*.  Beyond the line 256 x 6416 x 2048 23.8 / 41 / 29 / 24.5, 512 x 3216 x 1024 11.6 / 28 / 20 / 15.6.
+// Over all products of the layer at 128 to 4096 channels and 65 to 8000 rows within the line (432 of them, one shape behind the other) the time is 0.77 of the BLAS library's, geometric mean.  By themselves some
+// are slower: turned, many rows over long sums (1500 x 512 x 1792 13.1 / 14.0, 2000 x 512 x 1792 13.3 / 15.5, 4000 x 256 x 1024 10.4 / 11.0) and weights of 32 MB and more (160 x 3072 x 9496 49.1 / 53.0,
+// 256 x 4096 x 4096 24.9 / 26.5); 65 to 80 x 4880 x 1536 8.8 / 9.7.  Within a step, where their operands come from the launch before, they are not: as a graph's replay, which has no host to
+// gain by, training steps with these two kinds by BLAS / by this took 1 x 1500 tokens of 512 channels 197.5 / 197.1, 4 x 500 186.1 / 186.4, 4 x 1000 of 256 197.3 / 196.7, 1 x 200 of
+// 4096 423.0 / 421.9, 1 x 256 438.3 / 439.4.  So one line serves both, and calls and replays have the same bits.
 #include "row_tile.cuh"
 #include "host_path.h"
 
