@@ -110,7 +110,8 @@ __device__ __forceinline__ void chunk_grad_common_pair(const ChunkArgs<T>& p, in
 // CG_EACH (2-byte elements): one launch for no more pairs than the device holds at once, where occupancy is nothing and a workgroup may have more registers: each does its own pair,
 // flagged or not.  us a training step as
 // a graph's replay, two launches -> one: 32 pairs of K = V = 64 36.0 -> 34.2, 252 82.7 -> 80.4 (beta form), 480 54.4 -> 50.1 (beta form), 512 64.6 -> 61.9; K = V = 128, 14 37.7 -> 36.2,
-// 256 (beta form, with less to store and read in the scans) 65.4 -> 62.7.  Beyond, with one workgroup a compute unit: 960 of K = V = 64 62.5 -> 68.4, K = V = 128 528 90 -> 96, 1552 159 -> 188.
+// 256 (beta form, with less to store and read in the scans) 65.4 -> 62.7; 256, ab form, K = 64, V = 128 42.9 -> 40.4, K = 128, V = 64 44.9 -> 42.6, with fp32 decays 43.6 -> 41.2, 46.4 -> 44.3; of
+// 82 shapes, forms and types of decays at 4 to 512 pairs all are 0.8 to 3.9 faster.  Beyond, with one workgroup a compute unit: 960 of K = V = 64 62.5 -> 68.4, K = V = 128 528 90 -> 96, 1552 159 -> 188.
 enum CgPairs { CG_COMMON, CG_FLAGGED, CG_ALL, CG_EACH };
 constexpr int CG_STRONG_GRID = 256;
 // CG_EACH's waves per SIMD, and so workgroups a compute unit: what its registers allow
