@@ -343,7 +343,8 @@ template <typename T>
 void bind_ws(ChunkArgs<T>& a, const hdla_dims* d, const WsLayout& LP, void* prep_ws, const WsLayout& LS, void* scan_ws, int nch) {
     char* base = static_cast<char*>(prep_ws);
     auto at = [&](size_t o) { return reinterpret_cast<T*>(base + o); };
-    a.ws.W = at(LP.W); a.ws.UT = LP.UT ? at(LP.UT) : nullptr; a.ws.KGT = at(LP.KGT); a.ws.BGT = at(LP.BGT);
+    a.ws.W = at(LP.W); a.ws.UT = LP.UT ? at(LP.UT) : nullptr; a.ws.BGT = at(LP.BGT);
+    a.ws.KGT = sizeof(T) == 2 && a.beta && d->route != HDLA_ROUTE_CLASSIC ? nullptr : at(LP.KGT);   // (nobody's, then: prep.hip, KG_IS_B)
     a.ws.VTT = LP.VTT ? at(LP.VTT) : nullptr; a.ws.AAK = at(LP.AAK); a.ws.aak_stride = AAK_STRIDE;
     a.ws.SUM = reinterpret_cast<float*>(base + LP.SUM);
     a.ws.QG = at(LP.QG); a.ws.AQK = at(LP.AQK); a.ws.AQB = at(LP.AQB);

@@ -97,7 +97,7 @@ struct WsLayout {
     // written by prep, read by the scans
     size_t W;      // tiles  [2][K/16]   F(w_s)        rows token, inner channel
     size_t UT;     // tiles  [2][V/16]   F(u_s^T)      rows value, inner token
-    size_t KGT;    // tiles  [K/16]      F(kg^T)       rows channel, inner token (HDLA parameterisation, 2-byte elements: not written, b_2's gated copy is k's)
+    size_t KGT;    // tiles  [K/16]      F(kg^T)       rows channel, inner token (HDLA parameterisation, 2-byte elements: under HDLA_ROUTE_CLASSIC only, else null, b_2's gated copy being k's)
     size_t BGT;    // tiles  [2][K/16]   F(bg_s^T)     rows channel, inner token
     size_t VTT;    // tiles  [V/16]      F(v^T)        rows value, inner token
     size_t AAK;    // tiles  [2]         F(A_ak^s)     rows i, inner j: 2-byte elements, where the scan forms u from it, TM and v

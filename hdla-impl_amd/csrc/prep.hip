@@ -703,6 +703,21 @@ static int clearing_workgroups(int N, int T, const PackedOut& out, int fill = 51
     const long long most = max(32, min(fill, (1 << 20) / N));
     return (int)min((bytes + 16383) / 16384, most);
 }
+// kg^T out of bg_2^T for those who look at the classic route's buffers (KG_IS_B above; a store of its own in prep_kernel cost all calls 0.5 us of 48).  RANKS: the pairs are the ranks of a tile.
+// A workgroup a slot, of 64 threads
+template <int K, bool RANKS>
+__global__ __launch_bounds__(64) void kg_of_b_kernel(const bf16* bgt, bf16* kgt, int stride) {
+    typedef uint2 Four;                               // four elements
+    const int64_t at = (int64_t)blockIdx.x * stride;
+    const Four* const from = reinterpret_cast<const Four*>(bgt + at);
+    Four* const to = reinterpret_cast<Four*>(kgt + at);
+    const int l = lane_id();
+#pragma unroll
+    for (int pair = 0; pair < K / 32; ++pair)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+            to[pair * (PAIR / 4) + 2 * l + s] = RANKS ? from[(2 * pair + s) * (PAIR / 4) + 2 * l + 1] : from[(K / 32 + pair) * (PAIR / 4) + 2 * l + s];
+}
 template <typename T, int K, int V, bool HD>
 static hipError_t launch_prep_kv(const ChunkArgs<T>& a, int mode, const FewTable& few, hipStream_t stream) {
     const int makers = few.chunk_off ? 2 + clearing_workgroups(a.st.N, a.st.T, few.out, FEW_CLEARERS) : 0;
@@ -724,6 +739,13 @@ static hipError_t launch_prep_kv(const ChunkArgs<T>& a, int mode, const FewTable
         else HDLA_PREP_LAUNCH(kAlwaysF32, STATES);
     }
 #undef HDLA_PREP_LAUNCH
+    if constexpr (HD && sizeof(T) == 2) {
+        if (a.ws.KGT) {
+            const int stride = a.ws.sa_stride / (int)sizeof(T);
+            if (mode == PREP_FWD) hipLaunchKernelGGL((kg_of_b_kernel<K, true>), dim3(a.st.nch * a.H), dim3(64), 0, stream, a.ws.BGT, a.ws.KGT, stride);
+            else hipLaunchKernelGGL((kg_of_b_kernel<K, false>), dim3(a.st.nch * a.H), dim3(64), 0, stream, a.ws.BGT, a.ws.KGT, stride);
+        }
+    }
     return hipGetLastError();
 }
 

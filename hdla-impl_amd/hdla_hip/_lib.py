@@ -12,7 +12,7 @@ from typing import Optional, Tuple
 import torch
 
 HDLA_BF16, HDLA_FP32 = 0, 1
-HDLA_VERSION = 210          # the header this binding was written against (struct layouts, entry points)
+HDLA_VERSION = 211          # the header this binding was written against (struct layouts, entry points)
 ROUTE_AUTO, ROUTE_CLASSIC, ROUTE_FUSED, ROUTE_PLAIN = 0, 1, 2, 4
 _ROUTES = {"": ROUTE_AUTO, "auto": ROUTE_AUTO, "classic": ROUTE_CLASSIC, "plain": ROUTE_PLAIN, "fused": ROUTE_FUSED}
 _HERE = os.path.dirname(os.path.abspath(__file__))

@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-#define HDLA_VERSION 210
+#define HDLA_VERSION 211
 
 enum { HDLA_BF16 = 0, HDLA_FP32 = 1 };
 
@@ -100,7 +100,8 @@ typedef struct hdla_dims {
  * (and W, UT where chunk_grad reads them instead of rebuilding them: fp32 decays beside bf16 inputs) are written, in the backward pass.  In a forward pass on bf16 inputs (HDLA_PASS_FWD, classic route) the scan forms u
  * itself: there is no UT and no VTT, TM holds three tile pairs a slot, the blocks of (I - A_ab)^-1 (not transposed: rows i, inner j) and
  * the two ranks of A_ak, and the tile pairs of BGT are the two ranks of a channel tile.  The other passes' scans of bf16 inputs form u themselves
- * as well: there is VTT in a backward pass, and UT there and in HDLA_PASS_FWD_KEEP, under HDLA_ROUTE_CLASSIC only (UT also beside fp32 decays). */
+ * as well: there is VTT in a backward pass, and UT there and in HDLA_PASS_FWD_KEEP, under HDLA_ROUTE_CLASSIC only (UT also beside fp32 decays).  Where beta is given and the
+ * inputs are bf16, KGT, which is the second rank's half of BGT then, is written under HDLA_ROUTE_CLASSIC only, in every pass (since version 211; before, always). */
 typedef struct hdla_ws_layout {
     int64_t nch;               /* chunk slots per head */
     int64_t W, UT, KGT, BGT, VTT, EGL, QG, AQK, AQB, AQBT, QGT, TM, HC, DHC, DVN;

@@ -10,7 +10,8 @@ from hdla_hip import _lib
 
 HEADER = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "include", "hdla_hip.h")
 # the declarations of each number, without comments and white space: a change of them takes the next number and a line here
-DECLARED = {207: "97db2afde6266b58", 208: "96a58c1f76b34102", 209: "e3395d06f819a037", 210: "8dfa88fe5cdbd04b"}
+DECLARED = {207: "97db2afde6266b58", 208: "96a58c1f76b34102", 209: "e3395d06f819a037", 210: "8dfa88fe5cdbd04b",
+            211: "8dfa88fe5cdbd04b"}                        # (what a workspace holds)
 
 
 def declarations(text):

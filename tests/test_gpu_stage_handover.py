@@ -61,6 +61,35 @@ def test_a_ak_and_the_sums(B, T, H, K, V, route, segments, kept, form):
         assert bool(real.any()) and O.rel_l2(got[real], want[real]) <= 1e-5       # 64 or 128 positive terms in 32 bits
 
 
+@pytest.mark.parametrize("pass_", [_lib.PASS_FWD, _lib.PASS_BWD, _lib.PASS_FWD_KEEP])
+@pytest.mark.parametrize("K,V,gk", [(64, 64, BF), (128, 128, BF), (64, 128, torch.float32), (128, 64, BF)])
+def test_ks_gated_copy_under_the_classic_route(K, V, gk, pass_):
+    """With the HDLA parameterisation no kernel reads it: for those who look, it is what the same k has beside plain a, b."""
+    B, T, H, P, lib = 2, 40, 3, _lib.ptr, _lib.load()
+    inp = make_inputs(62, B, T, H, K, V, gk_div=1.0)
+    k, beta = torch.nn.functional.normalize(inp.k, dim=-1), 2.0 * torch.rand(B, T, H, generator=torch.Generator().manual_seed(8))
+    d = {n: t.to(BF).to(DEV) for n, t in (("q", inp.q), ("k", k), ("v", inp.v), ("a", inp.a), ("b", inp.b), ("beta", beta), ("do", inp.do))}
+    d["gk"], h0 = inp.gk.to(gk).to(DEV), inp.h0.to(DEV)
+    dims = _lib.make_dims(B, T, H, K, V, 2, B, BF, gk, 0.7, None, route=_lib.ROUTE_CLASSIC, segments=0)
+    L, got = _lib.workspace_layout(dims, pass_), []
+    for form in ("ab", "beta"):
+        ws = torch.full((lib.hdla_workspace_bytes(ctypes.byref(dims), pass_),), 255, dtype=torch.uint8, device=DEV)
+        head = [P(d["q"]), P(d["k"]), P(d["v"])] + ([P(d["a"]), P(d["b"]), None] if form == "ab" else [None, None, P(d["beta"])]) + [P(d["gk"]), P(h0)]
+        o, ht, stream = torch.empty_like(d["v"]), torch.empty_like(h0), _lib.current_stream(DEV)
+        if pass_ == _lib.PASS_FWD:
+            rc = lib.hdla_chunk_fwd_b(ctypes.byref(dims), *head, P(o), P(ht), None, 0, P(ws), ws.numel(), stream)
+        elif pass_ == _lib.PASS_FWD_KEEP:
+            rc = lib.hdla_chunk_fwd_keep(ctypes.byref(dims), *head, P(o), P(ht), P(ws), ws.numel(), stream)
+        else:
+            g = [torch.empty_like(d[n]) for n in ("q", "k", "v", "a", "b", "beta", "gk")] + [torch.empty_like(h0)]
+            out = [P(t) for t in g]
+            rc = lib.hdla_chunk_bwd_b(ctypes.byref(dims), *head, P(d["do"]), None, *out, None, 0, P(ws), ws.numel(), stream)
+        assert rc == 0
+        torch.cuda.synchronize()
+        got.append(G.pair_tiles(ws, L["KGT"], BF, H, L["nch"], K // 16, stride=L["SA_STRIDE"]))
+    assert torch.isfinite(got[0]).all() and torch.equal(got[0], got[1])
+
+
 def test_passes_that_have_none():
     for dtype, pass_ in ((BF, _lib.PASS_FWD), (BF, _lib.PASS_BWD_KEPT), (torch.float32, _lib.PASS_BWD), (torch.float32, _lib.PASS_FWD_KEEP)):
         L = _lib.workspace_layout(_lib.make_dims(1, 64, 2, 128, 128, 2, 1, dtype, dtype, 1.0, None), pass_)
