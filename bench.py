@@ -182,12 +182,13 @@ def measured_traffic(workload, kernel_key, K, V):
             if fused_mode is not None and k.startswith("fused_kernel<") and targs[2:] == [str(K), str(V), fused_mode, "false"]:
                 return rec["hbm_bytes_per_launch"]
             continue
-        # scan_out<K, V, NWC, KEPT> (the forward pass's scan), scan_grad<K, V, NWC> (both of the backward pass); of packed sequences that share
-        # the device by their lengths scan_out_share<K, V, KEPT> and scan_grad_share<K, V>
+        # scan_out<K, V, NWC, KEPT, HD> (the forward pass's scan; KEPT 0: nothing is left for a backward pass), scan_grad<K, V, NWC, HD> (both of the backward pass); of packed
+        # sequences that share the device by their lengths scan_out_share<K, V, KEPT, HD> and scan_grad_share<K, V, HD>; in older summaries KEPT is false or true, and there is no HD
         if name in ("scan_fwd", "scan_pair"):
-            if k.startswith(("scan_out_kernel<", "scan_out_share_kernel<") if name == "scan_fwd" else ("scan_grad_kernel<", "scan_grad_share_kernel<")) and \
-                    targs[:2] == [str(K), str(V)] and targs[-1] != "true":
-                return rec["hbm_bytes_per_launch"]
+            kind, rest = k.split("<")[0], targs[2:]
+            for of, width in ((("scan_out_kernel", 1), ("scan_out_share_kernel", 0)) if name == "scan_fwd" else (("scan_grad_kernel", 1), ("scan_grad_share_kernel", 0))):
+                if kind == of and targs[:2] == [str(K), str(V)] and rest[width:] in ([["0", "false"], ["false"]] if name == "scan_fwd" else [["false"], []]):
+                    return rec["hbm_bytes_per_launch"]
             continue
         if not k.startswith(name + "_kernel<"):
             continue

@@ -530,8 +530,8 @@ extern "C" int hdla_rows_gemm_norm(int32_t M, int32_t N, int32_t K, const float*
     const bf16* wp = static_cast<const bf16*>(w);
     bf16* yp = static_cast<bf16*>(y);
     // Waves and blocks a go as ask for all of K at once, as far as the registers reach: sixteen waves for K = 2048, where eight asked twice.  us a decode step of
-    // the layer, as a graph's replay, eight / sixteen: 16 sequences, 2048 channels 24.4 / 23.4, 4 21.4 / 20.5, 1 20.9 / 19.8; 16, 1024 channels, whose K eight have in one
-    // go, 13.9 / 14.6.
+    // the layer, as a graph's replay, eight / sixteen: 16 sequences, 2048 channels 24.4 / 23.4, 4 21.4 / 20.5, 1 20.9 / 19.8; 16, 1152 channels 22.5 / 21.3, 1536 22.9 / 22.1, 1792 23.9 / 23.5; 16, 1024
+    // channels, whose K eight have in one go, 13.9 / 14.6.
 #define HDLA_ROWS(UNR, WAVES)                                                                                                                       \
     hipLaunchKernelGGL((rows_gemm_kernel<1, 1, UNR, true, WAVES>), grid, dim3(64 * WAVES), 0, s, nullptr, 0LL, wp, (long long)ldw, yp, (long long)ldy, M, N, K, nrm)
     if (K <= 64 * ROW_WAVES) HDLA_ROWS(2, ROW_WAVES);

@@ -1,5 +1,6 @@
 """The kernels that bench.py looks up in the committed counter summary are in it under the names that they have."""
 import importlib.util
+import json
 import os
 
 import pytest
@@ -29,3 +30,16 @@ def test_the_norm(bench, rows):
     # stays in the last-level cache
     least = 5 * 2 * 1024 * rows
     assert 0.9 * least < bench.norm_traffic(rows) < 1.2 * least
+
+
+def test_launches_of_other_kinds_are_not_taken(bench, tmp_path, monkeypatch):
+    """Scans that leave something for a backward pass, and those of the HDLA parameterisation, whatever their place in the summary."""
+    names = {"scan_out_kernel<128, 128, 2, 1, false>": 1, "scan_out_kernel<128, 128, 2, 2, false>": 2, "scan_out_kernel<128, 128, 2, 0, true>": 3, "scan_out_share_kernel<128, 128, 2, false>": 4,
+             "scan_out_share_kernel<128, 128, 0, true>": 5, "scan_grad_kernel<128, 128, 2, true>": 6, "scan_grad_share_kernel<128, 128, true>": 7, "scan_rev_share_kernel<128, 128>": 8}
+    (tmp_path / "profiles").mkdir()
+    monkeypatch.setattr(bench, "ROOT", str(tmp_path))
+    for more, want in (({}, (None, None)), ({"scan_out_share_kernel<128, 128, 0, false>": 10, "scan_grad_share_kernel<128, 128, false>": 11}, (10, 11)),
+                       ({"scan_out_kernel<128, 128, 4, 0, false>": 12, "scan_grad_kernel<128, 128, 4, false>": 13}, (12, 13))):
+        table = {"varlen": {n: {"hbm_bytes_per_launch": b} for n, b in {**names, **more}.items()}}
+        (tmp_path / "profiles" / "hbm_traffic.json").write_text(json.dumps(table))
+        assert tuple(bench.measured_traffic("varlen", k, 128, 128) for k in ("fwd.scan_fwd", "bwd.scan_pair")) == want
