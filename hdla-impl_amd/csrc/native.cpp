@@ -230,9 +230,16 @@ void chunk_forward(const ChunkIn& x, const hdla_dims& d, bool want_ht, Plan* pla
             size_t ws_fwd = 0, ws_bwd = 0;
             const size_t all = api.states_plan(&d, &ws_fwd, &ws_bwd);
             if (all) left = kept_room(x.q, (int64_t)all);
+            Tensor ws;
+            if (left.defined()) {
+                try {
+                    ws = bytes_like(x.q, ws_fwd);
+                } catch (const c10::OutOfMemoryError&) {
+                    left = Tensor();                      // (a call without the buffer needs less)
+                }
+            }
             if (left.defined()) {
                 plan->keep = KEEP_STATES;
-                const Tensor ws = bytes_like(x.q, ws_fwd);
                 check(api.chunk_fwd_states(&d, ptr(x.q), ptr(x.k), ptr(x.v), ptr(x.a), ptr(x.b), ptr(x.beta), ptr(x.gk), fptr(x.h0), ptr(o), fptr(ht),
                                            ptr(left), all, ptr(ws), ws_fwd, stream_of(x.q)), "hdla_chunk_fwd_states");
                 return;

@@ -145,8 +145,9 @@ def test_who_finds_room():
 
 
 @pytest.mark.gpu
-def test_where_the_states_cannot_be_had():
-    """A limit of torch's allocator between what the call needs and what it would keep."""
+@pytest.mark.parametrize("missing", ["buffer", "scratch"])
+def test_where_the_states_cannot_be_had(missing):
+    """A limit of torch's allocator between what the call needs and what it would keep, or between that and what it needs beside it."""
     gc.collect()
     torch.cuda.empty_cache()                                      # (or the inputs may lie in a block that has room for the buffer too)
     call = _Call(4, 2048, 16, 128, 128)
@@ -154,10 +155,22 @@ def test_where_the_states_cannot_be_had():
     gc.collect()
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
-    room = _lib.load().hdla_workspace_bytes(ctypes.byref(d), _lib.PASS_FWD) + call.do.numel() * 2 + (24 << 20)   # (the allocator's blocks of 2 and 20 MiB)
-    assert room < call.states
+    blocks = 24 << 20                                             # (the allocator's blocks of 2 and 20 MiB)
+    room = _lib.load().hdla_workspace_bytes(ctypes.byref(d), _lib.PASS_FWD) + call.do.numel() * 2 + blocks
+    assert room < call.states and blocks < _plan(4, 2048, 16, 128, 128)[1]
+    if missing == "scratch":
+        room = call.states + call.do.numel() * 2 + blocks
+    limit = lambda more: torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + more) / torch.cuda.get_device_properties(0).total_memory)
+    gaps = []                                                     # what is free in the blocks of what is held
     try:
-        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + room) / torch.cuda.get_device_properties(0).total_memory)
+        limit(0)
+        for size in (64 << 20, 16 << 20, 2 << 20):
+            try:
+                while True:
+                    gaps.append(torch.empty(size, dtype=torch.uint8, device=DEV))
+            except torch.OutOfMemoryError:
+                pass
+        limit(room)
         held = call.forward()
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
