@@ -273,7 +273,8 @@ def chunk_hrdplr_delta_rule(
     until the backward pass (1.1 to 1.7 times the bytes of q, k, v, a, b, gk together), which then skips recomputing
     them; False is closest to the reference's behaviour, where only the inputs are kept (hrdplr.py:137) and the backward pass
     recomputes (:161-198): here the fused route's record is kept beside them.  None (and HDLA_HIP_KEEP_FORWARD unset): kept
-    where that is at most 256 MiB and the route has no record, and only as long as all calls whose backward pass is still to come hold
+    where that is at most 256 MiB and the route has no record, or, of larger bf16 calls of many (sequence, head) pairs, together with the states
+    that enter the chunks, and only as long as all calls whose backward pass is still to come hold
     at most 1 GiB a device that way; beyond, and where the memory cannot be had, the same bits are recomputed.
     HDLA_HIP_INPUTS_ONLY=1: strictly the inputs, unless True.  Results agree to rounding.
     """
