@@ -25,7 +25,7 @@ def test_against_the_python_code(B, T, d, H):
     got = step()
     m._forward_native = lambda *_: None
     want = step()
-    # every stage of both rounds its result to bf16 (2^-9 of it at the most), a dozen of them one behind the other, in other orders of sums
+    # every stage of both rounds its result to bf16 (2^-8 of it at the most), a dozen of them one behind the other, in other orders of sums
     for n, a, b in zip(["y", *names], got, want):
         assert a.shape == b.shape and torch.isfinite(a.float()).all(), n
         rel = (a.double() - b.double()).norm() / b.double().norm().clamp_min(1e-30)

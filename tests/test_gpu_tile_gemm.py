@@ -44,7 +44,7 @@ def test_against_float64(M, N, K):
         y = torch.full((M + 1, N + 8), nan, dtype=torch.bfloat16, device=DEV)
         assert f(M, N, K, xs.data_ptr(), xs.stride(0), ws.data_ptr(), ws.stride(0), turned, y.data_ptr(), y.stride(0), torch.cuda.current_stream().cuda_stream) == 0
         got = y[:M, :N].double()
-        # rounding to bf16: half a unit, 2^-9 of each value; sums of K products in 32 bits: K 2^-24 of the sum of their absolute values
+        # rounding to bf16: half a unit, at most 2^-8 of each value; sums of K products in 32 bits: K 2^-24 of the sum of their absolute values
         bound = want.abs() * 2.0 ** -8 + K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T).to(DEV)
         assert ((got - want).abs() <= bound).all()
         assert torch.isnan(y[M]).all() and torch.isnan(y[:, N:]).all()
